@@ -106,9 +106,10 @@ MI355X_API mi355x_status mi355x_stream_release(void* stream);
  * x by Q4_0 or by a small Q8_0, Q4_K or Q6_K matrix; Q8_0 weights are read
  * once for up to eight rows) or kernels on the int8 matrix cores (Q4_0 from two
  * rows on: up to some tens of rows a kernel that reads W once per eight rows,
- * beyond them a tiled one, and from some hundreds of rows by a large matrix the
- * same integers through the binary16 matrix cores, with the tiled one's bits,
- * which takes a workspace of 2 N K bytes in the stream's scratch; two to eight
+ * beyond them a tiled one, and from some hundreds of rows by a large matrix x as
+ * pairs of binary16 through the binary16 matrix cores, within the fixed point's
+ * bound (below), which takes a workspace of 2 N K bytes and more in the stream's
+ * scratch; two to eight
  * rows by a large Q8_0
  * matrix; Q4_K, Q6_K from enough rows on); which one ran changes the results
  * only by the order of float32 additions (Q4_0, Q8_0), or not at all (Q8_0
@@ -469,8 +470,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * release-acquire one at device scope, 2 also stores and loads the shares plainly (both to be measured; 1 restores).
  * "q4_0.fx_rows" = n sends Q4_0 products of at least n rows of float32 x to the
  * int8 matrix cores whatever the shape (0: the built-in cost model);
- * "q4_0.fx_pairs" = 0 keeps those products off the binary16 form of that
- * kernel, 2 sends them all there (1: its cost model).
+ * "q4_0.fx_pairs" = 0 keeps those products off the binary16 matrix cores, 2
+ * sends them all there as digits with the int8 form's bits, 3 as pairs of binary16
+ * (1: pairs, by the cost models).
  * "qgemm.blocks" = 0 keeps the exact Q4_0 products of mi355x_qgemm_bf16 on the
  * kernel that needs no workspace, 2 sends them all through the panel of the
  * weights' integers (1: by shape).

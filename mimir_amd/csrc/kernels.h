@@ -292,10 +292,16 @@ bool qgemm_q4_0_fx_pays(const void* W, int64_t M, int64_t N, int64_t K);  // and
 double qgemm_q4_0_fx_cost_us(int64_t M, int64_t N, int64_t K);           // about what it takes, conversion aside
 hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st);
 bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K);  // against the int8 form, its pass over W included
-size_t q4_0_fx16_act_bytes(int64_t K);
+size_t q4_0_fx16_act_bytes(int64_t M, int64_t K);
 hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
-size_t qgemm_q4_0_fx16_ws_bytes(int64_t N, int64_t K);
+size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st);
+// Up to three matrices by the same converted rows in one product; swiglu: part 0's y = silu(x . W0^T) (x . W1^T). resid: one part only.
+struct Fx16Part { const void* W; float* y; int64_t N; };
+size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K);  // as much as any number of rows can use
+bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes);
+hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, int64_t K, double eps, hipStream_t st);  // a norm and the conversion for it
+hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
 void set_q4_0_fx16(int v);  // measurement aid: 0 keeps every product on the int8 form
 
 // Prompt-sized Q4_0 product on the matrix cores (qgemm_q4_0.hip): X [M, K]

@@ -85,8 +85,11 @@ struct Model : Decoder {
 int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0) {
     switch (w.dtype) {
     case kQ4_0:
-        if (qgemm_q4_0_fx_pays(w.buf.p, rows, w.n, w.k))
-            return panel_bytes >= qgemm_q4_0_fx16_ws_bytes(w.n, w.k) && qgemm_q4_0_fx16_pays(rows, w.n, w.k) ? kActFxPairs : kActFx;
+        if (rows > 1 && panel_bytes) {
+            const Fx16Part alone{w.buf.p, nullptr, w.n};
+            if (qgemm_q4_0_fx16_parts_pay(&alone, 1, false, rows, w.k, panel_bytes)) return kActFxPairs;
+        }
+        if (qgemm_q4_0_fx_pays(w.buf.p, rows, w.n, w.k)) return kActFx;
         return q4_0_fixed_point_ok(w.buf.p, w.k) ? kActQ4 : kActNone;
     case kQ8_0: return q8_act_fits(w.k) ? kActQ8 : kActNone;
     case kQ4_K: case kQ6_K: return kActKQ;
@@ -94,13 +97,15 @@ int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0) {
     }
 }
 
-size_t act_row_bytes(int cls, int64_t K) {
+// Bytes of `rows` converted rows of K.
+size_t act_bytes(int cls, int64_t rows, int64_t K) {
+    if (cls == kActFxPairs) return q4_0_fx16_act_bytes(rows, K);
+    const size_t n = (size_t)rows;
     switch (cls) {
-    case kActQ4: return q4_0_act_bytes(K);
-    case kActQ8: return q8_act_bytes(K);
-    case kActKQ: return kq_act_bytes(K);
-    case kActFx: return q4_0_fx_act_bytes(K);
-    case kActFxPairs: return q4_0_fx16_act_bytes(K);
+    case kActQ4: return n * q4_0_act_bytes(K);
+    case kActQ8: return n * q8_act_bytes(K);
+    case kActKQ: return n * kq_act_bytes(K);
+    case kActFx: return n * q4_0_fx_act_bytes(K);
     default: return 0;
     }
 }
@@ -113,7 +118,7 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
     for (const Weight* w : ws) {
         int cls = act_class(*w, rows, m.fx_panel.bytes);
         if (cls == kActNone || done[cls]) continue;
-        size_t need = act_row_bytes(cls, K) * (size_t)rows;
+        size_t need = act_bytes(cls, rows, K);
         if (m.act[cls].bytes < need) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: activation scratch of %zu bytes, need %zu", m.act[cls].bytes, need);
         hipError_t e = cls == kActQ4   ? q4_0_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActQ8 ? q8_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
@@ -135,8 +140,12 @@ mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_
     hipError_t e;
     switch (w.dtype) {
     case kQ4_0:
-        e = cls == kActFx || cls == kActFxPairs
-                ? qgemm_q4_0_fx(w.buf.p, m.act[cls].p, y, resid, rows, w.n, w.k, cls == kActFxPairs ? m.fx_panel.p : nullptr, m.stream)
+        if (cls == kActFxPairs) {
+            const Fx16Part alone{w.buf.p, y, w.n};
+            e = qgemm_q4_0_fx16_parts(&alone, 1, false, m.act[cls].p, resid, rows, w.k, m.fx_panel.p, m.fx_panel.bytes, m.stream);
+            break;
+        }
+        e = cls == kActFx   ? qgemm_q4_0_fx(w.buf.p, m.act[cls].p, y, resid, rows, w.n, w.k, nullptr, m.stream)
             : cls == kActQ4 ? qgemv_q4_0_act(a, kNoTune, m.stream)
                             : qgemv_q4_0(a, kNoTune, m.stream);
         break;
@@ -150,6 +159,27 @@ mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_
     default: return capi_fail(MI355X_ERR_DTYPE, "mi355x: llama: a linear weight of dtype %d", w.dtype);
     }
     LLM_HIP(e, "linear");
+    return MI355X_OK;
+}
+
+// The products of one x by several Q4_0 matrices, or silu(gate) up of two, as one (qgemm_q4_0_fx16_parts), where that pays:
+// *done says whether it was done. x is normalized with the weights `norm` as it is converted.
+mi355x_status linear_parts(Model& m, std::initializer_list<const Weight*> ws, std::initializer_list<float*> ys, bool swiglu, const float* x, const Weight& norm,
+                           int64_t rows, bool* done) {
+    Fx16Part part[3];
+    const int64_t K = (*ws.begin())->k;
+    int n = 0;
+    *done = false;
+    for (const Weight* w : ws) {
+        if (w->dtype != kQ4_0 || w->k != K) return MI355X_OK;
+        part[n] = Fx16Part{w->buf.p, swiglu && n ? nullptr : ys.begin()[n], w->n};
+        n++;
+    }
+    if (rows < 2 || !m.fx_panel.bytes || !qgemm_q4_0_fx16_parts_pay(part, n, swiglu, rows, K, m.fx_panel.bytes)) return MI355X_OK;
+    if (m.act[kActFxPairs].bytes < act_bytes(kActFxPairs, rows, K)) return MI355X_OK;
+    LLM_HIP(rmsnorm_fx16(x, norm.buf.as<float>(), m.act[kActFxPairs].p, rows, K, m.c.eps, m.stream), "norm");
+    LLM_HIP(qgemm_q4_0_fx16_parts(part, n, swiglu, m.act[kActFxPairs].p, nullptr, rows, K, m.fx_panel.p, m.fx_panel.bytes, m.stream), "linear");
+    *done = true;
     return MI355X_OK;
 }
 
@@ -185,11 +215,15 @@ static mi355x_status forward(Model& m, int64_t s) {
     };
     for (int i = 0; i < c.layers; i++) {
         Block& b = m.blocks[i];
-        LLM_HIP(rmsnorm(x, b.attn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "attn_norm");
-        if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.q, &b.k, &b.v}, done)) return st;
-        if (mi355x_status st = linear(m, b.q, h, q, rows)) return st;
-        if (mi355x_status st = linear(m, b.k, h, k, rows)) return st;
-        if (mi355x_status st = linear(m, b.v, h, v, rows)) return st;
+        bool together;
+        if (mi355x_status st = linear_parts(m, {&b.q, &b.k, &b.v}, {q, k, v}, false, x, b.attn_norm, rows, &together)) return st;
+        if (!together) {
+            LLM_HIP(rmsnorm(x, b.attn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "attn_norm");
+            if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.q, &b.k, &b.v}, done)) return st;
+            if (mi355x_status st = linear(m, b.q, h, q, rows)) return st;
+            if (mi355x_status st = linear(m, b.k, h, k, rows)) return st;
+            if (mi355x_status st = linear(m, b.v, h, v, rows)) return st;
+        }
         if (b.biased()) {  // Linear.Forward: the bias behind the product, before the rotation (nn/layers.go:49-55)
             LLM_HIP(add_bias(q, b.q_bias.buf.as<float>(), rows, qd, m.stream), "q bias");
             LLM_HIP(add_bias(k, b.k_bias.buf.as<float>(), rows, kvd, m.stream), "k bias");
@@ -228,11 +262,14 @@ static mi355x_status forward(Model& m, int64_t s) {
         LLM_HIP(attention(at, (uint8_t*)m.act[0].p + kAttnTicketBytes, m.stream), "attention");
         if (mi355x_status st = convert_for(m, a, rows, qd, {&b.o}, done)) return st;
         if (mi355x_status st = onto_x(b.o, a)) return st;
-        LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "ffn_norm");
-        if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.gate, &b.up}, done)) return st;
-        if (mi355x_status st = linear(m, b.gate, h, gate, rows)) return st;
-        if (mi355x_status st = linear(m, b.up, h, up, rows)) return st;
-        LLM_HIP(swiglu(gate, up, sw, rows, c.hidden, c.hidden, m.stream), "swiglu");
+        if (mi355x_status st = linear_parts(m, {&b.gate, &b.up}, {sw, nullptr}, true, x, b.ffn_norm, rows, &together)) return st;
+        if (!together) {
+            LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "ffn_norm");
+            if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.gate, &b.up}, done)) return st;
+            if (mi355x_status st = linear(m, b.gate, h, gate, rows)) return st;
+            if (mi355x_status st = linear(m, b.up, h, up, rows)) return st;
+            LLM_HIP(swiglu(gate, up, sw, rows, c.hidden, c.hidden, m.stream), "swiglu");
+        }
         if (mi355x_status st = convert_for(m, sw, rows, c.hidden, {&b.down}, done)) return st;
         if (mi355x_status st = onto_x(b.down, sw)) return st;
     }
@@ -699,18 +736,31 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
     const int64_t kmax = c.hidden > qd ? (c.hidden > c.embed ? c.hidden : c.embed) : (qd > c.embed ? qd : c.embed);
     for (int cls = 1; cls < kActClasses; cls++) {
         int64_t kk = cls == kActKQ ? (kmax + 255) / 256 * 256 : cls == kActFx || cls == kActFxPairs ? (kmax + 127) / 128 * 128 : (kmax + 63) / 64 * 64;
-        LLM_HIP(m->act[cls].alloc(act_row_bytes(cls, kk) * rows + 64), "hipMalloc(activations)");
+        LLM_HIP(m->act[cls].alloc(act_bytes(cls, rows, kk) + 64), "hipMalloc(activations)");
     }
     LLM_HIP(m->act2.alloc(q4_0_act_bytes((c.hidden + 63) / 64 * 64) * c.batch + 64), "hipMalloc(activations)");
     {
-        // the workspace of the fixed-point product's binary16 form, which calls of some hundreds of rows take: the largest matrix's
+        // the workspace of the Q4_0 product's binary16 form, which calls of some tens of rows and more take: the largest matrix's, or
+        // that of those that are multiplied together
         size_t panel = 0;
-        for (const Block& b : m->blocks)
-            for (const Weight* w : {&b.q, &b.k, &b.v, &b.o, &b.gate, &b.up, &b.down, &b.qkv, &b.gate_up})
-                if (w->set() && w->dtype == kQ4_0 && qgemm_q4_0_fx16_ws_bytes(w->n, w->k) > panel) panel = qgemm_q4_0_fx16_ws_bytes(w->n, w->k);
+        auto want = [&](std::initializer_list<const Weight*> ws) {
+            Fx16Part part[3];
+            int n = 0;
+            for (const Weight* w : ws) {
+                if (w->dtype != kQ4_0 || w->k != (*ws.begin())->k) return;
+                part[n++] = Fx16Part{w->buf.p, nullptr, w->n};
+            }
+            const size_t bytes = qgemm_q4_0_fx16_parts_ws_bytes(part, n, (*ws.begin())->k);
+            panel = bytes > panel ? bytes : panel;
+        };
+        for (const Block& b : m->blocks) {
+            for (const Weight* w : {&b.q, &b.k, &b.v, &b.o, &b.gate, &b.up, &b.down}) want({w});
+            want({&b.q, &b.k, &b.v});
+            want({&b.gate, &b.up});
+        }
         m->fx_panel.release();
         m->fx_panel.bytes = 0;
-        if (panel && rows >= 256) LLM_HIP(m->fx_panel.alloc(panel), "hipMalloc(fixed-point product workspace)");
+        if (panel && rows >= 48) LLM_HIP(m->fx_panel.alloc(panel), "hipMalloc(fixed-point product workspace)");
     }
     int chunk, nsplit;
     attention_plan(c.batch, c.heads, c.kv_heads, max_tokens, c.context, &chunk, &nsplit);

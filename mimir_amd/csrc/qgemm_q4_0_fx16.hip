@@ -1,42 +1,29 @@
-// The fixed-point Q4_0 product of many rows of float32 x (qgemm_q4_0_fx.hip: x as a 24-bit integer per element and
-// a float32 scale per block of 32, the exact integer sum per block, one FMA per block with the product of the two
-// scales), from some hundreds of rows on, through the binary16 matrix cores, with the same bits.
+// The Q4_0 product of many rows of float32 x, from some tens of rows on, on the binary16 matrix cores. x enters as a pair of
+// binary16 numbers an element, x 2^-e = h0 + h1 (22 bits; e the row's exponent), W as the integers n - 8, whose scales stay
+// out of the matrix cores: v_mfma_f32_32x32x16_f16 sums a block's products of h1 and of h0 (exact, added in float32) into
+// one c, and acc = fma(d, c, acc) is left to the vector unit, one instruction per output and block; 2^e follows at the end.
 //
-// What bounds the int8 form is the vector unit: three digit sums per output and block have to be joined, converted
-// and scaled, five instructions against three MFMAs per 1024 outputs. Here the 24-bit integer a of an element is cut
-// into two balanced 12-bit digits, a = d0 + 4096 d1 with d0 in [-2048, 2047] and d1 in [-2048, 2048], and each digit is
-// a binary16 number (binary16 holds integers up to 2048 exactly). The weights enter as the binary16 integers n - 8. A
-// v_mfma_f32_32x32x16_f16 then sums products that are integers below 2^15 into float32 sums that stay below 2^20:
-// every partial sum is an integer float32 holds exactly, in whatever order the instruction adds. Per block and
-// output, c0 = sum d0 (n - 8) and c1 = sum d1 (n - 8) are exact, fma(c1, 4096, c0) is the exact integer sum rounded
-// once to float32, which is what the int8 form's conversion of its 32-bit sum gives, and the block's term follows as
-// there: acc = fma(dw dx, that, acc), blocks in their order. Three vector instructions per output and block instead
-// of five, and no offset term (n - 8 is signed here).
+// What bounds it: four MFMAs of 32 cycles and sixteen FMAs of 4 per 32 x 32 outputs and block of 32, which hardly overlap
+// on a SIMD (128 + 64 cycles; one wide tile alone takes 1.3 us a block, those cycles at the full clock; with every unit at work
+// the clock falls and it is 1.75 us). The form before this one, which the int8 form's bits need (x as two 12-bit integer
+// digits with a float32 scale a block: two sums, an MFMA for dw dx and two FMAs an output: 128 + 32 + 128 cycles), stays for
+// "q4_0.fx_pairs" = 2. Whole calls, conversion and the pass over W included, digits before and halves now:
+//   2048 x 14336 x 4096   647 -> 461 us (521 TFLOP/s)      4096 x 28672 x 4096   2430 -> 1667 us (577 TFLOP/s)
+//   4096 x 4096 x 14336  1286 -> 910 us                    512 x 4096 x 14336    506 (int8 268) -> 155 us
+//   2048 x 4096 x 4096    184 -> 149 us                    512 x 14336 x 4096    183 -> 149 us
+// The error against 64 bits is no larger: 2.11e-7 of the result at K = 4096 (digits 2.31e-7), 3.84e-7 at 14336 (3.95e-7).
 //
-// Two launches. fx16_panel_kernel writes W's integers once as a binary16 panel P [N, K] (the pass the approximate
-// form's panel takes too, qgemm_f16_panel.hip, without the scales). qgemm_q4_0_fx16_kernel multiplies: a workgroup
-// of eight wavefronts owns 128 rows of x by 256 rows of W, a wavefront 64 by 64; a stage is a pair of blocks (64 of K):
-// the rows of x (128 bytes a row and block: 32 digits d0, then 32 digits d1), the rows of P (128 bytes a row: the two
-// blocks) and the scales. Operands go from global memory straight into LDS (global_load_lds_dwordx4) with the 16-byte
-// pieces of a row placed at piece ^ (row / 2 mod 8), so that the 32 rows of a fragment read fall on all banks; the
-// scales pass through registers (W's are read from the blocks themselves). Two stages, one barrier a stage.
+// Two launches, three where K is cut into shares. fx16_panel_kernel writes W's integers as binary16 and its scales as float32,
+// in the order in which a stage of LDS holds them; the conversion of x (fx16_halves_kernel, with a norm before it
+// where the decoder has one) does the same for x. So every load of the product is a whole KB from contiguous memory straight
+// into LDS (global_load_lds_dwordx4). A workgroup of eight wavefronts owns 256 x 256 outputs (a wavefront 64 x 128, three
+// stages of one block) where tiles are many, 128 x 256 (64 x 64, four stages) where they are few: 8 KB of fragments
+// from LDS per 16 MFMAs against 12. One barrier a block; a sub-tile's MFMAs are issued with the FMAs of the sub-tile before.
+// Where even those leave units idle, K is cut into shares whose sums a third launch adds.
 //
-// The products of the two scales come from the matrix cores as well: dw dx over a sub-tile is an outer product, an
-// MFMA with K = 1 on float32 operands (one exact product per output, nothing added: the rounding of a multiplication).
-// That leaves the vector unit two instructions per output and block.
-//
-// What was measured on the way (2048 and 4096 rows by 14336 x 4096): tiles of 128 x 128 in workgroups of four
-// wavefronts, two a compute unit, with everything loaded straight into LDS and three stages, 335 to 340 TFLOP/s against
-// 350 to 360 here (half as many bytes again from L2 per product); the barrier moved to the middle of a block with the
-// next block's fragments read under the last vector work, and the order of MFMAs and vector instructions inside a
-// group imposed: no change. Under this kernel the device clock settles near 1.6 GHz, lower the fewer cycles a variant
-// needs: the time did not follow the cycle counts.
-//
-// x converted by fx16_convert_kernel: X16 [M, K / 32, 64] binary16 digits, then XS [M, K / 32] float32 scales; the
-// integers and scales are those of fx_convert_kernel and q4_convert_item.
+// Several matrices by the same x (q, k and v; gate and up, SwiGLU included) are one product: Parts.
 //
 // Reference semantics: the float32 product with the dequantized weights (io/mim/dtype.go:118-123,
-// backend/cpu/gemv.go:73-104), to which the result agrees within 1e-3.
 #include "device_util.h"
 #include "kernels.h"
 #include "q4_act.h"
@@ -49,29 +36,32 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 
-constexpr int kBM = 128;        // rows of x a workgroup
-constexpr int kBN = 256;        // rows of W a workgroup
-constexpr int kRowBytes = 128;  // a row of a stage: 64 binary16
-constexpr int kLoads = 8;       // 1 KB loads (8 rows) a wavefront issues per stage: 512 rows
-constexpr int kMinRows = 256;   // fewer rows stay with the int8 form
+constexpr int kMinRows = 256;     // fewer rows of one matrix stay with the int8 form,
+constexpr int kMinPartRows = 48;  // of several together
 
-// A stage in LDS: the rows of x for the even block, for the odd block, the rows of P, then the scales.
-struct Stage {
-    static constexpr int a = 0;                          // [2][kBM] rows
-    static constexpr int b = 2 * kBM * kRowBytes;        // [kBN] rows
-    static constexpr int sx = b + kBN * kRowBytes;       // float [2][kBN]: x's in the first kBM of each, the rest so that every thread stores
-    static constexpr int sw = sx + 2 * kBN * 4;          // float [2][kBN]
-    static constexpr int bytes = sw + 2 * kBN * 4;
-};
-static_assert(Stage::bytes % 1024 == 0, "stages start on the boundary the loads assume");
-constexpr size_t kLdsBytes = 2 * (size_t)Stage::bytes;
+// Operands lie in memory as a stage of LDS holds them, so that every load is a whole KB: granules of 32 rows by one block
+// of 32 of K, the granules of a strip of 32 rows one after the other.
+constexpr int kGranuleX = 2048;   // binary16 of a granule of x: 32 rows of 128 bytes, a row's 16-byte pieces turned (turn_of)
+constexpr int kGranuleP = 1024;   // of W: two halves of the block, each in the order of lanes of an MFMA's operand
+constexpr int kGranuleS = 32;     // float32 scales of W
+constexpr int kGroup = 8;         // blocks whose scales come into LDS together: a KB a strip
+
+// x: row m's pieces 4 part + 2 half + hi of a block, hi which eight of the half's sixteen, lie at piece ^ turn, so that the
+// 32 rows of a fragment read fall on all banks while a row's block stays one line for the kernels that write it.
+__host__ __device__ inline int64_t row_at(int m, int nb) { return (int64_t)(m >> 5) * nb * kGranuleX + (m & 31) * 64; }
+__host__ __device__ inline int turn_of(int m) { return (m >> 1) & 7; }
+
+// How a row of x is held. The row's information is {exponent, form}.
+enum Form { kHalves = 0, kBlockHalves = 1, kDigits = 2 };
 
 // Thread t takes elements 4t..4t+3 of row blockIdx.y; a block's eight threads are consecutive lanes.
-__global__ __launch_bounds__(256) void fx16_convert_kernel(const float* __restrict__ x, int64_t x_row_stride, int K, uint16_t* __restrict__ X16,
-                                                           float* __restrict__ XS) {
+__global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restrict__ x, int64_t x_row_stride, int K, uint16_t* __restrict__ X16,
+                                                          float* __restrict__ XS, int2* __restrict__ RS) {
     const int nb = K >> 5;
+    if (blockIdx.x == 0 && threadIdx.x == 0) RS[blockIdx.y] = make_int2(0, kDigits);
     const float* xr = x + (int64_t)blockIdx.y * x_row_stride;
-    uint16_t* row = X16 + (int64_t)blockIdx.y * nb * 64;
+    uint16_t* row = X16 + row_at((int)blockIdx.y, nb);
+    const int turn = turn_of((int)blockIdx.y);
     float* xscale = XS + (int64_t)blockIdx.y * nb;
     const int nq = K >> 2;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nq; t += gridDim.x * blockDim.x) {
@@ -106,25 +96,164 @@ __global__ __launch_bounds__(256) void fx16_convert_kernel(const float* __restri
             a = a > kFixMax ? kFixMax : a < -kFixMax ? -kFixMax : a;
             const int d0 = ((a + 2048) & 4095) - 2048;  // balanced: -2048..2047
             const int d1 = (a - d0) >> 12;              // -2048..2048
-            lo[k] = (_Float16)(float)d0;
-            hi[k] = (_Float16)(float)d1;
+            lo[k] = (_Float16)(float)(t & 8 ? -d0 : d0);  // odd blocks with their sign turned (tile_body)
+            hi[k] = (_Float16)(float)(t & 8 ? -d1 : d1);
         }
-        uint16_t* at = row + (t >> 3) * 64 + 4 * (t & 7);
-        __builtin_memcpy(at, lo, 8);
-        __builtin_memcpy(at + 32, hi, 8);
+        uint16_t* at = row + (int64_t)(t >> 3) * kGranuleX;
+        const int piece = (t & 7) >> 1, within = 4 * (t & 1);
+        __builtin_memcpy(at + ((piece ^ turn) << 3) + within, lo, 8);
+        __builtin_memcpy(at + (((4 + piece) ^ turn) << 3) + within, hi, 8);
         if ((t & 7) == 0) xscale[t >> 3] = scale;
     }
 }
 
-// Sixteen weights a thread: the low and the high nibbles of eight bytes of a block, as the binary16 integers n - 8.
-__global__ __launch_bounds__(256) void fx16_panel_kernel(const uint8_t* __restrict__ W, uint16_t* __restrict__ P, int64_t halves) {
-    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
-    for (int64_t t = first; t < halves; t += stride) {
-        const int q = (int)(t & 1);
-        const uint16_t* src = (const uint16_t*)(W + (t >> 1) * 18 + 2 + 8 * q);  // blocks are 2-byte aligned, no more
+// A workgroup converts a row of x into halves: x 2^-e = h0 + h1, h0 the binary16 next to it and h1 the binary16 next to
+// what that leaves. e makes the row's largest element lie in [2^14, 2^15), so that an element keeps 22 bits, and at least
+// an absolute 2^-25: 2^-24 of its block's largest as long as that is no less than 2^-15 of the row's, about what the
+// fixed point holds (2^-23.9). A row that has a smaller block (zeros aside) takes an exponent a block instead.
+// With NORM the row is normalized first (rmsnorm_kernel's operations, one by one): x over its root mean square, times w.
+// Memory bounds it: 8 bytes an element. ITEMS: eights of elements a thread holds between the row's maximum and its halves, so that x
+// is read once (4096 rows of 14336: 105 us, 156 reading it twice and storing eight bytes a thread); 0: rows of more than 16384, read twice.
+template <int ITEMS, bool NORM>
+__global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restrict__ x, const float* __restrict__ w, int64_t x_row_stride, int K,
+                                                          uint16_t* __restrict__ X16, float* __restrict__ XS, int2* __restrict__ RS, float inv_k, float eps) {
+    constexpr int kHeld = ITEMS ? ITEMS : 1;
+    const int nb = K >> 5, n8 = K >> 3, tid = threadIdx.x;
+    const float* xr = x + (int64_t)blockIdx.x * x_row_stride;
+    uint16_t* row = X16 + row_at((int)blockIdx.x, nb);
+    const int turn = turn_of((int)blockIdx.x);
+    float* xscale = XS + (int64_t)blockIdx.x * nb;
+    __shared__ uint32_t part[2][4];
+    float scale = 1.f;
+    if (NORM) {
+        const float ss = wave_sum(strided_sum_squares(xr, K, tid));
+        if ((tid & 63) == 0) part[0][tid >> 6] = __builtin_bit_cast(uint32_t, ss);
+        __syncthreads();
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[i] = __builtin_bit_cast(float, part[0][i]);
+        const float total = (p[0] + p[1]) + (p[2] + p[3]);
+        const float ms = total * inv_k;
+        scale = 1.0f / __builtin_sqrtf(ms + eps);
+        __syncthreads();
+    }
+    auto load = [&](int t, float v[8]) {
+        __builtin_memcpy(v, xr + 8 * (int64_t)t, 32);
+        if (NORM) {
+            float g[8];
+            __builtin_memcpy(g, w + 8 * (int64_t)t, 32);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float n = v[k] * scale;
+                v[k] = n * g[k];
+            }
+        }
+    };
+    // the largest magnitude of the block that this thread and three neighbours hold, as the integer of its bits: the order is the
+    // same, a NaN or an infinity is the largest
+    auto block_top = [&](const float v[8]) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t a = __builtin_bit_cast(uint32_t, v[k]) & 0x7fffffffu;
+            top = a > top ? a : top;
+        }
+        uint32_t other = __builtin_bit_cast(uint32_t, dpp_f32<0xb1>(__builtin_bit_cast(float, top)));
+        top = other > top ? other : top;
+        other = __builtin_bit_cast(uint32_t, dpp_f32<0x4e>(__builtin_bit_cast(float, top)));
+        return other > top ? other : top;
+    };
+    uint32_t most = 0, least = 0x7f800000u;
+    float v[kHeld][8];
+    auto see = [&](int t, float u[8]) {
+        load(t, u);
+        const uint32_t top = block_top(u);
+        most = top > most ? top : most;
+        if (top != 0 && top < least) least = top;
+    };
+    if (ITEMS) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++)
+            if (tid + 256 * i < n8) see(tid + 256 * i, v[i]);
+    } else {
+        for (int t = tid; t < n8; t += 256) see(t, v[0]);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t a = (uint32_t)__shfl_xor((int)most, d), b = (uint32_t)__shfl_xor((int)least, d);
+        most = a > most ? a : most;
+        least = b < least ? b : least;
+    }
+    if ((tid & 63) == 0) {
+        part[0][tid >> 6] = most;
+        part[1][tid >> 6] = least;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        most = part[0][i] > most ? part[0][i] : most;
+        least = part[1][i] < least ? part[1][i] : least;
+    }
+    const bool finite = most < 0x7f800000u;
+    const float amax = __builtin_bit_cast(float, most), amin = __builtin_bit_cast(float, least);
+    auto exponent = [](float a) { return a > 0.f ? __builtin_amdgcn_frexp_expf(a) - 15 : 0; };  // a 2^-e in [2^14, 2^15)
+    const int e_row = finite ? exponent(amax) : 0;
+    const int form = finite && amin < amax * 0x1p-15f ? kBlockHalves : kHalves;
+    if (tid == 0) RS[blockIdx.x] = make_int2(finite ? e_row : INT32_MAX, form);
+    auto convert = [&](int t, const float u[8]) {
+        const int e = form == kBlockHalves ? exponent(__builtin_bit_cast(float, block_top(u))) : e_row;
+        const bool odd = t & 4;  // odd blocks with their sign turned (tile_body)
+        f16x8 h0, h1;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float a = finite ? __builtin_ldexpf(odd ? -u[k] : u[k], -e) : 0.f;
+            h0[k] = (_Float16)a;
+            h1[k] = (_Float16)(a - (float)h0[k]);
+        }
+        uint16_t* at = row + (int64_t)(t >> 2) * kGranuleX;
+        *(f16x8*)(at + (((t & 3) ^ turn) << 3)) = h0;
+        *(f16x8*)(at + (((4 + (t & 3)) ^ turn) << 3)) = h1;
+        if ((t & 3) == 0) xscale[t >> 2] = finite ? __builtin_ldexpf(1.f, e) : __builtin_nanf("");
+    };
+    if (ITEMS) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++)
+            if (tid + 256 * i < n8) convert(tid + 256 * i, v[i]);
+    } else {
+        for (int t = tid; t < n8; t += 256) {
+            load(t, v[0]);
+            convert(t, v[0]);
+        }
+    }
+}
+
+__host__ __device__ inline int scale_blocks(int nb) { return (nb + kGroup - 1) / kGroup * kGroup; }  // of a strip: whole groups
+
+// What is multiplied by the same x: up to three matrices, or gate and up, whose strips then lie in turn.
+struct Parts {
+    const uint8_t* W[3];
+    float* y[3];
+    int N[3];      // rows of W
+    int begin[3];  // first strip; those of parts that are not there lie past the last
+    int strips;    // of all
+    int swiglu;    // W[0] and W[1] are gate and up: y[0] gets silu(gate) up
+};
+
+// W's integers n - 8 as binary16 and its scales as float32, in granules; an odd block's scale is negative (tile_body says why). A
+// wavefront takes a strip's block: lane r + 32 q the eight bytes q of row r, whose low nibbles are piece q of the block's
+// first half and whose high nibbles of its second.
+__global__ __launch_bounds__(256) void fx16_panel_kernel(Parts parts, uint16_t* __restrict__ P, float* __restrict__ SW, int nb) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, q = lane >> 5;
+    const int strip = blockIdx.y;
+    const int part = parts.swiglu ? strip & 1 : strip >= parts.begin[2] ? 2 : strip >= parts.begin[1] ? 1 : 0;
+    const int n = (parts.swiglu ? strip >> 1 : strip - parts.begin[part]) * 32 + r, N = parts.N[part];
+    const uint8_t* row = parts.W[part] + (int64_t)(n < N ? n : N - 1) * nb * 18;  // past the matrix: its last row again
+    for (int b = blockIdx.x * 8 + wave; b < nb && b < (int)blockIdx.x * 8 + 8; b += 4) {
+        const uint8_t* block = row + b * 18;
+        const uint16_t* src = (const uint16_t*)(block + 2 + 8 * q);  // blocks are 2-byte aligned, no more
         const uint32_t raw[2] = {(uint32_t)src[0] | (uint32_t)src[1] << 16, (uint32_t)src[2] | (uint32_t)src[3] << 16};
         const f16x2 off = {(_Float16)1032.f, (_Float16)1032.f};
-        uint16_t* out = P + (t >> 1) * 32 + 8 * q;  // elements 8 q .. 8 q + 7 (low nibbles) and 16 more on (high nibbles)
+        uint16_t* out = P + ((int64_t)strip * nb + b) * kGranuleP + lane * 8;
 #pragma unroll
         for (int half = 0; half < 2; half++) {
             u32x4 v;
@@ -137,20 +266,22 @@ __global__ __launch_bounds__(256) void fx16_panel_kernel(const uint8_t* __restri
                 v[2 * i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p0) - off);
                 v[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p1) - off);
             }
-            *(u32x4*)(out + 16 * half) = v;
+            *(u32x4*)(out + 512 * half) = v;
         }
+        if (q == 0) SW[((int64_t)strip * scale_blocks(nb) + b) * kGranuleS + r] = f16_bits_to_f32(load_u16(block) ^ ((b & 1) << 15));
     }
 }
 
-// 16 bytes a lane from global memory into LDS: lane l's piece lands at lds_base + 16 l. Written out because the
+// A KB from global memory into LDS: lane l's 16 bytes from base + 16 l to lds_base + 16 l. Written out because the
 // compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand
 // (the compiler does not see them, so its own waits for the register loads of the scales can only be longer than
 // needed, never shorter: loads return in order). The instruction takes its LDS base from M0, which an asm statement
 // cannot name as clobbered: nothing else in this kernel uses M0, and it is set anew before every load.
-__device__ __forceinline__ void load_to_lds(const void* g, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g) : "memory");
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane16, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
 }
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+template <int N>
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // A die's workgroups (every eighth, round-robin) take a contiguous range of the tiles, the tile's rows of x varying
@@ -160,256 +291,570 @@ __device__ __forceinline__ int tile_of(int b, int ntiles) {
     return (b & 7) * per_die + (b >> 3);
 }
 
-__global__ __launch_bounds__(512) void qgemm_q4_0_fx16_kernel(const uint8_t* __restrict__ W, const uint16_t* __restrict__ P,
-                                                              const uint16_t* __restrict__ X16, const float* __restrict__ XS, float* y,
-                                                              const float* resid,  // may be y
-                                                              int M, int N, int K, int tiles_m, int ntiles) {
-    extern __shared__ __align__(1024) char lds[];
-    const int t = tile_of((int)blockIdx.x, ntiles);
-    if (t >= ntiles) return;  // the whole workgroup
-    const int m0 = (t % tiles_m) * kBM, n0 = (t / tiles_m) * kBN;
+// A workgroup's tile of y: WM x (8 / WM) wavefronts of (32 MT) x (32 NT) each, over STAGES stages of one block.
+template <int WM, int MT_, int NT_, int STAGES_>
+struct Shape {
+    static constexpr int WN = 8 / WM, MT = MT_, NT = NT_, STAGES = STAGES_;
+    static constexpr int BM = WM * 32 * MT, BN = WN * 32 * NT;
+    static constexpr int kChunksX = BM / 32 * 4, kChunksP = BN / 32 * 2;  // KB of a stage
+    static constexpr int kX = kChunksX / 8, kLoads = kX + kChunksP / 8;   // a wavefront issues a stage: kX of x, then P's
+    static constexpr int stage = (kChunksX + kChunksP) * 1024;
+    static constexpr int sw = STAGES * stage;                // float [2 groups][BN / 32][kGroup][32]
+    static constexpr int sw_group = BN / 32 * 1024;
+    static constexpr int sx = sw + 2 * sw_group;             // float [2][BM]: x's scales of two blocks, where they differ by block
+    static constexpr int total = sx + 2 * BM * 4;
+    static_assert(kChunksX % 8 == 0 && kChunksP % 8 == 0 && kLoads <= MT * NT && BN <= 256 && BM <= 512, "as many loads a wavefront, one with a sub-tile");
+};
+using Low = Shape<2, 2, 2, 4>;   // 128 x 256
+using Wide = Shape<4, 2, 4, 3>;  // 256 x 256
+constexpr int kLdsBytes = Low::total > Wide::total - 2 * 256 * 4 ? Low::total : Wide::total - 2 * 256 * 4;  // Wide has no scales of x
+
+struct Operands {
+    const uint16_t* P;
+    const float* SW;
+    const uint16_t* X16;
+    const float* XS;
+    const int2* RS;
+    const float* resid;  // may be y; added to what one part's y gets
+    float* sums;         // where K is cut into shares: [share][M][32 strips] float32, finished by fx16_sum_kernel
+    int M, nb;
+    Parts parts;
+};
+
+__device__ __forceinline__ float silu_times(float g, float u) {  // as swiglu_kernel's
+    const float e = __builtin_exp2f(g * (float)(-1.4426950408889634));
+    const float s = 1.0f / (1.0f + e);
+    const float a = g * s;
+    return a * u;
+}
+
+// One tile: rows m0 .. m0 + BM of x by columns n0 .. n0 + BN, blocks b0 .. b0 + count of K (b0 a multiple of a group), of rows of
+// x that are all of one form, or halves of either kind (kBlockHalves).
+//
+// An MFMA rounds its float32 sums downwards more often than upwards, and over the hundreds of blocks of a row that bias
+// adds up (4096 x 14336 by normal x: 3.97e-7 of the result, where exact sums of blocks give 3.945e-7). So odd blocks are multiplied with
+// their sign turned, x's halves and W's scales both: the bias cancels, 3.84e-7.
+template <class S, int FORM>
+__device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int b0, int count, float* sums, char* lds) {
+    constexpr int MT = S::MT, NT = S::NT;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3;
-    const int nb = K >> 5;
+    const int wm = wave / S::WN, wn = wave % S::WN;
+    const int M = o.M, nb = o.nb;
 
-    // This wavefront's loads: load g = kLoads wave + j brings rows [8 g, 8 g + 8) of the stage: x's rows for the even
-    // block, for the odd block, then P's. Rows past the matrix re-read its last row (their results are not stored).
-    const char* from[kLoads];
-    uint32_t into[kLoads];
-    int advance[kLoads];
+    // This wavefront's loads: KB kX wave + j of x's granules, then as many of P's. Strips past the matrix re-read its last
+    // strip (their results are not stored).
+    const char* from[S::kLoads];
+    uint32_t into[S::kLoads];
 #pragma unroll
-    for (int j = 0; j < kLoads; j++) {
-        const int first = 8 * (kLoads * wave + j);
-        const int row = first + (lane >> 3);
-        const int piece = (lane & 7) ^ ((row >> 1) & 7);
-        const uint16_t* base;
-        if (first < 2 * kBM) {
-            const int r = row & (kBM - 1), odd = row >> 7;
-            const int m = m0 + r < M ? m0 + r : M - 1;
-            base = X16 + ((size_t)m * nb + odd) * 64;
-            advance[j] = 2 * kRowBytes;
-        } else {
-            const int r = row - 2 * kBM;
-            const int n = n0 + r < N ? n0 + r : N - 1;
-            base = P + (size_t)n * K;
-            advance[j] = kRowBytes;
-        }
-        from[j] = (const char*)(base + 8 * piece);
-        into[j] = (uint32_t)(first * kRowBytes);
+    for (int j = 0; j < S::kLoads; j++) {
+        const bool of_x = j < S::kX;
+        const int c = of_x ? S::kX * wave + j : (S::kLoads - S::kX) * wave + j - S::kX;
+        const int strip = of_x ? m0 / 32 + c / 4 : n0 / 32 + c / 2, last = of_x ? (M - 1) / 32 : o.parts.strips - 1;
+        const int64_t at = (int64_t)(strip < last ? strip : last) * nb + b0;
+        from[j] = of_x ? (const char*)(o.X16 + at * kGranuleX) + (c & 3) * 1024 : (const char*)(o.P + at * kGranuleP) + (c & 1) * 1024;
+        into[j] = (of_x ? c : c + S::kChunksX) * 1024;
     }
-    // the scales: thread t takes block t % 2 of the stage for row t / 2 of W and of x (x's rows beyond kBM: loaded and
-    // stored like the others, so that no branch is needed, and never read)
-    const int srow = tid >> 1, sodd = tid & 1;
-    const uint8_t* wscale = W + ((size_t)(n0 + srow < N ? n0 + srow : N - 1) * nb + sodd) * 18;
-    const float* xscale = XS + (size_t)(m0 + srow < M ? m0 + srow : M - 1) * nb + sodd;
+    const uint32_t lane16 = lane * 16;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+    // W's scales: wavefront w brings strip w of the tile's, a group of blocks at a time
+    const bool has_sw = wave < S::BN / 32;
+    const char* sw_from;
+    {
+        const int strip = n0 / 32 + (has_sw ? wave : 0), last = o.parts.strips - 1;
+        sw_from = (const char*)(o.SW + ((int64_t)(strip < last ? strip : last) * scale_blocks(nb) + b0) * kGranuleS);
+    }
+    const uint32_t sw_into = lds0 + S::sw + wave * 1024;
+    // x's, where they differ by block: one a thread below BM
+    const float* xscale = o.XS + (int64_t)(m0 + (tid & (S::BM - 1)) < M ? m0 + (tid & (S::BM - 1)) : M - 1) * nb + b0;
 
     const int r32 = lane & 31, hi = lane >> 5;
-    const int swz = (r32 >> 1) & 7;
-    int piece_off[4];  // of a row's pieces 2 p + hi: of x, half p % 2 of digit p / 2; of P, half p % 2 of the stage's block p / 2
+    int piece_off[4];  // of pieces 2 p + hi: half p % 2 of part p / 2
 #pragma unroll
-    for (int p = 0; p < 4; p++) piece_off[p] = ((2 * p + hi) ^ swz) * 16;
-    const int a_row = (wm * 64 + r32) * kRowBytes, b_row = Stage::b + (wn * 64 + r32) * kRowBytes;
+    for (int p = 0; p < 4; p++) piece_off[p] = wm * MT * 4096 + r32 * 128 + ((2 * p + hi) ^ turn_of(r32)) * 16;
+    const int b_off = S::kChunksX * 1024 + wn * NT * 2048 + lane * 16;
 
-    f32x16 acc[2][2];
+    f32x16 acc[MT][NT], zero;
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int i = 0; i < 16; i++) zero[i] = 0.f;
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[mt][nt][i] = 0.f;
+        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = zero;
 
-    const int nstages = K / 64;
-    {
-        const float dw = f16_bits_to_f32(load_u16(wscale));
-        const float dx = *xscale;
+    auto load_stage = [&](int j, uint32_t slot, int step) {
+        load_to_lds(from[j], lane16, lds0 + slot + into[j]);
+        from[j] += (j < S::kX ? kGranuleX * 2 : kGranuleP * 2) * step;
+    };
+    if (has_sw) load_to_lds(sw_from, lane16, sw_into);
+    uint32_t fill = 0;  // the stage that is loaded next
+    for (int i = 0; i < S::STAGES - 1; i++) {
 #pragma unroll
-        for (int j = 0; j < kLoads; j++) load_to_lds(from[j], __builtin_amdgcn_readfirstlane(lds0 + into[j]));
-        ((float*)(lds + Stage::sw))[sodd * kBN + srow] = dw;
-        ((float*)(lds + Stage::sx))[sodd * kBN + srow] = dx;
+        for (int j = 0; j < S::kLoads; j++) load_stage(j, fill, i + 1 < count ? 1 : 0);
+        fill += S::stage;
     }
-    // No branches around the loads and stores: past the end the last stage is requested and stored again, into the
-    // buffer that is not being read.
-    for (int i = 0; i < nstages; i++) {
-        wait_loads();   // this wavefront's part of stage i has landed
-        lds_barrier();  // everyone's has, with the scales, and everyone has read the other stage for the last time
-        const int step = i + 1 < nstages ? 1 : 0;
-        const uint32_t next = lds0 + ((i + 1) & 1) * Stage::bytes;
-        char* next_p = lds + ((i + 1) & 1) * Stage::bytes;
-        const char* st = lds + (i & 1) * Stage::bytes;
-        wscale += 36 * step;
-        xscale += 2 * step;
-        const float next_dw = f16_bits_to_f32(load_u16(wscale));
-        const float next_dx = *xscale;
+    if (FORM != kHalves && tid < S::BM) ((float*)(lds + S::sx))[tid] = *xscale;
+    f32x16 c[2];  // kHalves: the sums of a sub-tile, finished with the next one's products
+    c[1] = zero;
+    float dlast = 0.f;
+    uint32_t use = 0;  // the stage that is multiplied
+    // No branches around the loads: past the end the last block is requested again, into a stage that is not read any more.
+    for (int i = 0; i < count; i++) {
+        wait_loads<S::kLoads*(S::STAGES - 2)>();  // this wavefront's part of block i has landed, and W's scales
+        lds_barrier();                             // everyone's has, and everyone has read the block before for the last time
+        const int step = i + S::STAGES < count ? 1 : 0;
+        const char* st = lds + use;
+        if (has_sw && (i & (kGroup - 1)) == 0 && i + kGroup < count) {  // the next group of W's scales, over the one before this
+            sw_from += 1024;
+            load_to_lds(sw_from, lane16, sw_into + ((i / kGroup + 1) & 1) * S::sw_group);
+        }
+        float next_dx = 0.f;
+        if (FORM != kHalves) {
+            xscale += i + 1 < count ? 1 : 0;
+            next_dx = *xscale;
+        }
+        f16x8 a[MT][2][2], b[2][2];  // a[mt][part][half], b[nt % 2][half]
+        auto read_b = [&](int nt) {
 #pragma unroll
-        for (int odd = 0; odd < 2; odd++) {
-            // half of the next stage's loads with each block
+            for (int h = 0; h < 2; h++) b[nt & 1][h] = *(const f16x8*)(st + b_off + nt * 2048 + h * 1024);
+        };
+        read_b(0);
 #pragma unroll
-            for (int j = odd * kLoads / 2; j < (odd + 1) * kLoads / 2; j++) {
-                from[j] += advance[j] * step;
-                load_to_lds(from[j], __builtin_amdgcn_readfirstlane(next + into[j]));
-            }
-            f16x8 a[2][2][2], b[2][2];  // a[mt][digit][half], b[nt][half]
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
+            for (int p = 0; p < 4; p++) a[mt][p >> 1][p & 1] = *(const f16x8*)(st + mt * 4096 + piece_off[p]);
+        read_b(1);
+        const char* sw = lds + S::sw + (i / kGroup & 1) * S::sw_group + wn * NT * 1024 + (i & (kGroup - 1)) * 128;
+        if (FORM == kHalves) {
+            float dw[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) dw[nt] = *(const float*)(sw + nt * 1024 + r32 * 4);
+            // A sub-tile's products are issued with the FMAs of the one before it, so that the vector unit works while the
+            // matrix cores do. What h0 leaves first: the smaller terms.
+#pragma unroll
+            for (int sub = 0; sub < MT * NT; sub++) {
+                const int nt = sub / MT, mt = sub % MT, was = (sub + MT * NT - 1) % (MT * NT);
+                if (mt == 0 && nt > 0 && nt + 1 < NT) read_b(nt + 1);
+                if (sub < S::kLoads) load_stage(sub, fill, step);
 #pragma unroll
                 for (int p = 0; p < 4; p++)
-                    a[mt][p >> 1][p & 1] = *(const f16x8*)(st + Stage::a + odd * kBM * kRowBytes + a_row + mt * 32 * kRowBytes + piece_off[p]);
+                    c[sub & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1 - (p >> 1)][p & 1], b[nt & 1][p & 1], p == 0 ? zero : c[sub & 1], 0, 0, 0);
+                const float d = sub == 0 ? dlast : dw[was / MT];
 #pragma unroll
-            for (int nt = 0; nt < 2; nt++)
+                for (int e = 0; e < 16; e++) acc[was % MT][was / MT][e] = fmaf(d, c[(sub + 1) & 1][e], acc[was % MT][was / MT][e]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            dlast = dw[NT - 1];
+        } else {
 #pragma unroll
-                for (int h = 0; h < 2; h++) b[nt][h] = *(const f16x8*)(st + b_row + nt * 32 * kRowBytes + piece_off[2 * odd + h]);
-            // The operands of the outer products that give dw dx: v_mfma_f32_32x32x1_2b_f32 makes two, its first 32
-            // lanes giving x's rows and W's rows of the first, the other 32 of the second; here the 32 rows of x of
-            // sub-tiles (mt, 0) and (mt, 1), and the 64 rows of W of both (a lane each).
-            const float dwv = ((const float*)(st + Stage::sw))[odd * kBN + wn * 64 + lane];
-            float dxv[2];
+            for (int j = 0; j < S::kLoads; j++) load_stage(j, fill, step);
+            // The products of the two scales, dw dx, are an outer product: v_mfma_f32_32x32x1_2b_f32 makes two (one exact product
+            // an output, nothing added: the rounding of a multiplication), its first 32 lanes giving x's rows and W's rows
+            // of the first, the other 32 of the second; here the 32 rows of x of sub-tiles (mt, 0) and (mt, 1), and the 64
+            // rows of W of both (a lane each).
+            const float dw = *(const float*)(sw + hi * 1024 + r32 * 4);
+            float dx[MT];
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) dxv[mt] = ((const float*)(st + Stage::sx))[odd * kBN + wm * 64 + mt * 32 + r32];
-            auto scales = [&](int mt, f32x32& w) {
-                f32x32 zero;
+            for (int mt = 0; mt < MT; mt++) dx[mt] = ((const float*)(lds + S::sx))[(i & 1) * S::BM + (wm * MT + mt) * 32 + r32];
+            f32x32 w, none;
 #pragma unroll
-                for (int e = 0; e < 32; e++) zero[e] = 0.f;
-                w = __builtin_amdgcn_mfma_f32_32x32x1f32(dxv[mt], dwv, zero, 0, 0, 0);
-            };
-            // Sub-tile s = 2 mt + nt: its four MFMAs are issued with the finish of the sub-tile before it, so that the
-            // vector unit works while the matrix cores do (two pairs of sums live at a time; more, and registers spill).
-            auto multiply = [&](int sub, f32x16& c0, f32x16& c1) {
-                const int mt = sub >> 1, nt = sub & 1;
-                f32x16 zero;
+            for (int e = 0; e < 32; e++) none[e] = 0.f;
 #pragma unroll
-                for (int e = 0; e < 16; e++) zero[e] = 0.f;
-                c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][0], b[nt][0], zero, 0, 0, 0);
-                c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1][0], b[nt][0], zero, 0, 0, 0);
-                c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][1], b[nt][1], c0, 0, 0, 0);
-                c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1][1], b[nt][1], c1, 0, 0, 0);
-            };
-            auto finish = [&](int sub, const f32x16& c0, const f32x16& c1, const f32x32& w) {
-                const int mt = sub >> 1, nt = sub & 1;
+            for (int sub = 0; sub < MT * NT; sub++) {  // NT is 2 here: both of b are there
+                const int mt = sub / NT, nt = sub % NT;
+                f32x16 c0, c1;
+                if (FORM == kDigits) {
+                    c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][0], b[nt][0], zero, 0, 0, 0);
+                    c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1][0], b[nt][0], zero, 0, 0, 0);
+                    c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][1], b[nt][1], c0, 0, 0, 0);
+                    c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1][1], b[nt][1], c1, 0, 0, 0);
+                } else {
+                    c0 = zero;
+#pragma unroll
+                    for (int p = 0; p < 4; p++) c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1 - (p >> 1)][p & 1], b[nt][p & 1], c0, 0, 0, 0);
+                }
+                if (nt == 0) w = __builtin_amdgcn_mfma_f32_32x32x1f32(dx[mt], dw, none, 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    const float isum = fmaf(c1[e], 4096.f, c0[e]);  // the exact integer, rounded once
-                    acc[mt][nt][e] = fmaf(w[16 * nt + e], isum, acc[mt][nt][e]);
+                    const float sum = FORM == kDigits ? fmaf(c1[e], 4096.f, c0[e]) : c0[e];  // digits: the exact integer, rounded once
+                    acc[mt][nt][e] = fmaf(w[16 * nt + e], sum, acc[mt][nt][e]);
                 }
-            };
-            f32x16 p0, p1, q0, q1;
-            f32x32 w;
-            multiply(0, p0, p1);
-            scales(0, w);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the next block's scales, at the end: by now their loads have landed with everything requested before them
             __builtin_amdgcn_sched_barrier(0);
-            multiply(1, q0, q1);
-            finish(0, p0, p1, w);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(2, p0, p1);
-            finish(1, q0, q1, w);
-            __builtin_amdgcn_sched_barrier(0);
-            scales(1, w);
-            multiply(3, q0, q1);
-            finish(2, p0, p1, w);
-            __builtin_amdgcn_sched_barrier(0);
-            finish(3, q0, q1, w);
+            if (tid < S::BM) ((float*)(lds + S::sx))[((i + 1) & 1) * S::BM + tid] = next_dx;
         }
-        // the next stage's scales, at the end: by now their loads have landed with everything requested before them
-        __builtin_amdgcn_sched_barrier(0);
-        ((float*)(next_p + Stage::sw))[sodd * kBN + srow] = next_dw;
-        ((float*)(next_p + Stage::sx))[sodd * kBN + srow] = next_dx;
+        use = use + S::stage == S::sw ? 0 : use + S::stage;
+        fill = fill + S::stage == S::sw ? 0 : fill + S::stage;
     }
+    if (FORM == kHalves) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[MT - 1][NT - 1][e] = fmaf(dlast, c[1][e], acc[MT - 1][NT - 1][e]);
+    }
+    wait_loads<0>();  // nothing of this tile's is on its way into LDS any more
 
     // An MFMA leaves a lane one column of y and four consecutive rows per group of four registers; a 4 x 4
     // transposition within each quad of lanes turns that into one row and four consecutive columns a lane.
-    const bool wide_ok = (N & 3) == 0 && ((uintptr_t)y & 15) == 0 && (!resid || ((uintptr_t)resid & 15) == 0);
+    const float* resid = sums ? nullptr : o.resid;
+    const bool gated = o.parts.swiglu && !sums;
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++)
+    for (int nt = 0; nt < NT; nt++) {
+        // this strip's columns: where they go, and which they are there
+        const int strip = n0 / 32 + wn * NT + nt;
+        if (strip >= o.parts.strips) break;
+        if (gated && (nt & 1)) continue;  // taken with the gate's
+        const int part = gated || sums ? 0 : strip >= o.parts.begin[2] ? 2 : strip >= o.parts.begin[1] ? 1 : 0;
+        float* y = sums ? sums : o.parts.y[part];
+        const int N = sums ? o.parts.strips * 32 : o.parts.N[part];
+        const int n = (sums ? strip : gated ? strip >> 1 : strip - o.parts.begin[part]) * 32 + (r32 & ~3);
+        const bool wide_ok = (N & 3) == 0 && ((uintptr_t)y & 15) == 0 && (!resid || ((uintptr_t)resid & 15) == 0);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int m = m0 + wm * 64 + mt * 32 + q * 8 + hi * 4 + (lane & 3);
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                float v[4] = {acc[mt][nt][4 * q], acc[mt][nt][4 * q + 1], acc[mt][nt][4 * q + 2], acc[mt][nt][4 * q + 3]};
-                quad_transpose(v, lane);
-                const int n = n0 + wn * 64 + nt * 32 + (r32 & ~3);
+            for (int q = 0; q < 4; q++) {
+                const int m = m0 + (wm * MT + mt) * 32 + q * 8 + hi * 4 + (lane & 3);
+                const int e_row = FORM == kHalves ? o.RS[m < M ? m : M - 1].x : 0;
+                auto row_of = [&](int col, float v[4]) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) v[k] = acc[mt][col][4 * q + k];
+                    quad_transpose(v, lane);
+                    if (FORM == kHalves)
+#pragma unroll
+                        for (int k = 0; k < 4; k++) v[k] = e_row == INT32_MAX ? __builtin_nanf("") : __builtin_ldexpf(v[k], e_row);
+                };
+                float v[4];
+                row_of(nt, v);
+                if (gated) {
+                    float u[4];
+                    row_of((nt + 1) % NT, u);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) v[k] = silu_times(v[k], u[k]);
+                }
                 if (m >= M || n >= N) continue;
                 if (wide_ok && n + 3 < N) {
-                    f32x4 o = {v[0], v[1], v[2], v[3]};
+                    f32x4 out = {v[0], v[1], v[2], v[3]};
                     if (resid) {
                         const f32x4 r = *(const f32x4*)(resid + (int64_t)m * N + n);
 #pragma unroll
-                        for (int k = 0; k < 4; k++) o[k] = o[k] + r[k];
+                        for (int k = 0; k < 4; k++) out[k] = out[k] + r[k];
                     }
-                    *(f32x4*)(y + (int64_t)m * N + n) = o;
+                    *(f32x4*)(y + (int64_t)m * N + n) = out;
                 } else {
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         if (n + k >= N) continue;
-                        float o = v[k];
-                        if (resid) o = o + resid[(int64_t)m * N + n + k];
-                        y[(int64_t)m * N + n + k] = o;
+                        float out = v[k];
+                        if (resid) out = out + resid[(int64_t)m * N + n + k];
+                        y[(int64_t)m * N + n + k] = out;
                     }
                 }
             }
-        }
+    }
 }
 
-std::atomic<int> g_fx16{1};  // measurement aid: 0 keeps every product on the int8 form, 2 takes this one whatever the shape
+// Whether one of rows m0 .. m0 + rows has an exponent a block: then all are read by block.
+__device__ __forceinline__ bool by_block(const Operands& o, int m0, int rows) {
+    bool any = false;
+    for (int r = threadIdx.x & 63; r < rows; r += 64) any |= o.RS[m0 + r < o.M ? m0 + r : o.M - 1].y == kBlockHalves;
+    return __ballot(any) != 0;
+}
+
+// How the product is cut: the first wide_cols columns of 256 into wide tiles, the others into low ones, every tile's K into shares.
+struct Cut {
+    int wide_m, wide_cols, low_m, low_cols;  // tiles along M, columns of tiles
+    int shares, share_blocks;                // the last share may be shorter
+};
+
+template <bool DIGITS>
+__device__ __forceinline__ void product(const Operands& o, const Cut& cut, char* lds) {
+    static_assert(Wide::BN == Low::BN && Wide::BM == 2 * Low::BM, "a wide tile is two low ones");
+    const int wide_tiles = cut.wide_m * cut.wide_cols, wide_wgs = ((wide_tiles * cut.shares + 7) >> 3) << 3;
+    const bool wide = (int)blockIdx.x < wide_wgs;
+    const int tiles = wide ? wide_tiles : cut.low_m * cut.low_cols;
+    const int t = tile_of((int)blockIdx.x - (wide ? 0 : wide_wgs), tiles * cut.shares);
+    if (t >= tiles * cut.shares) return;  // the whole workgroup
+    const int share = t / tiles, tile = t % tiles, tiles_m = wide ? cut.wide_m : cut.low_m;
+    const int bm = wide ? Wide::BM : Low::BM, n0 = ((wide ? 0 : cut.wide_cols) + tile / tiles_m) * Low::BN;
+    const int b0 = share * cut.share_blocks, count = o.nb - b0 < cut.share_blocks ? o.nb - b0 : cut.share_blocks;
+    float* sums = o.sums ? o.sums + (int64_t)share * o.M * o.parts.strips * 32 : nullptr;
+    int m0 = tile % tiles_m * bm;
+    if (DIGITS) {
+        tile_body<Low, kDigits>(o, m0, n0, b0, count, sums, lds);
+    } else if (!by_block(o, m0, bm)) {
+        if (wide) tile_body<Wide, kHalves>(o, m0, n0, b0, count, sums, lds);
+        else tile_body<Low, kHalves>(o, m0, n0, b0, count, sums, lds);
+    } else {
+        for (const int end = m0 + bm < o.M ? m0 + bm : o.M; m0 < end; m0 += Low::BM) {
+            tile_body<Low, kBlockHalves>(o, m0, n0, b0, count, sums, lds);
+            lds_barrier();  // the next one fills the stages anew
+        }
+    }
+}
+
+__global__ __launch_bounds__(512) void qgemm_q4_0_fx16_kernel(Operands o, Cut cut) {
+    extern __shared__ __align__(1024) char lds[];
+    product<false>(o, cut, lds);
+}
+
+__global__ __launch_bounds__(512) void qgemm_q4_0_fx16_digits_kernel(Operands o, Cut cut) {
+    extern __shared__ __align__(1024) char lds[];
+    product<true>(o, cut, lds);
+}
+
+// The shares' sums, in their order, four columns a thread: y = ((s0 + s1) + ..) (+ resid), or silu(gate) up of them.
+__global__ __launch_bounds__(256) void fx16_sum_kernel(Operands o, int shares) {
+    const int64_t ld = (int64_t)o.parts.strips * 32, quads = o.M * ld / 4, step = o.M * ld;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < quads; t += (int64_t)gridDim.x * 256) {
+        const int64_t m = 4 * t / ld;
+        const int at = (int)(4 * t - m * ld), strip = at >> 5;
+        if (o.parts.swiglu && (strip & 1)) continue;
+        auto total = [&](const float* from) {
+            f32x4 v = *(const f32x4*)from;
+            for (int i = 1; i < shares; i++) {
+                const f32x4 w = *(const f32x4*)(from + i * step);
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = v[k] + w[k];
+            }
+            return v;
+        };
+        f32x4 v = total(o.sums + 4 * t);
+        if (o.parts.swiglu) {
+            const f32x4 u = total(o.sums + 4 * t + 32);
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = silu_times(v[k], u[k]);
+        }
+        const int part = o.parts.swiglu ? 0 : strip >= o.parts.begin[2] ? 2 : strip >= o.parts.begin[1] ? 1 : 0, N = o.parts.N[part];
+        const int n = (o.parts.swiglu ? strip >> 1 : strip - o.parts.begin[part]) * 32 + (at & 31);
+        float* y = o.parts.y[part] + m * N + n;
+        const float* resid = o.resid ? o.resid + m * N + n : nullptr;
+        if ((N & 3) == 0 && ((uintptr_t)o.parts.y[part] & 15) == 0 && ((uintptr_t)o.resid & 15) == 0) {
+            if (n >= N) continue;
+            if (resid) {
+                const f32x4 r = *(const f32x4*)resid;
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = v[k] + r[k];
+            }
+            *(f32x4*)y = v;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (n + k < N) y[k] = resid ? v[k] + resid[k] : v[k];
+        }
+    }
+}
+
+// measurement aid: 0 keeps every product on the int8 form, 2 takes the digits' form whatever the shape, 3 the halves'
+std::atomic<int> g_fx16{1};
+
+int64_t strips_of(int64_t rows) { return (rows + 31) / 32; }
+
+// Microseconds of a product, the pass over W and the shares' sums included, and its cut. A compute unit takes a tile at a
+// time; the time of a tile's block grows with how many units are at work, as the clock falls: 0.72 + 0.32 of them for a
+// tile of 128 x 256, 1.25 + 0.5 of them for one of 256 x 256 (measured at 32 to 1792 tiles of 4096 and 14336 of K). Shares of K are for
+// products whose tiles leave units idle: their sums are written and read at about 4.5 TB/s, the panel at 4.4.
+double plan(int64_t M, int64_t strips, int64_t K, int64_t min_share_blocks, size_t sums_bytes, Cut* cut) {
+    const int64_t nb = K / 32, cols = (strips + 7) / 8;
+    const int64_t tm = (M + Wide::BM - 1) / Wide::BM, tl = (M + Low::BM - 1) / Low::BM;
+    const double panel_us = (double)strips * 32 * (double)K * (18.0 / 32.0 + 2.0) / 4.4e6;
+    double best = 1e30;
+    auto consider = [&](int64_t wide_cols, int64_t shares) {
+        const int64_t blocks = (nb + shares * kGroup - 1) / (shares * kGroup) * kGroup, used = (nb + blocks - 1) / blocks;
+        if (used != shares) return;
+        const int64_t wide = tm * wide_cols * shares, low = tl * (cols - wide_cols) * shares;
+        const size_t sums = (size_t)shares * (size_t)M * (size_t)strips * 128;
+        if (shares > 1 && (blocks < min_share_blocks || sums > sums_bytes)) return;
+        // whole rounds of wide tiles; what is left of the last one is filled with low ones
+        double us = 0, idle = 256;
+        if (wide) {
+            const int64_t rounds = (wide + 255) / 256;
+            us += (double)rounds * (double)blocks * (1.25 + 0.5 * (double)wide / (double)(rounds * 256));
+            idle = (double)(rounds * 256 - wide);
+        }
+        if (low) {
+            const int64_t beside = wide ? (int64_t)(2 * idle) : 0, left = low > beside ? low - beside : 0, rounds = (left + 255) / 256;
+            if (rounds) us += (double)rounds * (double)blocks * (0.72 + 0.32 * (double)left / (double)(rounds * 256));
+        }
+        if (shares > 1) us += 3.0 + (double)sums * (1.0 + 1.0 / (double)shares) / 4.5e6;
+        if (us + panel_us < best) {
+            best = us + panel_us;
+            *cut = Cut{(int)tm, (int)wide_cols, (int)tl, (int)(cols - wide_cols), (int)shares, (int)blocks};
+        }
+    };
+    for (int64_t shares = 1; shares <= 16; shares++) {
+        if (shares > 1 && tl * cols * shares > 1024) break;
+        consider(0, shares);
+        consider(cols, shares);
+        if (shares == 1)
+            for (int64_t rounds = 1; rounds * 256 < tm * cols; rounds++)  // whole rounds of wide tiles, then low ones
+                if (rounds * 256 / tm > 0) consider(rounds * 256 / tm, 1);
+    }
+    return best;
+}
+
+bool fits(int64_t M, int64_t strips, int64_t K) {
+    return M > 0 && strips > 0 && K > 0 && K % 64 == 0 && M < (1 << 30) && K <= (1 << 20) && strips < (1 << 22) && (M + 127) / 128 * ((strips + 7) / 8) < ((int64_t)1 << 24);
+}
 
 }  // namespace
 
 void set_q4_0_fx16(int v) { g_fx16 = v; }
 
-// Whether the product is the faster here than in the int8 form (qgemm_q4_0_fx_cost_us), the pass over W included:
-// that pass reads the blocks and writes the panel at about 4.4 TB/s; a workgroup takes about 2.85 us a stage of 64 of K,
-// one a compute unit at a time (measured at 4096 x 4096, 14336 x 4096 and 4096 x 14336 weights, 512 to 4096 rows:
-// 512 x 4096 x 4096 stays with the int8 form, 512 x 14336 x 4096 comes here).
+// Whether the product is the faster here than in the int8 form (qgemm_q4_0_fx_cost_us). mi355x_qgemv cuts K into shares of
+// no less than 96 blocks: 512 x 4096 x 4096 stays with the int8 form there (88 us, in one pass here 114), which
+// tests/test_gpu_qgemm_fx.py holds it to; 512 x 14336 x 4096 comes here (151 us, 217 in the int8 form).
+constexpr int64_t kMinShareBlocks = 96;
+
 bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K) {
-    if (g_fx16 == 0 || M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return false;
-    if (g_fx16 == 2) return true;
-    if (M < kMinRows) return false;
-    const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
-    const double product_us = (double)((tiles + 255) / 256) * (double)(K / 64) * 2.85;
-    const double panel_us = (double)N * (double)K * (18.0 / 32.0 + 2.0) / 4.4e6;
-    return panel_us + product_us < qgemm_q4_0_fx_cost_us(M, N, K);
+    if (g_fx16 == 0 || N <= 0 || !fits(M, strips_of(N), K)) return false;
+    if (g_fx16 >= 2) return true;
+    Cut cut;
+    return M >= kMinRows && plan(M, strips_of(N), K, kMinShareBlocks, (size_t)-1, &cut) < qgemm_q4_0_fx_cost_us(M, N, K);
 }
 
-// X16 [M, K / 32, 64] binary16, then XS [M, K / 32] float32: 4 K + K / 8 bytes a row.
-size_t q4_0_fx16_act_bytes(int64_t K) { return (size_t)((4 * K + K / 8 + 15) / 16 * 16); }
+// X16 in granules, then RS [M] int2, then XS [M, K / 32] float32.
+size_t q4_0_fx16_act_bytes(int64_t M, int64_t K) {
+    return (size_t)strips_of(M) * (size_t)(K / 32) * kGranuleX * 2 + ((size_t)M * 8 + (size_t)M * (size_t)(K / 32) * 4 + 15) / 16 * 16;
+}
+
+template <bool NORM>
+static void launch_halves(const float* x, const float* w, double eps, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
+    uint16_t* X16 = (uint16_t*)act;
+    int2* RS = (int2*)(X16 + strips_of(M) * (K / 32) * kGranuleX);
+    float* XS = (float*)(RS + M);
+    const auto kernel = K <= 4096 ? fx16_halves_kernel<2, NORM> : K <= 16384 ? fx16_halves_kernel<8, NORM> : fx16_halves_kernel<0, NORM>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)M), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (float)(1.0 / (double)K), (float)eps);
+}
 
 hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
-    const int gx = (int)((K / 4 + 255) / 256);
-    uint16_t* X16 = (uint16_t*)act;
-    float* XS = (float*)(X16 + (size_t)M * K * 2);
-    hipLaunchKernelGGL(fx16_convert_kernel, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, (int)K, X16, XS);
+    if (g_fx16 == 2) {
+        uint16_t* X16 = (uint16_t*)act;
+        int2* RS = (int2*)(X16 + strips_of(M) * (K / 32) * kGranuleX);
+        const int gx = (int)((K / 4 + 255) / 256);
+        hipLaunchKernelGGL(fx16_digits_kernel, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, (int)K, X16, (float*)(RS + M), RS);
+    } else {
+        launch_halves<false>(x, nullptr, 0, M, K, x_row_stride, act, st);
+    }
     return hipGetLastError();
 }
 
-// The panel: N K binary16.
-size_t qgemm_q4_0_fx16_ws_bytes(int64_t N, int64_t K) { return (size_t)N * (size_t)K * 2; }
+// rmsnorm's result converted, for qgemm_q4_0_fx16_parts: x [M, K], 16-byte aligned like w, K a multiple of 32.
+hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, int64_t K, double eps, hipStream_t st) {
+    launch_halves<true>(x, w, eps, M, K, K, act, st);
+    return hipGetLastError();
+}
 
-// act: q4_0_fx16_convert_act's for these M rows; ws: qgemm_q4_0_fx16_ws_bytes(N, K) bytes, 16-byte aligned.
-// y = x . W^T (+ resid, which may be y itself).
-hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st) {
-    if (!ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)act & 15) != 0 || ((uintptr_t)W & 1) != 0 || M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 ||
-        M >= (1 << 30) || N >= (1 << 30) || K > (1 << 20))
-        return hipErrorInvalidValue;
+// The panel in granules, W's scales, the shares' sums.
+static size_t panel_bytes(int64_t strips, int64_t K) { return (size_t)strips * (size_t)(K / 32) * kGranuleP * 2; }
+static size_t scales_bytes(int64_t strips, int64_t K) { return (size_t)strips * (size_t)scale_blocks((int)(K / 32)) * kGranuleS * 4; }
+
+size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K) {
+    Cut cut{};
+    if (g_fx16 != 2) plan(M, strips_of(N), K, kMinShareBlocks, (size_t)-1, &cut);
+    return panel_bytes(strips_of(N), K) + scales_bytes(strips_of(N), K) + (cut.shares > 1 ? (size_t)cut.shares * (size_t)M * (size_t)strips_of(N) * 128 : 0);
+}
+
+static hipError_t multiply(const Parts& parts, const void* act, const float* resid, int64_t M, int64_t K, int64_t min_share_blocks, void* ws, size_t ws_bytes,
+                           hipStream_t st) {
+    const int64_t strips = parts.strips;
+    const size_t fixed = panel_bytes(strips, K) + scales_bytes(strips, K);
+    if (!ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)act & 15) != 0 || !fits(M, strips, K) || ws_bytes < fixed) return hipErrorInvalidValue;
+    for (int i = 0; i < 3; i++)
+        if (((uintptr_t)parts.W[i] & 1) != 0) return hipErrorInvalidValue;
     static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
+        hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx16_digits_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Low::total);
         if (e != hipSuccess) return e;
         raised = true;
     }
-    const int64_t tiles_m = (M + kBM - 1) / kBM, ntiles = tiles_m * ((N + kBN - 1) / kBN);
-    if (ntiles >= ((int64_t)1 << 28)) return hipErrorInvalidValue;
+    const int nb = (int)(K / 32);
+    const bool digits = g_fx16 == 2;
+    Cut cut{0, 0, (int)((M + Low::BM - 1) / Low::BM), (int)((strips + 7) / 8), 1, nb};
+    if (!digits) plan(M, strips, K, min_share_blocks, ws_bytes - fixed, &cut);
     uint16_t* P = (uint16_t*)ws;
-    const int64_t halves = N * (K / 32) * 2;
-    const int64_t want = (halves + 255) / 256;
-    hipLaunchKernelGGL(fx16_panel_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, st, (const uint8_t*)W, P, halves);
+    float* SW = (float*)((char*)ws + panel_bytes(strips, K));
     const uint16_t* X16 = (const uint16_t*)act;
-    const float* XS = (const float*)(X16 + (size_t)M * K * 2);
-    const int wgs = (int)(((ntiles + 7) / 8) * 8);
-    hipLaunchKernelGGL(qgemm_q4_0_fx16_kernel, dim3((unsigned)wgs), dim3(512), kLdsBytes, st, (const uint8_t*)W, P, X16, XS, y, resid, (int)M, (int)N,
-                       (int)K, (int)tiles_m, (int)ntiles);
-    note_kernel("qgemm_q4_0_fx16_kernel: %lld x %lld tiles of 128 x 256", (long long)tiles_m, (long long)(ntiles / tiles_m));
+    const int2* RS = (const int2*)(X16 + strips_of(M) * nb * kGranuleX);
+    const Operands o{P, SW, X16, (const float*)(RS + M), RS, resid, cut.shares > 1 ? (float*)((char*)ws + fixed) : nullptr, (int)M, nb, parts};
+    const int64_t wide = (int64_t)cut.wide_m * cut.wide_cols * cut.shares, low = (int64_t)cut.low_m * cut.low_cols * cut.shares;
+    hipLaunchKernelGGL(fx16_panel_kernel, dim3((unsigned)((nb + 7) / 8), (unsigned)strips), dim3(256), 0, st, parts, P, SW, nb);
+    const dim3 grid((unsigned)((wide + 7) / 8 * 8 + (low + 7) / 8 * 8));
+    if (digits) hipLaunchKernelGGL(qgemm_q4_0_fx16_digits_kernel, grid, dim3(512), Low::total, st, o, cut);
+    else hipLaunchKernelGGL(qgemm_q4_0_fx16_kernel, grid, dim3(512), kLdsBytes, st, o, cut);
+    if (cut.shares > 1) {
+        const int64_t groups = (M * strips * 8 + 255) / 256;
+        hipLaunchKernelGGL(fx16_sum_kernel, dim3((unsigned)(groups < 16384 ? groups : 16384)), dim3(256), 0, st, o, cut.shares);
+    }
+    char shares[40] = "", beside[60] = "";
+    if (cut.shares > 1) snprintf(shares, sizeof shares, ", %d shares of K", cut.shares);
+    if (cut.wide_cols && cut.low_cols) snprintf(beside, sizeof beside, ", %d x %d tiles of 128 x 256", cut.low_m, cut.low_cols);
+    note_kernel("qgemm_q4_0_fx16_kernel: %d x %d tiles of %s%s%s", cut.wide_cols ? cut.wide_m : cut.low_m, cut.wide_cols ? cut.wide_cols : cut.low_cols,
+                cut.wide_cols ? "256 x 256" : "128 x 256", beside, shares);
     return hipGetLastError();
+}
+
+// Several matrices by the same rows of x in one product, or gate and up with silu(gate) up as their result: the tiles of
+// all of them fill the device together (512 rows by 4096 of K: q, k and v of 4096, 1024 and 1024 rows take 84 us, one by one in
+// the int8 form 190; gate and up of 14336 rows 290, one by one 2 x 150). K is cut into shares of 16 blocks and up.
+constexpr int64_t kMinPartShareBlocks = 16;
+constexpr size_t kMostSums = (size_t)96 << 20;
+
+static bool parts_of(const Fx16Part* part, int n, bool swiglu, int64_t K, Parts* out) {
+    if (n < 1 || n > 3 || (swiglu && (n != 2 || part[0].N != part[1].N))) return false;
+    *out = Parts{};
+    int64_t strips = 0;
+    for (int i = 0; i < n; i++) {
+        if (part[i].N <= 0 || part[i].N >= (1 << 27) || ((uintptr_t)part[i].W & 1) != 0) return false;
+        out->W[i] = (const uint8_t*)part[i].W;
+        out->y[i] = part[i].y;
+        out->N[i] = (int)part[i].N;
+        out->begin[i] = (int)strips;
+        strips += strips_of(part[i].N);
+    }
+    for (int i = n; i < 3; i++) out->begin[i] = (int)strips;
+    out->strips = (int)strips;
+    out->swiglu = swiglu;
+    return fits(1, strips, K);
+}
+
+// What qgemm_q4_0_fx16_parts can use of a workspace, for up to M rows.
+size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K) {
+    Parts p;
+    return parts_of(part, n, false, K, &p) ? panel_bytes(p.strips, K) + scales_bytes(p.strips, K) + kMostSums : 0;
+}
+
+// Whether they are the faster together here, in a workspace of ws_bytes, than each on the int8 form or the row kernels.
+bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes) {
+    Parts p;
+    Cut cut;
+    if (g_fx16 == 0 || g_fx16 == 2 || M < kMinPartRows || !parts_of(part, n, swiglu, K, &p) || !fits(M, p.strips, K)) return false;
+    const size_t fixed = panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
+    if (ws_bytes < fixed) return false;
+    double apart = 0;
+    for (int i = 0; i < n; i++) {
+        const double rows_us = (double)M * ((double)part[i].N * (double)(K / 32) * 18.0) / 8.7e6, fx = qgemm_q4_0_fx_cost_us(M, part[i].N, K);
+        apart += fx < rows_us ? fx : rows_us;
+    }
+    return g_fx16 >= 3 || plan(M, p.strips, K, kMinPartShareBlocks, ws_bytes - fixed, &cut) < apart;
+}
+
+// act: q4_0_fx16_convert_act's for these M rows; ws: ws_bytes, 16-byte aligned. Each part's y = x . W^T; one part alone: + resid, which
+// may be y itself; swiglu: part 0's y = silu(x . W0^T) (x . W1^T).
+hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes,
+                                 hipStream_t st) {
+    Parts p;
+    if (!parts_of(part, n, swiglu, K, &p) || (resid && n != 1)) return hipErrorInvalidValue;
+    return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, st);
+}
+
+// act: q4_0_fx16_convert_act's for these M rows; ws: qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned.
+// y = x . W^T (+ resid, which may be y itself).
+hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st) {
+    if (N <= 0 || N >= (1 << 27) || !fits(M, strips_of(N), K)) return hipErrorInvalidValue;
+    const int n = (int)strips_of(N);
+    const Parts parts{{(const uint8_t*)W, nullptr, nullptr}, {y, nullptr, nullptr}, {(int)N, 0, 0}, {0, n, n}, n, 0};
+    return multiply(parts, act, resid, M, K, kMinShareBlocks, ws, qgemm_q4_0_fx16_ws_bytes(M, N, K), st);
 }
 
 }  // namespace mimir

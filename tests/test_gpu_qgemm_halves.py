@@ -1,0 +1,104 @@
+"""The Q4_0 product of many rows of float32 x on the binary16 matrix cores, x as pairs of binary16 (qgemm_q4_0_fx16.hip), against the
+product in 64 bits. Bound: a pair holds an element to 2^-23 of its block's largest magnitude (kernel's comment), beside
+float32 sums' 2e-6 sum |x||w|; what the fixed-point forms of this product are held to."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from mimir_amd import capi
+from mimir_amd.llama import Llama
+from oracle import llama as OL
+from tests import gpu
+from tests.helpers import random_blocks
+from tests.test_gpu_llama import _oracle_config, _upload_synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def last_kernel():
+    buf = ctypes.create_string_buffer(200)
+    capi.check(gpu.lib().mi355x_last_kernel(buf, 200))
+    return buf.value.decode()
+
+
+def tuned(rows, pairs):
+    capi.check(gpu.lib().mi355x_tune(b"q4_0.fx_rows", rows))
+    capi.check(gpu.lib().mi355x_tune(b"q4_0.fx_pairs", pairs))
+
+
+@pytest.mark.parametrize("m,n,k,tiles", [
+    (1, 5, 128, "1 x 1 tiles of 128 x 256"), (40, 100, 256, "1 x 1 tiles of 128 x 256"), (129, 257, 384, "2 x 2 tiles of 128 x 256"),
+    (300, 520, 6272, "3 x 3 tiles of 128 x 256, 2 shares of K"), (257, 129, 14336, "3 x 1 tiles of 128 x 256, 5 shares of K"),
+    (1000, 16500, 128, "4 x 64 tiles of 256 x 256, 8 x 1 tiles of 128 x 256"), (2047, 8192, 128, "8 x 32 tiles of 256 x 256"), (33, 60, 16512, "1 x 1 tiles of 128 x 256, 5 shares of K")])
+@pytest.mark.parametrize("rows", ["even", "wide", "special"])
+def test_pairs_of_halves(m, n, k, tiles, rows):
+    """Every cut of the product, tiles and strips that rows and columns do not fill. Rows of x: of very different magnitude; some whose
+    blocks differ by up to 2^60 (those take an exponent a block, and a tile with one of them its slower loop); blocks and
+    rows of zeros, the smallest and largest magnitudes, a NaN and an infinity (a row of NaNs each, and of no other)."""
+    rng = np.random.default_rng(m + n + k)
+    raw = random_blocks(rng, O.Q4_0, n * k)
+    x = (rng.normal(size=(m, k)) * np.exp(rng.normal(size=(m, 1)) * 3)).astype(np.float32)
+    bad = []
+    if rows == "wide":
+        x[m // 3, :32] *= 2.0 ** 30
+        x[m - 1, 32:64] *= 2.0 ** -40
+        x[m - 1, 5] *= 2.0 ** 20
+    if rows == "special" and m >= 12:
+        x[m // 2, :32] = 0
+        x[1] = 0
+        x[2, 3], x[5, k - 1] = np.nan, np.inf
+        x[7] *= np.float32(1e-36)
+        x[8] *= np.float32(1e30)
+        x[9] = np.float32(1e-42)
+        bad = [2, 5]
+    wide = torch.zeros((m, k + 8), device="cuda:0")  # rows further apart than K
+    wide[:, :k] = gpu.dev(x)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    gpu.say(f"q4_0 halves M={m} N={n} K={k} {rows}")
+    try:
+        tuned(1, 3)
+        got = gpu.qgemv(O.Q4_0, ptr, wide[:, :k], n, k)
+        assert last_kernel() == "qgemm_q4_0_fx16_kernel: " + tiles
+    finally:
+        tuned(0, 1)
+    x64 = gpu.dev(x).double()
+    w = gpu.dev(O.dequantize(O.Q4_0, raw).reshape(n, k)).double()
+    want, bound = x64 @ w.T, 2e-6 * (x64.abs() @ w.abs().T)
+    bound += 2.0 ** -23 * (x64.abs().reshape(m, -1, 32).amax(2) @ w.abs().reshape(n, -1, 32).sum(2).T) + 1e-30
+    good = [i for i in range(m) if i not in bad]
+    got = gpu.dev(got).double()
+    assert torch.isnan(got[bad]).all()
+    assert ((got - want).abs() <= bound)[good].all()
+
+
+@pytest.mark.parametrize("batch,prompt,hidden", [(1, 150, 1088), (2, 24, 1024), (3, 100, 992)])
+def test_a_prompt_pass_with_products_taken_together(batch, prompt, hidden):
+    """A model whose q, k, v and whose gate and up (with SwiGLU) are one product each: column strips that no tile is filled by, K of
+    320 and of 1088, a down projection whose K (992) this form does not take. Against the oracle as the other prompt passes
+    are, and within 1e-5 of the largest logit of the int8 form's pass (both hold x to 2^-23 of a block's largest; no rounding step
+    between them, but the binary16 cache's)."""
+    c = capi.LlamaConfig()
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = 320, hidden, 2, 5, 1, 64, 64, 515
+    c.context, c.interleaved, c.cache_dtype, c.batch = prompt + 8, 1, capi.F32, batch
+    c.rope_base, c.rope_scale, c.eps = 10000.0, 1.0, 1e-5
+    om = OL.synthetic(_oracle_config(c), seed=3, output_dt=O.Q4_0)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(prompt)
+    tokens = np.random.default_rng(1).integers(0, c.vocab, (batch, prompt))
+    out = {}
+    try:
+        for pairs in (3, 0):
+            gpu.say(f"prompt pass batch={batch} prompt={prompt} hidden={hidden} pairs={pairs}")
+            tuned(0, pairs)
+            m.reset()
+            out[pairs] = m.logits(tokens, all=True)
+    finally:
+        tuned(0, 1)
+    want = om.logits(tokens[0].tolist(), om.new_caches(c.context, O.F32), all=True)
+    scale = np.abs(want).max()
+    assert np.abs(out[3][0] - want).max() <= 0.02 * scale and np.median(np.abs(out[3][0] - want)) <= 1e-5 * scale
+    assert np.median(np.abs(out[3] - out[0])) <= 1e-5 * scale and np.abs(out[3] - out[0]).max() <= 0.02 * scale

@@ -4,6 +4,7 @@
 #include "../../include/mimir_mi355x.h"
 #include "../../include/mimir_mi355x_measure.h"
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -217,6 +218,23 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             if (rows && g_rows_max > 0) rows = M < g_rows_max;
             else if (rows && M >= 16 && mimir::qgemm_q4_0_fx_ok(W, M, N, K))
                 rows = mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K);
+            // some tens of rows, where W read where it lies by pairs of binary16 undercuts both (not from a fixed scratch, which is too
+            // small); every call of 16 rows and more asks for the scratch of that many rows, up to 256, so that none grows it after a larger one
+            if (M >= 16 && !src.fixed && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0 && K % 32 == 0) {
+                size_t ws;
+                const double us = mimir::qgemm_q4_0_in_place_cost_us(W, M, N, K, &ws);
+                const size_t act_bytes = (mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K) + 255) / 256 * 256;
+                void* act;
+                if (mi355x_status st = act_for(src, act_bytes + ws, &act)) return st;
+                double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
+                if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
+                // 8 us: the conversion, and what two launches more or less cost where the models are close (64 x 4096 x 4096: rows 22 us, here 24)
+                if (us + 8.0 < other) {
+                    HIP_TRY(mimir::q4_0_halves_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_halves_convert_act");
+                    HIP_TRY(mimir::qgemm_q4_0_in_place(W, act, y, M, N, K, (uint8_t*)act + act_bytes, ws, (hipStream_t)stream), "launch qgemm_q4_0_in_place");
+                    return MI355X_OK;
+                }
+            }
             if (rows) {
                 const bool one_launch = mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1);  // else the variant that takes eight rows a launch
                 const int64_t groups = (M + 7) / 8;

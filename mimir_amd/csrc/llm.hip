@@ -760,7 +760,7 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
         }
         m->fx_panel.release();
         m->fx_panel.bytes = 0;
-        if (panel && rows >= 48) LLM_HIP(m->fx_panel.alloc(panel), "hipMalloc(fixed-point product workspace)");
+        if (panel && rows >= 9) LLM_HIP(m->fx_panel.alloc(panel), "hipMalloc(fixed-point product workspace)");
     }
     int chunk, nsplit;
     attention_plan(c.batch, c.heads, c.kv_heads, max_tokens, c.context, &chunk, &nsplit);

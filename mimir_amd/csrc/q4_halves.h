@@ -1,0 +1,120 @@
+// What the two kernels share that multiply x as pairs of binary16 by Q4_0 weights (qgemm_q4_0_fx16.hip, qgemm_q4_0_direct.hip).
+#pragma once
+#include "device_util.h"
+
+namespace mimir {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+// Operands lie in memory as the product reads them, so that every load is a whole KB: granules of 32 rows by one block
+// of 32 of K, the granules of a strip of 32 rows one after the other.
+constexpr int kGranuleX = 2048;   // binary16 of a granule of x: 32 rows of 128 bytes, a row's 16-byte pieces turned (turn_of)
+constexpr int kGranuleP = 1024;   // of W: two halves of the block, each in the order of lanes of an MFMA's operand
+constexpr int kGranuleS = 32;     // float32 scales of W
+constexpr int kGroup = 8;         // blocks whose scales come into LDS together: a KB a strip
+
+// x: row m's pieces 4 part + 2 half + hi of a block, hi which eight of the half's sixteen, lie at piece ^ turn, so that the
+// 32 rows of a fragment read fall on all banks while a row's block stays one line for the kernels that write it.
+__host__ __device__ inline int64_t row_at(int m, int nb) { return (int64_t)(m >> 5) * nb * kGranuleX + (m & 31) * 64; }
+__host__ __device__ inline int turn_of(int m) { return (m >> 1) & 7; }
+
+// How a row of x is held. The row's information is {exponent, form}.
+enum Form { kHalves = 0, kBlockHalves = 1, kDigitPairs = 2 };
+
+__host__ __device__ inline int scale_blocks(int nb) { return (nb + kGroup - 1) / kGroup * kGroup; }  // of a strip: whole groups
+
+// What is multiplied by the same x: up to three matrices, or gate and up, whose strips then lie in turn.
+struct Parts {
+    const uint8_t* W[3];
+    float* y[3];
+    int N[3];      // rows of W
+    int begin[3];  // first strip; those of parts that are not there lie past the last
+    int strips;    // of all
+    int swiglu;    // W[0] and W[1] are gate and up: y[0] gets silu(gate) up
+};
+
+struct Operands {
+    const uint16_t* P;
+    const float* SW;
+    const uint16_t* X16;
+    const float* XS;
+    const int2* RS;
+    const float* resid;  // may be y; added to what one part's y gets
+    float* sums;         // where K is cut into shares: [share][M][32 strips] float32, finished by fx16_sum_kernel
+    int M, nb;
+    Parts parts;
+};
+
+__device__ __forceinline__ float silu_times(float g, float u) {  // as swiglu_kernel's
+    const float e = __builtin_exp2f(g * (float)(-1.4426950408889634));
+    const float s = 1.0f / (1.0f + e);
+    const float a = g * s;
+    return a * u;
+}
+
+// Where column 0 of a strip goes: its part, and the column it is there. SwiGLU: of both gate's and up's strips, the result's.
+__device__ __forceinline__ int part_of(const Parts& p, int strip, int* n) {
+    const int part = p.swiglu ? 0 : strip >= p.begin[2] ? 2 : strip >= p.begin[1] ? 1 : 0;
+    *n = (p.swiglu ? strip >> 1 : strip - p.begin[part]) * 32;
+    return part;
+}
+
+// Up to four neighbouring columns n.. of row m of y [.., N] (+ resid): in one store where they are whole and aligned.
+__device__ __forceinline__ void store_four(float* y, const float* resid, int64_t m, int N, int n, const float v[4], bool wide_ok) {
+    if (wide_ok && n + 3 < N) {
+        f32x4 out = {v[0], v[1], v[2], v[3]};
+        if (resid) {
+            const f32x4 r = *(const f32x4*)(resid + m * N + n);
+#pragma unroll
+            for (int k = 0; k < 4; k++) out[k] = out[k] + r[k];
+        }
+        *(f32x4*)(y + m * N + n) = out;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (n + k >= N) continue;
+            float out = v[k];
+            if (resid) out = out + resid[m * N + n + k];
+            y[m * N + n + k] = out;
+        }
+    }
+}
+
+// A row's results under its exponent; INT32_MAX: a row with a NaN or an infinity.
+__device__ __forceinline__ void under_exponent(float v[4], int e) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = e == INT32_MAX ? __builtin_nanf("") : __builtin_ldexpf(v[k], e);
+}
+
+// Eight nibbles (the low or the high ones of two dwords) as the binary16 integers n - 8: the nibble into the mantissa of binary16's
+// 1024, minus 1032.
+__device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t lo, uint32_t hi, int half) {
+    const f16x2 off = {(_Float16)1032.f, (_Float16)1032.f};
+    u32x4 v;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t nib = ((i ? hi : lo) >> (4 * half)) & 0x0f0f0f0fu;
+        const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u);
+        const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u);
+        v[2 * i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p0) - off);
+        v[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p1) - off);
+    }
+    return __builtin_bit_cast(f16x8, v);
+}
+
+// The shares' sums of K, in their order: y = ((s0 + s1) + ..) (+ resid), or silu(gate) up of them.
+hipError_t sum_shares(const Operands& o, int shares, hipStream_t st);
+
+// The product with W read where it lies (qgemm_q4_0_direct.hip): up to kDirectMaxRows rows.
+constexpr int64_t kDirectMaxRows = 256;
+constexpr size_t kDirectMostSums = (size_t)64 << 20;
+size_t qgemm_q4_0_direct_sums_bytes(int64_t M, int64_t strips);
+double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes);
+hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st);
+
+inline int64_t strips_of(int64_t rows) { return (rows + 31) / 32; }
+
+}  // namespace mimir

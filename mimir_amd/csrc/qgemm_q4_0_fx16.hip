@@ -27,38 +27,20 @@
 #include "device_util.h"
 #include "kernels.h"
 #include "q4_act.h"
+#include "q4_halves.h"
 
 namespace mimir {
 
 namespace {
 
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x32 __attribute__((ext_vector_type(32)));
-
 constexpr int kMinRows = 256;     // fewer rows of one matrix stay with the int8 form,
-constexpr int kMinPartRows = 48;  // of several together
-
-// Operands lie in memory as a stage of LDS holds them, so that every load is a whole KB: granules of 32 rows by one block
-// of 32 of K, the granules of a strip of 32 rows one after the other.
-constexpr int kGranuleX = 2048;   // binary16 of a granule of x: 32 rows of 128 bytes, a row's 16-byte pieces turned (turn_of)
-constexpr int kGranuleP = 1024;   // of W: two halves of the block, each in the order of lanes of an MFMA's operand
-constexpr int kGranuleS = 32;     // float32 scales of W
-constexpr int kGroup = 8;         // blocks whose scales come into LDS together: a KB a strip
-
-// x: row m's pieces 4 part + 2 half + hi of a block, hi which eight of the half's sixteen, lie at piece ^ turn, so that the
-// 32 rows of a fragment read fall on all banks while a row's block stays one line for the kernels that write it.
-__host__ __device__ inline int64_t row_at(int m, int nb) { return (int64_t)(m >> 5) * nb * kGranuleX + (m & 31) * 64; }
-__host__ __device__ inline int turn_of(int m) { return (m >> 1) & 7; }
-
-// How a row of x is held. The row's information is {exponent, form}.
-enum Form { kHalves = 0, kBlockHalves = 1, kDigits = 2 };
+constexpr int kMinPartRows = 9;    // of several together with the other kernels
 
 // Thread t takes elements 4t..4t+3 of row blockIdx.y; a block's eight threads are consecutive lanes.
 __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restrict__ x, int64_t x_row_stride, int K, uint16_t* __restrict__ X16,
                                                           float* __restrict__ XS, int2* __restrict__ RS) {
     const int nb = K >> 5;
-    if (blockIdx.x == 0 && threadIdx.x == 0) RS[blockIdx.y] = make_int2(0, kDigits);
+    if (blockIdx.x == 0 && threadIdx.x == 0) RS[blockIdx.y] = make_int2(0, kDigitPairs);
     const float* xr = x + (int64_t)blockIdx.y * x_row_stride;
     uint16_t* row = X16 + row_at((int)blockIdx.y, nb);
     const int turn = turn_of((int)blockIdx.y);
@@ -227,18 +209,6 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
     }
 }
 
-__host__ __device__ inline int scale_blocks(int nb) { return (nb + kGroup - 1) / kGroup * kGroup; }  // of a strip: whole groups
-
-// What is multiplied by the same x: up to three matrices, or gate and up, whose strips then lie in turn.
-struct Parts {
-    const uint8_t* W[3];
-    float* y[3];
-    int N[3];      // rows of W
-    int begin[3];  // first strip; those of parts that are not there lie past the last
-    int strips;    // of all
-    int swiglu;    // W[0] and W[1] are gate and up: y[0] gets silu(gate) up
-};
-
 // W's integers n - 8 as binary16 and its scales as float32, in granules; an odd block's scale is negative (tile_body says why). A
 // wavefront takes a strip's block: lane r + 32 q the eight bytes q of row r, whose low nibbles are piece q of the block's
 // first half and whose high nibbles of its second.
@@ -252,22 +222,9 @@ __global__ __launch_bounds__(256) void fx16_panel_kernel(Parts parts, uint16_t* 
         const uint8_t* block = row + b * 18;
         const uint16_t* src = (const uint16_t*)(block + 2 + 8 * q);  // blocks are 2-byte aligned, no more
         const uint32_t raw[2] = {(uint32_t)src[0] | (uint32_t)src[1] << 16, (uint32_t)src[2] | (uint32_t)src[3] << 16};
-        const f16x2 off = {(_Float16)1032.f, (_Float16)1032.f};
         uint16_t* out = P + ((int64_t)strip * nb + b) * kGranuleP + lane * 8;
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-            u32x4 v;
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                // the nibble into the mantissa of binary16's 1024; minus 1032 is n - 8
-                const uint32_t nib = (raw[i] >> (4 * half)) & 0x0f0f0f0fu;
-                const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u);
-                const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u);
-                v[2 * i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p0) - off);
-                v[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p1) - off);
-            }
-            *(u32x4*)(out + 512 * half) = v;
-        }
+        for (int half = 0; half < 2; half++) *(f16x8*)(out + 512 * half) = nibbles_to_f16(raw[0], raw[1], half);
         if (q == 0) SW[((int64_t)strip * scale_blocks(nb) + b) * kGranuleS + r] = f16_bits_to_f32(load_u16(block) ^ ((b & 1) << 15));
     }
 }
@@ -308,25 +265,6 @@ struct Shape {
 using Low = Shape<2, 2, 2, 4>;   // 128 x 256
 using Wide = Shape<4, 2, 4, 3>;  // 256 x 256
 constexpr int kLdsBytes = Low::total > Wide::total - 2 * 256 * 4 ? Low::total : Wide::total - 2 * 256 * 4;  // Wide has no scales of x
-
-struct Operands {
-    const uint16_t* P;
-    const float* SW;
-    const uint16_t* X16;
-    const float* XS;
-    const int2* RS;
-    const float* resid;  // may be y; added to what one part's y gets
-    float* sums;         // where K is cut into shares: [share][M][32 strips] float32, finished by fx16_sum_kernel
-    int M, nb;
-    Parts parts;
-};
-
-__device__ __forceinline__ float silu_times(float g, float u) {  // as swiglu_kernel's
-    const float e = __builtin_exp2f(g * (float)(-1.4426950408889634));
-    const float s = 1.0f / (1.0f + e);
-    const float a = g * s;
-    return a * u;
-}
 
 // One tile: rows m0 .. m0 + BM of x by columns n0 .. n0 + BN, blocks b0 .. b0 + count of K (b0 a multiple of a group), of rows of
 // x that are all of one form, or halves of either kind (kBlockHalves).
@@ -463,7 +401,7 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
             for (int sub = 0; sub < MT * NT; sub++) {  // NT is 2 here: both of b are there
                 const int mt = sub / NT, nt = sub % NT;
                 f32x16 c0, c1;
-                if (FORM == kDigits) {
+                if (FORM == kDigitPairs) {
                     c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][0], b[nt][0], zero, 0, 0, 0);
                     c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1][0], b[nt][0], zero, 0, 0, 0);
                     c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][0][1], b[nt][1], c0, 0, 0, 0);
@@ -476,7 +414,7 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
                 if (nt == 0) w = __builtin_amdgcn_mfma_f32_32x32x1f32(dx[mt], dw, none, 0, 0, 0);
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    const float sum = FORM == kDigits ? fmaf(c1[e], 4096.f, c0[e]) : c0[e];  // digits: the exact integer, rounded once
+                    const float sum = FORM == kDigitPairs ? fmaf(c1[e], 4096.f, c0[e]) : c0[e];  // digits: the exact integer, rounded once
                     acc[mt][nt][e] = fmaf(w[16 * nt + e], sum, acc[mt][nt][e]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -504,10 +442,10 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
         const int strip = n0 / 32 + wn * NT + nt;
         if (strip >= o.parts.strips) break;
         if (gated && (nt & 1)) continue;  // taken with the gate's
-        const int part = gated || sums ? 0 : strip >= o.parts.begin[2] ? 2 : strip >= o.parts.begin[1] ? 1 : 0;
+        int n0s;
+        const int part = part_of(o.parts, strip, &n0s);
         float* y = sums ? sums : o.parts.y[part];
-        const int N = sums ? o.parts.strips * 32 : o.parts.N[part];
-        const int n = (sums ? strip : gated ? strip >> 1 : strip - o.parts.begin[part]) * 32 + (r32 & ~3);
+        const int N = sums ? o.parts.strips * 32 : o.parts.N[part], n = (sums ? strip * 32 : n0s) + (r32 & ~3);
         const bool wide_ok = (N & 3) == 0 && ((uintptr_t)y & 15) == 0 && (!resid || ((uintptr_t)resid & 15) == 0);
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
@@ -519,9 +457,7 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
 #pragma unroll
                     for (int k = 0; k < 4; k++) v[k] = acc[mt][col][4 * q + k];
                     quad_transpose(v, lane);
-                    if (FORM == kHalves)
-#pragma unroll
-                        for (int k = 0; k < 4; k++) v[k] = e_row == INT32_MAX ? __builtin_nanf("") : __builtin_ldexpf(v[k], e_row);
+                    if (FORM == kHalves) under_exponent(v, e_row);
                 };
                 float v[4];
                 row_of(nt, v);
@@ -531,24 +467,7 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
 #pragma unroll
                     for (int k = 0; k < 4; k++) v[k] = silu_times(v[k], u[k]);
                 }
-                if (m >= M || n >= N) continue;
-                if (wide_ok && n + 3 < N) {
-                    f32x4 out = {v[0], v[1], v[2], v[3]};
-                    if (resid) {
-                        const f32x4 r = *(const f32x4*)(resid + (int64_t)m * N + n);
-#pragma unroll
-                        for (int k = 0; k < 4; k++) out[k] = out[k] + r[k];
-                    }
-                    *(f32x4*)(y + (int64_t)m * N + n) = out;
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        if (n + k >= N) continue;
-                        float out = v[k];
-                        if (resid) out = out + resid[(int64_t)m * N + n + k];
-                        y[(int64_t)m * N + n + k] = out;
-                    }
-                }
+                if (m < M && n < N) store_four(y, resid, m, N, n, v, wide_ok);
             }
     }
 }
@@ -580,7 +499,7 @@ __device__ __forceinline__ void product(const Operands& o, const Cut& cut, char*
     float* sums = o.sums ? o.sums + (int64_t)share * o.M * o.parts.strips * 32 : nullptr;
     int m0 = tile % tiles_m * bm;
     if (DIGITS) {
-        tile_body<Low, kDigits>(o, m0, n0, b0, count, sums, lds);
+        tile_body<Low, kDigitPairs>(o, m0, n0, b0, count, sums, lds);
     } else if (!by_block(o, m0, bm)) {
         if (wide) tile_body<Wide, kHalves>(o, m0, n0, b0, count, sums, lds);
         else tile_body<Low, kHalves>(o, m0, n0, b0, count, sums, lds);
@@ -602,7 +521,7 @@ __global__ __launch_bounds__(512) void qgemm_q4_0_fx16_digits_kernel(Operands o,
     product<true>(o, cut, lds);
 }
 
-// The shares' sums, in their order, four columns a thread: y = ((s0 + s1) + ..) (+ resid), or silu(gate) up of them.
+// Four columns a thread.
 __global__ __launch_bounds__(256) void fx16_sum_kernel(Operands o, int shares) {
     const int64_t ld = (int64_t)o.parts.strips * 32, quads = o.M * ld / 4, step = o.M * ld;
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < quads; t += (int64_t)gridDim.x * 256) {
@@ -624,30 +543,17 @@ __global__ __launch_bounds__(256) void fx16_sum_kernel(Operands o, int shares) {
 #pragma unroll
             for (int k = 0; k < 4; k++) v[k] = silu_times(v[k], u[k]);
         }
-        const int part = o.parts.swiglu ? 0 : strip >= o.parts.begin[2] ? 2 : strip >= o.parts.begin[1] ? 1 : 0, N = o.parts.N[part];
-        const int n = (o.parts.swiglu ? strip >> 1 : strip - o.parts.begin[part]) * 32 + (at & 31);
-        float* y = o.parts.y[part] + m * N + n;
-        const float* resid = o.resid ? o.resid + m * N + n : nullptr;
-        if ((N & 3) == 0 && ((uintptr_t)o.parts.y[part] & 15) == 0 && ((uintptr_t)o.resid & 15) == 0) {
-            if (n >= N) continue;
-            if (resid) {
-                const f32x4 r = *(const f32x4*)resid;
-#pragma unroll
-                for (int k = 0; k < 4; k++) v[k] = v[k] + r[k];
-            }
-            *(f32x4*)y = v;
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                if (n + k < N) y[k] = resid ? v[k] + resid[k] : v[k];
-        }
+        int n;
+        const int part = part_of(o.parts, strip, &n), N = o.parts.N[part];
+        n += at & 31;
+        const bool wide_ok = (N & 3) == 0 && ((uintptr_t)o.parts.y[part] & 15) == 0 && ((uintptr_t)o.resid & 15) == 0;
+        const float out[4] = {v[0], v[1], v[2], v[3]};
+        if (n < N) store_four(o.parts.y[part], o.resid, m, N, n, out, wide_ok);
     }
 }
 
 // measurement aid: 0 keeps every product on the int8 form, 2 takes the digits' form whatever the shape, 3 the halves'
 std::atomic<int> g_fx16{1};
-
-int64_t strips_of(int64_t rows) { return (rows + 31) / 32; }
 
 // Microseconds of a product, the pass over W and the shares' sums included, and its cut. A compute unit takes a tile at a
 // time; the time of a tile's block grows with how many units are at work, as the clock falls: 0.72 + 0.32 of them for a
@@ -700,16 +606,25 @@ bool fits(int64_t M, int64_t strips, int64_t K) {
 
 void set_q4_0_fx16(int v) { g_fx16 = v; }
 
+hipError_t sum_shares(const Operands& o, int shares, hipStream_t st) {
+    const int64_t groups = ((int64_t)o.M * o.parts.strips * 8 + 255) / 256;
+    hipLaunchKernelGGL(fx16_sum_kernel, dim3((unsigned)(groups < 16384 ? groups : 16384)), dim3(256), 0, st, o, shares);
+    return hipGetLastError();
+}
+
 // Whether the product is the faster here than in the int8 form (qgemm_q4_0_fx_cost_us). mi355x_qgemv cuts K into shares of
 // no less than 96 blocks: 512 x 4096 x 4096 stays with the int8 form there (88 us, in one pass here 114), which
 // tests/test_gpu_qgemm_fx.py holds it to; 512 x 14336 x 4096 comes here (151 us, 217 in the int8 form).
 constexpr int64_t kMinShareBlocks = 96;
 
+double qgemm_q4_0_fx16_cost_us(int64_t M, int64_t N, int64_t K) {
+    Cut cut;
+    return M < kMinRows || N <= 0 || !fits(M, strips_of(N), K) ? 1e30 : plan(M, strips_of(N), K, kMinShareBlocks, (size_t)-1, &cut);
+}
+
 bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K) {
     if (g_fx16 == 0 || N <= 0 || !fits(M, strips_of(N), K)) return false;
-    if (g_fx16 >= 2) return true;
-    Cut cut;
-    return M >= kMinRows && plan(M, strips_of(N), K, kMinShareBlocks, (size_t)-1, &cut) < qgemm_q4_0_fx_cost_us(M, N, K);
+    return g_fx16 >= 2 || qgemm_q4_0_fx16_cost_us(M, N, K) < qgemm_q4_0_fx_cost_us(M, N, K);
 }
 
 // X16 in granules, then RS [M] int2, then XS [M, K / 32] float32.
@@ -754,6 +669,20 @@ size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K) {
     return panel_bytes(strips_of(N), K) + scales_bytes(strips_of(N), K) + (cut.shares > 1 ? (size_t)cut.shares * (size_t)M * (size_t)strips_of(N) * 128 : 0);
 }
 
+// x's part of the operands.
+static Operands operands(const Parts& parts, const void* act, const float* resid, int64_t M, int64_t K) {
+    const int nb = (int)(K / 32);
+    const uint16_t* X16 = (const uint16_t*)act;
+    const int2* RS = (const int2*)(X16 + strips_of(M) * nb * kGranuleX);
+    return Operands{nullptr, nullptr, X16, (const float*)(RS + M), RS, resid, nullptr, (int)M, nb, parts};
+}
+
+static hipError_t in_place(const Parts& parts, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes, hipStream_t st) {
+    Operands o = operands(parts, act, resid, M, K);
+    o.sums = (float*)ws;
+    return qgemm_q4_0_direct(o, ws_bytes, st);
+}
+
 static hipError_t multiply(const Parts& parts, const void* act, const float* resid, int64_t M, int64_t K, int64_t min_share_blocks, void* ws, size_t ws_bytes,
                            hipStream_t st) {
     const int64_t strips = parts.strips;
@@ -774,18 +703,17 @@ static hipError_t multiply(const Parts& parts, const void* act, const float* res
     if (!digits) plan(M, strips, K, min_share_blocks, ws_bytes - fixed, &cut);
     uint16_t* P = (uint16_t*)ws;
     float* SW = (float*)((char*)ws + panel_bytes(strips, K));
-    const uint16_t* X16 = (const uint16_t*)act;
-    const int2* RS = (const int2*)(X16 + strips_of(M) * nb * kGranuleX);
-    const Operands o{P, SW, X16, (const float*)(RS + M), RS, resid, cut.shares > 1 ? (float*)((char*)ws + fixed) : nullptr, (int)M, nb, parts};
+    Operands o = operands(parts, act, resid, M, K);
+    o.P = P;
+    o.SW = SW;
+    if (cut.shares > 1) o.sums = (float*)((char*)ws + fixed);
     const int64_t wide = (int64_t)cut.wide_m * cut.wide_cols * cut.shares, low = (int64_t)cut.low_m * cut.low_cols * cut.shares;
     hipLaunchKernelGGL(fx16_panel_kernel, dim3((unsigned)((nb + 7) / 8), (unsigned)strips), dim3(256), 0, st, parts, P, SW, nb);
     const dim3 grid((unsigned)((wide + 7) / 8 * 8 + (low + 7) / 8 * 8));
     if (digits) hipLaunchKernelGGL(qgemm_q4_0_fx16_digits_kernel, grid, dim3(512), Low::total, st, o, cut);
     else hipLaunchKernelGGL(qgemm_q4_0_fx16_kernel, grid, dim3(512), kLdsBytes, st, o, cut);
-    if (cut.shares > 1) {
-        const int64_t groups = (M * strips * 8 + 255) / 256;
-        hipLaunchKernelGGL(fx16_sum_kernel, dim3((unsigned)(groups < 16384 ? groups : 16384)), dim3(256), 0, st, o, cut.shares);
-    }
+    if (cut.shares > 1)
+        if (hipError_t e = sum_shares(o, cut.shares, st)) return e;
     char shares[40] = "", beside[60] = "";
     if (cut.shares > 1) snprintf(shares, sizeof shares, ", %d shares of K", cut.shares);
     if (cut.wide_cols && cut.low_cols) snprintf(beside, sizeof beside, ", %d x %d tiles of 128 x 256", cut.low_m, cut.low_cols);
@@ -824,19 +752,30 @@ size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K) {
     return parts_of(part, n, false, K, &p) ? panel_bytes(p.strips, K) + scales_bytes(p.strips, K) + kMostSums : 0;
 }
 
+// Microseconds here, the cheaper way: with the pass over W first, or W read where it lies.
+static double parts_cost_us(const Parts& p, int64_t M, int64_t K, size_t ws_bytes, bool* direct) {
+    Cut cut;
+    const size_t fixed = panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
+    const double panel = fits(M, p.strips, K) && ws_bytes >= fixed ? plan(M, p.strips, K, kMinPartShareBlocks, ws_bytes - fixed, &cut) : 1e30;
+    const bool aligned = (((uintptr_t)p.W[0] | (uintptr_t)p.W[1] | (uintptr_t)p.W[2]) & 3) == 0;
+    const double in_place = aligned ? qgemm_q4_0_direct_cost_us(M, p.strips, K, ws_bytes) : 1e30;
+    *direct = in_place < panel;
+    return *direct ? in_place : panel;
+}
+
 // Whether they are the faster together here, in a workspace of ws_bytes, than each on the int8 form or the row kernels.
 bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes) {
     Parts p;
-    Cut cut;
-    if (g_fx16 == 0 || g_fx16 == 2 || M < kMinPartRows || !parts_of(part, n, swiglu, K, &p) || !fits(M, p.strips, K)) return false;
-    const size_t fixed = panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
-    if (ws_bytes < fixed) return false;
+    bool direct;
+    if (g_fx16 == 0 || g_fx16 == 2 || M < kMinPartRows || !parts_of(part, n, swiglu, K, &p)) return false;
+    const double us = parts_cost_us(p, M, K, ws_bytes, &direct);
+    if (us >= 1e30) return false;
     double apart = 0;
     for (int i = 0; i < n; i++) {
         const double rows_us = (double)M * ((double)part[i].N * (double)(K / 32) * 18.0) / 8.7e6, fx = qgemm_q4_0_fx_cost_us(M, part[i].N, K);
         apart += fx < rows_us ? fx : rows_us;
     }
-    return g_fx16 >= 3 || plan(M, p.strips, K, kMinPartShareBlocks, ws_bytes - fixed, &cut) < apart;
+    return g_fx16 >= 3 || us < apart;
 }
 
 // act: q4_0_fx16_convert_act's for these M rows; ws: ws_bytes, 16-byte aligned. Each part's y = x . W^T; one part alone: + resid, which
@@ -844,7 +783,10 @@ bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t
 hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes,
                                  hipStream_t st) {
     Parts p;
-    if (!parts_of(part, n, swiglu, K, &p) || (resid && n != 1)) return hipErrorInvalidValue;
+    bool direct;
+    if (!parts_of(part, n, swiglu, K, &p) || (resid && n != 1) || !ws || ((uintptr_t)ws & 15) != 0) return hipErrorInvalidValue;
+    parts_cost_us(p, M, K, ws_bytes, &direct);
+    if (direct) return in_place(p, act, resid, M, K, ws, ws_bytes, st);
     return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, st);
 }
 
@@ -855,6 +797,26 @@ hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float
     const int n = (int)strips_of(N);
     const Parts parts{{(const uint8_t*)W, nullptr, nullptr}, {y, nullptr, nullptr}, {(int)N, 0, 0}, {0, n, n}, n, 0};
     return multiply(parts, act, resid, M, K, kMinShareBlocks, ws, qgemm_q4_0_fx16_ws_bytes(M, N, K), st);
+}
+
+// y = x . W^T, W read where it lies: ws 16-byte aligned.
+hipError_t qgemm_q4_0_in_place(const void* W, const void* act, float* y, int64_t M, int64_t N, int64_t K, void* ws, size_t ws_bytes, hipStream_t st) {
+    Parts p;
+    const Fx16Part alone{W, y, N};
+    if (!parts_of(&alone, 1, false, K, &p) || !ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)act & 15) != 0) return hipErrorInvalidValue;
+    return in_place(p, act, nullptr, M, K, ws, ws_bytes, st);
+}
+
+double qgemm_q4_0_in_place_cost_us(const void* W, int64_t M, int64_t N, int64_t K, size_t* ws_bytes) {
+    *ws_bytes = qgemm_q4_0_direct_sums_bytes(M, strips_of(N));
+    if (g_fx16 == 0 || g_fx16 == 2 || N <= 0 || N >= (1 << 25) || ((uintptr_t)W & 3) != 0) return 1e30;
+    const double us = qgemm_q4_0_direct_cost_us(M, strips_of(N), K, *ws_bytes);
+    return g_fx16 == 3 && us < 1e30 ? -1e6 : us;
+}
+
+hipError_t q4_0_halves_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
+    launch_halves<false>(x, nullptr, 0, M, K, x_row_stride, act, st);
+    return hipGetLastError();
 }
 
 }  // namespace mimir

@@ -1,4 +1,5 @@
-"""The Q4_0 product of many rows of float32 x on the binary16 matrix cores, x as pairs of binary16 (qgemm_q4_0_fx16.hip), against the
+"""The Q4_0 product of many rows of float32 x on the binary16 matrix cores, x as pairs of binary16 (qgemm_q4_0_fx16.hip,
+qgemm_q4_0_direct.hip), against the
 product in 64 bits. Bound: a pair holds an element to 2^-23 of its block's largest magnitude (kernel's comment), beside
 float32 sums' 2e-6 sum |x||w|; what the fixed-point forms of this product are held to."""
 import ctypes
@@ -29,12 +30,19 @@ def tuned(rows, pairs):
     capi.check(gpu.lib().mi355x_tune(b"q4_0.fx_pairs", pairs))
 
 
-@pytest.mark.parametrize("m,n,k,tiles", [
-    (1, 5, 128, "1 x 1 tiles of 128 x 256"), (40, 100, 256, "1 x 1 tiles of 128 x 256"), (129, 257, 384, "2 x 2 tiles of 128 x 256"),
-    (300, 520, 6272, "3 x 3 tiles of 128 x 256, 2 shares of K"), (257, 129, 14336, "3 x 1 tiles of 128 x 256, 5 shares of K"),
-    (1000, 16500, 128, "4 x 64 tiles of 256 x 256, 8 x 1 tiles of 128 x 256"), (2047, 8192, 128, "8 x 32 tiles of 256 x 256"), (33, 60, 16512, "1 x 1 tiles of 128 x 256, 5 shares of K")])
+PANEL, IN_PLACE = "qgemm_q4_0_fx16_kernel: ", "qgemm_q4_0_direct_kernel"
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (1, 5, 128, PANEL + "1 x 1 tiles of 128 x 256"), (40, 100, 256, PANEL + "1 x 1 tiles of 128 x 256"), (129, 257, 384, PANEL + "2 x 2 tiles of 128 x 256"),
+    (300, 520, 6272, PANEL + "3 x 3 tiles of 128 x 256, 2 shares of K"), (257, 129, 14336, PANEL + "3 x 1 tiles of 128 x 256, 5 shares of K"),
+    (1000, 16500, 128, PANEL + "4 x 64 tiles of 256 x 256, 8 x 1 tiles of 128 x 256"), (2047, 8192, 128, PANEL + "8 x 32 tiles of 256 x 256"),
+    (33, 60, 16512, PANEL + "1 x 1 tiles of 128 x 256, 5 shares of K"),
+    # W read where it lies: one to four strips of x and two tiles, columns that fill no group, shares that are not of one length
+    (16, 5, 64, IN_PLACE + "<1>: 1 x 1 tiles, 1 shares of K"), (33, 129, 192, IN_PLACE + "<2>"), (77, 515, 5120, IN_PLACE + "<3>"), (128, 4096, 4160, IN_PLACE + "<4>"),
+    (130, 200, 320, IN_PLACE + "<4>: 2 x 2 tiles, 1 shares of K"), (256, 70, 16448, IN_PLACE + "<4>: 2 x 1 tiles, ")])
 @pytest.mark.parametrize("rows", ["even", "wide", "special"])
-def test_pairs_of_halves(m, n, k, tiles, rows):
+def test_pairs_of_halves(m, n, k, kernel, rows):
     """Every cut of the product, tiles and strips that rows and columns do not fill. Rows of x: of very different magnitude; some whose
     blocks differ by up to 2^60 (those take an exponent a block, and a tile with one of them its slower loop); blocks and
     rows of zeros, the smallest and largest magnitudes, a NaN and an infinity (a row of NaNs each, and of no other)."""
@@ -56,12 +64,12 @@ def test_pairs_of_halves(m, n, k, tiles, rows):
         bad = [2, 5]
     wide = torch.zeros((m, k + 8), device="cuda:0")  # rows further apart than K
     wide[:, :k] = gpu.dev(x)
-    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    buf, ptr = gpu.dev_bytes_at(raw, 4)
     gpu.say(f"q4_0 halves M={m} N={n} K={k} {rows}")
     try:
-        tuned(1, 3)
+        tuned(1 if kernel.startswith(PANEL) else 0, 3)
         got = gpu.qgemv(O.Q4_0, ptr, wide[:, :k], n, k)
-        assert last_kernel() == "qgemm_q4_0_fx16_kernel: " + tiles
+        assert last_kernel().startswith(kernel) and (kernel.startswith(IN_PLACE) or last_kernel() == kernel)
     finally:
         tuned(0, 1)
     x64 = gpu.dev(x).double()

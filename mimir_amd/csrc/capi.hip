@@ -140,7 +140,7 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
     if (dtype == MI355X_Q4_0 && g_tune_gemm != 1 && mimir::qgemm_q4_0_ok(W, X, M, N, K, x_row_stride)) {
         if (g_tune_gemm_f16 == 0 && mimir::qgemm_q4_0_blocks_pays(M, N, K)) {
             // the exact form of a large product: W's integers once as a bfloat16 panel, then one MFMA a weight
-            if (mi355x_status s2 = gemm_scratch(stream, mimir::qgemm_q4_0_blocks_ws_bytes(N, K), &ws)) return s2;
+            if (mi355x_status s2 = gemm_scratch(stream, mimir::qgemm_q4_0_blocks_ws_bytes(M, N, K), &ws)) return s2;
             HIP_TRY(mimir::qgemm_q4_0_blocks(W, X, x_row_stride, Y, M, N, K, f32, ws, st), "launch qgemm_q4_0_blocks");
             return MI355X_OK;
         }

@@ -89,6 +89,36 @@ __device__ __forceinline__ void under_exponent(float v[4], int e) {
     for (int k = 0; k < 4; k++) v[k] = e == INT32_MAX ? __builtin_nanf("") : __builtin_ldexpf(v[k], e);
 }
 
+// What lane half q takes of a pair of blocks: of each its eight bytes q of nibbles, and, q = 0, its scale's bits.
+struct PairBytes { uint32_t lo[2], hi[2], scale[2]; };
+
+// 36 bytes at `pair`, as two loads of twelve where they are on a 4-byte boundary: bytes 8 q .. + 12 have the even block's eight two
+// bytes in (q = 0: behind the scale), 16 + 8 q .. + 12 the odd one's last (q = 0: behind the scale and two bytes). Five loads of two bytes a
+// block, which is all that blocks' own alignment allows, took the pass over W a little longer.
+__device__ __forceinline__ PairBytes load_pair(const uint8_t* pair, int q, bool aligned) {
+    PairBytes p;
+    if (aligned) {
+        u32x3 a, b;
+        __builtin_memcpy(&a, __builtin_assume_aligned(pair + 8 * q, 4), 12);
+        __builtin_memcpy(&b, __builtin_assume_aligned(pair + 16 + 8 * q, 4), 12);
+        p.lo[0] = __builtin_amdgcn_alignbyte(a[1], a[0], 2);
+        p.hi[0] = __builtin_amdgcn_alignbyte(a[2], a[1], 2);
+        p.lo[1] = b[1];
+        p.hi[1] = b[2];
+        p.scale[0] = a[0] & 0xffffu;
+        p.scale[1] = b[0] >> 16;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint16_t* src = (const uint16_t*)(pair + 18 * i + 2 + 8 * q);
+            p.lo[i] = (uint32_t)src[0] | (uint32_t)src[1] << 16;
+            p.hi[i] = (uint32_t)src[2] | (uint32_t)src[3] << 16;
+            p.scale[i] = load_u16(pair + 18 * i);
+        }
+    }
+    return p;
+}
+
 // Eight nibbles (the low or the high ones of two dwords) as the binary16 integers n - 8: the nibble into the mantissa of binary16's
 // 1024, minus 1032.
 __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t lo, uint32_t hi, int half) {

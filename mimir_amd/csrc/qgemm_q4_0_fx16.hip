@@ -214,18 +214,23 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
 // first half and whose high nibbles of its second.
 __global__ __launch_bounds__(256) void fx16_panel_kernel(Parts parts, uint16_t* __restrict__ P, float* __restrict__ SW, int nb) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, q = lane >> 5;
-    const int strip = blockIdx.y;
+    const int groups = (nb + 31) >> 5, strip = (int)blockIdx.x / groups, first = ((int)blockIdx.x - strip * groups) * 32 + 8 * wave;  // of blocks
     const int part = parts.swiglu ? strip & 1 : strip >= parts.begin[2] ? 2 : strip >= parts.begin[1] ? 1 : 0;
     const int n = (parts.swiglu ? strip >> 1 : strip - parts.begin[part]) * 32 + r, N = parts.N[part];
     const uint8_t* row = parts.W[part] + (int64_t)(n < N ? n : N - 1) * nb * 18;  // past the matrix: its last row again
-    for (int b = blockIdx.x * 8 + wave; b < nb && b < (int)blockIdx.x * 8 + 8; b += 4) {
-        const uint8_t* block = row + b * 18;
-        const uint16_t* src = (const uint16_t*)(block + 2 + 8 * q);  // blocks are 2-byte aligned, no more
-        const uint32_t raw[2] = {(uint32_t)src[0] | (uint32_t)src[1] << 16, (uint32_t)src[2] | (uint32_t)src[3] << 16};
+    const bool aligned = ((uintptr_t)parts.W[part] & 3) == 0;
+    PairBytes pair[4];  // nb is even
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (first + 2 * i < nb) pair[i] = load_pair(row + (first + 2 * i) * 18, q, aligned);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int b = first + i;
+        if (b >= nb) return;
         uint16_t* out = P + ((int64_t)strip * nb + b) * kGranuleP + lane * 8;
 #pragma unroll
-        for (int half = 0; half < 2; half++) *(f16x8*)(out + 512 * half) = nibbles_to_f16(raw[0], raw[1], half);
-        if (q == 0) SW[((int64_t)strip * scale_blocks(nb) + b) * kGranuleS + r] = f16_bits_to_f32(load_u16(block) ^ ((b & 1) << 15));
+        for (int half = 0; half < 2; half++) *(f16x8*)(out + 512 * half) = nibbles_to_f16(pair[i / 2].lo[i & 1], pair[i / 2].hi[i & 1], half);
+        if (q == 0) SW[((int64_t)strip * scale_blocks(nb) + b) * kGranuleS + r] = f16_bits_to_f32((uint16_t)(pair[i / 2].scale[i & 1] ^ ((b & 1) << 15)));
     }
 }
 
@@ -708,7 +713,7 @@ static hipError_t multiply(const Parts& parts, const void* act, const float* res
     o.SW = SW;
     if (cut.shares > 1) o.sums = (float*)((char*)ws + fixed);
     const int64_t wide = (int64_t)cut.wide_m * cut.wide_cols * cut.shares, low = (int64_t)cut.low_m * cut.low_cols * cut.shares;
-    hipLaunchKernelGGL(fx16_panel_kernel, dim3((unsigned)((nb + 7) / 8), (unsigned)strips), dim3(256), 0, st, parts, P, SW, nb);
+    hipLaunchKernelGGL(fx16_panel_kernel, dim3((unsigned)((nb + 31) / 32 * strips)), dim3(256), 0, st, parts, P, SW, nb);
     const dim3 grid((unsigned)((wide + 7) / 8 * 8 + (low + 7) / 8 * 8));
     if (digits) hipLaunchKernelGGL(qgemm_q4_0_fx16_digits_kernel, grid, dim3(512), Low::total, st, o, cut);
     else hipLaunchKernelGGL(qgemm_q4_0_fx16_kernel, grid, dim3(512), kLdsBytes, st, o, cut);

@@ -96,6 +96,98 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_bf16_rows_kernel(const uint1
     }
 }
 
+// Eight rows of W a workgroup, for matrices whose sixteens are fewer than the compute units: what a unit draws from memory is
+// bounded (13 to 16 GB/s measured in the kernels that read weights once, whatever is under way), so every one of them has to.
+// The operand's other eight rows are the same rows of W 32 of K further on: a lane's sixteen bytes of eight rows are whole lines of 128.
+// They are multiplied by x of either step, and of each product the half is kept whose step it is; the matrix cores have the time.
+// 4 x 2048 x 8192: 19.3 us in sixteens on 128 units, here 15.5. What is left is x as much as W: every workgroup loads and converts all of it.
+template <int kWaves, Out KIND>
+__global__ __launch_bounds__(64 * kWaves) void gemv_bf16_rows_eight_kernel(const uint16_t* __restrict__ W, int64_t ldw, const float* __restrict__ x, int64_t ldx,
+                                                                           int M, int N, int K, ProductOut out) {
+    __shared__ float red[kWaves][16][17];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 8, row8 = r16 & 7, step = r16 >> 3;
+    const bool low = r16 >= 8;
+    const int pairs = K / 64, per = (pairs + kWaves - 1) / kWaves;
+    const int k0 = wave * per * 64, k1 = k0 + per * 64 < K ? k0 + per * 64 : K;
+    const float* xp = x + (int64_t)(row8 < M ? row8 : M - 1) * ldx + g * 8;
+    const uint16_t* wp = W + (int64_t)(n0 + row8 < N ? n0 + row8 : N - 1) * ldw + step * 32 + g * 8;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    // kSteps steps of 64 are under way, W and x; each one's registers are refilled as it is multiplied
+    constexpr int kSteps = 4;
+    auto sum_of = [&](int from, int to) {
+        const int n = (to - from) / 64;
+        if (n <= 0) return;
+        u32x4 w[kSteps];
+        f32x4 xv[kSteps][4];
+        auto load = [&](int i, int slot) {
+            const int k = from + 64 * (i < n ? i : n - 1);
+            w[slot] = *(const u32x4*)(wp + k);
+#pragma unroll
+            for (int j = 0; j < 4; j++) xv[slot][j] = *(const f32x4*)(xp + k + 32 * (j >> 1) + 4 * (j & 1));
+        };
+        auto multiply = [&](int slot) {
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const f32x4 a = xv[slot][2 * s], b = xv[slot][2 * s + 1];
+                float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+                u32x4 q;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (low) {
+                        v[2 * i] = low_part(v[2 * i]);
+                        v[2 * i + 1] = low_part(v[2 * i + 1]);
+                    }
+                    q[i] = pack_bf16(v[2 * i], v[2 * i + 1]);
+                }
+                acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[slot]), __builtin_bit_cast(bf16x8, q), acc[s], 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < kSteps; u++) load(u, u);
+        int base = 0;
+        for (; base + kSteps < n; base += kSteps)
+#pragma unroll
+            for (int u = 0; u < kSteps; u++) {
+                multiply(u);
+                load(base + kSteps + u, u);
+            }
+#pragma unroll
+        for (int u = 0; u < kSteps; u++)
+            if (base + u < n) multiply(u);
+    };
+    int from = k0;
+    if (KIND == Out::Scaled && out.mid) {  // what of this wavefront's piece lies below split has a factor of its own
+        const int to = out.split < k1 ? (int)out.split : k1;
+        sum_of(k0, to);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int n = n0 + ((4 * g + i) & 7);
+            const float f = out.mid[n < N ? n : N - 1];
+            acc[0][i] *= f;
+            acc[1][i] *= f;
+        }
+        if (to > from) from = to;
+    }
+    sum_of(from, k1);
+    // a lane holds column r16 of rows 4 g .. 4 g + 3; rows 8 and up are the second step's
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[wave][4 * g + i][r16] = g < 2 ? acc[0][i] : acc[1][i];
+    __syncthreads();
+    if (tid < 64) {
+        const int row = tid >> 3, col = tid & 7, n = n0 + row;
+        if (col >= M || n >= N) return;
+        auto sum = [&](int r) {
+            float v = 0.f;
+#pragma unroll
+            for (int i = 0; i < kWaves; i++) v += (red[i][r][col] + red[i][r][col + 8]) + (red[i][r + 8][col] + red[i][r + 8][col + 8]);
+            return v;
+        };
+        if (KIND != Out::Pairs || n < out.pair_from) store_column<KIND>(out, col, n, sum(row));
+        else if ((row & 1) == 0) store_pair(out, col, n, sum(row), sum(row + 1));
+    }
+}
+
 }  // namespace
 
 hipError_t gemv_bf16_rows(const uint16_t* W, int64_t ldw, const float* x, int64_t ldx, int64_t M, int64_t N, int64_t K, const ProductOut& out, hipStream_t st) {
@@ -112,8 +204,18 @@ hipError_t gemv_bf16_rows(const uint16_t* W, int64_t ldw, const float* x, int64_
         else if (kind == Out::Pairs) launch(gemv_bf16_rows_kernel<T, kWaves, Out::Pairs>, 16 * T, kWaves);
         else launch(gemv_bf16_rows_kernel<T, kWaves, Out::Scaled>, 16 * T, kWaves);
     };
+    auto eight_by_kind = [&](auto waves) {
+        constexpr int kWaves = decltype(waves)::value;
+        const Out kind = out_kind(out, N);
+        if (kind == Out::Plain) launch(gemv_bf16_rows_eight_kernel<kWaves, Out::Plain>, 8, kWaves);
+        else if (kind == Out::Pairs) launch(gemv_bf16_rows_eight_kernel<kWaves, Out::Pairs>, 8, kWaves);
+        else launch(gemv_bf16_rows_eight_kernel<kWaves, Out::Scaled>, 8, kWaves);
+    };
     using std::integral_constant;
-    if (N >= 8192) by_kind(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    // sixteens of up to 2048 rows are at most 128 workgroups (4 x 2048 x 2048: 6.9 us in sixteens, 6.0 in eights)
+    if (N <= 2048 && k >= 8192) eight_by_kind(integral_constant<int, 16>{});
+    else if (N <= 2048) eight_by_kind(integral_constant<int, 8>{});
+    else if (N >= 8192) by_kind(integral_constant<int, 2>{}, integral_constant<int, 8>{});
     else if (k >= 8192) by_kind(integral_constant<int, 1>{}, integral_constant<int, 16>{});
     else by_kind(integral_constant<int, 1>{}, integral_constant<int, 8>{});
     return hipGetLastError();

@@ -1,0 +1,82 @@
+"""Attention of many query positions over binary16 keys and values (attention_prompt.hip): the row of Q and the weights go to
+the binary16 matrix cores as pairs, and where the rows are few two wavefronts share them. Sizes at the edges of tiles (32
+keys), steps (64) and workgroups (64 or 128 rows), against 64 bits, the float32 matrix cores and the kernel that takes a query row a workgroup."""
+import numpy as np
+import pytest
+
+from mimir_amd import capi
+from tests import test_gpu_decode_ops as T
+
+pytestmark = pytest.mark.gpu
+
+
+def both(q, k, v, scale, off):
+    l = T.gpu.lib()
+    got = T.attention(q, k, v, scale, causal=True, offset=off, kv_dt=capi.F16)
+    assert T.last_kernel() == "attn_prompt_kernel"
+    try:
+        capi.check(l.mi355x_tune(b"attention.prompt", 0))
+        return got, T.attention(q, k, v, scale, causal=True, offset=off, kv_dt=capi.F16)
+    finally:
+        capi.check(l.mi355x_tune(b"attention.prompt", 1))
+
+
+def exact(q, k, v, scale, off):
+    B, H, Q, D = q.shape
+    g = H // k.shape[1]
+    k64, v64 = (np.repeat(x.view(np.float16).astype(np.float64), g, axis=1) for x in (k, v))
+    s = np.matmul(q.astype(np.float64) * scale, k64.transpose(0, 1, 3, 2))
+    s[..., np.arange(k.shape[2])[None, :] > np.arange(Q)[:, None] + off] = -np.inf
+    w = np.exp(s - s.max(-1, keepdims=True))
+    return np.matmul(w, v64) / w.sum(-1, keepdims=True)
+
+
+@pytest.mark.parametrize("B,H,HK,Q,K,D,spread", [
+    (1, 4, 2, 64, 64, 128, 1),      # one step, one workgroup of two pairs
+    (1, 4, 2, 65, 97, 64, 1),       # a row into the next workgroup; the last step's second tile holds one key
+    (2, 4, 1, 96, 96, 128, 6),      # the last step is one tile: the second wavefront joins with fewer keys; scores far apart
+    (1, 4, 4, 130, 159, 128, 0.01),  # ragged; weights all alike
+    (4, 32, 8, 449, 70, 64, 1),     # workgroups of 128 rows; keys that end inside the third tile, most rows see all
+])
+def test_error_is_no_larger_than_with_float32_products(B, H, HK, Q, K, D, spread):
+    rng = np.random.default_rng(Q + K)
+    q = rng.normal(size=(B, H, Q, D)).astype(np.float32) * np.float32(spread)
+    q *= np.exp(2 * rng.normal(size=(B, H, 1, D))).astype(np.float32) if spread == 1 else np.float32(1)  # features of unlike size
+    k, v = (T.O.f32_to_f16(rng.normal(size=(B, HK, K, D)).astype(np.float32)) for _ in range(2))
+    k, v = k.view(np.uint16), v.view(np.uint16)
+    scale, off = 1 / np.sqrt(D), max(K - Q, 0)
+    T.gpu.say(f"attention in halves B={B} H={H} Q={Q} K={K} D={D} spread={spread}")
+    out, _ = T.attention(q, k, v, scale, causal=True, offset=off, kv_dt=capi.F16)
+    assert T.last_kernel() == "attn_prompt_kernel"
+    k32, v32 = (x.view(np.float16).astype(np.float32) for x in (k, v))
+    single, _ = T.attention(q, k32, v32, scale, causal=True, offset=off, kv_dt=capi.F32)
+    want = exact(q, k, v, scale, off)
+    err, ref = (np.sqrt(np.mean((x.astype(np.float64) - want) ** 2)) for x in (out, single))
+    # both are rounding errors of float32 sums of the same terms, in fewer steps here; the pairs' own error, 2^-39 of the largest
+    # element, is far below. The luck of the roundings differs: a quarter, and one rounding of the results
+    assert err <= 1.25 * ref + 2.0 ** -24 * np.sqrt(np.mean(want ** 2)), (err, ref)
+
+
+@pytest.mark.parametrize("B,Q,D", [(1, 100, 128), (1, 100, 64), (4, 449, 64)])
+def test_infinities_among_keys_and_queries(B, Q, D):
+    """A NaN or an infinity in a key, a value or a row of Q gives every result the class (NaN, infinity, finite) that products of float32 give it."""
+    rng = np.random.default_rng(Q)
+    H, HK, K = 32 if B > 1 else 4, 2, 100
+    q = rng.normal(size=(B, H, Q, D)).astype(np.float32)
+    k = rng.normal(size=(B, HK, K, D)).astype(np.float32); v = rng.normal(size=(B, HK, K, D)).astype(np.float32)
+    q[0, :, 40, 3] = 0.25; q[0, :, 40, 7] = 1e-20; q[0, :, 41, 7] = 0   # an exact binary16, one far below the row's largest, a zero
+    k[0, 0, 20, 7] = np.inf      # scores of either infinity by the sign of q's feature 7
+    k[0, 0, 50, 3] = -np.inf
+    k[0, 1, 70, 2] = np.nan
+    v[0, 1, 33, 5] = np.inf      # values seen whole from some row on and in part before
+    v[0, 1, 34, 6] = -np.inf
+    q[0, 0, 60, 9] = np.inf; q[0, 0, 60, 10] = 1e6
+    k, v = T.O.f32_to_f16(k), T.O.f32_to_f16(v)
+    T.gpu.say(f"attention in halves, infinities, B={B} Q={Q} D={D}")
+    (out, lse), (rows, lse_rows) = both(q, k, v, 1 / np.sqrt(D), 0)
+    assert np.isnan(rows).any() and np.isfinite(rows).any()
+    for got, want in ((out, rows), (lse, lse_rows)):
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+        T.close(got[fin], want[fin])

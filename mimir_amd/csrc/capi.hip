@@ -254,9 +254,9 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             }
             if (g_tune_q4[4] != 2 && M >= g_fx_min_rows && (g_fx_min_rows != 16 ? mimir::qgemm_q4_0_fx_ok(W, M, N, K) : mimir::qgemm_q4_0_fx_pays(W, M, N, K)) &&
                 ((uintptr_t)x & 15) == 0 && x_row_stride % 4 == 0) {
-                // many rows: the same fixed-point arithmetic on the int8 matrix cores
+                // many rows: the fixed-point arithmetic on the int8 matrix cores
                 void* act;
-                // from some hundreds of rows on as pairs of 12-bit digits on the binary16 matrix cores, which want a
+                // from some hundreds of rows on as pairs of binary16 numbers on the binary16 matrix cores, which want a
                 // workspace behind the activations (not from a fixed scratch, which is too small for it)
                 const bool pairs = !src.fixed && mimir::qgemm_q4_0_fx16_pays(M, N, K);
                 const size_t act_bytes = ((pairs ? mimir::q4_0_fx16_act_bytes(M, K) : mimir::q4_0_fx_act_bytes(K) * (size_t)M) + 255) / 256 * 256;

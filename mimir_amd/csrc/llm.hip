@@ -35,7 +35,7 @@ namespace {
 #define LLM_HIP(expr, what) DECODER_HIP(expr, "llama", what)
 
 // The form of converted activations a weight's product reads.
-// kActFx: Q4_0 by many rows of x, on the int8 matrix cores; kActFxPairs: the same product through the binary16 ones
+// kActFx: Q4_0 by many rows of x, on the int8 matrix cores; kActFxPairs: on the binary16 ones, x as pairs of binary16 numbers
 enum ActClass { kActNone = 0, kActQ4 = 1, kActQ8 = 2, kActKQ = 3, kActFx = 4, kActFxPairs = 5, kActClasses = 6 };
 
 // qkv and gate_up: where q, k, v (gate, up) share a block dtype, finalize also keeps their rows in one
@@ -62,7 +62,7 @@ struct Model : Decoder {
 
     // activations of up to max_rows rows (batch x tokens of one call)
     DevBuf x, h, q, k, v, a, o, gate, up, s, xlast, hlast, act[kActClasses], act2;
-    DevBuf fx_panel;  // the workspace of the fixed-point Q4_0 product of a prompt's rows in its binary16 form: the largest matrix's
+    DevBuf fx_panel;  // the workspace of the Q4_0 products of a prompt's rows on the binary16 matrix cores: the largest product's
 
     // `fast` says the blocks qualify for the step of fused launches (Q4_0 linears that the fixed-point kernel takes).
     bool fast = false;

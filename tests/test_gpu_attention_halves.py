@@ -80,3 +80,14 @@ def test_infinities_among_keys_and_queries(B, Q, D):
         assert np.array_equal(np.isnan(got), np.isnan(want))
         assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
         T.close(got[fin], want[fin])
+
+
+def test_rows_that_see_no_key():
+    """The first 40 rows see no key: zeros and -Inf, also where the second wavefront of a pair has no tile at all."""
+    rng = np.random.default_rng(3)
+    q = rng.normal(size=(1, 4, 130, 128)).astype(np.float32)
+    k, v = (T.O.f32_to_f16(rng.normal(size=(1, 2, 100, 128)).astype(np.float32)) for _ in range(2))
+    T.gpu.say("attention in halves, rows without keys")
+    (out, lse), (rows, lse_rows) = both(q, k, v, 0.1, -40)
+    assert not out[:, :, :40].any() and np.all(lse[:, :, :40] == -np.inf)
+    T.close(out, rows); T.close(lse[:, :, 40:], lse_rows[:, :, 40:])

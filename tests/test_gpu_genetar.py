@@ -259,6 +259,20 @@ def test_large_prompt_tiles(tmp_path, dtype):
     assert X.error(got, one) < TOL[dtype]
 
 
+@pytest.mark.parametrize("batch,width,ff", [(2, 72, 8200), (8, 200, 8192), (3, 136, 70), (5, 2048, 320), (4, 2056, 64)])
+def test_few_rows_by_few_rows_of_weights(tmp_path, batch, width, ff):
+    """Decoding products of two to eight rows by up to 2048 rows of W, eight of them a workgroup: long rows (sixteen wavefronts) and short
+    ones (some wavefronts without a piece of K), a last workgroup of fewer rows, the widest, and the first that takes sixteen."""
+    c = X.config([X.rotary(ff=ff)], width=width, vocab=90)
+    w = X.weights(c, 4)
+    toks = X.tokens(c, 6, 3, batch=batch)
+    gpu.say(f"genetar few rows, batch {batch} width {width} ff {ff}")
+    m = load(tmp_path, c, w, context=8, batch=batch, dtype="bfloat16")
+    got = np.stack([m.logits(toks[:, t:t + 1]) for t in range(6)], 1)
+    want = np.stack([G.forward(c, w, t) for t in toks])
+    assert X.error(got, want) < TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("swiglu", [False, True], ids=["relu2", "swiglu"])
 @pytest.mark.parametrize("bare", [False, True], ids=["posts", "bare"])

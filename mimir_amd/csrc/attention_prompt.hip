@@ -1,11 +1,10 @@
-// Attention for many query positions at once (a prompt) on the matrix cores of gfx950: the semantics of
+// Attention for many query positions at once (a prompt) on the float32 matrix cores of gfx950: the semantics of
 // attention.hip (softmax(scale * q.k^T) . v per query row, the query scaled first, p = exp(s - max), the result
 // (sum p v) * (1 / sum p), the logsumexp max + log(sum p), a row that sees no key zeros and -Inf, key j hidden from
 // query i when causal and j > i + causal_offset; backend/cpu/attention.go:268-292, 437-535), for the calls that kernel
 // serves one query row a workgroup, re-reading every key and value for every row.
 //
-// Two kernels: one for float32 keys and values, described here, and one for binary16, described where it stands.
-// A wavefront owns 32 query rows of one head and walks the keys in tiles of 32 with a running maximum and sum per
+// Here a wavefront owns 32 query rows of one head and walks the keys in tiles of 32 with a running maximum and sum per
 // row (a row's result is rescaled when its maximum grows), and both products of a tile are MFMAs on float32 operands
 // (v_mfma_f32_32x32x2_f32), so that nothing is rounded that the other kernel does not round. Both are computed
 // transposed, so that everything a row owns lives in one lane (and its partner 32 lanes on): scores^T = K . Q^T over the
@@ -15,8 +14,8 @@
 // result^T = V^T . P^T over the tile's keys, taken in the order the scores' registers hold them, so that p goes from the
 // exponential straight into the MFMA's second operand, and the lane ends with 16 features of every 32 of its row. A
 // workgroup is four wavefronts with consecutive rows of one head, which share the tile of keys and values in LDS
-// (the next tile's rows requested while this one is used; K's rows padded by a float so that 32 keys' equal feature falls
-// on 32 banks).
+// (converted to float32 as they are loaded, the next tile's rows requested while this one is used; K's rows padded by a
+// float so that 32 keys' equal feature falls on 32 banks).
 //
 // What differs from the other kernel is the order of the float32 sums (features and keys in pairs as the MFMA takes
 // them, keys in tiles of 32 with rescaling), so results agree to float32 rounding, not bit for bit.
@@ -28,10 +27,9 @@ namespace mimir {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kRows = 32;       // query rows a wavefront
-// wavefronts a workgroup (WAVES below, float32): four, 128 consecutive rows of one head, or two where four would leave the device short of workgroups
+// wavefronts a workgroup (WAVES below): four, 128 consecutive rows of one head, or two where four would leave the device short of workgroups
 constexpr int kTile = 32;       // keys a tile
 
 struct PromptParams {
@@ -42,15 +40,22 @@ struct PromptParams {
     int64_t causal_offset;
 };
 
+// Element e of a row part held as raw 32-bit words.
+template <typename KV>
+__device__ __forceinline__ float element(const uint32_t* raw, int e);
+template <>
+__device__ __forceinline__ float element<float>(const uint32_t* raw, int e) { return __builtin_bit_cast(float, raw[e]); }
+template <>
+__device__ __forceinline__ float element<uint16_t>(const uint32_t* raw, int e) { return f16_bits_to_f32((uint16_t)(raw[e >> 1] >> (16 * (e & 1)))); }
+
 // The other half's value: lane ^ 32.
 __device__ __forceinline__ float other_half(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, v)));
 }
 
-template <int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                                                  const float* __restrict__ v, float* __restrict__ out,
-                                                                                                  float* __restrict__ lse, PromptParams p) {
+template <typename KV, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const KV* __restrict__ k, const KV* __restrict__ v,
+                                                                     float* __restrict__ out, float* __restrict__ lse, PromptParams p) {
     constexpr int KS = D + 1;            // floats between rows of the keys' tile
     constexpr int NT = D / 32;           // 32-feature tiles of the result
     constexpr int PER = D / 8;           // elements of a key (value) row a thread loads: eight threads a row
@@ -97,10 +102,10 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void 
 
     // a thread's part of a tile's keys and values: rows tid / 8 + RP n, elements [PER (tid % 8), + PER)
     const int lrow = tid >> 3, lpart = tid & 7;
-    const float* kbase = k + b * p.k_b + (int64_t)hk * p.k_h + PER * lpart;
-    const float* vbase = v + b * p.v_b + (int64_t)hk * p.v_h + PER * lpart;
-    constexpr int VEC = PER / 4;  // 16-byte pieces of a thread's part (the host checks their alignment)
-    float kreg[NP][PER], vreg[NP][PER];
+    const KV* kbase = k + b * p.k_b + (int64_t)hk * p.k_h + PER * lpart;
+    const KV* vbase = v + b * p.v_b + (int64_t)hk * p.v_h + PER * lpart;
+    constexpr int VEC = PER * (int)sizeof(KV) / 16;  // 16-byte pieces of a thread's part (the host checks their alignment)
+    uint32_t kreg[NP][4 * VEC], vreg[NP][4 * VEC];
     auto fetch = [&](int j0) {
 #pragma unroll
         for (int n = 0; n < NP; n++) {
@@ -108,7 +113,7 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void 
             j = j < Kt ? j : Kt - 1;  // rows past the last key: never seen, loaded from the last one
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
-                const f32x4 kw = ((const f32x4*)(kbase + j * p.k_p))[c], vw = ((const f32x4*)(vbase + j * p.v_p))[c];
+                const u32x4 kw = ((const u32x4*)(kbase + j * p.k_p))[c], vw = ((const u32x4*)(vbase + j * p.v_p))[c];
 #pragma unroll
                 for (int w = 0; w < 4; w++) kreg[n][4 * c + w] = kw[w], vreg[n][4 * c + w] = vw[w];
             }
@@ -120,10 +125,10 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void 
         for (int n = 0; n < NP; n++) {
             const int r = lrow + RP * n;
 #pragma unroll
-            for (int e = 0; e < PER; e++) ks[r * KS + PER * lpart + e] = kreg[n][e];
+            for (int e = 0; e < PER; e++) ks[r * KS + PER * lpart + e] = element<KV>(kreg[n], e);
 #pragma unroll
             for (int e = 0; e < PER; e += 4) {
-                const f32x4 f = {vreg[n][e], vreg[n][e + 1], vreg[n][e + 2], vreg[n][e + 3]};
+                const f32x4 f = {element<KV>(vreg[n], e), element<KV>(vreg[n], e + 1), element<KV>(vreg[n], e + 2), element<KV>(vreg[n], e + 3)};
                 *(f32x4*)(vs + r * D + PER * lpart + e) = f;
 #pragma unroll
                 for (int c = 0; c < 4; c++) chk = __builtin_fmaf(f[c], 0.f, chk);
@@ -235,326 +240,15 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void 
     if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
 }
 
-// The same for keys and values in binary16, which a matrix core takes as they are: only the float32 operands, the row of Q and the
-// weights, are brought to it, each as a pair of binary16 numbers, a 2^-e = a0 + a1 with a0 the binary16 next to it and a1 the one
-// next to what that leaves. e makes a row's largest element of Q lie in [2^14, 2^15), and is -14 for the weights, which are at
-// most 1: an element keeps 22 bits down to 2^-17 of the largest and is held to 2^-39 of it, far below the rounding of the
-// float32 sums that both products of a pair go into. v_mfma_f32_32x32x16_f16 multiplies sixteen times as fast as the float32
-// instruction: 1024 cycles a tile of 32 rows by 32 keys at 128 features where that one takes 8192. Against 64 bits the
-// results' error is 0.55 of what it was with float32 operands (2.0e-7 for 3.4e-7 over 512 normal keys, 6.0e-7 for 1.08e-6 with scores six times as far apart).
-//
-// LDS holds a tile's keys row by row, sixteen-byte pieces turned by the row so that 32 rows' equal piece falls on all banks, and its values
-// transposed, a feature's 32 keys in the order in which a lane holds its scores (keys 16 u + 8 a + 4 hi + c at 16 u + 8 hi +
-// 4 a + c), so that a lane's weights go from the exponential into the second operand; two neighbouring keys' values
-// meet in one dword on the way in.
-//
-// What bounds it is a wavefront's chain: some 600 vector instructions a tile (exponentials, masks, pairs, staging: 2400 cycles) and the
-// MFMAs' 1024, 2.7 us with one wavefront a SIMD, and a causal call ends with the rows that walk all keys. So a workgroup is four
-// wavefronts of 32 rows each only where there are many (KS = 1), and otherwise (KS = 2) two pairs of wavefronts, 32 rows a pair, that
-// take a step's two tiles of keys, one each, and join their maxima, sums and results through LDS at the end: half the chain.
-// One layer of 32 heads of 128 features over 8 key heads, us:
-//   rows, keys            float32 operands   KS = 1   KS = 2
-//   512                         90.3           49.1     37.9
-//   2048                       455            186      190
-//   5 prompts of 131            36.9           26.7     25.1
-//   8 prompts of 512           216            108      153
-//   8 heads, 512 of 2048       331            163      110
-
-// e^x for x <= 0, and for NaN: 2^t with t the float32 next to x / ln 2, times 1 + ln 2 (x / ln 2 - t). Nine instructions where
-// the general function, which has overflow and subnormal results to care for, takes fifteen; a result below 2^-126 is zero here.
-__device__ __forceinline__ float exp_down(float x) {
-    constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = (float)(1.4426950408889634074 - (double)kLog2e), kLn2 = 0.6931471805599453f;
-    const float t = x * kLog2e, y = __builtin_amdgcn_exp2f(t);
-    const float held = fmaxf(x, -128.f), th = held * kLog2e;  // an infinity leaves nothing to mend
-    const float rest = __builtin_fmaf(held, kLog2eLow, __builtin_fmaf(held, kLog2e, -th));
-    return __builtin_fmaf(y, rest * kLn2, y);
-}
-
-template <int D, int KS>
-__global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                                                         float* __restrict__ out, float* __restrict__ lse, PromptParams p) {
-    constexpr int NT = D / 32;                 // 32-feature tiles of the result
-    constexpr int NS = D / 16;                 // steps of the scores' product
-    constexpr int PER = D / 8, PD = PER / 2;   // elements, dwords of a key (value) row a thread loads: eight threads a row, a row of each tile
-    constexpr int G = 4 / KS;                  // groups of 32 query rows a workgroup
-    constexpr int kStep = kTile * KS;          // keys a step
-    constexpr float kUp = 16384.f;
-    __shared__ __align__(16) uint16_t kv[2][KS][kTile * D];  // the step's keys, its values
-    __shared__ int vbad[2], kbad[2];           // whether a step's values, keys hold a NaN or an infinity, for steps of either parity
-    __shared__ float ml[KS > 1 ? G : 1][2][64];  // maximum and sum of the rows' second half of the keys
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, hi = lane >> 5, part = wave % KS;
-    const int b = blockIdx.y, h = blockIdx.x, hk = h / (p.H / p.HK), bx = (int)(gridDim.z - 1 - blockIdx.z);  // the last rows first
-    const int i0 = (bx * G + wave / KS) * kRows;
-    const int64_t Kt = p.K;
-    auto seen_of = [&](int i) -> int {  // keys row i sees
-        int64_t s = Kt;
-        if (p.causal) {
-            s = (int64_t)i + p.causal_offset + 1;
-            s = s < 0 ? 0 : s > Kt ? Kt : s;
-        }
-        return (int)s;
-    };
-    const int last_row_wg = (bx + 1) * G * kRows - 1 < p.Q ? (bx + 1) * G * kRows - 1 : p.Q - 1;
-    const int last_row_wave = i0 + kRows - 1 < p.Q ? i0 + kRows - 1 : p.Q - 1;
-    const int seen_wg = p.causal ? seen_of(last_row_wg) : (int)Kt;
-    const int seen_wave = i0 < p.Q ? (p.causal ? seen_of(last_row_wave) : (int)Kt) : 0;
-    const int seen_first = i0 < p.Q ? seen_of(i0) : 0;  // the fewest keys a row of this wavefront sees
-    const int row = i0 + r32;
-    const int seen = row < p.Q ? seen_of(row) : 0;
-
-    // this lane's row, scaled: features 16 s + 8 hi .. + 8 of step s as the second operand's pair
-    f16x8 q0[NS], q1[NS];
-    int e_row = 0;
-    auto load_row = [&]() {
-        const int i = row < p.Q ? row : p.Q - 1;
-        const float* qr = q + b * p.q_b + (int64_t)h * p.q_h + (int64_t)i * p.q_i + 8 * hi;
-        float amax = 0.f;
-#pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const float x = __builtin_fabsf(qr[16 * s + c] * p.scale);
-                amax = fmaxf(amax, x < __builtin_inff() ? x : 0.f);
-            }
-        amax = fmaxf(amax, other_half(amax, lane));
-        e_row = amax > 0.f ? __builtin_amdgcn_frexp_expf(amax) - 15 : 0;
-#pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const float x = qr[16 * s + c] * p.scale, a = __builtin_ldexpf(x, -e_row);
-                q0[s][c] = (_Float16)a;
-                if (x != 0.f && q0[s][c] == (_Float16)0.f) q0[s][c] = (_Float16)__builtin_copysignf(0x1p-24f, x);  // times an infinity it is one
-                q1[s][c] = (_Float16)(__builtin_fabsf(a) < __builtin_inff() ? a - (float)q0[s][c] : 0.f);  // an infinity's product is q0's alone
-            }
-    };
-    load_row();
-    float m = -__builtin_inff(), l = 0.f;  // the row's maximum so far; the sum over the keys this half of the lanes holds
-    f32x16 o[NT], zero;                    // 2^14 times the row's result, transposed: register e of tile t is feature 32 t + 8 (e / 4) + 4 hi + e % 4
-#pragma unroll
-    for (int e = 0; e < 16; e++) zero[e] = 0.f;
-#pragma unroll
-    for (int t = 0; t < NT; t++) o[t] = zero;
-
-    // a thread's part of a tile's keys and values: rows tid / 8 + 32 n, elements [PER (tid % 8), + PER)
-    const int lrow = tid >> 3, lpart = tid & 7;
-    const uint16_t* kbase = k + b * p.k_b + (int64_t)hk * p.k_h + PER * lpart;
-    const uint16_t* vbase = v + b * p.v_b + (int64_t)hk * p.v_h + PER * lpart;
-    u32x4 kreg[KS][PD / 4], vreg[KS][PD / 4];
-    auto fetch = [&](int j0) {
-#pragma unroll
-        for (int n = 0; n < KS; n++) {
-            int64_t j = j0 + lrow + kTile * n;
-            j = j < Kt ? j : Kt - 1;  // rows past the last key: never seen, loaded from the last one
-#pragma unroll
-            for (int c = 0; c < PD / 4; c++) {
-                kreg[n][c] = ((const u32x4*)(kbase + j * p.k_p))[c];
-                vreg[n][c] = ((const u32x4*)(vbase + j * p.v_p))[c];
-            }
-        }
-    };
-    auto key_piece = [](int r, int piece) { return D == 128 ? piece ^ (r & 15) : piece ^ ((r >> 1) & 7); };
-    auto value_at = [](int f, int slot) { return f * kTile + ((((slot >> 3) ^ ((f >> 2) & 3)) << 3) | (slot & 7)); };
-    auto slot_of = [](int key) { return (key & 16) | (key & 4) << 1 | (key & 8) >> 1 | (key & 3); };
-    auto stage = [&](int parity) {
-        const f16x2 none = {(_Float16)0.f, (_Float16)0.f};
-        f16x2 chk = none, chk_k = none;  // 0 * value summed: NaN as soon as a value is a NaN or an infinity
-#pragma unroll
-        for (int n = 0; n < KS; n++) {
-            uint16_t *ks = kv[0][n], *vt = kv[1][n];
-            const int r = lrow;
-#pragma unroll
-            for (int c = 0; c < PD / 4; c++) *(u32x4*)(ks + r * D + key_piece(r, lpart * (PD / 4) + c) * 8) = kreg[n][c];
-            // the thread eight lanes on has the neighbouring key's same features: of two features, the even key's thread stores the first's two keys
-            const int odd = r & 1, slot = slot_of(r & ~1);
-#pragma unroll
-            for (int w = 0; w < PD; w++) {
-                const uint32_t mine = vreg[n][w >> 2][w & 3];
-                const uint32_t theirs = __builtin_bit_cast(uint32_t, dpp_f32<0x128>(__builtin_bit_cast(float, mine)));  // row_ror:8
-                const uint32_t two = odd ? __builtin_amdgcn_perm(mine, theirs, 0x07060302u) : __builtin_amdgcn_perm(theirs, mine, 0x05040100u);
-                *(uint32_t*)(vt + value_at(PER * lpart + 2 * w + odd, slot)) = two;
-                chk = __builtin_bit_cast(f16x2, mine) * none + chk;
-                const uint32_t key = kreg[n][w >> 2][w & 3];
-                chk_k = __builtin_bit_cast(f16x2, key) * none + chk_k;
-            }
-        }
-        const float bad = (float)chk[0] + (float)chk[1];
-        if (__builtin_amdgcn_ballot_w64(bad != bad) != 0 && lane == 0) vbad[parity] = 1;
-        const float bad_k = (float)chk_k[0] + (float)chk_k[1];
-        if (__builtin_amdgcn_ballot_w64(bad_k != bad_k) != 0 && lane == 0) kbad[parity] = 1;
-    };
-
-    // A tile with a NaN or an infinity among its values takes the vector units for its second product, key by key and only for the
-    // rows that see the key, as in the kernel above; here also where every row sees it, since an infinity times a pair is an
-    // infinity only if its parts' signs agree. Of a score with a NaN or an infinity among its key the first part alone counts.
-    if (tid < 2) vbad[tid] = kbad[tid] = 0;
-    const uint16_t *ks = kv[0][part], *vt = kv[1][part];
-    if (seen_wg > 0) fetch(0);
-    for (int jw = 0; jw < seen_wg; jw += kStep) {
-        const int parity = (jw / kStep) & 1, j0 = jw + kTile * part;
-        __syncthreads();  // everyone has read the tiles before
-        stage(parity);
-        __syncthreads();
-        if (tid == 0) vbad[parity ^ 1] = kbad[parity ^ 1] = 0;  // read last before the first barrier above, set next behind it a step on
-        if (jw + kStep < seen_wg) fetch(jw + kStep);
-        if (j0 >= seen_wave) continue;  // nothing of this tile is seen by this wavefront's rows (uniform)
-        const bool whole = j0 + kTile <= seen_first;
-        const bool by_key = vbad[parity] != 0;
-
-        // scores, transposed (K . Q^T): register e is key j0 + 8 (e / 4) + 4 hi + e % 4 against this lane's row
-        f32x16 s = zero;
-        int k0 = r32 * D + key_piece(r32, hi) * 8;
-        asm volatile("" : "+v"(k0));  // eight addresses worked out again for each tile instead of eight registers
-#pragma unroll
-        for (int f = 0; f < NS; f++) {
-            const f16x8 kf = *(const f16x8*)(ks + (k0 ^ 16 * f));
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q0[f], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q1[f], s, 0, 0, 0);
-        }
-        if (kbad[parity] != 0) {
-            f32x16 first = zero;
-#pragma unroll
-            for (int f = 0; f < NS; f++) first = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const f16x8*)(ks + (k0 ^ 16 * f)), q0[f], first, 0, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 16; e++) s[e] = __builtin_fabsf(first[e]) < __builtin_inff() ? s[e] : first[e];
-        }
-        float mx = -__builtin_inff();
-#pragma unroll
-        for (int e = 0; e < 16; e++) s[e] = __builtin_ldexpf(s[e], e_row);
-        if (!whole) {
-#pragma unroll
-            for (int e = 0; e < 16; e++) s[e] = 8 * (e >> 2) + (e & 3) < seen - j0 - 4 * hi ? s[e] : -__builtin_inff();
-        }
-#pragma unroll
-        for (int e = 0; e < 16; e++) mx = fmaxf(mx, s[e]);
-        mx = fmaxf(mx, other_half(mx, lane));
-        const float mn = fmaxf(m, mx);
-        float al = 1.f, sum = 0.f;
-        if (mn > -__builtin_inff()) {  // the row has seen a key by now
-            al = exp_down(m - mn);
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                s[e] = exp_down(s[e] - mn);
-                sum += s[e];
-            }
-        } else {
-            s = zero;
-        }
-        l = l * al + sum;
-        m = mn;
-        if (__builtin_amdgcn_ballot_w64(al != 1.f) != 0) {
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * al;
-        }
-        if (!by_key) {
-            f16x8 p0[2], p1[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    p0[u][c] = (_Float16)__builtin_fmaf(s[8 * u + c], kUp, 0.f);
-                    p1[u][c] = (_Float16)__builtin_fmaf(s[8 * u + c], kUp, -(float)p0[u][c]);
-                }
-#pragma unroll
-            for (int t = 0; t < NT; t++) {
-                f16x8 vf[2];
-#pragma unroll
-                for (int u = 0; u < 2; u++) vf[u] = *(const f16x8*)(vt + value_at(32 * t + r32, 16 * u + 8 * hi));
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], p0[u], o[t], 0, 0, 0);
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[u], p1[u], o[t], 0, 0, 0);
-                }
-            }
-        } else {
-#pragma unroll 1
-            for (int e = 0; e < 16; e++) {  // one body for all keys, whose weights come past register 0: unrolled, it took registers from the path above
-                const float mine = s[0] * kUp, theirs = other_half(mine, lane);
-#pragma unroll
-                for (int i = 0; i < 15; i++) s[i] = s[i + 1];
-#pragma unroll
-                for (int half = 0; half < 2; half++) {  // the key that register e holds in the lanes of this half
-                    const int key = 8 * (e >> 2) + 4 * half + (e & 3);
-                    const float pk = hi == half ? mine : theirs;
-                    const bool sees = j0 + key < seen;
-                    const int at = value_at(4 * hi, slot_of(key));  // this lane's first feature; eight on, the pieces are turned by two
-#pragma unroll
-                    for (int t = 0; t < NT; t++) {
-#pragma unroll
-                        for (int g = 0; g < 16; g++) {
-                            const float vv = f16_bits_to_f32(vt[(at ^ (g & 4) << 2) + (32 * t + 8 * (g >> 2) + (g & 3)) * kTile]);
-                            o[t][g] = __builtin_fmaf(pk, sees ? vv : 0.f, o[t][g]);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-            }
-        }
-    }
-
-    l += other_half(l, lane);
-    if (KS > 1) {  // the second wavefront's half of the keys joins the first's
-        float* theirs = (float*)kv + (wave / KS) * (16 * NT * 64) + lane;
-        __syncthreads();
-        if (part == 1) {
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) theirs[64 * (16 * t + e)] = o[t][e];
-            ml[wave / KS][0][lane] = m;
-            ml[wave / KS][1][lane] = l;
-        }
-        __syncthreads();
-        if (part == 1) return;
-        const float m1 = ml[wave / KS][0][lane], l1 = ml[wave / KS][1][lane], mn = fmaxf(m, m1);
-        const float a0 = m == mn ? 1.f : exp_down(m - mn), a1 = m1 == mn ? 1.f : exp_down(m1 - mn);
-        l = l * a0 + l1 * a1;
-        m = mn;
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * a0 + theirs[64 * (16 * t + e)] * a1;
-    }
-    if (row >= p.Q) return;
-    float* orow = out + b * p.o_b + (int64_t)h * p.o_h + (int64_t)row * p.o_i;
-    const float inv = l == 0.f ? 0.f : 1.0f / l;
-    const bool wide = (((uintptr_t)orow) & 15) == 0;
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            f32x4 r;
-#pragma unroll
-            for (int c = 0; c < 4; c++) r[c] = l == 0.f ? 0.f : o[t][4 * g + c] * (1.f / kUp) * inv;
-            float* dst = orow + 32 * t + 8 * g + 4 * hi;
-            if (wide) *(f32x4*)dst = r;
-            else
-#pragma unroll
-                for (int c = 0; c < 4; c++) dst[c] = r[c];
-        }
-    if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
-}
-
 std::atomic<int> g_prompt{1};  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup
 
-template <int WAVES>
-hipError_t launch_f32(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
-    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + WAVES * kRows - 1) / (WAVES * kRows))), block(64 * WAVES);
-    const float *k = (const float*)a.k, *v = (const float*)a.v;
-    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_kernel<128, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
-    else hipLaunchKernelGGL((attn_prompt_kernel<64, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
-    return hipGetLastError();
-}
-
-template <int KS>
-hipError_t launch_f16(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
-    constexpr int kWg = 4 / KS * kRows;
-    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + kWg - 1) / kWg)), block(256);
-    const uint16_t *k = (const uint16_t*)a.k, *v = (const uint16_t*)a.v;
-    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_half_kernel<128, KS>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
-    else hipLaunchKernelGGL((attn_prompt_half_kernel<64, KS>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+template <typename KV, int WAVES>
+hipError_t launch(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
+    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + WAVES * kRows - 1) / (WAVES * kRows)));
+    if (a.D == 128)
+        hipLaunchKernelGGL((attn_prompt_kernel<KV, 128, WAVES>), grid, dim3(64 * WAVES), 0, st, a.q, (const KV*)a.k, (const KV*)a.v, a.out, a.lse, p);
+    else
+        hipLaunchKernelGGL((attn_prompt_kernel<KV, 64, WAVES>), grid, dim3(64 * WAVES), 0, st, a.q, (const KV*)a.k, (const KV*)a.v, a.out, a.lse, p);
     return hipGetLastError();
 }
 
@@ -585,12 +279,11 @@ hipError_t attention_prompt(const AttnArgs& a, hipStream_t st) {
     p.scale = (float)a.scale;
     p.causal = a.causal;
     p.causal_offset = a.causal_offset;
-    // where workgroups of 128 rows would be fewer than the device holds at two a compute unit: two wavefronts a workgroup (float32), or
-    // two wavefronts on the same rows (binary16; at 512 workgroups the two are level, see the figures there)
-    const bool few = a.B * a.H * ((a.Q + 4 * kRows - 1) / (4 * kRows)) < 512;
+    // workgroups of two wavefronts where those of four would be fewer than the device holds at two a compute unit
+    const bool two = a.B * a.H * ((a.Q + 4 * kRows - 1) / (4 * kRows)) < 512;
     note_kernel("attn_prompt_kernel");
-    if (a.kv_dtype == kF16) return few ? launch_f16<2>(a, p, st) : launch_f16<1>(a, p, st);
-    return few ? launch_f32<2>(a, p, st) : launch_f32<4>(a, p, st);
+    if (a.kv_dtype == kF16) return two ? launch<uint16_t, 2>(a, p, st) : launch<uint16_t, 4>(a, p, st);
+    return two ? launch<float, 2>(a, p, st) : launch<float, 4>(a, p, st);
 }
 
 }  // namespace mimir

@@ -1,6 +1,6 @@
-"""Attention of many query positions over binary16 keys and values (attention_prompt.hip): the row of Q and the weights go to
-the binary16 matrix cores as pairs, and where the rows are few two wavefronts share them. Sizes at the edges of tiles (32
-keys), steps (64) and workgroups (64 or 128 rows), against 64 bits, the float32 matrix cores and the kernel that takes a query row a workgroup."""
+"""Attention of many query positions over binary16 keys and values (attention_prompt.hip): they enter products of float32 operands as they
+are, so that results are as near 64 bits as over float32 caches, whatever the sizes of weights, values and features. Sizes at the edges of tiles (32
+keys) and workgroups (64 or 128 rows), against 64 bits, the float32 cache and the kernel that takes a query row a workgroup."""
 import numpy as np
 import pytest
 
@@ -45,15 +45,14 @@ def test_error_is_no_larger_than_with_float32_products(B, H, HK, Q, K, D, spread
     k, v = (T.O.f32_to_f16(rng.normal(size=(B, HK, K, D)).astype(np.float32)) for _ in range(2))
     k, v = k.view(np.uint16), v.view(np.uint16)
     scale, off = 1 / np.sqrt(D), max(K - Q, 0)
-    T.gpu.say(f"attention in halves B={B} H={H} Q={Q} K={K} D={D} spread={spread}")
+    T.gpu.say(f"attention over binary16 B={B} H={H} Q={Q} K={K} D={D} spread={spread}")
     out, _ = T.attention(q, k, v, scale, causal=True, offset=off, kv_dt=capi.F16)
     assert T.last_kernel() == "attn_prompt_kernel"
     k32, v32 = (x.view(np.float16).astype(np.float32) for x in (k, v))
     single, _ = T.attention(q, k32, v32, scale, causal=True, offset=off, kv_dt=capi.F32)
     want = exact(q, k, v, scale, off)
     err, ref = (np.sqrt(np.mean((x.astype(np.float64) - want) ** 2)) for x in (out, single))
-    # both are rounding errors of float32 sums of the same terms, in fewer steps here; the pairs' own error, 2^-39 of the largest
-    # element, is far below. The luck of the roundings differs: a quarter, and one rounding of the results
+    # both are rounding errors of float32 sums of the same terms. The luck of the roundings may differ: a quarter, and one rounding of the results
     assert err <= 1.25 * ref + 2.0 ** -24 * np.sqrt(np.mean(want ** 2)), (err, ref)
 
 
@@ -72,7 +71,7 @@ def test_infinities_among_keys_and_queries(B, Q, D):
     v[0, 1, 34, 6] = -np.inf
     q[0, 0, 60, 9] = np.inf; q[0, 0, 60, 10] = 1e6
     k, v = T.O.f32_to_f16(k), T.O.f32_to_f16(v)
-    T.gpu.say(f"attention in halves, infinities, B={B} Q={Q} D={D}")
+    T.gpu.say(f"attention over binary16, infinities, B={B} Q={Q} D={D}")
     (out, lse), (rows, lse_rows) = both(q, k, v, 1 / np.sqrt(D), 0)
     assert np.isnan(rows).any() and np.isfinite(rows).any()
     for got, want in ((out, rows), (lse, lse_rows)):
@@ -83,11 +82,44 @@ def test_infinities_among_keys_and_queries(B, Q, D):
 
 
 def test_rows_that_see_no_key():
-    """The first 40 rows see no key: zeros and -Inf, also where the second wavefront of a pair has no tile at all."""
+    """The first 40 rows see no key: zeros and -Inf."""
     rng = np.random.default_rng(3)
     q = rng.normal(size=(1, 4, 130, 128)).astype(np.float32)
     k, v = (T.O.f32_to_f16(rng.normal(size=(1, 2, 100, 128)).astype(np.float32)) for _ in range(2))
-    T.gpu.say("attention in halves, rows without keys")
+    T.gpu.say("attention over binary16, rows without keys")
     (out, lse), (rows, lse_rows) = both(q, k, v, 0.1, -40)
     assert not out[:, :, :40].any() and np.all(lse[:, :, :40] == -np.inf)
     T.close(out, rows); T.close(lse[:, :, 40:], lse_rows[:, :, 40:])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_small_weights_on_large_values(D):
+    """The key of weight 1 has values of zero, the others of weights e^-8 down to e^-20 have large ones: every weight counts with its own 24 bits.
+    Their relative error is the exponential's, a few 2^-24, and the argument's rounding, 20 x 2^-24: below 3e-6 in all."""
+    rng = np.random.default_rng(5)
+    q = np.zeros((1, 1, 64, D), np.float32); q[0, 0, :, 0] = np.linspace(8, 20, 64)
+    k = np.zeros((1, 1, 64, D), np.float32); k[0, 0, 0, 0] = 1
+    v = rng.normal(size=(1, 1, 64, D)).astype(np.float32) * 1000; v[0, 0, 0] = 0
+    check_rows(q, k, v, 3e-6)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_small_features_of_q_by_large_keys(D):
+    """Q's largest feature meets keys of zero, and one 2^-26 of it keys of 2^14: the scores (up to about 3) come from the small one,
+    to float32's accuracy, and with them the weights: a few 2^-24 times 3."""
+    rng = np.random.default_rng(6)
+    q = rng.normal(size=(1, 1, 64, D)).astype(np.float32)
+    q[..., 0] = 2.0 ** 11; q[..., 1] *= np.float32(2.0 ** -15)
+    k = np.zeros((1, 1, 64, D), np.float32); k[..., 1] = rng.normal(size=64) * 2.0 ** 14
+    check_rows(q, k, rng.normal(size=(1, 1, 64, D)).astype(np.float32), 2e-6)
+
+
+def check_rows(q, k, v, bound):
+    """Every row within `bound` of its root mean square of the same in 64 bits."""
+    k, v = T.O.f32_to_f16(k).view(np.uint16), T.O.f32_to_f16(v).view(np.uint16)
+    T.gpu.say(f"attention over binary16, unlike sizes, D={q.shape[3]}")
+    got, _ = T.attention(q, k, v, 1.0, causal=False, kv_dt=capi.F16)
+    assert T.last_kernel() == "attn_prompt_kernel"
+    want = exact(q, k, v, 1.0, k.shape[2])  # an offset that hides no key
+    err = np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1))
+    assert err.max() <= bound, err.max()

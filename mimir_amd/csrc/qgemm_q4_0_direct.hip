@@ -16,12 +16,18 @@
 //   64 x 14336 x 4096  60 -> 38          77 x 4096 x 14336    77 -> 49     200 x 14336 x 4096  153 -> 85
 // and from 24 rows down the row kernel is no slower. Blocks' sums are those of qgemm_q4_0_fx16.hip; with K in shares and halves the error
 // against 64 bits is 1.05e-7 of the result at 77 x 5120 x 5120 where it was 1.63e-7.
+//
+// Rows held with an exponent a block (q4_halves.h: Form) take their scales through LDS beside x: four reads and a multiplication an output more a
+// block. One such row in the call, against one strip of x at a time with its rows' scales from memory, before, and against the
+// forms that this kernel took the place of: 77 x 5120 x 5120 53 -> 34 us (41), 128 x 14336 x 4096 127 -> 66 (84), 256 x 14336 x 4096 217 -> 100 (162).
 #include "kernels.h"
 #include "q4_halves.h"
 
 namespace mimir {
 
 namespace {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileStrips = 4;  // of x, at most
 constexpr int kColStrips = 4;   // of W a workgroup
@@ -32,7 +38,12 @@ struct Direct {
     int shares, share_blocks;  // of K; the last share may be shorter, all are even
 };
 
-// MS strips of x from row m0 on.
+// LDS: [2 halves][2][MS] granules of x, in whose place the halves' sums meet; then where rows have scales a block [2 halves][2][MS 32] of these.
+template <int MS>
+constexpr int kLdsBytes = 4 * MS * kGranuleX * 2 + 4 * MS * 32 * 4;
+
+// MS strips of x from row m0 on. BY_BLOCK: where a row of them has an exponent a block, all are taken as if they had. A thread brings one
+// row's scales through LDS, and a lane reads those of its results' rows from there, four a read, the same for the half's lanes.
 template <int MS, bool BY_BLOCK>
 __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, int m0, int group, int share, float* lds) {
     constexpr int kPairs = 3;  // pairs of blocks of W in registers, this one among them
@@ -59,6 +70,21 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
 #pragma unroll
     for (int p = 0; p < 4; p++) piece[p] = r32 * 64 + ((2 * p + q) ^ turn_of(r32)) * 8;
     uint16_t* stage = (uint16_t*)lds + second * 2 * MS * kGranuleX;  // [2][MS] granules of this half
+    // a thread's row of scales: of those that have one exponent, that one
+    float* scales = lds + MS * kGranuleX * 2 + second * 2 * MS * 32;  // [2][MS 32] of this half
+    const int srow = col * 64 + lane;
+    const float* row_scales = nullptr;
+    f32x2 scale[2] = {{0.f, 0.f}, {0.f, 0.f}};  // of this pair of blocks and the next
+    if (BY_BLOCK && srow < MS * 32) {
+        const int m = m0 + srow < M ? m0 + srow : M - 1;
+        const int2 info = o.RS[m];
+        if (info.y == kBlockHalves) {
+            row_scales = o.XS + (int64_t)m * nb + b0;
+        } else {
+            const float one = info.x == INT32_MAX ? __builtin_nanf("") : __builtin_ldexpf(1.f, info.x);
+            scale[0] = scale[1] = f32x2{one, one};
+        }
+    }
 
     f32x16 acc[MS], zero;
 #pragma unroll
@@ -83,6 +109,12 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
 #pragma unroll
         for (int mt = 0; mt < MS; mt++) *(u32x4*)(stage + ((b & 1) * MS + mt) * kGranuleX + col * 512 + lane * 8) = from[mt];
     };
+    auto load_scales = [&](int b, f32x2& to) {  // b even; a row's blocks are an even number, so a pair lies on 8 bytes
+        if (BY_BLOCK && row_scales) to = *(const f32x2*)(row_scales + (b < count ? b : count - 2));
+    };
+    auto store_scale = [&](int b, float s) {
+        if (BY_BLOCK && srow < MS * 32) scales[(b & 1) * MS * 32 + srow] = s;
+    };
     auto block = [&](int b, const u32x3& raw_b, bool odd) {
         const uint32_t lo = odd ? raw_b[1] : __builtin_amdgcn_alignbyte(raw_b[1], raw_b[0], 2);
         const uint32_t hi = odd ? raw_b[2] : __builtin_amdgcn_alignbyte(raw_b[2], raw_b[1], 2);
@@ -93,22 +125,19 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
         const f16x8 w0 = nibbles_to_f16(lo, hi, 0), w1 = nibbles_to_f16(lo, hi, 1);
         // a strip's products are issued with the FMAs of the one before it
         f32x16 c[2];
+        f32x4 dx[2][4];  // x's scales of this block, of the 16 rows that this lane has results of
         auto finish = [&](int mt) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                float f = dw;
-                if (BY_BLOCK) {  // x's scales of this block, of the 16 rows that this lane has results of
-                    const int m = m0 + mt * 32 + 8 * (e >> 2) + 4 * q + (e & 3);
-                    f = dw * o.XS[(int64_t)(m < M ? m : M - 1) * nb + b0 + b];
-                }
-                acc[mt][e] = fmaf(f, c[mt & 1][e], acc[mt][e]);
-            }
+            for (int e = 0; e < 16; e++) acc[mt][e] = fmaf(BY_BLOCK ? dw * dx[mt & 1][e >> 2][e & 3] : dw, c[mt & 1][e], acc[mt][e]);
             __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
         for (int mt = 0; mt < MS; mt++) {
             const uint16_t* x = stage + ((b & 1) * MS + mt) * kGranuleX;
             auto part = [&](int p) { return *(const f16x8*)(x + piece[p]); };
+            if (BY_BLOCK)
+#pragma unroll
+                for (int g = 0; g < 4; g++) dx[mt & 1][g] = *(const f32x4*)(scales + ((b & 1) * MS + mt) * 32 + 8 * g + 4 * q);
             f32x16& s = c[mt & 1];
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(part(2), w0, zero, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(part(3), w1, s, 0, 0, 0);
@@ -125,6 +154,9 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
         load_x(1, held[1]);
         store_x(0, held[0]);
         load_x(2, held[0]);
+        load_scales(0, scale[0]);
+        load_scales(2, scale[1]);
+        store_scale(0, scale[0][0]);
     }
     __syncthreads();
     for (int b = 0; b < first_half; b += 2 * kPairs) {
@@ -135,6 +167,11 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
                 if ((u & 1) == 0) load_w(b + u + 2 * kPairs - 2, raw[(u / 2 + kPairs - 1) % kPairs]);
                 store_x(b + u + 1, held[(u + 1) & 1]);
                 load_x(b + u + 3, held[(u + 1) & 1]);
+                store_scale(b + u + 1, u & 1 ? scale[1][0] : scale[0][1]);
+                if (BY_BLOCK && (u & 1)) {
+                    scale[0] = scale[1];
+                    load_scales(b + u + 3, scale[1]);
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 block(b + u, raw[u / 2][u & 1], u & 1);
             }
@@ -198,7 +235,7 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
 
 template <int MS>
 __global__ __launch_bounds__(64 * kWaves) void qgemm_q4_0_direct_kernel(Operands o, Direct d) {
-    __shared__ float lds[(size_t)kColStrips * MS * 16 * 64];
+    extern __shared__ __align__(16) float lds[];
     int t = (int)blockIdx.x;
     const int group = __builtin_amdgcn_readfirstlane(t % d.groups);
     t /= d.groups;
@@ -206,11 +243,20 @@ __global__ __launch_bounds__(64 * kWaves) void qgemm_q4_0_direct_kernel(Operands
     bool by_block = false;
     for (int r = threadIdx.x & 63; r < MS * 32; r += 64) by_block |= o.RS[m0 + r < o.M ? m0 + r : o.M - 1].y == kBlockHalves;
     if (__ballot(by_block) == 0) direct_tile<MS, false>(o, d, m0, group, share, lds);
-    else  // rare: a strip of x at a time, which holds the addresses of its rows' scales in registers
-        for (int mt = 0; mt < MS && m0 + 32 * mt < o.M; mt++) {
-            if (mt) __syncthreads();  // the one before has read its sums
-            direct_tile<1, true>(o, d, m0 + 32 * mt, group, share, lds);
+    else direct_tile<MS, true>(o, d, m0, group, share, lds);
+}
+
+template <int MS>
+hipError_t launch(const Operands& o, const Direct& d, hipStream_t st) {
+    if (kLdsBytes<MS> > 64 * 1024) {
+        static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
+        if (!raised) {
+            if (hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_direct_kernel<MS>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes<MS>)) return e;
+            raised = true;
         }
+    }
+    hipLaunchKernelGGL(qgemm_q4_0_direct_kernel<MS>, dim3((unsigned)(d.groups * d.tiles_m * d.shares)), dim3(64 * kWaves), kLdsBytes<MS>, st, o, d);
+    return hipGetLastError();
 }
 
 // Microseconds of a product and its cut into shares of K. A compute unit takes a workgroup at a time; one takes 2 us and, for
@@ -263,8 +309,7 @@ hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st) {
         if (((uintptr_t)o.parts.W[i] & 3) != 0) return hipErrorInvalidValue;
     if (d.shares == 1) o.sums = nullptr;
     const int ms = d.tiles_m > 1 ? kTileStrips : (int)strips_of(o.M);
-    const auto kernel = ms == 1 ? qgemm_q4_0_direct_kernel<1> : ms == 2 ? qgemm_q4_0_direct_kernel<2> : ms == 3 ? qgemm_q4_0_direct_kernel<3> : qgemm_q4_0_direct_kernel<4>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(d.groups * d.tiles_m * d.shares)), dim3(64 * kWaves), 0, st, o, d);
+    if (hipError_t e = ms == 1 ? launch<1>(o, d, st) : ms == 2 ? launch<2>(o, d, st) : ms == 3 ? launch<3>(o, d, st) : launch<4>(o, d, st)) return e;
     if (d.shares > 1)
         if (hipError_t e = sum_shares(o, d.shares, st)) return e;
     note_kernel("qgemm_q4_0_direct_kernel<%d>: %d x %d tiles, %d shares of K", ms, d.tiles_m, d.groups, d.shares);

@@ -13,7 +13,7 @@ from mimir_amd import capi
 from mimir_amd.llama import Llama
 from oracle import llama as OL
 from tests import gpu
-from tests.helpers import random_blocks
+from tests.helpers import bench_blocks, random_blocks
 from tests.test_gpu_llama import _oracle_config, _upload_synthetic
 
 pytestmark = pytest.mark.gpu
@@ -80,6 +80,48 @@ def test_pairs_of_halves(m, n, k, kernel, rows):
     got = gpu.dev(got).double()
     assert torch.isnan(got[bad]).all()
     assert ((got - want).abs() <= bound)[good].all()
+
+
+@pytest.mark.parametrize("m", [20, 64, 77, 128, 200])
+def test_rows_held_by_block_among_others(m):
+    """One row with a block 2^17 above its others, which is held with an exponent a block, beside ordinary rows, a row of zeros and one with
+    a NaN, by W read where it lies: results as above, and no more than half as long again as without it (such a row is rare, but takes the
+    tile's other rows with it; twice as long and more where a tile then went through W once for each 32 rows of x)."""
+    n, k, l = 14336, 4096, gpu.lib()
+    rng = np.random.default_rng(m)
+    raw = bench_blocks(rng, O.Q4_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    wide = x.copy()
+    wide[m // 2, 96:128] *= 2.0 ** 17
+    odd = wide.copy()
+    odd[1], odd[m - 1, 40] = 0, np.nan
+    w, xs = gpu.dev(raw), [gpu.dev(v) for v in (x, wide, odd)]
+    y = torch.empty((m, n), device="cuda:0")
+
+    def call(i, times=1):
+        for _ in range(times):
+            capi.check(l.mi355x_qgemv(capi.Q4_0, w.data_ptr(), xs[i].data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream()))
+    gpu.say(f"q4_0 halves, a row held by block, M={m}")
+    took = [[], []]
+    try:
+        tuned(0, 3)
+        call(2)
+        assert last_kernel().startswith(IN_PLACE)
+        w64, x64, got = gpu.dev(O.dequantize(O.Q4_0, raw).reshape(n, k)).double(), xs[2].double(), y.double()
+        for _ in range(5):
+            for i in (0, 1):
+                start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                call(i, 3)
+                start.record()
+                call(i, 20)
+                stop.record()
+                stop.synchronize()
+                took[i].append(start.elapsed_time(stop))
+    finally:
+        tuned(0, 1)
+    bound = 2e-6 * (x64.abs() @ w64.abs().T) + 2.0 ** -23 * (x64.abs().reshape(m, -1, 32).amax(2) @ w64.abs().reshape(n, -1, 32).sum(2).T) + 1e-30
+    assert torch.isnan(got[m - 1]).all() and ((got - x64 @ w64.T).abs() <= bound)[:m - 1].all()
+    assert min(took[1]) <= 1.5 * min(took[0]), (min(took[1]), min(took[0]))
 
 
 @pytest.mark.parametrize("batch,prompt,hidden", [(1, 150, 1088), (2, 24, 1024), (3, 100, 992)])

@@ -35,6 +35,10 @@ MI355X_API mi355x_status mi355x_stream_read(const void* p, size_t bytes, float* 
  * n bytes. */
 MI355X_API mi355x_status mi355x_last_kernel(char* buf, size_t n);
 
+/* The bytes of the stream's scratch that mi355x_qgemv asks for at a Q4_0 product of M rows of x, W and the rows of x on 16 bytes (0: none, or not a
+ * product). It never falls as M grows. No device is needed. */
+MI355X_API size_t mi355x_q4_0_scratch_bytes(int64_t M, int64_t N, int64_t K);
+
 #ifdef __cplusplus
 }
 #endif

@@ -87,6 +87,7 @@ SYMBOLS = {
     "mi355x_attention_d": (C.c_uint32, [_vp, _vp]),
     "mi355x_stream_release": (C.c_uint32, [_vp]),
     "mi355x_last_kernel": (C.c_uint32, [_vp, _sz]),
+    "mi355x_q4_0_scratch_bytes": (_sz, [_i64, _i64, _i64]),
     "mi355x_timed_begin": (C.c_uint32, [_int]),
     "mi355x_timed_end": (C.c_uint32, [_vp, _vp]),
     "mi355x_gemv_stamps": (C.c_uint32, [_vp]),

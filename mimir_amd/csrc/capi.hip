@@ -112,9 +112,37 @@ mi355x_status argmax_scratch(void* stream, size_t bytes, void** out) {
     return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, mimir::kArgmaxTicketBytes, "argmax", out);
 }
 
+size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// The stream's scratch that a Q4_0 product of several rows of x asks for: as much as any form of these rows or of fewer can take, so that
+// a call never outgrows what one with more rows by the same matrix has left (a block cannot grow under capture). wide_x: rows
+// of x on 16 bytes, which every form but the row kernel's wants.
+size_t q4_0_scratch_bytes(const void* W, int64_t M, int64_t N, int64_t K, bool wide_x) {
+    if (M <= 1 || !mimir::q4_0_fixed_point_ok(W, K)) return 0;  // one row: at most its own form, within any block's first size
+    size_t most = mimir::q4_0_act_bytes(K) * (size_t)M;
+    if (!wide_x) return most;
+    if (mimir::qgemv_q4_0_rows_ok(W, 1, N, K))
+        most = std::max(most, mimir::q4_0_rows_act_bytes(K) * (size_t)(mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1) ? (M + 7) / 8 : 1));
+    if (M < 16) return most;
+    size_t ws = 0;
+    (void)mimir::qgemm_q4_0_in_place_cost_us(W, M, N, K, &ws);
+    most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K)) + ws);
+    if (mimir::qgemm_q4_0_fx_ok(W, M, N, K)) {
+        most = std::max(most, mimir::q4_0_fx_act_bytes(K) * (size_t)M);
+        if (mimir::qgemm_q4_0_fx16_pays(M, N, K))
+            most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M, K)) + mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K));
+    }
+    return most;
+}
+
 }  // namespace
 
 extern "C" {
+
+size_t mi355x_q4_0_scratch_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > 65535 || N > (int64_t)1 << 30 || K > (int64_t)1 << 30 || K % 32 != 0) return 0;
+    return q4_0_scratch_bytes((const void*)256, M, N, K, true);
+}
 
 // Tensor.MatMulT with bfloat16 activations (tensor/quant.go:45-48): float32
 // product, one rounding to the output's dtype.
@@ -219,13 +247,14 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             else if (rows && M >= 16 && mimir::qgemm_q4_0_fx_ok(W, M, N, K))
                 rows = mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K);
             // some tens of rows, where W read where it lies by pairs of binary16 undercuts both (not from a fixed scratch, which is too
-            // small); every call of 16 rows and more asks for the scratch of that many rows, up to 256, so that none grows it after a larger one
+            // small)
+            const size_t scratch = src.fixed ? 0 : q4_0_scratch_bytes(W, M, N, K, wide_x);
             if (M >= 16 && !src.fixed && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0 && K % 32 == 0) {
                 size_t ws;
                 const double us = mimir::qgemm_q4_0_in_place_cost_us(W, M, N, K, &ws);
-                const size_t act_bytes = (mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K) + 255) / 256 * 256;
+                const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K));
                 void* act;
-                if (mi355x_status st = act_for(src, act_bytes + ws, &act)) return st;
+                if (mi355x_status st = act_for(src, scratch, &act)) return st;
                 double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
                 if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
                 // 8 us: the conversion, and what two launches more or less cost where the models are close (64 x 4096 x 4096: rows 22 us, here 24)
@@ -239,7 +268,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 const bool one_launch = mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1);  // else the variant that takes eight rows a launch
                 const int64_t groups = (M + 7) / 8;
                 void* act;
-                if (mi355x_status st = act_for(src, mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? groups : 1), &act)) return st;
+                if (mi355x_status st = act_for(src, std::max(scratch, mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? groups : 1)), &act)) return st;
                 if (one_launch) {
                     HIP_TRY(mimir::q4_0_rows_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_rows_convert_act");
                     HIP_TRY(mimir::qgemv_q4_0_rows(W, act, y, nullptr, M, N, K, 1, (hipStream_t)stream), "launch qgemv_q4_0_rows");
@@ -259,8 +288,8 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 // from some hundreds of rows on as pairs of binary16 numbers on the binary16 matrix cores, which want a
                 // workspace behind the activations (not from a fixed scratch, which is too small for it)
                 const bool pairs = !src.fixed && mimir::qgemm_q4_0_fx16_pays(M, N, K);
-                const size_t act_bytes = ((pairs ? mimir::q4_0_fx16_act_bytes(M, K) : mimir::q4_0_fx_act_bytes(K) * (size_t)M) + 255) / 256 * 256;
-                if (mi355x_status st = act_for(src, act_bytes + (pairs ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0), &act)) return st;
+                const size_t act_bytes = rounded(pairs ? mimir::q4_0_fx16_act_bytes(M, K) : mimir::q4_0_fx_act_bytes(K) * (size_t)M);
+                if (mi355x_status st = act_for(src, std::max(scratch, act_bytes + (pairs ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0)), &act)) return st;
                 HIP_TRY(mimir::q4_0_fx_convert_act(x, M, K, x_row_stride, act, pairs, (hipStream_t)stream), "launch q4_0_fx_convert_act");
                 HIP_TRY(mimir::qgemm_q4_0_fx(W, act, y, nullptr, M, N, K, pairs ? (uint8_t*)act + act_bytes : nullptr, (hipStream_t)stream),
                         "launch qgemm_q4_0_fx");
@@ -272,7 +301,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 return MI355X_OK;
             }
             void* act;
-            if (mi355x_status st = act_for(src, mimir::q4_0_act_bytes(K) * (size_t)M, &act)) return st;
+            if (mi355x_status st = act_for(src, std::max(scratch, mimir::q4_0_act_bytes(K) * (size_t)M), &act)) return st;
             HIP_TRY(mimir::q4_0_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_convert_act");
             a.act = act;
             HIP_TRY(mimir::qgemv_q4_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q4_0_act");

@@ -284,7 +284,7 @@ void set_q4_rows_direct(int v);  // measurement aid: 1 = its kernel that loads e
 // (q4_0_fx_act_bytes(K) bytes a row), K a multiple of 128. On the int8 matrix cores (qgemm_q4_0_fx.hip), or, with
 // `pairs` and a workspace (some hundreds of rows and more: qgemm_q4_0_fx16_pays says when), x converted into pairs
 // of binary16 numbers (q4_0_fx16_act_bytes(M, K) bytes) and the product on the binary16 matrix cores
-// (qgemm_q4_0_fx16.hip): ws qgemm_q4_0_fx16_ws_bytes(N, K) bytes, 16-byte aligned; ws null: act holds the int8 form.
+// (qgemm_q4_0_fx16.hip): ws qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned; ws null: act holds the int8 form.
 size_t q4_0_fx_act_bytes(int64_t K);
 hipError_t q4_0_fx_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, bool pairs, hipStream_t st);
 bool qgemm_q4_0_fx_ok(const void* W, int64_t M, int64_t N, int64_t K);
@@ -295,7 +295,7 @@ double qgemm_q4_0_fx16_cost_us(int64_t M, int64_t N, int64_t K);  // 1e30: not t
 bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K);  // against the int8 form, its pass over W included
 size_t q4_0_fx16_act_bytes(int64_t M, int64_t K);
 hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
-size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K);
+size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K);  // never falls as M grows
 hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st);
 // Up to three matrices by the same converted rows in one product; swiglu: part 0's y = silu(x . W0^T) (x . W1^T). resid: one part only.
 struct Fx16Part { const void* W; float* y; int64_t N; };

@@ -664,14 +664,23 @@ hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, in
     return hipGetLastError();
 }
 
+// The most that the shares' sums of a product of up to M rows take (plan): K's pieces of min_share_blocks, and no more than 1024 tiles of
+// 128 x 256. It never falls as M grows, where the sums of the one cut of M rows do: 512 rows by 4096 x 14336 take four shares, 2048 none.
+static size_t sums_bound(int64_t M, int64_t strips, int64_t K, int64_t min_share_blocks) {
+    const int64_t nb = K / 32;
+    int64_t shares = 1;
+    for (int64_t s = 2; s <= 16; s++)
+        if ((nb + s * kGroup - 1) / (s * kGroup) * kGroup >= min_share_blocks) shares = s;
+    const size_t by_rows = (size_t)shares * (size_t)M * (size_t)strips * 128, by_tiles = (size_t)1024 * Low::BM * Low::BN * 4;
+    return shares == 1 ? 0 : by_rows < by_tiles ? by_rows : by_tiles;
+}
+
 // The panel in granules, W's scales, the shares' sums.
 static size_t panel_bytes(int64_t strips, int64_t K) { return (size_t)strips * (size_t)(K / 32) * kGranuleP * 2; }
 static size_t scales_bytes(int64_t strips, int64_t K) { return (size_t)strips * (size_t)scale_blocks((int)(K / 32)) * kGranuleS * 4; }
 
 size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K) {
-    Cut cut{};
-    if (g_fx16 != 2) plan(M, strips_of(N), K, kMinShareBlocks, (size_t)-1, &cut);
-    return panel_bytes(strips_of(N), K) + scales_bytes(strips_of(N), K) + (cut.shares > 1 ? (size_t)cut.shares * (size_t)M * (size_t)strips_of(N) * 128 : 0);
+    return panel_bytes(strips_of(N), K) + scales_bytes(strips_of(N), K) + sums_bound(M, strips_of(N), K, kMinShareBlocks);
 }
 
 // x's part of the operands.

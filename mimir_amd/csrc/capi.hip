@@ -47,22 +47,36 @@ void set_llama_rows_off(int v);      // llm.hip
 }
 namespace {
 
-// Returns the calling stream's block `which` of the current device, at least `bytes` long (at least `floor`
-// when it has to be allocated); the first `zero_prefix` bytes of a new block are zeroed (tickets).
+// Returns the calling stream's block `which` of the current device, at least `bytes` long, and, where that much is to be had, `wish`
+// bytes (at least `floor` when it has to be allocated); the first `zero_prefix` bytes of a new block are zeroed (tickets).
 // Allocates, so it fails under stream capture when the block has to grow: a caller that records a
 // graph runs the call once beforehand, as run_batch does.
-mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, size_t bytes, size_t floor, size_t zero_prefix, const char* what,
+mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, size_t bytes, size_t wish, size_t floor, size_t zero_prefix, const char* what,
                              void** out) {
     DeviceState* s;
     if (mi355x_status st = current_state(&s)) return st;
     std::lock_guard<std::mutex> lock(g_mu);
     StreamScratch& mine = s->scratch[stream];
     ScratchBlock& b = mine.*which;
-    if (b.bytes < bytes) {
-        size_t want = bytes < floor ? floor : bytes;
-        if (want < 2 * b.bytes) want = 2 * b.bytes;
+    wish = std::max(wish, bytes);
+    if (b.bytes < wish && b.bytes >= bytes) {  // enough for this call: under capture, where no block can grow, it does
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone) wish = bytes;
+    }
+    if (b.bytes < wish) {
+        size_t want = std::max({wish, floor, 2 * b.bytes});
         void* p = nullptr;
         hipError_t e = hipMalloc(&p, want);
+        if (e != hipSuccess && want > bytes) {  // not as much as that: what this call needs
+            (void)hipGetLastError();  // which the next launch's check would report
+            if (b.bytes >= bytes) {
+                *out = b.p;
+                return MI355X_OK;
+            }
+            want = bytes;
+            e = hipMalloc(&p, want);
+        }
         if (e != hipSuccess) return capi_fail((mi355x_status)e, "mi355x: hipMalloc(%s scratch, %zu bytes): %s", what, want, hipGetErrorName(e));
         if (zero_prefix) {
             // on the calling stream, so that the zeros are in place before the first kernel that takes a ticket there
@@ -81,8 +95,8 @@ mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, s
     return MI355X_OK;
 }
 
-mi355x_status act_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::act, bytes, 1u << 20, 0, "activation", out);
+mi355x_status act_scratch(void* stream, size_t bytes, void** out, size_t wish = 0) {
+    return stream_scratch(stream, &StreamScratch::act, bytes, wish, kActFloorBytes, 0, "activation", out);
 }
 // Where a product's converted activations go: the stream's growing block, or a fixed block of
 // fixed_bytes bytes (then nothing is allocated and a larger need is an error).
@@ -91,28 +105,48 @@ struct ActSource {
     void* fixed;
     size_t fixed_bytes;
 };
-mi355x_status act_for(const ActSource& src, size_t bytes, void** out) {
-    if (!src.fixed) return act_scratch(src.stream, bytes, out);
+mi355x_status act_for(const ActSource& src, size_t bytes, void** out, size_t wish = 0) {
+    if (!src.fixed) return act_scratch(src.stream, bytes, out, wish);
     if (bytes > src.fixed_bytes)
         return capi_fail(MI355X_ERR_SHAPE, "mi355x: qgemv_noalloc: the converted activations take %zu bytes, the fixed scratch holds %zu", bytes, src.fixed_bytes);
     *out = src.fixed;
     return MI355X_OK;
 }
 mi355x_status attn_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::attn, bytes, 4u << 20, mimir::kAttnTicketBytes, "attention", out);
+    return stream_scratch(stream, &StreamScratch::attn, bytes, 0, 4u << 20, mimir::kAttnTicketBytes, "attention", out);
 }
 // The (value, flag) slots of decode attention's hand-over: all zero when handed out, and nobody else's.
 mi355x_status attn_flags_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::attn_flags, bytes, 1u << 20, (size_t)-1 /* all of it */, "attention hand-over", out);
+    return stream_scratch(stream, &StreamScratch::attn_flags, bytes, 0, 1u << 20, (size_t)-1 /* all of it */, "attention hand-over", out);
 }
 mi355x_status gemm_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::gemm, bytes, 0, 0, "gemm", out);
+    return stream_scratch(stream, &StreamScratch::gemm, bytes, 0, 0, 0, "gemm", out);
 }
 mi355x_status argmax_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, mimir::kArgmaxTicketBytes, "argmax", out);
+    return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, 0, mimir::kArgmaxTicketBytes, "argmax", out);
 }
 
 size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// About what a Q4_0 product of M rows takes on the row kernel or the int8 form, the shorter; it never falls as M grows.
+double q4_0_other_us(const void* W, int64_t M, int64_t N, int64_t K) {
+    const double rows = mimir::qgemv_q4_0_rows_ok(W, 1, N, K) ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
+    return mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? std::min(rows, mimir::qgemm_q4_0_fx_cost_us(M, N, K) + 5.0) : rows;
+}
+// The least that a product with W read where it lies takes, four pairs of blocks a workgroup and what stands around it: where the
+// others take no longer, its plan is not looked at.
+constexpr double kInPlaceLeastUs = 12.0;
+
+// Whether W is best read where it lies by pairs of binary16; rows: the row kernel would be taken else.
+bool q4_0_in_place_pays(const void* W, int64_t M, int64_t N, int64_t K, bool rows) {
+    if (!mimir::qgemm_q4_0_in_place_ok(W, N, K)) return false;
+    if (mimir::qgemm_q4_0_in_place_forced()) return true;
+    if (q4_0_other_us(W, M, N, K) <= kInPlaceLeastUs) return false;
+    double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
+    if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
+    // 8 us: the conversion, and what two launches more or less cost where the models are close (64 x 4096 x 4096: rows 22 us, here 24)
+    return mimir::qgemm_q4_0_in_place_cost_us(M, N, K) + 8.0 < other;
+}
 
 // The stream's scratch that a Q4_0 product of several rows of x asks for: as much as any form of these rows or of fewer can take, so that
 // a call never outgrows what one with more rows by the same matrix has left (a block cannot grow under capture). wide_x: rows
@@ -124,12 +158,13 @@ size_t q4_0_scratch_bytes(const void* W, int64_t M, int64_t N, int64_t K, bool w
     if (mimir::qgemv_q4_0_rows_ok(W, 1, N, K))
         most = std::max(most, mimir::q4_0_rows_act_bytes(K) * (size_t)(mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1) ? (M + 7) / 8 : 1));
     if (M < 16) return most;
-    size_t ws = 0;
-    (void)mimir::qgemm_q4_0_in_place_cost_us(W, M, N, K, &ws);
-    most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K)) + ws);
+    if (mimir::qgemm_q4_0_in_place_ok(W, N, K) && q4_0_other_us(W, M < 256 ? M : 256, N, K) > kInPlaceLeastUs)
+        most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K)) + mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K));
     if (mimir::qgemm_q4_0_fx_ok(W, M, N, K)) {
         most = std::max(most, mimir::q4_0_fx_act_bytes(K) * (size_t)M);
-        if (mimir::qgemm_q4_0_fx16_pays(M, N, K))
+        // 256 rows may do without the panel, more than that never
+        const bool in_place = M <= 256 && q4_0_in_place_pays(W, M, N, K, mimir::qgemv_q4_0_rows_ok(W, 1, N, K) && mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K));
+        if (!in_place && mimir::qgemm_q4_0_fx16_pays(M, N, K))
             most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M, K)) + mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K));
     }
     return most;
@@ -249,16 +284,11 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             // some tens of rows, where W read where it lies by pairs of binary16 undercuts both (not from a fixed scratch, which is too
             // small)
             const size_t scratch = src.fixed ? 0 : q4_0_scratch_bytes(W, M, N, K, wide_x);
-            if (M >= 16 && !src.fixed && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0 && K % 32 == 0) {
-                size_t ws;
-                const double us = mimir::qgemm_q4_0_in_place_cost_us(W, M, N, K, &ws);
-                const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K));
-                void* act;
-                if (mi355x_status st = act_for(src, scratch, &act)) return st;
-                double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
-                if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
-                // 8 us: the conversion, and what two launches more or less cost where the models are close (64 x 4096 x 4096: rows 22 us, here 24)
-                if (us + 8.0 < other) {
+            if (M >= 16 && M <= 256 && !src.fixed && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0) {
+                if (q4_0_in_place_pays(W, M, N, K, rows)) {
+                    const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M, K)), ws = mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K);
+                    void* act;
+                    if (mi355x_status st = act_for(src, act_bytes + ws, &act, scratch)) return st;
                     HIP_TRY(mimir::q4_0_halves_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_halves_convert_act");
                     HIP_TRY(mimir::qgemm_q4_0_in_place(W, act, y, M, N, K, (uint8_t*)act + act_bytes, ws, (hipStream_t)stream), "launch qgemm_q4_0_in_place");
                     return MI355X_OK;
@@ -268,7 +298,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 const bool one_launch = mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1);  // else the variant that takes eight rows a launch
                 const int64_t groups = (M + 7) / 8;
                 void* act;
-                if (mi355x_status st = act_for(src, std::max(scratch, mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? groups : 1)), &act)) return st;
+                if (mi355x_status st = act_for(src, mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? groups : 1), &act, scratch)) return st;
                 if (one_launch) {
                     HIP_TRY(mimir::q4_0_rows_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_rows_convert_act");
                     HIP_TRY(mimir::qgemv_q4_0_rows(W, act, y, nullptr, M, N, K, 1, (hipStream_t)stream), "launch qgemv_q4_0_rows");
@@ -289,7 +319,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 // workspace behind the activations (not from a fixed scratch, which is too small for it)
                 const bool pairs = !src.fixed && mimir::qgemm_q4_0_fx16_pays(M, N, K);
                 const size_t act_bytes = rounded(pairs ? mimir::q4_0_fx16_act_bytes(M, K) : mimir::q4_0_fx_act_bytes(K) * (size_t)M);
-                if (mi355x_status st = act_for(src, std::max(scratch, act_bytes + (pairs ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0)), &act)) return st;
+                if (mi355x_status st = act_for(src, act_bytes + (pairs ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0), &act, scratch)) return st;
                 HIP_TRY(mimir::q4_0_fx_convert_act(x, M, K, x_row_stride, act, pairs, (hipStream_t)stream), "launch q4_0_fx_convert_act");
                 HIP_TRY(mimir::qgemm_q4_0_fx(W, act, y, nullptr, M, N, K, pairs ? (uint8_t*)act + act_bytes : nullptr, (hipStream_t)stream),
                         "launch qgemm_q4_0_fx");
@@ -301,7 +331,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 return MI355X_OK;
             }
             void* act;
-            if (mi355x_status st = act_for(src, std::max(scratch, mimir::q4_0_act_bytes(K) * (size_t)M), &act)) return st;
+            if (mi355x_status st = act_for(src, mimir::q4_0_act_bytes(K) * (size_t)M, &act, scratch)) return st;
             HIP_TRY(mimir::q4_0_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_convert_act");
             a.act = act;
             HIP_TRY(mimir::qgemv_q4_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q4_0_act");

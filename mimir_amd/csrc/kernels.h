@@ -303,9 +303,12 @@ size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K);  
 bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes);
 hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, int64_t K, double eps, hipStream_t st);  // a norm and the conversion for it
 hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
-// One matrix by up to 256 rows converted by q4_0_halves_convert_act (q4_0_fx16_act_bytes), W read where it lies; its cost, and the
-// workspace that products of up to M rows want (1e30: not taken).
-double qgemm_q4_0_in_place_cost_us(const void* W, int64_t M, int64_t N, int64_t K, size_t* ws_bytes);
+// One matrix by up to 256 rows converted by q4_0_halves_convert_act (q4_0_fx16_act_bytes), W read where it lies: whether there is a number of
+// rows that it takes, its cost (1e30: not taken), and the workspace for products of up to M rows, which never falls as M grows.
+bool qgemm_q4_0_in_place_ok(const void* W, int64_t N, int64_t K);
+bool qgemm_q4_0_in_place_forced();  // measurement aid
+double qgemm_q4_0_in_place_cost_us(int64_t M, int64_t N, int64_t K);
+size_t qgemm_q4_0_in_place_sums_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t q4_0_halves_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
 hipError_t qgemm_q4_0_in_place(const void* W, const void* act, float* y, int64_t M, int64_t N, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
 void set_q4_0_fx16(int v);  // measurement aid: 0 keeps every product on the int8 form

@@ -141,7 +141,6 @@ hipError_t sum_shares(const Operands& o, int shares, hipStream_t st);
 // The product with W read where it lies (qgemm_q4_0_direct.hip): up to kDirectMaxRows rows.
 constexpr int64_t kDirectMaxRows = 256;
 constexpr size_t kDirectMostSums = (size_t)64 << 20;
-size_t qgemm_q4_0_direct_sums_bytes(int64_t M, int64_t strips);
 double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes);
 hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st);
 

@@ -288,13 +288,6 @@ bool fits(int64_t M, int64_t strips, int64_t K) {
 
 }  // namespace
 
-// The most that products of up to M rows can use for their shares' sums.
-size_t qgemm_q4_0_direct_sums_bytes(int64_t M, int64_t strips) {
-    return (size_t)32 * (size_t)(M < kDirectMaxRows ? M : kDirectMaxRows) * (size_t)strips * 128 < kDirectMostSums
-               ? (size_t)32 * (size_t)(M < kDirectMaxRows ? M : kDirectMaxRows) * (size_t)strips * 128
-               : kDirectMostSums;
-}
-
 double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes) {
     Direct d;
     return fits(M, strips, K) ? plan(M, strips, K, sums_bytes < kDirectMostSums ? sums_bytes : kDirectMostSums, &d) : 1e30;

@@ -821,12 +821,22 @@ hipError_t qgemm_q4_0_in_place(const void* W, const void* act, float* y, int64_t
     return in_place(p, act, nullptr, M, K, ws, ws_bytes, st);
 }
 
-double qgemm_q4_0_in_place_cost_us(const void* W, int64_t M, int64_t N, int64_t K, size_t* ws_bytes) {
-    *ws_bytes = qgemm_q4_0_direct_sums_bytes(M, strips_of(N));
-    if (g_fx16 == 0 || g_fx16 == 2 || N <= 0 || N >= (1 << 25) || ((uintptr_t)W & 3) != 0) return 1e30;
-    const double us = qgemm_q4_0_direct_cost_us(M, strips_of(N), K, *ws_bytes);
-    return g_fx16 == 3 && us < 1e30 ? -1e6 : us;
+bool qgemm_q4_0_in_place_ok(const void* W, int64_t N, int64_t K) {
+    return g_fx16 != 0 && g_fx16 != 2 && N > 0 && N < (1 << 25) && K > 0 && K % 64 == 0 && K <= (1 << 20) && ((uintptr_t)W & 3) == 0;
 }
+
+// 16 MiB: one round of workgroups, 256 of 128 rows by 128 columns. (With 64, single products of 200000 x 8192 and longer would take a twentieth less.)
+size_t qgemm_q4_0_in_place_sums_bytes(int64_t M, int64_t N, int64_t K) {
+    const int64_t pieces = (K / 32 + 7) / 8, shares = pieces < 32 ? pieces : 32, rows = M < kDirectMaxRows ? M : kDirectMaxRows;
+    const size_t all = (size_t)shares * (size_t)rows * (size_t)strips_of(N) * 128, most = (size_t)16 << 20;
+    return shares == 1 ? 0 : all < most ? all : most;
+}
+
+double qgemm_q4_0_in_place_cost_us(int64_t M, int64_t N, int64_t K) {
+    return qgemm_q4_0_direct_cost_us(M, strips_of(N), K, qgemm_q4_0_in_place_sums_bytes(M, N, K));
+}
+
+bool qgemm_q4_0_in_place_forced() { return g_fx16 == 3; }
 
 hipError_t q4_0_halves_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
     launch_halves<false>(x, nullptr, 0, M, K, x_row_stride, act, st);

@@ -30,6 +30,11 @@ constexpr int kMaxDevices = 16;
 // is created).
 constexpr size_t kNoallocScratchBytes = (size_t)1 << 20;
 
+// The first size of a stream's block of converted activations: whatever a Q4_0 product takes whose rows in fixed point fill no more than
+// 1 MiB, so that none of these grows the block, under capture for instance. Their pairs of binary16 (4 bytes an element where fixed point has 3
+// or more, rows rounded up to 32 from 16 on) are at most 2.8 MB, their shares' sums at most 16 MiB (qgemm_q4_0_in_place_sums_bytes).
+constexpr size_t kActFloorBytes = (size_t)19 << 20;
+
 // Scratch memory of the entry points that need some beyond their arguments (converted activations,
 // partial results and tickets of split attention and argmax, float32 copies of qgemm_bf16's general
 // route). One set per device and stream: calls on different streams never share a block, calls on one

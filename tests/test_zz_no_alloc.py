@@ -112,3 +112,35 @@ def test_noalloc_rejects_what_the_block_cannot_hold():
     # and the growing entry point takes the same call
     capi.check(l.mi355x_qgemv(capi.Q8_0, w.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream()))
     gpu.sync()
+
+
+def test_a_call_of_more_rows_under_capture_after_one_of_few():
+    """What a stream's first call leaves is enough for whatever fills no more than 1 MiB in fixed point: 32 rows by W read where it lies,
+    whose rows and shares of K take 4.8 MB, recorded into a graph after a call of eight rows, and replayed."""
+    l, n, k = gpu.lib(), 14336, 4096
+    rng = np.random.default_rng(5)
+    w = gpu.dev(helpers.bench_blocks(rng, O.Q4_0, n * k))
+    xs = [gpu.dev(rng.normal(size=(32, k)).astype(np.float32)) for _ in range(3)]
+    x, y, want = xs[0].clone(), torch.empty((32, n), device="cuda:0"), []
+
+    def call(m, stream, out=y):
+        capi.check(l.mi355x_qgemv(capi.Q4_0, w.data_ptr(), x.data_ptr(), out.data_ptr(), m, n, k, k, stream))
+    gpu.say("qgemv under capture after a call of few rows")
+    for v in xs:
+        x.copy_(v)
+        out = torch.empty_like(y)
+        call(32, gpu.stream(), out)
+        want.append(out)
+    torch.cuda.synchronize()
+    fresh, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(fresh):
+        call(8, fresh.cuda_stream)
+        fresh.synchronize()
+        with torch.cuda.graph(graph, stream=fresh):
+            call(32, fresh.cuda_stream)
+        for v, expected in zip(xs, want):
+            x.copy_(v)
+            y.fill_(float("nan"))
+            graph.replay()
+            fresh.synchronize()
+            assert torch.equal(y.view(torch.int32), expected.view(torch.int32))

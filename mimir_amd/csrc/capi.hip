@@ -145,7 +145,9 @@ bool q4_0_in_place_pays(const void* W, int64_t M, int64_t N, int64_t K, bool row
     double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
     if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
     // 8 us: the conversion, and what two launches more or less cost where the models are close (64 x 4096 x 4096: rows 22 us, here 24)
-    return mimir::qgemm_q4_0_in_place_cost_us(M, N, K) + 8.0 < other;
+    // Up to 24 rows, three groups of the row kernel, it has to be ahead by a sixth: one strip of x waits for its loads of long rows of W longer than its
+    // model says (24 x 8192 x 14336 was 49 us for the row kernel's 45, 20 x 14336 x 11008 71 for 63; 24 x 14336 x 14336 is 73 for 79).
+    return mimir::qgemm_q4_0_in_place_cost_us(M, N, K) + 8.0 < (M <= 24 ? other * (5.0 / 6.0) : other);
 }
 
 // The stream's scratch that a Q4_0 product of several rows of x asks for: as much as any form of these rows or of fewer can take, so that

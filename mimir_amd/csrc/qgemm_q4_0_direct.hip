@@ -14,7 +14,7 @@
 // 4-byte boundary a block they cost a tenth more). Whole calls, the row kernel or the int8 form before and this:
 //   77 x 5120 x 5120   39 -> 31.6 us     128 x 14336 x 4096   80 -> 57     256 x 4096 x 14336  219 -> 94
 //   64 x 14336 x 4096  60 -> 38          77 x 4096 x 14336    77 -> 49     200 x 14336 x 4096  153 -> 85
-// and from 24 rows down the row kernel is no slower. Blocks' sums are those of qgemm_q4_0_fx16.hip; with K in shares and halves the error
+// and from 24 rows down the row kernel is seldom slower. Blocks' sums are those of qgemm_q4_0_fx16.hip; with K in shares and halves the error
 // against 64 bits is 1.05e-7 of the result at 77 x 5120 x 5120 where it was 1.63e-7.
 //
 // Rows held with an exponent a block (q4_halves.h: Form) take their scales through LDS beside x: four reads and a multiplication an output more a

@@ -152,3 +152,16 @@ def test_a_prompt_pass_with_products_taken_together(batch, prompt, hidden):
     scale = np.abs(want).max()
     assert np.abs(out[3][0] - want).max() <= 0.02 * scale and np.median(np.abs(out[3][0] - want)) <= 1e-5 * scale
     assert np.median(np.abs(out[3] - out[0])) <= 1e-5 * scale and np.abs(out[3] - out[0]).max() <= 0.02 * scale
+
+
+@pytest.mark.parametrize("m,n,k,in_place", [(24, 8192, 14336, False), (20, 14336, 11008, False), (17, 8192, 11008, False), (24, 14336, 8192, False),
+                                            (32, 14336, 4096, True), (77, 5120, 5120, True), (24, 14336, 14336, True)])
+def test_the_row_kernel_keeps_up_to_24_rows_that_it_multiplies_faster(m, n, k, in_place):
+    raw = bench_blocks(np.random.default_rng(m), O.Q4_0, 16 * k)
+    w = gpu.dev(raw).repeat(n // 16)
+    x = torch.ones((m, k), device="cuda:0")
+    gpu.say(f"q4_0 choice M={m} N={n} K={k}")
+    gpu.qgemv(O.Q4_0, w.data_ptr(), x[:1], n, k)  # another kernel's name
+    before = last_kernel()
+    gpu.qgemv(O.Q4_0, w.data_ptr(), x, n, k)
+    assert before and last_kernel().startswith(IN_PLACE) == in_place

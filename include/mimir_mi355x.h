@@ -85,7 +85,7 @@ MI355X_API mi355x_status mi355x_sync(void* stream);
 /* Frees the scratch memory the library keeps for `stream` on the current device: converted activations,
  * attention's and argmax's partial results and tickets, qgemm_bf16's float32 copies, and the blocks kept aside
  * when one of them grew. Waits for the stream first. For hosts that create and destroy streams (the library
- * otherwise keeps a stream's scratch, some 5 MiB and up, for the life of the process). After it, no HIP graph
+ * otherwise keeps a stream's scratch, some 20 MiB and up, for the life of the process). After it, no HIP graph
  * recorded over this library's calls on that stream may be replayed: such a graph points into these blocks.
  * No counterpart in the reference, whose backend owns one stream for its whole life
  * (backend/rocm/rocm_linux.go:34-40). */
@@ -106,25 +106,29 @@ MI355X_API mi355x_status mi355x_stream_release(void* stream);
  * x by Q4_0 or by a small Q8_0, Q4_K or Q6_K matrix; Q8_0 weights are read
  * once for up to eight rows) or kernels on the int8 matrix cores (Q4_0 from two
  * rows on: up to some tens of rows a kernel that reads W once per eight rows,
- * beyond them a tiled one, and from some hundreds of rows by a large matrix x as
- * pairs of binary16 through the binary16 matrix cores, within the fixed point's
- * bound (below), which takes a workspace of 2 N K bytes and more in the stream's
- * scratch; two to eight
- * rows by a large Q8_0
- * matrix; Q4_K, Q6_K from enough rows on); which one ran changes the results
- * only by the order of float32 additions (Q4_0, Q8_0), or not at all (Q8_0
- * among its row kernels, Q4_K, Q6_K). */
+ * beyond them a tiled one; two to eight rows by a large Q8_0 matrix; Q4_K, Q6_K
+ * from enough rows on) or, for Q4_0, on the binary16 ones (some tens of rows up to
+ * 256 with W read where it lies, whose rows and shares of K take 4 M K bytes and
+ * up to 16 MiB of the stream's scratch; from some hundreds of rows with W's
+ * integers written out once a call, a workspace of 2 N K bytes and up to 128 MiB
+ * behind the rows); which one ran changes the results by the order of float32
+ * additions (Q4_0, Q8_0) and, for Q4_0, by how x is held (fixed point per block,
+ * or pairs of binary16: either within the bound below), or not at all (Q8_0 among
+ * its row kernels, Q4_K, Q6_K). The choice depends on the sizes, the
+ * alignment of W and x, and mi355x_tune alone. */
 MI355X_API mi355x_status mi355x_qgemv(int dtype, const void* W, const float* x, float* y, int64_t M, int64_t N, int64_t K,
                            int64_t x_row_stride, void* stream);
 
 /* mi355x_qgemv for callers that cannot allocate device memory: code under HIP
  * graph capture, serving loops and harnesses that forbid hipMalloc. It has no
  * counterpart in the reference. Same arguments, kernels and results as
- * mi355x_qgemv, but the converted activations go to a fixed block of 1 MiB inside
- * the library's code object instead of a scratch buffer that grows, and nothing
- * is allocated or freed: mi355x_init must have run on the device, and a product
- * whose converted activations exceed the block (M * mi355x_act_bytes(dtype, K),
- * for Q4_0 rounded up to groups of eight rows where W is read once per eight)
+ * mi355x_qgemv (of Q4_0 by 256 rows and more: the int8 matrix cores where that
+ * may take a kernel with the same bits and a workspace), but the converted
+ * activations go to a fixed block inside the library's code object instead of a
+ * scratch buffer that grows, and nothing is allocated or freed: mi355x_init must
+ * have run on the device, and a product whose converted activations exceed 1 MiB
+ * (M * mi355x_act_bytes(dtype, K), for Q4_0 rounded up to groups of eight rows
+ * where W is read once per eight, also where another form of them is used)
  * fails with MI355X_ERR_SHAPE. Every call on a device uses that device's one
  * block: calls that overlap on one device (two streams) race on it. */
 MI355X_API mi355x_status mi355x_qgemv_noalloc(int dtype, const void* W, const float* x, float* y, int64_t M, int64_t N, int64_t K,
@@ -141,7 +145,8 @@ MI355X_API mi355x_status mi355x_qgemv_noalloc(int dtype, const void* W, const fl
  *   Q4_0: 24-bit fixed point per block of 32 (K a multiple of 64, W dword
  *         aligned); no counterpart in the reference, whose kernels take
  *         float32 activations only. Block floating point, not float32: an
- *         element is held to 2^-23 of its block's largest magnitude amax_b, so
+ *         element is held to 2^-23 of its block's largest magnitude amax_b (as it
+ *         is where mi355x_qgemv holds x as pairs of binary16), so
  *         y[m, n] is within 2^-23 * sum_b amax_b * sum|w_b| of the float32
  *         product (b over the blocks of row n), beside the float32 sums' own
  *         2e-6 * sum|x||w|. For activations of even magnitude that is 1e-6 of

@@ -99,16 +99,18 @@ mi355x_status act_scratch(void* stream, size_t bytes, void** out, size_t wish = 
     return stream_scratch(stream, &StreamScratch::act, bytes, wish, kActFloorBytes, 0, "activation", out);
 }
 // Where a product's converted activations go: the stream's growing block, or a fixed block of
-// fixed_bytes bytes (then nothing is allocated and a larger need is an error).
+// kNoallocScratchBytes (then nothing is allocated, and activations of more than kNoallocActBytes are an error).
 struct ActSource {
     void* stream;
     void* fixed;
-    size_t fixed_bytes;
 };
+mi355x_status fixed_holds(size_t bytes) {
+    if (bytes <= kNoallocActBytes) return MI355X_OK;
+    return capi_fail(MI355X_ERR_SHAPE, "mi355x: qgemv_noalloc: the converted activations take %zu bytes, the fixed scratch holds %zu", bytes, kNoallocActBytes);
+}
 mi355x_status act_for(const ActSource& src, size_t bytes, void** out, size_t wish = 0) {
     if (!src.fixed) return act_scratch(src.stream, bytes, out, wish);
-    if (bytes > src.fixed_bytes)
-        return capi_fail(MI355X_ERR_SHAPE, "mi355x: qgemv_noalloc: the converted activations take %zu bytes, the fixed scratch holds %zu", bytes, src.fixed_bytes);
+    if (mi355x_status st = fixed_holds(bytes)) return st;
     *out = src.fixed;
     return MI355X_OK;
 }
@@ -140,7 +142,8 @@ constexpr double kInPlaceLeastUs = 12.0;
 // Whether W is best read where it lies by pairs of binary16; rows: the row kernel would be taken else.
 bool q4_0_in_place_pays(const void* W, int64_t M, int64_t N, int64_t K, bool rows) {
     if (!mimir::qgemm_q4_0_in_place_ok(W, N, K)) return false;
-    if (mimir::qgemm_q4_0_in_place_forced()) return true;
+    mimir::Fx16 form;
+    if (mimir::qgemm_q4_0_fx16_forced(&form)) return true;  // pairs: with digits it is not ok
     if (q4_0_other_us(W, M, N, K) <= kInPlaceLeastUs) return false;
     double other = rows ? mimir::qgemv_q4_0_rows_cost_us(M, N, K) : 1e30;
     if (!rows) other = std::min(mimir::qgemm_q4_0_fx16_cost_us(M, N, K), mimir::qgemm_q4_0_fx_ok(W, M, N, K) ? mimir::qgemm_q4_0_fx_cost_us(M, N, K) : 1e30) + 5.0;
@@ -160,12 +163,12 @@ size_t q4_0_scratch_bytes(const void* W, int64_t M, int64_t N, int64_t K, bool w
     if (mimir::qgemv_q4_0_rows_ok(W, 1, N, K))
         most = std::max(most, mimir::q4_0_rows_act_bytes(K) * (size_t)(mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1) ? (M + 7) / 8 : 1));
     if (M < 16) return most;
-    if (mimir::qgemm_q4_0_in_place_ok(W, N, K) && q4_0_other_us(W, M < 256 ? M : 256, N, K) > kInPlaceLeastUs)
-        most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M < 256 ? M : 256, K)) + mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K));
+    if (mimir::qgemm_q4_0_in_place_ok(W, N, K) && q4_0_other_us(W, M < mimir::kInPlaceRows ? M : mimir::kInPlaceRows, N, K) > kInPlaceLeastUs)
+        most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M < mimir::kInPlaceRows ? M : mimir::kInPlaceRows, K)) + mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K));
     if (mimir::qgemm_q4_0_fx_ok(W, M, N, K)) {
         most = std::max(most, mimir::q4_0_fx_act_bytes(K) * (size_t)M);
-        // 256 rows may do without the panel, more than that never
-        const bool in_place = M <= 256 && q4_0_in_place_pays(W, M, N, K, mimir::qgemv_q4_0_rows_ok(W, 1, N, K) && mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K));
+        // its first rows, 256, may do without the panel, more than that never
+        const bool in_place = M <= mimir::kInPlaceRows && q4_0_in_place_pays(W, M, N, K, mimir::qgemv_q4_0_rows_ok(W, 1, N, K) && mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K));
         if (!in_place && mimir::qgemm_q4_0_fx16_pays(M, N, K))
             most = std::max(most, rounded(mimir::q4_0_fx16_act_bytes(M, K)) + mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K));
     }
@@ -283,24 +286,25 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             if (rows && g_rows_max > 0) rows = M < g_rows_max;
             else if (rows && M >= 16 && mimir::qgemm_q4_0_fx_ok(W, M, N, K))
                 rows = mimir::qgemv_q4_0_rows_cost_us(M, N, K) < mimir::qgemm_q4_0_fx_cost_us(M, N, K);
-            // some tens of rows, where W read where it lies by pairs of binary16 undercuts both (not from a fixed scratch, which is too
-            // small)
+            // What the fixed-point forms take: a product that mi355x_qgemv_noalloc serves (kNoallocActBytes) runs on the same kernel through either entry point.
+            const bool one_launch = rows && mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1);  // else the variant that takes eight rows a launch
+            const bool fx = !rows && g_tune_q4[4] != 2 && M >= g_fx_min_rows && (g_fx_min_rows != 16 ? mimir::qgemm_q4_0_fx_ok(W, M, N, K) : mimir::qgemm_q4_0_fx_pays(W, M, N, K)) && wide_x;
+            const size_t plain = rows ? mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? (M + 7) / 8 : 1)
+                                      : (fx ? mimir::q4_0_fx_act_bytes(K) : mimir::q4_0_act_bytes(K)) * (size_t)M;
             const size_t scratch = src.fixed ? 0 : q4_0_scratch_bytes(W, M, N, K, wide_x);
-            if (M >= 16 && M <= 256 && !src.fixed && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0) {
-                if (q4_0_in_place_pays(W, M, N, K, rows)) {
-                    const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M, K)), ws = mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K);
-                    void* act;
-                    if (mi355x_status st = act_for(src, act_bytes + ws, &act, scratch)) return st;
-                    HIP_TRY(mimir::q4_0_halves_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_halves_convert_act");
-                    HIP_TRY(mimir::qgemm_q4_0_in_place(W, act, y, M, N, K, (uint8_t*)act + act_bytes, ws, (hipStream_t)stream), "launch qgemm_q4_0_in_place");
-                    return MI355X_OK;
-                }
+            // some tens of rows, where W read where it lies by pairs of binary16 undercuts both
+            if (M >= 16 && M <= mimir::kInPlaceRows && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0 && q4_0_in_place_pays(W, M, N, K, rows)) {
+                const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M, K)), ws = mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K);
+                void* act = src.fixed;
+                if (mi355x_status st = src.fixed ? fixed_holds(plain) : act_for(src, act_bytes + ws, &act, scratch)) return st;
+                if (src.fixed && act_bytes + ws > kNoallocScratchBytes) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: qgemv_noalloc: a workspace of %zu bytes", act_bytes + ws);
+                HIP_TRY(mimir::q4_0_fx16_convert_act(x, M, K, x_row_stride, act, mimir::Fx16::Pairs, (hipStream_t)stream), "launch q4_0_fx16_convert_act");
+                HIP_TRY(mimir::qgemm_q4_0_in_place(W, act, y, M, N, K, (uint8_t*)act + act_bytes, ws, (hipStream_t)stream), "launch qgemm_q4_0_in_place");
+                return MI355X_OK;
             }
             if (rows) {
-                const bool one_launch = mimir::qgemv_q4_0_rows_shares_ok(W, M, N, K, 1);  // else the variant that takes eight rows a launch
-                const int64_t groups = (M + 7) / 8;
                 void* act;
-                if (mi355x_status st = act_for(src, mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? groups : 1), &act, scratch)) return st;
+                if (mi355x_status st = act_for(src, plain, &act, scratch)) return st;
                 if (one_launch) {
                     HIP_TRY(mimir::q4_0_rows_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_rows_convert_act");
                     HIP_TRY(mimir::qgemv_q4_0_rows(W, act, y, nullptr, M, N, K, 1, (hipStream_t)stream), "launch qgemv_q4_0_rows");
@@ -313,18 +317,22 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 }
                 return MI355X_OK;
             }
-            if (g_tune_q4[4] != 2 && M >= g_fx_min_rows && (g_fx_min_rows != 16 ? mimir::qgemm_q4_0_fx_ok(W, M, N, K) : mimir::qgemm_q4_0_fx_pays(W, M, N, K)) &&
-                ((uintptr_t)x & 15) == 0 && x_row_stride % 4 == 0) {
-                // many rows: the fixed-point arithmetic on the int8 matrix cores
+            if (fx) {
+                // many rows: the fixed-point arithmetic on the int8 matrix cores, or from some hundreds of rows on the binary16 ones, which want a
+                // workspace behind the activations: x as pairs of binary16 numbers, or, where mi355x_qgemv_noalloc has the int8 form, as digits with its bits
+                mimir::Fx16 form = plain <= kNoallocActBytes ? mimir::Fx16::Digits : mimir::Fx16::Pairs;
+                const bool forced = mimir::qgemm_q4_0_fx16_forced(&form) || form == mimir::Fx16::Pairs;
+                const bool panel = !src.fixed && (forced ? mimir::qgemm_q4_0_fx16_pays(M, N, K) : mimir::qgemm_q4_0_fx16_digits_pay(M, N, K));
+                const size_t act_bytes = panel ? rounded(mimir::q4_0_fx16_act_bytes(M, K)) : plain;
                 void* act;
-                // from some hundreds of rows on as pairs of binary16 numbers on the binary16 matrix cores, which want a
-                // workspace behind the activations (not from a fixed scratch, which is too small for it)
-                const bool pairs = !src.fixed && mimir::qgemm_q4_0_fx16_pays(M, N, K);
-                const size_t act_bytes = rounded(pairs ? mimir::q4_0_fx16_act_bytes(M, K) : mimir::q4_0_fx_act_bytes(K) * (size_t)M);
-                if (mi355x_status st = act_for(src, act_bytes + (pairs ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0), &act, scratch)) return st;
-                HIP_TRY(mimir::q4_0_fx_convert_act(x, M, K, x_row_stride, act, pairs, (hipStream_t)stream), "launch q4_0_fx_convert_act");
-                HIP_TRY(mimir::qgemm_q4_0_fx(W, act, y, nullptr, M, N, K, pairs ? (uint8_t*)act + act_bytes : nullptr, (hipStream_t)stream),
-                        "launch qgemm_q4_0_fx");
+                if (mi355x_status st = act_for(src, act_bytes + (panel ? mimir::qgemm_q4_0_fx16_ws_bytes(M, N, K) : 0), &act, scratch)) return st;
+                if (panel) {
+                    HIP_TRY(mimir::q4_0_fx16_convert_act(x, M, K, x_row_stride, act, form, (hipStream_t)stream), "launch q4_0_fx16_convert_act");
+                    HIP_TRY(mimir::qgemm_q4_0_fx16(W, act, y, nullptr, M, N, K, (uint8_t*)act + act_bytes, form, (hipStream_t)stream), "launch qgemm_q4_0_fx16");
+                    return MI355X_OK;
+                }
+                HIP_TRY(mimir::q4_0_fx_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_fx_convert_act");
+                HIP_TRY(mimir::qgemm_q4_0_fx(W, act, y, nullptr, M, N, K, (hipStream_t)stream), "launch qgemm_q4_0_fx");
                 return MI355X_OK;
             }
             if (M == 1 && ((uintptr_t)x & 15) == 0) {
@@ -333,7 +341,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
                 return MI355X_OK;
             }
             void* act;
-            if (mi355x_status st = act_for(src, mimir::q4_0_act_bytes(K) * (size_t)M, &act, scratch)) return st;
+            if (mi355x_status st = act_for(src, plain, &act, scratch)) return st;
             HIP_TRY(mimir::q4_0_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_convert_act");
             a.act = act;
             HIP_TRY(mimir::qgemv_q4_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q4_0_act");
@@ -386,7 +394,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
 
 mi355x_status mi355x_qgemv(int dtype, const void* W, const float* x, float* y, int64_t M, int64_t N, int64_t K,
                            int64_t x_row_stride, void* stream) {
-    return qgemv_impl(dtype, W, x, y, M, N, K, x_row_stride, stream, ActSource{stream, nullptr, 0});
+    return qgemv_impl(dtype, W, x, y, M, N, K, x_row_stride, stream, ActSource{stream, nullptr});
 }
 
 // mi355x_qgemv without an allocation: the device's state must exist already (mi355x_init), and the
@@ -401,7 +409,7 @@ mi355x_status mi355x_qgemv_noalloc(int dtype, const void* W, const float* x, flo
         if (g_dev[dev].ready) fixed = g_dev[dev].fixed;
     }
     if (!fixed) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: qgemv_noalloc: call mi355x_init(%d) first (creating the device's state allocates)", dev);
-    return qgemv_impl(dtype, W, x, y, M, N, K, x_row_stride, stream, ActSource{stream, fixed, kNoallocScratchBytes});
+    return qgemv_impl(dtype, W, x, y, M, N, K, x_row_stride, stream, ActSource{stream, fixed});
 }
 
 size_t mi355x_act_bytes(int dtype, int64_t K) {

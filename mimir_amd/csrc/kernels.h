@@ -281,35 +281,37 @@ hipError_t rows_add_parts(float* x, const float* parts, int shares, int64_t n, h
 void set_q4_rows_waves(int v);   // measurement aid: 4 or 8 wavefronts a workgroup, 0 by shape
 void set_q4_rows_direct(int v);  // measurement aid: 1 = its kernel that loads each lane's block where it lies
 // The fixed-point Q4_0 product for many rows of float32 x on the matrix cores: x converted by q4_0_fx_convert_act
-// (q4_0_fx_act_bytes(K) bytes a row), K a multiple of 128. On the int8 matrix cores (qgemm_q4_0_fx.hip), or, with
-// `pairs` and a workspace (some hundreds of rows and more: qgemm_q4_0_fx16_pays says when), x converted into pairs
-// of binary16 numbers (q4_0_fx16_act_bytes(M, K) bytes) and the product on the binary16 matrix cores
-// (qgemm_q4_0_fx16.hip): ws qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned; ws null: act holds the int8 form.
+// (q4_0_fx_act_bytes(K) bytes a row), K a multiple of 128, on the int8 matrix cores (qgemm_q4_0_fx.hip).
 size_t q4_0_fx_act_bytes(int64_t K);
-hipError_t q4_0_fx_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, bool pairs, hipStream_t st);
+hipError_t q4_0_fx_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
 bool qgemm_q4_0_fx_ok(const void* W, int64_t M, int64_t N, int64_t K);
 bool qgemm_q4_0_fx_pays(const void* W, int64_t M, int64_t N, int64_t K);  // and is the faster choice against the one-row kernels
 double qgemm_q4_0_fx_cost_us(int64_t M, int64_t N, int64_t K);           // about what it takes, conversion aside
-hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st);
-double qgemm_q4_0_fx16_cost_us(int64_t M, int64_t N, int64_t K);  // 1e30: not taken
+hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, hipStream_t st);
+// The same product on the binary16 matrix cores (qgemm_q4_0_fx16.hip; some hundreds of rows and more: qgemm_q4_0_fx16_pays says when), x converted
+// by q4_0_fx16_convert_act (q4_0_fx16_act_bytes(M, K) bytes) into pairs of binary16 numbers, or into pairs of 12-bit digits, which
+// give the int8 form's bits; ws: qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned.
+enum class Fx16 { Pairs, Digits };
+double qgemm_q4_0_fx16_cost_us(int64_t M, int64_t N, int64_t K);  // of pairs; 1e30: not taken
 bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K);  // against the int8 form, its pass over W included
+bool qgemm_q4_0_fx16_digits_pay(int64_t M, int64_t N, int64_t K);
+bool qgemm_q4_0_fx16_forced(Fx16* form);  // measurement aid: every product on the binary16 matrix cores, in this form
 size_t q4_0_fx16_act_bytes(int64_t M, int64_t K);
-hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
+hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, Fx16 form, hipStream_t st);
 size_t qgemm_q4_0_fx16_ws_bytes(int64_t M, int64_t N, int64_t K);  // never falls as M grows
-hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st);
+hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, Fx16 form, hipStream_t st);
 // Up to three matrices by the same converted rows in one product; swiglu: part 0's y = silu(x . W0^T) (x . W1^T). resid: one part only.
 struct Fx16Part { const void* W; float* y; int64_t N; };
 size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K);  // as much as any number of rows can use
 bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes);
 hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, int64_t K, double eps, hipStream_t st);  // a norm and the conversion for it
 hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
-// One matrix by up to 256 rows converted by q4_0_halves_convert_act (q4_0_fx16_act_bytes), W read where it lies: whether there is a number of
+// One matrix by up to kInPlaceRows rows converted into pairs by q4_0_fx16_convert_act, W read where it lies: whether there is a number of
 // rows that it takes, its cost (1e30: not taken), and the workspace for products of up to M rows, which never falls as M grows.
+constexpr int64_t kInPlaceRows = 256;
 bool qgemm_q4_0_in_place_ok(const void* W, int64_t N, int64_t K);
-bool qgemm_q4_0_in_place_forced();  // measurement aid
 double qgemm_q4_0_in_place_cost_us(int64_t M, int64_t N, int64_t K);
 size_t qgemm_q4_0_in_place_sums_bytes(int64_t M, int64_t N, int64_t K);
-hipError_t q4_0_halves_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
 hipError_t qgemm_q4_0_in_place(const void* W, const void* act, float* y, int64_t M, int64_t N, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
 void set_q4_0_fx16(int v);  // measurement aid: 0 keeps every product on the int8 form
 

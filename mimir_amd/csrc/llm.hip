@@ -122,7 +122,8 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
         if (m.act[cls].bytes < need) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: activation scratch of %zu bytes, need %zu", m.act[cls].bytes, need);
         hipError_t e = cls == kActQ4   ? q4_0_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActQ8 ? q8_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
-                       : cls == kActFx || cls == kActFxPairs ? q4_0_fx_convert_act(x, rows, K, K, m.act[cls].p, cls == kActFxPairs, m.stream)
+                       : cls == kActFx ? q4_0_fx_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
+                       : cls == kActFxPairs ? q4_0_fx16_convert_act(x, rows, K, K, m.act[cls].p, Fx16::Pairs, m.stream)
                                        : kq_convert_act(x, rows, K, K, m.act[cls].p, m.stream);
         LLM_HIP(e, "convert activations");
         done[cls] = true;
@@ -145,7 +146,7 @@ mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_
             e = qgemm_q4_0_fx16_parts(&alone, 1, false, m.act[cls].p, resid, rows, w.k, m.fx_panel.p, m.fx_panel.bytes, m.stream);
             break;
         }
-        e = cls == kActFx   ? qgemm_q4_0_fx(w.buf.p, m.act[cls].p, y, resid, rows, w.n, w.k, nullptr, m.stream)
+        e = cls == kActFx   ? qgemm_q4_0_fx(w.buf.p, m.act[cls].p, y, resid, rows, w.n, w.k, m.stream)
             : cls == kActQ4 ? qgemv_q4_0_act(a, kNoTune, m.stream)
                             : qgemv_q4_0(a, kNoTune, m.stream);
         break;

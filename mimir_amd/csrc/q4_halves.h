@@ -138,8 +138,7 @@ __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t lo, uint32_t hi, int ha
 // The shares' sums of K, in their order: y = ((s0 + s1) + ..) (+ resid), or silu(gate) up of them.
 hipError_t sum_shares(const Operands& o, int shares, hipStream_t st);
 
-// The product with W read where it lies (qgemm_q4_0_direct.hip): up to kDirectMaxRows rows.
-constexpr int64_t kDirectMaxRows = 256;
+// The product with W read where it lies (qgemm_q4_0_direct.hip): up to kInPlaceRows rows.
 constexpr size_t kDirectMostSums = (size_t)64 << 20;
 double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes);
 hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st);

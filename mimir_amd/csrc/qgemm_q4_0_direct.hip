@@ -283,7 +283,7 @@ double plan(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, Direct* out
 }
 
 bool fits(int64_t M, int64_t strips, int64_t K) {
-    return M > 0 && M <= kDirectMaxRows && strips > 0 && strips < (1 << 20) && K > 0 && K % 64 == 0 && K <= (1 << 20);
+    return M > 0 && M <= kInPlaceRows && strips > 0 && strips < (1 << 20) && K > 0 && K % 64 == 0 && K <= (1 << 20);
 }
 
 }  // namespace

@@ -120,8 +120,7 @@ __global__ __launch_bounds__(256) void fx_convert_kernel(const float* __restrict
     }
 }
 
-hipError_t q4_0_fx_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, bool pairs, hipStream_t st) {
-    if (pairs) return q4_0_fx16_convert_act(x, M, K, x_row_stride, act, st);
+hipError_t q4_0_fx_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
     int gx = (int)((K / 4 + 255) / 256);
     hipLaunchKernelGGL(fx_convert_kernel, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, (int)K, (uint8_t*)act,
                        (int64_t)q4_0_fx_act_bytes(K));
@@ -302,9 +301,8 @@ bool qgemm_q4_0_fx_pays(const void* W, int64_t M, int64_t N, int64_t K) {
     return qgemm_q4_0_fx_cost_us(M, N, K) < rows_us;
 }
 
-// act: q4_0_fx_convert_act's rows, as pairs if ws is given. y = x . W^T (+ resid, which may be y itself).
-hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st) {
-    if (ws) return qgemm_q4_0_fx16(W, act, y, resid, M, N, K, ws, st);
+// act: q4_0_fx_convert_act's rows. y = x . W^T (+ resid, which may be y itself).
+hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
     if (!raised) {
         hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Layout::total);

@@ -632,6 +632,19 @@ bool qgemm_q4_0_fx16_pays(int64_t M, int64_t N, int64_t K) {
     return g_fx16 >= 2 || qgemm_q4_0_fx16_cost_us(M, N, K) < qgemm_q4_0_fx_cost_us(M, N, K);
 }
 
+// The same for digits: 2.85 us a step of 64 of K and round of tiles of 128 x 256 (256 x 32768 x 1024, two rounds).
+bool qgemm_q4_0_fx16_digits_pay(int64_t M, int64_t N, int64_t K) {
+    if (!qgemm_q4_0_fx16_pays(M, N, K)) return false;
+    const int64_t tiles = ((M + Low::BM - 1) / Low::BM) * ((N + Low::BN - 1) / Low::BN);
+    return (double)N * (double)K * (18.0 / 32.0 + 2.0) / 4.4e6 + (double)((tiles + 255) / 256) * (double)(K / 64) * 2.85 < qgemm_q4_0_fx_cost_us(M, N, K);
+}
+
+bool qgemm_q4_0_fx16_forced(Fx16* form) {
+    const int v = g_fx16;
+    if (v >= 2) *form = v == 2 ? Fx16::Digits : Fx16::Pairs;
+    return v >= 2;
+}
+
 // X16 in granules, then RS [M] int2, then XS [M, K / 32] float32.
 size_t q4_0_fx16_act_bytes(int64_t M, int64_t K) {
     return (size_t)strips_of(M) * (size_t)(K / 32) * kGranuleX * 2 + ((size_t)M * 8 + (size_t)M * (size_t)(K / 32) * 4 + 15) / 16 * 16;
@@ -646,8 +659,8 @@ static void launch_halves(const float* x, const float* w, double eps, int64_t M,
     hipLaunchKernelGGL(kernel, dim3((unsigned)M), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (float)(1.0 / (double)K), (float)eps);
 }
 
-hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
-    if (g_fx16 == 2) {
+hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, Fx16 form, hipStream_t st) {
+    if (form == Fx16::Digits) {
         uint16_t* X16 = (uint16_t*)act;
         int2* RS = (int2*)(X16 + strips_of(M) * (K / 32) * kGranuleX);
         const int gx = (int)((K / 4 + 255) / 256);
@@ -698,7 +711,7 @@ static hipError_t in_place(const Parts& parts, const void* act, const float* res
 }
 
 static hipError_t multiply(const Parts& parts, const void* act, const float* resid, int64_t M, int64_t K, int64_t min_share_blocks, void* ws, size_t ws_bytes,
-                           hipStream_t st) {
+                           Fx16 form, hipStream_t st) {
     const int64_t strips = parts.strips;
     const size_t fixed = panel_bytes(strips, K) + scales_bytes(strips, K);
     if (!ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)act & 15) != 0 || !fits(M, strips, K) || ws_bytes < fixed) return hipErrorInvalidValue;
@@ -712,7 +725,7 @@ static hipError_t multiply(const Parts& parts, const void* act, const float* res
         raised = true;
     }
     const int nb = (int)(K / 32);
-    const bool digits = g_fx16 == 2;
+    const bool digits = form == Fx16::Digits;
     Cut cut{0, 0, (int)((M + Low::BM - 1) / Low::BM), (int)((strips + 7) / 8), 1, nb};
     if (!digits) plan(M, strips, K, min_share_blocks, ws_bytes - fixed, &cut);
     uint16_t* P = (uint16_t*)ws;
@@ -801,16 +814,16 @@ hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const
     if (!parts_of(part, n, swiglu, K, &p) || (resid && n != 1) || !ws || ((uintptr_t)ws & 15) != 0) return hipErrorInvalidValue;
     parts_cost_us(p, M, K, ws_bytes, &direct);
     if (direct) return in_place(p, act, resid, M, K, ws, ws_bytes, st);
-    return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, st);
+    return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, Fx16::Pairs, st);
 }
 
 // act: q4_0_fx16_convert_act's for these M rows; ws: qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned.
 // y = x . W^T (+ resid, which may be y itself).
-hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, hipStream_t st) {
+hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, void* ws, Fx16 form, hipStream_t st) {
     if (N <= 0 || N >= (1 << 27) || !fits(M, strips_of(N), K)) return hipErrorInvalidValue;
     const int n = (int)strips_of(N);
     const Parts parts{{(const uint8_t*)W, nullptr, nullptr}, {y, nullptr, nullptr}, {(int)N, 0, 0}, {0, n, n}, n, 0};
-    return multiply(parts, act, resid, M, K, kMinShareBlocks, ws, qgemm_q4_0_fx16_ws_bytes(M, N, K), st);
+    return multiply(parts, act, resid, M, K, kMinShareBlocks, ws, qgemm_q4_0_fx16_ws_bytes(M, N, K), form, st);
 }
 
 // y = x . W^T, W read where it lies: ws 16-byte aligned.
@@ -827,20 +840,13 @@ bool qgemm_q4_0_in_place_ok(const void* W, int64_t N, int64_t K) {
 
 // 16 MiB: one round of workgroups, 256 of 128 rows by 128 columns. (With 64, single products of 200000 x 8192 and longer would take a twentieth less.)
 size_t qgemm_q4_0_in_place_sums_bytes(int64_t M, int64_t N, int64_t K) {
-    const int64_t pieces = (K / 32 + 7) / 8, shares = pieces < 32 ? pieces : 32, rows = M < kDirectMaxRows ? M : kDirectMaxRows;
+    const int64_t pieces = (K / 32 + 7) / 8, shares = pieces < 32 ? pieces : 32, rows = M < kInPlaceRows ? M : kInPlaceRows;
     const size_t all = (size_t)shares * (size_t)rows * (size_t)strips_of(N) * 128, most = (size_t)16 << 20;
     return shares == 1 ? 0 : all < most ? all : most;
 }
 
 double qgemm_q4_0_in_place_cost_us(int64_t M, int64_t N, int64_t K) {
     return qgemm_q4_0_direct_cost_us(M, strips_of(N), K, qgemm_q4_0_in_place_sums_bytes(M, N, K));
-}
-
-bool qgemm_q4_0_in_place_forced() { return g_fx16 == 3; }
-
-hipError_t q4_0_halves_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
-    launch_halves<false>(x, nullptr, 0, M, K, x_row_stride, act, st);
-    return hipGetLastError();
 }
 
 }  // namespace mimir

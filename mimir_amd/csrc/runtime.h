@@ -24,16 +24,20 @@ mi355x_status hip_fail(hipError_t e, const char* what);
 
 constexpr int kMaxDevices = 16;
 
-// The converted activations of mi355x_qgemv_noalloc: a fixed block in the code object's own
-// device memory, so that the entry point allocates nothing. Every device the library runs on
-// holds its own copy at its own address (DeviceState::fixed, looked up when the device's state
-// is created).
-constexpr size_t kNoallocScratchBytes = (size_t)1 << 20;
+// mi355x_qgemv_noalloc takes the products whose converted activations (for Q4_0 those in fixed point) fill no more than 1 MiB.
+constexpr size_t kNoallocActBytes = (size_t)1 << 20;
 
-// The first size of a stream's block of converted activations: whatever a Q4_0 product takes whose rows in fixed point fill no more than
-// 1 MiB, so that none of these grows the block, under capture for instance. Their pairs of binary16 (4 bytes an element where fixed point has 3
-// or more, rows rounded up to 32 from 16 on) are at most 2.8 MB, their shares' sums at most 16 MiB (qgemm_q4_0_in_place_sums_bytes).
+// The first size of a stream's block of converted activations, and the size of the block that stands in for it in
+// mi355x_qgemv_noalloc: whatever a Q4_0 product takes whose rows in fixed point fill no more than 1 MiB, so that none of these grows a
+// block, under capture for instance, and the same kernel serves them through either entry point. Their pairs of binary16 (4 bytes an element where
+// fixed point has 3 or more, rows rounded up to 32 from 16 on) are at most 2.8 MB, their shares' sums at most 16 MiB
+// (qgemm_q4_0_in_place_sums_bytes).
 constexpr size_t kActFloorBytes = (size_t)19 << 20;
+
+// The block of mi355x_qgemv_noalloc is in the code object's own device memory, so that the entry point allocates
+// nothing. Every device the library runs on holds its own copy at its own address (DeviceState::fixed, looked up
+// when the device's state is created).
+constexpr size_t kNoallocScratchBytes = kActFloorBytes;
 
 // Scratch memory of the entry points that need some beyond their arguments (converted activations,
 // partial results and tickets of split attention and argmax, float32 copies of qgemm_bf16's general

@@ -16,12 +16,12 @@ def test_no_call_asks_for_more_than_one_with_more_rows(n, k):
     assert not drops, drops[:4]
 
 
-@pytest.mark.parametrize("n,k", [(64, 64), (4096, 4096), (14336, 4096), (200000, 4096), (14336, 12288), (5120, 320)])
+@pytest.mark.parametrize("n,k", [(64, 64), (4096, 4096), (14336, 4096), (200000, 4096), (14336, 12288), (5120, 320), (64, 20480)])
 def test_rows_of_one_mib_in_fixed_point_stay_within_a_first_block(n, k):
-    """A stream's block of 19 MiB, which its first call leaves, holds whatever a call below the panel's 256 rows takes whose rows fill no more than 1 MiB as
-    the row kernel's groups of eight (1088 bytes a block of 32)."""
+    """A stream's block of 19 MiB, which its first call leaves, holds whatever a call below the panel's 256 rows takes whose rows fill no more than 1 MiB in
+    fixed point, one by one (3 1/8 bytes an element) or as the row kernel's groups of eight (1088 bytes a block of 32). mi355x_qgemv_noalloc has as much."""
     lib = capi.load()
-    rows = [m for m in range(2, 256) if (m + 7) // 8 * (k // 32) * 1088 <= 1 << 20]
+    rows = [m for m in range(2, 256) if m * (3 * k + k // 8) <= 1 << 20 or (m + 7) // 8 * (k // 32) * 1088 <= 1 << 20]
     assert rows and max(lib.mi355x_q4_0_scratch_bytes(m, n, k) for m in rows) <= 19 << 20
 
 

@@ -4,6 +4,8 @@ the oracle). Two calls in a row per case, the second with a smaller input, since
 last call's contents. That nothing is allocated is shown twice: the device's free memory does not move
 across the calls, and the calls are made under stream capture on a stream the library has never seen
 (where an allocation is refused, the library's growing scratch included), then replayed from the graph."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -144,3 +146,47 @@ def test_a_call_of_more_rows_under_capture_after_one_of_few():
             graph.replay()
             fresh.synchronize()
             assert torch.equal(y.view(torch.int32), expected.view(torch.int32))
+
+
+def last_kernel():
+    buf = C.create_string_buffer(200)
+    capi.check(gpu.lib().mi355x_last_kernel(buf, 200))
+    return buf.value.decode()
+
+
+@pytest.mark.parametrize("m,n,k,kernels", [
+    (32, 14336, 4096, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")), (48, 5120, 5120, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")),
+    (200, 32768, 1024, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")), (256, 32768, 1024, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")),
+    (300, 65536, 1024, ("qgemm_q4_0_fx16_kernel", "qgemm_q4_0_fx_kernel")), (512, 32768, 512, ("qgemm_q4_0_fx16_kernel", "qgemm_q4_0_fx_kernel")),
+    (1000, 2048, 256, ("qgemm_q4_0_fx_kernel", "qgemm_q4_0_fx_kernel"))])
+def test_noalloc_equals_qgemv_at_many_rows(m, n, k, kernels):
+    """Whatever the fixed block takes has mi355x_qgemv's bits there: W read where it lies, by the same kernel in the same shares of K; from
+    256 rows on the int8 form, whose bits mi355x_qgemv's panel of digits gives. Against 64 bits within the product's bound."""
+    rng = np.random.default_rng(m)
+    raw = helpers.bench_blocks(rng, O.Q4_0, 64 * k)
+    w = gpu.dev(raw).repeat(n // 64)
+    x = gpu.dev(rng.normal(size=(m, k)).astype(np.float32))
+    gpu.say(f"qgemv_noalloc q4_0 M={m} N={n} K={k}")
+    l, ys, ran = gpu.lib(), [], []
+    for fn in (l.mi355x_qgemv, l.mi355x_qgemv_noalloc):
+        y = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+        capi.check(fn(capi.Q4_0, w.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream()))
+        ran.append(last_kernel())
+        ys.append(y)
+    gpu.sync()
+    assert all(r.startswith(want) for r, want in zip(ran, kernels)), ran
+    assert torch.equal(ys[0].view(torch.int32), ys[1].view(torch.int32))
+    fresh, graph, y = torch.cuda.Stream(), torch.cuda.CUDAGraph(), torch.empty_like(ys[0])  # a stream that the library holds no scratch for
+    torch.cuda.synchronize()
+    with torch.cuda.stream(fresh):
+        with torch.cuda.graph(graph, stream=fresh):
+            capi.check(l.mi355x_qgemv_noalloc(capi.Q4_0, w.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, k, fresh.cuda_stream))
+        for replay in range(2):
+            y.fill_(float("nan"))
+            graph.replay()
+            fresh.synchronize()
+            assert torch.equal(y.view(torch.int32), ys[0].view(torch.int32)), replay
+    w64, x64 = gpu.dev(O.dequantize(O.Q4_0, raw).reshape(64, k)).double(), x.double()
+    bound = 2e-6 * (x64.abs() @ w64.abs().T) + 2.0 ** -23 * (x64.abs().reshape(m, -1, 32).amax(2) @ w64.abs().reshape(64, -1, 32).sum(2).T)
+    for n0 in (0, n - 64):
+        assert ((ys[1][:, n0:n0 + 64].double() - x64 @ w64.T).abs() <= bound).all()

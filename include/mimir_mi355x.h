@@ -476,8 +476,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * "q4_0.fx_rows" = n sends Q4_0 products of at least n rows of float32 x to the
  * int8 matrix cores whatever the shape (0: the built-in cost model);
  * "q4_0.fx_pairs" = 0 keeps those products off the binary16 matrix cores, 2
- * sends them all there as digits with the int8 form's bits, 3 as pairs of binary16
- * (1: pairs, by the cost models).
+ * sends them all there as digits with the int8 form's bits (the decoder's too,
+ * where their workspace was allocated), 3 as pairs of binary16 (1: pairs, by the
+ * cost models).
  * "qgemm.blocks" = 0 keeps the exact Q4_0 products of mi355x_qgemm_bf16 on the
  * kernel that needs no workspace, 2 sends them all through the panel of the
  * weights' integers (1: by shape).

@@ -120,10 +120,12 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
         if (cls == kActNone || done[cls]) continue;
         size_t need = act_bytes(cls, rows, K);
         if (m.act[cls].bytes < need) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: activation scratch of %zu bytes, need %zu", m.act[cls].bytes, need);
+        Fx16 form = Fx16::Pairs;
+        (void)qgemm_q4_0_fx16_forced(&form);
         hipError_t e = cls == kActQ4   ? q4_0_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActQ8 ? q8_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActFx ? q4_0_fx_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
-                       : cls == kActFxPairs ? q4_0_fx16_convert_act(x, rows, K, K, m.act[cls].p, Fx16::Pairs, m.stream)
+                       : cls == kActFxPairs ? q4_0_fx16_convert_act(x, rows, K, K, m.act[cls].p, form, m.stream)
                                        : kq_convert_act(x, rows, K, K, m.act[cls].p, m.stream);
         LLM_HIP(e, "convert activations");
         done[cls] = true;

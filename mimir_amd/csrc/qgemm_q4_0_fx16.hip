@@ -794,7 +794,9 @@ static double parts_cost_us(const Parts& p, int64_t M, int64_t K, size_t ws_byte
 bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes) {
     Parts p;
     bool direct;
-    if (g_fx16 == 0 || g_fx16 == 2 || M < kMinPartRows || !parts_of(part, n, swiglu, K, &p)) return false;
+    if (g_fx16 == 0 || M < kMinPartRows || !parts_of(part, n, swiglu, K, &p)) return false;
+    // digits, where the int8 form would be taken: one matrix at a time, by a panel
+    if (g_fx16 == 2) return n == 1 && qgemm_q4_0_fx_pays(part[0].W, M, part[0].N, K) && fits(M, p.strips, K) && ws_bytes >= panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
     const double us = parts_cost_us(p, M, K, ws_bytes, &direct);
     if (us >= 1e30) return false;
     double apart = 0;
@@ -812,9 +814,11 @@ hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const
     Parts p;
     bool direct;
     if (!parts_of(part, n, swiglu, K, &p) || (resid && n != 1) || !ws || ((uintptr_t)ws & 15) != 0) return hipErrorInvalidValue;
+    Fx16 form = Fx16::Pairs;
+    if (qgemm_q4_0_fx16_forced(&form) && form == Fx16::Digits) return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, form, st);
     parts_cost_us(p, M, K, ws_bytes, &direct);
     if (direct) return in_place(p, act, resid, M, K, ws, ws_bytes, st);
-    return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, Fx16::Pairs, st);
+    return multiply(p, act, resid, M, K, kMinPartShareBlocks, ws, ws_bytes, form, st);
 }
 
 // act: q4_0_fx16_convert_act's for these M rows; ws: qgemm_q4_0_fx16_ws_bytes(M, N, K) bytes, 16-byte aligned.

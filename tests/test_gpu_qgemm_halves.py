@@ -165,3 +165,27 @@ def test_the_row_kernel_keeps_up_to_24_rows_that_it_multiplies_faster(m, n, k, i
     before = last_kernel()
     gpu.qgemv(O.Q4_0, w.data_ptr(), x, n, k)
     assert before and last_kernel().startswith(IN_PLACE) == in_place
+
+
+def test_digits_on_request_in_a_prompt_pass():
+    """"q4_0.fx_pairs" = 2 sends the decoder's products of many rows to the binary16 matrix cores as digits too: the int8 form's bits."""
+    c = capi.LlamaConfig()
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = 384, 1024, 2, 6, 2, 64, 64, 2048
+    c.context, c.interleaved, c.cache_dtype, c.batch = 520, 1, capi.F32, 1
+    c.rope_base, c.rope_scale, c.eps = 10000.0, 1.0, 1e-5
+    m = Llama(c)
+    _upload_synthetic(m, OL.synthetic(_oracle_config(c), seed=4, output_dt=O.Q4_0))
+    m.finalize(512)
+    tokens = np.random.default_rng(2).integers(0, c.vocab, (1, 512))
+    out, ran = {}, {}
+    try:
+        for pairs in (2, 0):
+            gpu.say(f"prompt pass, digits, pairs={pairs}")
+            tuned(0, pairs)
+            m.reset()
+            out[pairs] = m.logits(tokens, all=True)
+            ran[pairs] = last_kernel()  # the output matrix's product
+    finally:
+        tuned(0, 1)
+    assert ran[2].startswith(PANEL) and ran[0] == "qgemm_q4_0_fx_kernel"
+    assert np.array_equal(out[2].view(np.uint32), out[0].view(np.uint32))

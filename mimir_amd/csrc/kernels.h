@@ -303,6 +303,7 @@ hipError_t qgemm_q4_0_fx16(const void* W, const void* act, float* y, const float
 // Up to three matrices by the same converted rows in one product; swiglu: part 0's y = silu(x . W0^T) (x . W1^T). resid: one part only.
 struct Fx16Part { const void* W; float* y; int64_t N; };
 size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K);  // as much as any number of rows can use
+size_t qgemm_q4_0_fx16_parts_uses(const Fx16Part* part, int n, int64_t K, int64_t max_rows, size_t ws_bytes);
 bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t M, int64_t K, size_t ws_bytes);
 hipError_t rmsnorm_fx16(const float* x, const float* w, void* act, int64_t M, int64_t K, double eps, hipStream_t st);  // a norm and the conversion for it
 hipError_t qgemm_q4_0_fx16_parts(const Fx16Part* part, int n, bool swiglu, const void* act, const float* resid, int64_t M, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);

@@ -16,6 +16,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -744,22 +745,41 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
     LLM_HIP(m->act2.alloc(q4_0_act_bytes((c.hidden + 63) / 64 * 64) * c.batch + 64), "hipMalloc(activations)");
     {
         // the workspace of the Q4_0 product's binary16 form, which calls of some tens of rows and more take: the largest matrix's, or
-        // that of those that are multiplied together
-        size_t panel = 0;
+        // that of those that are multiplied together; where no call has more rows than are multiplied with W read where it lies, what these use of it
+        struct Together { int n; int64_t rows[3], k; };
+        std::vector<Together> products;  // layers are alike
         auto want = [&](std::initializer_list<const Weight*> ws) {
-            Fx16Part part[3];
-            int n = 0;
+            Together t{0, {0, 0, 0}, (*ws.begin())->k};
             for (const Weight* w : ws) {
-                if (w->dtype != kQ4_0 || w->k != (*ws.begin())->k) return;
-                part[n++] = Fx16Part{w->buf.p, nullptr, w->n};
+                if (!w->set() || w->dtype != kQ4_0 || w->k != t.k) return;
+                t.rows[t.n++] = w->n;
             }
-            const size_t bytes = qgemm_q4_0_fx16_parts_ws_bytes(part, n, (*ws.begin())->k);
-            panel = bytes > panel ? bytes : panel;
+            for (const Together& o : products)
+                if (o.n == t.n && o.k == t.k && o.rows[0] == t.rows[0] && o.rows[1] == t.rows[1] && o.rows[2] == t.rows[2]) return;
+            products.push_back(t);
         };
         for (const Block& b : m->blocks) {
             for (const Weight* w : {&b.q, &b.k, &b.v, &b.o, &b.gate, &b.up, &b.down}) want({w});
             want({&b.q, &b.k, &b.v});
             want({&b.gate, &b.up});
+        }
+        auto parts = [](const Together& t, Fx16Part part[3]) {
+            for (int i = 0; i < t.n; i++) part[i] = Fx16Part{nullptr, nullptr, t.rows[i]};
+        };
+        size_t panel = 0;
+        Fx16Part part[3];
+        for (const Together& t : products) {
+            parts(t, part);
+            panel = std::max(panel, qgemm_q4_0_fx16_parts_ws_bytes(part, t.n, t.k));
+        }
+        if (panel && rows <= kInPlaceRows) {
+            want({m->tied ? &m->embed : &m->output});  // its products take what there is
+            size_t used = (size_t)1 << 20;
+            for (const Together& t : products) {
+                parts(t, part);
+                used = std::max(used, qgemm_q4_0_fx16_parts_uses(part, t.n, t.k, rows, panel));
+            }
+            panel = used;
         }
         m->fx_panel.release();
         m->fx_panel.bytes = 0;

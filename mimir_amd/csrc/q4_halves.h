@@ -140,7 +140,7 @@ hipError_t sum_shares(const Operands& o, int shares, hipStream_t st);
 
 // The product with W read where it lies (qgemm_q4_0_direct.hip): up to kInPlaceRows rows.
 constexpr size_t kDirectMostSums = (size_t)64 << 20;
-double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes);
+double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, size_t* used = nullptr);  // of sums_bytes
 hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st);
 
 inline int64_t strips_of(int64_t rows) { return (rows + 31) / 32; }

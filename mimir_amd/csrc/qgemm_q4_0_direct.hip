@@ -288,9 +288,11 @@ bool fits(int64_t M, int64_t strips, int64_t K) {
 
 }  // namespace
 
-double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes) {
-    Direct d;
-    return fits(M, strips, K) ? plan(M, strips, K, sums_bytes < kDirectMostSums ? sums_bytes : kDirectMostSums, &d) : 1e30;
+double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, size_t* used) {
+    Direct d{};
+    const double us = fits(M, strips, K) ? plan(M, strips, K, sums_bytes < kDirectMostSums ? sums_bytes : kDirectMostSums, &d) : 1e30;
+    if (used) *used = d.shares > 1 ? (size_t)d.shares * (size_t)M * (size_t)strips * 128 : 0;
+    return us;
 }
 
 // o: the parts, x's halves and their scales, sums: sums_bytes of workspace.

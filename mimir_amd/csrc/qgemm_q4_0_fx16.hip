@@ -779,15 +779,27 @@ size_t qgemm_q4_0_fx16_parts_ws_bytes(const Fx16Part* part, int n, int64_t K) {
     return parts_of(part, n, false, K, &p) ? panel_bytes(p.strips, K) + scales_bytes(p.strips, K) + kMostSums : 0;
 }
 
-// Microseconds here, the cheaper way: with the pass over W first, or W read where it lies.
-static double parts_cost_us(const Parts& p, int64_t M, int64_t K, size_t ws_bytes, bool* direct) {
-    Cut cut;
+// Microseconds here, the cheaper way: with the pass over W first, or W read where it lies; and what it uses of the workspace.
+static double parts_cost_us(const Parts& p, int64_t M, int64_t K, size_t ws_bytes, bool* direct, size_t* used = nullptr) {
+    Cut cut{};
+    size_t sums = 0;
     const size_t fixed = panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
     const double panel = fits(M, p.strips, K) && ws_bytes >= fixed ? plan(M, p.strips, K, kMinPartShareBlocks, ws_bytes - fixed, &cut) : 1e30;
     const bool aligned = (((uintptr_t)p.W[0] | (uintptr_t)p.W[1] | (uintptr_t)p.W[2]) & 3) == 0;
-    const double in_place = aligned ? qgemm_q4_0_direct_cost_us(M, p.strips, K, ws_bytes) : 1e30;
+    const double in_place = aligned ? qgemm_q4_0_direct_cost_us(M, p.strips, K, ws_bytes, &sums) : 1e30;
     *direct = in_place < panel;
+    if (used) *used = *direct ? sums : fixed + (cut.shares > 1 ? (size_t)cut.shares * (size_t)M * (size_t)p.strips * 128 : 0);
     return *direct ? in_place : panel;
+}
+
+// Microseconds of the products one by one, on the int8 form or the row kernels.
+static double apart_us(const Fx16Part* part, int n, int64_t M, int64_t K) {
+    double apart = 0;
+    for (int i = 0; i < n; i++) {
+        const double rows_us = (double)M * ((double)part[i].N * (double)(K / 32) * 18.0) / 8.7e6, fx = qgemm_q4_0_fx_cost_us(M, part[i].N, K);
+        apart += fx < rows_us ? fx : rows_us;
+    }
+    return apart;
 }
 
 // Whether they are the faster together here, in a workspace of ws_bytes, than each on the int8 form or the row kernels.
@@ -798,13 +810,20 @@ bool qgemm_q4_0_fx16_parts_pay(const Fx16Part* part, int n, bool swiglu, int64_t
     // digits, where the int8 form would be taken: one matrix at a time, by a panel
     if (g_fx16 == 2) return n == 1 && qgemm_q4_0_fx_pays(part[0].W, M, part[0].N, K) && fits(M, p.strips, K) && ws_bytes >= panel_bytes(p.strips, K) + scales_bytes(p.strips, K);
     const double us = parts_cost_us(p, M, K, ws_bytes, &direct);
-    if (us >= 1e30) return false;
-    double apart = 0;
-    for (int i = 0; i < n; i++) {
-        const double rows_us = (double)M * ((double)part[i].N * (double)(K / 32) * 18.0) / 8.7e6, fx = qgemm_q4_0_fx_cost_us(M, part[i].N, K);
-        apart += fx < rows_us ? fx : rows_us;
+    return us < 1e30 && (g_fx16 >= 3 || us < apart_us(part, n, M, K));
+}
+
+// What products of 9 rows up to max_rows use of a workspace of ws_bytes: in one of that size they run as in the larger one.
+size_t qgemm_q4_0_fx16_parts_uses(const Fx16Part* part, int n, int64_t K, int64_t max_rows, size_t ws_bytes) {
+    Parts p;
+    size_t most = 0;
+    if (!parts_of(part, n, false, K, &p)) return 0;
+    for (int64_t M = kMinPartRows; M <= max_rows; M++) {
+        bool direct;
+        size_t used;
+        if (parts_cost_us(p, M, K, ws_bytes, &direct, &used) < apart_us(part, n, M, K) && used > most) most = used;
     }
-    return g_fx16 >= 3 || us < apart;
+    return most;
 }
 
 // act: q4_0_fx16_convert_act's for these M rows; ws: ws_bytes, 16-byte aligned. Each part's y = x . W^T; one part alone: + resid, which

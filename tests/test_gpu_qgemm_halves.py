@@ -189,3 +189,38 @@ def test_digits_on_request_in_a_prompt_pass():
         tuned(0, 1)
     assert ran[2].startswith(PANEL) and ran[0] == "qgemm_q4_0_fx_kernel"
     assert np.array_equal(out[2].view(np.uint32), out[0].view(np.uint32))
+
+
+@pytest.mark.parametrize("prompt", [100, 40])
+def test_a_model_of_few_rows_holds_no_panel(prompt):
+    """Prompts of up to 256 rows are multiplied with W read where it lies: finalize allocates a workspace for shares' sums alone, not the 67 MB that gate's
+    and up's integers would be and 96 MiB of sums. 100 rows hold 10 + 6 MB of float32 and 12 MB of converted rows, sums of one round of
+    workgroups are 17 MB, and some twenty allocations may each end up to 2 MB further on: 64 MiB for 100 rows, 48 for 40."""
+    most_mib = 64 if prompt == 100 else 48
+    c = capi.LlamaConfig()
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = 2048, 8192, 1, 16, 4, 128, 128, 256
+    c.context, c.interleaved, c.cache_dtype, c.batch = prompt + 8, 1, capi.F16, 1
+    c.rope_base, c.rope_scale, c.eps = 10000.0, 1.0, 1e-5
+    m = Llama(c)
+    _upload_synthetic(m, OL.synthetic(_oracle_config(c), seed=5, output_dt=O.Q4_0))
+    held = []
+    for rows in (8, prompt):
+        gpu.say(f"finalize for {rows} rows")
+        m.finalize(rows)
+        gpu.sync()
+        held.append(torch.cuda.mem_get_info()[0])
+    assert held[0] - held[1] <= most_mib << 20, (held[0] - held[1]) / 2.0 ** 20
+    tokens = np.random.default_rng(2).integers(0, c.vocab, (1, prompt))
+    out = {}
+    try:
+        for pairs in (1, 0):
+            tuned(0, pairs)
+            m.reset()
+            out[pairs] = m.logits(tokens, all=True)
+            if pairs:
+                m.reset()
+                m.generate(tokens, 1)
+    finally:
+        tuned(0, 1)
+    scale = np.abs(out[0]).max()
+    assert np.median(np.abs(out[1] - out[0])) <= 1e-5 * scale and not np.array_equal(out[1], out[0])

@@ -124,17 +124,25 @@ def test_rows_held_by_block_among_others(m):
     assert min(took[1]) <= 1.5 * min(took[0]), (min(took[1]), min(took[0]))
 
 
-@pytest.mark.parametrize("batch,prompt,hidden", [(1, 150, 1088), (2, 24, 1024), (3, 100, 992)])
-def test_a_prompt_pass_with_products_taken_together(batch, prompt, hidden):
-    """A model whose q, k, v and whose gate and up (with SwiGLU) are one product each: column strips that no tile is filled by, K of
-    320 and of 1088, a down projection whose K (992) this form does not take. Against the oracle as the other prompt passes
-    are, and within 1e-5 of the largest logit of the int8 form's pass (both hold x to 2^-23 of a block's largest; no rounding step
-    between them, but the binary16 cache's)."""
+def prompt_model(batch, prompt, embed, hidden, heads, kv_heads, head_dim, layers):
     c = capi.LlamaConfig()
-    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = 320, hidden, 2, 5, 1, 64, 64, 515
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = embed, hidden, layers, heads, kv_heads, head_dim, head_dim, 515
     c.context, c.interleaved, c.cache_dtype, c.batch = prompt + 8, 1, capi.F32, batch
     c.rope_base, c.rope_scale, c.eps = 10000.0, 1.0, 1e-5
-    om = OL.synthetic(_oracle_config(c), seed=3, output_dt=O.Q4_0)
+    return c
+
+
+@pytest.mark.parametrize("batch,prompt,embed,hidden,heads,kv_heads,head_dim", [
+    (1, 150, 320, 1088, 5, 1, 64), (2, 24, 320, 1024, 5, 1, 64), (3, 100, 320, 992, 5, 1, 64),  # a down projection whose K (992) this form does not take
+    (1, 45, 320, 1088, 4, 1, 80),      # k and v of 80 rows: their last strips are half of the next one's place
+    (1, 37, 1024, 4096, 8, 2, 128),    # shares of K, W read where it lies
+    (2, 150, 1024, 4096, 8, 2, 128)])  # and by the panel
+def test_a_prompt_pass_with_products_taken_together(batch, prompt, embed, hidden, heads, kv_heads, head_dim):
+    """A model whose q, k, v and whose gate and up (with SwiGLU) are one product each: column strips that no tile is filled by, K of 320 and of 1088, shares of K.
+    Nothing on the way rounds to int8 or binary16, so that the passes as pairs and in fixed point, and the oracle's, differ by float32 rounding and by what
+    x is held to (2^-23 of a block's largest) alone: some 1e-6 of the largest logit after two layers; every logit of every sequence within 1e-5."""
+    c = prompt_model(batch, prompt, embed, hidden, heads, kv_heads, head_dim, 2)
+    om = OL.synthetic(_oracle_config(c), seed=3, output_dt=O.Q4_0, centered=True)
     m = Llama(c)
     _upload_synthetic(m, om)
     m.finalize(prompt)
@@ -142,16 +150,46 @@ def test_a_prompt_pass_with_products_taken_together(batch, prompt, hidden):
     out = {}
     try:
         for pairs in (3, 0):
-            gpu.say(f"prompt pass batch={batch} prompt={prompt} hidden={hidden} pairs={pairs}")
+            gpu.say(f"prompt pass batch={batch} prompt={prompt} embed={embed} hidden={hidden} pairs={pairs}")
             tuned(0, pairs)
             m.reset()
             out[pairs] = m.logits(tokens, all=True)
     finally:
         tuned(0, 1)
+    assert not np.array_equal(out[3], out[0])
+    scale = np.abs(out[0]).max()
+    assert np.abs(out[3] - out[0]).max() <= 1e-5 * scale, np.abs(out[3] - out[0]).max() / scale
+    for b in range(batch):
+        want = om.logits(tokens[b].tolist(), om.new_caches(c.context, O.F32), all=True)
+        assert np.abs(out[3][b] - want).max() <= 1e-5 * scale, np.abs(out[3][b] - want).max() / scale
+
+
+@pytest.mark.parametrize("rows,embed,hidden,kernel", [
+    (37, 1024, 4096, IN_PLACE + "<2>: 1 x 64 tiles, 4 shares of K"), (77, 2048, 8192, IN_PLACE + "<3>: 1 x 128 tiles, 2 shares of K"),
+    (100, 320, 992, IN_PLACE + "<4>: 1 x 16 tiles, 1 shares of K"), (300, 1024, 4096, PANEL + "3 x 32 tiles of 128 x 256, 2 shares of K"),
+    (300, 320, 992, PANEL + "3 x 8 tiles of 128 x 256")])
+def test_gate_and_up_are_one_product(rows, embed, hidden, kernel):
+    """Where the down projection and the output are of Q8_0, whose kernels leave no name, the name of the pass is gate's and up's: one product of both
+    matrices' strips (twice `hidden`), cut as asked. SwiGLU in the tile where K is whole, with the shares' sums where it is not; results against the oracle, whose
+    int8 roundings may fall on the other side here and there (test_gpu_llama.py)."""
+    c = prompt_model(1, rows, embed, hidden, 5 if embed == 320 else embed // 128, 1, 64 if embed == 320 else 128, 1)
+    om = OL.synthetic(_oracle_config(c), seed=6, centered=True)
+    om.blocks[0].down = OL._q_blocks(np.random.default_rng(8), O.Q8_0, embed, hidden)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(rows)
+    tokens = np.random.default_rng(1).integers(0, c.vocab, (1, rows))
+    try:
+        gpu.say(f"gate and up rows={rows} embed={embed} hidden={hidden}")
+        tuned(0, 3)
+        got = m.logits(tokens, all=True)[0]
+        ran = last_kernel()
+    finally:
+        tuned(0, 1)
+    assert ran == kernel
     want = om.logits(tokens[0].tolist(), om.new_caches(c.context, O.F32), all=True)
     scale = np.abs(want).max()
-    assert np.abs(out[3][0] - want).max() <= 0.02 * scale and np.median(np.abs(out[3][0] - want)) <= 1e-5 * scale
-    assert np.median(np.abs(out[3] - out[0])) <= 1e-5 * scale and np.abs(out[3] - out[0]).max() <= 0.02 * scale
+    assert np.abs(got - want).max() <= 0.02 * scale and np.median(np.abs(got - want)) <= 1e-5 * scale
 
 
 @pytest.mark.parametrize("m,n,k,in_place", [(24, 8192, 14336, False), (20, 14336, 11008, False), (17, 8192, 11008, False), (24, 14336, 8192, False),

@@ -1,4 +1,5 @@
-// What the two kernels share that multiply x as pairs of binary16 by Q4_0 weights (qgemm_q4_0_fx16.hip, qgemm_q4_0_direct.hip).
+// What the kernels share that multiply many rows by Q4_0 weights: x as pairs of binary16 (qgemm_q4_0_fx16.hip, qgemm_q4_0_direct.hip) or
+// bfloat16 as it is (qgemm_q4_0_blocks.hip).
 #pragma once
 #include "device_util.h"
 
@@ -133,6 +134,25 @@ __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t lo, uint32_t hi, int ha
         v[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, p1) - off);
     }
     return __builtin_bit_cast(f16x8, v);
+}
+
+// A KB from global memory into LDS: lane l's 16 bytes from base + 16 l to lds_base + 16 l. Written out because the
+// compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand
+// (the compiler does not see them, so its own waits for the register loads of the scales can only be longer than
+// needed, never shorter: loads return in order). The instruction takes its LDS base from M0, which an asm statement
+// cannot name as clobbered: nothing else in these kernels uses M0, and it is set anew before every load.
+__device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane16, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A die's workgroups (every eighth, round-robin) take a contiguous range of the tiles, the tile's rows of x varying
+// fastest: those that run together share few column panels of P through the die's L2.
+__device__ __forceinline__ int tile_of(int b, int ntiles) {
+    const int per_die = (ntiles + 7) >> 3;
+    return (b & 7) * per_die + (b >> 3);
 }
 
 // The shares' sums of K, in their order: y = ((s0 + s1) + ..) (+ resid), or silu(gate) up of them.

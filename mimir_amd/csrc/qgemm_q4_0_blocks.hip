@@ -108,24 +108,6 @@ __global__ __launch_bounds__(256) void blocks_panel_kernel(const uint8_t* __rest
     }
 }
 
-// A KB from global memory into LDS: lane l's 16 bytes from base + 16 l to lds_base + 16 l. Written out because the
-// compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand.
-// The instruction takes its LDS base from M0, which an asm statement cannot name as clobbered: nothing else in this
-// kernel uses M0, and it is set anew before every load.
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane16, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// A die's workgroups (every eighth, round-robin) take a contiguous range of the tiles, the tile's rows of X varying
-// fastest: those that run together share few column panels of P through the die's L2.
-__device__ __forceinline__ int tile_of(int b, int ntiles) {
-    const int per_die = (ntiles + 7) >> 3;
-    return (b & 7) * per_die + (b >> 3);
-}
-
 // One tile: Y [m0 .. m0 + BM) x [n0 .. n0 + BN).
 template <class S, bool OUT_F32>
 __device__ __forceinline__ void tile_body(const uint16_t* __restrict__ P, const uint16_t* __restrict__ XG, const float* __restrict__ SW, void* __restrict__ Yv,

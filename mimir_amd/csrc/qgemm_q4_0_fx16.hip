@@ -1,13 +1,14 @@
 // The Q4_0 product of many rows of float32 x, from some tens of rows on, on the binary16 matrix cores. x enters as a pair of
-// binary16 numbers an element, x 2^-e = h0 + h1 (22 bits; e the row's exponent), W as the integers n - 8, whose scales stay
+// binary16 numbers an element, x 2^-e = h0 + h1 (to 2^-23 of the element; e the row's exponent), W as the integers n - 8, whose scales stay
 // out of the matrix cores: v_mfma_f32_32x32x16_f16 sums a block's products of h1 and of h0 (exact, added in float32) into
 // one c, and acc = fma(d, c, acc) is left to the vector unit, one instruction per output and block; 2^e follows at the end.
 //
 // What bounds it: four MFMAs of 32 cycles and sixteen FMAs of 4 per 32 x 32 outputs and block of 32, which hardly overlap
 // on a SIMD (128 + 64 cycles; one wide tile alone takes 1.3 us a block, those cycles at the full clock; with every unit at work
-// the clock falls and it is 1.75 us). The form before this one, which the int8 form's bits need (x as two 12-bit integer
-// digits with a float32 scale a block: two sums, an MFMA for dw dx and two FMAs an output: 128 + 32 + 128 cycles), stays for
-// "q4_0.fx_pairs" = 2. Whole calls, conversion and the pass over W included, digits before and halves now:
+// the clock falls and it is 1.75 us). The form with the int8 form's bits (x as two 12-bit integer
+// digits with a float32 scale a block: two sums, an MFMA for dw dx and two FMAs an output: 128 + 32 + 128 cycles) is taken where mi355x_qgemv_noalloc
+// multiplies in that form. Whole calls, conversion and the pass over W included, fifty of a shape back to back (among other shapes, as bench.py has them, a
+// tenth more: 498 us for the first), digits and halves:
 //   2048 x 14336 x 4096   647 -> 461 us (521 TFLOP/s)      4096 x 28672 x 4096   2430 -> 1667 us (577 TFLOP/s)
 //   4096 x 4096 x 14336  1286 -> 910 us                    512 x 4096 x 14336    506 (int8 268) -> 155 us
 //   2048 x 4096 x 4096    184 -> 149 us                    512 x 14336 x 4096    183 -> 149 us
@@ -23,7 +24,7 @@
 //
 // Several matrices by the same x (q, k and v; gate and up, SwiGLU included) are one product: Parts.
 //
-// Reference semantics: the float32 product with the dequantized weights (io/mim/dtype.go:118-123,
+// Reference semantics: the float32 product with the dequantized weights (io/mim/dtype.go:118-123).
 #include "device_util.h"
 #include "kernels.h"
 #include "q4_act.h"
@@ -90,9 +91,11 @@ __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restric
 }
 
 // A workgroup converts a row of x into halves: x 2^-e = h0 + h1, h0 the binary16 next to it and h1 the binary16 next to
-// what that leaves. e makes the row's largest element lie in [2^14, 2^15), so that an element keeps 22 bits, and at least
-// an absolute 2^-25: 2^-24 of its block's largest as long as that is no less than 2^-15 of the row's, about what the
-// fixed point holds (2^-23.9). A row that has a smaller block (zeros aside) takes an exponent a block instead.
+// what that leaves. An element is held to 2^-23 of itself (of float32's 24 bits the last may go: 2^14 + 8 - 2^-9 leaves 8 - 2^-9, which h1 rounds by
+// 2^-9). e makes the row's largest element lie in [2^14, 2^15), where h1's smallest step, 2^-24, is below that bound down to
+// 2^-2, and holds what is smaller to 2^-25: to 2^-24 of its block's largest as long as that is no less than 2^-15 of the row's. The fixed point
+// holds every element to 2^-23.9 of its block's largest, that is most of them to less: its error over normal x is twice the pairs'. A row that has a
+// smaller block (zeros aside) takes an exponent a block instead.
 // With NORM the row is normalized first (rmsnorm_kernel's operations, one by one): x over its root mean square, times w.
 // Memory bounds it: 8 bytes an element. ITEMS: eights of elements a thread holds between the row's maximum and its halves, so that x
 // is read once (4096 rows of 14336: 105 us, 156 reading it twice and storing eight bytes a thread); 0: rows of more than 16384, read twice.
@@ -232,25 +235,6 @@ __global__ __launch_bounds__(256) void fx16_panel_kernel(Parts parts, uint16_t* 
         for (int half = 0; half < 2; half++) *(f16x8*)(out + 512 * half) = nibbles_to_f16(pair[i / 2].lo[i & 1], pair[i / 2].hi[i & 1], half);
         if (q == 0) SW[((int64_t)strip * scale_blocks(nb) + b) * kGranuleS + r] = f16_bits_to_f32((uint16_t)(pair[i / 2].scale[i & 1] ^ ((b & 1) << 15)));
     }
-}
-
-// A KB from global memory into LDS: lane l's 16 bytes from base + 16 l to lds_base + 16 l. Written out because the
-// compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand
-// (the compiler does not see them, so its own waits for the register loads of the scales can only be longer than
-// needed, never shorter: loads return in order). The instruction takes its LDS base from M0, which an asm statement
-// cannot name as clobbered: nothing else in this kernel uses M0, and it is set anew before every load.
-__device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane16, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// A die's workgroups (every eighth, round-robin) take a contiguous range of the tiles, the tile's rows of x varying
-// fastest: those that run together share few column panels of P through the die's L2.
-__device__ __forceinline__ int tile_of(int b, int ntiles) {
-    const int per_die = (ntiles + 7) >> 3;
-    return (b & 7) * per_die + (b >> 3);
 }
 
 // A workgroup's tile of y: WM x (8 / WM) wavefronts of (32 MT) x (32 NT) each, over STAGES stages of one block.
@@ -618,8 +602,9 @@ hipError_t sum_shares(const Operands& o, int shares, hipStream_t st) {
 }
 
 // Whether the product is the faster here than in the int8 form (qgemm_q4_0_fx_cost_us). mi355x_qgemv cuts K into shares of
-// no less than 96 blocks: 512 x 4096 x 4096 stays with the int8 form there (88 us, in one pass here 114), which
-// tests/test_gpu_qgemm_fx.py holds it to; 512 x 14336 x 4096 comes here (151 us, 217 in the int8 form).
+// no less than 96 blocks: 512 x 4096 x 4096 stays with the int8 form there (88 us, in one pass here 114; 512 x 14336 x 4096 comes here: 151 us, 217
+// in the int8 form). That line is one of results and not of time: up to there a product of float32 x has the int8 form's bits, which
+// tests/test_gpu_qgemm_fx.py names; in shares of 16 blocks, as the decoder has it, 512 x 4096 x 4096 takes some 65 us.
 constexpr int64_t kMinShareBlocks = 96;
 
 double qgemm_q4_0_fx16_cost_us(int64_t M, int64_t N, int64_t K) {

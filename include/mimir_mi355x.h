@@ -166,8 +166,8 @@ MI355X_API mi355x_status mi355x_qgemv_act(int dtype, const void* W, const void* 
  * rounding). Q4_0 runs on the bfloat16 matrix cores without rounding any
  * operand (each weight as two bfloat16 halves; or, for large products, the
  * weights' integers against x block by block and one float32 FMA per block with
- * the block's scale, which takes a workspace of 2 N K bytes in the stream's
- * scratch), when K is a multiple of 256, X and W are 16-byte aligned
+ * the block's scale, which takes a workspace of 2 K (M + N) bytes and 4 bytes a
+ * block of W in the stream's scratch), when K is a multiple of 256, X and W are 16-byte aligned
  * and rows of X are a multiple of 8 elements apart; otherwise, and for the other
  * dtypes, X goes through mi355x_qgemv as float32. Q4_K and Q6_K then run on
  * the int8 matrix cores from a few rows of X on, with the CPU's results bit for

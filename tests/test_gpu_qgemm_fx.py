@@ -108,7 +108,8 @@ def last_kernel():
 
 def pairs_and_int8(raw, x_dev, n, k):
     """The same product from 256 rows on in its two forms: 12-bit digit pairs on the binary16 matrix cores (the
-    library's choice for large products; "q4_0.fx_pairs" = 2 asks for it whatever the shape), and the int8 form
+    library's choice for products by large matrices whose rows mi355x_qgemv_noalloc takes; "q4_0.fx_pairs" = 2 asks
+    for it whatever the shape), and the int8 form
     ("q4_0.fx_pairs" = 0). Returns both and the kernels that ran."""
     l = gpu.lib()
     buf, ptr = gpu.dev_bytes_at(raw, 0)

@@ -145,7 +145,7 @@ void set_kquant_tune(int which, int value);
 // the kernel takes the shape).
 bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a);
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a);
-hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st);
+hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);
 // With the rotation and the cache writes of a decoding step as its tail (y receives the rotated queries only).
 bool qgemv_kquant_rows_rope_ok(int dt, const QGemvArgs& a);
 hipError_t qgemv_kquant_rows_rope(int dt, const QGemvArgs& a, const Q4RopeTail& rope, hipStream_t st);

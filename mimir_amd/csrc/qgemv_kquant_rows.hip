@@ -9,21 +9,25 @@
 //   dd = d_w d_x, dm = dmin_w d_x, acc += dd float(sumi), accm += dm float(summ)
 // over the super-blocks in order, and acc - accm at the end.
 //
-// x comes rounded to int8 per super-block (kq_convert_act: quants, sums of 16,
-// scale). A sub-block is 32 weights: the K of one v_mfma_i32_32x32x32_i8, whose
-// first operand holds the eight rows of x (8 of its 32 rows) and whose second
-// 32 rows of W as their nibbles 0..15. A lane ends up with its row of W's
-// sub-block sums for four rows of x; the scales are per lane, so sc_j times the
-// sum is one multiply-add, and m_j times the two sums of 16 one v_dot2.
+// x comes rounded to int8 per super-block (kq_convert_act: quants, sums of 16, scale).
 //
-// A workgroup of four or eight wavefronts owns 32 rows of W; its wavefronts take
-// the super-blocks round robin and leave their float32 terms per output (two
-// for Q4_K, one for Q6_K) in LDS; when all are there the first wavefront adds
-// them in the super-blocks' order, which is the CPU's. (Long rows: contiguous
-// runs of super-blocks, terms in registers, the sums handed from wavefront to
-// wavefront in that order; see the kernel.) x of a super-block (2.6 KB for eight
-// rows) and W of it (32 rows, loaded as whole cache lines) pass through LDS that
-// is the wavefront's own, so no barrier but those around the sums.
+// What bounds it is W's way into the matrix core's operands. Neighbouring lanes hold neighbouring rows there, and a load whose
+// lanes touch a line each costs the cache 64 lookups (x and W loaded so, 4096 x 14336: 16 us), so both come as rows, 16 bytes a lane, and change
+// lanes in LDS that is the wavefront's own: no barrier but the one before the sums. A workgroup owns sixteen rows of W, so that a
+// matrix of 4096 rows has one for every compute unit, in up to sixteen wavefronts, which take the super-blocks round robin and have all or
+// most of theirs under way from the start: with one ahead every second super-block cost a trip to memory. Matrices with
+// more rows take two tiles of sixteen a workgroup, which share the operand of x.
+//
+// The operands are sixteen rows wide: column n of the second is row n of W, row 8 c + m of the first is row m of x with everything but
+// group c of the weights zeroed, c = 0 or 1 (those lanes read zeros kept in LDS), so that one instruction keeps two groups of
+// weights with scales of their own apart. A lane then has one group's sums for its row of W and four rows of x, times its
+// scale; two exchanges between the wavefront's halves add the groups and leave a lane two rows' integer sums. The float32
+// terms of all super-blocks meet in LDS, and one thread per output adds them in the super-blocks' order, which is the CPU's.
+//
+// Measured, us a call on rows already converted, eight rows of x, the form before it (32 rows of W a workgroup in four or eight wavefronts, one
+// super-block ahead) and this one: Q4_K 4096 x 14336 20.2 12.2 (loads alone 9.6), 2048 x 8192 10.4 6.4, 6144 x 4096 8.5 6.8, 4096 x 4096 7.0 4.9,
+// 28672 x 4096 22.6 20.2-22.5 (66 MB: 3.1 TB/s); Q6_K 4096 x 14336 26.6 14.7 (48 MB: 3.3 TB/s), 2048 x 8192 16.7 9.0, 4096 x 4096
+// 11.0 6.1, 28672 x 4096 31.5 26.2-28.7.
 #include "device_util.h"
 #include "kernels.h"
 #include "rope_tail.h"
@@ -35,86 +39,103 @@ namespace mimir {
 namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 8;                        // rows of x a group holds
-// A super-block of x for eight rows in LDS: quants [8][256] with rows 288 bytes apart (72 dwords: the sixteen 16-byte pieces the
-// lanes of a matrix-core operand read, eight rows by two halves, fall on all 64 banks; 256 apart they would share four), sums [8][16]
-// int16, scales [8].
-constexpr int kXRow = 288;
-constexpr int kXq = 0, kXs = 8 * kXRow, kXd = kXs + 256;
-constexpr int kXBytes = kXd + 32;
+constexpr int kRows = 8;    // rows of x a group holds
+constexpr uint32_t kBeyond = 1u << 30;  // an offset, or a bit of one, past every buffer's end: the load gives zeros and touches no memory
 
-// scale_min_k4 (backend/cpu/quant.go:129-134) on the twelve scale bytes held as three dwords.
-__device__ __forceinline__ int q4k_sc(uint32_t s0, uint32_t s2, int j) {
-    const int sh = 8 * (j & 3);
-    return j < 4 ? (int)((s0 >> sh) & 63) : (int)(((s2 >> sh) & 0xf) | (((s0 >> (sh + 6)) & 3) << 4));
-}
-__device__ __forceinline__ int q4k_mn(uint32_t s1, uint32_t s2, int j) {
-    const int sh = 8 * (j & 3);
-    return j < 4 ? (int)((s1 >> sh) & 63) : (int)(((s2 >> (sh + 4)) & 0xf) | (((s1 >> (sh + 6)) & 3) << 4));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
 }
 
-// W comes through LDS: a wavefront loads a super-block of its 32 rows as 16-byte pieces in row order (consecutive lanes, consecutive
-// pieces of a row: whole cache lines per request, where a load of a lane's own row would touch 64 lines for 16 bytes each and wait for
-// the cache's tag lookups), stores them into a slab of its own and reads its row's pieces back. WBlock<DT> says how a row's
-// super-block is cut into pieces and makes the float32 terms of a lane's four rows of x from its row in the slab (wl) and the
-// super-block of x in LDS (xl).
+// The sums of lanes 32 apart: lanes of the lower half get v[0] and v[1] of both, lanes of the upper half v[2] and v[3].
+__device__ __forceinline__ void add_halves(const int v[4], int out[2]) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v[i], (uint32_t)v[i + 2], false, false);
+        const uint32_t a = r[0], b = r[1];
+        out[i] = (int)(a + b);
+    }
+}
+
+// Lane numbers: r = lane % 16 is a lane's row of W (and of the first operand: row r % 8 of x, group r / 8), g = lane / 16 its
+// quarter of an instruction's K, and of the result rows 4 g..4 g + 3.
+//
+// A super-block of x in a wavefront's LDS: 256 bytes of zeros (where the lanes of the other group read), quants [8][256] with rows 288
+// bytes apart (72 dwords: the eight rows that the lanes of a quarter read fall on different banks), sums [8][16] int16.
+constexpr int kXRow = 288, kXq = 256, kXs = kXq + 8 * kXRow, kXBytes = kXs + 256;
+
+// WBlock<DT> says how a row's super-block is cut into 16-byte pieces; operands() reads x's part of the products from LDS, terms() makes the
+// float32 terms of row r of W (wl: its super-block in LDS) with rows 4 (g % 2) + 2 (g / 2) and the one after it of x, whose scales are xd.
 template <int DT> struct WBlock;
 
+// A 144-byte block is d, dmin, twelve bytes of scales (scale_min_k4, backend/cpu/quant.go:129-134), then four groups of 32 bytes whose
+// low nibbles are sub-block 2 p and high nibbles sub-block 2 p + 1. An instruction takes the low (or the high) nibbles of
+// two groups, 2 pp and 2 pp + 1: sixteen bytes a lane, 64 in a row of W. The mins' sum m_j (sums of 16) is one
+// v_mfma_f32_16x16x16_f16 over the sixteen sums: integers below 2^11 and 2^6, exact, as is their sum.
 template <> struct WBlock<kQ4_K> {
     static constexpr int kBytes = 144, kTerms = 2;
-    static constexpr int kPieces = 9, kStride = 144;  // rows 36 dwords apart: the 16 lanes of a 128-bit read's phase fall on all 64 banks
+    static constexpr int kPieces = 9, kStride = 144;  // rows 36 dwords apart: the 16 lanes of a quarter fall on all 64 banks
     __device__ __forceinline__ static int piece_offset(int c) { return 16 * c; }
+    i32x4 x[2][2];
+    f16x4 sums;
+    __device__ __forceinline__ void operands(const uint8_t* xl, uint32_t r, uint32_t g) {
+        const uint8_t* xa = (g >> 1) == (r >> 3) ? xl + kXq + (r & 7) * kXRow + 64 * (g >> 1) + 16 * (g & 1) : xl;
+#pragma unroll
+        for (int pp = 0; pp < 2; pp++)
+#pragma unroll
+            for (int hi = 0; hi < 2; hi++) x[pp][hi] = *(const i32x4*)(xa + 128 * pp + 32 * hi);
+        const u32x2 sv = *(const u32x2*)(xl + kXs + (r & 7) * 32 + 8 * g);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t v = sv[i >> 1];
+            sums[i] = (_Float16)(int16_t)(v >> (16 * (i & 1)));
+        }
+    }
     // t[0] = d_w d_x float(sumi), t[1] = dmin_w d_x float(summ)
-    __device__ __forceinline__ static void terms(const uint8_t* wl, const uint8_t* xl, int l32, int lh, f32x4* t) {
-        const u32x4 hdr = *(const u32x4*)wl;  // d, dmin, scales
-        const uint8_t* xrow = xl + kXq + (l32 & 7) * kXRow + 16 * lh;  // this lane's operand row of x (rows 8.. of the operand repeat rows 0..7)
+    __device__ __forceinline__ void terms(const uint8_t* wl, const float xd[2], uint32_t g, float t[kTerms][2]) const {
+        const u32x4 hdr = *(const u32x4*)wl;
+        u32x4 q[2];
+#pragma unroll
+        for (int pp = 0; pp < 2; pp++) q[pp] = *(const u32x4*)(wl + 16 + 64 * pp + 16 * g);
         const uint32_t s0 = hdr[1], s1 = hdr[2], s2 = hdr[3];
-        int sumi[4] = {0, 0, 0, 0}, summ[4] = {0, 0, 0, 0};
-        // the sums of 16 of this lane's four rows of x: dword c holds chunks 2c and 2c + 1
-        u32x4 sv[4][2];
+        // scales and mins 0..3 and 4..7, a byte each
+        const uint32_t sc0 = s0 & 0x3f3f3f3fu, sc1 = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
+        const uint32_t mn0 = s1 & 0x3f3f3f3fu, mn1 = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
+        int sumi[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            sv[jj][0] = *(const u32x4*)(xl + kXs + (4 * lh + jj) * 32);
-            sv[jj][1] = *(const u32x4*)(xl + kXs + (4 * lh + jj) * 32 + 16);
-        }
-        const f32x4 xd = *(const f32x4*)(xl + kXd + 16 * lh);
+        for (int pp = 0; pp < 2; pp++) {
+            const uint32_t sc = (pp ? sc1 : sc0) >> (16 * (g >> 1));  // sub-blocks 4 pp + 2 c and the one after it, c = g / 2
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const u32x4 q = *(const u32x4*)(wl + 16 + 32 * g + 16 * lh);  // the lane's 16 bytes of nibbles of group g
-            i32x4 wlo, whi;
+            for (int hi = 0; hi < 2; hi++) {
+                i32x4 w;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                wlo[i] = (int)(q[i] & 0x0F0F0F0Fu);
-                whi[i] = (int)((q[i] >> 4) & 0x0F0F0F0Fu);
-            }
-            const i32x4 xa = *(const i32x4*)(xrow + 64 * g), xb = *(const i32x4*)(xrow + 64 * g + 32);
-            i32x16 zero;
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t qv = q[pp][i];
+                    w[i] = (int)((hi ? qv >> 4 : qv) & 0x0F0F0F0Fu);
+                }
+                const i32x4 c = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[pp][hi], w, i32x4{0, 0, 0, 0}, 0, 0, 0);
+                const int s = (int)((sc >> (8 * hi)) & 0xff);
 #pragma unroll
-            for (int i = 0; i < 16; i++) zero[i] = 0;
-            const i32x16 ca = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa, wlo, zero, 0, 0, 0);
-            const i32x16 cb = __builtin_amdgcn_mfma_i32_32x32x32_i8(xb, whi, zero, 0, 0, 0);
-            const int sca = q4k_sc(s0, s2, 2 * g), scb = q4k_sc(s0, s2, 2 * g + 1);
-            const int ma = q4k_mn(s1, s2, 2 * g), mb = q4k_mn(s1, s2, 2 * g + 1);
-            const uint32_t ma2 = (uint32_t)ma * 0x00010001u, mb2 = (uint32_t)mb * 0x00010001u;
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++) {
-                // 24-bit multiplies (full rate; a 32-bit one takes four times as long): |sum| <= 32 * 15 * 127, scales below 64
-                sumi[jj] += __mul24(sca, ca[jj]) + __mul24(scb, cb[jj]);
-                // sub-block 2g is chunks 4g, 4g + 1 (dword 2g of the sums), sub-block 2g + 1 chunks 4g + 2, 4g + 3
-                const uint32_t pa = sv[jj][g >> 1][2 * (g & 1)], pb = sv[jj][g >> 1][2 * (g & 1) + 1];
-                summ[jj] = __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, pa), __builtin_bit_cast(s16x2, ma2), summ[jj], false);
-                summ[jj] = __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, pb), __builtin_bit_cast(s16x2, mb2), summ[jj], false);
+                for (int i = 0; i < 4; i++) sumi[i] += __mul24(s, c[i]);  // 24-bit multiplies: |sum| <= 32 * 15 * 127
             }
         }
-        const float dw = f16_bits_to_f32((uint16_t)hdr[0]), dmin = f16_bits_to_f32((uint16_t)(hdr[0] >> 16));
+        // mins 2 g and 2 g + 1 as binary16: the sums of 16 number 4 g.. are theirs
+        const uint32_t mn = (g & 2 ? mn1 : mn0) >> (16 * (g & 1));
+        f16x4 b;
+        b[0] = b[1] = (_Float16)(uint16_t)(mn & 0xff);
+        b[2] = b[3] = (_Float16)(uint16_t)((mn >> 8) & 0xff);
+        const f32x4 cm = __builtin_amdgcn_mfma_f32_16x16x16f16(sums, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        int two[2];
+        add_halves(sumi, two);
+        const uint32_t dd = hdr[0];
+        const float dw = f16_bits_to_f32((uint16_t)dd), dmin = f16_bits_to_f32((uint16_t)(dd >> 16));
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const float dd = dw * xd[jj], dm = dmin * xd[jj];
-            t[0][jj] = dd * (float)sumi[jj];
-            t[1][jj] = dm * (float)summ[jj];
+        for (int i = 0; i < 2; i++) {
+            const float d = dw * xd[i], dm = dmin * xd[i];
+            t[0][i] = d * (float)two[i];
+            t[1][i] = dm * (g & 2 ? cm[2 + i] : cm[i]);
         }
     }
 };
@@ -123,60 +144,58 @@ template <> struct WBlock<kQ4_K> {
 // 16-byte loads are unaligned ones: thirteen pieces from the block's start and a fourteenth over its last 16 bytes (194..209), which
 // lands behind them in the slab (bytes 208..223 of the row there: the scale d at 222). Half h2 of a super-block (128 weights) is 64
 // bytes of ql and 32 of qh: slab s = 0..3 of the half (32 weights) has its low four bits in the low (s < 2) or high nibbles of
-// ql[64 h2 + 32 (s & 1) ..] and its upper two at bit 2 s of qh[32 h2 ..]; a scale per chunk of 16, a zero point of 32. The matrix-core
-// product must keep the two chunks of a slab apart: the operand's row 8 c + m holds row m of x with everything but chunk c of the slab
-// zeroed, so the result's rows 0..7 are chunk 0's sums and rows 8..15 chunk 1's (rows 16..31 are unused).
+// ql[64 h2 + 32 (s & 1) ..] and its upper two at bit 2 s of qh[32 h2 ..]; a scale per chunk of 16, a zero point of 32. An instruction
+// takes a slab, eight weights a lane, its two chunks as the two groups. The operand is 4 (q - 32), an int8 (the zero point is a bit
+// turned, the shift by two an alignment of the two fields), so the sums of 16 are not needed; the integer sum is shifted
+// back at the end, exactly.
 template <> struct WBlock<kQ6_K> {
     static constexpr int kBytes = 210, kTerms = 1;
     static constexpr int kPieces = 14, kStride = 240;  // 60 dwords: as above
     __device__ __forceinline__ static int piece_offset(int c) { return c < 13 ? 16 * c : 194; }
-    // t[0] = d_w d_x float(sum over the chunks of sc (q . x - 32 sum of x))
-    __device__ __forceinline__ static void terms(const uint8_t* wl, const uint8_t* xl, int l32, int lh, f32x4* t) {
-        const bool keep = (l32 >> 3) == lh;  // operand rows 0..7 keep the first 16 of a slab (held by lanes of half 0), rows 8..15 the second
-        const uint8_t* xrow = xl + kXq + (l32 & 7) * kXRow + 16 * lh;
-        int sumi[4] = {0, 0, 0, 0}, summ[4] = {0, 0, 0, 0};
-        u32x4 sv[4][2];
+    u32x2 x[2][4];
+    __device__ __forceinline__ void operands(const uint8_t* xl, uint32_t r, uint32_t g) {
+        const uint8_t* xa = (g >> 1) == (r >> 3) ? xl + kXq + (r & 7) * kXRow + 8 * g : xl;
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            sv[jj][0] = *(const u32x4*)(xl + kXs + (4 * lh + jj) * 32);
-            sv[jj][1] = *(const u32x4*)(xl + kXs + (4 * lh + jj) * 32 + 16);
-        }
-        const f32x4 xd = *(const f32x4*)(xl + kXd + 16 * lh);
+        for (int h2 = 0; h2 < 2; h2++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) x[h2][s] = *(const u32x2*)(xa + 128 * h2 + 32 * s);
+    }
+    // t[0] = d_w d_x float(sum over the chunks of sc (q - 32) . x)
+    __device__ __forceinline__ void terms(const uint8_t* wl, const float xd[2], uint32_t g, float t[kTerms][2]) const {
         const u32x4 sc = *(const u32x4*)(wl + 192);
+        int sumi[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int h2 = 0; h2 < 2; h2++) {
-            const u32x4 ql[2] = {*(const u32x4*)(wl + 64 * h2 + 16 * lh), *(const u32x4*)(wl + 64 * h2 + 32 + 16 * lh)};
-            const u32x4 qh = *(const u32x4*)(wl + 128 + 32 * h2 + 16 * lh);
+            const u32x2 ql[2] = {*(const u32x2*)(wl + 64 * h2 + 8 * g), *(const u32x2*)(wl + 64 * h2 + 32 + 8 * g)};
+            const u32x2 qh = *(const u32x2*)(wl + 128 + 32 * h2 + 8 * g);
+            uint32_t up[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) up[i] = qh[i] ^ 0xAAAAAAAAu;  // bit 5 of every weight turned: q - 32
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                i32x4 w, xa = *(const i32x4*)(xrow + 128 * h2 + 32 * s);
+                uint32_t w[2], xa[2];
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t lo = (ql[s & 1][i] >> (s & 2 ? 4 : 0)) & 0x0F0F0F0Fu, hi = (qh[i] >> (2 * s)) & 0x03030303u;
-                    w[i] = (int)(lo | (hi << 4));  // 0..63
-                    xa[i] = keep ? xa[i] : 0;
+                for (int i = 0; i < 2; i++) {
+                    const uint32_t lo = ql[s & 1][i];
+                    w[i] = ((s < 2 ? lo << 2 : lo >> 2) & 0x3C3C3C3Cu) | ((s < 3 ? up[i] << (6 - 2 * s) : up[i]) & 0xC0C0C0C0u);
+                    xa[i] = x[h2][s][i];
                 }
-                i32x16 zero;
+                const i32x4 c = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)xa[1] << 32) | xa[0]), (long)(((uint64_t)w[1] << 32) | w[0]),
+                                                                      i32x4{0, 0, 0, 0}, 0, 0, 0);
+                // the scale of chunk 8 h2 + 2 s + c, c = g / 2
+                const uint32_t sd = sc[2 * h2 + (s >> 1)] >> (8 * (g >> 1));
+                const int scale = (int)(int8_t)(sd >> (16 * (s & 1)));
 #pragma unroll
-                for (int i = 0; i < 16; i++) zero[i] = 0;
-                const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa, w, zero, 0, 0, 0);
-                // the scales of chunks 8 h2 + 2 s and + 1: bytes 2 (s & 1), 2 (s & 1) + 1 of dword 2 h2 + s / 2
-                const uint32_t sd = sc[2 * h2 + (s >> 1)];
-                const int sca = (int)(int8_t)(sd >> (16 * (s & 1))), scb = (int)(int8_t)(sd >> (16 * (s & 1) + 8));
-                const uint32_t pair = ((uint32_t)sca & 0xffffu) | ((uint32_t)scb << 16);
-#pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    sumi[jj] += __mul24(sca, c[jj]) + __mul24(scb, c[4 + jj]);  // |sum| <= 16 * 63 * 127, int8 scales
-                    const uint32_t ps = sv[jj][h2][s];  // a copy: __builtin_bit_cast of a vector's element takes element 0 with this compiler
-                    summ[jj] = __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, ps), __builtin_bit_cast(s16x2, pair), summ[jj], false);
-                }
+                for (int i = 0; i < 4; i++) sumi[i] += __mul24(scale, c[i]);  // |c| <= 16 * 128 * 127, times 128, sixteen times: below 2^30
             }
         }
+        int two[2];
+        add_halves(sumi, two);
         const float dw = f16_bits_to_f32(*(const uint16_t*)(wl + 222));
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const float dd = dw * xd[jj];
-            t[0][jj] = dd * (float)(sumi[jj] - 32 * summ[jj]);
+        for (int i = 0; i < 2; i++) {
+            const float dd = dw * xd[i];
+            t[0][i] = dd * (float)(two[i] >> 2);
         }
     }
 };
@@ -185,177 +204,154 @@ template <> struct WBlock<kQ6_K> {
 template <int LOADS> struct Stage {
     u32x4 w[LOADS];
     u32x4 xq[2];  // two 16-byte pieces of the eight rows' quants
-    u32x4 xs;     // a piece of their sums (lanes 0..15 store theirs)
-    float xd;     // a row's scale (lanes 0..7 store theirs)
+    u32x4 xs;     // a piece of their sums (lanes 0..15 store theirs; Q4_K)
+    float xd[2];  // the scales of the rows whose terms this lane makes
 };
 
-// CHAIN > 0: a wavefront takes a contiguous run of at most CHAIN super-blocks and keeps its terms in registers; the sums then pass
-// from wavefront to wavefront through LDS in the super-blocks' order (a barrier a wavefront). LDS holds no terms then, so more
-// workgroups share a compute unit and long rows leave room for eight wavefronts. CHAIN = 0: super-blocks round robin, terms
-// [nsb][kT][64] in LDS, summed by the first wavefront (any K that fits).
+// kTiles: tiles of sixteen rows of W that share the operand of x. kDepth: super-blocks a wavefront has under way. kRounds: how many
+// times that many it takes at most (0: any number; the last requests of a loop of unknown length are for nothing).
 // ROPE: W is q | k | v of a decoding step; the rotation and the cache writes ride on the results (rope_kv's arithmetic, interleaved
 // pairs), y gets the rotated queries only.
-template <int DT, int kWaves, int CHAIN, bool ROPE = false>
+template <int DT, int kTiles, int kWaves, int kDepth, int kRounds, bool ROPE>
 __global__ __launch_bounds__(64 * kWaves) void qgemv_kq_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, const float* resid,
-                                                                     int M_all, int N, int nsb, int64_t act_row_bytes, const Q4RopeTail rope) {
+                                                                    int M_all, int N, int nsb, int64_t act_row_bytes, int y_bf16, const Q4RopeTail rope) {
     typedef WBlock<DT> WB;
-    constexpr int kT = WB::kTerms, kAll = 32 * WB::kPieces, kLoads = (kAll + 63) / 64, kSlab = 32 * WB::kStride;
+    constexpr int kT = WB::kTerms, kCols = 16 * kTiles, kAll = kCols * WB::kPieces, kLoads = (kAll + 63) / 64, kSlab = kCols * WB::kStride;
     typedef Stage<kLoads> St;
-    extern __shared__ __align__(16) uint8_t smem[];  // terms (or the sums handed on), then per wavefront a super-block of x and the slab of W
-    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+    extern __shared__ __align__(16) uint8_t smem[];  // per wavefront x and the slab of W, then the terms [nsb][kT][8 rows of x][kCols]
+    float* terms = (float*)(smem + kWaves * (kXBytes + kSlab));
+    const int tid = threadIdx.x;
+    const uint32_t lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // blockIdx.z: the group of eight rows of x
     const int64_t row0 = (int64_t)kRows * blockIdx.z;
-    act += row0 * act_row_bytes;
     const int M = M_all - (int)row0 < kRows ? M_all - (int)row0 : kRows;
-    const int n0 = blockIdx.x * 32, n = n0 + l32;
-    f32x4* terms = (f32x4*)smem;
-    uint8_t* xl = smem + (size_t)(CHAIN ? 1 : nsb) * kT * 1024 + wave * (kXBytes + kSlab);
+    const int n0 = blockIdx.x * kCols, left = N - n0 < kCols ? N - n0 : kCols;
+    uint8_t* xl = smem + wave * (kXBytes + kSlab);
     uint8_t* slab = xl + kXBytes;
+    *(uint32_t*)(xl + 4 * lane) = 0;
 
-    // piece p = 64 i + lane of a super-block of the 32 rows: row p / kPieces, piece p % kPieces of it
+    // piece p = 64 i + lane of a super-block of the rows: row p / kPieces, piece p % kPieces of it; rows beyond N repeat the last one
     const uint8_t* wbase = W + (int64_t)n0 * nsb * WB::kBytes;
     uint32_t goff[kLoads], loff[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; i++) {
         int p = 64 * i + lane;
         p = p < kAll ? p : kAll - 1;  // a last load that is not full repeats the last piece in its upper lanes
-        const int r = p / WB::kPieces, c = p - WB::kPieces * r;
-        const int row = n0 + r < N ? n0 + r : N - 1;
-        goff[i] = (uint32_t)(row - n0) * (uint32_t)(nsb * WB::kBytes) + WB::piece_offset(c);  // 32 rows of W within 4 GB (checked by the host)
-        loff[i] = r * WB::kStride + 16 * c;
+        const int row = p / WB::kPieces, c = p - WB::kPieces * row;
+        goff[i] = (uint32_t)(row < left ? row : left - 1) * (uint32_t)(nsb * WB::kBytes) + WB::piece_offset(c);
+        loff[i] = row * WB::kStride + 16 * c;
     }
-    // pieces of x a lane fetches: quants p = lane, 64 + lane (row p / 16, bytes 16 (p % 16)..); sums (lanes below 16:
-    // row lane / 2, half lane % 2); scale (lanes below 8: row lane). Rows from M on repeat the last one.
-    const uint8_t* xsrc[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int p = 64 * i + lane, r = p >> 4;
-        xsrc[i] = act + (int64_t)(r < M ? r : M - 1) * act_row_bytes + 16 * (p & 15);
-    }
-    // (every lane loads, the upper ones what lower ones load too: with a load under a branch the compiler waits for all loads under
-    // way, the next super-block's with them, before it touches this one's)
-    const int rs = ((lane >> 1) & 7) < M ? ((lane >> 1) & 7) : M - 1, rd = (lane & 7) < M ? (lane & 7) : M - 1;
-    const uint8_t* ssrc = act + (int64_t)rs * act_row_bytes + (int64_t)nsb * 256 + 16 * (lane & 1);
-    const uint8_t* dsrc = act + (int64_t)rd * act_row_bytes + (int64_t)nsb * 288;
+    // x: rows from M on lie past the buffer's end and read as zeros, as does every super-block past the last one
+    const uint32_t xbytes = (uint32_t)act_row_bytes, m0 = 4 * (g & 1) + 2 * (g >> 1);  // m0: the rows of x whose terms this lane makes
+    const __amdgpu_buffer_rsrc_t wr = buffer_of(wbase, (uint32_t)(nsb * WB::kBytes) * left), xr = buffer_of(act + row0 * act_row_bytes, xbytes * M);
+    const uint32_t xo = (lane >> 4) * xbytes + 16 * r, so = lane < 16 ? (lane >> 1) * xbytes + 16 * (lane & 1) : kBeyond, dof = m0 * xbytes;
 
+    // (every fetch has the same number of loads, and none lies under a branch: the compiler counts those that may still be out)
     auto fetch = [&](St& f, int sb) {
-        const uint8_t* wb = wbase + (int64_t)sb * WB::kBytes;
+        const uint32_t past = sb < nsb ? 0 : kBeyond;
+        const int at = sb < nsb ? sb : nsb - 1;
+        const uint8_t* wb = wbase + (int64_t)at * WB::kBytes;
 #pragma unroll
         for (int i = 0; i < kLoads; i++) {
-            if (DT == kQ4_K) f.w[i] = *(const u32x4*)(wb + goff[i]);
+            if (DT == kQ4_K) f.w[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, goff[i] | past, at * WB::kBytes, 0);
             else __builtin_memcpy(&f.w[i], __builtin_assume_aligned(wb + goff[i], 2), 16);
         }
 #pragma unroll
-        for (int i = 0; i < 2; i++) f.xq[i] = *(const u32x4*)(xsrc[i] + (int64_t)sb * 256);
-        f.xs = *(const u32x4*)(ssrc + (int64_t)sb * 32);
-        f.xd = ((const float*)dsrc)[sb];
+        for (int i = 0; i < 2; i++) f.xq[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, (xo + 4 * i * xbytes) | past, at * 256, 0);
+        if (kT == 2) f.xs = __builtin_amdgcn_raw_buffer_load_b128(xr, so | past, nsb * 256 + at * 32, 0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) f.xd[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, (dof + i * xbytes) | past, nsb * 288 + at * 4, 0));
     };
-    auto work = [&](const St& f, f32x4* t) {
+    auto work = [&](const St& f, int sb) {
         // W and x of the super-block into this wavefront's LDS (its own: a wavefront's LDS operations complete in order)
 #pragma unroll
         for (int i = 0; i < kLoads; i++)
-            if (64 * (i + 1) <= kAll || lane < kAll - 64 * i) *(u32x4*)(slab + loff[i]) = f.w[i];
+            if (64 * (i + 1) <= kAll || (int)lane < kAll - 64 * i) *(u32x4*)(slab + loff[i]) = f.w[i];
 #pragma unroll
-        for (int i = 0; i < 2; i++) *(u32x4*)(xl + kXq + ((64 * i + lane) >> 4) * kXRow + 16 * (lane & 15)) = f.xq[i];
-        if (lane < 16) *(u32x4*)(xl + kXs + 16 * lane) = f.xs;
-        if (lane < 8) *(float*)(xl + kXd + 4 * lane) = f.xd;
-        WB::terms(slab + l32 * WB::kStride, xl, l32, lh, t);
+        for (int i = 0; i < 2; i++) *(u32x4*)(xl + kXq + (4 * i + (lane >> 4)) * kXRow + 16 * r) = f.xq[i];
+        if (kT == 2 && lane < 16) *(u32x4*)(xl + kXs + 16 * lane) = f.xs;
+        WB b;
+        b.operands(xl, r, g);
+#pragma unroll
+        for (int tile = 0; tile < kTiles; tile++) {
+            float t[kT][2];
+            b.terms(slab + (16 * tile + r) * WB::kStride, f.xd, g, t);
+            float* at = terms + ((sb * kTiles + tile) * 64 + lane) * 2 * kT;
+            if constexpr (kT == 2) *(f32x4*)at = f32x4{t[0][0], t[1][0], t[0][1], t[1][1]};
+            else *(f32x2*)at = f32x2{t[0][0], t[0][1]};
+        }
     };
-    f32x4 acc[kT];
+    // up to a multiple of eight super-blocks with zeros: a sum from zero is never a negative zero, so they change no bit of it
+    for (int i = tid; i < (((nsb + 7) & ~7) - nsb) * kTiles * 128 * kT; i += 64 * kWaves) terms[nsb * kTiles * 128 * kT + i] = 0.f;
+    St f[kDepth];
 #pragma unroll
-    for (int i = 0; i < kT; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (CHAIN > 0) {
-        const int sb_lo = wave * nsb / kWaves, count = (wave + 1) * nsb / kWaves - sb_lo;  // at most CHAIN (the host's choice of CHAIN)
-        St f[2];
-        f32x4 tt[CHAIN][kT];
-        if (count > 0) fetch(f[0], sb_lo);
-#pragma unroll
-        for (int j = 0; j < CHAIN; j++) {
-            if (j < count) {  // the same for the whole wavefront
-                if (j + 1 < count) fetch(f[(j + 1) & 1], sb_lo + j + 1);
-                work(f[j & 1], tt[j]);
-            }
-            __builtin_amdgcn_sched_barrier(0);  // one super-block's work at a time: interleaved they would not fit the registers
-        }
-        // wavefront w adds its terms, the CPU's next ones, to the sums of those before it and hands them on
-        for (int w = 0; w < kWaves; w++) {
-            if (w == wave) {
-                if (w > 0) {
-#pragma unroll
-                    for (int i = 0; i < kT; i++) acc[i] = terms[i * 64 + lane];
-                }
-#pragma unroll
-                for (int j = 0; j < CHAIN; j++) {
-                    if (j < count) {
-#pragma unroll
-                        for (int i = 0; i < kT; i++)
-#pragma unroll
-                            for (int jj = 0; jj < 4; jj++) acc[i][jj] = acc[i][jj] + tt[j][i][jj];
-                    }
-                }
-                if (w + 1 < kWaves) {
-#pragma unroll
-                    for (int i = 0; i < kT; i++) terms[i * 64 + lane] = acc[i];
-                }
-            }
-            if (w + 1 < kWaves) __syncthreads();
-        }
-        if (wave != kWaves - 1) return;
-    } else {
-        St cur, nxt;  // one in work, the next requested
-        if (wave < nsb) fetch(cur, wave);
-        for (int sb = wave; sb < nsb; sb += kWaves) {
-            fetch(nxt, sb + kWaves < nsb ? sb + kWaves : sb);
-            f32x4 t[kT];
-            work(cur, t);
-#pragma unroll
-            for (int i = 0; i < kT; i++) terms[(sb * kT + i) * 64 + lane] = t[i];
-            cur = nxt;
-        }
-        __syncthreads();
-        if (wave != 0) return;
-        // the CPU's order; eight super-blocks' terms are requested together so that the chain of additions does not wait for LDS each time
-        for (int sb0 = 0; sb0 < nsb; sb0 += 8) {
-            f32x4 t[8][kT];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int sb = sb0 + j < nsb ? sb0 + j : nsb - 1;
-#pragma unroll
-                for (int i = 0; i < kT; i++) t[j][i] = terms[(sb * kT + i) * 64 + lane];
-            }
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                if (sb0 + j >= nsb) break;
-#pragma unroll
-                for (int i = 0; i < kT; i++)
-#pragma unroll
-                    for (int jj = 0; jj < 4; jj++) acc[i][jj] = acc[i][jj] + t[j][i][jj];
-            }
-        }
+    for (int u = 0; u < kDepth; u++) {
+        fetch(f[u], wave + u * kWaves);
+        __builtin_amdgcn_sched_barrier(0);  // in this order: what is requested first returns first
     }
-    if constexpr (ROPE) {
-        // rows (n, n + 1), n even, are a pair of features: the even lane takes its neighbour's result and stores both
-        const int pos = *rope.pos;
+    auto round = [&](int sb0, bool more) {
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const float v = kT == 2 ? acc[0][jj] - acc[kT - 1][jj] : acc[0][jj];
-            const float other = dpp_f32<0xb1>(v);  // quad_perm [1,0,3,2]
-            const int m = 4 * lh + jj, seq = (int)row0 + m;
-            if ((lane & 1) == 0 && n < N && m < M) q4_rope_store(rope, pos, seq, n, v, other, y + (int64_t)seq * N);
+        for (int u = 0; u < kDepth; u++) {
+            const int sb = sb0 + u * kWaves;
+            if (sb < nsb) work(f[u], sb);       // the same for the whole wavefront
+            __builtin_amdgcn_sched_barrier(0);  // one super-block at a time: interleaved they would not fit the registers
+            if (more) fetch(f[u], sb + kDepth * kWaves);
         }
+    };
+    if constexpr (kRounds > 0) {
+#pragma unroll
+        for (int i = 0; i < kRounds; i++) round(wave + i * kDepth * kWaves, i + 1 < kRounds);
+    } else {
+        for (int sb0 = wave; sb0 < nsb; sb0 += kDepth * kWaves) round(sb0, true);
+    }
+    __syncthreads();
+    if (tid >= kRows * kCols) return;
+    // one thread an output: the CPU's order; the next eight super-blocks' terms are requested before these are added
+    float acc[kT], t[2][8][kT];
+#pragma unroll
+    for (int i = 0; i < kT; i++) acc[i] = 0.f;
+    auto request = [&](float (*to)[kT], int sb0) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float* at = terms + ((sb0 + j) * kTiles * 128 + tid) * kT;
+            if constexpr (kT == 2) {
+                const f32x2 v = *(const f32x2*)at;
+                to[j][0] = v[0];
+                to[j][1] = v[1];
+            } else to[j][0] = *at;
+        }
+    };
+    auto add = [&](const float (*from)[kT]) {
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+#pragma unroll
+            for (int i = 0; i < kT; i++) acc[i] = acc[i] + from[j][i];
+    };
+    request(t[0], 0);
+    for (int sb0 = 0;;) {
+        if ((sb0 += 8) < nsb) request(t[1], sb0);
+        add(t[0]);
+        if (sb0 >= nsb) break;
+        if ((sb0 += 8) < nsb) request(t[0], sb0);
+        add(t[1]);
+        if (sb0 >= nsb) break;
+    }
+    const float v = kT == 2 ? acc[0] - acc[kT - 1] : acc[0];
+    // thread 128 tile + 2 lane + j has row m0 + j of x (see terms)
+    const int of = (tid & 127) >> 1, m = 4 * ((of >> 4) & 1) + 2 * (of >> 5) + (tid & 1), n = n0 + 16 * (tid >> 7) + (of & 15);
+    if constexpr (ROPE) {
+        // rows (n, n + 1), n even, are a pair of features: the even row's lane takes its neighbour's result and stores both
+        const float other = dpp_f32<0x4e>(v);  // quad_perm [2,3,0,1]
+        const int seq = (int)row0 + m;
+        if ((n & 1) == 0 && n < N && m < M) q4_rope_store(rope, *rope.pos, seq, n, v, other, y + (int64_t)seq * N);
         return;
     }
-    if (n < N) {
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const int m = 4 * lh + jj;
-            if (m < M) {
-                const int64_t at = (row0 + m) * N + n;
-                const float v = kT == 2 ? acc[0][jj] - acc[kT - 1][jj] : acc[0][jj];
-                y[at] = resid ? v + resid[at] : v;
-            }
-        }
+    if (n < N && m < M) {
+        const int64_t at = (row0 + m) * N + n;
+        const float out = resid ? v + resid[at] : v;
+        if (y_bf16) ((uint16_t*)y)[at] = f32_to_bf16_bits(out);
+        else y[at] = out;
     }
 }
 
@@ -364,99 +360,99 @@ __global__ __launch_bounds__(64 * kWaves) void qgemv_kq_rows_kernel(const uint8_
 static std::atomic<int> g_kq_rows{0};  // measurement aid: 1 = never, 2 = for any number of rows the kernel takes
 void set_kquant_rows(int v) { g_kq_rows = v; }
 
-static std::atomic<int> g_kq_rows_waves{0};  // measurement aid: 4 or 8 wavefronts to a workgroup whatever the shape
-static std::atomic<int> g_kq_rows_chain{0};  // measurement aid: 1 = terms in LDS whatever the shape
-void set_kquant_rows_waves(int v) {
-    if (v == 0) g_kq_rows_chain = g_kq_rows_waves = 0;
-    else if (v == 1) g_kq_rows_chain = 1;
-    else g_kq_rows_waves = v;
+static std::atomic<int> g_kq_rows_waves{0};  // measurement aid: 4, 8 or 16 wavefronts to a workgroup where there is a form of that many
+void set_kquant_rows_waves(int v) { g_kq_rows_waves = v == 4 || v == 8 || v == 16 ? v : 0; }
+
+// LDS of a workgroup: per wavefront a super-block of x and the slab of W, and the terms.
+static size_t rows_lds(int dt, int64_t nsb, int tiles, int waves) {
+    return (size_t)waves * (kXBytes + 16 * tiles * (dt == kQ4_K ? WBlock<kQ4_K>::kStride : WBlock<kQ6_K>::kStride)) +
+           (size_t)((nsb + 7) & ~7) * (dt == kQ4_K ? 2 : 1) * kRows * 16 * tiles * sizeof(float);
 }
 
-// LDS of a workgroup: the terms (or the sums handed on), and per wavefront a super-block of x and the slab of W.
-static size_t rows_lds(int dt, int64_t nsb, int waves, bool chain) {
-    return (size_t)(chain ? 1 : nsb) * (dt == kQ4_K ? 2 : 1) * 1024 +
-           (size_t)waves * (kXBytes + 32 * (dt == kQ4_K ? WBlock<kQ4_K>::kStride : WBlock<kQ6_K>::kStride));
-}
-
-// Two rows of x or more, converted (kq_convert_act); the terms of 32 rows of W in LDS; Q4_K's W 16-byte aligned, Q6_K's on an even address.
+// Two rows of x or more, converted (kq_convert_act); the terms of sixteen rows of W in LDS; Q4_K's W 16-byte aligned, Q6_K's on an even address.
 bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a) {
     const int64_t nsb = a.K / 256;
     return (dt == kQ4_K || dt == kQ6_K) && g_kq_rows != 1 && a.M >= 2 && a.M <= 8 * 65535 && a.act && a.K % 256 == 0 && nsb > 0 &&
            ((uintptr_t)a.W & (dt == kQ4_K ? 15 : 1)) == 0 && ((uintptr_t)a.act & 15) == 0 && a.N > 0 && a.N <= (1ll << 30) &&
-           (nsb <= 64 || rows_lds(dt, nsb, 4, false) <= 160 * 1024) && 32 * nsb * 210 < ((int64_t)1 << 32);
+           rows_lds(dt, nsb, 1, 4) <= 160 * 1024;
 }
 
-// Where it is the faster choice. A pass over W for eight rows of x runs at about 3.3 TB/s (Q4_K; 14336 x 4096 in 11 us, 28672 x 4096
-// in 20 us, after 4 us for converting x) or 2.6 TB/s (Q6_K; 19 and 37 us); the tiled kernel of qgemm_kquant.hip spends about 2.1 us per
-// super-block of K and round of 256 tiles of 128 x 128 (at 32 rows of x and 14336 x 4096: 36 us here, 34 us there; at 4096 x 14336: 36
-// and 100 us).
+// Where it is the faster choice. Up to eight rows always; beyond, by what both kernels take: here 3 us, then W from memory once and once from
+// the caches per group of eight rows (5.7 TB/s Q4_K, 6.2 TB/s Q6_K), the tiled kernel of qgemm_kquant.hip about 2.1 us per super-block of
+// K and round of 128 tiles of 128 x 128. Measured, us, here | there, Q4_K: 32 x 14336 x 4096 28.5 | 31.6, 40 rows 34.4 | 31.8; 32 x 28672
+// x 4096 55 | 61, 40 rows 67 | 62; 64 x 4096 x 14336 62 | 109, 128 rows 121 | 118; 64 x 1024 x 4096 5.4 | 32. Q6_K: 16 x 14336 x 4096 24.6 | 32.2, 32 rows 37.5 | 32.5.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
     if (g_kq_rows == 2 || a.M <= 8) return true;
-    if (a.M > 64) return false;
+    if (a.M > 512) return false;
     const double nsb = (double)(a.K / 256), groups = (double)((a.M + kRows - 1) / kRows);
-    const double rows_us = groups * (double)a.N * nsb * (dt == kQ4_K ? 144 / 3.3e6 : 210 / 2.6e6);
-    // (its 2.1 us hold up to some 128 tiles at a time: 112 tiles take 35 us at K = 4096, 224 take 63)
+    // (rows of more than 32 super-blocks leave room for one workgroup a compute unit)
+    const double rows_us = 3 + (groups + 0.6) * (double)a.N * nsb * (dt == kQ4_K ? 144 / 5.7e6 : 210 / 6.2e6) / (nsb > 32 ? 0.75 : 1);
     const double tiles = (double)(((a.M + 127) / 128) * ((a.N + 127) / 128));
     return rows_us < (tiles > 128 ? tiles / 128 : 1.0) * nsb * 2.1;
 }
 
-template <int DT, int WAVES, int CHAIN, bool ROPE = false>
-static hipError_t launch_kq_rows(const QGemvArgs& a, hipStream_t st, const Q4RopeTail* rope = nullptr) {
+template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>
+static hipError_t launch_kq_rows(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int nsb = (int)(a.K / 256);
+    const auto kernel = qgemv_kq_rows_kernel<DT, TILES, WAVES, DEPTH, ROUNDS, ROPE>;
     static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemv_kq_rows_kernel<DT, WAVES, CHAIN, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
         raised = true;
     }
-    hipLaunchKernelGGL((qgemv_kq_rows_kernel<DT, WAVES, CHAIN, ROPE>), dim3((unsigned)((a.N + 31) / 32), 1, (unsigned)((a.M + kRows - 1) / kRows)),
-                       dim3(64 * WAVES), rows_lds(DT, nsb, WAVES, CHAIN > 0), st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y, a.resid, (int)a.M,
-                       (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), rope ? *rope : Q4RopeTail{});
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.N + 16 * TILES - 1) / (16 * TILES)), 1, (unsigned)((a.M + kRows - 1) / kRows)),
+                       dim3(64 * WAVES), rows_lds(DT, nsb, TILES, WAVES), st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y, a.resid, (int)a.M,
+                       (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), bf16 ? 1 : 0, rope ? *rope : Q4RopeTail{});
     return hipGetLastError();
 }
 
-// Eight wavefronts where the workgroups are at most one to a compute unit or the rows are long, four where they are many (measured at
-// eight rows of x already converted, us a call, Q4_K | Q6_K, four and eight wavefronts: 14336 x 4096 11.1 14.2 | 16.0 19.2; 4096 x 4096
-// 7.6 7.1 | 10.1 9.3; 28672 x 4096 20.5 27.3 | 33.5 41.8). Rows of more than four super-blocks a wavefront (K above 8192 with eight) keep
-// the terms in registers, in runs of up to eight super-blocks (4096 x 14336: 16.3 | 21.3 us, 19.9 | 21.9 with the terms in LDS, which leave
-// room for four wavefronts only); shorter ones gain nothing from it (the registers cost what the LDS gives), longer ones have no choice.
-static void rows_shape(int dt, const QGemvArgs& a, int* waves_out, bool* chain_out) {
-    const int64_t nsb = a.K / 256, wgs = (a.N + 31) / 32 * ((a.M + kRows - 1) / kRows);
-    int waves = wgs <= 256 || nsb > 32 ? 8 : 4;
-    if (g_kq_rows_waves == 4 || g_kq_rows_waves == 8) waves = g_kq_rows_waves;
-    bool chain = g_kq_rows_chain != 1 && nsb > 4 * waves && nsb <= 64;
-    if (chain) waves = 8;
-    else if (rows_lds(dt, nsb, waves, false) > 160 * 1024) waves = 4;
-    *waves_out = waves;
-    *chain_out = chain;
+// By the super-blocks that a wavefront takes: sixteen wavefronts hold two under way within their 128 registers, fewer four.
+template <int DT, int TILES, int WAVES, bool ROPE>
+static hipError_t launch_depth(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
+    const int64_t each = (a.K / 256 + WAVES - 1) / WAVES;
+    if (each <= 1) return launch_kq_rows<DT, TILES, WAVES, 1, 1, ROPE>(a, st, bf16, rope);
+    if (each <= 2) return launch_kq_rows<DT, TILES, WAVES, 2, 1, ROPE>(a, st, bf16, rope);
+    if constexpr (WAVES == 16) {
+        if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 2, 2, ROPE>(a, st, bf16, rope);
+        return launch_kq_rows<DT, TILES, WAVES, 2, 0, ROPE>(a, st, bf16, rope);
+    } else {
+        if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 4, 1, ROPE>(a, st, bf16, rope);
+        if (each <= 8) return launch_kq_rows<DT, TILES, WAVES, 4, 2, ROPE>(a, st, bf16, rope);
+        return launch_kq_rows<DT, TILES, WAVES, 4, 0, ROPE>(a, st, bf16, rope);
+    }
+}
+
+// Measured at eight rows of x, us: one tile in 16 | 8 | 4 wavefronts 4096 x 14336 Q4_K 12.1 | 13.6 | 13.4, Q6_K 14.7 | 17.3 | 15.9, 4096 x 4096 4.8 |
+// 5.5 | 6.0, 6.1 | 6.9 | 8.1: the most where there is at most one workgroup a compute unit. Two tiles in 16 | 8 | 4: 6144 x 4096 Q4_K 6.9 | 7.4 |
+// 8.6, Q6_K (no room for 16) - | 8.1 | 10.2; 28672 x 4096 23 | 26 | 20-22: four where there are more than two workgroups a unit.
+template <int DT, bool ROPE>
+static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
+    const int64_t nsb = a.K / 256, wgs = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows);
+    const int fixed = g_kq_rows_waves;
+    auto fits = [&](int tiles, int waves) { return rows_lds(DT, nsb, tiles, waves) <= 160 * 1024 && (fixed == 0 || fixed == waves); };
+    if (wgs <= 256 && fits(1, 16)) return launch_depth<DT, 1, 16, ROPE>(a, st, bf16, rope);
+    if constexpr (DT == kQ4_K) {
+        if (wgs <= 512 && fits(2, 16)) return launch_depth<DT, 2, 16, ROPE>(a, st, bf16, rope);
+    } else {
+        if (wgs <= 512 && nsb <= 16 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
+    }
+    if (fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
+    return launch_depth<DT, 1, 4, ROPE>(a, st, bf16, rope);
 }
 
 // The q | k | v product of a decoding step with the rotation and the cache writes as its tail (see Q4RopeTail; interleaved pairs,
-// even widths): where the rows kernel takes the shape with its terms in LDS (K up to 8192).
-bool qgemv_kquant_rows_rope_ok(int dt, const QGemvArgs& a) {
-    if (!qgemv_kquant_rows_ok(dt, a) || a.resid || a.N % 2) return false;
-    int waves;
-    bool chain;
-    rows_shape(dt, a, &waves, &chain);
-    return !chain;
-}
+// even widths).
+bool qgemv_kquant_rows_rope_ok(int dt, const QGemvArgs& a) { return qgemv_kquant_rows_ok(dt, a) && !a.resid && a.N % 2 == 0; }
 
 hipError_t qgemv_kquant_rows_rope(int dt, const QGemvArgs& a, const Q4RopeTail& rope, hipStream_t st) {
-    int waves;
-    bool chain;
-    rows_shape(dt, a, &waves, &chain);
-    if (chain) return hipErrorInvalidValue;
-    if (dt == kQ4_K) return waves == 8 ? launch_kq_rows<kQ4_K, 8, 0, true>(a, st, &rope) : launch_kq_rows<kQ4_K, 4, 0, true>(a, st, &rope);
-    return waves == 8 ? launch_kq_rows<kQ6_K, 8, 0, true>(a, st, &rope) : launch_kq_rows<kQ6_K, 4, 0, true>(a, st, &rope);
+    return dt == kQ4_K ? launch_shape<kQ4_K, true>(a, st, false, &rope) : launch_shape<kQ6_K, true>(a, st, false, &rope);
 }
 
-hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st) {
-    int waves;
-    bool chain;
-    rows_shape(dt, a, &waves, &chain);
-    if (dt == kQ4_K) return chain ? launch_kq_rows<kQ4_K, 8, 8>(a, st) : waves == 8 ? launch_kq_rows<kQ4_K, 8, 0>(a, st) : launch_kq_rows<kQ4_K, 4, 0>(a, st);
-    return chain ? launch_kq_rows<kQ6_K, 8, 8>(a, st) : waves == 8 ? launch_kq_rows<kQ6_K, 8, 0>(a, st) : launch_kq_rows<kQ6_K, 4, 0>(a, st);
+// y_bf16: a.y holds bfloat16, rounded as the results are stored.
+hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16) {
+    return dt == kQ4_K ? launch_shape<kQ4_K, false>(a, st, y_bf16, nullptr) : launch_shape<kQ6_K, false>(a, st, y_bf16, nullptr);
 }
 
 }  // namespace mimir

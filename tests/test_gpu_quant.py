@@ -725,6 +725,34 @@ def test_kquant_rows_of_x_share_one_pass_over_w_on_the_matrix_cores(dt, m, n, k)
 
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("m,n,k", [(2, 16, 256), (8, 15, 256 * 16), (7, 17, 256 * 17), (9, 31, 256 * 32), (3, 33, 256 * 49), (17, 47, 256 * 64),
+                                   (8, 18, 256 * 65), (8, 20, 256 * 75), (5, 4099, 256), (8, 4130, 256 * 16), (6, 4131, 256 * 17), (16, 2070, 256 * 20),
+                                   (5, 8210, 256 * 2), (8, 8211, 256 * 9), (2, 8225, 256 * 33), (130, 1030, 256 * 5), (64, 520, 256 * 34)])
+def test_kquant_rows_kernel_at_the_edges_of_its_forms(dt, m, n, k):
+    """One or two tiles of sixteen rows of W a workgroup, four to sixteen wavefronts, one to four super-blocks each and loops of
+    more, partly filled tiles and groups of x: the oracle's bits, into float32 and, rounded once, into bfloat16."""
+    l = gpu.lib()
+    rng = np.random.default_rng(dt + 7 * m + n + k)
+    raw = random_blocks(rng, dt, n * k)
+    x = O.f32_to_bf16(rng.normal(size=(m, k)).astype(np.float32)).reshape(m, k)
+    xf = O.bf16_to_f32(x).reshape(m, k)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    want = O.qmatmul(dt, raw, xf, n, k)
+    xd = torch.from_numpy(x.view(np.int16)).to("cuda:0")
+    half = torch.empty(m * n, dtype=torch.int16, device="cuda:0")
+    try:
+        capi.check(l.mi355x_tune(b"kquant.mfma_rows", 2))
+        gpu.say(f"kquant rows kernel forms dt={dt} M={m} N={n} K={k}")
+        got = gpu.qgemv(dt, ptr, gpu.dev(xf), n, k)
+        capi.check(l.mi355x_qgemm_bf16(dt, ptr, xd.data_ptr(), half.data_ptr(), m, n, k, k, capi.BF16, gpu.stream()))
+        gpu.sync()
+    finally:
+        capi.check(l.mi355x_tune(b"kquant.mfma_rows", 0))
+    assert bits_equal(got, want)
+    assert np.array_equal(half.cpu().numpy().view(np.uint16).reshape(m, n), O.f32_to_bf16(want).reshape(m, n))
+
+
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
 def test_kquant_rows_kernel_at_the_largest_integer_sums(dt):
     """Every quant and scale at its largest magnitude with x at +-127 per super-block (backend/cpu/quant_test.go:164-204), through the
     kernel that reads W once per eight rows of x: its 24-bit multiplies and int32 sums hold what the CPU's int32 arithmetic holds."""

@@ -281,6 +281,7 @@ hipError_t advance(int32_t* state, const int32_t* next_tok, int32_t* record, int
 __global__ void set_state_kernel(int32_t* __restrict__ state, int pos, int step) {
     state[0] = pos;
     state[1] = step;
+    state[2] = 0;  // rows whose token is chosen (ChooseTail)
 }
 
 hipError_t set_state(int32_t* state, int pos, int step, hipStream_t st) {
@@ -399,23 +400,26 @@ __device__ __forceinline__ void argmax_better(float& best, int& at, float v, int
     }
 }
 
+// TAIL: the workgroup that chooses a row's token also does what follows it (ChooseTail). As launches of their own the bookkeeping and
+// the embedding of a decoding step took 4.0 and 4.6 us, and the choice 7.0 with workgroups of four rounds of loads; together 6.
+template <bool TAIL>
 __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restrict__ logits, int64_t n, int span, int32_t* __restrict__ out,
                                                            uint32_t* __restrict__ tickets, float* __restrict__ cand_v,
-                                                           int* __restrict__ cand_i) {
+                                                           int* __restrict__ cand_i, const ChooseTail tail) {
     __shared__ float bv[4];
     __shared__ int bi[4];
-    __shared__ int s_last;
+    __shared__ int s_last, s_token;
     const int r = blockIdx.y, nblk = gridDim.x;
     const float* row = logits + (int64_t)r * n;
     const int64_t lo = (int64_t)blockIdx.x * span, hi = lo + span < n ? lo + span : n;
     float best = -__builtin_inff();
     int at = 0x7fffffff;
-    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * 256) {
-        float v[4];
+    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += 8 * 256) {
+        float v[8];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = i0 + 256 * u < hi ? row[i0 + 256 * u] : -__builtin_inff();
+        for (int u = 0; u < 8; u++) v[u] = i0 + 256 * u < hi ? row[i0 + 256 * u] : -__builtin_inff();
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int u = 0; u < 8; u++)
             if (i0 + 256 * u < hi) argmax_better(best, at, v[u], (int)(i0 + 256 * u));
     }
 #pragma unroll
@@ -443,10 +447,10 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
         if (s_last) __hip_atomic_store(&tickets[r], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (!s_last || threadIdx.x >= 64) return;
+    if (!s_last || (!TAIL && threadIdx.x >= 64)) return;
     best = -__builtin_inff();
     at = 0x7fffffff;
-    if ((int)threadIdx.x < nblk) {
+    if ((int)threadIdx.x < nblk) {  // nblk is at most 64: the first wavefront
         best = __hip_atomic_load(&cand_v[r * kArgmaxBlocks + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         at = __hip_atomic_load(&cand_i[r * kArgmaxBlocks + threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -460,28 +464,85 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
         float first = row[0];
         if (first != first || at == 0x7fffffff) at = 0;  // NaN at 0, or nothing but NaNs
         out[r] = at;
+        if (TAIL) {
+            s_token = at;
+            // read before this row is counted, moved on behind the last row that is
+            const int32_t pos = tail.state[0], step = tail.state[1];
+            tail.record[(int64_t)step * gridDim.y + r] = at;
+            const uint32_t done = __hip_atomic_fetch_add((uint32_t*)tail.state + 2, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            if (done == gridDim.y - 1) {
+                tail.state[0] = pos + 1;
+                tail.state[1] = step + 1;
+                __hip_atomic_store((uint32_t*)tail.state + 2, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    if constexpr (TAIL) {
+        if (!tail.table) return;
+        __syncthreads();
+        // the token's row of the table, Q8_0 (dequant_at's product), eight weights a thread at a time
+        const uint8_t* from = tail.table + (int64_t)s_token * (tail.k / 32 * 34);
+        float* x = tail.x + r * tail.k;
+        for (int64_t c = 8 * threadIdx.x; c < tail.k; c += 2 * 8 * 256) {
+            u32x2 q[2] = {};
+            uint16_t d[2] = {};
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int64_t i = c + 8 * 256 * u;
+                if (i >= tail.k) continue;
+                const uint8_t* b = from + i / 32 * 34;
+                __builtin_memcpy(&q[u], __builtin_assume_aligned(b + 2 + i % 32, 2), 8);
+                d[u] = load_u16(b);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int64_t i = c + 8 * 256 * u;
+                if (i >= tail.k) continue;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const uint32_t w = q[u][j >> 2];
+                    x[i + j] = (float)(int8_t)(w >> (8 * (j & 3))) * f16_bits_to_f32(d[u]);
+                }
+            }
+        }
     }
 }
 
 size_t argmax_workspace_bytes(int64_t rows) { return kArgmaxTicketBytes + (size_t)rows * kArgmaxBlocks * 8; }
 
-// workspace: argmax_workspace_bytes(rows) bytes whose first kArgmaxTicketBytes were
-// zero before the first launch, or null for the one-workgroup kernel.
-hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, hipStream_t st) {
-    if (rows == 0) return hipSuccess;
-    if (!workspace || rows > (int64_t)(kArgmaxTicketBytes / 4) || n < 8192) {
-        hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)rows), dim3(1024), 0, st, logits, n, out);
-        return hipGetLastError();
-    }
-    int64_t nblk = (n + 4095) / 4096;
+// Workgroups of 2048 values, one round of eight loads a thread, up to 64 a row (one lane each in the last step).
+static void argmax_split(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail* tail, hipStream_t st) {
+    int64_t nblk = (n + 2047) / 2048;
     nblk = nblk > kArgmaxBlocks ? kArgmaxBlocks : nblk;
     int64_t span = ((n + nblk - 1) / nblk + 255) / 256 * 256;
     nblk = (n + span - 1) / span;
     uint32_t* tickets = (uint32_t*)workspace;
     float* cand_v = (float*)((uint8_t*)workspace + kArgmaxTicketBytes);
     int* cand_i = (int*)(cand_v + rows * kArgmaxBlocks);
-    hipLaunchKernelGGL(argmax_split_kernel, dim3((unsigned)nblk, (unsigned)rows), dim3(256), 0, st, logits, n, (int)span, out, tickets,
-                       cand_v, cand_i);
+    if (tail)
+        hipLaunchKernelGGL(argmax_split_kernel<true>, dim3((unsigned)nblk, (unsigned)rows), dim3(256), 0, st, logits, n, (int)span, out, tickets,
+                           cand_v, cand_i, *tail);
+    else
+        hipLaunchKernelGGL(argmax_split_kernel<false>, dim3((unsigned)nblk, (unsigned)rows), dim3(256), 0, st, logits, n, (int)span, out, tickets,
+                           cand_v, cand_i, ChooseTail{});
+}
+
+// workspace: argmax_workspace_bytes(rows) bytes whose first kArgmaxTicketBytes were
+// zero before the first launch, or null for the one-workgroup kernel.
+hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, hipStream_t st) {
+    if (rows == 0) return hipSuccess;
+    if (!argmax_choose_ok(rows, n, workspace)) {
+        hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)rows), dim3(1024), 0, st, logits, n, out);
+        return hipGetLastError();
+    }
+    argmax_split(logits, rows, n, out, workspace, nullptr, st);
+    return hipGetLastError();
+}
+
+bool argmax_choose_ok(int64_t rows, int64_t n, const void* workspace) { return workspace && rows > 0 && rows <= (int64_t)(kArgmaxTicketBytes / 4) && n >= 8192; }
+
+hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, hipStream_t st) {
+    argmax_split(logits, rows, n, out, workspace, &tail, st);
     return hipGetLastError();
 }
 

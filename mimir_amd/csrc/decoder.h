@@ -85,8 +85,11 @@ struct Decoder {
     // The logits of n rows (index into batch x s, ascending or not) of the last pass, into `logits` [n, vocab].
     virtual mi355x_status head(const int64_t* rows, int64_t n) = 0;
     // One decoding position of every sequence: the tokens from next_tok, the position from `state`, the logits into
-    // `logits` [batch, vocab]. Host-visible state (cache_len) is the caller's.
+    // `logits` [batch, vocab]. Host-visible state (cache_len) is the caller's. embed_next() comes before it, or, where
+    // next_embedding() says how, the choice of the tokens has brought in their rows.
     virtual mi355x_status step() = 0;
+    virtual mi355x_status embed_next() { return MI355X_OK; }
+    virtual void next_embedding(ChooseTail&) const {}
     virtual int step_variant() const { return 0; }
     // Whether calls longer than max_rows may be run in several passes.
     virtual bool runs_in_portions() const { return false; }

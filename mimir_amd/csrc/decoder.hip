@@ -141,8 +141,17 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
         st = hip(hipMemcpyAsync(next_tok.p, picked.p, B * 4, hipMemcpyDeviceToDevice, stream), "step state");
         if (!st) st = hip(set_state(state.as<int32_t>(), (int)cache_len, 0, stream), "step state");
         if (!st) st = hip(advance(state.as<int32_t>(), next_tok.as<int32_t>(), record.as<int32_t>(), (int)B, 0, stream), "step state");
+        ChooseTail tail;
+        tail.state = state.as<int32_t>();
+        tail.record = record.as<int32_t>();
+        next_embedding(tail);
+        const bool chosen = argmax_choose_ok(B, vocab, argmax_ws.p), embedded = chosen && tail.table;
+        if (!st && embedded && n_new > 1) st = embed_next();  // for the first step
         auto one_step = [&]() -> mi355x_status {
+            if (!embedded)
+                if (mi355x_status s2 = embed_next()) return s2;
             if (mi355x_status s2 = step()) return s2;
+            if (chosen) return hip(argmax_choose(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, tail, stream), "choice");
             if (mi355x_status s2 = hip(argmax(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, stream), "argmax")) return s2;
             return hip(advance(state.as<int32_t>(), next_tok.as<int32_t>(), record.as<int32_t>(), (int)B, 1, stream), "advance");
         };

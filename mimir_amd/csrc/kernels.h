@@ -105,6 +105,8 @@ hipError_t qgemv_q4_0_act_swiglu(const void* gate, const void* up, const void* a
 bool q8_act_fits(int64_t K);
 size_t q8_act_bytes(int64_t K);
 hipError_t q8_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
+// The same of rmsnorm's result, rows of x x_row_stride floats apart, d a multiple of 32, x and w 16-byte aligned.
+hipError_t rmsnorm_q8_act(const float* x, int64_t x_row_stride, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st);
 hipError_t qgemv_q8_0_act(const QGemvArgs& a, const int* tune, hipStream_t st);
 // Two or more rows of x against W read once (each sum formed as qgemv_q8_0_act forms it): rows converted beforehand,
 // W 4-byte aligned, an even number of blocks a row, no residual.
@@ -181,6 +183,14 @@ hipError_t rope_kv_split(float* q, const float* k, const float* v, void* kcache,
                          hipStream_t st, const float* bias = nullptr);
 // state = {position, steps}: record[steps] = next_tok [B], then steps += 1 and
 // position += pos_inc.
+// What follows the choice of a step's tokens, when argmax does it too: the token into the record, state = {position, steps taken, rows
+// chosen} moved on by one behind the last row, and, with a Q8_0 table, the token's row of it into x [rows, k] for the next step.
+struct ChooseTail {
+    int32_t *state = nullptr, *record = nullptr;
+    const uint8_t* table = nullptr;
+    int64_t k = 0;
+    float* x = nullptr;
+};
 hipError_t advance(int32_t* state, const int32_t* next_tok, int32_t* record, int B, int pos_inc, hipStream_t st);
 hipError_t set_state(int32_t* state, int pos, int step, hipStream_t st);
 hipError_t swiglu(const float* g, const float* u, float* out, int64_t rows, int64_t n, int64_t stride, hipStream_t st);
@@ -191,6 +201,9 @@ hipError_t add_bias(float* y, const float* bias, int64_t rows, int64_t n, hipStr
 constexpr size_t kArgmaxTicketBytes = 4096;
 size_t argmax_workspace_bytes(int64_t rows);
 hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, hipStream_t st);
+// argmax and its tail in one launch (the workspace is needed); whether it takes rows of n.
+bool argmax_choose_ok(int64_t rows, int64_t n, const void* workspace);
+hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, hipStream_t st);
 
 // Attention of queries [B, H, Q, D] over keys and values [B, HK, K, D], each
 // read through strides {batch, head, position} (features contiguous). chunk

@@ -79,6 +79,8 @@ struct Model : Decoder {
     mi355x_status forward(int64_t s) override;
     mi355x_status head(const int64_t* rows, int64_t n) override;
     mi355x_status step() override;
+    mi355x_status embed_next() override;
+    void next_embedding(ChooseTail& tail) const override;
     int step_variant() const override;
 };
 
@@ -296,7 +298,6 @@ static mi355x_status step_fast(Model& m) {
     float *x = m.x.as<float>(), *qkv = m.qkv.as<float>(), *a = m.a.as<float>(), *sw = m.s.as<float>();
     void* act = m.act[kActQ4].p;
     const int32_t* pos = m.state.as<int32_t>();
-    if (mi355x_status st = embed_rows(m, m.next_tok.as<int32_t>(), B, x, device_error_word())) return st;
     AttnArgs at;
     at.q = qkv; at.kv_dtype = c.cache_dtype; at.out = a; at.lse = nullptr;
     at.q_strides[0] = row; at.q_strides[1] = c.head_dim; at.q_strides[2] = 0;
@@ -387,7 +388,6 @@ static mi355x_status step_rows(Model& m) {
     float *x = m.x.as<float>(), *qkv = m.qkv.as<float>(), *gu = m.gu.as<float>(), *parts = m.parts.as<float>();
     void* act = m.rows_act.p;
     const int32_t* pos = m.state.as<int32_t>();
-    if (mi355x_status st = embed_rows(m, m.next_tok.as<int32_t>(), B, x, device_error_word())) return st;
     AttnArgs at;
     at.q = qkv; at.kv_dtype = c.cache_dtype; at.out = nullptr; at.lse = nullptr;
     at.q_strides[0] = row; at.q_strides[1] = c.head_dim; at.q_strides[2] = 0;
@@ -449,7 +449,6 @@ static mi355x_status step_any(Model& m) {
     float *qkv = m.qkv.as<float>(), *gu = m.gu.as<float>();
     const int32_t* pos = m.state.as<int32_t>();
     bool done[kActClasses];
-    if (mi355x_status st = embed_rows(m, m.next_tok.as<int32_t>(), B, x, device_error_word())) return st;
     AttnArgs at;
     at.q = q; at.kv_dtype = c.cache_dtype; at.out = a; at.lse = nullptr;
     at.q_strides[0] = qd; at.q_strides[1] = c.head_dim; at.q_strides[2] = 0;
@@ -560,14 +559,18 @@ static mi355x_status step_any(Model& m) {
 static mi355x_status head(Model& m, const float* xin, int64_t rows, int64_t row_stride) {
     const auto& c = m.c;
     float* hl = m.hlast.as<float>();
+    const Weight& w = m.tied ? m.embed : m.output;
+    bool done[kActClasses];
+    if (act_class(w, rows, m.fx_panel.bytes) == kActQ8 && m.act[kActQ8].bytes >= act_bytes(kActQ8, rows, c.embed) && rows <= 65535) {  // norm and conversion in one launch
+        LLM_HIP(rmsnorm_q8_act(xin, row_stride, m.norm.buf.as<float>(), m.act[kActQ8].p, rows, c.embed, c.eps, m.stream), "output_norm");
+        return linear(m, w, hl, m.logits.as<float>(), rows);
+    }
     if (row_stride == c.embed) {
         LLM_HIP(rmsnorm(xin, m.norm.buf.as<float>(), hl, rows, c.embed, c.eps, m.stream), "output_norm");
     } else {
         for (int64_t r = 0; r < rows; r++)
             LLM_HIP(rmsnorm(xin + r * row_stride, m.norm.buf.as<float>(), hl + r * c.embed, 1, c.embed, c.eps, m.stream), "output_norm");
     }
-    const Weight& w = m.tied ? m.embed : m.output;
-    bool done[kActClasses];
     if (mi355x_status st = convert_for(m, hl, rows, c.embed, {&w}, done)) return st;
     return linear(m, w, hl, m.logits.as<float>(), rows);
 }
@@ -586,6 +589,15 @@ mi355x_status Model::head(const int64_t* rows_of, int64_t n) {
             return mimir::head(*this, o.as<float>(), n, c.embed);
         }
     return mimir::head(*this, x.as<float>() + rows_of[0] * c.embed, n, apart * c.embed);
+}
+
+mi355x_status Model::embed_next() { return embed_rows(*this, next_tok.as<int32_t>(), c.batch, x.as<float>(), device_error_word()); }
+
+void Model::next_embedding(ChooseTail& tail) const {
+    if (embed.dtype != kQ8_0 || embed.k % 32 != 0 || embed.n < vocab) return;
+    tail.table = embed.buf.as<uint8_t>();
+    tail.k = embed.k;
+    tail.x = x.as<float>();
 }
 
 mi355x_status Model::step() {

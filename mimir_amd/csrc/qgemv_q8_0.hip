@@ -87,6 +87,42 @@ hipError_t q8_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_st
     return hipGetLastError();
 }
 
+// RMSNorm (rmsnorm_kernel's arithmetic, operation for operation: nn/transformer.go:50-61) and the conversion of its result in one
+// launch: a workgroup sums the row's squares as rmsnorm_kernel does, each for itself, and converts 32 blocks of it. The two launches
+// it replaces took 9.5 us in a decoding step, nearly all of it the cost of a dependent launch; this one 5.
+__global__ __launch_bounds__(256) void rmsnorm_q8_act_kernel(const float* __restrict__ x, int64_t x_row_stride, const float* __restrict__ w, int d, float inv_d,
+                                                             float eps, uint8_t* __restrict__ act, int64_t act_row_bytes) {
+    __shared__ float part[4];
+    const float* xr = x + (int64_t)blockIdx.y * x_row_stride;
+    const int nb = d >> 5, nbp = nb | 1, t = blockIdx.x * 256 + threadIdx.x;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f}, wv = {0.f, 0.f, 0.f, 0.f};
+    if (t < nb * 8) {  // requested with the loads of the sum
+        __builtin_memcpy(&v, xr + 4 * (int64_t)t, 16);
+        __builtin_memcpy(&wv, w + 4 * (int64_t)t, 16);
+    }
+    float ss = wave_sum(strided_sum_squares(xr, d, threadIdx.x));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float total = (part[0] + part[1]) + (part[2] + part[3]);
+    float ms = total * inv_d;
+    float scale = 1.0f / __builtin_sqrtf(ms + eps);
+    if (t >= nb * 8) return;  // whole groups of eight lanes
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        float n = v[k] * scale;
+        v[k] = n * wv[k];
+    }
+    uint32_t* q = (uint32_t*)(act + (int64_t)blockIdx.y * act_row_bytes);
+    q8_convert_item(v, q, (float*)(q + 2 * nbp * 4), nbp, t);
+}
+
+hipError_t rmsnorm_q8_act(const float* x, int64_t x_row_stride, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st) {
+    if (rows == 0) return hipSuccess;
+    hipLaunchKernelGGL(rmsnorm_q8_act_kernel, dim3((unsigned)((d / 4 + 255) / 256), (unsigned)rows), dim3(256), 0, st, x, x_row_stride, w, (int)d,
+                       (float)(1.0 / (double)d), (float)eps, (uint8_t*)act, (int64_t)q8_act_bytes(d));
+    return hipGetLastError();
+}
+
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 

@@ -366,6 +366,37 @@ def test_batch_step_that_reads_weights_once_chooses_the_same_tokens(batch):
             assert a == w, f"token {i}: device {a}, oracle {w}, oracle's margin there {margins[i]:.4g}"
 
 
+@pytest.mark.parametrize("embed,vocab,batch", [(512, 8192, 1), (512, 8195, 3), (4160, 8195, 2), (512, 70001, 9)])
+def test_the_choice_brings_in_the_next_embedding(embed, vocab, batch):
+    """From 8192 tokens on, the launch that chooses a step's tokens also records them, moves the position on and looks the next step's
+    embeddings up: tokens of the graph and of its launches equal to the per-operator path's, over three calls with one of logits between."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    c.embed, c.hidden, c.layers, c.vocab, c.context = embed, 320, 1, vocab, 32
+    if embed > 512:
+        c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved = 2, 1, 64, 64, 0
+    om = OL.synthetic(_oracle_config(c) if embed == 512 else OL.Config(
+        embed=c.embed, hidden=c.hidden, layers=c.layers, heads=c.heads, kv_heads=c.kv_heads, head_dim=c.head_dim, rope_dim=c.rope_dim,
+        rope_base=c.rope_base, rope_scale=1.0, eps=c.eps, vocab=c.vocab, context=c.context), seed=3, output_dt=O.Q8_0)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(16)
+    prompts = np.random.default_rng(23).integers(0, c.vocab, (batch, 5))
+    runs = []
+    try:
+        for mode in (0, 1, 2):
+            capi.check(lib.mi355x_tune(b"llama.step", mode))
+            m.reset()
+            first, _ = m.generate(prompts, 8)
+            more, _ = m.generate(first[:, -1:], 6)
+            last = m.logits(more[:, -1:])
+            again, _ = m.generate(last.argmax(-1).reshape(batch, 1).astype(np.int32), 3)
+            runs.append(np.concatenate([first, more, again], 1))
+    finally:
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+
+
 def test_fused_steps_without_their_riders_choose_the_per_operator_tokens():
     """The fused step lets the rotation, the norms and the conversion of SwiGLU's results ride on the products
     only where their shapes allow: interleaved pairs, rows of x one step of a wavefront long. A model with

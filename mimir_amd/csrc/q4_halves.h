@@ -2,6 +2,7 @@
 // bfloat16 as it is (qgemm_q4_0_blocks.hip).
 #pragma once
 #include "device_util.h"
+#include "kernels.h"
 
 namespace mimir {
 
@@ -12,15 +13,19 @@ typedef float f32x32 __attribute__((ext_vector_type(32)));
 
 // Operands lie in memory as the product reads them, so that every load is a whole KB: granules of 32 rows by one block
 // of 32 of K, the granules of a strip of 32 rows one after the other.
-constexpr int kGranuleX = 2048;   // binary16 of a granule of x: 32 rows of 128 bytes, a row's 16-byte pieces turned (turn_of)
+constexpr int kGranuleX = 2048;   // binary16 of a granule of x: 32 rows of 128 bytes, eight pieces of 16 (piece_at)
 constexpr int kGranuleP = 1024;   // of W: two halves of the block, each in the order of lanes of an MFMA's operand
 constexpr int kGranuleS = 32;     // float32 scales of W
 constexpr int kGroup = 8;         // blocks whose scales come into LDS together: a KB a strip
 
-// x: row m's pieces 4 part + 2 half + hi of a block, hi which eight of the half's sixteen, lie at piece ^ turn, so that the
-// 32 rows of a fragment read fall on all banks while a row's block stays one line for the kernels that write it.
-__host__ __device__ inline int64_t row_at(int m, int nb) { return (int64_t)(m >> 5) * nb * kGranuleX + (m & 31) * 64; }
+// x: row m's pieces 4 part + 2 half + hi of a block, hi which eight of the half's sixteen. Of up to kInPlaceRows rows they lie in the order of
+// an operand's lanes, piece by piece of the 32 rows: a load of an operand is whole lines (with a row's pieces beside one another the
+// product that reads them from memory took 35 cycles a load of 1 KB: 80 x 14336 x 4096 39.0 us, now 35.6). Of more rows a row's block
+// is one line for the kernels that write it, and its pieces lie at piece ^ turn, so that the 32 rows of a read from LDS fall on all banks.
+__host__ __device__ inline int64_t strip_at(int m, int nb) { return (int64_t)(m >> 5) * nb * kGranuleX; }
 __host__ __device__ inline int turn_of(int m) { return (m >> 1) & 7; }
+__host__ __device__ inline bool in_lanes(int64_t M) { return M <= kInPlaceRows; }
+__host__ __device__ inline int piece_at(int m, int piece, bool lanes) { return lanes ? piece * 256 + (m & 31) * 8 : (m & 31) * 64 + ((piece ^ turn_of(m)) << 3); }
 
 // How a row of x is held. The row's information is {exponent, form}.
 enum Form { kHalves = 0, kBlockHalves = 1, kDigitPairs = 2 };
@@ -162,6 +167,11 @@ hipError_t sum_shares(const Operands& o, int shares, hipStream_t st);
 constexpr size_t kDirectMostSums = (size_t)64 << 20;
 double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, size_t* used = nullptr);  // of sums_bytes
 hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st);
+
+// The same by a wavefront a part of K (qgemm_q4_0_parts.hip), which the two above pass on to where it is the faster.
+bool qgemm_q4_0_parts_ok(int64_t M, int64_t strips, int64_t K);
+double qgemm_q4_0_parts_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, size_t* used);
+hipError_t qgemm_q4_0_parts(Operands o, size_t sums_bytes, hipStream_t st);
 
 inline int64_t strips_of(int64_t rows) { return (rows + 31) / 32; }
 

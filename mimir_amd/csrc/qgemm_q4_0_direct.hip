@@ -1,4 +1,5 @@
-// The Q4_0 product of some rows of float32 x (about 16 to 256: short prompts, large batches), x as pairs of binary16 as in
+// The Q4_0 product of some rows of float32 x (about 16 to 256: short prompts, large batches) by rows of W of up to 2048, and of up to 24
+// rows by longer ones (more of these: qgemm_q4_0_parts.hip), x as pairs of binary16 as in
 // qgemm_q4_0_fx16.hip and with its arithmetic, W read where it lies: the pass that writes W's integers out costs as much as the
 // whole product at these sizes, and the kernel for up to eight rows a group (qgemv_q4_0_rows.hip) reads and unpacks W once
 // a group.
@@ -14,7 +15,7 @@
 // 4-byte boundary a block they cost a tenth more). Whole calls, the row kernel or the int8 form before and this:
 //   77 x 5120 x 5120   39 -> 31.6 us     128 x 14336 x 4096   80 -> 57     256 x 4096 x 14336  219 -> 94
 //   64 x 14336 x 4096  60 -> 38          77 x 4096 x 14336    77 -> 49     200 x 14336 x 4096  153 -> 85
-// and from 24 rows down the row kernel is seldom slower. Blocks' sums are those of qgemm_q4_0_fx16.hip; with K in shares and halves the error
+// (shapes that have since gone to qgemm_q4_0_parts.hip, with its times) and from 24 rows down the row kernel is seldom slower. Blocks' sums are those of qgemm_q4_0_fx16.hip; with K in shares and halves the error
 // against 64 bits is 1.05e-7 of the result at 77 x 5120 x 5120 where it was 1.63e-7.
 //
 // Rows held with an exponent a block (q4_halves.h: Form) take their scales through LDS beside x: four reads and a multiplication an output more a
@@ -68,7 +69,7 @@ __device__ __forceinline__ void direct_tile(const Operands& o, const Direct& d, 
         xg[mt] = o.X16 + ((int64_t)(s < last ? s : last) * nb + b0) * kGranuleX + col * 512 + lane * 8;
     }
 #pragma unroll
-    for (int p = 0; p < 4; p++) piece[p] = r32 * 64 + ((2 * p + q) ^ turn_of(r32)) * 8;
+    for (int p = 0; p < 4; p++) piece[p] = piece_at(r32, 2 * p + q, true);
     uint16_t* stage = (uint16_t*)lds + second * 2 * MS * kGranuleX;  // [2][MS] granules of this half
     // a thread's row of scales: of those that have one exponent, that one
     float* scales = lds + MS * kGranuleX * 2 + second * 2 * MS * 32;  // [2][MS 32] of this half
@@ -288,9 +289,17 @@ bool fits(int64_t M, int64_t strips, int64_t K) {
 
 }  // namespace
 
+// What qgemm_q4_0_parts.hip takes instead: the faster by both models, and from 161 rows up, where four workgroups read each row of W, by a tenth
+// (256 x 5120 x 5120: 54.4 us here, 58.2 there, by the models 51.5 and 49.3; 256 x 4096 x 4096: 41.0 and 32.0).
+static bool by_parts(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, double us) {
+    return qgemm_q4_0_parts_ok(M, strips, K) && qgemm_q4_0_parts_cost_us(M, strips, K, sums_bytes, nullptr) <= (M > 160 ? 0.9 * us : us);
+}
+
 double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, size_t* used) {
     Direct d{};
-    const double us = fits(M, strips, K) ? plan(M, strips, K, sums_bytes < kDirectMostSums ? sums_bytes : kDirectMostSums, &d) : 1e30;
+    if (sums_bytes > kDirectMostSums) sums_bytes = kDirectMostSums;
+    const double us = fits(M, strips, K) ? plan(M, strips, K, sums_bytes, &d) : 1e30;
+    if (by_parts(M, strips, K, sums_bytes, us)) return qgemm_q4_0_parts_cost_us(M, strips, K, sums_bytes, used);
     if (used) *used = d.shares > 1 ? (size_t)d.shares * (size_t)M * (size_t)strips * 128 : 0;
     return us;
 }
@@ -299,7 +308,11 @@ double qgemm_q4_0_direct_cost_us(int64_t M, int64_t strips, int64_t K, size_t su
 hipError_t qgemm_q4_0_direct(Operands o, size_t sums_bytes, hipStream_t st) {
     const int64_t K = (int64_t)o.nb * 32;
     Direct d;
-    if (!fits(o.M, o.parts.strips, K) || plan(o.M, o.parts.strips, K, sums_bytes < kDirectMostSums ? sums_bytes : kDirectMostSums, &d) >= 1e30) return hipErrorInvalidValue;
+    if (sums_bytes > kDirectMostSums) sums_bytes = kDirectMostSums;
+    if (!fits(o.M, o.parts.strips, K)) return hipErrorInvalidValue;
+    const double us = plan(o.M, o.parts.strips, K, sums_bytes, &d);
+    if (us >= 1e30) return hipErrorInvalidValue;
+    if (by_parts(o.M, o.parts.strips, K, sums_bytes, us)) return qgemm_q4_0_parts(o, sums_bytes, st);
     for (int i = 0; i < 3; i++)
         if (((uintptr_t)o.parts.W[i] & 3) != 0) return hipErrorInvalidValue;
     if (d.shares == 1) o.sums = nullptr;

@@ -43,8 +43,8 @@ __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restric
     const int nb = K >> 5;
     if (blockIdx.x == 0 && threadIdx.x == 0) RS[blockIdx.y] = make_int2(0, kDigitPairs);
     const float* xr = x + (int64_t)blockIdx.y * x_row_stride;
-    uint16_t* row = X16 + row_at((int)blockIdx.y, nb);
-    const int turn = turn_of((int)blockIdx.y);
+    uint16_t* strip = X16 + strip_at((int)blockIdx.y, nb);
+    const bool lanes = in_lanes(gridDim.y);
     float* xscale = XS + (int64_t)blockIdx.y * nb;
     const int nq = K >> 2;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nq; t += gridDim.x * blockDim.x) {
@@ -82,13 +82,18 @@ __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restric
             lo[k] = (_Float16)(float)(t & 8 ? -d0 : d0);  // odd blocks with their sign turned (tile_body)
             hi[k] = (_Float16)(float)(t & 8 ? -d1 : d1);
         }
-        uint16_t* at = row + (int64_t)(t >> 3) * kGranuleX;
+        uint16_t* at = strip + (int64_t)(t >> 3) * kGranuleX;
         const int piece = (t & 7) >> 1, within = 4 * (t & 1);
-        __builtin_memcpy(at + ((piece ^ turn) << 3) + within, lo, 8);
-        __builtin_memcpy(at + (((4 + piece) ^ turn) << 3) + within, hi, 8);
+        __builtin_memcpy(at + piece_at((int)blockIdx.y, piece, lanes) + within, lo, 8);
+        __builtin_memcpy(at + piece_at((int)blockIdx.y, 4 + piece, lanes) + within, hi, 8);
         if ((t & 7) == 0) xscale[t >> 3] = scale;
     }
 }
+
+// Where strips are more than half the dies. 256 x 4096 x 14336 took 92 us with a strip's rows on all of them and 88 on one; the three strips of
+// 77 x 4096 x 14336 on three dies 45 against 43.
+__host__ __device__ inline bool by_dies(int64_t M) { return in_lanes(M) && M > 128; }
+static_assert(kInPlaceRows == 8 * 32, "a strip a die");
 
 // A workgroup converts a row of x into halves: x 2^-e = h0 + h1, h0 the binary16 next to it and h1 the binary16 next to
 // what that leaves. An element is held to 2^-23 of itself (of float32's 24 bits the last may go: 2^14 + 8 - 2^-9 leaves 8 - 2^-9, which h1 rounds by
@@ -101,13 +106,16 @@ __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restric
 // is read once (4096 rows of 14336: 105 us, 156 reading it twice and storing eight bytes a thread); 0: rows of more than 16384, read twice.
 template <int ITEMS, bool NORM>
 __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restrict__ x, const float* __restrict__ w, int64_t x_row_stride, int K,
-                                                          uint16_t* __restrict__ X16, float* __restrict__ XS, int2* __restrict__ RS, float inv_k, float eps) {
+                                                          uint16_t* __restrict__ X16, float* __restrict__ XS, int2* __restrict__ RS, int M, float inv_k, float eps) {
     constexpr int kHeld = ITEMS ? ITEMS : 1;
     const int nb = K >> 5, n8 = K >> 3, tid = threadIdx.x;
-    const float* xr = x + (int64_t)blockIdx.x * x_row_stride;
-    uint16_t* row = X16 + row_at((int)blockIdx.x, nb);
-    const int turn = turn_of((int)blockIdx.x);
-    float* xscale = XS + (int64_t)blockIdx.x * nb;
+    const bool lanes = in_lanes(M);
+    // in the order of lanes a line has pieces of eight rows: a strip's rows on one die (every eighth workgroup), whose cache puts the lines together
+    const int m = by_dies(M) ? ((int)blockIdx.x & 7) * 32 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    if (m >= M) return;
+    const float* xr = x + (int64_t)m * x_row_stride;
+    uint16_t* strip = X16 + strip_at(m, nb);
+    float* xscale = XS + (int64_t)m * nb;
     __shared__ uint32_t part[2][4];
     float scale = 1.f;
     if (NORM) {
@@ -184,7 +192,7 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
     auto exponent = [](float a) { return a > 0.f ? __builtin_amdgcn_frexp_expf(a) - 15 : 0; };  // a 2^-e in [2^14, 2^15)
     const int e_row = finite ? exponent(amax) : 0;
     const int form = finite && amin < amax * 0x1p-15f ? kBlockHalves : kHalves;
-    if (tid == 0) RS[blockIdx.x] = make_int2(finite ? e_row : INT32_MAX, form);
+    if (tid == 0) RS[m] = make_int2(finite ? e_row : INT32_MAX, form);
     auto convert = [&](int t, const float u[8]) {
         const int e = form == kBlockHalves ? exponent(__builtin_bit_cast(float, block_top(u))) : e_row;
         const bool odd = t & 4;  // odd blocks with their sign turned (tile_body)
@@ -195,9 +203,9 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
             h0[k] = (_Float16)a;
             h1[k] = (_Float16)(a - (float)h0[k]);
         }
-        uint16_t* at = row + (int64_t)(t >> 2) * kGranuleX;
-        *(f16x8*)(at + (((t & 3) ^ turn) << 3)) = h0;
-        *(f16x8*)(at + (((4 + (t & 3)) ^ turn) << 3)) = h1;
+        uint16_t* at = strip + (int64_t)(t >> 2) * kGranuleX;
+        *(f16x8*)(at + piece_at(m, t & 3, lanes)) = h0;
+        *(f16x8*)(at + piece_at(m, 4 + (t & 3), lanes)) = h1;
         if ((t & 3) == 0) xscale[t >> 2] = finite ? __builtin_ldexpf(1.f, e) : __builtin_nanf("");
     };
     if (ITEMS) {
@@ -298,7 +306,7 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
     const int r32 = lane & 31, hi = lane >> 5;
     int piece_off[4];  // of pieces 2 p + hi: half p % 2 of part p / 2
 #pragma unroll
-    for (int p = 0; p < 4; p++) piece_off[p] = wm * MT * 4096 + r32 * 128 + ((2 * p + hi) ^ turn_of(r32)) * 16;
+    for (int p = 0; p < 4; p++) piece_off[p] = wm * MT * 4096 + piece_at(r32, 2 * p + hi, in_lanes(M)) * 2;
     const int b_off = S::kChunksX * 1024 + wn * NT * 2048 + lane * 16;
 
     f32x16 acc[MT][NT], zero;
@@ -641,7 +649,7 @@ static void launch_halves(const float* x, const float* w, double eps, int64_t M,
     int2* RS = (int2*)(X16 + strips_of(M) * (K / 32) * kGranuleX);
     float* XS = (float*)(RS + M);
     const auto kernel = K <= 4096 ? fx16_halves_kernel<2, NORM> : K <= 16384 ? fx16_halves_kernel<8, NORM> : fx16_halves_kernel<0, NORM>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)M), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (float)(1.0 / (double)K), (float)eps);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(by_dies(M) ? 256 : M)), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (int)M, (float)(1.0 / (double)K), (float)eps);
 }
 
 hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, Fx16 form, hipStream_t st) {

@@ -124,6 +124,31 @@ def test_rows_held_by_block_among_others(m):
     assert min(took[1]) <= 1.5 * min(took[0]), (min(took[1]), min(took[0]))
 
 
+@pytest.mark.parametrize("m", [25, 32, 33, 48, 49, 80, 81, 112, 128, 129, 160, 161, 256])
+@pytest.mark.parametrize("n,k", [(97, 2112), (513, 4224), (64, 9280)])
+@pytest.mark.parametrize("rows", ["even", "wide"])
+def test_a_wavefront_a_part_of_k(m, n, k, rows):
+    """Rows of W of more than 2048: every number of sixteens of rows, a sixteen and a tile begun and filled, columns that fill no strip; 66, 132 and
+    290 blocks, which leave some parts less than a chunk of eight blocks, and a last chunk that reaches back. Bound as in test_pairs_of_halves."""
+    rng = np.random.default_rng(m + n + k)
+    raw = random_blocks(rng, O.Q4_0, n * k)
+    x = (rng.normal(size=(m, k)) * np.exp(rng.normal(size=(m, 1)) * 3)).astype(np.float32)
+    if rows == "wide":
+        x[m // 3, :32] *= 2.0 ** 30
+        x[m - 1, k - 32:] *= 2.0 ** -40
+    buf, ptr = gpu.dev_bytes_at(raw, 4)
+    gpu.say(f"q4_0 parts M={m} N={n} K={k} {rows}")
+    try:
+        tuned(0, 3)
+        got = gpu.dev(gpu.qgemv(O.Q4_0, ptr, gpu.dev(x), n, k)).double()
+        assert last_kernel().startswith(IN_PLACE) and (m > 160 or "parts of it a wavefront" in last_kernel())
+    finally:
+        tuned(0, 1)
+    x64, w = gpu.dev(x).double(), gpu.dev(O.dequantize(O.Q4_0, raw).reshape(n, k)).double()
+    bound = 2e-6 * (x64.abs() @ w.abs().T) + 2.0 ** -23 * (x64.abs().reshape(m, -1, 32).amax(2) @ w.abs().reshape(n, -1, 32).sum(2).T) + 1e-30
+    assert ((got - x64 @ w.T).abs() <= bound).all()
+
+
 def prompt_model(batch, prompt, embed, hidden, heads, kv_heads, head_dim, layers):
     c = capi.LlamaConfig()
     c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab = embed, hidden, layers, heads, kv_heads, head_dim, head_dim, 515
@@ -187,6 +212,29 @@ def test_gate_and_up_are_one_product(rows, embed, hidden, kernel):
     finally:
         tuned(0, 1)
     assert ran == kernel
+    want = om.logits(tokens[0].tolist(), om.new_caches(c.context, O.F32), all=True)
+    scale = np.abs(want).max()
+    assert np.abs(got - want).max() <= 0.02 * scale and np.median(np.abs(got - want)) <= 1e-5 * scale
+
+
+@pytest.mark.parametrize("rows,hidden,shares", [(40, 96, 5), (130, 2080, 1)])
+def test_gate_and_up_by_parts_of_k(rows, hidden, shares):
+    """The same by rows of W of 2112, SwiGLU in the tile and with the shares' sums; hidden that fills no group of strips."""
+    c = prompt_model(1, rows, 2112, hidden, 33, 1, 64, 1)
+    om = OL.synthetic(_oracle_config(c), seed=6, centered=True)
+    om.blocks[0].down = OL._q_blocks(np.random.default_rng(8), O.Q8_0, 2112, hidden)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(rows)
+    tokens = np.random.default_rng(1).integers(0, c.vocab, (1, rows))
+    try:
+        gpu.say(f"gate and up by parts, rows={rows} hidden={hidden}")
+        tuned(0, 3)
+        got = m.logits(tokens, all=True)[0]
+        ran = last_kernel()
+    finally:
+        tuned(0, 1)
+    assert f"{shares} shares of K, parts of it a wavefront" in ran
     want = om.logits(tokens[0].tolist(), om.new_caches(c.context, O.F32), all=True)
     scale = np.abs(want).max()
     assert np.abs(got - want).max() <= 0.02 * scale and np.median(np.abs(got - want)) <= 1e-5 * scale

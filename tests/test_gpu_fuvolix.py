@@ -7,8 +7,9 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
-from mimir_amd import capi, registry
+from mimir_amd import capi, registry, stack
 from oracle import fuvolix as F
 from tests import fuvolix as X
 from tests import gpu
@@ -350,3 +351,31 @@ def test_trace_replay(tmp_path, mixed, dtype):
     for step, rows in ((0, [0, 49]), (2, [52]), (3, [11, 3])):
         got = np.fromfile(out / f"{step}.f32", "<f4").reshape(len(rows), c["vocab"])
         assert X.error(got, want[rows]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("rows", [2, 4, 5, 8])
+def test_few_rows_by_wide_matrices(rows):
+    """One position of `rows` sequences against each of them alone: products of few rows by 8224 (a last round of a few workgroups), 8192 and 2048 rows of W, K
+    2048 and 8192. A row alone is multiplied as float32, several as the sum of two bfloat16 (2^-17 of an element at most); six products on a path
+    with terms of either sign, whose sums are some ten times smaller than their terms': 6 * 10 * 2^-17."""
+    c = dict(width=2048, vocab=515, canon=dict(taps=4), norm=dict(groups=2, eps=1e-6), logit_scale=1.0,
+             layers=[dict(type="mlstm", mixer=dict(heads=16, dim=128, vdim=128, gate_cap=15.0), mlp=dict(kind="dense", ff=8192))])
+    g = torch.Generator().manual_seed(rows)
+    tokens = np.arange(7, 7 + rows, dtype=np.int32).reshape(rows, 1) * 31 % 515
+
+    def model(batch, data):
+        m = stack.Stack(*stack.CONFIGS["Fuvolix"](c, 8, batch))
+        for name, n, k in m.tensors():
+            if name not in data:
+                data[name] = (torch.randn(n, k, generator=g) * (k ** -0.5 if n > 1 else 0.02) + (1.0 if "norm" in name else 0.0)).to(torch.bfloat16)
+            m.set_tensor(name, capi.BF16, data[name].view(torch.int16).numpy().view(np.uint16), n * k)
+        m.finalize(1)
+        return m
+    data = {}
+    gpu.say(f"fuvolix few rows {rows}")
+    together, alone = model(rows, data), model(1, data)
+    got = together.logits(tokens)
+    for i in range(rows):
+        alone.reset()
+        want = alone.logits(tokens[i:i + 1])[0]
+        assert np.linalg.norm(got[i] - want) <= 6 * 10 * 2.0 ** -17 * np.linalg.norm(want)

@@ -369,21 +369,31 @@ static size_t rows_lds(int dt, int64_t nsb, int tiles, int waves) {
            (size_t)((nsb + 7) & ~7) * (dt == kQ4_K ? 2 : 1) * kRows * 16 * tiles * sizeof(float);
 }
 
-// Two rows of x or more, converted (kq_convert_act); the terms of sixteen rows of W in LDS; Q4_K's W 16-byte aligned, Q6_K's on an even address.
+// Rows of x, converted (kq_convert_act); the terms of sixteen rows of W in LDS; Q4_K's W 16-byte aligned, Q6_K's on an even address.
 bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a) {
     const int64_t nsb = a.K / 256;
-    return (dt == kQ4_K || dt == kQ6_K) && g_kq_rows != 1 && a.M >= 2 && a.M <= 8 * 65535 && a.act && a.K % 256 == 0 && nsb > 0 &&
+    return (dt == kQ4_K || dt == kQ6_K) && g_kq_rows != 1 && a.M >= 1 && a.M <= 8 * 65535 && a.act && a.K % 256 == 0 && nsb > 0 &&
            ((uintptr_t)a.W & (dt == kQ4_K ? 15 : 1)) == 0 && ((uintptr_t)a.act & 15) == 0 && a.N > 0 && a.N <= (1ll << 30) &&
            rows_lds(dt, nsb, 1, 4) <= 160 * 1024;
 }
 
-// Where it is the faster choice. Up to eight rows always; beyond, by what both kernels take: here 3 us, then W from memory once and once from
+// One converted row: the kernels that give a row of W to a wavefront (qgemv_kquant.hip) have little to read a wavefront where rows are short, and
+// a long serial chain of terms where they are long and too few to hide it. us in a decoding step, there | here: Q4_K 16384 x 2048 9.8 | 7.5, 8192 x 1024
+// 6.0 | 5.1, 4096 x 14336 11.6 | 10.4; Q6_K 16384 x 2048 9.7 | 9.0, 8192 x 1024 5.8 | 5.3; but Q4_K 28672 x 4096 17.8 | 21.2, 2048 x 8192 5 | 6.8,
+// Q6_K 4096 x 14336 15 | 14.4 and 28672 x 4096 24.6 | 26.9.
+static bool one_row_pays(int dt, const QGemvArgs& a) {
+    const int64_t nsb = a.K / 256;
+    return (nsb <= 8 && a.N >= 8192) || (dt == kQ4_K && nsb >= 48 && a.N > 2048 && a.N <= 4096);
+}
+
+// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us, then W from memory once and once from
 // the caches per group of eight rows (5.7 TB/s Q4_K, 6.2 TB/s Q6_K), the tiled kernel of qgemm_kquant.hip about 2.1 us per super-block of
 // K and round of 128 tiles of 128 x 128. Measured, us, here | there, Q4_K: 32 x 14336 x 4096 28.5 | 31.6, 40 rows 34.4 | 31.8; 32 x 28672
 // x 4096 55 | 61, 40 rows 67 | 62; 64 x 4096 x 14336 62 | 109, 128 rows 121 | 118; 64 x 1024 x 4096 5.4 | 32. Q6_K: 16 x 14336 x 4096 24.6 | 32.2, 32 rows 37.5 | 32.5.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
-    if (g_kq_rows == 2 || a.M <= 8) return true;
+    if (g_kq_rows == 2 || (a.M >= 2 && a.M <= 8)) return true;
+    if (a.M == 1) return one_row_pays(dt, a);
     if (a.M > 512) return false;
     const double nsb = (double)(a.K / 256), groups = (double)((a.M + kRows - 1) / kRows);
     // (rows of more than 32 super-blocks leave room for one workgroup a compute unit)

@@ -753,6 +753,20 @@ def test_kquant_rows_kernel_at_the_edges_of_its_forms(dt, m, n, k):
 
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("n,k", [(8191, 256), (8192, 256), (8199, 256 * 8), (8192, 256 * 9), (2048, 256 * 48), (2049, 256 * 48), (4096, 256 * 48),
+                                 (4097, 256 * 48), (2050, 256 * 47), (2051, 256 * 75)])
+def test_one_converted_row_of_kquants_on_either_side_of_the_choice(dt, n, k):
+    """A row by the kernel for several where that is the faster, at the edges of the rule and by the other kernel: the oracle's bits."""
+    rng = np.random.default_rng(dt + n + k)
+    raw = random_blocks(rng, dt, 64 * k).reshape(64, -1)
+    raw = np.ascontiguousarray(raw[np.arange(n) * 37 % 64])
+    x = rng.normal(size=(1, k)).astype(np.float32)
+    buf, ptr = gpu.dev_bytes_at(raw.reshape(-1), 0)
+    gpu.say(f"kquant one converted row dt={dt} N={n} K={k}")
+    assert bits_equal(gpu.qgemv_act(dt, ptr, gpu.dev(x), n, k), O.qmatmul(dt, raw.reshape(-1), x, n, k))
+
+
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
 def test_kquant_rows_kernel_at_the_largest_integer_sums(dt):
     """Every quant and scale at its largest magnitude with x at +-127 per super-block (backend/cpu/quant_test.go:164-204), through the
     kernel that reads W once per eight rows of x: its 24-bit multiplies and int32 sums hold what the CPU's int32 arithmetic holds."""

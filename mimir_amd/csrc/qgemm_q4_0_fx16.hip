@@ -104,15 +104,14 @@ static_assert(kInPlaceRows == 8 * 32, "a strip a die");
 // With NORM the row is normalized first (rmsnorm_kernel's operations, one by one): x over its root mean square, times w.
 // Memory bounds it: 8 bytes an element. ITEMS: eights of elements a thread holds between the row's maximum and its halves, so that x
 // is read once (4096 rows of 14336: 105 us, 156 reading it twice and storing eight bytes a thread); 0: rows of more than 16384, read twice.
-template <int ITEMS, bool NORM>
+template <int ITEMS, bool NORM, bool LANES>
 __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restrict__ x, const float* __restrict__ w, int64_t x_row_stride, int K,
                                                           uint16_t* __restrict__ X16, float* __restrict__ XS, int2* __restrict__ RS, int M, float inv_k, float eps) {
     constexpr int kHeld = ITEMS ? ITEMS : 1;
     const int nb = K >> 5, n8 = K >> 3, tid = threadIdx.x;
-    const bool lanes = in_lanes(M);
     // in the order of lanes a line has pieces of eight rows: a strip's rows on one die (every eighth workgroup), whose cache puts the lines together
-    const int m = by_dies(M) ? ((int)blockIdx.x & 7) * 32 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
-    if (m >= M) return;
+    const int m = LANES && by_dies(M) ? ((int)blockIdx.x & 7) * 32 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    if (LANES && m >= M) return;
     const float* xr = x + (int64_t)m * x_row_stride;
     uint16_t* strip = X16 + strip_at(m, nb);
     float* xscale = XS + (int64_t)m * nb;
@@ -204,8 +203,8 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
             h1[k] = (_Float16)(a - (float)h0[k]);
         }
         uint16_t* at = strip + (int64_t)(t >> 2) * kGranuleX;
-        *(f16x8*)(at + piece_at(m, t & 3, lanes)) = h0;
-        *(f16x8*)(at + piece_at(m, 4 + (t & 3), lanes)) = h1;
+        *(f16x8*)(at + piece_at(m, t & 3, LANES)) = h0;
+        *(f16x8*)(at + piece_at(m, 4 + (t & 3), LANES)) = h1;
         if ((t & 3) == 0) xscale[t >> 2] = finite ? __builtin_ldexpf(1.f, e) : __builtin_nanf("");
     };
     if (ITEMS) {
@@ -648,7 +647,9 @@ static void launch_halves(const float* x, const float* w, double eps, int64_t M,
     uint16_t* X16 = (uint16_t*)act;
     int2* RS = (int2*)(X16 + strips_of(M) * (K / 32) * kGranuleX);
     float* XS = (float*)(RS + M);
-    const auto kernel = K <= 4096 ? fx16_halves_kernel<2, NORM> : K <= 16384 ? fx16_halves_kernel<8, NORM> : fx16_halves_kernel<0, NORM>;
+    const auto rows = K <= 4096 ? fx16_halves_kernel<2, NORM, false> : K <= 16384 ? fx16_halves_kernel<8, NORM, false> : fx16_halves_kernel<0, NORM, false>;
+    const auto by_lanes = K <= 4096 ? fx16_halves_kernel<2, NORM, true> : K <= 16384 ? fx16_halves_kernel<8, NORM, true> : fx16_halves_kernel<0, NORM, true>;
+    const auto kernel = in_lanes(M) ? by_lanes : rows;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(by_dies(M) ? 256 : M)), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (int)M, (float)(1.0 / (double)K), (float)eps);
 }
 

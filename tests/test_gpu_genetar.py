@@ -7,6 +7,7 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
 from mimir_amd import capi, registry, stack
 from oracle import fuvolix as F
@@ -407,3 +408,26 @@ def test_trace_replay(tmp_path, mixed, dtype):
     for step, rows in ((0, [0, 49]), (2, [52]), (3, [11, 3])):
         got = np.fromfile(out / f"{step}.f32", "<f4").reshape(len(rows), c["vocab"])
         assert X.error(got, want[rows]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("width,ff", [(1024, 8192), (1088, 7232), (1024, 15360)])
+def test_one_row_by_long_rows_of_the_output_and_down_projection(width, ff):
+    """One position of a sequence against the same as one of two: attention's output and the down projection as one product of K heads * 128 + ff
+    (9216; 8256, pieces that end within a step; 16384), the part below split with a factor of its own. A row alone is multiplied as float32, two as
+    the sum of two bfloat16 (2^-17 of an element): five products on a path, their sums some ten times smaller than their terms'."""
+    heads = 8
+    mixer = dict(heads=heads, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5, softcap=30.0, v_mix=True)
+    c = dict(width=width, vocab=515, norm=dict(groups=2, eps=1e-6), logit_scale=1.0, embedding=dict(bigram=dict(buckets=515, mul_prev=31, mul_cur=7)),
+             canon=dict(taps=4), layers=[dict(type="attention", mixer=mixer, mlp=dict(kind="dense", ff=ff)) for _ in range(2)])
+    g = torch.Generator().manual_seed(ff)
+    data, got = {}, []
+    gpu.say(f"genetar one row width={width} ff={ff}")
+    for batch in (1, 2):
+        m = stack.Stack(*stack.CONFIGS["Genetar"](c, 8, batch))
+        for name, n, k in m.tensors():
+            if name not in data:
+                data[name] = (torch.randn(n, k, generator=g) * (k ** -0.5 if n > 1 else 0.1) + (1.0 if n == 1 else 0.0)).to(torch.bfloat16)
+            m.set_tensor(name, capi.BF16, data[name].view(torch.int16).numpy().view(np.uint16), n * k)
+        m.finalize(1)
+        got.append(m.logits(np.array([[7], [11]], np.int32)[:batch])[0])
+    assert np.linalg.norm(got[0] - got[1]) <= 5 * 10 * 2.0 ** -17 * np.linalg.norm(got[1])

@@ -446,7 +446,8 @@ static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, co
     if constexpr (DT == kQ4_K) {
         if (wgs <= 512 && fits(2, 16)) return launch_depth<DT, 2, 16, ROPE>(a, st, bf16, rope);
     } else {
-        if (wgs <= 512 && nsb <= 16 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
+        // (eight wavefronts to 32 super-blocks, two rounds of theirs: 8 x 8192 x 7168 19.4 -> 18.2 us, 2 x 4975 x 4352 13.3 -> 12.1)
+        if (wgs <= 512 && nsb <= 32 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
     }
     if (fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     return launch_depth<DT, 1, 4, ROPE>(a, st, bf16, rope);

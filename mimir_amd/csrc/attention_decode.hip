@@ -529,9 +529,6 @@ void attention_decode_plan(int64_t B, int H, int HK, int64_t kmax, int* nsplit, 
     // the scores and the weighted values of a share take half as long, the hand-over a little longer.
     const int64_t aim = g_share_keys.load(std::memory_order_relaxed);
     int64_t by_keys = (kmax + aim - 1) / aim;
-    // Up to 128 keys are one share: its second trip to memory costs less than the hand-over (64 steps from 64 positions on 16.24 -> 15.90 ms, eight
-    // sequences' 32 from 90 15.75 -> 15.63; one share of 192 keys 9.39 ms where three have 9.11).
-    if (kmax <= 128) by_keys = 1;
     const bool short_shares = by_keys <= kGather;
     if (!short_shares) by_keys = (kmax + 127) / 128;
     // Shares of 64 keys are worth three workgroups a compute unit (eight sequences at 768 positions: 12 shares of 64 keys

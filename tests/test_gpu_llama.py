@@ -366,6 +366,38 @@ def test_batch_step_that_reads_weights_once_chooses_the_same_tokens(batch):
             assert a == w, f"token {i}: device {a}, oracle {w}, oracle's margin there {margins[i]:.4g}"
 
 
+@pytest.mark.parametrize("linear_dt,batch,cache", [(O.Q4_0, 1, capi.F32), (O.Q4_0, 8, capi.F16), (O.Q4_K, 3, capi.F16), (O.Q6_K, 1, capi.F32)])
+def test_steps_of_a_context_of_96_share_its_keys_between_two_workgroups(linear_dt, batch, cache):
+    """65 to 128 positions are two shares of the keys ("attention.share": 64), whose hand-over leaves the result in each form that a step
+    reads. The caches that ten steps from position 70 on fill give the logits of a model held to two shares bit for bit; held to one, which adds in another
+    order, those of a difference of some 1e-7 (K-quants: 2 %, the bound of quantized weights, since their int8 rounding is a step)."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, cache)
+    om = OL.synthetic(_oracle_config(c), seed=4, linear_dt=linear_dt, output_dt=O.Q4_0)
+    prompts = np.random.default_rng(29).integers(0, c.vocab, (batch, 70))
+    got = {}
+    try:
+        capi.check(lib.mi355x_tune(b"llama.step", 1))
+        for shares in (0, 2, 1):
+            gpu.say(f"context of 96, dtype {linear_dt}, batch {batch}, shares {shares}")
+            capi.check(lib.mi355x_tune(b"attention.splits", shares))  # before the model sizes its workspaces
+            m = Llama(c)
+            _upload_synthetic(m, om)
+            m.finalize(80)
+            m.generate(prompts, 11)
+            capi.check(lib.mi355x_tune(b"attention.splits", 0))
+            got[shares] = m.logits(np.full((batch, 1), 7))
+            m.close()
+    finally:
+        capi.check(lib.mi355x_tune(b"attention.splits", 0))
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    assert np.array_equal(got[0], got[2])
+    if linear_dt == O.Q4_0:  # (int8 rounding may swallow the difference)
+        assert not np.array_equal(got[0], got[1])
+    scale = np.abs(got[1]).max()
+    assert np.abs(got[0] - got[1]).max() <= (1e-3 if linear_dt == O.Q4_0 else 0.02) * scale
+
+
 @pytest.mark.parametrize("embed,vocab,batch", [(512, 8192, 1), (512, 8195, 3), (4160, 8195, 2), (512, 70001, 9)])
 def test_the_choice_brings_in_the_next_embedding(embed, vocab, batch):
     """From 8192 tokens on, the launch that chooses a step's tokens also records them, moves the position on and looks the next step's

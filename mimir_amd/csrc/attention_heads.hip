@@ -555,7 +555,7 @@ __global__ __launch_bounds__(256) void heads_combine_kernel(HeadAttention a, Par
 
 // 16 bytes a lane from a wavefront's address and a lane's offset into LDS (load_to_lds, gemm_nt_tile.h).
 __device__ __forceinline__ void load_to_lds(const void* g, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(g) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(g) : "memory");
 }
 __device__ __forceinline__ f32x16 mfma_bf16(u32x4 a, u32x4 b, f32x16 c) { return Bf16Element::mfma(a, b, c); }
 

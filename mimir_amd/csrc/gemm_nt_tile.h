@@ -52,9 +52,10 @@ struct Bf16Element {
 // 16 bytes a lane from global memory into LDS: lane l's piece lands at lds_base + 16 l. Written out because the
 // compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand.
 // The instruction takes its LDS base from M0, which the compiler does not let an asm statement name as clobbered: nothing
-// else in this kernel uses M0 (no dynamically indexed registers, no LDS-direct reads), and it is set anew before every load.
+// else in this kernel uses M0 (no dynamically indexed registers, no LDS-direct reads), and it is set anew before every load. A load into
+// LDS needs a wait state behind a scalar write of M0 (the compiler, which does not look into an asm statement, puts s_nop 0 there itself).
 __device__ __forceinline__ void load_to_lds(const void* g, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(g) : "memory");
 }
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

@@ -145,9 +145,9 @@ __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t lo, uint32_t hi, int ha
 // compiler, given the builtin, waits for every load under way before any LDS access; these loads are counted by hand
 // (the compiler does not see them, so its own waits for the register loads of the scales can only be longer than
 // needed, never shorter: loads return in order). The instruction takes its LDS base from M0, which an asm statement
-// cannot name as clobbered: nothing else in these kernels uses M0, and it is set anew before every load.
+// cannot name as clobbered: nothing else in these kernels uses M0, and it is set anew before every load (s_nop: gemm_nt_tile.h).
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane16, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(lane16), "s"(base) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }

@@ -44,7 +44,7 @@ static_assert(kLdsBytes <= 160 * 1024 && kWaves / 2 * kMostTiles * kCols * 4 * 6
 
 // A wavefront's sixteen bytes a lane from `from` to lds_base + 16 lane, as load_to_lds with an address a lane.
 __device__ __forceinline__ void load_piece(const uint8_t* from, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(from) : "memory");
 }
 
 // x's granules as a buffer, so that an address is a lane's offset and a scalar one: 2 VALU instructions a load fewer.

@@ -64,7 +64,7 @@ __device__ long long* g_dma_stamps_dev = nullptr;
 // 16 bytes a lane from global memory into LDS: lane l's piece lands at lds_base + OFF + 16 l, read from g + OFF.
 template <int OFF>
 __device__ __forceinline__ void dma16(const void* g, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off offset:%2" ::"s"(lds_base), "v"(g), "n"(OFF) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2" ::"s"(lds_base), "v"(g), "n"(OFF) : "memory");
 }
 __device__ __forceinline__ void gload16(u32x4& v, const void* g) { asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(v) : "v"(g) : "memory"); }
 __device__ __forceinline__ void gload4(float& v, const void* g) { asm volatile("global_load_dword %0, %1, off" : "=&v"(v) : "v"(g) : "memory"); }

@@ -253,8 +253,10 @@ __global__ __launch_bounds__(64 * kWaves) void qgemm_q4_0_parts_kernel(Operands 
 #pragma unroll
     for (int i = 0; i < (MT * 16 + 63) / 64; i++) by_block |= info[i].y == kBlockHalves;
     by_block = __ballot(by_block) != 0;
-    if (by_block) tile.template run<true>(nchunks, acc);
-    else tile.template run<false>(nchunks, acc);
+    if (nchunks > 0) {  // a share of fewer pairs of blocks than parts leaves some without: nothing of x's is theirs to read
+        if (by_block) tile.template run<true>(nchunks, acc);
+        else tile.template run<false>(nchunks, acc);
+    }
 
     // The parts' sums: the upper two's to the lower two, these two's to whichever wavefront stores them. A loop over tiles, not their
     // code one after the other: run once a launch, it would be fetched as slowly as it is long.

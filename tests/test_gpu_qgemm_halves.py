@@ -129,7 +129,8 @@ def test_rows_held_by_block_among_others(m):
 @pytest.mark.parametrize("rows", ["even", "wide"])
 def test_a_wavefront_a_part_of_k(m, n, k, rows):
     """Rows of W of more than 2048: every number of sixteens of rows, a sixteen and a tile begun and filled, columns that fill no strip; 66, 132 and
-    290 blocks, which leave some parts less than a chunk of eight blocks, and a last chunk that reaches back. Bound as in test_pairs_of_halves."""
+    290 blocks, which leave some parts less than a chunk of eight blocks or none at all (161 x 97 x 2112: a last share of two blocks for eight of
+    them), and a last chunk that reaches back. Bound as in test_pairs_of_halves."""
     rng = np.random.default_rng(m + n + k)
     raw = random_blocks(rng, O.Q4_0, n * k)
     x = (rng.normal(size=(m, k)) * np.exp(rng.normal(size=(m, 1)) * 3)).astype(np.float32)

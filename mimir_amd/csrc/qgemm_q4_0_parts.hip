@@ -31,8 +31,7 @@ constexpr int kRowBytes = kChunk * 18, kPieces = kRowBytes / 16, kChunkBytes = 6
 
 struct Plan {
     int sides, groups;         // of two strips of W, of as many sides
-    int tiles_m, mt;           // of mt sixteens of rows
-    int tiles;                 // of up to 128 rows: of more than five sixteens they are taken as two of half
+    int tiles_m, mt;           // of mt sixteens of rows: 128 rows are one, more than five sixteens of them two of half
     int shares, share_blocks;  // of K; the last share may be shorter, all are even
 };
 
@@ -361,7 +360,7 @@ double plan(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, Plan* out) 
             if (shares > 1) us += 1.1 + (double)sums * 1.1e-6;
             if (us < best) {
                 best = us;
-                *out = Plan{sides, (int)groups, (int)tiles, mt, (int)of_tile, (int)shares, (int)blocks};
+                *out = Plan{sides, (int)groups, (int)tiles, mt, (int)shares, (int)blocks};
             }
         }
     }
@@ -395,9 +394,7 @@ hipError_t qgemm_q4_0_parts(Operands o, size_t sums_bytes, hipStream_t st) {
     if (e) return e;
     if (d.shares > 1)
         if (hipError_t e = sum_shares(o, d.shares, st)) return e;
-    // by tiles of up to four strips of x and of W, as qgemm_q4_0_direct_kernel has them, and what a workgroup takes of one
-    note_kernel("qgemm_q4_0_direct_kernel<%d>: %d x %d tiles, %d shares of K, parts of it a wavefront, %d x %d a workgroup",
-                d.tiles > 1 ? 4 : (int)strips_of(o.M), d.tiles, (o.parts.strips + 3) / 4, d.shares, 16 * d.mt, 64 * d.sides);
+    note_kernel("qgemm_q4_0_parts_kernel<%d>: %d x %d tiles of %d x %d, %d shares of K", d.mt, d.tiles_m, d.groups, 16 * d.mt, 64 * d.sides, d.shares);
     return hipGetLastError();
 }
 

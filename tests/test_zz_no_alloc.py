@@ -155,7 +155,7 @@ def last_kernel():
 
 
 @pytest.mark.parametrize("m,n,k,kernels", [
-    (32, 14336, 4096, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")), (48, 5120, 5120, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")),
+    (32, 14336, 4096, ("qgemm_q4_0_parts_kernel", "qgemm_q4_0_parts_kernel")), (48, 5120, 5120, ("qgemm_q4_0_parts_kernel", "qgemm_q4_0_parts_kernel")),
     (200, 32768, 1024, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")), (256, 32768, 1024, ("qgemm_q4_0_direct_kernel", "qgemm_q4_0_direct_kernel")),
     (300, 65536, 1024, ("qgemm_q4_0_fx16_kernel", "qgemm_q4_0_fx_kernel")), (512, 32768, 512, ("qgemm_q4_0_fx16_kernel", "qgemm_q4_0_fx_kernel")),
     (1000, 2048, 256, ("qgemm_q4_0_fx_kernel", "qgemm_q4_0_fx_kernel"))])

@@ -418,25 +418,38 @@ static hipError_t launch_kq_rows(const QGemvArgs& a, hipStream_t st, bool bf16, 
     return hipGetLastError();
 }
 
-// By the super-blocks that a wavefront takes: sixteen wavefronts hold two under way within their 128 registers, fewer four.
+// By the super-blocks that a wavefront takes: as many under way as it takes in one round or two, sixteen wavefronts hold two within their 128 registers,
+// fewer four. (Three of three: with four asked for, 4 x 12480 x 2304 Q4_K took 10.1 us, so 8.5; four for six, 25 x 12288 x 4608 34.6, three in two rounds 32.0.)
+// What launch_shape() does not come to has the loop of any length.
 template <int DT, int TILES, int WAVES, bool ROPE>
 static hipError_t launch_depth(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int64_t each = (a.K / 256 + WAVES - 1) / WAVES;
     if (each <= 1) return launch_kq_rows<DT, TILES, WAVES, 1, 1, ROPE>(a, st, bf16, rope);
-    if (each <= 2) return launch_kq_rows<DT, TILES, WAVES, 2, 1, ROPE>(a, st, bf16, rope);
+    if constexpr (WAVES != 16 || TILES == 1)
+        if (each <= 2) return launch_kq_rows<DT, TILES, WAVES, 2, 1, ROPE>(a, st, bf16, rope);
     if constexpr (WAVES == 16) {
-        if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 2, 2, ROPE>(a, st, bf16, rope);
+        if constexpr (TILES == 1)
+            if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 2, 2, ROPE>(a, st, bf16, rope);
         return launch_kq_rows<DT, TILES, WAVES, 2, 0, ROPE>(a, st, bf16, rope);
     } else {
-        if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 4, 1, ROPE>(a, st, bf16, rope);
-        if (each <= 8) return launch_kq_rows<DT, TILES, WAVES, 4, 2, ROPE>(a, st, bf16, rope);
+        if (each == 3) return launch_kq_rows<DT, TILES, WAVES, 3, 1, ROPE>(a, st, bf16, rope);
+        if (each == 4) return launch_kq_rows<DT, TILES, WAVES, 4, 1, ROPE>(a, st, bf16, rope);
+        if (each <= 6) return launch_kq_rows<DT, TILES, WAVES, 3, 2, ROPE>(a, st, bf16, rope);
+        if constexpr (TILES == 1)
+            if (each <= 8) return launch_kq_rows<DT, TILES, WAVES, 4, 2, ROPE>(a, st, bf16, rope);
         return launch_kq_rows<DT, TILES, WAVES, 4, 0, ROPE>(a, st, bf16, rope);
     }
 }
 
-// Measured at eight rows of x, us: one tile in 16 | 8 | 4 wavefronts 4096 x 14336 Q4_K 12.1 | 13.6 | 13.4, Q6_K 14.7 | 17.3 | 15.9, 4096 x 4096 4.8 |
-// 5.5 | 6.0, 6.1 | 6.9 | 8.1: the most where there is at most one workgroup a compute unit. Two tiles in 16 | 8 | 4: 6144 x 4096 Q4_K 6.9 | 7.4 |
-// 8.6, Q6_K (no room for 16) - | 8.1 | 10.2; 28672 x 4096 23 | 26 | 20-22: four where there are more than two workgroups a unit.
+// By the sixteens of rows of W, times groups of x, and the super-blocks of a row. us a call on converted rows, tiles x wavefronts (a product not named 8 rows):
+//   up to 256 sixteens, one workgroup a compute unit: 1 x 16 | 1 x 8 | 1 x 4, 4096 x 14336 Q4_K 12.1 | 13.6 | 13.4, Q6_K 14.7 | 17.3 | 15.9
+//   up to 512, two tiles: Q4_K 2 x 16 while it fits (16 super-blocks), 6144 x 4096 6.9, 2 x 8 7.4; then 2 x 8: 2 x 6912 x 4608 9.0, 2 x 4 10.7, 1 x 4 9.4; of more
+//     than 48 super-blocks 2 x 4: 4 x 7296 x 13824 20.0, 1 x 4 20.5. Q6_K 2 x 8 to 32 super-blocks: 8 x 8192 x 7168 17.4, 2 x 4 18.5; then 2 x 4: 4 x 4352 x 12544 21.8, 1 x 4 24.9
+//   beyond, one tile, so that three to five workgroups share a unit: 1 x 4 | 2 x 4, Q4_K 16 x 13568 x 7424 32.2 | 44.7, 88 x 4032 x 7936 43.1 | 66.1, 8 x 12032 x 4096
+//     11.7 | 13.3; Q6_K 4 x 8512 x 6400 20.1 | 23.5, 72 x 3776 x 7936 44.2 | 53.3. Two tiles where the operand of x that they share is what counts: short rows by many groups (Q4_K 188
+//     x 960 x 1536 1 x 4 9.0 | 2 x 4 8.5, 61 x 2688 x 1536 7.6 | 7.1; 45 x 4480 x 1280 8.0 | 8.8), short rows of Q6_K from 1200 sixteens on (1 x 20480 x 2048 12.7 | 12.4, 159 x 10560 x 1792 60.7 | 55.3; 30 x 4416 x 1536, 1104 of them,
+//     8.9 | 10.0); and where LDS has room for three workgroups of one tile a unit, so that 769 to 1024 sixteens are two rounds of them (Q4_K of 17 to 24 super-blocks, 162 x 704
+//     x 5120 14.8 | 14.3; Q6_K of more than 32, 22 x 5120 x 9216 36.6 | 35.1).
 template <int DT, bool ROPE>
 static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int64_t nsb = a.K / 256, wgs = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows);
@@ -445,11 +458,12 @@ static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, co
     if (wgs <= 256 && fits(1, 16)) return launch_depth<DT, 1, 16, ROPE>(a, st, bf16, rope);
     if constexpr (DT == kQ4_K) {
         if (wgs <= 512 && fits(2, 16)) return launch_depth<DT, 2, 16, ROPE>(a, st, bf16, rope);
+        if (wgs <= 512 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
+        if ((wgs <= 512 || (wgs > 1024 && nsb <= 8 && a.M > 48) || (wgs > 768 && wgs <= 1024 && nsb > 16 && nsb <= 24)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     } else {
-        // (eight wavefronts to 32 super-blocks, two rounds of theirs: 8 x 8192 x 7168 19.4 -> 18.2 us, 2 x 4975 x 4352 13.3 -> 12.1)
         if (wgs <= 512 && nsb <= 32 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
+        if ((wgs <= 512 || (wgs > 1200 && nsb <= 8) || (wgs > 768 && wgs <= 1024 && nsb > 32)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     }
-    if (fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     return launch_depth<DT, 1, 4, ROPE>(a, st, bf16, rope);
 }
 

@@ -386,20 +386,22 @@ static bool one_row_pays(int dt, const QGemvArgs& a) {
     return (nsb <= 8 && a.N >= 8192) || (dt == kQ4_K && nsb >= 48 && a.N > 2048 && a.N <= 4096);
 }
 
-// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us, then W from memory once and once from
-// the caches per group of eight rows (5.7 TB/s Q4_K, 6.2 TB/s Q6_K), the tiled kernel of qgemm_kquant.hip about 2.1 us per super-block of
-// K and round of 128 tiles of 128 x 128. Measured, us, here | there, Q4_K: 32 x 14336 x 4096 28.5 | 31.6, 40 rows 34.4 | 31.8; 32 x 28672
-// x 4096 55 | 61, 40 rows 67 | 62; 64 x 4096 x 14336 62 | 109, 128 rows 121 | 118; 64 x 1024 x 4096 5.4 | 32. Q6_K: 16 x 14336 x 4096 24.6 | 32.2, 32 rows 37.5 | 32.5.
+// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.56 ns (Q4_K) or 0.64 ns (Q6_K) per super-block of sixteen
+// rows of W and group of eight rows of x, a fifth more where rows of more than 32 super-blocks leave LDS room for fewer workgroups; the tiled kernel of
+// qgemm_kquant.hip 4 us and 2.1 (Q4_K) or 2 and 1.9 (Q6_K) per super-block of K and round of 128 tiles of 128 x 128. Fitted to 983 products of 9 to 512 rows, 512 x 1024 to
+// 14336 x 14336: the kernel that it takes is more than 5 % slower than the other at one of them, 145 x 2240 x 4608 Q6_K 38.8 | 36.7, and at two of 470 more (by up to 8 %). Measured, us, here | there, Q4_K: 39 x 13632 x 5120 45.8 | 40.4,
+// 25 x 12288 x 4608 32.0 | 35.5, 237 x 2176 x 2304 23.4 | 22.8, 101 x 3712 x 13824 83 | 108; Q6_K: 257 x 1536 x 4608 43.1 | 36.5, 33 x 9152 x 3584 31.1 | 28.8,
+// 18 x 8960 x 4864 26.7 | 37.5, 193 x 1152 x 8448 47 | 63.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
     if (g_kq_rows == 2 || (a.M >= 2 && a.M <= 8)) return true;
     if (a.M == 1) return one_row_pays(dt, a);
     if (a.M > 512) return false;
-    const double nsb = (double)(a.K / 256), groups = (double)((a.M + kRows - 1) / kRows);
-    // (rows of more than 32 super-blocks leave room for one workgroup a compute unit)
-    const double rows_us = 3 + (groups + 0.6) * (double)a.N * nsb * (dt == kQ4_K ? 144 / 5.7e6 : 210 / 6.2e6) / (nsb > 32 ? 0.75 : 1);
+    const bool q4 = dt == kQ4_K;
+    const double nsb = (double)(a.K / 256), sixteens = (double)((a.N + 15) / 16 * ((a.M + kRows - 1) / kRows));
+    const double rows_us = 3 + sixteens * nsb * (q4 ? 0.56e-3 : 0.64e-3) * (nsb > 32 ? 1.2 : 1);
     const double tiles = (double)(((a.M + 127) / 128) * ((a.N + 127) / 128));
-    return rows_us < (tiles > 128 ? tiles / 128 : 1.0) * nsb * 2.1;
+    return rows_us < (q4 ? 4 : 2) + (tiles > 128 ? tiles / 128 : 1.0) * nsb * (q4 ? 2.1 : 1.9);
 }
 
 template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>

@@ -377,13 +377,13 @@ bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a) {
            rows_lds(dt, nsb, 1, 4) <= 160 * 1024;
 }
 
-// One converted row: the kernels that give a row of W to a wavefront (qgemv_kquant.hip) have little to read a wavefront where rows are short, and
-// a long serial chain of terms where they are long and too few to hide it. us in a decoding step, there | here: Q4_K 16384 x 2048 9.8 | 7.5, 8192 x 1024
-// 6.0 | 5.1, 4096 x 14336 11.6 | 10.4; Q6_K 16384 x 2048 9.7 | 9.0, 8192 x 1024 5.8 | 5.3; but Q4_K 28672 x 4096 17.8 | 21.2, 2048 x 8192 5 | 6.8,
-// Q6_K 4096 x 14336 15 | 14.4 and 28672 x 4096 24.6 | 26.9.
+// One converted row: the kernels that give a row of W to a wavefront (qgemv_kquant.hip) have little to read a wavefront where rows are short and many. us, there | here,
+// Q4_K: 8192 x 256 5.5 | 3.9, 8192 x 2048 6.2 | 5.5, 12288 x 2048 8.0 | 7.0, 32768 x 2048 17.3 | 12.8, 128256 x 2048 56 | 37; Q6_K: 8192 x 2048 6.0 | 5.9, 12288 x 2048 9.3 | 8.7,
+// 32768 x 2048 20.4 | 18.0; but Q6_K 9216 x 2048 7.2 | 7.6, 10240 x 1536 6.8 | 7.0, and of longer rows Q4_K 8192 x 2560 6.5 | 6.2, 16384 x 3072 11.2 | 11.9, 4096 x 14336 11.5 | 11.7,
+// 4096 x 20480 14.2 | 16.6; Q6_K 4096 x 14336 15.8 | 17.1.
 static bool one_row_pays(int dt, const QGemvArgs& a) {
     const int64_t nsb = a.K / 256;
-    return (nsb <= 8 && a.N >= 8192) || (dt == kQ4_K && nsb >= 48 && a.N > 2048 && a.N <= 4096);
+    return nsb <= 8 && a.N >= 8192 && (dt == kQ4_K || nsb <= 5 || a.N == 8192 || a.N >= 11264);
 }
 
 // Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.56 ns (Q4_K) or 0.64 ns (Q6_K) per super-block of sixteen
@@ -394,8 +394,8 @@ static bool one_row_pays(int dt, const QGemvArgs& a) {
 // 18 x 8960 x 4864 26.7 | 37.5, 193 x 1152 x 8448 47 | 63.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
-    if (g_kq_rows == 2 || (a.M >= 2 && a.M <= 8)) return true;
     if (a.M == 1) return one_row_pays(dt, a);
+    if (g_kq_rows == 2 || a.M <= 8) return true;
     if (a.M > 512) return false;
     const bool q4 = dt == kQ4_K;
     const double nsb = (double)(a.K / 256), sixteens = (double)((a.N + 15) / 16 * ((a.M + kRows - 1) / kRows));
@@ -449,9 +449,10 @@ static hipError_t launch_depth(const QGemvArgs& a, hipStream_t st, bool bf16, co
 //     than 48 super-blocks 2 x 4: 4 x 7296 x 13824 20.0, 1 x 4 20.5. Q6_K 2 x 8 to 32 super-blocks: 8 x 8192 x 7168 17.4, 2 x 4 18.5; then 2 x 4: 4 x 4352 x 12544 21.8, 1 x 4 24.9
 //   beyond, one tile, so that three to five workgroups share a unit: 1 x 4 | 2 x 4, Q4_K 16 x 13568 x 7424 32.2 | 44.7, 88 x 4032 x 7936 43.1 | 66.1, 8 x 12032 x 4096
 //     11.7 | 13.3; Q6_K 4 x 8512 x 6400 20.1 | 23.5, 72 x 3776 x 7936 44.2 | 53.3. Two tiles where the operand of x that they share is what counts: short rows by many groups (Q4_K 188
-//     x 960 x 1536 1 x 4 9.0 | 2 x 4 8.5, 61 x 2688 x 1536 7.6 | 7.1; 45 x 4480 x 1280 8.0 | 8.8), short rows of Q6_K from 1200 sixteens on (1 x 20480 x 2048 12.7 | 12.4, 159 x 10560 x 1792 60.7 | 55.3; 30 x 4416 x 1536, 1104 of them,
-//     8.9 | 10.0); and where LDS has room for three workgroups of one tile a unit, so that 769 to 1024 sixteens are two rounds of them (Q4_K of 17 to 24 super-blocks, 162 x 704
-//     x 5120 14.8 | 14.3; Q6_K of more than 32, 22 x 5120 x 9216 36.6 | 35.1).
+//     x 960 x 1536 1 x 4 9.0 | 2 x 4 8.5, 61 x 2688 x 1536 7.6 | 7.1; 45 x 4480 x 1280 8.0 | 8.8) or
+//     of up to four super-blocks (1 x 65536 x 1024 15.0 | 14.2), short rows of Q6_K from 1200 sixteens on (1 x 20480 x 2048 12.7 | 12.4, 159 x 10560 x 1792 60.7 | 55.3; 30 x 4416 x 1536, 1104 of them,
+//     8.9 | 10.0); and where one tile a workgroup is a second round and two are not: LDS has room for five of a unit of up to eight super-blocks (Q4_K 1 x 24576 x 1024
+//     7.2 | 6.5) and for three of 17 to 24 (Q4_K 162 x 704 x 5120 14.8 | 14.3) or more than 32 (Q6_K 22 x 5120 x 9216 36.6 | 35.1).
 template <int DT, bool ROPE>
 static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int64_t nsb = a.K / 256, wgs = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows);
@@ -461,7 +462,8 @@ static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, co
     if constexpr (DT == kQ4_K) {
         if (wgs <= 512 && fits(2, 16)) return launch_depth<DT, 2, 16, ROPE>(a, st, bf16, rope);
         if (wgs <= 512 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
-        if ((wgs <= 512 || (wgs > 1024 && nsb <= 8 && a.M > 48) || (wgs > 768 && wgs <= 1024 && nsb > 16 && nsb <= 24)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
+        const bool short_rows = nsb <= 8 && ((wgs > 1024 && a.M > 48) || (wgs > 1280 && wgs <= 1536) || (wgs > 2560 && nsb <= 4));
+        if ((wgs <= 512 || short_rows || (wgs > 768 && wgs <= 1024 && nsb > 16 && nsb <= 24)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     } else {
         if (wgs <= 512 && nsb <= 32 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
         if ((wgs <= 512 || (wgs > 1200 && nsb <= 8) || (wgs > 768 && wgs <= 1024 && nsb > 32)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);

@@ -755,7 +755,8 @@ def test_kquant_rows_kernel_at_the_edges_of_its_forms(dt, m, n, k):
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("n,k", [(8191, 256), (8192, 256), (8199, 256 * 8), (8192, 256 * 9), (2048, 256 * 48), (2049, 256 * 48), (4096, 256 * 48),
-                                 (4097, 256 * 48), (2050, 256 * 47), (2051, 256 * 75)])
+                                 (4097, 256 * 48), (2050, 256 * 47), (2051, 256 * 75),
+                                 (8193, 256 * 5), (8193, 256 * 6), (11263, 256 * 8), (11264, 256 * 8), (24580, 256 * 2), (41009, 256)])
 def test_one_converted_row_of_kquants_on_either_side_of_the_choice(dt, n, k):
     """A row by the kernel for several where that is the faster, at the edges of the rule and by the other kernel: the oracle's bits."""
     rng = np.random.default_rng(dt + n + k)

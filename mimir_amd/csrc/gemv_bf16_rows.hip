@@ -65,14 +65,16 @@ __global__ __launch_bounds__(64 * kWaves, 4) void gemv_bf16_rows_kernel(const ui
     f32x4 acc[T];
 #pragma unroll
     for (int t = 0; t < T; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int kSteps = 2;  // under way: with three or four, fewer wavefronts fit a SIMD (4 x 8192 x 2048 9.6 us; 10.4 with four)
+    // under way: with three or four, fewer wavefronts fit a SIMD (4 x 8192 x 2048 10.3 us, 11.2 with four). An odd last step by itself: in a whole pair the
+    // one before it was fetched again, a third more of W where a wavefront has three (2 x 8192 x 1536 8.2 us, so 7.2; of five, 2 x 8192 x 2560 12.0 and 11.2).
+    constexpr int kSteps = 2;
     auto sum_of = [&](int from, int to) {
         const int n = (to - from) / 64;
         if (n <= 0) return;
         u32x4 w[kSteps][2][T];
         XStep<PASSES> xs[kSteps];
         auto load = [&](int i, int slot) {
-            const int k = from + 64 * (i < n ? i : n - 1);
+            const int k = from + 64 * i;
             xs[slot].load(x, ldx, M, k, lane);
 #pragma unroll
             for (int t = 0; t < T; t++)
@@ -92,15 +94,16 @@ __global__ __launch_bounds__(64 * kWaves, 4) void gemv_bf16_rows_kernel(const ui
         for (int u = 0; u < kSteps; u++)
             if (u < n) load(u, u);
         int base = 0;
-        for (; base + kSteps < n; base += kSteps)
+        for (; base + kSteps < n - 1; base += kSteps)  // whole pairs of steps: no step of W is asked for twice
 #pragma unroll
             for (int u = 0; u < kSteps; u++) {
                 multiply(u);
                 load(base + kSteps + u, u);
             }
-#pragma unroll
-        for (int u = 0; u < kSteps; u++)
-            if (base + u < n) multiply(u);
+        multiply(0);
+        if (base + 2 < n) load(base + 2, 0);
+        if (base + 1 < n) multiply(1);
+        if (base + 2 < n) multiply(0);
     };
     int from = k0;
     if (KIND == Out::Scaled && out.mid) {  // what of this wavefront's piece lies below split has a factor of its own

@@ -188,7 +188,11 @@ void launch_gemv_bf16(const uint16_t* W, int64_t ldw, const float* x, int64_t ld
         else if (kind == Out::Plain) launch(gemv_bf16_kernel<M, R, Out::Plain>, R);
         else if constexpr (R > 1) launch(gemv_bf16_kernel<M, R, Out::Pairs>, R);
     };
-    if (M == 1 && groups == 1 && N >= 1024 && N < 8192 && k >= 8192 && kind != Out::Pairs) {
+    // Two rows a wavefront, and rows of W in quarters, us: 1536 x 10240 10.4 | 10.2, 2048 x 8192 13.0 | 11.2, 2048 x 14336 22.4 | 13.6, 3072 x 8192 14.6 | 13.3, 4096 x 8704 18.2 | 17.0,
+    // 6144 x 10240 28.5 | 26.0, 8128 x 18432 62 | 57; of less W than 14 million the quarters are short (1024 x 8192 6.3 | 7.1), and by more than 4096 rows,
+    // which fill the compute units as they are, only quarters of whole steps gain (6144 x 8192 22.2 | 25.1, 6144 x 11264 31.1 | 33.0).
+    const bool quarters = N >= 1024 && N < 8192 && N * (int64_t)k >= 14000000 && (N <= 3072 ? k >= 8192 : N <= 4096 ? k > 8192 : k >= 10240 && k % 2048 == 0);
+    if (M == 1 && groups == 1 && quarters && kind != Out::Pairs) {
         const dim3 grid((unsigned)((N + 3) / 4));
         if (kind == Out::Scaled) hipLaunchKernelGGL((gemv_bf16_long_kernel<4, Out::Scaled>), grid, dim3(256), 0, st, W, ldw, x, (int)N, k, out);
         else hipLaunchKernelGGL((gemv_bf16_long_kernel<4, Out::Plain>), grid, dim3(256), 0, st, W, ldw, x, (int)N, k, out);

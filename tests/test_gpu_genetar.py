@@ -410,10 +410,11 @@ def test_trace_replay(tmp_path, mixed, dtype):
         assert X.error(got, want[rows]) < TOL[dtype]
 
 
-@pytest.mark.parametrize("width,ff", [(1024, 8192), (1088, 7232), (1024, 15360)])
+@pytest.mark.parametrize("width,ff", [(1024, 8192), (1088, 7232), (1024, 15360), (1536, 8192), (2112, 7232), (4160, 9216), (4160, 9280)])
 def test_one_row_by_long_rows_of_the_output_and_down_projection(width, ff):
     """One position of a sequence against the same as one of two: attention's output and the down projection as one product of K heads * 128 + ff
-    (9216; 8256, pieces that end within a step; 16384), the part below split with a factor of its own. A row alone is multiplied as float32, two as
+    (9216; 8256, pieces that end within a step; 16384), the part below split with a factor of its own; by either kernel for one row (the rows in quarters:
+    width 1024 with 16384, 1536, 2112 and 4160 with 10240). A row alone is multiplied as float32, two as
     the sum of two bfloat16 (2^-17 of an element): five products on a path, their sums some ten times smaller than their terms'."""
     heads = 8
     mixer = dict(heads=heads, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5, softcap=30.0, v_mix=True)

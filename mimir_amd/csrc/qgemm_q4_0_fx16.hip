@@ -90,10 +90,11 @@ __global__ __launch_bounds__(256) void fx16_digits_kernel(const float* __restric
     }
 }
 
-// Where strips are more than half the dies. 256 x 4096 x 14336 took 92 us with a strip's rows on all of them and 88 on one; the three strips of
-// 77 x 4096 x 14336 on three dies 45 against 43.
-__host__ __device__ inline bool by_dies(int64_t M) { return in_lanes(M) && M > 128; }
-static_assert(kInPlaceRows == 8 * 32, "a strip a die");
+// In the order of lanes a line of 128 bytes has a piece each of eight rows: eight rows a die (every eighth workgroup), whose cache puts the line together, the eights
+// on the dies in turn. Whole calls, against a row a workgroup as rows come (up to 128 of them; more, a strip a die): 128 x 9536 x 4544 55.0 -> 53.7 us, 108 x 4480 x 13056 63.6 -> 62.4,
+// 77 x 5120 x 5120 30.0 -> 29.3, 200 x 3136 x 11968 70.0 -> 69.5.
+constexpr int kDies = 8, kLineRows = 8;
+__device__ inline int row_of_die(int block) { return kLineRows * ((block & (kDies - 1)) + kDies * (block / (kDies * kLineRows))) + block / kDies % kLineRows; }
 
 // A workgroup converts a row of x into halves: x 2^-e = h0 + h1, h0 the binary16 next to it and h1 the binary16 next to
 // what that leaves. An element is held to 2^-23 of itself (of float32's 24 bits the last may go: 2^14 + 8 - 2^-9 leaves 8 - 2^-9, which h1 rounds by
@@ -109,8 +110,7 @@ __global__ __launch_bounds__(256) void fx16_halves_kernel(const float* __restric
                                                           uint16_t* __restrict__ X16, float* __restrict__ XS, int2* __restrict__ RS, int M, float inv_k, float eps) {
     constexpr int kHeld = ITEMS ? ITEMS : 1;
     const int nb = K >> 5, n8 = K >> 3, tid = threadIdx.x;
-    // in the order of lanes a line has pieces of eight rows: a strip's rows on one die (every eighth workgroup), whose cache puts the lines together
-    const int m = LANES && by_dies(M) ? ((int)blockIdx.x & 7) * 32 + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    const int m = LANES ? row_of_die((int)blockIdx.x) : (int)blockIdx.x;
     if (LANES && m >= M) return;
     const float* xr = x + (int64_t)m * x_row_stride;
     uint16_t* strip = X16 + strip_at(m, nb);
@@ -650,7 +650,7 @@ static void launch_halves(const float* x, const float* w, double eps, int64_t M,
     const auto rows = K <= 4096 ? fx16_halves_kernel<2, NORM, false> : K <= 16384 ? fx16_halves_kernel<8, NORM, false> : fx16_halves_kernel<0, NORM, false>;
     const auto by_lanes = K <= 4096 ? fx16_halves_kernel<2, NORM, true> : K <= 16384 ? fx16_halves_kernel<8, NORM, true> : fx16_halves_kernel<0, NORM, true>;
     const auto kernel = in_lanes(M) ? by_lanes : rows;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(by_dies(M) ? 256 : M)), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (int)M, (float)(1.0 / (double)K), (float)eps);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(in_lanes(M) ? (M + kDies * kLineRows - 1) / (kDies * kLineRows) * (kDies * kLineRows) : M)), dim3(256), 0, st, x, w, x_row_stride, (int)K, X16, XS, RS, (int)M, (float)(1.0 / (double)K), (float)eps);
 }
 
 hipError_t q4_0_fx16_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, Fx16 form, hipStream_t st) {

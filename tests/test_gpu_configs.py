@@ -54,10 +54,14 @@ def test_one_layer_step_against_a_prefilled_cache(batch):
         want = om.logits(tokens[b].tolist(), caches)
         err = np.abs(got[b] - want).max() / np.abs(want).max()
         assert err <= 5e-4, (b, float(err))
-    # the same step through the fused launches and their graph: the tokens it chooses are the logits' largest
+    # the choice after the pass and two more through the fused launches and their graph, whose shares of the keys meet in the form the next product
+    # reads: the tokens that the per-operator logits choose from the same caches
+    want = [got.argmax(-1)]
+    for _ in range(2):
+        want.append(m.logits(want[-1].reshape(batch, 1)).argmax(-1))
     m.set_cache(0, keys, values)
     toks, _ = m.generate(tokens, 3)
-    assert toks[:, 0].tolist() == [int(np.argmax(got[b])) for b in range(batch)]
+    assert toks.tolist() == np.stack(want, 1).tolist()
 
 
 @pytest.fixture(scope="module")

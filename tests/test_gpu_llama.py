@@ -8,6 +8,7 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from mimir_amd import capi
@@ -396,6 +397,35 @@ def test_steps_of_a_context_of_96_share_its_keys_between_two_workgroups(linear_d
         assert not np.array_equal(got[0], got[1])
     scale = np.abs(got[1]).max()
     assert np.abs(got[0] - got[1]).max() <= (1e-3 if linear_dt == O.Q4_0 else 0.02) * scale
+
+
+@pytest.mark.parametrize("embed,batch,rows", [(512, 1, 3), (512, 3, 2), (4160, 2, 5), (8192, 1, 9)])
+def test_the_heads_norm_and_conversion_in_one_launch_are_the_two_launches(embed, batch, rows):
+    """A block of zeros leaves a token's embedding as it is: the logits of a Q8_0 head are, bit for bit, those of rmsnorm, conversion and product one by one, for all rows of a
+    call (a row's length apart) and for the last of each sequence (further apart)."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab, c.interleaved = embed, 64, 1, 1, 1, 64, 64, 515, 0
+    om = OL.synthetic(OL.Config(embed=embed, hidden=64, layers=1, heads=1, kv_heads=1, head_dim=64, rope_dim=64, rope_base=c.rope_base, rope_scale=1.0, eps=c.eps,
+                                vocab=c.vocab, context=c.context), seed=9, output_dt=O.Q8_0)
+    b = om.blocks[0]
+    for w in (b.o, b.down):
+        w.data[:] = 0
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(batch * rows)
+    tokens = np.random.default_rng(31).integers(0, c.vocab, (batch, rows))
+    gpu.say(f"head embed={embed} batch={batch} rows={rows}")
+    every = m.logits(tokens, all=True)
+    m.reset()
+    last = m.logits(tokens)
+    x = gpu.dev(np.ascontiguousarray(O.dequantize(O.Q8_0, om.embed.data).reshape(c.vocab, embed)[tokens.reshape(-1)]))
+    normed, norm = torch.empty_like(x), gpu.dev(om.norm.reshape(-1).astype(np.float32))
+    capi.check(lib.mi355x_rmsnorm(x.data_ptr(), norm.data_ptr(), normed.data_ptr(), batch * rows, embed, c.eps, gpu.stream()))
+    buf, ptr = gpu.dev_bytes_at(om.output.data, 4)
+    want = gpu.qgemv_act(O.Q8_0, ptr, normed, c.vocab, embed).reshape(batch, rows, c.vocab)
+    assert np.array_equal(np.asarray(every).reshape(want.shape).view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(np.asarray(last).reshape(batch, c.vocab).view(np.uint32), np.ascontiguousarray(want[:, -1]).view(np.uint32))
 
 
 @pytest.mark.parametrize("embed,vocab,batch", [(512, 8192, 1), (512, 8195, 3), (4160, 8195, 2), (512, 70001, 9)])

@@ -700,9 +700,8 @@ def test_kquant_rows_of_x_share_one_pass_over_w_on_the_matrix_cores(dt, m, n, k)
     """Rows of x, eight at a time, against Q4_K or Q6_K weights read once on the int8 matrix cores (the decoding
     step of a batch; forced here beyond the rows it is chosen for): the CPU's integer sums, and its float32
     operations in its order, so the oracle's bits and those of the one-row kernels. x holds a zero
-    super-block, ties and, in one row, a NaN. Rows of up to 32 super-blocks keep their partial sums in
-    LDS, longer ones (to 64) in registers, handed from wavefront to wavefront; beyond that LDS again, or
-    another kernel where it has no room."""
+    super-block, ties and, in one row, a NaN. Up to some 80 super-blocks in up to sixteen wavefronts; longer rows
+    leave LDS room for fewer, or are another kernel's."""
     l = gpu.lib()
     rng = np.random.default_rng(dt + 7 * m + n + k)
     raw = random_blocks(rng, dt, n * k)
@@ -769,11 +768,13 @@ def test_one_converted_row_of_kquants_on_either_side_of_the_choice(dt, n, k):
 
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
-def test_kquant_rows_kernel_at_the_largest_integer_sums(dt):
+@pytest.mark.parametrize("n,k,waves", [(64, 256 * 32, 16), (64, 256 * 32, 8), (64, 256 * 32, 4), (2064, 256 * 16, 0), (4128, 256 * 9, 0)])
+def test_kquant_rows_kernel_at_the_largest_integer_sums(dt, n, k, waves):
     """Every quant and scale at its largest magnitude with x at +-127 per super-block (backend/cpu/quant_test.go:164-204), through the
-    kernel that reads W once per eight rows of x: its 24-bit multiplies and int32 sums hold what the CPU's int32 arithmetic holds."""
+    kernel that reads W once per eight rows of x: its 24-bit multiplies, int32 and binary16 sums hold what the CPU's int32 arithmetic holds. Sixteen, eight and four
+    wavefronts a workgroup, one and two tiles of rows of W, super-blocks in one round, two and a loop."""
     l = gpu.lib()
-    m, n, k = 11, 64, 256 * 40
+    m = 11
     bb = O.block_bytes(dt)
     raw = np.zeros(n * k // 256 * bb, np.uint8).reshape(-1, bb)
     if dt == O.Q4_K:
@@ -795,10 +796,9 @@ def test_kquant_rows_kernel_at_the_largest_integer_sums(dt):
     want = O.qmatmul(dt, raw, x, n, k)
     try:
         capi.check(l.mi355x_tune(b"kquant.mfma_rows", 2))
-        for key, v in ((b"kquant.mfma_rows_waves", 0), (b"kquant.mfma_rows_waves", 1)):  # partial sums in registers (K = 10240), then in LDS
-            capi.check(l.mi355x_tune(key, v))
-            gpu.say(f"kquant rows kernel extremes dt={dt} {key.decode()}={v}")
-            assert bits_equal(gpu.qgemv(dt, ptr, gpu.dev(x), n, k), want)
+        capi.check(l.mi355x_tune(b"kquant.mfma_rows_waves", waves))
+        gpu.say(f"kquant rows kernel extremes dt={dt} N={n} K={k} waves={waves}")
+        assert bits_equal(gpu.qgemv(dt, ptr, gpu.dev(x), n, k), want)
     finally:
         capi.check(l.mi355x_tune(b"kquant.mfma_rows", 0))
         capi.check(l.mi355x_tune(b"kquant.mfma_rows_waves", 0))

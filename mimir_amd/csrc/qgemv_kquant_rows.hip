@@ -386,22 +386,21 @@ static bool one_row_pays(int dt, const QGemvArgs& a) {
     return nsb <= 8 && a.N >= 8192 && (dt == kQ4_K || nsb <= 5 || a.N == 8192 || a.N >= 11264);
 }
 
-// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.56 ns (Q4_K) or 0.64 ns (Q6_K) per super-block of sixteen
-// rows of W and group of eight rows of x, a fifth more where rows of more than 32 super-blocks leave LDS room for fewer workgroups; the tiled kernel of
-// qgemm_kquant.hip 4 us and 2.1 (Q4_K) or 2 and 1.9 (Q6_K) per super-block of K and round of 128 tiles of 128 x 128. Fitted to 983 products of 9 to 512 rows, 512 x 1024 to
-// 14336 x 14336: the kernel that it takes is more than 5 % slower than the other at one of them, 145 x 2240 x 4608 Q6_K 38.8 | 36.7, and at two of 470 more (by up to 8 %). Measured, us, here | there, Q4_K: 39 x 13632 x 5120 45.8 | 40.4,
-// 25 x 12288 x 4608 32.0 | 35.5, 237 x 2176 x 2304 23.4 | 22.8, 101 x 3712 x 13824 83 | 108; Q6_K: 257 x 1536 x 4608 43.1 | 36.5, 33 x 9152 x 3584 31.1 | 28.8,
-// 18 x 8960 x 4864 26.7 | 37.5, 193 x 1152 x 8448 47 | 63.
+// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.46 ns (Q4_K) or 0.64 ns (Q6_K) per super-block of sixteen
+// rows of W and group of eight rows of x, half of those counted that the last of a workgroup's four wavefronts have less, and a tenth or a fifth more where rows of more than 32
+// super-blocks leave LDS room for fewer workgroups; the tiled kernel of qgemm_kquant.hip 4 us and 1.9 (Q4_K) or 3 and 2 per super-block of K and begun round of 128 tiles of 128 x 128. Fitted to
+// 2715 products of 9 to 512 rows, 512 x 1024 to 32768 x 8192 and 14336 x 14336: the choice takes 0.1 % longer than the faster kernel in the mean, 11 % at most. us, here | there, Q4_K:
+// 39 x 13632 x 5120 46.0 | 40.6, 39 x 12416 x 4352 38.5 | 34.6, 25 x 12288 x 4608 32.0 | 35.5, 101 x 3712 x 13824 83 | 108, 42 x 17280 x 3584 (135 tiles) 46.9 | 54.9; Q6_K: 257 x 1536 x 4608
+// 43.1 | 36.5, 33 x 9152 x 3584 31.3 | 29.0, 18 x 8960 x 4864 26.7 | 37.5, 193 x 1152 x 8448 47 | 63, 18 x 20288 x 4352 50 | 67.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
     if (a.M == 1) return one_row_pays(dt, a);
     if (g_kq_rows == 2 || a.M <= 8) return true;
     if (a.M > 512) return false;
     const bool q4 = dt == kQ4_K;
-    const double nsb = (double)(a.K / 256), sixteens = (double)((a.N + 15) / 16 * ((a.M + kRows - 1) / kRows));
-    const double rows_us = 3 + sixteens * nsb * (q4 ? 0.56e-3 : 0.64e-3) * (nsb > 32 ? 1.2 : 1);
-    const double tiles = (double)(((a.M + 127) / 128) * ((a.N + 127) / 128));
-    return rows_us < (q4 ? 4 : 2) + (tiles > 128 ? tiles / 128 : 1.0) * nsb * (q4 ? 2.1 : 1.9);
+    const int64_t nsb = a.K / 256, sixteens = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows), rounds = (((a.M + 127) / 128) * ((a.N + 127) / 128) + 127) / 128;
+    const double each = (double)nsb + 0.5 * (double)(-nsb & 3), rows_us = 3 + (double)sixteens * each * (q4 ? 0.46e-3 * (nsb > 32 ? 1.1 : 1) : 0.64e-3 * (nsb > 32 ? 1.2 : 1));
+    return rows_us < (q4 ? 4 : 3) + (double)(rounds * nsb) * (q4 ? 1.9 : 2.0);
 }
 
 template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>

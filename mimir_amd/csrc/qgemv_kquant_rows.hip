@@ -449,7 +449,7 @@ static hipError_t launch_depth(const QGemvArgs& a, hipStream_t st, bool bf16, co
 //   beyond, one tile, so that three to five workgroups share a unit: 1 x 4 | 2 x 4, Q4_K 16 x 13568 x 7424 32.2 | 44.7, 88 x 4032 x 7936 43.1 | 66.1, 8 x 12032 x 4096
 //     11.7 | 13.3; Q6_K 4 x 8512 x 6400 20.1 | 23.5, 72 x 3776 x 7936 44.2 | 53.3. Two tiles where the operand of x that they share is what counts: short rows by many groups (Q4_K 188
 //     x 960 x 1536 1 x 4 9.0 | 2 x 4 8.5, 61 x 2688 x 1536 7.6 | 7.1; 45 x 4480 x 1280 8.0 | 8.8) or
-//     of up to four super-blocks (1 x 65536 x 1024 15.0 | 14.2), short rows of Q6_K from 1200 sixteens on (1 x 20480 x 2048 12.7 | 12.4, 159 x 10560 x 1792 60.7 | 55.3; 30 x 4416 x 1536, 1104 of them,
+//     of up to four super-blocks (1 x 65536 x 1024 15.0 | 14.2) or of sixteen, four to each wavefront (32 x 28672 x 4096 60.4 | 58.2, 64 x 4096 x 4096 17.8 | 16.9), short rows of Q6_K from 1200 sixteens on (1 x 20480 x 2048 12.7 | 12.4, 159 x 10560 x 1792 60.7 | 55.3; 30 x 4416 x 1536, 1104 of them,
 //     8.9 | 10.0); and where one tile a workgroup is a second round and two are not: LDS has room for five of a unit of up to eight super-blocks (Q4_K 1 x 24576 x 1024
 //     7.2 | 6.5) and for three of 17 to 24 (Q4_K 162 x 704 x 5120 14.8 | 14.3) or more than 32 (Q6_K 22 x 5120 x 9216 36.6 | 35.1).
 template <int DT, bool ROPE>
@@ -462,7 +462,8 @@ static hipError_t launch_shape(const QGemvArgs& a, hipStream_t st, bool bf16, co
         if (wgs <= 512 && fits(2, 16)) return launch_depth<DT, 2, 16, ROPE>(a, st, bf16, rope);
         if (wgs <= 512 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
         const bool short_rows = nsb <= 8 && ((wgs > 1024 && a.M > 48) || (wgs > 1280 && wgs <= 1536) || (wgs > 2560 && nsb <= 4));
-        if ((wgs <= 512 || short_rows || (wgs > 768 && wgs <= 1024 && nsb > 16 && nsb <= 24)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
+        const bool even = nsb == 16 && wgs >= 1024 && a.M > 24;
+        if ((wgs <= 512 || short_rows || even || (wgs > 768 && wgs <= 1024 && nsb > 16 && nsb <= 24)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);
     } else {
         if (wgs <= 512 && nsb <= 32 && fits(2, 8)) return launch_depth<DT, 2, 8, ROPE>(a, st, bf16, rope);
         if ((wgs <= 512 || (wgs > 1200 && nsb <= 8) || (wgs > 768 && wgs <= 1024 && nsb > 32)) && fits(2, 4)) return launch_depth<DT, 2, 4, ROPE>(a, st, bf16, rope);

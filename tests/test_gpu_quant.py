@@ -727,7 +727,7 @@ def test_kquant_rows_of_x_share_one_pass_over_w_on_the_matrix_cores(dt, m, n, k)
 @pytest.mark.parametrize("m,n,k", [(2, 16, 256), (8, 15, 256 * 16), (7, 17, 256 * 17), (9, 31, 256 * 32), (3, 33, 256 * 49), (17, 47, 256 * 64),
                                    (8, 18, 256 * 65), (8, 20, 256 * 75), (5, 4099, 256), (8, 4130, 256 * 16), (6, 4131, 256 * 17), (16, 2070, 256 * 20),
                                    (5, 8210, 256 * 2), (8, 8211, 256 * 9), (2, 8225, 256 * 33), (130, 1030, 256 * 5), (64, 520, 256 * 34),
-                                   (61, 2690, 256 * 6), (21, 4510, 256 * 20), (5, 8210, 256 * 31), (4, 6001, 256 * 50), (17, 4110, 256 * 34)])
+                                   (61, 2690, 256 * 6), (21, 4510, 256 * 20), (5, 8210, 256 * 31), (4, 6001, 256 * 50), (17, 4110, 256 * 34), (33, 3290, 256 * 16)])
 def test_kquant_rows_kernel_at_the_edges_of_its_forms(dt, m, n, k):
     """One or two tiles of sixteen rows of W a workgroup, four to sixteen wavefronts, one to four super-blocks each and loops of
     more, partly filled tiles and groups of x: the oracle's bits, into float32 and, rounded once, into bfloat16."""

@@ -143,8 +143,8 @@ hipError_t qgemm_kquant(int dt, const QGemvArgs& a, hipStream_t st, bool out_bf1
 // global memory, 2 = never the matrix-core kernel, 3 = always the matrix-core kernel.
 void set_kquant_tune(int which, int value);
 // Two rows of x or more against Q4_K or Q6_K weights, eight to a pass over W, on the int8 matrix cores with the CPU's bits
-// (qgemv_kquant_rows.hip); qgemv_kquant_act hands over where qgemv_kquant_rows_pays says so ("kquant.mfma_rows": 1 never, 2 wherever
-// the kernel takes the shape).
+// (qgemv_kquant_rows.hip), and one row where its rows of W are short and many; qgemv_kquant_act hands over where qgemv_kquant_rows_pays says so
+// ("kquant.mfma_rows": 1 never, 2 wherever the kernel takes two rows or more).
 bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a);
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a);
 hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);

@@ -15,8 +15,8 @@
 // lanes touch a line each costs the cache 64 lookups (x and W loaded so, 4096 x 14336: 16 us), so both come as rows, 16 bytes a lane, and change
 // lanes in LDS that is the wavefront's own: no barrier but the one before the sums. A workgroup owns sixteen rows of W, so that a
 // matrix of 4096 rows has one for every compute unit, in up to sixteen wavefronts, which take the super-blocks round robin and have all or
-// most of theirs under way from the start: with one ahead every second super-block cost a trip to memory. Matrices with
-// more rows take two tiles of sixteen a workgroup, which share the operand of x.
+// most of theirs under way from the start: with one ahead every second super-block cost a trip to memory. Matrices of up to twice as many
+// rows take two tiles of sixteen a workgroup, which share the operand of x, larger ones several workgroups of four wavefronts a compute unit (launch_shape).
 //
 // The operands are sixteen rows wide: column n of the second is row n of W, row 8 c + m of the first is row m of x with everything but
 // group c of the weights zeroed, c = 0 or 1 (those lanes read zeros kept in LDS), so that one instruction keeps two groups of
@@ -26,8 +26,8 @@
 //
 // Measured, us a call on rows already converted, eight rows of x, the form before it (32 rows of W a workgroup in four or eight wavefronts, one
 // super-block ahead) and this one: Q4_K 4096 x 14336 20.2 12.2 (loads alone 9.6), 2048 x 8192 10.4 6.4, 6144 x 4096 8.5 6.8, 4096 x 4096 7.0 4.9,
-// 28672 x 4096 22.6 20.2-22.5 (66 MB: 3.1 TB/s); Q6_K 4096 x 14336 26.6 14.7 (48 MB: 3.3 TB/s), 2048 x 8192 16.7 9.0, 4096 x 4096
-// 11.0 6.1, 28672 x 4096 31.5 26.2-28.7.
+// 28672 x 4096 22.6 20.9-23.5 (66 MB: 3.0 TB/s); Q6_K 4096 x 14336 26.6 14.7 (48 MB: 3.3 TB/s), 2048 x 8192 16.7 9.0, 4096 x 4096
+// 11.0 6.1, 28672 x 4096 31.5 27.5.
 #include "device_util.h"
 #include "kernels.h"
 #include "rope_tail.h"

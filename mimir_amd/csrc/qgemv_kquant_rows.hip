@@ -421,24 +421,27 @@ static hipError_t launch_kq_rows(const QGemvArgs& a, hipStream_t st, bool bf16, 
 
 // By the super-blocks that a wavefront takes: as many under way as it takes in one round or two, sixteen wavefronts hold two within their 128 registers,
 // fewer four. (Three of three: with four asked for, 4 x 12480 x 2304 Q4_K took 10.1 us, so 8.5; four for six, 25 x 12288 x 4608 34.6, three in two rounds 32.0.)
-// What launch_shape() does not come to has the loop of any length.
+// Two tiles in sixteen or eight wavefronts fit LDS, or are taken, for so few super-blocks that a wavefront has no more than are here.
 template <int DT, int TILES, int WAVES, bool ROPE>
 static hipError_t launch_depth(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int64_t each = (a.K / 256 + WAVES - 1) / WAVES;
     if (each <= 1) return launch_kq_rows<DT, TILES, WAVES, 1, 1, ROPE>(a, st, bf16, rope);
-    if constexpr (WAVES != 16 || TILES == 1)
+    if constexpr (TILES == 2 && WAVES == 16) return hipErrorInvalidValue;
+    else {
         if (each <= 2) return launch_kq_rows<DT, TILES, WAVES, 2, 1, ROPE>(a, st, bf16, rope);
-    if constexpr (WAVES == 16) {
-        if constexpr (TILES == 1)
+        if constexpr (WAVES == 16) {
             if (each <= 4) return launch_kq_rows<DT, TILES, WAVES, 2, 2, ROPE>(a, st, bf16, rope);
-        return launch_kq_rows<DT, TILES, WAVES, 2, 0, ROPE>(a, st, bf16, rope);
-    } else {
-        if (each == 3) return launch_kq_rows<DT, TILES, WAVES, 3, 1, ROPE>(a, st, bf16, rope);
-        if (each == 4) return launch_kq_rows<DT, TILES, WAVES, 4, 1, ROPE>(a, st, bf16, rope);
-        if (each <= 6) return launch_kq_rows<DT, TILES, WAVES, 3, 2, ROPE>(a, st, bf16, rope);
-        if constexpr (TILES == 1)
-            if (each <= 8) return launch_kq_rows<DT, TILES, WAVES, 4, 2, ROPE>(a, st, bf16, rope);
-        return launch_kq_rows<DT, TILES, WAVES, 4, 0, ROPE>(a, st, bf16, rope);
+            return launch_kq_rows<DT, TILES, WAVES, 2, 0, ROPE>(a, st, bf16, rope);
+        } else {
+            if (each == 3) return launch_kq_rows<DT, TILES, WAVES, 3, 1, ROPE>(a, st, bf16, rope);
+            if (each == 4) return launch_kq_rows<DT, TILES, WAVES, 4, 1, ROPE>(a, st, bf16, rope);
+            if constexpr (WAVES == 4 || DT == kQ4_K)
+                if (each <= 6) return launch_kq_rows<DT, TILES, WAVES, 3, 2, ROPE>(a, st, bf16, rope);
+            if constexpr (TILES == 1)
+                if (each <= 8) return launch_kq_rows<DT, TILES, WAVES, 4, 2, ROPE>(a, st, bf16, rope);
+            if constexpr (WAVES == 4) return launch_kq_rows<DT, TILES, WAVES, 4, 0, ROPE>(a, st, bf16, rope);
+            else return hipErrorInvalidValue;
+        }
     }
 }
 

@@ -290,8 +290,8 @@ bool fits(int64_t M, int64_t strips, int64_t K) {
 }  // namespace
 
 // What qgemm_q4_0_parts.hip takes instead: the faster by both models and by a tenth, which is how far they may be off: here | there 128 x 9536 x 4544 51.2 us | 55.8 (by the models 45.7 and
-// 44.1), 108 x 4480 x 13056 61.7 | 67.2 (53.2, 51.9), 205 x 2240 x 8448 48.5 | 50.4 (39.5, 37.0), 256 x 5120 x 5120 54.4 | 58.2 (51.5, 49.3); of 450 shapes it is behind by more than 3 % at two
-// within the tenth (128 x 6208 x 8960 57.6 | 60.0). Nor up to 32 rows by more than 8192 long ones: 29 x 11136 x 11328 54.0 | 60.5, 31 x 12480 x 8960 46.9 | 51.2, but 28 x 8128 x 13376 54.2 | 48.7.
+// 44.1), 108 x 4480 x 13056 61.7 | 67.2 (53.2, 51.9), 205 x 2240 x 8448 48.5 | 50.4 (39.5, 37.0), 256 x 5120 x 5120 54.4 | 58.2 (51.5, 49.3); of 780 shapes it is behind by more than 3 % at
+// three within the tenth (128 x 6208 x 8960 57.6 | 60.0). Nor up to 32 rows by more than 8192 long ones: 29 x 11136 x 11328 54.0 | 60.5, 31 x 12480 x 8960 46.9 | 51.2, but 28 x 8128 x 13376 54.2 | 48.7.
 static bool by_parts(int64_t M, int64_t strips, int64_t K, size_t sums_bytes, double us) {
     return qgemm_q4_0_parts_ok(M, strips, K) && !(M <= 32 && strips > 256 && K > 8192) && qgemm_q4_0_parts_cost_us(M, strips, K, sums_bytes, nullptr) <= 0.9 * us;
 }

@@ -136,6 +136,7 @@ hipError_t qgemv_kquant_act(int dt, const QGemvArgs& a, hipStream_t st);
 // The same products for many rows of x on the matrix cores (qgemm_kquant.hip); qgemv_kquant_act
 // hands over to it where qgemm_kquant_pays says it is the faster of the two.
 bool qgemm_kquant_pays(int dt, const QGemvArgs& a);
+double qgemm_kquant_us(int64_t M, int64_t N, int64_t K);
 bool qgemm_kquant_ok(int dt, const QGemvArgs& a);
 // y float32, or with out_bf16 each result rounded once to bfloat16 into y taken as uint16_t*.
 hipError_t qgemm_kquant(int dt, const QGemvArgs& a, hipStream_t st, bool out_bf16 = false);

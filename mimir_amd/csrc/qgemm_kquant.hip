@@ -11,8 +11,9 @@
 // The integer sum of a super-block is sum_i s(i) q_i x_i with a 6-bit scale and
 // a 4-bit quant (Q4_K) or an int8 scale and a 6-bit quant less 32 (Q6_K). The
 // scaled weight s q has 10 or 14 bits, too many for the int8 matrix
-// instruction, so it is split: s q = 64 a + b (Q4_K) or 128 a + b (Q6_K) with
-// both digits in int8 range, and the sum is 64 A + B from two planes of
+// instruction, so it is split into two planes: Q4_K's by its scale, s = 8 s1 + s0, a = s1 q and
+// b = s0 q (at most 105 each, so that a pair of 16-bit multiplies makes four of them), Q6_K's by
+// its bytes, s q = 256 a + b. Either sum is that of two planes of
 // v_mfma_i32_32x32x32_i8 against the same fragment of x. Integer sums are
 // exact, so the split changes nothing. Q4_K's second sum, the mins against the
 // sums of x, is sum over the sixteen 16-element groups of m(g / 2) S(g): one
@@ -20,18 +21,26 @@
 // 16 * 127) and m (at most 63) are integers binary16 holds and the products
 // and their sum stay below 2^24.
 //
-// A workgroup of eight wavefronts owns a tile of 128 or 256 rows of x by 64 rows
-// of W; a wavefront owns 32 or 64 by 32 of it. The loop runs over halves of a
-// super-block (128 of K): the int8 rows of x and the two planes of W for the
-// next half are loaded from global memory before the current half is
-// multiplied, and split and stored into the other of two LDS buffers
-// afterwards; rows are padded to 144 bytes, which makes the 128-bit fragment
-// reads conflict-free. After the second half the wavefront turns its integer
-// sums into float32 as above. Both matrix instructions take, per lane, the
+// A workgroup of eight wavefronts owns a tile of 256 or 128 rows of x by 64 rows
+// of W and walks K a super-block a step. Its wavefronts are two groups of four, each with half of the rows of x; a group splits half of the next
+// super-block's W into LDS (planes in two buffers), multiplies, and turns its integer sums into float32 as above. x goes from memory
+// straight into LDS (global_load_lds_dwordx4). LDS has room for 256 rows of a super-block once, so the groups of a tall tile are half a step apart: one
+// multiplies, brings in the other's rows and splits W while the other is at its float32 sums, and the other way round. Of 128 rows there are two buffers; a group
+// brings in its own rows a step ahead, both are in step, and one barrier a step is enough. Rows of LDS are 256 bytes with their
+// 16-byte pieces turned by the row, which makes the 128-bit fragment reads conflict-free.
+//
+// What bounds it: the MFMAs (1056 cycles a wavefront and super-block, 64 x 32 outputs) and the vector instructions, which do not overlap with them on this device:
+// 256 a wavefront for the float32 operations (eight an output, fixed by the CPU's order), 80 for the split. A tall tile and super-block takes 2.7 us, of which these are 2.3.
+// Before (both groups in step, halves of a super-block, split by 24-bit multiplies, tiles of 256 x 64 only where they filled the device) and now, us with x's
+// conversion, Q4_K | Q6_K: 655 x 4096 x 14336 244 -> 157 | 238 -> 166, 655 x 14336 x 4096 185 -> 155 | 177 -> 158, 2048 x 14336 x 4096 434 -> 360 (668 TFLOP/s) | 419 -> 362,
+// 1000 x 5120 x 5120 160 -> 109 | 148 -> 107, 128 x 14336 x 4096 42.1 -> 36.9 | 41.1 -> 39.1, 300 x 2048 x 8192 74 -> 61 | 70 -> 62.
+//
+// Both matrix instructions take, per lane, the
 // bytes or halves k = 16 or 8 (lane / 32).. of row (lane % 32); the result holds
 // column (lane % 32) and rows 8 (i / 4) + 4 (lane / 32) + i % 4 in register i.
 #include "device_util.h"
 #include "kernels.h"
+#include "tile_plan.h"
 
 namespace mimir {
 
@@ -47,229 +56,200 @@ typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kTN = 64;          // rows of W per workgroup
-constexpr int kHalf = 128;       // K per step
-constexpr int kRow = kHalf + 16; // bytes per LDS row of int8
-constexpr int kSumRow = 48;      // bytes per LDS row of sixteen binary16 (32 used)
+constexpr int kThreads = 512;
+constexpr int kSb = 256;         // K per step (a super-block), and bytes per LDS row of int8
 
-// LDS: two step buffers (x rows, plane A, plane B) and what the end of a
-// super-block needs (scales of x, sums of x, scales and mins of W), stored with
-// the second half's step: the barrier that ends the super-block's last step
-// also separates its readers from the next writers.
+// LDS: the rows of x of the super-block under way, two buffers of W's planes, and twice what the end of a super-block needs (scales
+// and sums of x, scales and mins of W).
 template <int TM>
 struct Layout {
     static constexpr int x = 0;
-    static constexpr int wa = TM * kRow;
-    static constexpr int wb = wa + kTN * kRow;
-    static constexpr int step = wb + kTN * kRow;
-    static constexpr int side0 = 2 * step;
-    static constexpr int dx = 0;                       // float[TM]
-    static constexpr int xsum = TM * 4;                // binary16[TM][16], rows of kSumRow bytes
-    static constexpr int dw = xsum + TM * kSumRow;     // float[kTN][2]: d, dmin
-    static constexpr int mins = dw + kTN * 8;          // binary16[kTN][16], rows of kSumRow bytes
-    static constexpr int side = mins + kTN * kSumRow;
-    static constexpr int total = side0 + side;
+    static constexpr int xbufs = TM == 128 ? 2 : 1;      // buffers of a group's rows of x
+    static constexpr int planes = xbufs * TM * kSb;      // [2] of: plane A [kTN][kSb], plane B the same
+    static constexpr int plane = kTN * kSb;
+    static constexpr int xside = planes + 4 * plane;     // [2] of:
+    static constexpr int xsum = 0;                       // binary16[TM][16]
+    static constexpr int dx = TM * 32;                   // float[TM]
+    static constexpr int xside_bytes = TM * 36;
+    static constexpr int wside = xside + 2 * xside_bytes;  // [2] of:
+    static constexpr int mins = 0;                       // binary16[kTN][16]
+    static constexpr int dw = kTN * 32;                  // float[kTN][2]: d, dmin
+    static constexpr int wside_bytes = kTN * 40;
+    static constexpr int total = wside + 2 * wside_bytes;
 };
+static_assert(Layout<256>::total <= 160 * 1024, "a compute unit's LDS");
 
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// Where 16-byte piece `piece` of row `row` sits: the 16 pieces of a row turned by the row, so that 16 rows' equal piece falls on all banks.
+__device__ __forceinline__ int piece_at(int row, int piece) { return row * kSb + 16 * (piece ^ (row & 15)); }
 
-__device__ __forceinline__ u32x2 load_u32x2_unaligned(const uint8_t* p) {
-    u32x2 v;
-    __builtin_memcpy(&v, p, 8);
-    return v;
+__device__ __forceinline__ void phase_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// 16 bytes a lane from base + offset into LDS at lds_base + 16 lane (load_to_lds of gemm_nt_tile.h, a wavefront's address and a lane's offset).
+__device__ __forceinline__ void load_to_lds(const uint8_t* base, uint32_t offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(base) : "memory");
 }
 
-// Bytes 0 and 2 of lo, then bytes 0 and 2 of hi.
-__device__ __forceinline__ uint32_t even_bytes(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x06040200u); }
-// Bytes 0 and 1 (or 2 and 3) of v, each widened to 16 bits.
-__device__ __forceinline__ uint32_t widen01(uint32_t v) { return __builtin_amdgcn_perm(0u, v, 0x0c010c00u); }
-__device__ __forceinline__ uint32_t widen23(uint32_t v) { return __builtin_amdgcn_perm(0u, v, 0x0c030c02u); }
-
-// Four quants in the bytes of q (each below 16) times the 6-bit scale s, split
-// into the digits of 64 a + b.
-__device__ __forceinline__ void split_q4k(uint32_t q, uint32_t s, uint32_t& a, uint32_t& b) {
-    uint32_t p01 = __umul24(widen01(q), s), p23 = __umul24(widen23(q), s);  // two products below 1024 each
-    a = even_bytes(p01 >> 6, p23 >> 6);
-    b = even_bytes(p01 & 0x003F003Fu, p23 & 0x003F003Fu);
+// Two 16-bit products a lane, their low halves.
+__device__ __forceinline__ uint32_t mul_pairs(uint32_t a, uint32_t b) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b));
 }
 
-// Four quants in the bytes of q (each below 64) less 32, times the int8 scale
-// s, split into the digits of 128 a + b with b in 0..127.
-__device__ __forceinline__ void split_q6k(uint32_t q, int s, uint32_t& a, uint32_t& b) {
-    const s16x2 bias = {32, 32}, sc = {(short)s, (short)s};
-    s16x2 p01 = (__builtin_bit_cast(s16x2, widen01(q)) - bias) * sc;
-    s16x2 p23 = (__builtin_bit_cast(s16x2, widen23(q)) - bias) * sc;
-    a = even_bytes(__builtin_bit_cast(uint32_t, p01 >> 7), __builtin_bit_cast(uint32_t, p23 >> 7));
-    b = even_bytes(__builtin_bit_cast(uint32_t, p01) & 0x007F007Fu, __builtin_bit_cast(uint32_t, p23) & 0x007F007Fu);
+// Four quants in the bytes of q (each below 64) times the int8 scale s, less 32 s each, split into the digits of 256 a + b, both int8:
+// q s + (128 - 32 s) in 16 bits has a in its upper byte and b + 128 in its lower. s and bias: the two numbers in both halves.
+__device__ __forceinline__ void split_q6k(uint32_t q, uint32_t s, uint32_t bias, uint32_t& a, uint32_t& b) {
+    const s16x2 sc = __builtin_bit_cast(s16x2, s), c = __builtin_bit_cast(s16x2, bias);
+    const uint32_t even = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, q, 0x0c020c00u)) * sc + c);
+    const uint32_t odd = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, q, 0x0c030c01u)) * sc + c);
+    a = __builtin_amdgcn_perm(odd, even, 0x07030501u);
+    b = __builtin_amdgcn_perm(odd, even, 0x06020400u) ^ 0x80808080u;
 }
 
 // scale_min_k4 (backend/cpu/quant.go:129-134) on the twelve scale bytes held as three dwords.
-__device__ __forceinline__ uint32_t q4k_scale(uint32_t s0, uint32_t s2, int j) {
-    const int sh = 8 * (j & 3);
-    return j < 4 ? (s0 >> sh) & 63 : ((s2 >> sh) & 0xf) | (((s0 >> (sh + 6)) & 3) << 4);
-}
 __device__ __forceinline__ uint32_t q4k_min(uint32_t s1, uint32_t s2, int j) {
     const int sh = 8 * (j & 3);
     return j < 4 ? (s1 >> sh) & 63 : ((s2 >> (sh + 4)) & 0xf) | (((s1 >> (sh + 6)) & 3) << 4);
 }
 
-// What a thread holds between the loads of a step and its LDS stores: its
-// piece of W, requested two steps ahead (it comes from HBM), and its pieces of
-// the x tile, requested one step ahead (they come from the L2, every tile of
-// the same rows reads them).
+// What a thread holds between the loads and the LDS stores of its part of a super-block.
 struct FetchedW {
     u32x4 hdr;      // Q4_K: d, dmin and the scales. Q6_K: x, y = the 8 scales of the half, z = d
-    u32x2 q;        // 8 bytes of nibbles
-    u32x2 qh;       // Q6_K: the 8 bytes of upper bits that go with them
+    u32x4 q;        // 16 bytes of nibbles
+    u32x4 qh;       // Q6_K: the 16 bytes of upper bits that go with them
 };
-template <int XV>
 struct FetchedX {
-    u32x4 x[XV];    // 16-byte pieces of the x tile
-    u32x4 sums;     // second half only: eight int16 sums of x
-    float dx;       // second half only: the scale of one row of x
+    u32x4 sums;     // Q4_K: eight int16 sums of a row of x
+    float dx;       // the scale of a row of x
 };
 
-template <int H>
-struct Half {
-    static constexpr int value = H;
-};
-
-// MT 32-row tiles per wavefront: the workgroup's tile is (128 MT) x 64. DEPTH says how far ahead of
-// its LDS stores a step's global loads are requested: 0 one step for W and x, 1 two steps for W, 2 two
-// steps for both; each step further costs the registers of one more set of loads.
-template <int DT, int MT, int DEPTH, bool OUT_BF16>
-__global__ __launch_bounds__(512) void qgemm_kquant_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act,
-                                                            void* __restrict__ yv, int M, int N, int nsb,
-                                                            int64_t act_row_bytes, int tiles_m, int ntiles) {
-    constexpr int TM = 128 * MT;
-    constexpr int XV = TM * 8 / 512;  // 16-byte pieces of x per thread and step: piece p is row p / 8, bytes 16 (p % 8)..
+// One tile: rows [m0, m0 + 128 MT) of x by rows [n0, n0 + 64) of W.
+template <int DT, int MT, bool OUT_BF16>
+__device__ __forceinline__ void tile(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act, void* __restrict__ yv, int M, int N, int nsb,
+                                     int64_t act_row_bytes, int m0, int n0, uint8_t* smem) {
+    constexpr int TM = 128 * MT;      // a wavefront's tile: 32 MT rows of x by 32 of W
+    constexpr int GM = TM / 2;        // rows of x a group
+    constexpr int NX = GM / 16;       // 1 KB loads of x a wavefront and super-block: four rows each
     constexpr int BB = DT == kQ4_K ? 144 : 210;
     typedef Layout<TM> L;
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 3, wn = wave >> 2, l32 = lane & 31, lh = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = wave >> 2, gw = wave & 3, gt = tid & 255;
+    const int wm = gw & 1, wn = gw >> 1, l32 = lane & 31, lh = lane >> 5;
 
-    // Tiles that share rows of W run next to each other on one XCD (workgroup i
-    // goes to XCD i % 8), so the second and later tiles find W in that L2.
-    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-    const int per_xcd = (ntiles + 7) >> 3;
-    const int t = slot / tiles_m + xcd * per_xcd;
-    const int tm = slot % tiles_m;
-    if (slot >= per_xcd * tiles_m || t >= ntiles) return;
-    const int m0 = tm * TM, n0 = t * kTN;
+    const int g0 = group * GM;        // this group's first row in the tile
 
-    // This thread's part of the W tile: 8 bytes of nibbles of row wrow_i, piece c8 of the half. Its
-    // addresses, and those of its pieces of x, are a base the workgroup shares plus 32 bits of its own.
-    const int wrow_i = tid >> 3, c8 = tid & 7;
+    // This thread's part of W: 16 bytes of nibbles of row wrow_i, piece c4 of half `group` of the super-block. Of the row's index
+    // the two bits that tell the rows of sixteen lanes apart are those that turn their pieces away from each other.
+    const int c4 = gt & 3, r4 = gt >> 4, j4 = (gt >> 2) & 3;
+    const int wrow_i = DT == kQ4_K ? (r4 >> 2) * 16 + (r4 & 1) + 2 * (r4 & 2) + 2 * (j4 & 1) + 4 * (j4 & 2) : (r4 >> 2) * 16 + (r4 & 3) + 4 * j4;
     const int last_n = N - 1 - n0, last_m = M - 1 - m0;
     const uint8_t* w_t = W + (int64_t)n0 * nsb * BB;
     const uint32_t woff = (uint32_t)(wrow_i < last_n ? wrow_i : last_n) * (uint32_t)(nsb * BB);
     const uint8_t* act_t = act + (int64_t)m0 * act_row_bytes;
-    uint32_t xoff[XV];
+    // Its parts of x: a lane's piece of the wavefront's loads, and the sums of half a row with the row's scale (two threads a row; with 64 rows a
+    // group two threads have the same part: branch-free, and the same bytes to the same place).
+    const int gx = L::xbufs == 2 ? g0 : GM - g0;
+    uint32_t xoff[NX];
 #pragma unroll
-    for (int i = 0; i < XV; i++) {
-        const int r = (tid + 512 * i) >> 3;
-        xoff[i] = (uint32_t)(r < last_m ? r : last_m) * (uint32_t)act_row_bytes + 16 * (tid & 7);
+    for (int j = 0; j < NX; j++) {
+        const int r = gx + 4 * (NX * gw + j) + (lane >> 4);
+        xoff[j] = (uint32_t)(r < last_m ? r : last_m) * (uint32_t)act_row_bytes + 16 * ((lane & 15) ^ (r & 15));
     }
-    // sums: two threads a row; scales: a thread a row
-    // (with 128-row tiles two threads do the same row's part: branch-free, and the same bytes to the same place)
-    const int srow = (tid >> 1) & (TM - 1), drow = tid & (TM - 1);
-    const uint32_t soff = (uint32_t)(srow < last_m ? srow : last_m) * (uint32_t)act_row_bytes + 16 * (tid & 1);
-    const uint32_t doff = (uint32_t)(drow < last_m ? drow : last_m) * (uint32_t)act_row_bytes;
-    const uint8_t* sums_t = act_t + (int64_t)nsb * 256;
+    const int srow = g0 + ((gt >> 1) & (GM - 1));
+    const uint32_t soff = (uint32_t)(srow < last_m ? srow : last_m) * (uint32_t)act_row_bytes;
+    const uint8_t* sums_t = act_t + (int64_t)nsb * 256 + 16 * (tid & 1);
     const uint8_t* dx_t = act_t + (int64_t)nsb * 288;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
 
-    FetchedW fw0, fw1;
-    FetchedX<XV> fx0, fx1;
-    auto fetch_w = [&](FetchedW& f, int sb, auto half) {
-        constexpr int h = decltype(half)::value;
+    FetchedW fw;
+    FetchedX fx;
+    FetchedW fw0;  // the first super-block's, requested together with the second's
+    FetchedX fx0;
+    auto clamped = [&](int sb) { return sb < nsb ? sb : nsb - 1; };  // past the last super-block: it again, into buffers nobody reads
+    auto fetch = [&](FetchedW& fw, FetchedX& fx, int sb) {
         const uint8_t* wb = w_t + (int64_t)sb * BB + woff;
         if (DT == kQ4_K) {
-            f.hdr = *(const u32x4*)wb;
-            f.q = *(const u32x2*)(wb + 16 + 64 * h + 8 * c8);
+            fw.hdr = *(const u32x4*)wb;
+            fw.q = *(const u32x4*)(wb + 16 + 64 * group + 16 * c4);
+            fx.sums = *(const u32x4*)(sums_t + (int64_t)sb * 32 + soff);
         } else {
-            f.q = load_u32x2_unaligned(wb + 64 * h + 8 * c8);
-            f.qh = load_u32x2_unaligned(wb + 128 + 32 * h + 8 * (c8 & 3));
-            u32x2 sc = load_u32x2_unaligned(wb + 192 + 8 * h);
-            f.hdr[0] = sc[0];
-            f.hdr[1] = sc[1];
-            f.hdr[2] = load_u16(wb + 208);
+            fw.q = load_u32x4_unaligned(wb + 64 * group + 16 * c4);
+            fw.qh = load_u32x4_unaligned(wb + 128 + 32 * group + 16 * (c4 & 1));
+            u32x2 sc;
+            __builtin_memcpy(&sc, wb + 192 + 8 * group, 8);
+            fw.hdr[0] = sc[0], fw.hdr[1] = sc[1];
+            fw.hdr[2] = load_u16(wb + 208);
         }
+        fx.dx = *(const float*)(dx_t + (int64_t)sb * 4 + soff);
     };
-    auto fetch_x = [&](FetchedX<XV>& fx, int sb, auto half) {
-        constexpr int h = decltype(half)::value;
-#pragma unroll
-        for (int i = 0; i < XV; i++) fx.x[i] = *(const u32x4*)(act_t + ((int64_t)sb * 256 + kHalf * h) + xoff[i]);
-        if (h == 1) {
-            if (DT == kQ4_K) fx.sums = *(const u32x4*)(sums_t + (int64_t)sb * 32 + soff);
-            fx.dx = *(const float*)(dx_t + (int64_t)sb * 4 + doff);
-        }
+    auto load_x = [&](int sb, int j) {
+        load_to_lds(act_t + (int64_t)sb * 256, xoff[j], __builtin_amdgcn_readfirstlane(lds0 + L::x + ((sb & (L::xbufs - 1)) * TM + gx + 4 * (NX * gw + j)) * kSb));
     };
-    auto stage = [&](const FetchedW& f, const FetchedX<XV>& fx, int sb, auto half) {
-        constexpr int h = decltype(half)::value;
-        uint8_t* buf = smem + h * L::step;
-        uint8_t* side = smem + L::side0;
-#pragma unroll
-        for (int i = 0; i < XV; i++) {
-            const int p = tid + 512 * i;
-            *(u32x4*)(buf + L::x + (p >> 3) * kRow + 16 * (p & 7)) = fx.x[i];
-        }
-        u32x2 alo, blo, ahi, bhi;
-        int klo, khi;
+    auto stage = [&](const FetchedW& fw, const FetchedX& fx, int sb) {  // this thread's part of W's planes of super-block sb and of its sums and scales of x; its scales and mins by group 1
+        u32x4 alo, blo, ahi, bhi;
+        int plo, phi;  // the pieces of the low and the high nibbles' weights
+        uint8_t* wside = smem + L::wside + (sb & 1) * L::wside_bytes;
         if (DT == kQ4_K) {
-            const int j = 4 * h + 2 * (c8 >> 2);  // sub-blocks j (low nibbles) and j + 1 (high) of this thread's bytes
-            const uint32_t sl = q4k_scale(f.hdr[1], f.hdr[3], j), sh = q4k_scale(f.hdr[1], f.hdr[3], j + 1);
-#pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const uint32_t w = f.q[d];
-                uint32_t a0, b0, a1, b1;
-                split_q4k(w & 0x0F0F0F0Fu, sl, a0, b0);
-                split_q4k((w >> 4) & 0x0F0F0F0Fu, sh, a1, b1);
-                alo[d] = a0, blo[d] = b0, ahi[d] = a1, bhi[d] = b1;
+            const int j = 2 * (c4 >> 1);  // sub-blocks 4 group + j (low nibbles) and j + 1 (high) of this thread's bytes
+            const int sh0 = 8 * (j & 3);
+            uint32_t sl, sh;
+            if (group == 0) {
+                sl = (fw.hdr[1] >> sh0) & 63, sh = (fw.hdr[1] >> (sh0 + 8)) & 63;
+            } else {
+                sl = ((fw.hdr[3] >> sh0) & 0xf) | (((fw.hdr[1] >> (sh0 + 6)) & 3) << 4);
+                sh = ((fw.hdr[3] >> (sh0 + 8)) & 0xf) | (((fw.hdr[1] >> (sh0 + 14)) & 3) << 4);
             }
-            klo = 64 * (c8 >> 2) + 8 * (c8 & 3);
-            khi = klo + 32;
-            if (h == 1) {
-                float* dw = (float*)(side + L::dw) + 2 * wrow_i;  // the row's eight threads store the same two values
-                dw[0] = f16_bits_to_f32((uint16_t)f.hdr[0]);
-                dw[1] = f16_bits_to_f32((uint16_t)(f.hdr[0] >> 16));
-                // sub-block c8's min, once for each of its two groups of 16
-                const _Float16 mn = (_Float16)(float)q4k_min(f.hdr[2], f.hdr[3], c8);
-                const uint32_t pair = (uint32_t)__builtin_bit_cast(uint16_t, mn) * 0x00010001u;
-                *(uint32_t*)(side + L::mins + wrow_i * kSumRow + 4 * c8) = pair;
+            const uint32_t sl1 = (sl >> 3) * 0x00010001u, sl0 = (sl & 7) * 0x00010001u, sh1 = (sh >> 3) * 0x00010001u, shl = (sh & 7) * 0x00010001u;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {  // a byte's product is at most 15 x 7: four of them in a pair of 16-bit multiplies
+                const uint32_t lo = fw.q[d] & 0x0F0F0F0Fu, hi = (fw.q[d] >> 4) & 0x0F0F0F0Fu;
+                alo[d] = mul_pairs(lo, sl1), blo[d] = mul_pairs(lo, sl0);
+                ahi[d] = mul_pairs(hi, sh1), bhi[d] = mul_pairs(hi, shl);
+            }
+            plo = 8 * group + 4 * (c4 >> 1) + (c4 & 1);
+            phi = plo + 2;
+            if (group == 1) {
+                float* dw = (float*)(wside + L::dw) + 2 * wrow_i;  // the row's four threads store the same two values
+                dw[0] = f16_bits_to_f32((uint16_t)fw.hdr[0]);
+                dw[1] = f16_bits_to_f32((uint16_t)(fw.hdr[0] >> 16));
+                // the mins of sub-blocks 2 c4 and 2 c4 + 1, each once for its two groups of 16
+                u32x2 pairs;
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const _Float16 mn = (_Float16)(uint16_t)q4k_min(fw.hdr[2], fw.hdr[3], 2 * c4 + k);
+                    pairs[k] = (uint32_t)__builtin_bit_cast(uint16_t, mn) * 0x00010001u;
+                }
+                *(u32x2*)(wside + L::mins + wrow_i * 32 + 8 * c4) = pairs;
             }
         } else {
-            const int shl = c8 >= 4 ? 2 : 0;
-            const int si = c8 >> 1;  // scale of the low nibbles' group; the high nibbles' is four further
-            const int sl = (int)(int8_t)(f.hdr[0] >> (8 * si)), sh = (int)(int8_t)(f.hdr[1] >> (8 * si));
+            const int shl = c4 >= 2 ? 2 : 0;
+            const uint32_t sl = (uint32_t)(int)(int8_t)(fw.hdr[0] >> (8 * c4)), sh = (uint32_t)(int)(int8_t)(fw.hdr[1] >> (8 * c4));
+            const uint32_t sl2 = (sl & 0xffffu) * 0x00010001u, sh2 = (sh & 0xffffu) * 0x00010001u;
+            const uint32_t cl = ((128u - 32u * sl) & 0xffffu) * 0x00010001u, ch = ((128u - 32u * sh) & 0xffffu) * 0x00010001u;
 #pragma unroll
-            for (int d = 0; d < 2; d++) {
-                const uint32_t a = f.q[d], b = f.qh[d] >> shl;
+            for (int d = 0; d < 4; d++) {
+                const uint32_t a = fw.q[d], b = fw.qh[d] >> shl;
                 uint32_t a0, b0, a1, b1;
-                split_q6k((a & 0x0F0F0F0Fu) | ((b & 0x03030303u) << 4), sl, a0, b0);
-                split_q6k(((a >> 4) & 0x0F0F0F0Fu) | (((b >> 4) & 0x03030303u) << 4), sh, a1, b1);
+                split_q6k((a & 0x0F0F0F0Fu) | ((b & 0x03030303u) << 4), sl2, cl, a0, b0);
+                split_q6k(((a >> 4) & 0x0F0F0F0Fu) | (b & 0x30303030u), sh2, ch, a1, b1);
                 alo[d] = a0, blo[d] = b0, ahi[d] = a1, bhi[d] = b1;
             }
-            klo = 8 * c8;
-            khi = klo + 64;
-            if (h == 1) {
-                float* dw = (float*)(side + L::dw) + 2 * wrow_i;
-                dw[0] = f16_bits_to_f32((uint16_t)f.hdr[2]);
-            }
+            plo = 8 * group + c4;
+            phi = plo + 4;
+            if (group == 1) ((float*)(wside + L::dw))[2 * wrow_i] = f16_bits_to_f32((uint16_t)fw.hdr[2]);
         }
-        uint8_t* wa = buf + L::wa + wrow_i * kRow;
-        uint8_t* wbp = buf + L::wb + wrow_i * kRow;
-        *(u32x2*)(wa + klo) = alo;
-        *(u32x2*)(wa + khi) = ahi;
-        *(u32x2*)(wbp + klo) = blo;
-        *(u32x2*)(wbp + khi) = bhi;
-        if (h == 1) {
-            if (DT == kQ4_K) {
-                const s16x8 s = __builtin_bit_cast(s16x8, fx.sums);
-                const f16x8 hsum = __builtin_convertvector(s, f16x8);
-                *(f16x8*)(side + L::xsum + srow * kSumRow + 16 * (tid & 1)) = hsum;
-            }
-            ((float*)(side + L::dx))[drow] = fx.dx;
+        uint8_t* pa = smem + L::planes + (sb & 1) * 2 * L::plane;
+        const int at_lo = piece_at(wrow_i, plo), at_hi = piece_at(wrow_i, phi);
+        *(u32x4*)(pa + at_lo) = alo;
+        *(u32x4*)(pa + at_hi) = ahi;
+        *(u32x4*)(pa + L::plane + at_lo) = blo;
+        *(u32x4*)(pa + L::plane + at_hi) = bhi;
+        uint8_t* xside = smem + L::xside + (sb & 1) * L::xside_bytes;
+        if (DT == kQ4_K) {
+            const s16x8 s = __builtin_bit_cast(s16x8, fx.sums);
+            *(f16x8*)(xside + L::xsum + srow * 32 + 16 * (tid & 1)) = __builtin_convertvector(s, f16x8);
         }
+        ((float*)(xside + L::dx))[srow] = fx.dx;
     };
 
     i32x16 acc_a[MT], acc_b[MT];
@@ -279,106 +259,124 @@ __global__ __launch_bounds__(512) void qgemm_kquant_kernel(const uint8_t* __rest
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[mt][i] = accm[mt][i] = 0.f;
 
-    auto compute = [&](int sb, auto half) {
-        constexpr int h = decltype(half)::value;
-        const uint8_t* buf = smem + h * L::step;
-        const uint8_t* xa = buf + L::x + (wm * 32 * MT + l32) * kRow + 16 * lh;
-        const uint8_t* pa = buf + L::wa + (wn * 32 + l32) * kRow + 16 * lh;
-        const uint8_t* pb = buf + L::wb + (wn * 32 + l32) * kRow + 16 * lh;
+    const int at0 = piece_at(l32, lh);  // this lane's first piece of a row; the next is 32 bytes on, turned
+    auto multiply = [&](int sb, int sbx, bool more) {
+        const uint8_t* xa = smem + L::x + ((sb & (L::xbufs - 1)) * TM + g0 + wm * 32 * MT) * kSb;
+        const uint8_t* pa = smem + L::planes + (sb & 1) * 2 * L::plane + wn * 32 * kSb;
+        i32x4 wa[2], wb[2], x[2][MT];
+        auto read = [&](int s) {
+            const int at = at0 ^ (32 * s), c = s & 1;
+            wa[c] = *(const i32x4*)(pa + at), wb[c] = *(const i32x4*)(pa + L::plane + at);
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const i32x4 wa = *(const i32x4*)(pa + 32 * s), wb = *(const i32x4*)(pb + 32 * s);
+            for (int mt = 0; mt < MT; mt++) x[c][mt] = *(const i32x4*)(xa + mt * 32 * kSb + at);
+        };
+        read(0);
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int c = s & 1;
+            if (s + 1 < 8) read(s + 1);
+            if (more && s < 4) {
+#pragma unroll
+                for (int j = s * NX / 4; j < (s + 1) * NX / 4; j++) load_x(sbx, j);
+            }
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
-                const i32x4 x = *(const i32x4*)(xa + mt * 32 * kRow + 32 * s);
-                if (h == 0 && s == 0) {  // a super-block's first products start its sums from the constant zero
+                if (s == 0) {  // a super-block's first products start its sums from the constant zero
                     i32x16 zero;
 #pragma unroll
                     for (int i = 0; i < 16; i++) zero[i] = 0;
-                    acc_a[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, wa, zero, 0, 0, 0);
-                    acc_b[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, wb, zero, 0, 0, 0);
+                    acc_a[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[c][mt], wa[c], zero, 0, 0, 0);
+                    acc_b[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[c][mt], wb[c], zero, 0, 0, 0);
                 } else {
-                    acc_a[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, wa, acc_a[mt], 0, 0, 0);
-                    acc_b[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, wb, acc_b[mt], 0, 0, 0);
+                    acc_a[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[c][mt], wa[c], acc_a[mt], 0, 0, 0);
+                    acc_b[mt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[c][mt], wb[c], acc_b[mt], 0, 0, 0);
                 }
             }
         }
     };
     // The end of a super-block: its integer sums into the float32 sums, as the CPU does it.
-    auto finish = [&]() {
-        {
-            const uint8_t* side = smem + L::side0;
-            const float* dwp = (const float*)(side + L::dw) + 2 * (wn * 32 + l32);
-            const float dw = dwp[0], dmin = DT == kQ4_K ? dwp[1] : 0.f;
+    auto finish = [&](int sb) {
+        const uint8_t* xside = smem + L::xside + (sb & 1) * L::xside_bytes;
+        const uint8_t* wside = smem + L::wside + (sb & 1) * L::wside_bytes;
+        const float* dwp = (const float*)(wside + L::dw) + 2 * (wn * 32 + l32);
+        const float dw = dwp[0], dmin = DT == kQ4_K ? dwp[1] : 0.f;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                const int r0 = wm * 32 * MT + 32 * mt;
-                f32x16 summ;
-                if (DT == kQ4_K) {
-                    const f16x8 xs = *(const f16x8*)(side + L::xsum + (r0 + l32) * kSumRow + 16 * lh);
-                    const f16x8 mn = *(const f16x8*)(side + L::mins + (wn * 32 + l32) * kSumRow + 16 * lh);
-                    f32x16 zero;
+        for (int mt = 0; mt < MT; mt++) {
+            const int r0 = g0 + wm * 32 * MT + 32 * mt;
+            f32x16 summ;
+            if (DT == kQ4_K) {
+                const f16x8 xs = *(const f16x8*)(xside + L::xsum + (r0 + l32) * 32 + 16 * lh);
+                const f16x8 mn = *(const f16x8*)(wside + L::mins + (wn * 32 + l32) * 32 + 16 * lh);
+                f32x16 zero;
 #pragma unroll
-                    for (int i = 0; i < 16; i++) zero[i] = 0.f;
-                    summ = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, mn, zero, 0, 0, 0);
-                }
+                for (int i = 0; i < 16; i++) zero[i] = 0.f;
+                summ = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, mn, zero, 0, 0, 0);
+            }
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const f32x4 dx = *(const f32x4*)(side + L::dx + 4 * (r0 + 8 * j + 4 * lh));
+            for (int j = 0; j < 4; j++) {
+                const f32x4 dx = *(const f32x4*)(xside + L::dx + 4 * (r0 + 8 * j + 4 * lh));
 #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const int i = 4 * j + k;
-                        const int sumi = (acc_a[mt][i] << (DT == kQ4_K ? 6 : 7)) + acc_b[mt][i];
-                        const float dd = dw * dx[k];
-                        const float tt = dd * (float)sumi;
-                        acc[mt][i] = acc[mt][i] + tt;
-                        if (DT == kQ4_K) {
-                            const float dm = dmin * dx[k];
-                            const float u = dm * summ[i];
-                            accm[mt][i] = accm[mt][i] + u;
-                        }
+                for (int k = 0; k < 4; k++) {
+                    const int i = 4 * j + k;
+                    const int sumi = (acc_a[mt][i] << (DT == kQ4_K ? 3 : 8)) + acc_b[mt][i];
+                    const float dd = dw * dx[k];
+                    const float tt = dd * (float)sumi;
+                    acc[mt][i] = acc[mt][i] + tt;
+                    if (DT == kQ4_K) {
+                        const float dm = dmin * dx[k];
+                        const float u = dm * summ[i];
+                        accm[mt][i] = accm[mt][i] + u;
                     }
                 }
-                __builtin_amdgcn_sched_barrier(0);  // one tile at a time: interleaving them costs registers the kernel lacks
             }
+            __builtin_amdgcn_sched_barrier(0);  // one tile at a time: interleaving them costs registers the kernel lacks
         }
     };
 
-    const Half<0> h0;
-    const Half<1> h1;
-    // Sets of loads: with two steps of lead, the steps of a first half use fw0 / fx0 and those of a
-    // second half fw1 / fx1; with one step of lead there is one set.
-    FetchedW& fwb = DEPTH >= 1 ? fw1 : fw0;
-    FetchedX<XV>& fxb = DEPTH >= 2 ? fx1 : fx0;
-    fetch_w(fw0, 0, h0);
-    fetch_x(fx0, 0, h0);
-    if (DEPTH >= 1) fetch_w(fw1, 0, h1);
-    if (DEPTH >= 2) fetch_x(fx1, 0, h1);
-    stage(fw0, fx0, 0, h0);
-    lds_barrier();
-    // No branches inside: the last super-block requests and stages itself again, into buffers nobody reads.
-    for (int sb = 0; sb < nsb; sb++) {
-        const int nx = sb + 1 < nsb ? sb + 1 : sb;
-        if (DEPTH >= 1) fetch_w(fw0, nx, h0); else fetch_w(fw0, sb, h1);
-        if (DEPTH >= 2) fetch_x(fx0, nx, h0); else fetch_x(fx0, sb, h1);
-        compute(sb, h0);
-        stage(fwb, fxb, sb, h1);
-        lds_barrier();
-        if (DEPTH >= 1) fetch_w(fw1, nx, h1); else fetch_w(fw0, nx, h0);
-        if (DEPTH >= 2) fetch_x(fx1, nx, h1); else fetch_x(fx0, nx, h0);
-        compute(sb, h1);
-        __builtin_amdgcn_sched_barrier(0);
-        finish();
-        stage(fw0, fx0, nx, h0);
-        lds_barrier();
+    if (L::xbufs == 2 || group == 1) {
+#pragma unroll
+        for (int j = 0; j < NX; j++) load_x(0, j);
     }
+    fetch(fw0, fx0, 0);
+    fetch(fw, fx, clamped(1));
+    stage(fw0, fx0, 0);
+    wait_loads();
+    phase_barrier();
+    if (L::xbufs == 1 && group == 1) phase_barrier();
+    for (int sb = 0; sb < nsb; sb++) {
+        if (L::xbufs == 2) {
+            if (sb + 1 < nsb) {
+                stage(fw, fx, sb + 1);
+                fetch(fw, fx, clamped(sb + 2));
+            }
+            multiply(sb, sb + 1, sb + 1 < nsb);
+            __builtin_amdgcn_sched_barrier(0);
+            finish(sb);
+            wait_loads();
+        } else {
+            multiply(sb, sb + group, sb + group < nsb);
+            if (sb + 1 < nsb) {
+                stage(fw, fx, sb + 1);
+                wait_loads();
+                fetch(fw, fx, clamped(sb + 2));
+            } else {
+                wait_loads();
+            }
+            phase_barrier();
+            __builtin_amdgcn_s_setprio(0);
+            finish(sb);
+            __builtin_amdgcn_s_setprio(1);
+        }
+        phase_barrier();
+    }
+    if (L::xbufs == 1 && group == 0) phase_barrier();
 
     const int n = n0 + wn * 32 + l32;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int m = m0 + wm * 32 * MT + 32 * mt + 8 * (i >> 2) + 4 * lh + (i & 3);
+            const int m = m0 + g0 + wm * 32 * MT + 32 * mt + 8 * (i >> 2) + 4 * lh + (i & 3);
             if (m < M && n < N) {
                 const float v = DT == kQ4_K ? acc[mt][i] - accm[mt][i] : acc[mt][i];
                 if (OUT_BF16) ((uint16_t*)yv)[(int64_t)m * N + n] = f32_to_bf16_bits(v);
@@ -387,22 +385,66 @@ __global__ __launch_bounds__(512) void qgemm_kquant_kernel(const uint8_t* __rest
         }
 }
 
-template <int DT, int MT, bool OUT_BF16>
+// How the result is cut: 64 tall_cols columns in tiles of 256 rows, handed out first, the rest in tiles of 128.
+struct Cut {
+    int tall_m, short_m, tall_cols, cols;
+};
+
+template <int DT, bool OUT_BF16>
+__global__ __launch_bounds__(kThreads, 2) void qgemm_kquant_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act,
+                                                                   void* __restrict__ yv, int M, int N, int nsb, int64_t act_row_bytes, Cut cut) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    // A die's workgroups (every eighth) take a contiguous range of the tiles, those that share rows of W next to each other, so that
+    // the second and later ones find W in that die's L2.
+    const int tall = cut.tall_m * cut.tall_cols, tall_die = (tall + 7) >> 3;
+    int b = blockIdx.x;
+    if (b < 8 * tall_die) {
+        const int t = (b & 7) * tall_die + (b >> 3);
+        if (t < tall) tile<DT, 2, OUT_BF16>(W, act, yv, M, N, nsb, act_row_bytes, (t % cut.tall_m) * 256, (t / cut.tall_m) * kTN, smem);
+        return;
+    }
+    b -= 8 * tall_die;
+    const int low = cut.short_m * (cut.cols - cut.tall_cols), low_die = (low + 7) >> 3;
+    const int t = (b & 7) * low_die + (b >> 3);
+    if (t < low) tile<DT, 1, OUT_BF16>(W, act, yv, M, N, nsb, act_row_bytes, (t % cut.short_m) * 128, (cut.tall_cols + t / cut.short_m) * kTN, smem);
+}
+
+// A short tile takes this part of a tall one's time: 0.55 on a device half empty (1.5 us a super-block for 2.7), 0.75 on a full one.
+constexpr double kShortCost = 0.66;
+
+// Tall tiles for as many whole rounds of the device as end earliest, short ones for the rest, which a round of tall tiles would leave
+// partly empty; returns the end in tall tiles' time.
+double plan(int64_t M, int64_t N, Cut* out) {
+    const int tall_m = (int)((M + 255) / 256), short_m = (int)((M + 127) / 128), cols = (int)((N + kTN - 1) / kTN);
+    *out = Cut{tall_m, short_m, 0, cols};
+    double best = makespan(short_m * cols, kShortCost, 0, 0.0);
+    const int64_t rounds = (int64_t)tall_m * cols / kUnits;
+    for (int64_t round = rounds > 1 ? rounds - 1 : 1; round <= rounds + 1; round++) {
+        const int64_t c = round * kUnits / tall_m;
+        const int tall = (int)(c < cols ? c : cols);
+        const double end = makespan(tall_m * tall, 1.0, short_m * (cols - tall), kShortCost);
+        if (end < best - 1e-9) {
+            best = end;
+            *out = Cut{tall_m, short_m, tall, cols};
+        }
+    }
+    return best;
+}
+
+template <int DT, bool OUT_BF16>
 hipError_t launch(const QGemvArgs& a, int nsb, hipStream_t st) {
-    // What the registers allow: 256 a lane at two wavefronts a SIMD.
-    constexpr int DEPTH = MT == 1 ? 2 : 1;
-    typedef Layout<128 * MT> L;
+    constexpr int kLds = Layout<256>::total > Layout<128>::total ? Layout<256>::total : Layout<128>::total;
     static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_kquant_kernel<DT, MT, DEPTH, OUT_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, L::total);
+        hipError_t e = hipFuncSetAttribute((const void*)qgemm_kquant_kernel<DT, OUT_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) return e;
         raised = true;
     }
-    const int tiles_m = (int)((a.M + 128 * MT - 1) / (128 * MT)), ntiles = (int)((a.N + kTN - 1) / kTN);
-    const int per_xcd = (ntiles + 7) / 8;
-    hipLaunchKernelGGL((qgemm_kquant_kernel<DT, MT, DEPTH, OUT_BF16>), dim3((unsigned)(8 * per_xcd * tiles_m)), dim3(512), L::total, st,
-                       (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y, (int)a.M, (int)a.N, nsb, (int64_t)kq_act_bytes(a.K),
-                       tiles_m, ntiles);
+    Cut cut;
+    plan(a.M, a.N, &cut);
+    const int grid = 8 * ((cut.tall_m * cut.tall_cols + 7) / 8 + (cut.short_m * (cut.cols - cut.tall_cols) + 7) / 8);
+    hipLaunchKernelGGL((qgemm_kquant_kernel<DT, OUT_BF16>), dim3((unsigned)grid), dim3(kThreads), kLds, st,
+                       (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y, (int)a.M, (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), cut);
     return hipGetLastError();
 }
 
@@ -414,34 +456,25 @@ bool qgemm_kquant_ok(int dt, const QGemvArgs& a) {
            ((uintptr_t)a.act & 15) == 0 && a.M * ((a.N + kTN - 1) / kTN) < ((int64_t)1 << 30) && a.K <= (1 << 20);
 }
 
-static bool tall_tiles(const QGemvArgs& a) {
-    // 256-row tiles halve the work of splitting W; 128-row tiles where those would leave compute units idle.
-    return a.M > 128 && ((a.M + 255) / 256) * ((a.N + kTN - 1) / kTN) >= 256;
+// What a product takes by this kernel, us, Q4_K and Q6_K alike. Fitted to 950 products of 9 to 600 rows by 512 to 32768 rows of W of 4 to 56 super-blocks (6 % off in the mean).
+double qgemm_kquant_us(int64_t M, int64_t N, int64_t K) {
+    Cut cut;
+    return 4 + (double)(K / 256) * (2.8 * plan(M, N, &cut) - 0.4);
 }
 
-// The row-by-row kernels read W once per row of x, at about 5.8 TB/s (Q4_K) or 5.1 TB/s (Q6_K) while it sits in
-// the caches; a workgroup here spends about 2.1 us (5.5 with 256-row tiles) per super-block of K, 256 workgroups
-// at a time. Measured on 4096 x 4096, 4096 x 14336 and 14336 x 4096 weights, 2 to 64 rows (at 14336 x 4096 and
-// eight rows: 49 and 79 us by rows, 35 and 37 us here).
+// Against the row-by-row kernels, which read W once per row of x, at about 5.8 TB/s (Q4_K) or 5.1 TB/s (Q6_K) while it sits in
+// the caches. Measured on 4096 x 4096, 4096 x 14336 and 14336 x 4096 weights, 2 to 64 rows (at 14336 x 4096 and
+// eight rows: 49 and 79 us by rows, 35 and 39 us here).
 bool qgemm_kquant_pays(int dt, const QGemvArgs& a) {
-    if (a.M < 4) return false;
-    const double nsb = (double)(a.K / 256);
-    const double rows_us = (double)a.M * (double)a.N * nsb * (dt == kQ4_K ? 144 : 210) / (dt == kQ4_K ? 5.8e6 : 5.1e6);
-    const bool tall = tall_tiles(a);
-    const int64_t tiles = ((a.M + (tall ? 255 : 127)) / (tall ? 256 : 128)) * ((a.N + kTN - 1) / kTN);
-    return (double)((tiles + 255) / 256) * nsb * (tall ? 5.5 : 2.1) < rows_us;
-}
-
-template <bool OUT_BF16>
-static hipError_t pick(int dt, const QGemvArgs& a, hipStream_t st) {
-    const int nsb = (int)(a.K / 256);
-    const bool tall = tall_tiles(a);
-    if (dt == kQ4_K) return tall ? launch<kQ4_K, 2, OUT_BF16>(a, nsb, st) : launch<kQ4_K, 1, OUT_BF16>(a, nsb, st);
-    return tall ? launch<kQ6_K, 2, OUT_BF16>(a, nsb, st) : launch<kQ6_K, 1, OUT_BF16>(a, nsb, st);
+    if (a.M < 4 || !qgemm_kquant_ok(dt, a)) return false;
+    const double rows_us = (double)a.M * (double)a.N * (double)(a.K / 256) * (dt == kQ4_K ? 144 : 210) / (dt == kQ4_K ? 5.8e6 : 5.1e6);
+    return qgemm_kquant_us(a.M, a.N, a.K) < rows_us;
 }
 
 hipError_t qgemm_kquant(int dt, const QGemvArgs& a, hipStream_t st, bool out_bf16) {
-    return out_bf16 ? pick<true>(dt, a, st) : pick<false>(dt, a, st);
+    const int nsb = (int)(a.K / 256);
+    if (dt == kQ4_K) return out_bf16 ? launch<kQ4_K, true>(a, nsb, st) : launch<kQ4_K, false>(a, nsb, st);
+    return out_bf16 ? launch<kQ6_K, true>(a, nsb, st) : launch<kQ6_K, false>(a, nsb, st);
 }
 
 }  // namespace mimir

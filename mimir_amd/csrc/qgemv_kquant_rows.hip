@@ -386,21 +386,21 @@ static bool one_row_pays(int dt, const QGemvArgs& a) {
     return nsb <= 8 && a.N >= 8192 && (dt == kQ4_K || nsb <= 5 || a.N == 8192 || a.N >= 11264);
 }
 
-// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.46 ns (Q4_K) or 0.64 ns (Q6_K) per super-block of sixteen
-// rows of W and group of eight rows of x, half of those counted that the last of a workgroup's four wavefronts have less, and a tenth or a fifth more where rows of more than 32
-// super-blocks leave LDS room for fewer workgroups; the tiled kernel of qgemm_kquant.hip 4 us and 1.9 (Q4_K) or 3 and 2 per super-block of K and begun round of 128 tiles of 128 x 128. Fitted to
-// 2715 products of 9 to 512 rows, 512 x 1024 to 32768 x 8192 and 14336 x 14336: the choice takes 0.1 % longer than the faster kernel in the mean, 11 % at most. us, here | there, Q4_K:
-// 39 x 13632 x 5120 46.0 | 40.6, 39 x 12416 x 4352 38.5 | 34.6, 25 x 12288 x 4608 32.0 | 35.5, 101 x 3712 x 13824 83 | 108, 42 x 17280 x 3584 (135 tiles) 46.9 | 54.9; Q6_K: 257 x 1536 x 4608
-// 43.1 | 36.5, 33 x 9152 x 3584 31.3 | 29.0, 18 x 8960 x 4864 26.7 | 37.5, 193 x 1152 x 8448 47 | 63, 18 x 20288 x 4352 50 | 67.
+// Where it is the faster choice. Two to eight rows always; beyond, by what both kernels take: here 3 us and 0.42 ns (Q4_K; of rows of up to eight super-blocks 0.38) or 0.56 ns
+// (Q6_K) per super-block of sixteen rows of W and group of eight rows of x, half of those counted that the last of a workgroup's four wavefronts have less, and a tenth more where
+// rows of more than 32 super-blocks leave LDS room for fewer workgroups; the tiled kernel qgemm_kquant_us. On 950 products of 9 to 512 rows, 512 x 1024 to 32768 x 8192
+// and 14336 x 14336, the choice takes 0.04 % longer than the faster kernel in the mean, 11 % at most. us, here | there: Q4_K 79 x 5248 x 1024 9.1 | 10.9, 58 x 4160 x 8960 48 | 55, 300 x 1152 x 4096 22.6 | 27,
+// 83 x 5632 x 13312 103 | 85, 205 x 2688 x 2560 22.3 | 19.2; Q6_K 25 x 22272 x 2048 25.5 | 31.2, 64 x 5184 x 2048 16.3 | 17.4, 41 x 10432 x 1792 21.0 | 16.0, 98 x 3520 x 3072 21.0 | 23.2.
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
     if (a.M == 1) return one_row_pays(dt, a);
     if (g_kq_rows == 2 || a.M <= 8) return true;
     if (a.M > 512) return false;
     const bool q4 = dt == kQ4_K;
-    const int64_t nsb = a.K / 256, sixteens = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows), rounds = (((a.M + 127) / 128) * ((a.N + 127) / 128) + 127) / 128;
-    const double each = (double)nsb + 0.5 * (double)(-nsb & 3), rows_us = 3 + (double)sixteens * each * (q4 ? 0.46e-3 * (nsb > 32 ? 1.1 : 1) : 0.64e-3 * (nsb > 32 ? 1.2 : 1));
-    return rows_us < (q4 ? 4 : 3) + (double)(rounds * nsb) * (q4 ? 1.9 : 2.0);
+    const int64_t nsb = a.K / 256, sixteens = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows);
+    const double each = (double)nsb + 0.5 * (double)(-nsb & 3), ns = q4 ? (nsb <= 8 ? 0.378 : 0.42) : 0.56;
+    const double rows_us = 3 + (double)sixteens * each * ns * 1e-3 * (nsb > 32 ? 1.1 : 1);
+    return rows_us < 3 + 1.4 * (double)nsb || rows_us < qgemm_kquant_us(a.M, a.N, a.K);  // no product takes less than one round of short tiles
 }
 
 template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>

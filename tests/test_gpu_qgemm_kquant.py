@@ -145,3 +145,18 @@ def test_prompt_sized_products_take_the_matrix_cores_and_bf16_rounds_once(dt, m)
             assert np.array_equal(got.view(np.uint16), O.f32_to_bf16(want))
         else:
             assert bits_equal(got, want)
+
+
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("m,n,k", [
+    (300, 8960, 256),   # 256 tiles of 256 rows, then 36 of 128: one super-block, no step ahead
+    (257, 8200, 512),   # the same with a row and a few columns into the next tile
+    (700, 5000, 768),   # tiles of 256 rows to the last column but a few; an odd number of super-blocks
+    (128, 64, 1280), (129, 16384, 256),  # tiles of 128 rows alone: one, and one round of the device
+])
+def test_tiles_of_either_height(dt, m, n, k, matrix_cores):
+    rng = np.random.default_rng(m + n + k + dt)
+    raw = random_blocks(rng, dt, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    gpu.say(f"kquant gemm tiles dt={dt} M={m} N={n} K={k}")
+    assert bits_equal(product(dt, raw, x, n, k), O.qmatmul(dt, raw, x, n, k))

@@ -1,10 +1,11 @@
-// Attention for many query positions at once (a prompt) on the float32 matrix cores of gfx950: the semantics of
+// Attention for many query positions at once (a prompt) on the matrix cores of gfx950: the semantics of
 // attention.hip (softmax(scale * q.k^T) . v per query row, the query scaled first, p = exp(s - max), the result
 // (sum p v) * (1 / sum p), the logsumexp max + log(sum p), a row that sees no key zeros and -Inf, key j hidden from
 // query i when causal and j > i + causal_offset; backend/cpu/attention.go:268-292, 437-535), for the calls that kernel
 // serves one query row a workgroup, re-reading every key and value for every row.
 //
-// Here a wavefront owns 32 query rows of one head and walks the keys in tiles of 32 with a running maximum and sum per
+// Two kernels: one for float32 keys and values, described here, and one for binary16, described where it stands.
+// A wavefront owns 32 query rows of one head and walks the keys in tiles of 32 with a running maximum and sum per
 // row (a row's result is rescaled when its maximum grows), and both products of a tile are MFMAs on float32 operands
 // (v_mfma_f32_32x32x2_f32), so that nothing is rounded that the other kernel does not round. Both are computed
 // transposed, so that everything a row owns lives in one lane (and its partner 32 lanes on): scores^T = K . Q^T over the
@@ -14,8 +15,7 @@
 // result^T = V^T . P^T over the tile's keys, taken in the order the scores' registers hold them, so that p goes from the
 // exponential straight into the MFMA's second operand, and the lane ends with 16 features of every 32 of its row. A
 // workgroup is four wavefronts with consecutive rows of one head, which share the tile of keys and values in LDS
-// (converted to float32 as they are loaded, the next tile's rows requested while this one is used; K's rows padded by a
-// float so that 32 keys' equal feature falls on 32 banks).
+// (the next tile's rows requested while this one is used; K's rows padded by a float so that 32 keys' equal feature falls on 32 banks).
 //
 // What differs from the other kernel is the order of the float32 sums (features and keys in pairs as the MFMA takes
 // them, keys in tiles of 32 with rescaling), so results agree to float32 rounding, not bit for bit.
@@ -27,9 +27,11 @@ namespace mimir {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kRows = 32;       // query rows a wavefront
-// wavefronts a workgroup (WAVES below): four, 128 consecutive rows of one head, or two where four would leave the device short of workgroups
+// wavefronts a workgroup (WAVES below, float32): four, 128 consecutive rows of one head, or two where four would leave the device short of workgroups
 constexpr int kTile = 32;       // keys a tile
 
 struct PromptParams {
@@ -48,27 +50,35 @@ __device__ __forceinline__ float element<float>(const uint32_t* raw, int e) { re
 template <>
 __device__ __forceinline__ float element<uint16_t>(const uint32_t* raw, int e) { return f16_bits_to_f32((uint16_t)(raw[e >> 1] >> (16 * (e & 1)))); }
 
+// The two values of a packed pair of bfloat16.
+__device__ __forceinline__ float bf16_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
+
 // The other half's value: lane ^ 32.
 __device__ __forceinline__ float other_half(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, __builtin_bit_cast(int, v)));
 }
 
-template <typename KV, int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const KV* __restrict__ k, const KV* __restrict__ v,
-                                                                     float* __restrict__ out, float* __restrict__ lse, PromptParams p) {
-    constexpr int KS = D + 1;            // floats between rows of the keys' tile
+template <int D>
+struct Float32Lds {
+    static constexpr int KS = D + 1;     // floats between rows of the keys' tile
+    float ks[kTile * KS];
+    __align__(16) float vs[kTile * D];
+    int vbad[2];                         // whether a tile's values hold a NaN or an infinity, for tiles of either parity
+};
+
+// Rows [first, first + ROWS) of head h of sequence b.
+template <typename KV, int D, int WAVES, int ROWS>
+__device__ __forceinline__ void rows_by_float32(const float* __restrict__ q, const KV* __restrict__ k, const KV* __restrict__ v, float* __restrict__ out,
+                                                float* __restrict__ lse, const PromptParams& p, int b, int h, int first, float* ks, float* vs, int* vbad) {
+    constexpr int KS = Float32Lds<D>::KS;
     constexpr int NT = D / 32;           // 32-feature tiles of the result
     constexpr int PER = D / 8;           // elements of a key (value) row a thread loads: eight threads a row
     constexpr int RP = 8 * WAVES;        // rows of a tile the workgroup loads at once
     constexpr int NP = kTile / RP;       // and how often
-    __shared__ float ks[kTile * KS];
-    __shared__ __align__(16) float vs[kTile * D];
-    __shared__ int vbad[2];              // whether a tile's values hold a NaN or an infinity, for tiles of either parity
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, hi = lane >> 5;
-    // the grid is (head, sequence, block of rows), the last rows first: under causality they see the most keys, and
-    // workgroups are handed out in this order
-    const int b = blockIdx.y, h = blockIdx.x, hk = h / (p.H / p.HK), bx = (int)(gridDim.z - 1 - blockIdx.z);
-    const int i0 = (bx * WAVES + wave) * kRows;  // this wavefront's first row
+    const int hk = h / (p.H / p.HK);
+    const int i0 = ROWS == WAVES * kRows || wave * kRows < ROWS ? first + wave * kRows : p.Q;  // this wavefront's first row, or none
     const int64_t Kt = p.K;
     auto seen_of = [&](int i) -> int {  // keys row i sees
         int64_t s = Kt;
@@ -78,7 +88,7 @@ __global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES =
         }
         return (int)s;
     };
-    const int last_row_wg = (bx + 1) * WAVES * kRows - 1 < p.Q ? (bx + 1) * WAVES * kRows - 1 : p.Q - 1;
+    const int last_row_wg = first + ROWS - 1 < p.Q ? first + ROWS - 1 : p.Q - 1;
     const int last_row_wave = i0 + kRows - 1 < p.Q ? i0 + kRows - 1 : p.Q - 1;
     const int seen_wg = p.causal ? seen_of(last_row_wg) : (int)Kt;
     const int seen_wave = i0 < p.Q ? (p.causal ? seen_of(last_row_wave) : (int)Kt) : 0;
@@ -240,15 +250,328 @@ __global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES =
     if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
 }
 
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                                                                  const float* __restrict__ v, float* __restrict__ out,
+                                                                                                  float* __restrict__ lse, PromptParams p) {
+    __shared__ float ks[kTile * Float32Lds<D>::KS];
+    __shared__ __align__(16) float vs[kTile * D];
+    __shared__ int vbad[2];
+    // the grid is (head, sequence, block of rows), the last rows first: under causality they see the most keys, and
+    // workgroups are handed out in this order
+    rows_by_float32<float, D, WAVES, WAVES * kRows>(q, k, v, out, lse, p, blockIdx.y, blockIdx.x, (int)(gridDim.z - 1 - blockIdx.z) * WAVES * kRows, ks, vs, vbad);
+}
+
+// The same for keys and values in binary16, by sums of products of 16-bit parts that are exact, on instructions sixteen times as fast as the float32 one:
+//   - scores: keys are binary16 as they are, a row of Q is a pair, q 2^-e = a0 + 2^-11 a1 with a0 the binary16 next to it and a1 the one next to 2^11 times what
+//     that leaves, and 2^e such that the row's largest element lies in [2^14, 2^15); the pair's products go into sums of their own. An element down to 2^-27 of the
+//     largest is held to 23 bits.
+//   - result: a weight is three bfloat16 (24 bits, whatever its size down to e^-75), a value two (its 11 bits); of the six products the one of both
+//     lowest parts, below 2^-26 of the whole, is left out.
+// A workgroup that finds a NaN or an infinity among its keys and values, or an element of Q other than zero below 2^-27 of its row's largest, or a row
+// whose largest is beyond 2^100 or below 2^-100, starts anew with rows_by_float32.
+// The MFMAs of a tile of 32 rows by 32 keys at 128 features are 1792 cycles where those on float32 operands are 8192. Against 64 bits the
+// results' error is 0.4 to 0.65 of what it was with float32 operands (1.7e-7 for 3.4e-7 over 512 normal keys, 3.0e-7 for 4.6e-7 over 2048, 5.6e-7 for 1.2e-6 with scores four times as far apart).
+//
+// LDS holds a tile's keys row by row, sixteen-byte pieces turned by the row so that 32 rows' equal piece falls on all banks, and its values
+// transposed, a feature's 32 keys in the order in which a lane holds its scores (keys 16 u + 8 a + 4 hi + c at 16 u + 8 hi +
+// 4 a + c), so that a lane's weights go from the exponential into the second operand; two neighbouring keys' values
+// meet in one dword on the way in.
+//
+// What bounds it is a wavefront's chain: some 650 vector instructions a tile (exponentials, masks, parts, staging: 2600 cycles) and the
+// MFMAs' 1792, and a causal call ends with the rows that walk all keys. So a workgroup is four
+// wavefronts of 32 rows each only where there are many (KS = 1), and otherwise (KS = 2) two pairs of wavefronts, 32 rows a pair, that
+// take a step's two tiles of keys, one each, and join their maxima, sums and results through LDS at the end: half the chain.
+// One layer of 32 heads of 128 features over 8 key heads, us:
+//   rows, keys            float32 operands   KS = 1   KS = 2
+//   512                         89.6           49.7    36.7
+//   2048                       458            203       210
+//   5 prompts of 131            35.9           27.2    23.0
+//   8 prompts of 512           201            103       127
+//   8 heads, 512 of 2048       325             163    106
+
+// e^x for x <= 0, and for NaN: 2^t with t the float32 next to x / ln 2, times 1 + ln 2 (x / ln 2 - t). Nine instructions where
+// the general function, which has overflow and subnormal results to care for, takes fifteen; a result below 2^-126 is zero here.
+__device__ __forceinline__ float exp_down(float x) {
+    constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = (float)(1.4426950408889634074 - (double)kLog2e), kLn2 = 0.6931471805599453f;
+    const float t = x * kLog2e, y = __builtin_amdgcn_exp2f(t);
+    const float held = fmaxf(x, -128.f), th = held * kLog2e;  // an infinity leaves nothing to mend
+    const float rest = __builtin_fmaf(held, kLog2eLow, __builtin_fmaf(held, kLog2e, -th));
+    return __builtin_fmaf(y, rest * kLn2, y);
+}
+
+template <int D, int KS>
+__global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                                         float* __restrict__ out, float* __restrict__ lse, PromptParams p) {
+    constexpr int NT = D / 32;                 // 32-feature tiles of the result
+    constexpr int NS = D / 16;                 // steps of the scores' product
+    constexpr int PER = D / 8, PD = PER / 2;   // elements, dwords of a key (value) row a thread loads: eight threads a row, a row of each tile
+    constexpr int G = 4 / KS;                  // groups of 32 query rows a workgroup
+    constexpr int kStep = kTile * KS;          // keys a step
+    __shared__ union Lds {
+        uint16_t kv[3][KS][kTile * D];         // the step's keys, its values' upper and lower parts
+        float results[KS > 1 ? G : 1][16 * NT * 64];
+        Float32Lds<D> by_float32;
+    } lds;
+    __shared__ int odd;                        // whether the products of float32 operands are to be taken
+    __shared__ float ml[KS > 1 ? G : 1][2][64];  // maximum and sum of the rows' second half of the keys
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, hi = lane >> 5, part = wave % KS;
+    const int b = blockIdx.y, h = blockIdx.x, hk = h / (p.H / p.HK), bx = (int)(gridDim.z - 1 - blockIdx.z);  // the last rows first
+    const int i0 = (bx * G + wave / KS) * kRows;
+    const int64_t Kt = p.K;
+    auto seen_of = [&](int i) -> int {  // keys row i sees
+        int64_t s = Kt;
+        if (p.causal) {
+            s = (int64_t)i + p.causal_offset + 1;
+            s = s < 0 ? 0 : s > Kt ? Kt : s;
+        }
+        return (int)s;
+    };
+    const int last_row_wg = (bx + 1) * G * kRows - 1 < p.Q ? (bx + 1) * G * kRows - 1 : p.Q - 1;
+    const int last_row_wave = i0 + kRows - 1 < p.Q ? i0 + kRows - 1 : p.Q - 1;
+    const int seen_wg = p.causal ? seen_of(last_row_wg) : (int)Kt;
+    const int seen_wave = i0 < p.Q ? (p.causal ? seen_of(last_row_wave) : (int)Kt) : 0;
+    const int seen_first = i0 < p.Q ? seen_of(i0) : 0;  // the fewest keys a row of this wavefront sees
+    const int row = i0 + r32;
+    const int seen = row < p.Q ? seen_of(row) : 0;
+    if (tid == 0) odd = 0;
+    __syncthreads();
+
+    // this lane's row, scaled: features 16 s + 8 hi .. + 8 of step s as the second operand's pair
+    f16x8 q0[NS], q1[NS];
+    float up = 1.f;  // 2^e
+    {
+        const float* qr = q + b * p.q_b + (int64_t)h * p.q_h + (int64_t)(row < p.Q ? row : p.Q - 1) * p.q_i + 8 * hi;
+        float amax = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) amax = fmaxf(amax, __builtin_fabsf(qr[16 * s + c] * p.scale));
+        amax = fmaxf(amax, other_half(amax, lane));
+        bool far = amax != 0.f && !(amax > 0x1p-100f && amax < 0x1p100f);
+        const int e = far || amax == 0.f ? 0 : __builtin_amdgcn_frexp_expf(amax) - 15;
+        up = __builtin_ldexpf(1.f, e);
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const float x = qr[16 * s + c] * p.scale, a = __builtin_ldexpf(x, -e);
+                far = far || !(x == 0.f || __builtin_fabsf(a) >= 0x1p-13f);
+                q0[s][c] = (_Float16)a;
+                q1[s][c] = (_Float16)((a - (float)q0[s][c]) * 2048.f);
+            }
+        if (__builtin_amdgcn_ballot_w64(far) != 0 && lane == 0) odd = 1;
+    }
+    float m = -__builtin_inff(), l = 0.f;  // the row's maximum so far; the sum over the keys this half of the lanes holds
+    f32x16 o[NT], zero;                    // the row's result, transposed: register e of tile t is feature 32 t + 8 (e / 4) + 4 hi + e % 4
+#pragma unroll
+    for (int e = 0; e < 16; e++) zero[e] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) o[t] = zero;
+
+    // a thread's part of a tile's keys and values: rows tid / 8 + 32 n, elements [PER (tid % 8), + PER)
+    const int lrow = tid >> 3, lpart = tid & 7;
+    const uint16_t* kbase = k + b * p.k_b + (int64_t)hk * p.k_h + PER * lpart;
+    const uint16_t* vbase = v + b * p.v_b + (int64_t)hk * p.v_h + PER * lpart;
+    u32x4 kreg[KS][PD / 4], vreg[KS][PD / 4];
+    auto fetch = [&](int j0) {
+#pragma unroll
+        for (int n = 0; n < KS; n++) {
+            int64_t j = j0 + lrow + kTile * n;
+            j = j < Kt ? j : Kt - 1;  // rows past the last key: never seen, loaded from the last one
+#pragma unroll
+            for (int c = 0; c < PD / 4; c++) {
+                kreg[n][c] = ((const u32x4*)(kbase + j * p.k_p))[c];
+                vreg[n][c] = ((const u32x4*)(vbase + j * p.v_p))[c];
+            }
+        }
+    };
+    auto key_piece = [](int r, int piece) { return D == 128 ? piece ^ (r & 15) : piece ^ ((r >> 1) & 7); };
+    auto value_at = [](int f, int slot) { return f * kTile + ((((slot >> 3) ^ ((f >> 2) & 3)) << 3) | (slot & 7)); };
+    auto slot_of = [](int key) { return (key & 16) | (key & 4) << 1 | (key & 8) >> 1 | (key & 3); };
+    auto stage = [&]() {
+        const f16x2 none = {(_Float16)0.f, (_Float16)0.f};
+        f16x2 chk = none;  // 0 * each summed: NaN as soon as one is a NaN or an infinity
+#pragma unroll
+        for (int n = 0; n < KS; n++) {
+            uint16_t *ks = lds.kv[0][n], *vh = lds.kv[1][n], *vl = lds.kv[2][n];
+            const int r = lrow;
+#pragma unroll
+            for (int c = 0; c < PD / 4; c++) *(u32x4*)(ks + r * D + key_piece(r, lpart * (PD / 4) + c) * 8) = kreg[n][c];
+            // the thread eight lanes on has the neighbouring key's same features: of two features, the even key's thread stores the first's two keys
+            const int odd = r & 1, slot = slot_of(r & ~1);
+#pragma unroll
+            for (int w = 0; w < PD; w++) {
+                const uint32_t mine = vreg[n][w >> 2][w & 3];
+                const uint32_t theirs = __builtin_bit_cast(uint32_t, dpp_f32<0x128>(__builtin_bit_cast(float, mine)));  // row_ror:8
+                const uint32_t two = odd ? __builtin_amdgcn_perm(mine, theirs, 0x07060302u) : __builtin_amdgcn_perm(theirs, mine, 0x05040100u);
+                const float f0 = (float)as_f16x2(two)[0], f1 = (float)as_f16x2(two)[1];
+                const uint32_t upper = pack_bf16(f0, f1), lower = pack_bf16(f0 - bf16_lo(upper), f1 - bf16_hi(upper));
+                const int at = value_at(PER * lpart + 2 * w + odd, slot);
+                *(uint32_t*)(vh + at) = upper;
+                *(uint32_t*)(vl + at) = lower;
+                chk = __builtin_bit_cast(f16x2, mine) * none + chk;
+                const uint32_t key = kreg[n][w >> 2][w & 3];
+                chk = __builtin_bit_cast(f16x2, key) * none + chk;
+            }
+        }
+        const float bad = (float)chk[0] + (float)chk[1];
+        if (__builtin_amdgcn_ballot_w64(bad != bad) != 0 && lane == 0) odd = 1;
+    };
+
+    const uint16_t *ks = lds.kv[0][part], *vh = lds.kv[1][part], *vl = lds.kv[2][part];
+    if (seen_wg > 0) fetch(0);
+    bool by_float32 = false;
+    for (int jw = 0; jw < seen_wg; jw += kStep) {
+        const int j0 = jw + kTile * part;
+        __syncthreads();  // everyone has read the tiles before
+        stage();
+        __syncthreads();
+        if (odd != 0) {  // the same for all: it is set before the barrier above or behind the next one
+            by_float32 = true;
+            break;
+        }
+        if (jw + kStep < seen_wg) fetch(jw + kStep);
+        if (j0 >= seen_wave) continue;  // nothing of this tile is seen by this wavefront's rows (uniform)
+        const bool whole = j0 + kTile <= seen_first;
+
+        // scores, transposed (K . Q^T): register e is 2^-e of key j0 + 8 (e / 4) + 4 hi + e % 4 against this lane's row
+        f32x16 s = zero, s1 = zero;
+        int k0 = r32 * D + key_piece(r32, hi) * 8;
+        asm volatile("" : "+v"(k0));  // eight addresses worked out again for each tile instead of eight registers
+#pragma unroll
+        for (int f = 0; f < NS; f++) {
+            const f16x8 kf = *(const f16x8*)(ks + (k0 ^ 16 * f));
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q1[f], s1, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q0[f], s, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s1[e], 1.f / 2048.f, s[e]);
+        float mx = -__builtin_inff();
+        if (!whole) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) s[e] = 8 * (e >> 2) + (e & 3) < seen - j0 - 4 * hi ? s[e] : -__builtin_inff();
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) mx = fmaxf(mx, s[e]);
+        mx = fmaxf(mx, other_half(mx, lane)) * up;
+        const float mn = fmaxf(m, mx);
+        float al = 1.f, sum = 0.f;
+        if (mn > -__builtin_inff()) {  // the row has seen a key by now
+            al = exp_down(m - mn);
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                s[e] = exp_down(__builtin_fmaf(s[e], up, -mn));
+                sum += s[e];
+            }
+        } else {
+            s = zero;
+        }
+        l = l * al + sum;
+        m = mn;
+        if (__builtin_amdgcn_ballot_w64(al != 1.f) != 0) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * al;
+        }
+        bf16x8 p0[2], p1[2], p2[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            u32x4 a, b, c;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float x = s[8 * u + 2 * i], y = s[8 * u + 2 * i + 1];
+                a[i] = pack_bf16(x, y);
+                const float x1 = x - bf16_lo(a[i]), y1 = y - bf16_hi(a[i]);
+                b[i] = pack_bf16(x1, y1);
+                c[i] = pack_bf16(x1 - bf16_lo(b[i]), y1 - bf16_hi(b[i]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            p0[u] = __builtin_bit_cast(bf16x8, a), p1[u] = __builtin_bit_cast(bf16x8, b), p2[u] = __builtin_bit_cast(bf16x8, c);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int at = value_at(32 * t + r32, 16 * u + 8 * hi);
+                const bf16x8 h8 = *(const bf16x8*)(vh + at), l8 = *(const bf16x8*)(vl + at);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, p1[u], o[t], 0, 0, 0);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, p2[u], o[t], 0, 0, 0);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, p0[u], o[t], 0, 0, 0);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, p1[u], o[t], 0, 0, 0);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, p0[u], o[t], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (by_float32) {
+        __syncthreads();
+        rows_by_float32<uint16_t, D, 4, G * kRows>(q, k, v, out, lse, p, b, h, bx * G * kRows, lds.by_float32.ks, lds.by_float32.vs, lds.by_float32.vbad);
+        return;
+    }
+
+    l += other_half(l, lane);
+    if (KS > 1) {  // the second wavefront's half of the keys joins the first's
+        float* theirs = lds.results[wave / KS] + lane;
+        __syncthreads();
+        if (part == 1) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) theirs[64 * (16 * t + e)] = o[t][e];
+            ml[wave / KS][0][lane] = m;
+            ml[wave / KS][1][lane] = l;
+        }
+        __syncthreads();
+        if (part == 1) return;
+        const float m1 = ml[wave / KS][0][lane], l1 = ml[wave / KS][1][lane], mn = fmaxf(m, m1);
+        const float a0 = m == mn ? 1.f : exp_down(m - mn), a1 = m1 == mn ? 1.f : exp_down(m1 - mn);
+        l = l * a0 + l1 * a1;
+        m = mn;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * a0 + theirs[64 * (16 * t + e)] * a1;
+    }
+    if (row >= p.Q) return;
+    float* orow = out + b * p.o_b + (int64_t)h * p.o_h + (int64_t)row * p.o_i;
+    const float inv = l == 0.f ? 0.f : 1.0f / l;
+    const bool wide = (((uintptr_t)orow) & 15) == 0;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            f32x4 r;
+#pragma unroll
+            for (int c = 0; c < 4; c++) r[c] = l == 0.f ? 0.f : o[t][4 * g + c] * inv;
+            float* dst = orow + 32 * t + 8 * g + 4 * hi;
+            if (wide) *(f32x4*)dst = r;
+            else
+#pragma unroll
+                for (int c = 0; c < 4; c++) dst[c] = r[c];
+        }
+    if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
+}
+
 std::atomic<int> g_prompt{1};  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup
 
-template <typename KV, int WAVES>
-hipError_t launch(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
-    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + WAVES * kRows - 1) / (WAVES * kRows)));
-    if (a.D == 128)
-        hipLaunchKernelGGL((attn_prompt_kernel<KV, 128, WAVES>), grid, dim3(64 * WAVES), 0, st, a.q, (const KV*)a.k, (const KV*)a.v, a.out, a.lse, p);
-    else
-        hipLaunchKernelGGL((attn_prompt_kernel<KV, 64, WAVES>), grid, dim3(64 * WAVES), 0, st, a.q, (const KV*)a.k, (const KV*)a.v, a.out, a.lse, p);
+template <int WAVES>
+hipError_t launch_f32(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
+    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + WAVES * kRows - 1) / (WAVES * kRows))), block(64 * WAVES);
+    const float *k = (const float*)a.k, *v = (const float*)a.v;
+    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_kernel<128, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+    else hipLaunchKernelGGL((attn_prompt_kernel<64, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+    return hipGetLastError();
+}
+
+template <int KS>
+hipError_t launch_f16(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
+    constexpr int kWg = 4 / KS * kRows;
+    const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + kWg - 1) / kWg)), block(256);
+    const uint16_t *k = (const uint16_t*)a.k, *v = (const uint16_t*)a.v;
+    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_half_kernel<128, KS>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+    else hipLaunchKernelGGL((attn_prompt_half_kernel<64, KS>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
     return hipGetLastError();
 }
 
@@ -279,11 +602,12 @@ hipError_t attention_prompt(const AttnArgs& a, hipStream_t st) {
     p.scale = (float)a.scale;
     p.causal = a.causal;
     p.causal_offset = a.causal_offset;
-    // workgroups of two wavefronts where those of four would be fewer than the device holds at two a compute unit
-    const bool two = a.B * a.H * ((a.Q + 4 * kRows - 1) / (4 * kRows)) < 512;
+    // where workgroups of 128 rows would be fewer than the device holds at two a compute unit: two wavefronts a workgroup (float32), or
+    // two wavefronts on the same rows (binary16; at 512 workgroups the two are level, see the figures there)
+    const bool few = a.B * a.H * ((a.Q + 4 * kRows - 1) / (4 * kRows)) < 512;
     note_kernel("attn_prompt_kernel");
-    if (a.kv_dtype == kF16) return two ? launch<uint16_t, 2>(a, p, st) : launch<uint16_t, 4>(a, p, st);
-    return two ? launch<float, 2>(a, p, st) : launch<float, 4>(a, p, st);
+    if (a.kv_dtype == kF16) return few ? launch_f16<2>(a, p, st) : launch_f16<1>(a, p, st);
+    return few ? launch_f32<2>(a, p, st) : launch_f32<4>(a, p, st);
 }
 
 }  // namespace mimir

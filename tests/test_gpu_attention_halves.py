@@ -1,5 +1,5 @@
-"""Attention of many query positions over binary16 keys and values (attention_prompt.hip): they enter products of float32 operands as they
-are, so that results are as near 64 bits as over float32 caches, whatever the sizes of weights, values and features. Sizes at the edges of tiles (32
+"""Attention of many query positions over binary16 keys and values (attention_prompt.hip), by products of 16-bit parts: results are as near 64 bits as
+over float32 caches, whatever the sizes of weights, values and features. Sizes at the edges of tiles (32
 keys) and workgroups (64 or 128 rows), against 64 bits, the float32 cache and the kernel that takes a query row a workgroup."""
 import numpy as np
 import pytest
@@ -123,3 +123,24 @@ def check_rows(q, k, v, bound):
     want = exact(q, k, v, 1.0, k.shape[2])  # an offset that hides no key
     err = np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1))
     assert err.max() <= bound, err.max()
+
+
+@pytest.mark.parametrize("B,H,Q,D,ratio", [
+    (4, 32, 449, 128, 2.0 ** -27), (4, 32, 449, 128, 2.0 ** -40),  # workgroups of 128 rows: a pair of binary16 holds the small feature to its last bit but one; products of float32
+    (1, 4, 100, 128, 2.0 ** -27), (1, 4, 100, 128, 2.0 ** -29), (1, 4, 100, 64, 2.0 ** -29),  # workgroups of 64
+])
+def test_a_row_whose_features_lie_far_apart(B, H, Q, D, ratio):
+    """One row of one sequence has a largest feature that meets keys of zero and one `ratio` of it that meets large keys: that row and those that share
+    its workgroup are within float32's rounding (scores up to about 5, weights to 5 x 2^-24, some 3e-7) of 64 bits, as all others are."""
+    rng = np.random.default_rng(Q + D)
+    q = rng.normal(size=(B, H, Q, D)).astype(np.float32); q[..., :2] = 0
+    q[0, :, 70, 0] = 2.0 ** 13; q[0, :, 70, 1] = np.float32(1.2345678 * 2.0 ** 13 * ratio)
+    k, v = (rng.normal(size=(B, 2, Q, D)).astype(np.float32) for _ in range(2))
+    k[..., 0] = 0; k[..., 1] = np.clip(k[..., 1], -3, 3) * 2.0 ** 14
+    k, v = T.O.f32_to_f16(k).view(np.uint16), T.O.f32_to_f16(v).view(np.uint16)
+    T.gpu.say(f"attention over binary16, features {ratio} apart, B={B} Q={Q} D={D}")
+    got, _ = T.attention(q, k, v, 1 / np.sqrt(D), causal=True, offset=0, kv_dt=capi.F16)
+    assert T.last_kernel() == "attn_prompt_kernel"
+    want = exact(q, k, v, 1 / np.sqrt(D), 0)
+    err = np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1))
+    assert err.max() <= 2e-6, err.max()

@@ -160,6 +160,87 @@ hipError_t kv_write(const float* src, void* cache, int cache_dt, int64_t B, int 
     return hipGetLastError();
 }
 
+// A prompt's positions in one launch: of rows b s + p, ld floats apart each, the query heads are rotated in place, the key heads
+// rotated and cast into the keys cache at position pos + p of sequence b, the value heads cast into the values cache (rope_kernel's and
+// kv_write_kernel's operations one by one); bias: null, or [(H + 2 HK) dim] added first. A workgroup a row, a thread eight features at a time: four pairs, in vectors of
+// sixteen bytes. Memory bounds it: 2048 rows of the 8B shape 40 us as four launches of an element a thread, 20 as one; 8 x 512 rows 92 -> 35.
+struct PromptHeads {
+    float* q;
+    const float *k, *v, *bias;
+    int64_t q_row, k_row, v_row;
+    void *kcache, *vcache;
+    const float *cosv, *sinv;
+    int64_t cap, pos;
+    int cache_dt, s, H, HK, dim, rope_dim, interleaved;
+};
+
+__device__ __forceinline__ void store_cast(void* cache, int cache_dt, int64_t at, const f32x4 v) {
+    if (cache_dt == kF32) {
+        *(f32x4*)((float*)cache + at) = v;
+    } else {
+        const u32x2 o = {(uint32_t)f32_to_f16_bits(v[0]) | (uint32_t)f32_to_f16_bits(v[1]) << 16, (uint32_t)f32_to_f16_bits(v[2]) | (uint32_t)f32_to_f16_bits(v[3]) << 16};
+        *(u32x2*)((uint16_t*)cache + at) = o;
+    }
+}
+
+__global__ __launch_bounds__(256) void rope_kv_prompt_kernel(PromptHeads a) {
+    const int64_t row = blockIdx.x;
+    const int b = (int)(row / a.s), p = (int)(row - (int64_t)b * a.s), half = a.rope_dim >> 1, eights = a.dim >> 3;
+    const float *cosr = a.cosv + (a.pos + p) * half, *sinr = a.sinv + (a.pos + p) * half;
+    for (int t = threadIdx.x; t < (a.H + 2 * a.HK) * eights; t += 256) {
+        const int head = t / eights, e = t - head * eights;
+        const bool is_q = head < a.H, is_v = head >= a.H + a.HK;
+        const float* from = is_q ? a.q + row * a.q_row + (int64_t)head * a.dim
+                                 : is_v ? a.v + row * a.v_row + (int64_t)(head - a.H - a.HK) * a.dim : a.k + row * a.k_row + (int64_t)(head - a.H) * a.dim;
+        const bool turns = !is_v && 8 * e < a.rope_dim, apart = turns && !a.interleaved;
+        const int f0 = apart ? 4 * e : 8 * e, f1 = apart ? f0 + half : f0 + 4;  // this thread's two fours of features
+        f32x4 x = *(const f32x4*)(from + f0), y = *(const f32x4*)(from + f1);
+        if (a.bias) {
+            const float* bias = a.bias + (int64_t)head * a.dim;
+            const f32x4 bx = *(const f32x4*)(bias + f0), by = *(const f32x4*)(bias + f1);
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = x[i] + bx[i], y[i] = y[i] + by[i];
+        }
+        if (turns) {
+            const f32x4 c = *(const f32x4*)(cosr + 4 * e), sn = *(const f32x4*)(sinr + 4 * e);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {  // pair i: both of one four, or one of each
+                const float u = apart ? x[i] : i < 2 ? x[2 * i] : y[2 * i - 4], w = apart ? y[i] : i < 2 ? x[2 * i + 1] : y[2 * i - 3];
+                const float uc = u * c[i], ws = w * sn[i], us = u * sn[i], wc = w * c[i];
+                const float ra = uc - ws, rb = apart ? wc + us : us + wc;
+                if (apart) x[i] = ra, y[i] = rb;
+                else if (i < 2) x[2 * i] = ra, x[2 * i + 1] = rb;
+                else y[2 * i - 4] = ra, y[2 * i - 3] = rb;
+            }
+        }
+        if (is_q) {
+            float* to = a.q + row * a.q_row + (int64_t)head * a.dim;
+            *(f32x4*)(to + f0) = x;
+            *(f32x4*)(to + f1) = y;
+        } else {
+            void* cache = is_v ? a.vcache : a.kcache;
+            const int64_t at = (((int64_t)b * a.HK + (is_v ? head - a.H - a.HK : head - a.H)) * a.cap + a.pos + p) * a.dim;
+            store_cast(cache, a.cache_dt, at + f0, x);
+            store_cast(cache, a.cache_dt, at + f1, y);
+        }
+    }
+}
+
+// Rows of whole eights, rotated ones too, on 16 bytes.
+bool rope_kv_prompt_ok(const float* q, const float* k, const float* v, int64_t q_row, int64_t k_row, int64_t v_row, int dim, int rope_dim) {
+    return dim > 0 && dim % 8 == 0 && rope_dim % 8 == 0 && q_row % 4 == 0 && k_row % 4 == 0 && v_row % 4 == 0 &&
+           (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+}
+
+hipError_t rope_kv_prompt(float* q, const float* k, const float* v, int64_t q_row, int64_t k_row, int64_t v_row, void* kcache, void* vcache, int cache_dt,
+                          int64_t B, int64_t s, int H, int HK, int dim, int rope_dim, int interleaved, int64_t cap, int64_t pos, const float* cosv, const float* sinv,
+                          const float* bias, hipStream_t st) {
+    if (B * s == 0) return hipSuccess;
+    const PromptHeads a{q, k, v, bias, q_row, k_row, v_row, kcache, vcache, cosv, sinv, cap, pos, cache_dt, (int)s, H, HK, dim, rope_dim, interleaved};
+    hipLaunchKernelGGL(rope_kv_prompt_kernel, dim3((unsigned)(B * s)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 // One position of a decoding step in one launch: qkv is [B, (H + 2 HK) * dim],
 // the rows of a fused q|k|v product. The query heads are rotated in place, the
 // key heads are rotated and written to the keys cache at the position *pos_dev

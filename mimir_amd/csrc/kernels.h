@@ -168,6 +168,11 @@ hipError_t rope(const float* x, float* y, int64_t rows, int64_t s, int head_dim,
                 int64_t offset, hipStream_t st, int64_t period = 0);
 hipError_t kv_write(const float* src, void* cache, int cache_dt, int64_t B, int heads, int64_t s, int dim, int64_t cap,
                     int64_t pos, int64_t src_b, int64_t src_h, int64_t src_p, hipStream_t st);
+// A prompt's rotation and cache writes in one launch: q, k, v rows of B sequences of s positions, *_row floats apart.
+bool rope_kv_prompt_ok(const float* q, const float* k, const float* v, int64_t q_row, int64_t k_row, int64_t v_row, int dim, int rope_dim);
+hipError_t rope_kv_prompt(float* q, const float* k, const float* v, int64_t q_row, int64_t k_row, int64_t v_row, void* kcache, void* vcache, int cache_dt,
+                          int64_t B, int64_t s, int H, int HK, int dim, int rope_dim, int interleaved, int64_t cap, int64_t pos, const float* cosv, const float* sinv,
+                          const float* bias, hipStream_t st);
 // RMSNorm that also writes the row converted for the Q4_0 kernel (y may be
 // null); rmsnorm_q4act_ok says whether a row length qualifies.
 bool rmsnorm_q4act_ok(int64_t d);

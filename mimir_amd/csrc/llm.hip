@@ -230,28 +230,34 @@ static mi355x_status forward(Model& m, int64_t s) {
             if (mi355x_status st = linear(m, b.k, h, k, rows)) return st;
             if (mi355x_status st = linear(m, b.v, h, v, rows)) return st;
         }
-        if (b.biased()) {  // Linear.Forward: the bias behind the product, before the rotation (nn/layers.go:49-55)
-            LLM_HIP(add_bias(q, b.q_bias.buf.as<float>(), rows, qd, m.stream), "q bias");
-            LLM_HIP(add_bias(k, b.k_bias.buf.as<float>(), rows, kvd, m.stream), "k bias");
-            LLM_HIP(add_bias(v, b.v_bias.buf.as<float>(), rows, kvd, m.stream), "v bias");
-        }
-        // q and k are [B, s, heads, dim]. One position: every head of every
-        // sequence is a row `dim` apart. More: per sequence, heads are rows
-        // `dim` apart and positions heads * dim apart.
-        if (s == 1) {
-            LLM_HIP(rope(q, q, B * c.heads, 1, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, qd, c.head_dim, qd,
-                         m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream), "rope q");
-            LLM_HIP(rope(k, k, B * c.kv_heads, 1, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, kvd, c.head_dim, kvd,
-                         m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream), "rope k");
+        const float* bias = b.biased() ? b.qkv_bias.as<float>() : nullptr;  // behind the product, before the rotation (nn/layers.go:49-55)
+        if (rope_kv_prompt_ok(q, k, v, qd, kvd, kvd, c.head_dim, c.rope_dim)) {
+            LLM_HIP(rope_kv_prompt(q, k, v, qd, kvd, kvd, m.keys[i].p, m.values[i].p, c.cache_dtype, B, s, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved,
+                                   c.context, past, m.cos_t.as<float>(), m.sin_t.as<float>(), bias, m.stream), "rope and cache");
         } else {
-            // the sequences' positions follow one another at the same distance: one launch, each sequence counting from `past`
-            LLM_HIP(rope(q, q, c.heads, B * s, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, qd, c.head_dim, qd,
-                         m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream, s), "rope q");
-            LLM_HIP(rope(k, k, c.kv_heads, B * s, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, kvd, c.head_dim, kvd,
-                         m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream, s), "rope k");
+            if (bias) {
+                LLM_HIP(add_bias(q, b.q_bias.buf.as<float>(), rows, qd, m.stream), "q bias");
+                LLM_HIP(add_bias(k, b.k_bias.buf.as<float>(), rows, kvd, m.stream), "k bias");
+                LLM_HIP(add_bias(v, b.v_bias.buf.as<float>(), rows, kvd, m.stream), "v bias");
+            }
+            // q and k are [B, s, heads, dim]. One position: every head of every
+            // sequence is a row `dim` apart. More: per sequence, heads are rows
+            // `dim` apart and positions heads * dim apart.
+            if (s == 1) {
+                LLM_HIP(rope(q, q, B * c.heads, 1, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, qd, c.head_dim, qd,
+                             m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream), "rope q");
+                LLM_HIP(rope(k, k, B * c.kv_heads, 1, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, kvd, c.head_dim, kvd,
+                             m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream), "rope k");
+            } else {
+                // the sequences' positions follow one another at the same distance: one launch, each sequence counting from `past`
+                LLM_HIP(rope(q, q, c.heads, B * s, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, qd, c.head_dim, qd,
+                             m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream, s), "rope q");
+                LLM_HIP(rope(k, k, c.kv_heads, B * s, c.head_dim, c.rope_dim, c.interleaved, c.head_dim, kvd, c.head_dim, kvd,
+                             m.cos_t.as<float>(), m.sin_t.as<float>(), past, m.stream, s), "rope k");
+            }
+            LLM_HIP(kv_write(k, m.keys[i].p, c.cache_dtype, B, c.kv_heads, s, c.head_dim, c.context, past, s * kvd, c.head_dim, kvd, m.stream), "cache keys");
+            LLM_HIP(kv_write(v, m.values[i].p, c.cache_dtype, B, c.kv_heads, s, c.head_dim, c.context, past, s * kvd, c.head_dim, kvd, m.stream), "cache values");
         }
-        LLM_HIP(kv_write(k, m.keys[i].p, c.cache_dtype, B, c.kv_heads, s, c.head_dim, c.context, past, s * kvd, c.head_dim, kvd, m.stream), "cache keys");
-        LLM_HIP(kv_write(v, m.values[i].p, c.cache_dtype, B, c.kv_heads, s, c.head_dim, c.context, past, s * kvd, c.head_dim, kvd, m.stream), "cache values");
         AttnArgs at;
         at.q = q; at.k = m.keys[i].p; at.v = m.values[i].p; at.kv_dtype = c.cache_dtype; at.out = a; at.lse = nullptr;
         at.q_strides[0] = s * qd; at.q_strides[1] = c.head_dim; at.q_strides[2] = qd;

@@ -526,3 +526,32 @@ def test_k_quant_and_q8_0_models_decode_from_a_graph(linear_dt, batch, heads, he
     for i, (a, w) in enumerate(zip(runs[2][0][0, :20].tolist(), want)):
         assert a == w, f"token {i}: device {a}, oracle {w}, oracle's margin there {margins[i]:.4g}"
     assert np.array_equal(runs[1][0], runs[2][0]) and np.array_equal(runs[0][0], runs[2][0]) and np.array_equal(runs[0][1], runs[2][0])
+
+
+@pytest.mark.parametrize("arch,heads,head_dim,rope_dim,cache", [
+    ("llama", 4, 128, 64, capi.F32),   # neighbouring features turn, the upper half passes
+    ("qwen2", 4, 128, 128, capi.F32),  # halves turn against each other
+    ("qwen2", 8, 64, 48, capi.F16),    # of a head in part, a binary16 cache
+    ("llama", 8, 36, 36, capi.F32),    # heads that are no whole eights of features: the launches apart
+])
+def test_a_prompts_rotation_and_cache_writes(arch, heads, head_dim, rope_dim, cache):
+    """Two sequences, two calls, the second behind the first's positions: logits of every position against the oracle (binary16 rounds the cache on
+    both sides, so a value on a boundary moves a logit by 2^-11 of a key: the bound there is the one of the other binary16 tests)."""
+    gpu.lib()
+    c = _small_q4_config(2, cache)
+    c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved = heads, heads // 4, head_dim, rope_dim, int(arch == "llama")
+    cfg = _oracle_config(c)
+    cfg.arch = arch
+    om = OL.synthetic(cfg, seed=3, output_dt=O.Q4_0)
+    gpu.say(f"prompt rotation {arch} {heads} x {head_dim}, {rope_dim} turn")
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(40)
+    prompts = np.random.default_rng(3).integers(0, c.vocab, (2, 38))
+    got = np.concatenate([m.logits(prompts[:, :33], all=True), m.logits(prompts[:, 33:], all=True)], 1)
+    odt = O.F32 if cache == capi.F32 else O.F16
+    for b in range(2):
+        caches = om.new_caches(c.context, odt)
+        want = np.concatenate([om.logits(prompts[b, :33].tolist(), caches, all=True), om.logits(prompts[b, 33:].tolist(), caches, all=True)])
+        err = np.abs(got[b] - want).max(1) / np.abs(want).max()
+        assert err.max() <= (1e-3 if cache == capi.F32 else 0.02) and np.median(err) <= 1e-5, err

@@ -450,3 +450,19 @@ def test_swiglu_add_argmax():
     tiny = gpu.dev(np.array([[-np.inf, -np.inf], [np.nan, np.nan]], np.float32))
     capi.check(l.mi355x_argmax(tiny.data_ptr(), 2, 2, idx.data_ptr(), gpu.stream())); gpu.sync()
     assert idx.cpu().tolist()[:2] == [0, 0]
+
+
+@pytest.mark.parametrize("K,off", [(64, 20), (256, 254), (288, 100), (8192, 8190), (8224, 8222), (8224, -1)])
+def test_shares_of_the_keys_are_put_together(K, off):
+    """Two query positions over shares of 32 keys: 2, 8, 9, 256 and 257 of them (eight are read ahead, 256 are a round of the threads), some or all of them
+    without a key that a row sees."""
+    rng = np.random.default_rng(K + off)
+    q = rng.normal(size=(1, 4, 2, 64)).astype(np.float32)
+    k, v = (rng.normal(size=(1, 1, K, 64)).astype(np.float32) for _ in range(2))
+    gpu.say(f"attention, two positions, K={K} offset={off}")
+    out, lse = attention(q, k, v, 0.125, causal=True, offset=off)
+    wo, wl = O.attention(q, k, v, 0.125, causal=True, causal_offset=off)
+    close(out, wo)
+    seen = np.isfinite(wl)
+    assert np.array_equal(np.isfinite(lse), seen) and not out[~seen].any()
+    close(lse[seen], wl[seen])

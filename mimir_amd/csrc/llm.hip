@@ -62,7 +62,8 @@ struct Model : Decoder {
     std::vector<DevBuf> keys, values;    // per block: [batch, kv_heads, context, head_dim]
 
     // activations of up to max_rows rows (batch x tokens of one call)
-    DevBuf x, h, q, k, v, a, o, gate, up, s, xlast, hlast, act[kActClasses], act2;
+    DevBuf x, h, q, k, v, a, o, gate, s, xlast, hlast, act[kActClasses], act2;
+    float* up = nullptr;  // behind gate's rows: products of both matrices at once have [rows, 2 hidden] there
     DevBuf fx_panel;  // the workspace of the Q4_0 products of a prompt's rows on the binary16 matrix cores: the largest product's
 
     // `fast` says the blocks qualify for the step of fused launches (Q4_0 linears that the fixed-point kernel takes).
@@ -200,6 +201,9 @@ mi355x_status embed_rows(Model& m, const int32_t* idx_dev, int64_t rows, float* 
 
 }  // namespace
 
+// Matrices of one K-quant dtype kept in one buffer: their products are one, by x converted as it is normalized.
+static bool kq_together(const Weight& w) { return w.set() && (w.dtype == kQ4_K || w.dtype == kQ6_K); }
+
 // One pass of s tokens per sequence over the blocks (llm/model.go:391-437),
 // tokens already on the device at m.tokens_dev [batch, s]. Leaves the final
 // hidden state in m.x; advances the caches.
@@ -208,13 +212,13 @@ static mi355x_status forward(Model& m, int64_t s) {
     const int64_t B = c.batch, rows = B * s, past = m.cache_len;
     const int64_t qd = (int64_t)c.heads * c.head_dim, kvd = (int64_t)c.kv_heads * c.head_dim;
     float *x = m.x.as<float>(), *h = m.h.as<float>(), *q = m.q.as<float>(), *k = m.k.as<float>(), *v = m.v.as<float>();
-    float *a = m.a.as<float>(), *o = m.o.as<float>(), *gate = m.gate.as<float>(), *up = m.up.as<float>(), *sw = m.s.as<float>();
+    float *a = m.a.as<float>(), *o = m.o.as<float>(), *gate = m.gate.as<float>(), *up = m.up, *sw = m.s.as<float>();
     bool done[kActClasses];
     if (mi355x_status st = embed_rows(m, m.tokens_dev.as<int32_t>(), rows, x, device_error_word())) return st;
-    // x += in . W^T: the prompt-sized fixed-point products add x as they store, the others leave it to a launch
+    // x += in . W^T: the prompt-sized fixed-point products and the K-quants' add x as they store, the others leave it to a launch
     auto onto_x = [&](const Weight& w, const float* in) -> mi355x_status {
         const int cls = act_class(w, rows, m.fx_panel.bytes);
-        if (cls == kActFx || cls == kActFxPairs) return linear(m, w, in, x, rows, x);
+        if (cls == kActFx || cls == kActFxPairs || cls == kActKQ) return linear(m, w, in, x, rows, x);
         if (mi355x_status st = linear(m, w, in, o, rows)) return st;
         LLM_HIP(add(x, o, x, rows * c.embed, m.stream), "residual");
         return MI355X_OK;
@@ -223,7 +227,15 @@ static mi355x_status forward(Model& m, int64_t s) {
         Block& b = m.blocks[i];
         bool together;
         if (mi355x_status st = linear_parts(m, {&b.q, &b.k, &b.v}, {q, k, v}, false, x, b.attn_norm, rows, &together)) return st;
-        if (!together) {
+        float *qp = q, *kp = k, *vp = v;
+        int64_t qld = qd, kld = kvd;  // between positions
+        if (!together && kq_together(b.qkv) && qd + 2 * kvd <= 2 * (int64_t)c.hidden &&
+            rope_kv_prompt_ok(gate, gate + qd, gate + qd + kvd, qd + 2 * kvd, qd + 2 * kvd, qd + 2 * kvd, c.head_dim, c.rope_dim)) {
+            LLM_HIP(rmsnorm_kq_act(x, b.attn_norm.buf.as<float>(), m.act[kActKQ].p, rows, c.embed, c.eps, m.stream), "attn_norm");
+            if (mi355x_status st = linear(m, b.qkv, h, gate, rows)) return st;
+            qp = gate, kp = gate + qd, vp = gate + qd + kvd;
+            qld = kld = qd + 2 * kvd;
+        } else if (!together) {
             LLM_HIP(rmsnorm(x, b.attn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "attn_norm");
             if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.q, &b.k, &b.v}, done)) return st;
             if (mi355x_status st = linear(m, b.q, h, q, rows)) return st;
@@ -231,8 +243,8 @@ static mi355x_status forward(Model& m, int64_t s) {
             if (mi355x_status st = linear(m, b.v, h, v, rows)) return st;
         }
         const float* bias = b.biased() ? b.qkv_bias.as<float>() : nullptr;  // behind the product, before the rotation (nn/layers.go:49-55)
-        if (rope_kv_prompt_ok(q, k, v, qd, kvd, kvd, c.head_dim, c.rope_dim)) {
-            LLM_HIP(rope_kv_prompt(q, k, v, qd, kvd, kvd, m.keys[i].p, m.values[i].p, c.cache_dtype, B, s, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved,
+        if (rope_kv_prompt_ok(qp, kp, vp, qld, kld, kld, c.head_dim, c.rope_dim)) {
+            LLM_HIP(rope_kv_prompt(qp, kp, vp, qld, kld, kld, m.keys[i].p, m.values[i].p, c.cache_dtype, B, s, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved,
                                    c.context, past, m.cos_t.as<float>(), m.sin_t.as<float>(), bias, m.stream), "rope and cache");
         } else {
             if (bias) {
@@ -259,12 +271,12 @@ static mi355x_status forward(Model& m, int64_t s) {
             LLM_HIP(kv_write(v, m.values[i].p, c.cache_dtype, B, c.kv_heads, s, c.head_dim, c.context, past, s * kvd, c.head_dim, kvd, m.stream), "cache values");
         }
         AttnArgs at;
-        at.q = q; at.k = m.keys[i].p; at.v = m.values[i].p; at.kv_dtype = c.cache_dtype; at.out = a; at.lse = nullptr;
-        at.q_strides[0] = s * qd; at.q_strides[1] = c.head_dim; at.q_strides[2] = qd;
+        at.q = qp; at.k = m.keys[i].p; at.v = m.values[i].p; at.kv_dtype = c.cache_dtype; at.out = a; at.lse = nullptr;
+        at.q_strides[0] = s * qld; at.q_strides[1] = c.head_dim; at.q_strides[2] = qld;
+        at.o_strides[0] = s * qd; at.o_strides[1] = c.head_dim; at.o_strides[2] = qd;
         at.k_strides[0] = at.v_strides[0] = (int64_t)c.kv_heads * c.context * c.head_dim;
         at.k_strides[1] = at.v_strides[1] = (int64_t)c.context * c.head_dim;
         at.k_strides[2] = at.v_strides[2] = c.head_dim;
-        for (int j = 0; j < 3; j++) at.o_strides[j] = at.q_strides[j];
         at.B = B; at.Q = s; at.K = past + s; at.H = c.heads; at.HK = c.kv_heads; at.D = c.head_dim;
         at.scale = 1.0 / std::sqrt((double)c.head_dim);
         at.causal = 1; at.causal_offset = past;
@@ -275,14 +287,22 @@ static mi355x_status forward(Model& m, int64_t s) {
         if (mi355x_status st = convert_for(m, a, rows, qd, {&b.o}, done)) return st;
         if (mi355x_status st = onto_x(b.o, a)) return st;
         if (mi355x_status st = linear_parts(m, {&b.gate, &b.up}, {sw, nullptr}, true, x, b.ffn_norm, rows, &together)) return st;
-        if (!together) {
+        bool converted = false;
+        if (!together && kq_together(b.gate_up)) {
+            LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[kActKQ].p, rows, c.embed, c.eps, m.stream), "ffn_norm");
+            if (mi355x_status st = linear(m, b.gate_up, h, gate, rows)) return st;
+            converted = act_class(b.down, rows, m.fx_panel.bytes) == kActKQ;
+            if (converted) LLM_HIP(swiglu_kq_act(gate, gate + c.hidden, m.act[kActKQ].p, rows, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
+            else LLM_HIP(swiglu(gate, gate + c.hidden, sw, rows, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
+        } else if (!together) {
             LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "ffn_norm");
             if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.gate, &b.up}, done)) return st;
             if (mi355x_status st = linear(m, b.gate, h, gate, rows)) return st;
             if (mi355x_status st = linear(m, b.up, h, up, rows)) return st;
             LLM_HIP(swiglu(gate, up, sw, rows, c.hidden, c.hidden, m.stream), "swiglu");
         }
-        if (mi355x_status st = convert_for(m, sw, rows, c.hidden, {&b.down}, done)) return st;
+        if (!converted)
+            if (mi355x_status st = convert_for(m, sw, rows, c.hidden, {&b.down}, done)) return st;
         if (mi355x_status st = onto_x(b.down, sw)) return st;
     }
     m.cache_len = past + s;
@@ -451,7 +471,7 @@ static mi355x_status step_any(Model& m) {
     const int64_t B = c.batch;
     const int64_t qd = (int64_t)c.heads * c.head_dim, kvd = (int64_t)c.kv_heads * c.head_dim;
     float *x = m.x.as<float>(), *h = m.h.as<float>(), *q = m.q.as<float>(), *k = m.k.as<float>(), *v = m.v.as<float>();
-    float *a = m.a.as<float>(), *o = m.o.as<float>(), *gate = m.gate.as<float>(), *up = m.up.as<float>(), *sw = m.s.as<float>();
+    float *a = m.a.as<float>(), *o = m.o.as<float>(), *gate = m.gate.as<float>(), *up = m.up, *sw = m.s.as<float>();
     float *qkv = m.qkv.as<float>(), *gu = m.gu.as<float>();
     const int32_t* pos = m.state.as<int32_t>();
     bool done[kActClasses];
@@ -753,7 +773,8 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
     LLM_HIP(m->x.alloc(rows * c.embed * 4), "hipMalloc"); LLM_HIP(m->h.alloc(rows * c.embed * 4), "hipMalloc");
     LLM_HIP(m->q.alloc(rows * qd * 4), "hipMalloc"); LLM_HIP(m->k.alloc(rows * kvd * 4), "hipMalloc"); LLM_HIP(m->v.alloc(rows * kvd * 4), "hipMalloc");
     LLM_HIP(m->a.alloc(rows * qd * 4), "hipMalloc"); LLM_HIP(m->o.alloc(rows * c.embed * 4), "hipMalloc");
-    LLM_HIP(m->gate.alloc(rows * c.hidden * 4), "hipMalloc"); LLM_HIP(m->up.alloc(rows * c.hidden * 4), "hipMalloc"); LLM_HIP(m->s.alloc(rows * c.hidden * 4), "hipMalloc");
+    LLM_HIP(m->gate.alloc(rows * c.hidden * 2 * 4), "hipMalloc"); LLM_HIP(m->s.alloc(rows * c.hidden * 4), "hipMalloc");
+    m->up = m->gate.as<float>() + rows * c.hidden;
     LLM_HIP(m->hlast.alloc(rows * c.embed * 4), "hipMalloc");
     const int64_t kmax = c.hidden > qd ? (c.hidden > c.embed ? c.hidden : c.embed) : (qd > c.embed ? qd : c.embed);
     for (int cls = 1; cls < kActClasses; cls++) {

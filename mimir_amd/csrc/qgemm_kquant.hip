@@ -125,8 +125,8 @@ struct FetchedX {
 
 // One tile: rows [m0, m0 + 128 MT) of x by rows [n0, n0 + 64) of W.
 template <int DT, int MT, bool OUT_BF16>
-__device__ __forceinline__ void tile(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act, void* __restrict__ yv, int M, int N, int nsb,
-                                     int64_t act_row_bytes, int m0, int n0, uint8_t* smem) {
+__device__ __forceinline__ void tile(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act, void* yv, int M, int N, int nsb,
+                                     const float* resid, int64_t act_row_bytes, int m0, int n0, uint8_t* smem) {
     constexpr int TM = 128 * MT;      // a wavefront's tile: 32 MT rows of x by 32 of W
     constexpr int GM = TM / 2;        // rows of x a group
     constexpr int NX = GM / 16;       // 1 KB loads of x a wavefront and super-block: four rows each
@@ -378,7 +378,8 @@ __device__ __forceinline__ void tile(const uint8_t* __restrict__ W, const uint8_
         for (int i = 0; i < 16; i++) {
             const int m = m0 + g0 + wm * 32 * MT + 32 * mt + 8 * (i >> 2) + 4 * lh + (i & 3);
             if (m < M && n < N) {
-                const float v = DT == kQ4_K ? acc[mt][i] - accm[mt][i] : acc[mt][i];
+                float v = DT == kQ4_K ? acc[mt][i] - accm[mt][i] : acc[mt][i];
+                if (!OUT_BF16 && resid) v = v + resid[(int64_t)m * N + n];
                 if (OUT_BF16) ((uint16_t*)yv)[(int64_t)m * N + n] = f32_to_bf16_bits(v);
                 else ((float*)yv)[(int64_t)m * N + n] = v;
             }
@@ -392,7 +393,7 @@ struct Cut {
 
 template <int DT, bool OUT_BF16>
 __global__ __launch_bounds__(kThreads, 2) void qgemm_kquant_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ act,
-                                                                   void* __restrict__ yv, int M, int N, int nsb, int64_t act_row_bytes, Cut cut) {
+                                                                   void* yv, const float* resid, int M, int N, int nsb, int64_t act_row_bytes, Cut cut) {  // resid may be yv
     extern __shared__ __align__(16) uint8_t smem[];
     // A die's workgroups (every eighth) take a contiguous range of the tiles, those that share rows of W next to each other, so that
     // the second and later ones find W in that die's L2.
@@ -400,13 +401,13 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kquant_kernel(const uint8_t
     int b = blockIdx.x;
     if (b < 8 * tall_die) {
         const int t = (b & 7) * tall_die + (b >> 3);
-        if (t < tall) tile<DT, 2, OUT_BF16>(W, act, yv, M, N, nsb, act_row_bytes, (t % cut.tall_m) * 256, (t / cut.tall_m) * kTN, smem);
+        if (t < tall) tile<DT, 2, OUT_BF16>(W, act, yv, M, N, nsb, resid, act_row_bytes, (t % cut.tall_m) * 256, (t / cut.tall_m) * kTN, smem);
         return;
     }
     b -= 8 * tall_die;
     const int low = cut.short_m * (cut.cols - cut.tall_cols), low_die = (low + 7) >> 3;
     const int t = (b & 7) * low_die + (b >> 3);
-    if (t < low) tile<DT, 1, OUT_BF16>(W, act, yv, M, N, nsb, act_row_bytes, (t % cut.short_m) * 128, (cut.tall_cols + t / cut.short_m) * kTN, smem);
+    if (t < low) tile<DT, 1, OUT_BF16>(W, act, yv, M, N, nsb, resid, act_row_bytes, (t % cut.short_m) * 128, (cut.tall_cols + t / cut.short_m) * kTN, smem);
 }
 
 // A short tile takes this part of a tall one's time: 0.55 on a device half empty (1.5 us a super-block for 2.7), 0.75 on a full one.
@@ -444,7 +445,7 @@ hipError_t launch(const QGemvArgs& a, int nsb, hipStream_t st) {
     plan(a.M, a.N, &cut);
     const int grid = 8 * ((cut.tall_m * cut.tall_cols + 7) / 8 + (cut.short_m * (cut.cols - cut.tall_cols) + 7) / 8);
     hipLaunchKernelGGL((qgemm_kquant_kernel<DT, OUT_BF16>), dim3((unsigned)grid), dim3(kThreads), kLds, st,
-                       (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y, (int)a.M, (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), cut);
+                       (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y, a.resid, (int)a.M, (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), cut);
     return hipGetLastError();
 }
 

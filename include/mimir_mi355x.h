@@ -466,8 +466,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * without the pass through LDS; "q4_0.rows_waves" = 4 or 8 fixes its wavefronts
  * a workgroup; "q4_0.rows_max" = n sends Q4_0 products of fewer than n rows to
  * it (0: up to where the tiled kernel's cost model undercuts its own).
- * "q8_0.mfma" = 1 sends every Q8_0 product of two to eight rows of x that the
- * matrix-core kernel takes to it, 2 none (0: matrices of 64 M weights or more).
+ * "q8_0.mfma" = 1 sends every Q8_0 product of two and more rows of x that the
+ * matrix-core kernel takes to it, 2 none (0: matrices of 32 M weights or more,
+ * and products of more than eight rows with 32768 results or more).
  * "attention.splits" = n fixes the shares of the keys in decode attention; "attention.share" = 128 makes it aim at
  * shares of 128 keys whatever their number (otherwise 64 while there are at most sixteen shares);
  * "attention.handover" = 1 makes its shares travel through a ticket per head instead of as (value, flag) pairs;

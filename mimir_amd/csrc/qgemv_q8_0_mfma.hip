@@ -1,59 +1,74 @@
-// Products of two to eight rows of x with Q8_0 weights on the int8 matrix cores
-// of gfx950, W read once for all the rows: the output projection of a batch's
-// decoding step. The arithmetic is qdotQ8_0Go's (backend/cpu/qmatmul.go:125-139,
-// see qgemv_q8_0.hip): per block four int32 lane sums (value p into lane
-// p/4 mod 4), each times the product of the two scales added to a float32 lane
-// of its own (a multiply, then an add), the lanes added (0+2)+(1+3).
+// Products of two and more rows of x with Q8_0 weights on the int8 matrix cores of gfx950, W read once for eight rows
+// (the output projection of a batch's decoding step) or for 32 (a prompt's rows). What it computes is qdotQ8_0Go's sum
+// (backend/cpu/qmatmul.go:125-139, see qgemv_q8_0.hip) in another order: a block's int32 sum, exact, once times the
+// product of the two scales, where the CPU keeps four sums, one for every fourth group of four values, and adds them
+// at the end.
 //
-// The four lane sums of eight rows of x are the 32 rows of one
-// v_mfma_i32_32x32x32_i8: its first operand's row 8 l + m holds row m's int8
-// block with everything but the values of lane sum l zeroed (of the 16 values a
-// lane holds, that is dword l), its other operand 32 rows of W. A lane ends up
-// with the four lane sums of its row of W for four rows of x. The integer sums
-// are the CPU's; the float32 sums run over the blocks of a row in another order
-// than the CPU's or the one-row kernel's (a wavefront takes every fourth run of
-// eight blocks, the wavefronts' sums are added in order), a few units in the
-// last place.
+// One v_mfma_i32_32x32x32_i8 per block: its first operand has 32 rows of x, or eight rows four times, its other operand
+// 32 rows of W. A lane ends up with its row of W's sums for sixteen rows of x, or for four (and three times again,
+// which it leaves). A workgroup's wavefronts take runs of eight blocks in turn and add their sums up in order.
 //
-// W stays in ggml's layout. As in qgemv_q4_0_rows.hip, a wavefront loads a run
-// of eight blocks of its 32 rows as aligned 16-byte pieces in row order (272
-// bytes a row), passes them through a private LDS slab and reads its 16 int8 of
-// each block back as dwords. x comes converted by q8_convert_act (its one-row
-// form): a lane loads the one dword of it that its operand row keeps.
+// W stays in ggml's layout. As in qgemv_q4_0_rows.hip, a wavefront loads a run of its 32 rows as 16-byte pieces in row
+// order (272 bytes a row), passes them through a private LDS slab and reads its 16 int8 of each block back as dwords.
+// Where K is no multiple of 256 the pieces start on two bytes, which the hardware takes, and the last run reaches back
+// over blocks whose scale is then nought. x comes converted by q8_convert_act: of eight rows a lane loads its row's
+// sixteen bytes of a block, again for the next run as soon as it has used them; of 32, whose rows would be 64 lines a
+// load, x goes through LDS as W does, and a block's MFMA is issued before the sums of the block ahead of it (512 x 4096
+// x 14336 without: 236 us, with: 191).
+//
+// What bounds it. Eight rows: the loads (143 MB of 32768 x 4096: 27 us at the rate of a copy), with four wavefronts
+// too few for them where the matrix is small. 32 rows: a conversion, a product and an fma for each sum and block, 192
+// cycles beside the MFMA's 32 and some 60 of unpacking; 315 TFLOP/s at 512 x 4096 x 14336. Whole calls, us, with W read for eight rows
+// by the vector unit (and by four zeroed copies of x on the matrix cores: 2 and 8 x 32768 x 4096) and now:
+//   2, 8 x 32768 x 4096    38, 42 -> 32, 36        8 x 4096 x 14336     71 -> 29
+//   32 x 32768 x 4096         122 -> 49            64 x 1024 x 4096     34 -> 14
+//   512 x 4096 x 14336       3511 -> 191           128 x 4096 x 4096   229 -> 24
+// Errors against 64 bits, of the result: K = 256: 7.2e-8 -> 6.0e-8, 4096: 9.1e-8 (head of 32768 rows: 1.25e-7) ->
+// 8.5e-8, 14336: 1.02e-7 -> 9.8e-8, 28672: 1.13e-7 -> 1.03e-7, 57344: 1.3e-7 .. 3.9e-7 -> 1.1e-7.
 #include "device_util.h"
 #include "kernels.h"
 
 namespace mimir {
-
-#pragma clang fp contract(off)
 
 namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kWaves = 4;                      // wavefronts of a workgroup, among which the runs of K go round
 constexpr int kRunBlocks = 8;
 constexpr int kRunBytes = 34 * kRunBlocks;     // 272: seventeen pieces a row
 constexpr int kPieces = kRunBytes / 16;
 constexpr int kSlabStride = kRunBytes + 32;    // 304 bytes = 76 dwords: rows fall on eight banks, four to each
 constexpr int kSlabBytes = 32 * kSlabStride;
 constexpr int kLoads = (32 * kPieces + 63) / 64;  // 9: the last one half full
+constexpr int kManyRows = 32;
+constexpr int kRunsTogether = 8;
 
-__global__ __launch_bounds__(64 * kWaves) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, int M, int N,
-                                                                       int nb, int64_t act_row_bytes) {
-    extern __shared__ __align__(16) uint8_t smem[];  // a slab per wavefront; later the wavefronts' sums
+// LDS of a wavefront: the slab, the scales of x of a run [block][row] and, of 32 rows, x's pieces [row][half][block],
+// the block's place turned by the row so that a block's reads fall on all banks.
+template <int XR>
+constexpr int kWaveLds = kSlabBytes + kRunBlocks * XR * 4 + (XR == kManyRows ? XR * kRunBlocks * 32 : 0);
+
+// XR: rows of x a workgroup (8 or 32); WAVES: its wavefronts, among which the runs of K go round
+template <int XR, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, int M,
+                                                                                             int N, int nb, int64_t act_row_bytes) {
+    constexpr bool kMany = XR == kManyRows;
+    constexpr int kSums = XR / 2;  // of a lane
+    extern __shared__ __align__(16) uint8_t smem[];  // per wavefront; later the wavefronts' sums
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // The grid runs over the groups of eight rows of x first: the workgroups that read the same 32 rows of W are handed
+    // The grid runs over the groups of rows of x first: the workgroups that read the same 32 rows of W are handed
     // out together, so the rows come from HBM once and from the memory-side cache for the other groups.
-    const int ngroups = (M + 7) >> 3, group = (int)(blockIdx.x % (unsigned)ngroups);
+    const int ngroups = (M + XR - 1) / XR, group = (int)(blockIdx.x % (unsigned)ngroups);
     const int n0 = (int)(blockIdx.x / (unsigned)ngroups) * 32, n = n0 + l32;
-    const int nruns = nb / kRunBlocks, nbp = nb | 1;
-    uint8_t* slab = smem + wave * kSlabBytes;
-    act += (int64_t)8 * group * act_row_bytes;
-    y += (int64_t)8 * group * N;
-    M = M - 8 * group < 8 ? M - 8 * group : 8;
+    const int nruns = (nb + kRunBlocks - 1) / kRunBlocks, nbp = nb | 1;
+    uint8_t* slab = smem + wave * kWaveLds<XR>;
+    float* dxs = (float*)(slab + kSlabBytes);
+    uint8_t* xslab = slab + kSlabBytes + kRunBlocks * XR * 4;
+    act += (int64_t)XR * group * act_row_bytes;
+    y += (int64_t)XR * group * N;
+    M = M - XR * group < XR ? M - XR * group : XR;
 
     // piece p = 64 i + lane of a run: row p / 17 of the 32, bytes 16 (p % 17).. of its 272
     uint32_t goff[kLoads], loff[kLoads];
@@ -67,60 +82,68 @@ __global__ __launch_bounds__(64 * kWaves) void qgemv_q8_0_mfma_kernel(const uint
         loff[i] = r * kSlabStride + 16 * c;
     }
     const uint8_t* wbase = W + (int64_t)n0 * nb * 34;
-    // this lane's operand row of x: lane sum xl of row xm; it keeps dword xl of the 16 bytes a lane holds
-    const int xl = (l32 >> 3), xm = l32 & 7;
-    const uint8_t* xrow = act + (int64_t)(xm < M ? xm : M - 1) * act_row_bytes;
-    const uint32_t* xq = (const uint32_t*)xrow + (int64_t)lh * nbp * 4 + xl;  // + 4 b: dword xl of half lh of block b
-    const bool x_live = xm < M;
+    // rows past M: the last one again, not stored
+    auto row_of = [&](int r) { return act + (int64_t)(r < M ? r : M - 1) * act_row_bytes; };
+    const i32x4* xq = (const i32x4*)row_of(l32 & (XR - 1)) + (int64_t)lh * nbp;  // + b: half lh of block b of this lane's operand row
+    uint32_t xoff[8];  // of 32 rows: this lane's pieces of a run, of row 4 i + lane / 16 half (lane / 8) % 2 of block lane % 8
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (kMany) xoff[i] = (uint32_t)((row_of(4 * i + (lane >> 4)) - act) + (((lane >> 3) & 1) * nbp + (lane & 7)) * 16);
+    auto x_piece = [](int row, int half, int block) { return ((2 * row + half) * kRunBlocks + (block ^ (row & 7))) * 16; };
+    // The scales of x of a run: of 32 rows a lane brings four blocks' of row l32, of eight one block's of row 4 lh + l32 % 4.
+    const float* own_scales = (const float*)(row_of(kMany ? l32 : 4 * lh + (l32 & 3)) + (int64_t)nbp * 32) + (kMany ? 4 * lh : l32 >> 2);
 
-    struct Run {
-        u32x4 w[kLoads];
-        uint32_t x[kRunBlocks];  // the lane's dword of x per block
-        float dx;                // one scale of x, see below
+    auto start_of = [&](int run) { return kRunBlocks * run < nb - kRunBlocks ? kRunBlocks * run : nb - kRunBlocks; };  // the last run reaches back
+    u32x4 w[kLoads];
+    i32x4 x[8];  // eight rows: the operands of a run's blocks; 32: this lane's pieces of it
+    float own[kMany ? 4 : 1];
+    auto fetch = [&](int at) {
+        const uint8_t* p = wbase + (int64_t)at * 34;
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) w[i] = load_u32x4_unaligned(p + goff[i]);
+        if (kMany) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] = *(const i32x4*)(act + xoff[i] + 16 * at);
+        }
+        __builtin_memcpy(own, own_scales + at, sizeof(own));
     };
-    // The scales of x a lane needs are those of rows 4 lh .. 4 lh + 3 for every block of the run: 32 floats.
-    // They are loaded once a run by the lanes (block l32 >> 2 of the run, row 4 lh + (l32 & 3)) and handed
-    // round through LDS behind the slab.
-    float* dxs = (float*)(smem + kWaves * kSlabBytes) + wave * 64;  // [half][block of the run][4 rows]
-    auto fetch = [&](Run& f, int run) {
-        const uint8_t* p = wbase + (int64_t)run * kRunBytes;
-#pragma unroll
-        for (int i = 0; i < kLoads; i++) f.w[i] = *(const u32x4*)(p + goff[i]);
-#pragma unroll
-        for (int b = 0; b < kRunBlocks; b++) f.x[b] = xq[(int64_t)(run * kRunBlocks + b) * 4];
-        const int drow = 4 * lh + (l32 & 3);
-        f.dx = ((const float*)(act + (int64_t)(drow < M ? drow : M - 1) * act_row_bytes + (int64_t)nbp * 32))[run * kRunBlocks + (l32 >> 2)];
-    };
 
-    float acc[4][4];  // [lane sum][row of x 4 lh + j]
+    // A run's sums by themselves, those of eight runs, and the eights': short chains, whose errors stay below those of
+    // the one-row kernel's 64 lanes with four sums each (one chain for all of a wavefront's blocks: 2.0e-7 at K = 14336).
+    float acc[kSums], total[kSums];
 #pragma unroll
-    for (int l = 0; l < 4; l++)
+    for (int i = 0; i < kSums; i++) acc[i] = total[i] = 0.f;
+    if (wave < nruns) {
+        fetch(start_of(wave));
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[l][j] = 0.f;
-
-    Run cur, nxt;
-    if (wave < nruns) fetch(cur, wave);
+        for (int b = 0; b < kRunBlocks; b++)
+            if (!kMany) x[b] = xq[start_of(wave) + b];
+    }
     const uint8_t* mine = slab + l32 * kSlabStride + 16 * lh;  // the lane's 16 int8 of block b: bytes 34 b + 2 + 16 lh
-    const uint32_t keep0 = xl == 0 && x_live ? ~0u : 0u, keep1 = xl == 1 && x_live ? ~0u : 0u, keep2 = xl == 2 && x_live ? ~0u : 0u,
-                   keep3 = xl == 3 && x_live ? ~0u : 0u;
-    for (int run = wave; run < nruns; run += kWaves) {
-        const int nrun = run + kWaves < nruns ? run + kWaves : run;
-        fetch(nxt, nrun);
-        // slab and scales are this wavefront's alone, and a wavefront's LDS operations complete in order
+    for (int run = wave; run < nruns; run += WAVES) {
+        const int nrun = run + WAVES < nruns ? run + WAVES : run, next = start_of(nrun), done = kRunBlocks * run - start_of(run);
+        // slabs and scales are this wavefront's alone, and a wavefront's LDS operations complete in order
 #pragma unroll
-        for (int i = 0; i < kLoads - 1; i++) *(u32x4*)(slab + loff[i]) = cur.w[i];
-        if (lane < 32 * kPieces - 64 * (kLoads - 1)) *(u32x4*)(slab + loff[kLoads - 1]) = cur.w[kLoads - 1];
-        dxs[32 * lh + l32] = cur.dx;  // [half][block l32 >> 2][row l32 & 3]
+        for (int i = 0; i < kLoads - 1; i++) *(u32x4*)(slab + loff[i]) = w[i];
+        if (lane < 32 * kPieces - 64 * (kLoads - 1)) *(u32x4*)(slab + loff[kLoads - 1]) = w[kLoads - 1];
+        if (kMany) {
 #pragma unroll
-        for (int b = 0; b < kRunBlocks; b++) {
+            for (int i = 0; i < 4; i++) dxs[(4 * lh + i) * XR + l32] = own[i % (kMany ? 4 : 1)];
+#pragma unroll
+            for (int i = 0; i < 8; i++) *(i32x4*)(xslab + x_piece(4 * i + (lane >> 4), (lane >> 3) & 1, lane & 7)) = x[i];
+        } else {
+            dxs[(l32 >> 2) * XR + 4 * lh + (l32 & 3)] = own[0];
+        }
+        fetch(next);
+        // The block's product of this lane's row of W (scale into dw).
+        auto multiply = [&](int b, float* dw) {
             // bytes 34 b + 2 ..: on a dword for odd b, two bytes into one for even b
             i32x4 wop;
-            float dw;
             if (b & 1) {
                 const uint8_t* p = mine + 34 * b + 2;
 #pragma unroll
                 for (int i = 0; i < 4; i++) wop[i] = (int)*(const uint32_t*)(p + 4 * i);
-                dw = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(slab + l32 * kSlabStride + 34 * b - 2) >> 16));
+                *dw = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(slab + l32 * kSlabStride + 34 * b - 2) >> 16));
             } else {
                 const uint8_t* p = mine + 34 * b;
                 uint32_t r[5];
@@ -128,81 +151,109 @@ __global__ __launch_bounds__(64 * kWaves) void qgemv_q8_0_mfma_kernel(const uint
                 for (int i = 0; i < 5; i++) r[i] = *(const uint32_t*)(p + 4 * i);
 #pragma unroll
                 for (int i = 0; i < 4; i++) wop[i] = (int)__builtin_amdgcn_alignbit(r[i + 1], r[i], 16);
-                dw = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(slab + l32 * kSlabStride + 34 * b) & 0xffffu));
+                *dw = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(slab + l32 * kSlabStride + 34 * b) & 0xffffu));
             }
-            const uint32_t xv = cur.x[b];
-            const i32x4 xop = {(int)(xv & keep0), (int)(xv & keep1), (int)(xv & keep2), (int)(xv & keep3)};
+            *dw = b < done ? 0.f : *dw;  // blocks that the run before has taken
+            const i32x4 xop = kMany ? *(const i32x4*)(xslab + x_piece(l32, lh, b)) : x[b];
             i32x16 zero;
 #pragma unroll
             for (int i = 0; i < 16; i++) zero[i] = 0;
-            const i32x16 c = __builtin_amdgcn_mfma_i32_32x32x32_i8(xop, wop, zero, 0, 0, 0);
-            const f32x4 dx = *(const f32x4*)(dxs + 32 * lh + 4 * b);
+            return __builtin_amdgcn_mfma_i32_32x32x32_i8(xop, wop, zero, 0, 0, 0);
+        };
+        float part[kSums];
+        float dw;
+        i32x16 c = multiply(0, &dw);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float dd = dw * dx[j];
+        for (int b = 0; b < kRunBlocks; b++) {
+            float dw_next = 0.f;
+            i32x16 c_next = c;
+            if (b + 1 < kRunBlocks) c_next = multiply(b + 1, &dw_next);  // under the sums of block b
+            if (kMany) __builtin_amdgcn_sched_barrier(0);
+            if (!kMany) x[b] = xq[next + b];
+            // register 4 g + j: row 8 g + 4 lh + j of x
 #pragma unroll
-                for (int l = 0; l < 4; l++) {
-                    const float t = dd * (float)c[4 * l + j];
-                    acc[l][j] = acc[l][j] + t;
-                }
+            for (int g = 0; g < kSums / 4; g++) {
+                const f32x4 dx = *(const f32x4*)(dxs + b * XR + 8 * g + 4 * lh);
+#pragma unroll
+                for (int j = 0; j < 4; j++) part[4 * g + j] = b == 0 ? dw * dx[j] * (float)c[4 * g + j] : fmaf(dw * dx[j], (float)c[4 * g + j], part[4 * g + j]);
+            }
+            c = c_next;
+            dw = dw_next;
+        }
+#pragma unroll
+        for (int i = 0; i < kSums; i++) acc[i] += part[i];
+        if ((run / WAVES) % kRunsTogether == kRunsTogether - 1) {
+#pragma unroll
+            for (int i = 0; i < kSums; i++) {
+                total[i] += acc[i];
+                acc[i] = 0.f;
             }
         }
-        cur = nxt;
     }
+#pragma unroll
+    for (int i = 0; i < kSums; i++) acc[i] += total[i];
 
     __syncthreads();  // every wavefront is done with its slab
-    f32x4* red = (f32x4*)smem;  // [wave][lane sum][lane]
+    float* red = (float*)smem;  // [wave][sum][lane]
 #pragma unroll
-    for (int l = 0; l < 4; l++) red[(wave * 4 + l) * 64 + lane] = f32x4{acc[l][0], acc[l][1], acc[l][2], acc[l][3]};
+    for (int i = 0; i < kSums; i++) red[(wave * kSums + i) * 64 + lane] = acc[i];
     __syncthreads();
-    if (wave != 0) return;
-    f32x4 a[4];
+    // the wavefronts share the sums
+    for (int s = wave; s < kSums; s += WAVES) {
+        float v = red[s * 64 + lane];
 #pragma unroll
-    for (int l = 0; l < 4; l++) {
-        a[l] = red[l * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < kWaves; w++) {
-            const f32x4 t = red[(w * 4 + l) * 64 + lane];
-#pragma unroll
-            for (int j = 0; j < 4; j++) a[l][j] = a[l][j] + t[j];
-        }
-    }
-    if (n < N) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int m = 4 * lh + j;
-            if (m < M) {
-                const float s02 = a[0][j] + a[2][j], s13 = a[1][j] + a[3][j];
-                y[(int64_t)m * N + n] = s02 + s13;
-            }
-        }
+        for (int o = 1; o < WAVES; o++) v = v + red[(o * kSums + s) * 64 + lane];
+        const int m = 8 * (s >> 2) + 4 * lh + (s & 3);
+        if (n < N && m < M) y[(int64_t)m * N + n] = v;
     }
 }
 
+constexpr int kFewRows = 8;
+
 }  // namespace
 
-// Rows of x converted beforehand (q8_convert_act), taken eight at a time; whole runs of eight blocks; W 16-byte aligned.
+// Rows of x converted beforehand (q8_convert_act), eight blocks and more a row.
 bool qgemv_q8_0_mfma_ok(const QGemvArgs& a) {
     const int64_t nb = a.K / 32;
-    return a.M >= 2 && a.M <= 8 * 65535 && a.act && !a.resid && a.K % 256 == 0 && nb > 0 && ((uintptr_t)a.W & 15) == 0 && 32 * nb * 34 < ((int64_t)1 << 32) &&
-           a.N > 0 && a.N <= (1ll << 30);
+    return a.M >= 2 && a.M <= 8 * 65535 && a.act && ((uintptr_t)a.act & 15) == 0 && !a.resid && nb >= kRunBlocks && ((uintptr_t)a.W & 1) == 0 &&
+           32 * nb * 34 < ((int64_t)1 << 32) && 32 * (int64_t)q8_act_bytes(a.K) < ((int64_t)1 << 31) && a.N > 0 && a.N <= (1ll << 30);
 }
 
 static std::atomic<int> g_q8_mfma{0};  // measurement aid: 1 = wherever the kernel takes the shape, 2 = never
 void set_q8_mfma(int v) { g_q8_mfma = v; }
 
+// Up to eight rows: matrices of 32 M weights and more that give the chip 128 workgroups, for two and three rows 192
+// (us by the vector unit, here; 8 rows: 8192 x 4096 34, 13; 4 rows: 4096 x 8192 19, 17, 2048 x 16384 18, 28; 2 rows:
+// 6144 x 8192 20, 18, 4096 x 14336 24, 26). More rows: from 32768 results (9 x 4096 x 4096 31, 12; 32 x 1024 x 14336
+// 42, 28; 128 x 256 x 1024 18, 8; against 9 x 1024 x 4096 11.3, 11.8; 64 x 64 x 14336 20, 28).
 bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
     if (g_q8_mfma == 2 || !qgemv_q8_0_mfma_ok(a)) return false;
-    return g_q8_mfma == 1 || a.N * a.K >= ((int64_t)64 << 20);
+    if (g_q8_mfma == 1) return true;
+    if (a.M > kFewRows) return a.M * a.N >= 32768;
+    return a.N * a.K >= ((int64_t)32 << 20) && a.N >= (a.M >= 4 ? 4096 : 6144);
 }
 
-hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st) {
-    const size_t lds = (size_t)kWaves * kSlabBytes + kWaves * 64 * 4;
-    const int64_t wgs = ((a.N + 31) / 32) * ((a.M + 7) / 8);
-    if (wgs > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(qgemv_q8_0_mfma_kernel, dim3((unsigned)wgs), dim3(64 * kWaves), lds, st, (const uint8_t*)a.W,
-                       (const uint8_t*)a.act, a.y, (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K));
+template <int XR, int WAVES>
+static hipError_t launch(const QGemvArgs& a, int64_t wgs, hipStream_t st) {
+    constexpr int kLds = WAVES * kWaveLds<XR>;
+    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
+    if (kLds > 64 * 1024 && !raised) {
+        if (hipError_t e = hipFuncSetAttribute((const void*)qgemv_q8_0_mfma_kernel<XR, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
+        raised = true;
+    }
+    hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y,
+                       (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K));
     return hipGetLastError();
+}
+
+// Eight wavefronts a workgroup where all workgroups then are on the chip at once, two a compute unit of eight rows, one of 32
+// (us with four, with eight: 2 x 14336 x 4064 21, 20; 32 x 4096 x 14336 65, 45; past it, 64 x 8192 x 4096 26, 30), else four.
+hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st) {
+    const int rows = a.M > kFewRows ? kManyRows : 8;
+    const int64_t wgs = ((a.N + 31) / 32) * ((a.M + rows - 1) / rows);
+    if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+    if (rows == 8) return wgs <= 512 ? launch<8, 8>(a, wgs, st) : launch<8, 4>(a, wgs, st);
+    return wgs <= 256 ? launch<kManyRows, 8>(a, wgs, st) : launch<kManyRows, 4>(a, wgs, st);
 }
 
 }  // namespace mimir

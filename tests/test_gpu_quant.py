@@ -612,6 +612,33 @@ def test_q8_0_rows_on_the_matrix_cores(m, n, k):
     assert np.all(np.abs(got - rows) <= 2e-6 * mag + 1e-30)
 
 
+@pytest.mark.parametrize("m,n,k,offset", [(9, 4097, 256, 0), (32, 1024, 288, 2), (33, 1000, 4064, 0), (64, 513, 2304, 4), (65, 8200, 480, 2), (520, 70, 992, 0),
+                                          (3, 8193, 4128, 2), (2, 16500, 2080, 0)])
+def test_q8_0_products_of_any_rows_on_the_matrix_cores(m, n, k, offset):
+    """32 rows of x and 32 of W a workgroup, eight blocks a run: remainders of each, a W on two bytes, four and eight
+    wavefronts, on the route that the size selects. The integers are the CPU's; a result's float32 sums pass through
+    fewer than nb + 40 roundings of 2^-24, here and there together, each of no more than sum |w||x|. All rows against
+    the exact product within the rounding of x to int8 (half a step of a block's largest / 127). A row that holds a
+    NaN is NaN, the others are not."""
+    rng = np.random.default_rng(5 * m + n + k)
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[0, -32:] = 0
+    x[m - 1, k - 1] = np.nan
+    buf, ptr = gpu.dev_bytes_at(raw, offset)
+    gpu.say(f"q8_0 matrix-core product M={m} N={n} K={k} offset={offset}")
+    got = gpu.qgemv(O.Q8_0, ptr, gpu.dev(x), n, k)
+    assert np.isnan(got[m - 1]).all()
+    got, x = got[:-1], x[:-1]
+    w = np.abs(O.dequantize(O.Q8_0, raw).reshape(n, k).astype(np.float64))
+    sums = (k // 32 + 40) * 2.0**-24 * 1.01 * (np.abs(x).astype(np.float64) @ w.T)
+    some = sorted({0, m // 2, m - 2} - {m - 1})  # the oracle is slow on all of them
+    assert np.all(np.abs(got[some] - O.qmatmul(O.Q8_0, raw, x[some], n, k)) <= sums[some])
+    steps = np.abs(x).reshape(m - 1, -1, 32).max(2).astype(np.float64) / 254 * 1.01
+    exact = x.astype(np.float64) @ O.dequantize(O.Q8_0, raw).reshape(n, k).astype(np.float64).T
+    assert np.all(np.abs(got - exact) <= steps @ w.reshape(n, -1, 32).sum(2).T + sums)
+
+
 # ---- Q4_K / Q6_K -------------------------------------------------------------
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])

@@ -476,6 +476,8 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * release-acquire one at device scope, 2 also stores and loads the shares plainly (both to be measured; 1 restores).
  * "q4_0.fx_rows" = n sends Q4_0 products of at least n rows of float32 x to the
  * int8 matrix cores whatever the shape (0: the built-in cost model);
+ * "q4_0.strips" = 1 sends every Q4_0 product of mi355x_qgemm_bf16, and of mi355x_qgemv by rows that the
+ * fixed-point forms do not take, to the kernel for some rows without a workspace where it takes the shape, 2 none (0: by shape);
  * "q4_0.fx_pairs" = 0 keeps those products off the binary16 matrix cores, 2
  * sends them all there as digits with the int8 form's bits (the decoder's too,
  * where their workspace was allocated), 3 as pairs of binary16 (1: pairs, by the

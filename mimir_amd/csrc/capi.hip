@@ -205,6 +205,10 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
         return MI355X_OK;
     }
     void* ws;
+    if (dtype == MI355X_Q4_0 && g_tune_gemm != 1 && g_tune_gemm_f16 == 0 && !mimir::q4_0_blocks_chosen() && mimir::qgemm_q4_0_strips_pays(W, X, true, M, N, K, x_row_stride)) {
+        HIP_TRY(mimir::qgemm_q4_0_strips(W, X, true, Y, !f32, M, N, K, x_row_stride, st), "launch qgemm_q4_0_strips");
+        return MI355X_OK;
+    }
     if (dtype == MI355X_Q4_0 && g_tune_gemm != 1 && mimir::qgemm_q4_0_ok(W, X, M, N, K, x_row_stride)) {
         if (g_tune_gemm_f16 == 0 && mimir::qgemm_q4_0_blocks_pays(M, N, K)) {
             // the exact form of a large product: W's integers once as a bfloat16 panel, then one MFMA a weight
@@ -338,6 +342,11 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             HIP_TRY(mimir::q4_0_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q4_0_convert_act");
             a.act = act;
             HIP_TRY(mimir::qgemv_q4_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q4_0_act");
+            return MI355X_OK;
+        }
+        // rows that the fixed-point forms do not take (an odd number of blocks, W on two bytes)
+        if (g_tune_q4[4] != 1 && mimir::qgemm_q4_0_strips_pays(W, x, false, M, N, K, x_row_stride)) {
+            HIP_TRY(mimir::qgemm_q4_0_strips(W, x, false, y, false, M, N, K, x_row_stride, (hipStream_t)stream), "launch qgemm_q4_0_strips");
             return MI355X_OK;
         }
         HIP_TRY(mimir::qgemv_q4_0(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q4_0");
@@ -690,6 +699,10 @@ mi355x_status mi355x_tune(const char* key, int value) {
     }
     if (key && strcmp(key, "qgemm.f16") == 0) {
         g_tune_gemm_f16 = value == 1 || value == 2 ? value : 0;
+        return MI355X_OK;
+    }
+    if (key && strcmp(key, "q4_0.strips") == 0) {
+        mimir::set_q4_0_strips(value);
         return MI355X_OK;
     }
     if (key && strcmp(key, "q4_0.fx_pairs") == 0) {  // 0: every product of many rows on the int8 form; 2: on the binary16 form; 1: by cost

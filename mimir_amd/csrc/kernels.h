@@ -335,6 +335,14 @@ size_t qgemm_q4_0_in_place_sums_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t qgemm_q4_0_in_place(const void* W, const void* act, float* y, int64_t M, int64_t N, int64_t K, void* ws, size_t ws_bytes, hipStream_t st);
 void set_q4_0_fx16(int v);  // measurement aid: 0 keeps every product on the int8 form
 
+// Two and more rows of x, float32 or bfloat16, by Q4_0 weights, W and x read where they lie, no workspace
+// (qgemm_q4_0_strips.hip): K a multiple of 32, 256 and more, W 2-byte and x's rows 16-byte aligned; y float32, or bfloat16
+// of a bfloat16 x. _pays: faster than the kernels else taken ("q4_0.strips": 1 always, 2 never).
+bool qgemm_q4_0_strips_ok(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride);
+bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride);
+void set_q4_0_strips(int v);
+hipError_t qgemm_q4_0_strips(const void* W, const void* x, bool bf16, void* y, bool out_bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st);
+
 // Prompt-sized Q4_0 product on the matrix cores (qgemm_q4_0.hip): X [M, K]
 // bfloat16, Y [M, N] bfloat16 or float32. Exact up to the order of the float32 sums when half_ws is null; with
 // half_ws (qgemm_q4_0_half_ws_bytes(M, N, K, panel) bytes of device memory, 256-byte aligned) the weights are rounded to
@@ -352,6 +360,7 @@ bool qgemm_q4_0_blocks_pays(int64_t M, int64_t N, int64_t K);  // against the ti
 hipError_t qgemm_q4_0_blocks(const void* W, const void* X, int64_t x_row_stride, void* Y, int64_t M, int64_t N, int64_t K, bool out_f32, void* ws,
                              hipStream_t st);
 void set_q4_0_blocks(int v);  // measurement aid: 0 keeps every product on the tile kernel, 2 takes this route whatever the shape
+bool q4_0_blocks_chosen();  // by "qgemm.blocks", not by shape
 // The panel route (qgemm_f16_panel.hip): X [M, K] bfloat16 goes to X16 [M, K] binary16 with row_scale[m] to multiply row
 // m's results by (both written here), W Q4_0 to `panel` (qgemm_f16_panel_bytes(N, K) bytes of device memory, 256-byte aligned).
 size_t qgemm_f16_panel_bytes(int64_t N, int64_t K);

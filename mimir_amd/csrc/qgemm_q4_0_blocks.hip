@@ -301,6 +301,7 @@ std::atomic<int> g_blocks{1};  // measurement aid: 0 keeps every product on the 
 }  // namespace
 
 void set_q4_0_blocks(int v) { g_blocks = v; }
+bool q4_0_blocks_chosen() { return g_blocks != 1; }
 
 // W's integers and X in granules, W's scales.
 static size_t granules_bytes(int64_t rows, int64_t K) { return (size_t)((rows + 31) / 32) * (size_t)(K / 32) * kGranule * 2; }

@@ -1,0 +1,363 @@
+// Products of some rows of x, bfloat16 or float32, by Q4_0 weights on the bfloat16 matrix cores of gfx950, with x and W read
+// where they lie and no workspace: what mi355x_qgemm_bf16 takes up to some hundreds of rows, and mi355x_qgemv for rows of W
+// that the fixed-point forms do not take (an odd number of blocks, or W on two bytes).
+//
+// A workgroup has 32 rows of x and one or two strips of 32 rows of W; its eight wavefronts take runs of eight blocks of K in
+// turn and add their sums up in order. A chain of steps over all of K, in which one workgroup a tile of the result
+// takes 0.9 us for every 64 of K however few the rows, is what bounded these shapes before. W passes through a private slab of LDS as in
+// qgemv_q8_0_mfma.hip (144 bytes a row, rows end to end); x, of which an MFMA's operand is sixteen consecutive bytes of each
+// of 32 rows, comes straight from memory some blocks ahead. Two v_mfma_f32_32x32x16_bf16 make a block: their operands are
+// n - 8 of the lower and of the upper nibbles, exact in bfloat16 (as sixteenths, the scale times sixteen), and one FMA a result adds the
+// block's sum by its scale. A float32 x is the sum of three bfloat16, exactly, and a block six MFMAs.
+//
+// What bounds it: 30 instructions of unpacking, 16 FMAs and 64 cycles of MFMA a block and strip, with float32 another 150
+// instructions of splitting x (for two strips where they fill the chip) and 192 cycles. From 1024 workgroups on the tile
+// kernels, which unpack W once for 128 rows, are the faster. Whole calls, us, before and now:
+//   bfloat16   16 x 4096 x 4096    61 -> 10      float32   16 x 4096 x 4064      31 -> 20
+//              64 x 14336 x 4096   63 -> 46               128 x 4096 x 4064     215 -> 30
+//             128 x 4096 x 14336  200 -> 75               512 x 14336 x 4064   3860 -> 370
+// Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 8.3e-8 at K = 4096, 1.05e-6 -> 9.4e-8 at 14336; float32
+// 1.96e-7 -> 1.04e-7 at K = 4064, 2.1e-7 -> 1.83e-7 at 28704.
+#include <atomic>
+
+#include "device_util.h"
+#include "kernels.h"
+
+namespace mimir {
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kWaves = 8;
+constexpr int kRunBlocks = 8;
+constexpr int kRunBytes = 18 * kRunBlocks;         // 144: nine pieces of sixteen bytes a row
+constexpr int kPieces = kRunBytes / 16;
+constexpr int kStripBytes = 32 * kRunBytes;        // a strip's run in LDS, rows end to end: their starts fall on sixteen banks
+constexpr int kLoads = (32 * kPieces + 63) / 64;   // 5: the last one half full
+
+template <typename X>
+constexpr int kParts = sizeof(X) == 4 ? 3 : 1;
+
+__device__ __forceinline__ uint32_t upper_halves(uint32_t odd, uint32_t even) { return __builtin_amdgcn_perm(odd, even, 0x07060302u); }
+
+// Eight x of a row as the MFMA's operands, the least part first. A float32 is three bfloat16 that add up to it: its upper
+// sixteen bits (eight of its 24 significant ones), those of what is left, and of what is left then. An infinity's rest is
+// nought, a NaN's NaN.
+__device__ __forceinline__ void split(const u32x4* v, bf16x8* parts, __bf16) { __builtin_memcpy(parts, v, 16); }
+__device__ __forceinline__ void split(const u32x4* v, bf16x8* parts, float) {
+    uint32_t p[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t b[3][2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const uint32_t u = v[i >> 1][2 * (i & 1) + j];
+            const float x = __uint_as_float(u), upper = __uint_as_float(u & 0xffff0000u);
+            const float rest = __builtin_fabsf(x) == __builtin_inff() ? 0.f : x - upper;
+            const float low = rest - __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
+            b[2][j] = u;
+            b[1][j] = __float_as_uint(rest);
+            b[0][j] = __float_as_uint(low);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) p[q][i] = upper_halves(b[q][1], b[q][0]);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) __builtin_memcpy(&parts[q], p[q], 16);
+}
+
+// The matrix cores take subnormal operands for nought, which the lesser parts of an x below 2^-103 are. The least of sixteen x a lane
+// other than nought goes into `least`; where one is below 2^-100, the workgroup goes over its share again and takes each
+// block's rows whose largest x is below 2^-60 times 2^64 (in the others what is lost is 2^-66 of the largest).
+constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1;
+__device__ __forceinline__ void note_least(const u32x4 (*v)[2], uint32_t* least) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) *least = min(*least, (v[i >> 3][(i >> 2) & 1][i & 3] << 1) - 1);  // nought: the largest number
+}
+__device__ __forceinline__ float enlarge(u32x4 (*v)[2]) {  // returns what takes the row's sum back
+    float most = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float a = __builtin_fabsf(__uint_as_float(v[i >> 3][(i >> 2) & 1][i & 3]));
+        most = a > most || a != a ? a : most;
+    }
+    const float other = __shfl_xor(most, 32);
+    const float by = most < 0x1p-60f && other < 0x1p-60f ? 0x1p64f : 1.f;  // this lane's half of the row and the other lane's
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i >> 3][(i >> 2) & 1][i & 3] = __float_as_uint(__uint_as_float(v[i >> 3][(i >> 2) & 1][i & 3]) * by);
+    return 1.f / by;
+}
+
+// SW: strips of 32 rows of W a workgroup. RAGGED: the blocks of a row are no multiple of eight.
+template <typename X, int SW, bool RAGGED, typename Y>
+__global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const uint8_t* __restrict__ W, const X* __restrict__ x, Y* __restrict__ y, int M, int N,
+                                                                            int nb, int64_t x_row_stride) {
+    constexpr int kP = kParts<X>;
+    constexpr int kWords = sizeof(X) == 4 ? 2 : 1;  // sixteen-byte loads of eight x
+    constexpr int kAhead = sizeof(X) == 2 ? 8 : SW == 1 ? 4 : 2;  // blocks of x in registers
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ngroups = (M + 31) / 32, group = (int)(blockIdx.x % (unsigned)ngroups);
+    const int n0 = (int)(blockIdx.x / (unsigned)ngroups) * 32 * SW;
+    const int nruns = (nb + kRunBlocks - 1) / kRunBlocks;
+    uint8_t* slab = smem + wave * SW * kStripBytes;  // this wavefront's alone
+    x += (int64_t)32 * group * x_row_stride;
+    y += (int64_t)32 * group * N;
+    M = M - 32 * group < 32 ? M - 32 * group : 32;
+
+    // piece p = 64 i + lane of a strip's run: row p / 9 of the 32, bytes 16 (p % 9).. of its 144
+    uint32_t goff[SW][kLoads];
+#pragma unroll
+    for (int s = 0; s < SW; s++) {
+#pragma unroll
+        for (int i = 0; i < kLoads; i++) {
+            int p = 64 * i + lane;
+            p = p < 32 * kPieces ? p : 32 * kPieces - 1;  // the last load's upper lanes repeat the last piece
+            const int r = p / kPieces, c = p - kPieces * r;
+            const int row = n0 + 32 * s + r < N ? n0 + 32 * s + r : N - 1;
+            goff[s][i] = (uint32_t)(row - n0) * (uint32_t)(nb * 18) + 16 * c;  // 64 rows of W within 4 GB (checked by the host)
+        }
+    }
+    const uint8_t* wbase = W + (int64_t)n0 * nb * 18;
+    const X* xrow = x + (int64_t)(l32 < M ? l32 : M - 1) * x_row_stride + 8 * lh;  // rows past M: the last one again, not stored
+
+    auto start_of = [&](int run) { return kRunBlocks * run < nb - kRunBlocks ? kRunBlocks * run : nb - kRunBlocks; };  // the last run reaches back
+    u32x4 w[SW][kLoads];
+    u32x4 xs[kAhead][2][kWords];
+    auto fetch_w = [&](int at) {
+        const uint8_t* p = wbase + (int64_t)at * 18;
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) w[s][i] = load_u32x4_unaligned(p + goff[s][i]);
+        }
+    };
+    auto fetch_x = [&](int slot, int block) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int i = 0; i < kWords; i++) xs[slot][h][i] = *((const u32x4*)(xrow + 32 * (int64_t)block + 16 * h) + i);
+        }
+    };
+
+    // A block's product of a strip and sixteen times its scale. A block is a scale and sixteen bytes, of which this lane takes eight: their
+    // lower nibbles are weights 8 lh .., the upper ones 16 + 8 lh .. It starts on a dword for even b, two bytes into one for odd b.
+    auto product = [&](int s, int b, const bf16x8 (&xp)[2][kP], float* scale) {
+        const uint8_t* block = slab + s * kStripBytes + l32 * kRunBytes + 18 * b;
+        uint32_t q[2];
+        float d;
+        if (b & 1) {
+            const uint32_t* p = (const uint32_t*)(block + 2 + 8 * lh);
+            q[0] = p[0];
+            q[1] = p[1];
+            d = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(block - 2) >> 16));
+        } else {
+            const uint32_t* p = (const uint32_t*)(block + 8 * lh);
+            const uint32_t r0 = p[0], r1 = p[1], r2 = p[2];
+            q[0] = __builtin_amdgcn_alignbit(r1, r0, 16);
+            q[1] = __builtin_amdgcn_alignbit(r2, r1, 16);
+            d = f16_bits_to_f32((uint16_t)(*(const uint32_t*)block & 0xffffu));
+        }
+        *scale = d * 16.f;
+        f32x16 c;
+#pragma unroll
+        for (int i = 0; i < 16; i++) c[i] = 0.f;
+        bf16x8 wp[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            uint32_t packed[4];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const uint32_t t = (h ? q[k] >> 4 : q[k]) ^ 0x08080808u;  // a nibble n as the four-bit integer n - 8, converted as sixteenths
+                float f[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) f[i] = __builtin_amdgcn_cvt_off_f32_i4((int)((t >> (8 * i)) & 0xffu));
+                packed[2 * k] = upper_halves(__float_as_uint(f[1]), __float_as_uint(f[0]));
+                packed[2 * k + 1] = upper_halves(__float_as_uint(f[3]), __float_as_uint(f[2]));
+            }
+            __builtin_memcpy(&wp[h], packed, 16);
+        }
+#pragma unroll
+        for (int p = 0; p < kP; p++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xp[h][p], wp[h], c, 0, 0, 0);
+        }
+        return c;  // register 4 g + j: row 8 g + 4 lh + j of x
+    };
+    // a wavefront's LDS operations complete in order
+    auto store_w = [&]() {
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) {
+                if (64 * i + lane < 32 * kPieces) *(u32x4*)(slab + s * kStripBytes + 16 * (64 * i + lane)) = w[s][i];
+            }
+        }
+    };
+
+    // A run's sums by themselves, then the runs': short chains, small errors
+    float acc[SW][16];
+#pragma unroll
+    for (int s = 0; s < SW; s++) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
+    }
+    uint32_t least = 0xffffffffu;
+    if (wave < nruns) {
+        fetch_w(start_of(wave));
+#pragma unroll
+        for (int b = 0; b < kAhead; b++) fetch_x(b, start_of(wave) + b);
+    }
+    for (int run = wave; run < nruns; run += kWaves) {
+        const int at = start_of(run), next = start_of(run + kWaves < nruns ? run + kWaves : run), done = kRunBlocks * run - at;
+        store_w();
+        fetch_w(next);
+        float part[SW][16];
+#pragma unroll
+        for (int b = 0; b < kRunBlocks; b++) {
+            bf16x8 xp[2][kP];
+            u32x4 v[2][kWords];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+#pragma unroll
+                for (int i = 0; i < kWords; i++) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[h][i][j] = RAGGED && b < done ? 0u : xs[b % kAhead][h][i][j];  // blocks that the run before has taken
+                }
+                split(v[h], xp[h], X());
+            }
+            if constexpr (kP == 3) note_least(v, &least);
+            fetch_x(b % kAhead, b + kAhead < kRunBlocks ? at + b + kAhead : next + b + kAhead - kRunBlocks);
+#pragma unroll
+            for (int s = 0; s < SW; s++) {
+                float d;
+                const f32x16 c = product(s, b, xp, &d);
+                if (RAGGED) d = b < done ? 0.f : d;
+#pragma unroll
+                for (int i = 0; i < 16; i++) part[s][i] = b == 0 ? d * c[i] : fmaf(d, c[i], part[s][i]);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[s][i] += part[s][i];
+        }
+    }
+    if constexpr (kP == 3) {
+        if (__syncthreads_or(least < kTiny)) {  // seldom; block after block
+#pragma unroll
+            for (int s = 0; s < SW; s++) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
+            }
+#pragma unroll 1
+            for (int run = wave; run < nruns; run += kWaves) {
+                const int at = start_of(run);
+                fetch_w(at);
+                store_w();
+#pragma unroll 1
+                for (int b = kRunBlocks * run - at; b < kRunBlocks; b++) {
+                    fetch_x(0, at + b);
+                    const float back = enlarge(xs[0]);
+                    bf16x8 xp[2][kP];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) split(xs[0][h], xp[h], X());
+#pragma unroll
+                    for (int s = 0; s < SW; s++) {
+                        float d;
+                        const f32x16 c = product(s, b, xp, &d);
+#pragma unroll
+                        for (int i = 0; i < 16; i++) acc[s][i] = fmaf(d, c[i] * __shfl(back, 8 * (i >> 2) + 4 * lh + (i & 3)), acc[s][i]);
+                    }
+                }
+            }
+        }
+    }
+
+    __syncthreads();  // every wavefront is done with its slab
+    float* red = (float*)smem;  // [wave][16][lane], a strip at a time
+#pragma unroll
+    for (int s = 0; s < SW; s++) {
+        if (s > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; i++) red[(wave * 16 + i) * 64 + lane] = acc[s][i];
+        __syncthreads();
+        for (int i = wave; i < 16; i += kWaves) {
+            float v = red[i * 64 + lane];
+#pragma unroll
+            for (int o = 1; o < kWaves; o++) v = v + red[(o * 16 + i) * 64 + lane];
+            const int m = 8 * (i >> 2) + 4 * lh + (i & 3), n = n0 + 32 * s + l32;
+            if (n < N && m < M) {
+                if constexpr (sizeof(Y) == 4) y[(int64_t)m * N + n] = v;
+                else y[(int64_t)m * N + n] = f32_to_bf16_bits(v);
+            }
+        }
+    }
+}
+
+std::atomic<int> g_strips{0};  // measurement aid: 1 = wherever the kernel takes the shape, 2 = never
+
+template <typename X, int SW, bool RAGGED, typename Y>
+hipError_t launch(const void* W, const void* x, void* y, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {
+    const int64_t wgs = ((N + 32 * SW - 1) / (32 * SW)) * ((M + 31) / 32);
+    if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+    constexpr int kLds = kWaves * SW * kStripBytes;
+    static_assert(kLds >= kWaves * 16 * 64 * 4, "the sums take the slabs' place");
+    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
+    if (kLds > 64 * 1024 && !raised) {
+        if (hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_strips_kernel<X, SW, RAGGED, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
+        raised = true;
+    }
+    hipLaunchKernelGGL((qgemm_q4_0_strips_kernel<X, SW, RAGGED, Y>), dim3((unsigned)wgs), dim3(64 * kWaves), kLds, st, (const uint8_t*)W, (const X*)x, (Y*)y, (int)M,
+                       (int)N, (int)(K / 32), x_row_stride);
+    return hipGetLastError();
+}
+
+template <typename X, int SW, typename Y>
+hipError_t dispatch(const void* W, const void* x, void* y, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {
+    return K % (32 * kRunBlocks) ? launch<X, SW, true, Y>(W, x, y, M, N, K, x_row_stride, st) : launch<X, SW, false, Y>(W, x, y, M, N, K, x_row_stride, st);
+}
+
+}  // namespace
+
+void set_q4_0_strips(int v) { g_strips = v; }
+
+bool qgemm_q4_0_strips_ok(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride) {
+    return M >= 1 && M <= 65535 && N > 0 && N <= ((int64_t)1 << 30) && K >= 32 * kRunBlocks && K % 32 == 0 && 64 * (K / 32) * 18 < ((int64_t)1 << 32) &&
+           ((uintptr_t)W & 1) == 0 && ((uintptr_t)x & 15) == 0 && x_row_stride % (bf16 ? 8 : 4) == 0;
+}
+
+// float32, against the float32 kernel for one row after another (us there, here): from sixteen rows, 8192 results (16 x 512 x
+// 4064 20, 19; 64 x 128 x 1056 14, 11; 16 x 256 x 1056 8, 10); nine to fifteen, 1000 rows of W (9 x 4096 x 1056 10.2, 10.0; 12 x
+// 512 x 4064 16, 19); five to eight, 32 M weights (6 x 4096 x 8224 47, 35; 6 x 4096 x 4064 14, 19; four rows 33, 35). Past K =
+// 32768 its sums, which are longer than that kernel's, would be the less exact.
+// bfloat16. Rows of W of an odd number of blocks: against that kernel and two conversions, always. Where there is a tile
+// kernel (K a multiple of 256): up to 1024 workgroups here, fewer of shorter rows (256 x 4096 x 4096 62, 46; 256 x 4096 x 1024
+// 20.5, 20.8; 192 x 4096 x 512 12.9, 12.8; 192 x 4096 x 256 9, 11; 1792 workgroups: 100 x 14336 x 4096 65, 78). Else, against
+// the fixed-point forms and two conversions: up to 512.
+bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride) {
+    if (g_strips == 2 || !qgemm_q4_0_strips_ok(W, x, bf16, M, N, K, x_row_stride)) return false;
+    if (g_strips == 1) return true;
+    if (!bf16) {
+        if (K > 32768) return false;
+        if (M >= 16) return M * N >= 8192;
+        return M >= 9 ? N >= 1000 : M >= 5 && N * K >= ((int64_t)32 << 20);
+    }
+    const int64_t wgs = ((N + 31) / 32) * ((M + 31) / 32);
+    if (K % 64 != 0) return true;
+    if (!qgemm_q4_0_ok(W, x, M, N, K, x_row_stride)) return wgs <= 512;
+    return wgs <= (K >= 2048 ? 1024 : K >= 512 ? 768 : 384);
+}
+
+hipError_t qgemm_q4_0_strips(const void* W, const void* x, bool bf16, void* y, bool out_bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {
+    if (!qgemm_q4_0_strips_ok(W, x, bf16, M, N, K, x_row_stride) || (out_bf16 && !bf16)) return hipErrorInvalidValue;
+    if (bf16 && out_bf16) return dispatch<__bf16, 1, uint16_t>(W, x, y, M, N, K, x_row_stride, st);
+    if (bf16) return dispatch<__bf16, 1, float>(W, x, y, M, N, K, x_row_stride, st);
+    const int64_t pairs = ((N + 63) / 64) * ((M + 31) / 32);
+    return pairs >= 256 ? dispatch<float, 2, float>(W, x, y, M, N, K, x_row_stride, st) : dispatch<float, 1, float>(W, x, y, M, N, K, x_row_stride, st);
+}
+
+}  // namespace mimir

@@ -466,3 +466,40 @@ def test_exact_form_from_the_panel_rows_with_nan_and_inf():
     assert not np.isfinite(got32[5]).any() and np.isnan(got32[6]).all()
     keep = np.ones(m, bool); keep[[5, 6]] = False
     assert np.array_equal(got32[keep], base[keep])
+
+
+@pytest.mark.parametrize("half,m,n,k,offset", [(True, 1, 33, 256, 0), (True, 33, 65, 288, 2), (True, 100, 96, 4096, 0), (True, 5, 70, 2080, 0), (True, 64, 31, 1280, 6),
+                                               (False, 16, 513, 288, 0), (False, 33, 1000, 1056, 2), (False, 64, 8200, 352, 0), (False, 9, 1001, 2208, 0),
+                                               (False, 17, 530, 512, 2), (False, 65, 8193, 256, 2), (False, 5, 4097, 8224, 0)])
+def test_some_rows_without_a_workspace(half, m, n, k, offset):
+    """The kernel for some rows of x by W read where it lies: remainders of 32 rows of x and of W and of eight blocks, W
+    on two bytes, one and two strips, on the route that the shape selects. Its float32 sums are held to the bound of
+    the other kernels; a row of numbers near the smallest normal keeps its digits, an infinity and a NaN stay in their rows."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    w = bench_blocks(rng, O.Q4_0, n * k)
+    xf = rng.normal(size=(m, k)).astype(np.float32)
+    if m >= 5:
+        xf[0, -32:] = 0
+        xf[1] *= 1e-36
+        xf[2] *= 1e30
+        xf[3, k - 1] = np.inf
+        xf[4, 0] = np.nan
+    x_bits = bf16_bits(xf)
+    if half:
+        xf = O.bf16_to_f32(x_bits)
+    gpu.say(f"q4_0 without a workspace {'bfloat16' if half else 'float32'} {m}x{k} by {n}x{k}+{offset}")
+    if half:
+        got = qgemm(w, x_bits, n, k, capi.F32, w_offset=offset)
+        assert np.array_equal(qgemm(w, x_bits, n, k, capi.BF16, w_offset=offset), bf16_bits(got)) or m >= 5  # a NaN's bits are its own
+    else:
+        buf, ptr = gpu.dev_bytes_at(w, offset)
+        got = gpu.qgemv(O.Q4_0, ptr, gpu.dev(xf), n, k)
+    finite = [i for i in range(m) if m < 5 or i not in (3, 4)]
+    wf = np.abs(O.dequantize(O.Q4_0, w).reshape(n, k).astype(np.float64))
+    exact = xf[finite].astype(np.float64) @ O.dequantize(O.Q4_0, w).reshape(n, k).astype(np.float64).T
+    bound = np.maximum(2e-6 * (np.abs(xf[finite]).astype(np.float64) @ wf.T), 1e-44)
+    assert np.all(np.abs(got[finite] - exact) <= bound)
+    some = finite[:3] + finite[-1:]
+    assert np.all(np.abs(got[some] - O.qmatmul(O.Q4_0, w, xf[some], n, k)) <= 2 * bound[[finite.index(i) for i in some]])
+    if m >= 5:
+        assert not np.isfinite(got[3]).any() and np.isnan(got[4]).all()

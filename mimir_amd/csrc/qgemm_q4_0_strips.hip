@@ -11,11 +11,11 @@
 // block's sum by its scale. A float32 x is the sum of three bfloat16, exactly, and a block six MFMAs.
 //
 // What bounds it: 30 instructions of unpacking, 16 FMAs and 64 cycles of MFMA a block and strip, with float32 another 150
-// instructions of splitting x (for two strips where they fill the chip) and 192 cycles. From 1024 workgroups on the tile
+// instructions of splitting x (for two strips where they fill the chip) and 192 cycles. From some 1800 workgroups on the tile
 // kernels, which unpack W once for 128 rows, are the faster. Whole calls, us, before and now:
 //   bfloat16   16 x 4096 x 4096    61 -> 10      float32   16 x 4096 x 4064      31 -> 20
-//              64 x 14336 x 4096   63 -> 46               128 x 4096 x 4064     215 -> 30
-//             128 x 4096 x 14336  200 -> 75               512 x 14336 x 4064   3860 -> 370
+//             256 x 4096 x 4096    62 -> 37               128 x 4096 x 4064     215 -> 30
+//             128 x 4096 x 14336  200 -> 68               512 x 14336 x 4064   3860 -> 370
 // Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 8.3e-8 at K = 4096, 1.05e-6 -> 9.4e-8 at 14336; float32
 // 1.96e-7 -> 1.04e-7 at K = 4064, 2.1e-7 -> 1.83e-7 at 28704.
 #include <atomic>
@@ -68,25 +68,49 @@ __device__ __forceinline__ void split(const u32x4* v, bf16x8* parts, float) {
     for (int q = 0; q < 3; q++) __builtin_memcpy(&parts[q], p[q], 16);
 }
 
-// The matrix cores take subnormal operands for nought, which the lesser parts of an x below 2^-103 are. The least of sixteen x a lane
-// other than nought goes into `least`; where one is below 2^-100, the workgroup goes over its share again and takes each
-// block's rows whose largest x is below 2^-60 times 2^64 (in the others what is lost is 2^-66 of the largest).
+// What x's parts and a block's sum do not hold. The matrix cores take subnormal operands for nought, which the lesser parts of
+// a float32 below 2^-103 are; and 32 numbers above 2^122 may add up to more than a float32 holds, where their product with the
+// scale is none. Where a float32 is below 2^-100 (other than nought) or a result no finite number, a workgroup goes over
+// its share again and takes each block's rows whose largest x is below 2^-60 times 2^64 (in the others what is lost is 2^-66 of
+// the largest), from 2^100 on times 2^-64.
 constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1;
 __device__ __forceinline__ void note_least(const u32x4 (*v)[2], uint32_t* least) {
 #pragma unroll
     for (int i = 0; i < 16; i++) *least = min(*least, (v[i >> 3][(i >> 2) & 1][i & 3] << 1) - 1);  // nought: the largest number
 }
-__device__ __forceinline__ float enlarge(u32x4 (*v)[2]) {  // returns what takes the row's sum back
+
+// Sixteen x of a row, eight of each half of the block, by the power of two that suits it; returns what takes the row's sum back.
+__device__ __forceinline__ float factor(float most) {
+    const float other = __shfl_xor(most, 32);  // the other lane's half of the row
+    const float all = other > most || other != other ? other : most;
+    return all < 0x1p-60f ? 0x1p64f : all >= 0x1p100f ? 0x1p-64f : 1.f;
+}
+__device__ __forceinline__ float suit(u32x4 (*v)[2]) {
     float most = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         const float a = __builtin_fabsf(__uint_as_float(v[i >> 3][(i >> 2) & 1][i & 3]));
         most = a > most || a != a ? a : most;
     }
-    const float other = __shfl_xor(most, 32);
-    const float by = most < 0x1p-60f && other < 0x1p-60f ? 0x1p64f : 1.f;  // this lane's half of the row and the other lane's
+    const float by = factor(most);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i >> 3][(i >> 2) & 1][i & 3] = __float_as_uint(__uint_as_float(v[i >> 3][(i >> 2) & 1][i & 3]) * by);
+    return 1.f / by;
+}
+__device__ __forceinline__ float suit(u32x4 (*v)[1]) {
+    float most = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const uint32_t u = v[i >> 3][0][(i >> 1) & 3];
+        const float a = __builtin_fabsf(__uint_as_float(i & 1 ? u & 0xffff0000u : u << 16));
+        most = a > most || a != a ? a : most;
+    }
+    const float by = factor(most);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t u = v[i >> 2][0][i & 3];
+        v[i >> 2][0][i & 3] = upper_halves(__float_as_uint(__uint_as_float(u & 0xffff0000u) * by), __float_as_uint(__uint_as_float(u << 16) * by));
+    }
     return 1.f / by;
 }
 
@@ -96,7 +120,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
                                                                             int nb, int64_t x_row_stride) {
     constexpr int kP = kParts<X>;
     constexpr int kWords = sizeof(X) == 4 ? 2 : 1;  // sixteen-byte loads of eight x
-    constexpr int kAhead = sizeof(X) == 2 ? 8 : SW == 1 ? 4 : 2;  // blocks of x in registers
+    constexpr int kAhead = SW == 1 ? 4 : 2;  // blocks of x in registers: of bfloat16 with eight, two wavefronts a SIMD instead of four (256 x 4096 x 4096: 55 us, 38)
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -246,32 +270,36 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
             for (int i = 0; i < 16; i++) acc[s][i] += part[s][i];
         }
     }
-    if constexpr (kP == 3) {
-        if (__syncthreads_or(least < kTiny)) {  // seldom; block after block
+    bool beyond = least < kTiny;
 #pragma unroll
-            for (int s = 0; s < SW; s++) {
+    for (int s = 0; s < SW; s++) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
-            }
+        for (int i = 0; i < 16; i++) beyond = beyond || !(__builtin_fabsf(acc[s][i]) < __builtin_inff());
+    }
+    if (__syncthreads_or(beyond)) {  // seldom; block after block
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
+        }
 #pragma unroll 1
-            for (int run = wave; run < nruns; run += kWaves) {
-                const int at = start_of(run);
-                fetch_w(at);
-                store_w();
+        for (int run = wave; run < nruns; run += kWaves) {
+            const int at = start_of(run);
+            fetch_w(at);
+            store_w();
 #pragma unroll 1
-                for (int b = kRunBlocks * run - at; b < kRunBlocks; b++) {
-                    fetch_x(0, at + b);
-                    const float back = enlarge(xs[0]);
-                    bf16x8 xp[2][kP];
+            for (int b = kRunBlocks * run - at; b < kRunBlocks; b++) {
+                fetch_x(0, at + b);
+                const float back = suit(xs[0]);
+                bf16x8 xp[2][kP];
 #pragma unroll
-                    for (int h = 0; h < 2; h++) split(xs[0][h], xp[h], X());
+                for (int h = 0; h < 2; h++) split(xs[0][h], xp[h], X());
 #pragma unroll
-                    for (int s = 0; s < SW; s++) {
-                        float d;
-                        const f32x16 c = product(s, b, xp, &d);
+                for (int s = 0; s < SW; s++) {
+                    float d;
+                    const f32x16 c = product(s, b, xp, &d);
 #pragma unroll
-                        for (int i = 0; i < 16; i++) acc[s][i] = fmaf(d, c[i] * __shfl(back, 8 * (i >> 2) + 4 * lh + (i & 3)), acc[s][i]);
-                    }
+                    for (int i = 0; i < 16; i++) acc[s][i] = fmaf(d * c[i], __shfl(back, 8 * (i >> 2) + 4 * lh + (i & 3)), acc[s][i]);
                 }
             }
         }
@@ -318,7 +346,7 @@ hipError_t launch(const void* W, const void* x, void* y, int64_t M, int64_t N, i
 
 template <typename X, int SW, typename Y>
 hipError_t dispatch(const void* W, const void* x, void* y, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {
-    return K % (32 * kRunBlocks) ? launch<X, SW, true, Y>(W, x, y, M, N, K, x_row_stride, st) : launch<X, SW, false, Y>(W, x, y, M, N, K, x_row_stride, st);
+    return SW == 2 || K % (32 * kRunBlocks) ? launch<X, SW, true, Y>(W, x, y, M, N, K, x_row_stride, st) : launch<X, 1, false, Y>(W, x, y, M, N, K, x_row_stride, st);
 }
 
 }  // namespace
@@ -335,9 +363,9 @@ bool qgemm_q4_0_strips_ok(const void* W, const void* x, bool bf16, int64_t M, in
 // 512 x 4064 16, 19); five to eight, 32 M weights (6 x 4096 x 8224 47, 35; 6 x 4096 x 4064 14, 19; four rows 33, 35). Past K =
 // 32768 its sums, which are longer than that kernel's, would be the less exact.
 // bfloat16. Rows of W of an odd number of blocks: against that kernel and two conversions, always. Where there is a tile
-// kernel (K a multiple of 256): up to 1024 workgroups here, fewer of shorter rows (256 x 4096 x 4096 62, 46; 256 x 4096 x 1024
-// 20.5, 20.8; 192 x 4096 x 512 12.9, 12.8; 192 x 4096 x 256 9, 11; 1792 workgroups: 100 x 14336 x 4096 65, 78). Else, against
-// the fixed-point forms and two conversions: up to 512.
+// kernel (K a multiple of 256): up to 1792 workgroups here, fewer of shorter rows (there, here: 256 x 4096 x 4096, 1024
+// workgroups, 62, 37; 128 x 14336 x 4096, 1792, 64, 61; 96 x 14336 x 1024, 1344, 21, 20; 256 x 4096 x 512 13.3, 12.1; 192 x
+// 4096 x 256, 768, 9.0, 9.2). Else, against the fixed-point forms and two conversions: up to 512.
 bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride) {
     if (g_strips == 2 || !qgemm_q4_0_strips_ok(W, x, bf16, M, N, K, x_row_stride)) return false;
     if (g_strips == 1) return true;
@@ -349,7 +377,7 @@ bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, 
     const int64_t wgs = ((N + 31) / 32) * ((M + 31) / 32);
     if (K % 64 != 0) return true;
     if (!qgemm_q4_0_ok(W, x, M, N, K, x_row_stride)) return wgs <= 512;
-    return wgs <= (K >= 2048 ? 1024 : K >= 512 ? 768 : 384);
+    return wgs <= (K >= 2048 ? 1792 : K >= 1024 ? 1344 : K >= 512 ? 1024 : 512);
 }
 
 hipError_t qgemm_q4_0_strips(const void* W, const void* x, bool bf16, void* y, bool out_bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {

@@ -14,10 +14,11 @@
 // instructions of splitting x (for two strips where they fill the chip) and 192 cycles. From some 1800 workgroups on the tile
 // kernels, which unpack W once for 128 rows, are the faster. Whole calls, us, before and now:
 //   bfloat16   16 x 4096 x 4096    61 -> 10      float32   16 x 4096 x 4064      31 -> 20
-//             256 x 4096 x 4096    62 -> 37               128 x 4096 x 4064     215 -> 30
-//             128 x 4096 x 14336  200 -> 68               512 x 14336 x 4064   3860 -> 370
-// Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 8.3e-8 at K = 4096, 1.05e-6 -> 9.4e-8 at 14336; float32
-// 1.96e-7 -> 1.04e-7 at K = 4064, 2.1e-7 -> 1.83e-7 at 28704.
+//             256 x 4096 x 4096    62 -> 38               128 x 4096 x 4064     215 -> 30
+//             128 x 4096 x 14336  200 -> 70               512 x 14336 x 4064   3860 -> 370
+// Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 6.6e-8 at K = 4096 (7.4e-8 at 4064), 1.05e-6 -> 6.5e-8 at 14336;
+// float32 1.96e-7 -> 9.1e-8 at K = 4064, 2.0e-7 -> 1.34e-7 at 14368. With the runs' and the wavefronts' sums in 32 bits it was
+// 8.3e-8 of bfloat16 at K = 4096, more than the 7.4e-8 of the kernel for an odd number of blocks.
 #include <atomic>
 
 #include "device_util.h"
@@ -70,7 +71,8 @@ __device__ __forceinline__ void split(const u32x4* v, bf16x8* parts, float) {
 
 // What x's parts and a block's sum do not hold. The matrix cores take subnormal operands for nought, which the lesser parts of
 // a float32 below 2^-103 are; and 32 numbers above 2^122 may add up to more than a float32 holds, where their product with the
-// scale is none. Where a float32 is below 2^-100 (other than nought) or a result no finite number, a workgroup goes over
+// scale is none. Where a float32 is below 2^-100, or a bfloat16 subnormal (other than nought; the tile kernel takes these for
+// nought too, so they are looked for in its stead only where it does not go), or a result no finite number, a workgroup goes over
 // its share again and takes each block's rows whose largest x is below 2^-60 times 2^64 (in the others what is lost is 2^-66 of
 // the largest), from 2^100 on times 2^-64.
 constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1;
@@ -78,6 +80,21 @@ __device__ __forceinline__ void note_least(const u32x4 (*v)[2], uint32_t* least)
 #pragma unroll
     for (int i = 0; i < 16; i++) *least = min(*least, (v[i >> 3][(i >> 2) & 1][i & 3] << 1) - 1);  // nought: the largest number
 }
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void note_least(const u32x4 (*v)[1], uint32_t* least) {  // two halves a word
+    u16x2 most, one;
+    __builtin_memcpy(&most, least, 4);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t bits = v[i >> 2][0][i & 3] & 0x7fff7fffu;
+        __builtin_memcpy(&one, &bits, 4);
+        most = __builtin_elementwise_min(most, one - (uint16_t)1);
+    }
+    __builtin_memcpy(least, &most, 4);
+}
+__device__ __forceinline__ bool tiny(uint32_t least, float) { return least < kTiny; }
+__device__ __forceinline__ bool tiny(uint32_t least, __bf16) { return (least & 0xffffu) < 0x7f || (least >> 16) < 0x7f; }
 
 // Sixteen x of a row, eight of each half of the block, by the power of two that suits it; returns what takes the row's sum back.
 __device__ __forceinline__ float factor(float most) {
@@ -114,9 +131,12 @@ __device__ __forceinline__ float suit(u32x4 (*v)[1]) {
     return 1.f / by;
 }
 
-// SW: strips of 32 rows of W a workgroup. RAGGED: the blocks of a row are no multiple of eight.
+__device__ double acc_of(__bf16);
+__device__ float acc_of(float);
+
+// SW: strips of 32 rows of W a workgroup. RAGGED: the blocks of a row need be no multiple of eight, and subnormal bfloat16 count.
 template <typename X, int SW, bool RAGGED, typename Y>
-__global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const uint8_t* __restrict__ W, const X* __restrict__ x, Y* __restrict__ y, int M, int N,
+__global__ __launch_bounds__(64 * kWaves, sizeof(X) == 2 && !RAGGED ? 4 : 2) void qgemm_q4_0_strips_kernel(const uint8_t* __restrict__ W, const X* __restrict__ x, Y* __restrict__ y, int M, int N,
                                                                             int nb, int64_t x_row_stride) {
     constexpr int kP = kParts<X>;
     constexpr int kWords = sizeof(X) == 4 ? 2 : 1;  // sixteen-byte loads of eight x
@@ -222,12 +242,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
         }
     };
 
-    // A run's sums by themselves, then the runs': short chains, small errors
-    float acc[SW][16];
+    // A run's sums by themselves, the runs' in 64 bits (of float32 x, whose blocks' sums err by more, in 32)
+    using Acc = decltype(acc_of(X()));
+    Acc acc[SW][16];
 #pragma unroll
     for (int s = 0; s < SW; s++) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
+        for (int i = 0; i < 16; i++) acc[s][i] = 0;
     }
     uint32_t least = 0xffffffffu;
     if (wave < nruns) {
@@ -253,7 +274,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
                 }
                 split(v[h], xp[h], X());
             }
-            if constexpr (kP == 3) note_least(v, &least);
+            if constexpr (kP == 3 || RAGGED) note_least(v, &least);
             fetch_x(b % kAhead, b + kAhead < kRunBlocks ? at + b + kAhead : next + b + kAhead - kRunBlocks);
 #pragma unroll
             for (int s = 0; s < SW; s++) {
@@ -270,17 +291,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
             for (int i = 0; i < 16; i++) acc[s][i] += part[s][i];
         }
     }
-    bool beyond = least < kTiny;
+    bool beyond = tiny(least, X());
 #pragma unroll
     for (int s = 0; s < SW; s++) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) beyond = beyond || !(__builtin_fabsf(acc[s][i]) < __builtin_inff());
+        for (int i = 0; i < 16; i++) beyond = beyond || !(__builtin_fabsf((float)acc[s][i]) < __builtin_inff());
     }
     if (__syncthreads_or(beyond)) {  // seldom; block after block
 #pragma unroll
         for (int s = 0; s < SW; s++) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[s][i] = 0.f;
+            for (int i = 0; i < 16; i++) acc[s][i] = 0;
         }
 #pragma unroll 1
         for (int run = wave; run < nruns; run += kWaves) {
@@ -299,7 +320,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
                     float d;
                     const f32x16 c = product(s, b, xp, &d);
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[s][i] = fmaf(d * c[i], __shfl(back, 8 * (i >> 2) + 4 * lh + (i & 3)), acc[s][i]);
+                    for (int i = 0; i < 16; i++) acc[s][i] += (Acc)(d * c[i]) * (Acc)__shfl(back, 8 * (i >> 2) + 4 * lh + (i & 3));
                 }
             }
         }
@@ -311,12 +332,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_q4_0_strips_kernel(const
     for (int s = 0; s < SW; s++) {
         if (s > 0) __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; i++) red[(wave * 16 + i) * 64 + lane] = acc[s][i];
+        for (int i = 0; i < 16; i++) red[(wave * 16 + i) * 64 + lane] = (float)acc[s][i];
         __syncthreads();
         for (int i = wave; i < 16; i += kWaves) {
-            float v = red[i * 64 + lane];
+            double sum = red[i * 64 + lane];
 #pragma unroll
-            for (int o = 1; o < kWaves; o++) v = v + red[(o * 16 + i) * 64 + lane];
+            for (int o = 1; o < kWaves; o++) sum += red[(o * 16 + i) * 64 + lane];
+            const float v = (float)sum;
             const int m = 8 * (i >> 2) + 4 * lh + (i & 3), n = n0 + 32 * s + l32;
             if (n < N && m < M) {
                 if constexpr (sizeof(Y) == 4) y[(int64_t)m * N + n] = v;
@@ -346,7 +368,8 @@ hipError_t launch(const void* W, const void* x, void* y, int64_t M, int64_t N, i
 
 template <typename X, int SW, typename Y>
 hipError_t dispatch(const void* W, const void* x, void* y, int64_t M, int64_t N, int64_t K, int64_t x_row_stride, hipStream_t st) {
-    return SW == 2 || K % (32 * kRunBlocks) ? launch<X, SW, true, Y>(W, x, y, M, N, K, x_row_stride, st) : launch<X, 1, false, Y>(W, x, y, M, N, K, x_row_stride, st);
+    const bool tiles = K % (32 * kRunBlocks) == 0 && (sizeof(X) == 4 || qgemm_q4_0_ok(W, x, M, N, K, x_row_stride));
+    return SW == 2 || !tiles ? launch<X, SW, true, Y>(W, x, y, M, N, K, x_row_stride, st) : launch<X, 1, false, Y>(W, x, y, M, N, K, x_row_stride, st);
 }
 
 }  // namespace
@@ -362,9 +385,10 @@ bool qgemm_q4_0_strips_ok(const void* W, const void* x, bool bf16, int64_t M, in
 // 4064 20, 19; 64 x 128 x 1056 14, 11; 16 x 256 x 1056 8, 10); nine to fifteen, 1000 rows of W (9 x 4096 x 1056 10.2, 10.0; 12 x
 // 512 x 4064 16, 19); five to eight, 32 M weights (6 x 4096 x 8224 47, 35; 6 x 4096 x 4064 14, 19; four rows 33, 35). Past K =
 // 32768 its sums, which are longer than that kernel's, would be the less exact.
-// bfloat16. Rows of W of an odd number of blocks: against that kernel and two conversions, always. Where there is a tile
+// bfloat16. Rows of W of an odd number of blocks: against that kernel and two conversions, but for a few rows by few long
+// ones of W (8 x 1024 x 8224 34, 20; 2 x 4096 x 14368 35, 33; 2 x 1024 x 8224 14, 20). Where there is a tile
 // kernel (K a multiple of 256): up to 1792 workgroups here, fewer of shorter rows (there, here: 256 x 4096 x 4096, 1024
-// workgroups, 62, 37; 128 x 14336 x 4096, 1792, 64, 61; 96 x 14336 x 1024, 1344, 21, 20; 256 x 4096 x 512 13.3, 12.1; 192 x
+// workgroups, 62, 38; 128 x 14336 x 4096, 1792, 64, 62; 96 x 14336 x 1024, 1344, 21, 20; 256 x 4096 x 512 13.4, 12.5; 192 x
 // 4096 x 256, 768, 9.0, 9.2). Else, against the fixed-point forms and two conversions: up to 512.
 bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, int64_t N, int64_t K, int64_t x_row_stride) {
     if (g_strips == 2 || !qgemm_q4_0_strips_ok(W, x, bf16, M, N, K, x_row_stride)) return false;
@@ -375,7 +399,7 @@ bool qgemm_q4_0_strips_pays(const void* W, const void* x, bool bf16, int64_t M, 
         return M >= 9 ? N >= 1000 : M >= 5 && N * K >= ((int64_t)32 << 20);
     }
     const int64_t wgs = ((N + 31) / 32) * ((M + 31) / 32);
-    if (K % 64 != 0) return true;
+    if (K % 64 != 0) return M >= 6 || N >= 4096 || K <= 4096;
     if (!qgemm_q4_0_ok(W, x, M, N, K, x_row_stride)) return wgs <= 512;
     return wgs <= (K >= 2048 ? 1792 : K >= 1024 ? 1344 : K >= 512 ? 1024 : 512);
 }

@@ -481,7 +481,7 @@ def test_some_rows_without_a_workspace(half, m, n, k, offset):
     xf = rng.normal(size=(m, k)).astype(np.float32)
     if m >= 5:
         xf[0, -32:] = 0
-        xf[1] *= 1e-36
+        xf[1] *= 1e-39 if half and k % 256 else 1e-36  # subnormal bfloat16 where the tile kernel does not go
         xf[2] = 0
         xf[2, 32:64] = 1.2e38 * rng.uniform(0.5, 1.0, 32)  # a block's sum before its scale is now and then more than float32 holds
         xf[3, k - 1] = np.inf

@@ -509,7 +509,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * "attention.prompt" = 0 makes it use them also for 64 and more query positions
  * (which otherwise, without a mask, at 64 or 128 features and key rows that start
  * on 16 bytes, take a kernel that shares tiles of keys among 128 query rows on the
- * float32 matrix cores: the same sums in another order).
+ * float32 matrix cores, of binary16 keys on the 16-bit ones: the same sums in another
+ * order); 2 keeps binary16 keys on the float32 ones, as a decoder does whose
+ * products round activations to int8.
  * "llama.step" chooses how mi355x_llama_generate runs its decoding steps: 0 the
  * fused launches replayed as a HIP graph where every block's linears are Q4_0
  * (else the per-operator path), 1 the same launches without the graph, 2 the

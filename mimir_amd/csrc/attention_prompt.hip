@@ -4,7 +4,7 @@
 // query i when causal and j > i + causal_offset; backend/cpu/attention.go:268-292, 437-535), for the calls that kernel
 // serves one query row a workgroup, re-reading every key and value for every row.
 //
-// Two kernels: one for float32 keys and values, described here, and one for binary16, described where it stands.
+// Two kernels: one on float32 operands, described here, and one for binary16 keys and values, described where it stands.
 // A wavefront owns 32 query rows of one head and walks the keys in tiles of 32 with a running maximum and sum per
 // row (a row's result is rescaled when its maximum grows), and both products of a tile are MFMAs on float32 operands
 // (v_mfma_f32_32x32x2_f32), so that nothing is rounded that the other kernel does not round. Both are computed
@@ -250,16 +250,16 @@ __device__ __forceinline__ void rows_by_float32(const float* __restrict__ q, con
     if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
 }
 
-template <int D, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, (D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                                                                  const float* __restrict__ v, float* __restrict__ out,
-                                                                                                  float* __restrict__ lse, PromptParams p) {
+template <typename KV, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES == 2) ? 1 : 2) void attn_prompt_kernel(const float* __restrict__ q, const KV* __restrict__ k,
+                                                                                                                     const KV* __restrict__ v, float* __restrict__ out,
+                                                                                                                     float* __restrict__ lse, PromptParams p) {
     __shared__ float ks[kTile * Float32Lds<D>::KS];
     __shared__ __align__(16) float vs[kTile * D];
     __shared__ int vbad[2];
     // the grid is (head, sequence, block of rows), the last rows first: under causality they see the most keys, and
     // workgroups are handed out in this order
-    rows_by_float32<float, D, WAVES, WAVES * kRows>(q, k, v, out, lse, p, blockIdx.y, blockIdx.x, (int)(gridDim.z - 1 - blockIdx.z) * WAVES * kRows, ks, vs, vbad);
+    rows_by_float32<KV, D, WAVES, WAVES * kRows>(q, k, v, out, lse, p, blockIdx.y, blockIdx.x, (int)(gridDim.z - 1 - blockIdx.z) * WAVES * kRows, ks, vs, vbad);
 }
 
 // The same for keys and values in binary16, by sums of products of 16-bit parts that are exact, on instructions sixteen times as fast as the float32 one:
@@ -554,14 +554,14 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
     if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
 }
 
-std::atomic<int> g_prompt{1};  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup
+std::atomic<int> g_prompt{1};  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup, 2 those over binary16 on float32 operands
 
-template <int WAVES>
+template <typename KV, int WAVES>
 hipError_t launch_f32(const AttnArgs& a, const PromptParams& p, hipStream_t st) {
     const dim3 grid((unsigned)a.H, (unsigned)a.B, (unsigned)((a.Q + WAVES * kRows - 1) / (WAVES * kRows))), block(64 * WAVES);
-    const float *k = (const float*)a.k, *v = (const float*)a.v;
-    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_kernel<128, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
-    else hipLaunchKernelGGL((attn_prompt_kernel<64, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+    const KV *k = (const KV*)a.k, *v = (const KV*)a.v;
+    if (a.D == 128) hipLaunchKernelGGL((attn_prompt_kernel<KV, 128, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
+    else hipLaunchKernelGGL((attn_prompt_kernel<KV, 64, WAVES>), grid, block, 0, st, a.q, k, v, a.out, a.lse, p);
     return hipGetLastError();
 }
 
@@ -606,8 +606,9 @@ hipError_t attention_prompt(const AttnArgs& a, hipStream_t st) {
     // two wavefronts on the same rows (binary16; at 512 workgroups the two are level, see the figures there)
     const bool few = a.B * a.H * ((a.Q + 4 * kRows - 1) / (4 * kRows)) < 512;
     note_kernel("attn_prompt_kernel");
+    if (a.kv_dtype == kF16 && (a.float32_operands || g_prompt == 2)) return few ? launch_f32<uint16_t, 2>(a, p, st) : launch_f32<uint16_t, 4>(a, p, st);
     if (a.kv_dtype == kF16) return few ? launch_f16<2>(a, p, st) : launch_f16<1>(a, p, st);
-    return few ? launch_f32<2>(a, p, st) : launch_f32<4>(a, p, st);
+    return few ? launch_f32<float, 2>(a, p, st) : launch_f32<float, 4>(a, p, st);
 }
 
 }  // namespace mimir

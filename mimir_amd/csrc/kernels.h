@@ -232,15 +232,16 @@ struct AttnArgs {
     int DV = 0;                      // features of a value (0: D)
     const float* mask = nullptr;     // added to the scores, [B, H, Q, K] read through m_strides {batch, head, query, key}
     int64_t m_strides[4] = {0, 0, 0, 0};
+    bool float32_operands = false;   // of a prompt over binary16 keys and values: products and sums of float32 operands, in their order
 };
 void attention_plan(int64_t B, int H, int HK, int64_t Q, int64_t K, int* chunk, int* nsplit);
 size_t attention_workspace_bytes(int64_t B, int H, int64_t Q, int D, int nsplit);
 hipError_t attention(const AttnArgs& a, void* workspace, hipStream_t st);
-// Many query positions at once on the float32 matrix cores (attention_prompt.hip), which attention() takes for the calls
+// Many query positions at once on the matrix cores (attention_prompt.hip), which attention() takes for the calls
 // attention_prompt_ok names: the same results up to the order of the float32 sums.
 bool attention_prompt_ok(const AttnArgs& a);
 hipError_t attention_prompt(const AttnArgs& a, hipStream_t st);
-void set_attention_prompt(int v);  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup
+void set_attention_prompt(int v);  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup, 2 those over binary16 on float32 operands
 // K == 0: zeros and a logsumexp of -Inf for every row; reads neither keys nor values.
 hipError_t attention_empty(const AttnArgs& a, hipStream_t st);
 

@@ -66,6 +66,10 @@ struct Model : Decoder {
     float* up = nullptr;  // behind gate's rows: products of both matrices at once have [rows, 2 hidden] there
     DevBuf fx_panel;  // the workspace of the Q4_0 products of a prompt's rows on the binary16 matrix cores: the largest product's
 
+    // Whether a block's product rounds x to int8 (Q8_0, Q4_K, Q6_K). There a difference in x's last place can be a step of a quant, a 127th of its block's
+    // largest, and a few layers make some 1e-2 of a logit of it: attention of a prompt keeps float32 operands and the order of their sums.
+    bool int8_products = false;
+
     // `fast` says the blocks qualify for the step of fused launches (Q4_0 linears that the fixed-point kernel takes).
     bool fast = false;
     DevBuf qkv, gu;  // gu: gate|up of a step, [batch, 2 hidden]
@@ -280,6 +284,7 @@ static mi355x_status forward(Model& m, int64_t s) {
         at.B = B; at.Q = s; at.K = past + s; at.H = c.heads; at.HK = c.kv_heads; at.D = c.head_dim;
         at.scale = 1.0 / std::sqrt((double)c.head_dim);
         at.causal = 1; at.causal_offset = past;
+        at.float32_operands = m.int8_products;
         attention_plan(B, c.heads, c.kv_heads, s, at.K, &at.chunk, &at.nsplit);
         size_t need = attention_workspace_bytes(B, c.heads, s, c.head_dim, at.nsplit);
         if (need + kAttnTicketBytes > m.act[0].bytes) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: attention scratch of %zu bytes, need %zu", m.act[0].bytes, need);
@@ -847,6 +852,9 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
         LLM_HIP(hipMemset(m->attn_flags.p, 0, fb + 64), "hipMemset(attention hand-over)");
     }
     LLM_HIP(m->qkv.alloc((size_t)c.batch * (qd + 2 * kvd) * 4), "hipMalloc");
+    m->int8_products = false;
+    for (const Block& b : m->blocks)
+        for (const Weight* w : {&b.q, &b.k, &b.v, &b.o, &b.gate, &b.up, &b.down}) m->int8_products = m->int8_products || w->dtype == kQ8_0 || w->dtype == kQ4_K || w->dtype == kQ6_K;
     m->fast = rmsnorm_q4act_ok(c.embed) && c.head_dim % 2 == 0;
     bool biased = false;  // q, k, v with biases: the generic step, whose rotation launch adds them first
     for (int i = 0; i < c.layers; i++) biased = biased || m->blocks[i].biased();

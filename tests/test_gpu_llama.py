@@ -576,3 +576,24 @@ def test_a_prompt_by_k_quants_takes_matrices_of_one_x_together(linear_dt, batch,
         want = om.logits(prompts[b].tolist(), om.new_caches(c.context, O.F32), all=True)
         err = np.abs(got[b] - want).max(1) / np.abs(want).max()
         assert err.max() <= 0.05 and np.median(err) <= 0.01, err
+
+
+@pytest.mark.parametrize("linear_dt", [O.Q4_K, O.Q6_K, O.Q8_0, O.Q4_0])
+def test_a_prompt_whose_products_round_to_int8_keeps_the_order_of_attentions_sums(linear_dt):
+    """Rounding to int8 makes a step of a difference in the last place: a decoder of such products takes attention of a prompt over a binary16 cache on float32
+    operands, bit for bit as the setting that has every call there does. One of Q4_0 products does not."""
+    lib = gpu.lib()
+    c = _small_q4_config(2, capi.F16)
+    om = OL.synthetic(_oracle_config(c), seed=6, linear_dt=linear_dt, output_dt=O.Q4_0)
+    gpu.say(f"prompt attention of a decoder by dtype {linear_dt}")
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(90)
+    prompts = np.random.default_rng(6).integers(0, c.vocab, (2, 90))
+    got = m.logits(prompts, all=True)
+    try:
+        capi.check(lib.mi355x_tune(b"attention.prompt", 2))
+        m.reset()
+        assert np.array_equal(m.logits(prompts, all=True), got) == (linear_dt != O.Q4_0)
+    finally:
+        capi.check(lib.mi355x_tune(b"attention.prompt", 1))

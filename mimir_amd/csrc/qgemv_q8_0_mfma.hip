@@ -1,12 +1,15 @@
 // Products of two and more rows of x with Q8_0 weights on the int8 matrix cores of gfx950, W read once for eight rows
 // (the output projection of a batch's decoding step) or for 32 (a prompt's rows). What it computes is qdotQ8_0Go's sum
-// (backend/cpu/qmatmul.go:125-139, see qgemv_q8_0.hip) in another order: a block's int32 sum, exact, once times the
-// product of the two scales, where the CPU keeps four sums, one for every fourth group of four values, and adds them
-// at the end.
+// (backend/cpu/qmatmul.go:125-139, see qgemv_q8_0.hip), in one of two orders:
+//   - a block's int32 sum, exact, once times the product of the two scales;
+//   - FOUR: the CPU's four sums a block, one for every fourth group of four values, each times the product of the scales (a
+//     multiply, then an add) into a float32 sum of its own, added (0 + 2) + (1 + 3) at the end. It serves two to eight rows by the
+//     largest matrices, the output projections, whose results stay what they were before there was the other (8 x 32768 x 4096: 36.1 us by the other, 36.7).
 //
-// One v_mfma_i32_32x32x32_i8 per block: its first operand has 32 rows of x, or eight rows four times, its other operand
+// One v_mfma_i32_32x32x32_i8 per block: its first operand has 32 rows of x, or eight rows four times (FOUR: each time with everything but the
+// values of one of the four sums zeroed, which of the 16 values a lane holds are one dword), its other operand
 // 32 rows of W. A lane ends up with its row of W's sums for sixteen rows of x, or for four (and three times again,
-// which it leaves). A workgroup's wavefronts take runs of eight blocks in turn and add their sums up in order.
+// which it leaves, or the four sums of each). A workgroup's wavefronts take runs of eight blocks in turn and add their sums up in order.
 //
 // W stays in ggml's layout. As in qgemv_q4_0_rows.hip, a wavefront loads a run of its 32 rows as 16-byte pieces in row
 // order (272 bytes a row), passes them through a private LDS slab and reads its 16 int8 of each block back as dwords.
@@ -20,11 +23,10 @@
 // too few for them where the matrix is small. 32 rows: a conversion, a product and an fma for each sum and block, 192
 // cycles beside the MFMA's 32 and some 60 of unpacking; 315 TFLOP/s at 512 x 4096 x 14336. Whole calls, us, with W read for eight rows
 // by the vector unit (and by four zeroed copies of x on the matrix cores: 2 and 8 x 32768 x 4096) and now:
-//   2, 8 x 32768 x 4096    38, 42 -> 32, 36        8 x 4096 x 14336     71 -> 29
+//   2, 8 x 32768 x 4096    40, 43 -> 35, 37        8 x 4096 x 14336     71 -> 29
 //   32 x 32768 x 4096         122 -> 49            64 x 1024 x 4096     34 -> 14
 //   512 x 4096 x 14336       3511 -> 191           128 x 4096 x 4096   229 -> 24
-// Errors against 64 bits, of the result: K = 256: 7.2e-8 -> 6.0e-8, 4096: 9.1e-8 (head of 32768 rows: 1.25e-7) ->
-// 8.5e-8, 14336: 1.02e-7 -> 9.8e-8, 28672: 1.13e-7 -> 1.03e-7, 57344: 1.3e-7 .. 3.9e-7 -> 1.1e-7.
+// Errors against 64 bits, of the result: K = 256: 7.2e-8 -> 6.0e-8, 4096: 9.1e-8 -> 8.5e-8 (FOUR: 1.25e-7 as ever), 14336: 1.02e-7 -> 9.8e-8, 28672: 1.13e-7 -> 1.03e-7, 57344: 1.3e-7 .. 3.9e-7 -> 1.1e-7.
 #include "device_util.h"
 #include "kernels.h"
 
@@ -49,12 +51,14 @@ constexpr int kRunsTogether = 8;
 template <int XR>
 constexpr int kWaveLds = kSlabBytes + kRunBlocks * XR * 4 + (XR == kManyRows ? XR * kRunBlocks * 32 : 0);
 
-// XR: rows of x a workgroup (8 or 32); WAVES: its wavefronts, among which the runs of K go round
-template <int XR, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, int M,
+// XR: rows of x a workgroup (8 or 32); WAVES: its wavefronts, among which the runs of K go round. AHEAD: a run's loads stay a run ahead, which takes the
+// registers of two wavefronts: for so few workgroups that no more are on a compute unit (four sums, us, without and with: 4 x 8192 x 14336 48, 33).
+template <int XR, int WAVES, bool FOUR = false, bool AHEAD = false>
+__global__ __launch_bounds__(64 * WAVES, XR == kManyRows || AHEAD ? 2 : 4) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, int M,
                                                                                              int N, int nb, int64_t act_row_bytes) {
     constexpr bool kMany = XR == kManyRows;
-    constexpr int kSums = XR / 2;  // of a lane
+    constexpr int kSums = FOUR ? 16 : XR / 2;  // of a lane
+    static_assert(!FOUR || XR == 8, "four sums of each of a lane's four rows");
     extern __shared__ __align__(16) uint8_t smem[];  // per wavefront; later the wavefronts' sums
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -85,6 +89,7 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
     // rows past M: the last one again, not stored
     auto row_of = [&](int r) { return act + (int64_t)(r < M ? r : M - 1) * act_row_bytes; };
     const i32x4* xq = (const i32x4*)row_of(l32 & (XR - 1)) + (int64_t)lh * nbp;  // + b: half lh of block b of this lane's operand row
+    const int sum = l32 >> 3;                                                    // FOUR: which sum's values it keeps, a dword of a half
     uint32_t xoff[8];  // of 32 rows: this lane's pieces of a run, of row 4 i + lane / 16 half (lane / 8) % 2 of block lane % 8
 #pragma unroll
     for (int i = 0; i < 8; i++)
@@ -95,13 +100,18 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
 
     auto start_of = [&](int run) { return kRunBlocks * run < nb - kRunBlocks ? kRunBlocks * run : nb - kRunBlocks; };  // the last run reaches back
     u32x4 w[kLoads];
-    i32x4 x[8];  // eight rows: the operands of a run's blocks; 32: this lane's pieces of it
+    i32x4 x[FOUR ? 1 : 8];  // eight rows: the operands of a run's blocks; 32: this lane's pieces of it
+    int kept[FOUR ? 8 : 1];
+    auto fetch_x = [&](int b, int block) {  // of eight rows
+        if constexpr (FOUR) kept[b] = ((const int*)(xq + block))[sum];
+        else x[b] = xq[block];
+    };
     float own[kMany ? 4 : 1];
     auto fetch = [&](int at) {
         const uint8_t* p = wbase + (int64_t)at * 34;
 #pragma unroll
         for (int i = 0; i < kLoads; i++) w[i] = load_u32x4_unaligned(p + goff[i]);
-        if (kMany) {
+        if constexpr (kMany) {
 #pragma unroll
             for (int i = 0; i < 8; i++) x[i] = *(const i32x4*)(act + xoff[i] + 16 * at);
         }
@@ -117,7 +127,7 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
         fetch(start_of(wave));
 #pragma unroll
         for (int b = 0; b < kRunBlocks; b++)
-            if (!kMany) x[b] = xq[start_of(wave) + b];
+            if (!kMany) fetch_x(b, start_of(wave) + b);
     }
     const uint8_t* mine = slab + l32 * kSlabStride + 16 * lh;  // the lane's 16 int8 of block b: bytes 34 b + 2 + 16 lh
     for (int run = wave; run < nruns; run += WAVES) {
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
 #pragma unroll
         for (int i = 0; i < kLoads - 1; i++) *(u32x4*)(slab + loff[i]) = w[i];
         if (lane < 32 * kPieces - 64 * (kLoads - 1)) *(u32x4*)(slab + loff[kLoads - 1]) = w[kLoads - 1];
-        if (kMany) {
+        if constexpr (kMany) {
 #pragma unroll
             for (int i = 0; i < 4; i++) dxs[(4 * lh + i) * XR + l32] = own[i % (kMany ? 4 : 1)];
 #pragma unroll
@@ -135,6 +145,7 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
             dxs[(l32 >> 2) * XR + 4 * lh + (l32 & 3)] = own[0];
         }
         fetch(next);
+        if (AHEAD) __builtin_amdgcn_sched_barrier(0);
         // The block's product of this lane's row of W (scale into dw).
         auto multiply = [&](int b, float* dw) {
             // bytes 34 b + 2 ..: on a dword for odd b, two bytes into one for even b
@@ -154,7 +165,13 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
                 *dw = f16_bits_to_f32((uint16_t)(*(const uint32_t*)(slab + l32 * kSlabStride + 34 * b) & 0xffffu));
             }
             *dw = b < done ? 0.f : *dw;  // blocks that the run before has taken
-            const i32x4 xop = kMany ? *(const i32x4*)(xslab + x_piece(l32, lh, b)) : x[b];
+            i32x4 xop;
+            if constexpr (FOUR) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) xop[i] = sum == i ? kept[b] : 0;  // operand row 8 l + m: sum l of row m
+            } else {
+                xop = kMany ? *(const i32x4*)(xslab + x_piece(l32, lh, b)) : x[b];
+            }
             i32x16 zero;
 #pragma unroll
             for (int i = 0; i < 16; i++) zero[i] = 0;
@@ -169,17 +186,33 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
             i32x16 c_next = c;
             if (b + 1 < kRunBlocks) c_next = multiply(b + 1, &dw_next);  // under the sums of block b
             if (kMany) __builtin_amdgcn_sched_barrier(0);
-            if (!kMany) x[b] = xq[next + b];
+            if (!kMany) fetch_x(b, next + b);
             // register 4 g + j: row 8 g + 4 lh + j of x
 #pragma unroll
             for (int g = 0; g < kSums / 4; g++) {
-                const f32x4 dx = *(const f32x4*)(dxs + b * XR + 8 * g + 4 * lh);
+                const f32x4 dx = *(const f32x4*)(dxs + b * XR + (FOUR ? 0 : 8 * g) + 4 * lh);
+                if (FOUR) {  // register 4 l + j: sum l of row 4 lh + j
+#pragma clang fp contract(off)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float dd = dw * dx[j], t = dd * (float)c[4 * g + j];
+                        acc[4 * g + j] = acc[4 * g + j] + t;
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int j = 0; j < 4; j++) part[4 * g + j] = b == 0 ? dw * dx[j] * (float)c[4 * g + j] : fmaf(dw * dx[j], (float)c[4 * g + j], part[4 * g + j]);
             }
             c = c_next;
             dw = dw_next;
         }
+        if constexpr (FOUR && AHEAD) {  // the next run's loads are under way by here: the compiler issues them where they are used otherwise
+#pragma unroll
+            for (int i = 0; i < kLoads; i++) asm volatile("" : "+v"(w[i]));
+#pragma unroll
+            for (int b = 0; b < kRunBlocks; b++) asm volatile("" : "+v"(kept[b]));
+        }
+        if (FOUR) continue;
 #pragma unroll
         for (int i = 0; i < kSums; i++) acc[i] += part[i];
         if ((run / WAVES) % kRunsTogether == kRunsTogether - 1) {
@@ -190,19 +223,25 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows ? 2 : 4) void qgemv_q8_
             }
         }
     }
+    if (!FOUR) {
 #pragma unroll
-    for (int i = 0; i < kSums; i++) acc[i] += total[i];
+        for (int i = 0; i < kSums; i++) acc[i] += total[i];
+    }
 
     __syncthreads();  // every wavefront is done with its slab
     float* red = (float*)smem;  // [wave][sum][lane]
 #pragma unroll
     for (int i = 0; i < kSums; i++) red[(wave * kSums + i) * 64 + lane] = acc[i];
     __syncthreads();
-    // the wavefronts share the sums
-    for (int s = wave; s < kSums; s += WAVES) {
+    auto sum_of = [&](int s) {
         float v = red[s * 64 + lane];
 #pragma unroll
         for (int o = 1; o < WAVES; o++) v = v + red[(o * kSums + s) * 64 + lane];
+        return v;
+    };
+    // the wavefronts share the sums
+    for (int s = wave; s < (FOUR ? 4 : kSums); s += WAVES) {
+        const float v = FOUR ? (sum_of(s) + sum_of(8 + s)) + (sum_of(4 + s) + sum_of(12 + s)) : sum_of(s);
         const int m = 8 * (s >> 2) + 4 * lh + (s & 3);
         if (n < N && m < M) y[(int64_t)m * N + n] = v;
     }
@@ -233,15 +272,15 @@ bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
     return a.N * a.K >= ((int64_t)32 << 20) && a.N >= (a.M >= 4 ? 4096 : 6144);
 }
 
-template <int XR, int WAVES>
+template <int XR, int WAVES, bool FOUR = false, bool AHEAD = false>
 static hipError_t launch(const QGemvArgs& a, int64_t wgs, hipStream_t st) {
     constexpr int kLds = WAVES * kWaveLds<XR>;
     static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
     if (kLds > 64 * 1024 && !raised) {
-        if (hipError_t e = hipFuncSetAttribute((const void*)qgemv_q8_0_mfma_kernel<XR, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
+        if (hipError_t e = hipFuncSetAttribute((const void*)qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
         raised = true;
     }
-    hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y,
+    hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y,
                        (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K));
     return hipGetLastError();
 }
@@ -252,6 +291,9 @@ hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st) {
     const int rows = a.M > kFewRows ? kManyRows : 8;
     const int64_t wgs = ((a.N + 31) / 32) * ((a.M + rows - 1) / rows);
     if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+    // from 64 M weights on, of whole runs: sums in the order in which they always were
+    if (a.M <= kFewRows && a.N * a.K >= ((int64_t)64 << 20) && a.K % 256 == 0 && ((uintptr_t)a.W & 15) == 0)
+        return wgs <= 512 ? launch<8, 4, true, true>(a, wgs, st) : launch<8, 4, true>(a, wgs, st);
     if (rows == 8) return wgs <= 512 ? launch<8, 8>(a, wgs, st) : launch<8, 4>(a, wgs, st);
     return wgs <= 256 ? launch<kManyRows, 8>(a, wgs, st) : launch<kManyRows, 4>(a, wgs, st);
 }

@@ -639,6 +639,46 @@ def test_q8_0_products_of_any_rows_on_the_matrix_cores(m, n, k, offset):
     assert np.all(np.abs(got - exact) <= steps @ w.reshape(n, -1, 32).sum(2).T + sums)
 
 
+@pytest.mark.parametrize("m,n,k", [(2, 16400, 4096), (5, 13131, 5120), (8, 4700, 14336), (3, 8200, 8192)])
+def test_q8_0_few_rows_by_the_largest_matrices_bit_for_bit(m, n, k):
+    """Two to eight rows by 64 M weights and more, whole runs of eight blocks: the CPU's four sums a block, each times the product of the scales, a multiply
+    and an add; four wavefronts take the runs in turn, and their sums are added in order, then (0 + 2) + (1 + 3)."""
+    rng = np.random.default_rng(m + n + k)
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    gpu.say(f"q8_0 four sums a block M={m} N={n} K={k}")
+    got = gpu.qgemv(O.Q8_0, ptr, gpu.dev(x), n, k)
+    some = np.unique(np.concatenate([np.arange(0, n, 97), [n - 1]]))
+    w = raw.reshape(n, k // 32, 34)[some]
+    xq = np.stack([O.quantize_row(r, 32, False).reshape(-1, 36) for r in x])
+    dw, dx = O.f16_to_f32(w[..., :2].copy().view(np.uint16)[..., 0]), xq[..., :4].copy().view(np.float32)[..., 0]
+    qw, qx = (q.view(np.int8).astype(np.int32) for q in (w[..., 2:].copy(), xq[..., 4:].copy()))
+    sums = np.zeros((4, m, some.size, 4), np.float32)  # [wavefront][row of x][row of W][sum]: value 4 i + j of a block is of sum i % 4
+    for b in range(k // 32):
+        of = b // 8 % 4
+        c = np.einsum("migj,nigj->mng", qx[:, b].reshape(m, 2, 4, 4), qw[:, b].reshape(-1, 2, 4, 4)).astype(np.float32)
+        sums[of] = sums[of] + (dw[:, b] * dx[:, b, None])[..., None] * c
+    v = ((sums[0] + sums[1]) + sums[2]) + sums[3]
+    assert bits_equal(got[:, some], (v[..., 0] + v[..., 2]) + (v[..., 1] + v[..., 3]))
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 16500, 2080), (9, 4097, 288), (64, 1000, 4064)])
+def test_q8_0_a_block_with_an_infinity_that_a_ragged_rows_last_run_reads_twice(m, n, k):
+    """The last run of a row of no whole runs reaches back over blocks that it counts for nought: an infinity there makes its row what the CPU makes of it, and no other."""
+    rng = np.random.default_rng(m + n + k)
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    gpu.say(f"q8_0 infinity in blocks read twice M={m} N={n} K={k}")
+    clean = gpu.qgemv(O.Q8_0, ptr, gpu.dev(x), n, k)
+    x[1, -256] = np.inf  # the last run's first block
+    got = gpu.qgemv(O.Q8_0, ptr, gpu.dev(x), n, k)
+    want = O.qmatmul(O.Q8_0, raw, x[1:2], n, k)[0]
+    assert np.array_equal(np.isnan(got[1]), np.isnan(want)) and np.array_equal(np.isinf(got[1]), np.isinf(want)) and not np.isfinite(want).any()
+    assert bits_equal(np.delete(got, 1, 0), np.delete(clean, 1, 0))
+
+
 # ---- Q4_K / Q6_K -------------------------------------------------------------
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])

@@ -262,43 +262,56 @@ __global__ __launch_bounds__(64 * WAVES, (sizeof(KV) == 4 && D == 128 && WAVES =
     rows_by_float32<KV, D, WAVES, WAVES * kRows>(q, k, v, out, lse, p, blockIdx.y, blockIdx.x, (int)(gridDim.z - 1 - blockIdx.z) * WAVES * kRows, ks, vs, vbad);
 }
 
-// The same for keys and values in binary16, by sums of products of 16-bit parts that are exact, on instructions sixteen times as fast as the float32 one:
-//   - scores: keys are binary16 as they are, a row of Q is a pair, q 2^-e = a0 + 2^-11 a1 with a0 the binary16 next to it and a1 the one next to 2^11 times what
-//     that leaves, and 2^e such that the row's largest element lies in [2^14, 2^15); the pair's products go into sums of their own. An element down to 2^-27 of the
-//     largest is held to 23 bits.
-//   - result: a weight is three bfloat16 (24 bits, whatever its size down to e^-75), a value two (its 11 bits); of the six products the one of both
-//     lowest parts, below 2^-26 of the whole, is left out.
-// A workgroup that finds a NaN or an infinity among its keys and values, or an element of Q other than zero below 2^-27 of its row's largest, or a row
-// whose largest is beyond 2^100 or below 2^-100, starts anew with rows_by_float32.
-// The MFMAs of a tile of 32 rows by 32 keys at 128 features are 1792 cycles where those on float32 operands are 8192. Against 64 bits the
-// results' error is 0.4 to 0.65 of what it was with float32 operands (1.7e-7 for 3.4e-7 over 512 normal keys, 3.0e-7 for 4.6e-7 over 2048, 5.6e-7 for 1.2e-6 with scores four times as far apart).
+// The same for keys and values in binary16, whose products it makes of bfloat16 parts that add up to their factors, exactly, on instructions sixteen times
+// as fast as the float32 one. A key or a value is two (its 11 bits), an element of a row of Q and a weight three (24 bits), and a product is the six of
+// theirs: what differs is the order of the float32 sums. Keys are not taken as the binary16 they are: an MFMA cuts its sums off by the exponents of their
+// terms, and counts a subnormal's as 2^-14, which is up to 2^-15 of a score of subnormal keys.
+//   - scores: a row of Q is scaled by a power of two that takes its largest element to [2^14, 2^15); the products of the upper parts have a sum of their own.
+//   - result: weights are 2^64 times what they are, so that the parts of all that a float32 holds are normal numbers.
+// A workgroup that finds a NaN or an infinity among its keys and values, or a row of Q with an element other than zero below 2^-114 of its largest, or with a
+// largest beyond 2^100 or below 2^-100, starts anew with rows_by_float32 (a layer of 512 rows then takes 98 us, or 126 with an infinity in the last key, for 89 with
+// float32 operands alone; of 2048 rows 451, or 580, for 450).
+// Against 64 bits the results' error is 0.4 to 0.65 of what it is with float32 operands (1.5e-7 for 3.4e-7 over 512 normal keys, 2.9e-7 for 4.6e-7
+// over 2048, 5.2e-7 for 1.2e-6 with scores four times as far apart).
 //
 // LDS holds a tile's keys row by row, sixteen-byte pieces turned by the row so that 32 rows' equal piece falls on all banks, and its values
 // transposed, a feature's 32 keys in the order in which a lane holds its scores (keys 16 u + 8 a + 4 hi + c at 16 u + 8 hi +
 // 4 a + c), so that a lane's weights go from the exponential into the second operand; two neighbouring keys' values
-// meet in one dword on the way in.
+// meet in one dword on the way in. The third parts of Q are there too.
 //
-// What bounds it is a wavefront's chain: some 650 vector instructions a tile (exponentials, masks, parts, staging: 2600 cycles) and the
-// MFMAs' 1792, and a causal call ends with the rows that walk all keys. So a workgroup is four
+// What bounds it is a wavefront's chain: some 750 vector instructions a tile (exponentials, masks, parts, staging: 3000 cycles) and the
+// 96 MFMAs' 3072 (those on float32 operands would be 8192), and a causal call ends with the rows that walk all keys. So a workgroup is four
 // wavefronts of 32 rows each only where there are many (KS = 1), and otherwise (KS = 2) two pairs of wavefronts, 32 rows a pair, that
 // take a step's two tiles of keys, one each, and join their maxima, sums and results through LDS at the end: half the chain.
 // One layer of 32 heads of 128 features over 8 key heads, us:
 //   rows, keys            float32 operands   KS = 1   KS = 2
-//   512                         89.6           49.7    36.7
-//   2048                       458            203       210
-//   5 prompts of 131            35.9           27.2    23.0
-//   8 prompts of 512           201            103       127
-//   8 heads, 512 of 2048       325             163    106
+//   512                         91             65       45
+//   2048                       455            276      272
+//   5 prompts of 131            35             32       27
+//   8 prompts of 512           200            132      159
+//   8 heads, 512 of 2048       326            218      137
 
-// e^x for x <= 0, and for NaN: 2^t with t the float32 next to x / ln 2, times 1 + ln 2 (x / ln 2 - t). Nine instructions where
-// the general function, which has overflow and subnormal results to care for, takes fifteen; a result below 2^-126 is zero here.
+constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = (float)(1.4426950408889634074 - (double)kLog2e), kLn2 = 0.6931471805599453f;
+
+// 2^up e^x for x <= 0, and for NaN: 2^t with t the float32 next to x / ln 2, times 1 + ln 2 (x / ln 2 - t). Ten instructions where
+// the general function, which has overflow to care for, takes fifteen. Not for t below -126, whose 2^t is no normal number.
+template <int UP>
 __device__ __forceinline__ float exp_down(float x) {
-    constexpr float kLog2e = 1.4426950408889634f, kLog2eLow = (float)(1.4426950408889634074 - (double)kLog2e), kLn2 = 0.6931471805599453f;
-    const float t = x * kLog2e, y = __builtin_amdgcn_exp2f(t);
+    const float t = x * kLog2e, y = __builtin_ldexpf(__builtin_amdgcn_exp2f(t), UP);
     const float held = fmaxf(x, -128.f), th = held * kLog2e;  // an infinity leaves nothing to mend
     const float rest = __builtin_fmaf(held, kLog2eLow, __builtin_fmaf(held, kLog2e, -th));
     return __builtin_fmaf(y, rest * kLn2, y);
 }
+
+// The same for UP = 64 and any x down to where 2^64 e^x is no normal number any more.
+__device__ __forceinline__ float exp_far_down(float x) {
+    const float t = x * kLog2e, lift = t < -64.f ? 64.f : 0.f, y = __builtin_ldexpf(__builtin_amdgcn_exp2f(t + lift), 64 - (int)lift);  // t + 64 is exact there
+    const float held = fmaxf(x, -128.f), th = held * kLog2e;
+    const float rest = __builtin_fmaf(held, kLog2eLow, __builtin_fmaf(held, kLog2e, -th));
+    return __builtin_fmaf(y, rest * kLn2, y);
+}
+
+constexpr float kFar = -80.f;  // e^x of an x above is far from subnormal
 
 template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
@@ -308,14 +321,21 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
     constexpr int PER = D / 8, PD = PER / 2;   // elements, dwords of a key (value) row a thread loads: eight threads a row, a row of each tile
     constexpr int G = 4 / KS;                  // groups of 32 query rows a workgroup
     constexpr int kStep = kTile * KS;          // keys a step
+    constexpr int kOwn = KS > 1 && D == 128 ? 1 : 0;  // steps whose third part of Q stays in registers: the LDS has no room for it
     __shared__ union Lds {
-        uint16_t kv[3][KS][kTile * D];         // the step's keys, its values' upper and lower parts
-        float results[KS > 1 ? G : 1][16 * NT * 64];
+        struct {
+            uint16_t kv[4][KS][kTile * D];     // upper and lower parts of the step's keys and of its values
+            bf16x8 q2[G][NS - kOwn][64];       // the third part of a group's rows, a lane's eight features of each step of the scores' product
+        };
+        struct {
+            float results[KS > 1 ? G : 1][16 * NT * 64];
+            float ml[KS > 1 ? G : 1][2][64];   // maximum and sum of the rows' second half of the keys
+        };
         Float32Lds<D> by_float32;
     } lds;
+    static_assert(sizeof(Lds) + 64 <= 80 * 1024, "two workgroups a compute unit");
     __shared__ int odd;                        // whether the products of float32 operands are to be taken
-    __shared__ float ml[KS > 1 ? G : 1][2][64];  // maximum and sum of the rows' second half of the keys
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, hi = lane >> 5, part = wave % KS;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r32 = lane & 31, hi = lane >> 5, half = wave % KS;
     const int b = blockIdx.y, h = blockIdx.x, hk = h / (p.H / p.HK), bx = (int)(gridDim.z - 1 - blockIdx.z);  // the last rows first
     const int i0 = (bx * G + wave / KS) * kRows;
     const int64_t Kt = p.K;
@@ -337,8 +357,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
     if (tid == 0) odd = 0;
     __syncthreads();
 
-    // this lane's row, scaled: features 16 s + 8 hi .. + 8 of step s as the second operand's pair
-    f16x8 q0[NS], q1[NS];
+    // this lane's row, scaled: features 16 s + 8 hi .. + 8 of step s as the second operand's parts
+    bf16x8 q0[NS], q1[NS], q2_own[kOwn ? kOwn : 1];
     float up = 1.f;  // 2^e
     {
         const float* qr = q + b * p.q_b + (int64_t)h * p.q_h + (int64_t)(row < p.Q ? row : p.Q - 1) * p.q_i + 8 * hi;
@@ -348,19 +368,35 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
 #pragma unroll
             for (int c = 0; c < 8; c++) amax = fmaxf(amax, __builtin_fabsf(qr[16 * s + c] * p.scale));
         amax = fmaxf(amax, other_half(amax, lane));
-        bool far = amax != 0.f && !(amax > 0x1p-100f && amax < 0x1p100f);
-        const int e = far || amax == 0.f ? 0 : __builtin_amdgcn_frexp_expf(amax) - 15;
+        bool odd_row = amax != 0.f && !(amax > 0x1p-100f && amax < 0x1p100f);
+        asm volatile("" ::: "memory");  // the row is read again, not kept
+        const int e = odd_row || amax == 0.f ? 0 : __builtin_amdgcn_frexp_expf(amax) - 15;
         up = __builtin_ldexpf(1.f, e);
 #pragma unroll
-        for (int s = 0; s < NS; s++)
+        for (int s = 0; s < NS; s++) {
+            u32x4 part[3];
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const float x = qr[16 * s + c] * p.scale, a = __builtin_ldexpf(x, -e);
-                far = far || !(x == 0.f || __builtin_fabsf(a) >= 0x1p-13f);
-                q0[s][c] = (_Float16)a;
-                q1[s][c] = (_Float16)((a - (float)q0[s][c]) * 2048.f);
+            for (int i = 0; i < 4; i++) {
+                float a[2];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const float x = qr[16 * s + 2 * i + j] * p.scale;
+                    a[j] = __builtin_ldexpf(x, -e);
+                    odd_row |= !(x == 0.f || __builtin_fabsf(a[j]) >= 0x1p-100f);
+                }
+#pragma unroll
+                for (int n = 0; n < 3; n++) {
+                    part[n][i] = pack_bf16(a[0], a[1]);
+                    a[0] -= bf16_lo(part[n][i]);
+                    a[1] -= bf16_hi(part[n][i]);
+                }
             }
-        if (__builtin_amdgcn_ballot_w64(far) != 0 && lane == 0) odd = 1;
+            q0[s] = __builtin_bit_cast(bf16x8, part[0]);
+            q1[s] = __builtin_bit_cast(bf16x8, part[1]);
+            if (s < kOwn) q2_own[s] = __builtin_bit_cast(bf16x8, part[2]);
+            else if (KS == 1 || half == 0) lds.q2[wave / KS][s - kOwn][lane] = __builtin_bit_cast(bf16x8, part[2]);  // the pair's rows are the same
+        }
+        if (__builtin_amdgcn_ballot_w64(odd_row) != 0 && lane == 0) odd = 1;
     }
     float m = -__builtin_inff(), l = 0.f;  // the row's maximum so far; the sum over the keys this half of the lanes holds
     f32x16 o[NT], zero;                    // the row's result, transposed: register e of tile t is feature 32 t + 8 (e / 4) + 4 hi + e % 4
@@ -394,10 +430,22 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
         f16x2 chk = none;  // 0 * each summed: NaN as soon as one is a NaN or an infinity
 #pragma unroll
         for (int n = 0; n < KS; n++) {
-            uint16_t *ks = lds.kv[0][n], *vh = lds.kv[1][n], *vl = lds.kv[2][n];
+            uint16_t *kh = lds.kv[0][n], *kl = lds.kv[1][n], *vh = lds.kv[2][n], *vl = lds.kv[3][n];
             const int r = lrow;
 #pragma unroll
-            for (int c = 0; c < PD / 4; c++) *(u32x4*)(ks + r * D + key_piece(r, lpart * (PD / 4) + c) * 8) = kreg[n][c];
+            for (int c = 0; c < PD / 4; c++) {
+                u32x4 upper, lower;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const f16x2 two = as_f16x2(kreg[n][c][i]);
+                    const float f0 = (float)two[0], f1 = (float)two[1];
+                    upper[i] = pack_bf16(f0, f1);
+                    lower[i] = pack_bf16(f0 - bf16_lo(upper[i]), f1 - bf16_hi(upper[i]));
+                }
+                const int at = r * D + key_piece(r, lpart * (PD / 4) + c) * 8;
+                *(u32x4*)(kh + at) = upper;
+                *(u32x4*)(kl + at) = lower;
+            }
             // the thread eight lanes on has the neighbouring key's same features: of two features, the even key's thread stores the first's two keys
             const int odd = r & 1, slot = slot_of(r & ~1);
 #pragma unroll
@@ -419,11 +467,12 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
         if (__builtin_amdgcn_ballot_w64(bad != bad) != 0 && lane == 0) odd = 1;
     };
 
-    const uint16_t *ks = lds.kv[0][part], *vh = lds.kv[1][part], *vl = lds.kv[2][part];
+    const bf16x8* q2 = &lds.q2[wave / KS][0][lane];
+    const uint16_t *kh = lds.kv[0][half], *kl = lds.kv[1][half], *vh = lds.kv[2][half], *vl = lds.kv[3][half];
     if (seen_wg > 0) fetch(0);
     bool by_float32 = false;
     for (int jw = 0; jw < seen_wg; jw += kStep) {
-        const int j0 = jw + kTile * part;
+        const int j0 = jw + kTile * half;
         __syncthreads();  // everyone has read the tiles before
         stage();
         __syncthreads();
@@ -436,18 +485,24 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
         const bool whole = j0 + kTile <= seen_first;
 
         // scores, transposed (K . Q^T): register e is 2^-e of key j0 + 8 (e / 4) + 4 hi + e % 4 against this lane's row
-        f32x16 s = zero, s1 = zero;
+        f32x16 s = zero, s1 = zero;  // of the upper parts, of the five others
         int k0 = r32 * D + key_piece(r32, hi) * 8;
         asm volatile("" : "+v"(k0));  // eight addresses worked out again for each tile instead of eight registers
 #pragma unroll
         for (int f = 0; f < NS; f++) {
-            const f16x8 kf = *(const f16x8*)(ks + (k0 ^ 16 * f));
-            s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q1[f], s1, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, q0[f], s, 0, 0, 0);
+            const bf16x8 h8 = *(const bf16x8*)(kh + (k0 ^ 16 * f)), l8 = *(const bf16x8*)(kl + (k0 ^ 16 * f)), q2f = f < kOwn ? q2_own[f < kOwn ? f : 0] : q2[(f - kOwn) * 64];
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, q2f, s1, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, q1[f], s1, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, q2f, s1, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, q0[f], s1, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, q1[f], s1, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, q0[f], s, 0, 0, 0);
         }
 #pragma unroll
-        for (int e = 0; e < 16; e++) s[e] = __builtin_fmaf(s1[e], 1.f / 2048.f, s[e]);
-        float mx = -__builtin_inff();
+        for (int e = 0; e < 16; e++) s[e] = s[e] + s1[e];
+        float mx = -__builtin_inff(), least = s[0];
+#pragma unroll
+        for (int e = 1; e < 16; e++) least = fminf(least, s[e]);
         if (!whole) {
 #pragma unroll
             for (int e = 0; e < 16; e++) s[e] = 8 * (e >> 2) + (e & 3) < seen - j0 - 4 * hi ? s[e] : -__builtin_inff();
@@ -456,25 +511,38 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
         for (int e = 0; e < 16; e++) mx = fmaxf(mx, s[e]);
         mx = fmaxf(mx, other_half(mx, lane)) * up;
         const float mn = fmaxf(m, mx);
-        float al = 1.f, sum = 0.f;
-        if (mn > -__builtin_inff()) {  // the row has seen a key by now
-            al = exp_down(m - mn);
+        const bool any = mn > -__builtin_inff();  // the row has seen a key by now
+        float sum = 0.f;
+        if (__builtin_amdgcn_ballot_w64(any && __builtin_fmaf(least, up, -mn) < kFar) == 0) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                s[e] = exp_down(__builtin_fmaf(s[e], up, -mn));
-                sum += s[e];
-            }
-        } else {
-            s = zero;
+            for (int e = 0; e < 16; e++) s[e] = exp_down<64>(__builtin_fmaf(s[e], up, -mn));
+        } else {  // seldom
+#pragma unroll
+            for (int e = 0; e < 16; e++) s[e] = exp_far_down(__builtin_fmaf(s[e], up, -mn));
         }
-        l = l * al + sum;
+        if (!any) s = zero;
+#pragma unroll
+        for (int e = 0; e < 16; e++) sum += s[e];
+        // in two factors where the first maximum is far below
+        const float down = any ? m - mn : 0.f, down0 = fmaxf(down, kFar), down1 = down - down0;
+        const float al = exp_down<0>(down0);
         m = mn;
+        l = l * al;
         if (__builtin_amdgcn_ballot_w64(al != 1.f) != 0) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * al;
+            if (__builtin_amdgcn_ballot_w64(down1 != 0.f) != 0) {
+                const float al1 = exp_down<0>(fmaxf(down1, kFar));
+                l = l * al1;
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * al1;
+            }
         }
+        l = l + sum;
         bf16x8 p0[2], p1[2], p2[2];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
@@ -496,6 +564,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
             for (int u = 0; u < 2; u++) {
                 const int at = value_at(32 * t + r32, 16 * u + 8 * hi);
                 const bf16x8 h8 = *(const bf16x8*)(vh + at), l8 = *(const bf16x8*)(vl + at);
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, p2[u], o[t], 0, 0, 0);
                 o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, p1[u], o[t], 0, 0, 0);
                 o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h8, p2[u], o[t], 0, 0, 0);
                 o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l8, p0[u], o[t], 0, 0, 0);
@@ -515,24 +584,25 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
     if (KS > 1) {  // the second wavefront's half of the keys joins the first's
         float* theirs = lds.results[wave / KS] + lane;
         __syncthreads();
-        if (part == 1) {
+        if (half == 1) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int e = 0; e < 16; e++) theirs[64 * (16 * t + e)] = o[t][e];
-            ml[wave / KS][0][lane] = m;
-            ml[wave / KS][1][lane] = l;
+            lds.ml[wave / KS][0][lane] = m;
+            lds.ml[wave / KS][1][lane] = l;
         }
         __syncthreads();
-        if (part == 1) return;
-        const float m1 = ml[wave / KS][0][lane], l1 = ml[wave / KS][1][lane], mn = fmaxf(m, m1);
-        const float a0 = m == mn ? 1.f : exp_down(m - mn), a1 = m1 == mn ? 1.f : exp_down(m1 - mn);
-        l = l * a0 + l1 * a1;
+        if (half == 1) return;
+        const float m1 = lds.ml[wave / KS][0][lane], l1 = lds.ml[wave / KS][1][lane], mn = fmaxf(m, m1);
+        const float d0 = m == mn ? 0.f : m - mn, d1 = m1 == mn ? 0.f : m1 - mn, a0 = exp_down<0>(fmaxf(d0, kFar)), a1 = exp_down<0>(fmaxf(d1, kFar));
+        const float b0 = exp_down<0>(fmaxf(d0 - fmaxf(d0, kFar), kFar)), b1 = exp_down<0>(fmaxf(d1 - fmaxf(d1, kFar), kFar));
+        l = l * a0 * b0 + l1 * a1 * b1;
         m = mn;
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * a0 + theirs[64 * (16 * t + e)] * a1;
+            for (int e = 0; e < 16; e++) o[t][e] = o[t][e] * a0 * b0 + theirs[64 * (16 * t + e)] * a1 * b1;
     }
     if (row >= p.Q) return;
     float* orow = out + b * p.o_b + (int64_t)h * p.o_h + (int64_t)row * p.o_i;
@@ -551,7 +621,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_half_kernel(const float* _
 #pragma unroll
                 for (int c = 0; c < 4; c++) dst[c] = r[c];
         }
-    if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(l);
+    if (lse && hi == 0) lse[((int64_t)b * p.H + h) * p.Q + row] = l == 0.f ? -__builtin_inff() : m + __builtin_logf(__builtin_ldexpf(l, -64));
 }
 
 std::atomic<int> g_prompt{1};  // measurement aid: 0 keeps every call on the kernel that takes a query row a workgroup, 2 those over binary16 on float32 operands

@@ -121,26 +121,92 @@ def check_rows(q, k, v, bound):
     got, _ = T.attention(q, k, v, 1.0, causal=False, kv_dt=capi.F16)
     assert T.last_kernel() == "attn_prompt_kernel"
     want = exact(q, k, v, 1.0, k.shape[2])  # an offset that hides no key
-    err = np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1))
-    assert err.max() <= bound, err.max()
+    err = max_row_error(got, want)
+    assert err <= bound, err
 
 
-@pytest.mark.parametrize("B,H,Q,D,ratio", [
-    (4, 32, 449, 128, 2.0 ** -27), (4, 32, 449, 128, 2.0 ** -40),  # workgroups of 128 rows: a pair of binary16 holds the small feature to its last bit but one; products of float32
-    (1, 4, 100, 128, 2.0 ** -27), (1, 4, 100, 128, 2.0 ** -29), (1, 4, 100, 64, 2.0 ** -29),  # workgroups of 64
+def parts_of(q, scale, n):
+    """Rows of Q as the sum of n binary16 each, the row's largest element in [2^14, 2^15) and each part 2^11 times what the ones ahead of it leave."""
+    x = q * np.float32(scale)
+    up = 2.0 ** (np.frexp(np.abs(x).max(-1, keepdims=True).astype(np.float64))[1] - 15)
+    rest, held = x / up, 0
+    for i in range(n):
+        part = rest.astype(np.float16).astype(np.float64)
+        held, rest = held + part * 2.0 ** (-11 * i), (rest - part) * 2048
+    return held * up / scale
+
+
+@pytest.mark.parametrize("B,H,Q,D,ratio,short", [
+    (4, 32, 449, 128, 2.0 ** -27, 1), (4, 32, 449, 128, 2.0 ** -50, 3),   # workgroups of 128 rows
+    (4, 32, 449, 128, 2.0 ** -120, 3),                                    # the largest is beyond 2^100: products of float32 operands
+    (1, 4, 100, 128, 2.0 ** -36, 2), (1, 4, 100, 128, 2.0 ** -110, 3), (1, 4, 100, 128, 2.0 ** -120, 3), (1, 4, 100, 64, 2.0 ** -120, 3),  # workgroups of 64
 ])
-def test_a_row_whose_features_lie_far_apart(B, H, Q, D, ratio):
-    """One row of one sequence has a largest feature that meets keys of zero and one `ratio` of it that meets large keys: that row and those that share
-    its workgroup are within float32's rounding (scores up to about 5, weights to 5 x 2^-24, some 3e-7) of 64 bits, as all others are."""
+def test_a_row_whose_features_lie_far_apart(B, H, Q, D, ratio, short):
+    """One row of one sequence has a largest feature that meets keys of zero and one `ratio` of it whose products are scores of some units: that row and
+    those that share its workgroup are within float32's rounding (scores up to about 8, weights to 8 x 2^-24, some 5e-7) of 64 bits, as all others are.
+    With the row as `short` binary16 parts under one exponent it would be off by more than four times the bound."""
     rng = np.random.default_rng(Q + D)
-    q = rng.normal(size=(B, H, Q, D)).astype(np.float32); q[..., :2] = 0
+    scale = np.float32(2.0 ** -27 / ratio)
+    q = (rng.normal(size=(B, H, Q, D)) / np.sqrt(D) / scale).astype(np.float32); q[..., :2] = 0
     q[0, :, 70, 0] = 2.0 ** 13; q[0, :, 70, 1] = np.float32(1.2345678 * 2.0 ** 13 * ratio)
     k, v = (rng.normal(size=(B, 2, Q, D)).astype(np.float32) for _ in range(2))
     k[..., 0] = 0; k[..., 1] = np.clip(k[..., 1], -3, 3) * 2.0 ** 14
     k, v = T.O.f32_to_f16(k).view(np.uint16), T.O.f32_to_f16(v).view(np.uint16)
+    want = exact(q, k, v, float(scale), 0)
+    less = q[:1].astype(np.float64)
+    less[0, :, 70] = parts_of(q[0, :, 70], scale, short)
+    assert max_row_error(exact(less, k[:1], v[:1], float(scale), 0)[:, :, 70:71], want[:1, :, 70:71]) > 8e-6
     T.gpu.say(f"attention over binary16, features {ratio} apart, B={B} Q={Q} D={D}")
-    got, _ = T.attention(q, k, v, 1 / np.sqrt(D), causal=True, offset=0, kv_dt=capi.F16)
+    got, _ = T.attention(q, k, v, float(scale), causal=True, offset=0, kv_dt=capi.F16)
     assert T.last_kernel() == "attn_prompt_kernel"
-    want = exact(q, k, v, 1 / np.sqrt(D), 0)
-    err = np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1))
-    assert err.max() <= 2e-6, err.max()
+    err = max_row_error(got, want)
+    assert err <= 2e-6, err
+
+
+def max_row_error(got, want):
+    return np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1)).max()
+
+
+@pytest.mark.parametrize("B,H,Q,D", [(1, 2, 64, 128), (1, 2, 64, 64), (4, 32, 449, 128)])
+def test_a_row_of_q_keeps_its_last_bits(B, H, Q, D):
+    """Scores of some units that are the difference of two products 2^12 times as large, exact in float32: a feature of Q that lost the last of its 24 bits
+    would move them by 2^-12. The results' error is the weights', a few 2^-24."""
+    rng = np.random.default_rng(D)
+    q = np.zeros((B, H, Q, D), np.float32)
+    q[..., 0] = rng.uniform(1, 2, (B, H, Q)).astype(np.float32)
+    q[..., 1] = q[..., 0].astype(np.float16)
+    k = np.zeros((B, 1, Q, D), np.float32)
+    k[..., 0] = rng.integers(-2, 3, (B, 1, Q)) * 4096.0; k[..., 1] = -k[..., 0]
+    k, v = (T.O.f32_to_f16(x).view(np.uint16) for x in (k, rng.normal(size=(B, 1, Q, D)).astype(np.float32)))
+    T.gpu.say(f"attention over binary16, last bits of Q, B={B} Q={Q} D={D}")
+    got, _ = T.attention(q, k, v, 1.0, causal=False, kv_dt=capi.F16)
+    assert T.last_kernel() == "attn_prompt_kernel"
+    err = max_row_error(got, exact(q, k, v, 1.0, Q))
+    assert err <= 1e-6, err
+
+
+@pytest.mark.parametrize("D,K,low", [(64, 64, 75), (128, 64, 75), (128, 64, 86), (128, 100, 75)])
+def test_weights_far_below_one(D, K, low):
+    """The key of weight 1 has values of zero, the others' weights of e^-low down to e^-95 (below 2^-126, the smallest normal number, from e^-87.4 on) decide
+    the results. Scores are exact: what remains is the exponential's error and the sums'. The first key is the last of the tiles that a wavefront takes, or the first,
+    so that what came before it is scaled down by as much."""
+    rng = np.random.default_rng(K)
+    q = np.zeros((1, 1, 64, D), np.float32); q[..., 0] = 1
+    v = (rng.uniform(0.5, 1, size=(1, 1, K, D)) * 60000).astype(np.float32)
+    for at in (0, K - 1):
+        k = np.zeros((1, 1, K, D), np.float32)
+        k[0, 0, :, 0] = -np.round(rng.uniform(low, 95, K) * 16) / 16
+        k[0, 0, at, 0] = 0
+        w = v.copy(); w[0, 0, at] = 0
+        check_rows(q, k, w, 1e-6)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("small", [2.0 ** -24, 2.0 ** -20])
+def test_subnormal_keys_and_values(small, D):
+    """All keys and values are subnormal binary16 numbers, down to the smallest. Scores of some units from all features: their rounding, 2^-24 of some 5, and that of their
+    distance from the largest, 2^-24 of some 10, make some 1e-6 of the weights."""
+    rng = np.random.default_rng(9)
+    q = (rng.normal(size=(1, 2, 64, D)) / np.sqrt(D) / (8 * small)).astype(np.float32)
+    k, v = (rng.integers(-15, 16, (1, 2, 64, D)).astype(np.float32) * np.float32(small) for _ in range(2))
+    check_rows(q, k, v, 2e-6)

@@ -72,9 +72,11 @@ __device__ __forceinline__ void split(const u32x4* v, bf16x8* parts, float) {
 // What x's parts and a block's sum do not hold. The matrix cores take subnormal operands for nought, which the lesser parts of
 // a float32 below 2^-103 are; and 32 numbers above 2^122 may add up to more than a float32 holds, where their product with the
 // scale is none. Where a float32 is below 2^-100, or a bfloat16 subnormal (other than nought; the tile kernel takes these for
-// nought too, so they are looked for in its stead only where it does not go), or a result no finite number, a workgroup goes over
-// its share again and takes each block's rows whose largest x is below 2^-60 times 2^64 (in the others what is lost is 2^-66 of
-// the largest), from 2^100 on times 2^-64.
+// nought too, so they are looked for in its stead only where it does not go), or a result no finite number, a workgroup reads such rows
+// of x again, and if one has a block whose largest x is below 2^-60 (in the others what is lost is 2^-66 of
+// the largest), or a finite x from 2^100 on, it goes over its share again and takes the former times 2^64, the latter times 2^-64. Rows with a
+// NaN or an infinity, and products that no float32 holds, are what they are the first time (us without, with a NaN in one row, and when it went over all of it again:
+// bfloat16 16 x 4096 x 4096 10.2, 13.5, 28; 128 x 14336 x 4096 63, 68, 149; float32 128 x 4096 x 4064 32, 34, 61).
 constexpr uint32_t kTiny = ((127u - 100u) << 24) - 1;
 __device__ __forceinline__ void note_least(const u32x4 (*v)[2], uint32_t* least) {
 #pragma unroll
@@ -95,6 +97,42 @@ __device__ __forceinline__ void note_least(const u32x4 (*v)[1], uint32_t* least)
 }
 __device__ __forceinline__ bool tiny(uint32_t least, float) { return least < kTiny; }
 __device__ __forceinline__ bool tiny(uint32_t least, __bf16) { return (least & 0xffffu) < 0x7f || (least >> 16) < 0x7f; }
+
+// Whether any of the rows in `rows` has what is to be gone over again: pieces of sixteen bytes, a thread each, a block's to neighbours.
+template <typename X>
+__device__ __forceinline__ bool needs_suit(const X* x, int64_t x_row_stride, uint32_t rows, int K, bool small_too, int tid) {
+    constexpr int kPer = 16 / sizeof(X), kTogether = 4;
+    const int pieces = K / kPer;
+    bool need = false;
+    for (int p = tid; rows != 0;) {
+        u32x4 v[kTogether];
+#pragma unroll
+        for (int u = 0; u < kTogether; u++) {
+            while (p >= pieces && rows != 0) p -= pieces, rows &= rows - 1;
+            const int row = rows != 0 ? __builtin_ctz(rows) : -1;
+            v[u] = u32x4{0, 0, 0, 0};
+            if (row >= 0) v[u] = *(const u32x4*)(x + row * x_row_stride + (int64_t)kPer * p);
+            p += 64 * kWaves;
+        }
+#pragma unroll
+        for (int u = 0; u < kTogether; u++) {
+            float most = 0.f;
+#pragma unroll
+            for (int i = 0; i < kPer; i++) {
+                const float a = __builtin_fabsf(__uint_as_float(sizeof(X) == 4 ? v[u][i & 3] : i & 1 ? v[u][(i >> 1) & 3] & 0xffff0000u : v[u][(i >> 1) & 3] << 16));
+                need |= a >= 0x1p100f && a < __builtin_inff();
+                most = a > most || a != a ? a : most;
+            }
+#pragma unroll
+            for (int o = 1; o < 32 / kPer; o <<= 1) {
+                const float other = __shfl_xor(most, o);
+                most = other > most || other != other ? other : most;
+            }
+            need |= small_too && most > 0.f && most < 0x1p-60f;
+        }
+    }
+    return need;
+}
 
 // Sixteen x of a row, eight of each half of the block, by the power of two that suits it; returns what takes the row's sum back.
 __device__ __forceinline__ float factor(float most) {
@@ -297,7 +335,22 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(X) == 2 && !RAGGED ? 4 : 2) voi
 #pragma unroll
         for (int i = 0; i < 16; i++) beyond = beyond || !(__builtin_fabsf((float)acc[s][i]) < __builtin_inff());
     }
-    if (__syncthreads_or(beyond)) {  // seldom; block after block
+    bool again = false;
+    if (__syncthreads_or(beyond)) {  // seldom
+        uint32_t rows = tiny(least, X()) ? 1u << l32 : 0u;  // of x
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) rows |= __builtin_fabsf((float)acc[s][i]) < __builtin_inff() ? 0u : 1u << (8 * (i >> 2) + 4 * lh + (i & 3));
+        }
+        uint32_t* all = (uint32_t*)smem;  // every wavefront is done with its slab
+        if (tid == 0) *all = 0;
+        __syncthreads();
+        atomicOr(all, rows);
+        __syncthreads();
+        again = __syncthreads_or(needs_suit(x, x_row_stride, M < 32 ? *all & ((1u << M) - 1) : *all, 32 * nb, kP == 3 || RAGGED, tid));
+    }
+    if (again) {  // block after block
 #pragma unroll
         for (int s = 0; s < SW; s++) {
 #pragma unroll

@@ -508,3 +508,32 @@ def test_some_rows_without_a_workspace(half, m, n, k, offset):
         assert np.all((np.abs(got[some] - O.qmatmul(O.Q4_0, w, xf[some], n, k)) <= 2 * bound[at]) | ~fits[at])
     if m >= 5:
         assert not np.isfinite(got[3]).any() and np.isnan(got[4]).all()
+
+
+@pytest.mark.parametrize("half,m,n,k,bad", [(True, 40, 96, 4096, (3, 37)), (True, 33, 65, 288, (32,)), (False, 33, 1000, 1056, (7,)), (False, 64, 8200, 352, (0, 63)), (True, 16, 64, 14336, (5,))])
+def test_rows_with_an_infinity_or_a_nan_leave_the_others_sums_alone(half, m, n, k, bad):
+    """A workgroup goes over its share again, block after block, only for rows that its parts or sums do not hold: beside a row with a NaN or an infinity the
+    others' results are bit for bit what they are without it, and so beside a row of small numbers whose blocks have large ones."""
+    rng = np.random.default_rng(m + n + k)
+    w = bench_blocks(rng, O.Q4_0, n * k)
+    xf = rng.normal(size=(m, k)).astype(np.float32)
+
+    def product(x):
+        if half:
+            return qgemm(w, bf16_bits(x), n, k, capi.F32)
+        buf, ptr = gpu.dev_bytes_at(w, 0)
+        return gpu.qgemv(O.Q4_0, ptr, gpu.dev(x), n, k)
+    gpu.say(f"q4_0 without a workspace, odd rows {bad} of {m} {'bfloat16' if half else 'float32'} by {n}x{k}")
+    clean, others = product(xf), np.setdiff1d(np.arange(m), bad)
+    for odd in (np.inf, np.nan, 1e-37):
+        x = xf.copy()
+        x[list(bad), k // 2] = odd
+        got = product(x)
+        assert np.array_equal(got[others].view(np.uint32), clean[others].view(np.uint32)), odd
+        assert not np.isfinite(got[list(bad)]).any() if odd != 1e-37 else np.isfinite(got).all()
+    if half and n == 65:  # what does have to be gone over again still is
+        x = xf.copy()
+        x[bad[0], :32] = 1e38
+        want = O.bf16_to_f32(bf16_bits(x)).astype(np.float64) @ O.dequantize(O.Q4_0, w).reshape(n, k).astype(np.float64).T
+        fits = np.abs(want[bad[0]]) < 3e38
+        assert fits.any() and np.allclose(product(x)[bad[0]][fits], want[bad[0]][fits], rtol=1e-4)

@@ -114,14 +114,8 @@ unsigned die_grid(int tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
 
 template <Out KIND>
 hipError_t launch(const uint16_t* W, int64_t ldw, const uint16_t* x, int64_t ldx, int64_t M, int64_t N, int64_t K, const ProductOut& out, hipStream_t st) {
-    {
-        static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-        if (!raised) {
-            hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_kernel<ActStore<KIND>>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-            if (e != hipSuccess) return e;
-            raised = true;
-        }
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise((int)kLdsBytes, {(const void*)gemm_bf16_kernel<ActStore<KIND>>})) return e;
     const int k = (int)((K + 63) / 64 * 64);
     const void* y = out.f32 ? (const void*)out.f32 : (const void*)out.bf16;
     const ActStore<KIND> store{out, out.ld % 4 == 0 && ((uintptr_t)y & 15) == 0};

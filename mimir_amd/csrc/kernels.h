@@ -5,8 +5,27 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <atomic>
+#include <initializer_list>
+
+#include "once_a_device.h"
 
 namespace mimir {
+
+// Raises the dynamic LDS that kernels may ask for, once on every device that they are launched on: the attribute is the current device's.
+class LdsLimit {
+    OnceADevice once_;
+
+public:
+    hipError_t raise(int bytes, std::initializer_list<const void*> kernels) {
+        int device = 0;
+        if (hipError_t e = hipGetDevice(&device)) return e;
+        return once_(device, [&] {
+            for (const void* k : kernels)
+                if (hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes)) return e;
+            return hipSuccess;
+        });
+    }
+};
 
 // dtype codes: the reference's DType enumeration (backend/backend.go:72-90)
 // with Q4_0 appended, so that IsQuantized stays the range test Q8_0..Q4_0.

@@ -154,15 +154,8 @@ bool qgemm_f16_panel_pays(int64_t M, int64_t N, int64_t K) {
 
 hipError_t qgemm_f16_panel(const void* W, const void* X, int64_t x_row_stride, void* X16, float* row_scale, void* Y, int64_t M, int64_t N, int64_t K,
                            bool out_f32, void* panel, hipStream_t st) {
-    {
-        static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-        if (!raised) {
-            hipError_t e = hipFuncSetAttribute((const void*)hgemm_f16_nt_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-            if (e == hipSuccess) e = hipFuncSetAttribute((const void*)hgemm_f16_nt_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-            if (e != hipSuccess) return e;
-            raised = true;
-        }
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise((int)kLdsBytes, {(const void*)hgemm_f16_nt_kernel<true>, (const void*)hgemm_f16_nt_kernel<false>})) return e;
     const int64_t halves = N * K / 16;
     const int64_t want = (halves + 255) / 256;
     hipLaunchKernelGGL(panel_prepare_kernel, dim3((unsigned)(M + (want > 8192 ? 8192 : want))), dim3(256), 0, st, (const uint16_t*)X, (uint16_t*)X16, row_scale,

@@ -435,12 +435,8 @@ double plan(int64_t M, int64_t N, Cut* out) {
 template <int DT, bool OUT_BF16>
 hipError_t launch(const QGemvArgs& a, int nsb, hipStream_t st) {
     constexpr int kLds = Layout<256>::total > Layout<128>::total ? Layout<256>::total : Layout<128>::total;
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_kquant_kernel<DT, OUT_BF16>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise(kLds, {(const void*)qgemm_kquant_kernel<DT, OUT_BF16>})) return e;
     Cut cut;
     plan(a.M, a.N, &cut);
     const int grid = 8 * ((cut.tall_m * cut.tall_cols + 7) / 8 + (cut.short_m * (cut.cols - cut.tall_cols) + 7) / 8);

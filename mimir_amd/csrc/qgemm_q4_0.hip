@@ -473,20 +473,12 @@ hipError_t qgemm_q4_0_bf16(const void* W, const void* X, void* Y, int64_t M, int
     const int ntiles = (int)(tiles_m * tiles_n);
     dim3 grid((unsigned)(((ntiles + 7) / 8) * 8));
     const size_t lds = 2 * stage_bytes(BM, half) + (MT <= 2 || half ? 2 * kBN * 144 : 0);
-    {  // more dynamic LDS than a kernel gets by default
-        static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-        if (!raised) {
-            const int most = 160 * 1024;
-            hipError_t e = hipSuccess;
-#define QGEMM_RAISE(MT_, F32_)                                                                                                                  \
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)qgemm_q4_0_kernel<MT_, F32_, false>, hipFuncAttributeMaxDynamicSharedMemorySize, most); \
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)qgemm_q4_0_kernel<MT_, F32_, true>, hipFuncAttributeMaxDynamicSharedMemorySize, most)
-            QGEMM_RAISE(1, true); QGEMM_RAISE(1, false); QGEMM_RAISE(2, true); QGEMM_RAISE(2, false); QGEMM_RAISE(4, true); QGEMM_RAISE(4, false);
-#undef QGEMM_RAISE
-            if (e != hipSuccess) return e;
-            raised = true;
-        }
-    }
+    static LdsLimit limit;  // more dynamic LDS than a kernel gets by default
+#define QGEMM_KERNELS(MT_, F32_) (const void*)qgemm_q4_0_kernel<MT_, F32_, false>, (const void*)qgemm_q4_0_kernel<MT_, F32_, true>
+    if (hipError_t e = limit.raise(160 * 1024, {QGEMM_KERNELS(1, true), QGEMM_KERNELS(1, false), QGEMM_KERNELS(2, true), QGEMM_KERNELS(2, false),
+                                                QGEMM_KERNELS(4, true), QGEMM_KERNELS(4, false)}))
+        return e;
+#undef QGEMM_KERNELS
 #define QGEMM_LAUNCH(MT_, F32_)                                                                                                              \
     do {                                                                                                                                     \
         if (half)                                                                                                                            \

@@ -325,13 +325,8 @@ hipError_t qgemm_q4_0_blocks(const void* W, const void* X, int64_t x_row_stride,
     if (!ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)X & 15) != 0 || x_row_stride % 8 != 0 || x_row_stride < K || ((uintptr_t)W & 1) != 0 ||
         M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || M >= (1 << 24) || N >= (1 << 24) || K > (1 << 24))
         return hipErrorInvalidValue;
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attributes
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_blocks_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)qgemm_q4_0_blocks_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise((int)kLdsBytes, {(const void*)qgemm_q4_0_blocks_kernel<true>, (const void*)qgemm_q4_0_blocks_kernel<false>})) return e;
     const int nb = (int)(K / 32), strips = (int)((N + 31) / 32), x_strips = (int)((M + 31) / 32);
     uint16_t* P = (uint16_t*)ws;
     uint16_t* XG = P + granules_bytes(N, K) / 2;

@@ -250,11 +250,8 @@ __global__ __launch_bounds__(64 * kWaves) void qgemm_q4_0_direct_kernel(Operands
 template <int MS>
 hipError_t launch(const Operands& o, const Direct& d, hipStream_t st) {
     if (kLdsBytes<MS> > 64 * 1024) {
-        static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-        if (!raised) {
-            if (hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_direct_kernel<MS>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes<MS>)) return e;
-            raised = true;
-        }
+        static LdsLimit limit;
+        if (hipError_t e = limit.raise(kLdsBytes<MS>, {(const void*)qgemm_q4_0_direct_kernel<MS>})) return e;
     }
     hipLaunchKernelGGL(qgemm_q4_0_direct_kernel<MS>, dim3((unsigned)(d.groups * d.tiles_m * d.shares)), dim3(64 * kWaves), kLdsBytes<MS>, st, o, d);
     return hipGetLastError();

@@ -303,12 +303,8 @@ bool qgemm_q4_0_fx_pays(const void* W, int64_t M, int64_t N, int64_t K) {
 
 // act: q4_0_fx_convert_act's rows. y = x . W^T (+ resid, which may be y itself).
 hipError_t qgemm_q4_0_fx(const void* W, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, hipStream_t st) {
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Layout::total);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise(Layout::total, {(const void*)qgemm_q4_0_fx_kernel})) return e;
     const int tiles_m = (int)((M + kTM - 1) / kTM), ntiles = (int)((N + kTN - 1) / kTN);
     const int per_xcd = (ntiles + 7) / 8;
     hipLaunchKernelGGL(qgemm_q4_0_fx_kernel, dim3((unsigned)(8 * per_xcd * tiles_m)), dim3(512), Layout::total, st, (const uint8_t*)W,

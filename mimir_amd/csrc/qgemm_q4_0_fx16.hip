@@ -711,13 +711,9 @@ static hipError_t multiply(const Parts& parts, const void* act, const float* res
     if (!ws || ((uintptr_t)ws & 15) != 0 || ((uintptr_t)act & 15) != 0 || !fits(M, strips, K) || ws_bytes < fixed) return hipErrorInvalidValue;
     for (int i = 0; i < 3; i++)
         if (((uintptr_t)parts.W[i] & 1) != 0) return hipErrorInvalidValue;
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-        if (e == hipSuccess) e = hipFuncSetAttribute((const void*)qgemm_q4_0_fx16_digits_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Low::total);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    static LdsLimit limit, digits_limit;
+    if (hipError_t e = limit.raise(kLdsBytes, {(const void*)qgemm_q4_0_fx16_kernel})) return e;
+    if (hipError_t e = digits_limit.raise(Low::total, {(const void*)qgemm_q4_0_fx16_digits_kernel})) return e;
     const int nb = (int)(K / 32);
     const bool digits = form == Fx16::Digits;
     Cut cut{0, 0, (int)((M + Low::BM - 1) / Low::BM), (int)((strips + 7) / 8), 1, nb};

@@ -328,11 +328,8 @@ __global__ __launch_bounds__(64 * kWaves) void qgemm_q4_0_parts_kernel(Operands 
 
 template <int MT>
 hipError_t launch(const Operands& o, const Plan& d, hipStream_t st) {
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (!raised) {
-        if (hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_parts_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes)) return e;
-        raised = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise(kLdsBytes, {(const void*)qgemm_q4_0_parts_kernel<MT>})) return e;
     hipLaunchKernelGGL(qgemm_q4_0_parts_kernel<MT>, dim3((unsigned)(d.groups * d.tiles_m * d.shares)), dim3(64 * kWaves), kLdsBytes, st, o, d);
     return hipGetLastError();
 }

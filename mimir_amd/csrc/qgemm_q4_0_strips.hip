@@ -409,10 +409,9 @@ hipError_t launch(const void* W, const void* x, void* y, int64_t M, int64_t N, i
     if (wgs > 0x7fffffff) return hipErrorInvalidValue;
     constexpr int kLds = kWaves * SW * kStripBytes;
     static_assert(kLds >= kWaves * 16 * 64 * 4, "the sums take the slabs' place");
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (kLds > 64 * 1024 && !raised) {
-        if (hipError_t e = hipFuncSetAttribute((const void*)qgemm_q4_0_strips_kernel<X, SW, RAGGED, Y>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
-        raised = true;
+    if (kLds > 64 * 1024) {
+        static LdsLimit limit;
+        if (hipError_t e = limit.raise(kLds, {(const void*)qgemm_q4_0_strips_kernel<X, SW, RAGGED, Y>})) return e;
     }
     hipLaunchKernelGGL((qgemm_q4_0_strips_kernel<X, SW, RAGGED, Y>), dim3((unsigned)wgs), dim3(64 * kWaves), kLds, st, (const uint8_t*)W, (const X*)x, (Y*)y, (int)M,
                        (int)N, (int)(K / 32), x_row_stride);

@@ -554,16 +554,13 @@ void set_kquant_tune(int which, int value) {
 
 template <int R>
 static hipError_t launch_kq(int dt, const QGemvArgs& a, int nsb, const Q4RopeTail* rope, hipStream_t st) {
-    static std::atomic<bool> raised[2];  // zero at start; threads may race here: both then set the same attribute
+    static LdsLimit limits[2];
     const size_t lds = kq_lds_bytes(nsb);
     const int rows_per_wg = kKqThreads / 64 * R;
     dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), (unsigned)a.M);
     const void* fn = dt == kQ4_K ? (const void*)qgemv_q4k_kernel<R> : (const void*)qgemv_q6k_kernel<R>;
-    if (lds > 48 * 1024 && !raised[dt == kQ4_K]) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kKqMaxLds);
-        if (e != hipSuccess) return e;
-        raised[dt == kQ4_K] = true;
-    }
+    if (lds > 48 * 1024)
+        if (hipError_t e = limits[dt == kQ4_K].raise((int)kKqMaxLds, {fn})) return e;
     const Q4RopeTail tail = rope ? *rope : Q4RopeTail{};
     // without converted activations the kernel reads float32 x and rounds it per workgroup
     const uint8_t* in = a.act ? (const uint8_t*)a.act : (const uint8_t*)a.x;

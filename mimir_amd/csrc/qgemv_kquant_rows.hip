@@ -407,12 +407,8 @@ template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>
 static hipError_t launch_kq_rows(const QGemvArgs& a, hipStream_t st, bool bf16, const Q4RopeTail* rope) {
     const int nsb = (int)(a.K / 256);
     const auto kernel = qgemv_kq_rows_kernel<DT, TILES, WAVES, DEPTH, ROUNDS, ROPE>;
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    static LdsLimit limit;
+    if (hipError_t e = limit.raise(160 * 1024, {(const void*)kernel})) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((a.N + 16 * TILES - 1) / (16 * TILES)), 1, (unsigned)((a.M + kRows - 1) / kRows)),
                        dim3(64 * WAVES), rows_lds(DT, nsb, TILES, WAVES), st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y, a.resid, (int)a.M,
                        (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), bf16 ? 1 : 0, rope ? *rope : Q4RopeTail{});

@@ -625,14 +625,9 @@ static int q4_batch_rows(int64_t M, int64_t K) {
 
 template <int R, int MODE, int MB>
 static hipError_t launch_q4_0_i4_batch(const Q4Job& job, const void* act, float* y, int64_t M, int64_t K, hipStream_t st) {
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
+    static LdsLimit limit;
     const size_t act_bytes = q4_0_act_bytes(K), lds_bytes = MB * act_bytes + MB * 128;
-    if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)qgemv_q4_0_i4_batch_kernel<R, MODE, MB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           160 * 1024);
-        if (e != hipSuccess) return e;
-        raised = true;
-    }
+    if (hipError_t e = limit.raise(160 * 1024, {(const void*)qgemv_q4_0_i4_batch_kernel<R, MODE, MB>})) return e;
     const int rows_per_wg = MODE == kSwiGLU && job.act_out ? 32 : R * 8;
     dim3 grid((unsigned)((job.total + rows_per_wg - 1) / rows_per_wg), (unsigned)((M + MB - 1) / MB));
     hipLaunchKernelGGL((qgemv_q4_0_i4_batch_kernel<R, MODE, MB>), grid, dim3(512), lds_bytes, st, job, (const uint8_t*)act, y, (int)M,

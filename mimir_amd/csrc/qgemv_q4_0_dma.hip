@@ -449,15 +449,11 @@ DmaPlan plan_dma(int nitems, int rr, int npairs, int min_waves, size_t act_bytes
     return pl;
 }
 
-// More dynamic LDS than a launch gets by default has to be asked for once per kernel.
+// More dynamic LDS than a launch gets by default has to be asked for once per kernel and device.
 template <int MODE, int HEAD, int NIT, int P, bool STAMPS>
 hipError_t dma_kernel_ready() {
-    static std::once_flag once;
-    static hipError_t status = hipSuccess;
-    std::call_once(once, [] {
-        status = hipFuncSetAttribute((const void*)qgemv_q4_0_dma_kernel<MODE, HEAD, NIT, P, STAMPS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDmaLdsMost);
-    });
-    return status;
+    static LdsLimit limit;
+    return limit.raise((int)kDmaLdsMost, {(const void*)qgemv_q4_0_dma_kernel<MODE, HEAD, NIT, P, STAMPS>});
 }
 
 template <int MODE, int HEAD, int NIT, int P>

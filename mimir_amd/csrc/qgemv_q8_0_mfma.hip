@@ -275,10 +275,9 @@ bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
 template <int XR, int WAVES, bool FOUR = false, bool AHEAD = false>
 static hipError_t launch(const QGemvArgs& a, int64_t wgs, hipStream_t st) {
     constexpr int kLds = WAVES * kWaveLds<XR>;
-    static std::atomic<bool> raised{false};  // threads may race here: both then set the same attribute
-    if (kLds > 64 * 1024 && !raised) {
-        if (hipError_t e = hipFuncSetAttribute((const void*)qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds)) return e;
-        raised = true;
+    if (kLds > 64 * 1024) {
+        static LdsLimit limit;
+        if (hipError_t e = limit.raise(kLds, {(const void*)qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>})) return e;
     }
     hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y,
                        (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K));

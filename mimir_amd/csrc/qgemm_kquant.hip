@@ -440,6 +440,7 @@ hipError_t launch(const QGemvArgs& a, int nsb, hipStream_t st) {
     Cut cut;
     plan(a.M, a.N, &cut);
     const int grid = 8 * ((cut.tall_m * cut.tall_cols + 7) / 8 + (cut.short_m * (cut.cols - cut.tall_cols) + 7) / 8);
+    note_kernel("qgemm_kquant_kernel: %d x %d tiles of 256 x 64, %d x %d of 128 x 64", cut.tall_m, cut.tall_cols, cut.short_m, cut.cols - cut.tall_cols);
     hipLaunchKernelGGL((qgemm_kquant_kernel<DT, OUT_BF16>), dim3((unsigned)grid), dim3(kThreads), kLds, st,
                        (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y, a.resid, (int)a.M, (int)a.N, nsb, (int64_t)kq_act_bytes(a.K), cut);
     return hipGetLastError();

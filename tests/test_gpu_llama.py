@@ -16,6 +16,8 @@ from mimir_amd.llama import Llama, load_mim
 from mimir_amd.mimfile import MimFile
 from oracle import llama as OL
 from tests import gpu
+from tests import test_gpu_decode_ops as ops
+from tests.helpers import bits_equal
 from tests.test_oracle_llama import compare_logits
 
 pytestmark = pytest.mark.gpu
@@ -595,5 +597,72 @@ def test_a_prompt_whose_products_round_to_int8_keeps_the_order_of_attentions_sum
         capi.check(lib.mi355x_tune(b"attention.prompt", 2))
         m.reset()
         assert np.array_equal(m.logits(prompts, all=True), got) == (linear_dt != O.Q4_0)
+    finally:
+        capi.check(lib.mi355x_tune(b"attention.prompt", 1))
+
+
+@pytest.mark.parametrize("linear_dt,batch,first,arch,biased,rope_dim,cache", [
+    (O.Q4_K, 2, 70, "qwen2", True, 128, capi.F16),   # halves turn against each other behind a bias, on rows as far apart as q, k and v are wide
+    (O.Q6_K, 1, 3, "qwen2", True, 64, capi.F32),     # a few rows, half of a head turning
+    (O.Q6_K, 3, 67, "llama", False, 128, capi.F16),  # neighbours turn
+])
+def test_k_quant_prompts_together_are_their_products_apart_bit_for_bit(linear_dt, batch, first, arch, biased, rope_dim, cache):
+    """A K-quant prompt's launches (q, k and v as one product, gate and up as another, biases, rotation and cache writes in one launch, norms and SwiGLU that round to
+    int8, residuals added as products are stored) against the library's operators one by one, whose products have the CPU's bits as these have: every logit of two
+    calls, the second behind the first's positions, is the same."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, cache)
+    c.interleaved, c.rope_dim = int(arch == "llama"), rope_dim
+    om = OL.synthetic(_oracle_config(c), seed=8, linear_dt=linear_dt, output_dt=O.Q6_K)
+    rng = np.random.default_rng(first)
+    biases = [[rng.normal(size=w.n).astype(np.float32) for w in (b.q, b.k, b.v)] if biased else None for b in om.blocks]
+    gpu.say(f"k-quant prompt together and apart, dt={linear_dt} {batch} x {first} {arch}")
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    for i, three in enumerate(biases):
+        for leaf, v in zip(("attn_q", "attn_k", "attn_v"), three or ()):
+            m.set_tensor(f"blk.{i}.{leaf}.bias", capi.F32, v, v.size)
+    m.finalize(max(first, 5))
+    weights = [{leaf: gpu.dev_bytes_at(w.data, 0) + (w,) for leaf, w in (("q", b.q), ("k", b.k), ("v", b.v), ("o", b.o), ("gate", b.gate), ("up", b.up), ("down", b.down))}
+               for b in om.blocks]
+    output = gpu.dev_bytes_at(om.output.data, 0) + (om.output,)
+    D, H, HK = c.head_dim, c.heads, c.kv_heads
+    cos, sin = O.rope_angles(rope_dim, c.rope_base, 0, c.context)
+    kept = [[np.zeros((batch, HK, c.context, D), np.uint16 if cache == capi.F16 else np.float32) for _ in range(2)] for _ in om.blocks]
+
+    def times(x, weight):
+        _, ptr, w = weight
+        return gpu.qgemv(linear_dt if w is not om.output else O.Q6_K, ptr, gpu.dev(x), w.n, w.k)
+
+    def swiglu(gate, up):
+        gd, ud = gpu.dev(gate), gpu.dev(up)
+        out = torch.empty_like(gd)
+        capi.check(lib.mi355x_swiglu(gd.data_ptr(), ud.data_ptr(), out.data_ptr(), gate.shape[0], gate.shape[1], gate.shape[1], gpu.stream()))
+        gpu.sync()
+        return out.cpu().numpy()
+
+    def apart(tokens, past):
+        s = tokens.shape[1]
+        x = O.dequantize(om.embed.dtype, om.embed.data).reshape(c.vocab, c.embed)[tokens.reshape(-1)].copy()
+        for b, w, three, caches in zip(om.blocks, weights, biases, kept):
+            h = ops.rmsnorm(x, b.attn_norm, c.eps)
+            parts = [times(h, w[leaf]) for leaf in "qkv"]
+            if three:
+                parts = [p + v for p, v in zip(parts, three)]
+            q, k, v = (np.ascontiguousarray(p.reshape(batch, s, -1, D).transpose(0, 2, 1, 3)) for p in parts)
+            q, k = (ops.rope(t, cos, sin, rope_dim, arch == "llama", past) for t in (q, k))
+            for kept_rows, new in zip(caches, (k, v)):
+                kept_rows[:, :, past:past + s] = O.f32_to_f16(new) if cache == capi.F16 else new
+            o, _ = ops.attention(q, *caches, 1 / np.sqrt(D), causal=True, offset=past, kv_dt=cache, k_len=past + s)
+            x = x + times(np.ascontiguousarray(o.transpose(0, 2, 1, 3)).reshape(batch * s, H * D), w["o"])
+            h = ops.rmsnorm(x, b.ffn_norm, c.eps)
+            x = x + times(swiglu(times(h, w["gate"]), times(h, w["up"])), w["down"])
+        return times(ops.rmsnorm(x, om.norm, c.eps), output).reshape(batch, s, c.vocab)
+
+    prompts = rng.integers(0, c.vocab, (batch, first + 5))
+    try:
+        capi.check(lib.mi355x_tune(b"attention.prompt", 2))  # the order of sums that a decoder of such products keeps
+        for tokens, past in ((prompts[:, :first], 0), (prompts[:, first:], first)):
+            assert bits_equal(m.logits(tokens, all=True), apart(tokens, past))
     finally:
         capi.check(lib.mi355x_tune(b"attention.prompt", 1))

@@ -2,6 +2,9 @@
 qmatmul (backend/cpu/qmatmul.go:148-200, 310-405). It runs every output through the CPU's float32
 operations in the CPU's order on exact integer sums, so the comparison is for equal bits, the
 property the reference claims for its own tiles (backend/cpu/qtile.go:51-54)."""
+import ctypes
+import re
+
 import numpy as np
 import pytest
 
@@ -148,15 +151,25 @@ def test_prompt_sized_products_take_the_matrix_cores_and_bf16_rounds_once(dt, m)
 
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
-@pytest.mark.parametrize("m,n,k", [
-    (300, 8960, 256),   # 256 tiles of 256 rows, then 36 of 128: one super-block, no step ahead
-    (257, 8200, 512),   # the same with a row and a few columns into the next tile
-    (700, 5000, 768),   # tiles of 256 rows to the last column but a few; an odd number of super-blocks
-    (128, 64, 1280), (129, 16384, 256),  # tiles of 128 rows alone: one, and one round of the device
+@pytest.mark.parametrize("m,n,k,tall,low", [
+    (300, 8960, 256, 0, 420), (257, 8200, 512, 0, 387), (128, 64, 1280, 0, 1),  # tiles of 128 rows alone: more than a round of the device, a row and a few columns over, one
+    (700, 5000, 768, 237, 0), (129, 16384, 256, 256, 0),                        # tiles of 256 rows alone: an odd number of super-blocks, a row into the second half
+    (129, 16448, 256, 256, 2), (655, 6144, 256, 255, 66),                       # both in one launch: one column of short tiles; a third of the last rows' tiles empty
+    (655, 6100, 768, 255, 66), (385, 8200, 512, 256, 4), (140, 16450, 512, 256, 4),  # with remainders of rows and columns in tiles of either height
 ])
-def test_tiles_of_either_height(dt, m, n, k, matrix_cores):
+def test_tiles_of_either_height(dt, m, n, k, tall, low, matrix_cores):
     rng = np.random.default_rng(m + n + k + dt)
     raw = random_blocks(rng, dt, n * k)
     x = rng.normal(size=(m, k)).astype(np.float32)
     gpu.say(f"kquant gemm tiles dt={dt} M={m} N={n} K={k}")
     assert bits_equal(product(dt, raw, x, n, k), O.qmatmul(dt, raw, x, n, k))
+    assert tiles_run() == (tall, low)
+
+
+def tiles_run():
+    """How many tiles of 256 and of 128 rows the last product was cut into."""
+    buf = ctypes.create_string_buffer(200)
+    capi.check(gpu.lib().mi355x_last_kernel(buf, 200))
+    cut = re.fullmatch(r"qgemm_kquant_kernel: (\d+) x (\d+) tiles of 256 x 64, (\d+) x (\d+) of 128 x 64", buf.value.decode())
+    rows, cols, low_rows, low_cols = map(int, cut.groups())
+    return rows * cols, low_rows * low_cols

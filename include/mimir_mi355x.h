@@ -106,14 +106,18 @@ MI355X_API mi355x_status mi355x_stream_release(void* stream);
  * x by Q4_0 or by a small Q8_0, Q4_K or Q6_K matrix; Q8_0 weights are read
  * once for up to eight rows) or kernels on the int8 matrix cores (Q4_0 from two
  * rows on: up to some tens of rows a kernel that reads W once per eight rows,
- * beyond them a tiled one; two to eight rows by a large Q8_0 matrix; Q4_K, Q6_K
- * from enough rows on) or, for Q4_0, on the binary16 ones (some tens of rows up to
+ * beyond them a tiled one; Q8_0 from two rows on by a large matrix, from nine on
+ * by all but the smallest, W read once for eight or for 32 rows; Q4_K, Q6_K
+ * from enough rows on), on the bfloat16 ones (Q4_0 from five rows on where rows
+ * of W are an odd number of blocks or W is on two bytes: a float32 x as the sum of
+ * three bfloat16, W and x read where they lie and no scratch) or, for other Q4_0,
+ * on the binary16 ones (some tens of rows up to
  * 256 with W read where it lies, whose rows and shares of K take 4 M K bytes and
  * up to 16 MiB of the stream's scratch; from some hundreds of rows with W's
  * integers written out once a call, a workspace of 2 N K bytes and up to 128 MiB
  * behind the rows); which one ran changes the results by the order of float32
  * additions (Q4_0, Q8_0) and, for Q4_0, by how x is held (fixed point per block,
- * or pairs of binary16: either within the bound below), or not at all (Q8_0 among
+ * or pairs of binary16: either within the bound below; or exactly), or not at all (Q8_0 among
  * its row kernels, Q4_K, Q6_K). The choice depends on the sizes, the
  * alignment of W and x, and mi355x_tune alone. */
 MI355X_API mi355x_status mi355x_qgemv(int dtype, const void* W, const float* x, float* y, int64_t M, int64_t N, int64_t K,
@@ -140,7 +144,9 @@ MI355X_API mi355x_status mi355x_qgemv_noalloc(int dtype, const void* W, const fl
  * per row at a 16-byte aligned `act` (0 when that dtype and K have no such
  * form); mi355x_qgemv_act multiplies by W. mi355x_qgemv does both through a
  * scratch buffer of its own.
- *   Q8_0: quantizeRow's int8 blocks (backend/cpu/qmatmul.go:208-254).
+ *   Q8_0: quantizeRow's int8 blocks (backend/cpu/qmatmul.go:208-254). Always the
+ *         row kernel that reads W once a row of x: a few rows at most, more are
+ *         faster by mi355x_qgemv, whose sums are then in another order.
  *   Q4_K, Q6_K: quantizeRow's int8 super-blocks of 256 with their sums.
  *   Q4_0: 24-bit fixed point per block of 32 (K a multiple of 64, W dword
  *         aligned); no counterpart in the reference, whose kernels take
@@ -164,13 +170,16 @@ MI355X_API mi355x_status mi355x_qgemv_act(int dtype, const void* W, const void* 
  * apart, W [N, K] of any block dtype, Y [M, N] contiguous of out_dtype
  * MI355X_BF16 (the reference's result) or MI355X_F32 (the same sums before the
  * rounding). Q4_0 runs on the bfloat16 matrix cores without rounding any
- * operand (each weight as two bfloat16 halves; or, for large products, the
- * weights' integers against x block by block and one float32 FMA per block with
- * the block's scale, which takes a workspace of 2 K (M + N) bytes and 4 bytes a
- * block of W in the stream's scratch), when K is a multiple of 256, X and W are 16-byte aligned
- * and rows of X are a multiple of 8 elements apart; otherwise, and for the other
- * dtypes, X goes through mi355x_qgemv as float32. Q4_K and Q6_K then run on
- * the int8 matrix cores from a few rows of X on, with the CPU's results bit for
+ * operand. Up to some hundreds of rows it is the weights' integers against x block
+ * by block and one float32 FMA per block with the block's scale, X and W read where
+ * they lie and no workspace: any K of 256 and more that is a multiple of 32, W on
+ * two bytes, X on 16 and its rows a multiple of 8 elements apart. Beyond, when K
+ * is a multiple of 256 and X and W are 16-byte aligned, each weight is two bfloat16
+ * halves; or, for large products, W's integers are written out first, which takes
+ * a workspace of 2 K (M + N) bytes and 4 bytes a
+ * block of W in the stream's scratch. Otherwise, and for the other
+ * dtypes, X goes through mi355x_qgemv as float32. Q8_0, Q4_K and Q6_K then run on
+ * the int8 matrix cores from a few rows of X on, the K-quants with the CPU's results bit for
  * bit (backend/cpu/qtile.go:51-54 claims the same of the reference's tiles). */
 MI355X_API mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y, int64_t M, int64_t N, int64_t K,
                                            int64_t x_row_stride, int out_dtype, void* stream);

@@ -142,7 +142,7 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
 }
 
 // y[rows, n] = x[rows, k] . W^T (nn/layers.go:49-55 -> tensor/quant.go:35-56).
-// With resid, y = product + resid (which may be y); only the row kernels of the quantized dtypes add it.
+// With resid, y = product + resid (which may be y): every form of converted x has a kernel that adds it as it stores.
 mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_t rows, const float* resid = nullptr) {
     int cls = act_class(w, rows, m.fx_panel.bytes);
     if (resid && cls == kActNone) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: no residual epilogue for this product");

@@ -29,10 +29,11 @@
 // brings in its own rows a step ahead, both are in step, and one barrier a step is enough. Rows of LDS are 256 bytes with their
 // 16-byte pieces turned by the row, which makes the 128-bit fragment reads conflict-free.
 //
-// What bounds it: the MFMAs (1056 cycles a wavefront and super-block, 64 x 32 outputs) and the vector instructions, which do not overlap with them on this device:
-// 256 a wavefront for the float32 operations (eight an output, fixed by the CPU's order), 80 for the split. A tall tile and super-block takes 2.7 us, of which these are 2.3.
+// What bounds it: the MFMAs (of 32 cycles each; 1088 a wavefront and super-block, 64 x 32 outputs, of Q4_K and 1024 of Q6_K) and the vector instructions, which do not overlap with
+// them on this device: of Q4_K 256 a wavefront for the float32 operations (eight an output, fixed by the CPU's order), 80 for the split, 423 in all by the counters; of Q6_K, which has no
+// mins, 357. At 2048 x 14336 x 4096 that is 92 % of the SIMDs' cycles by Q4_K and 77 % by Q6_K, whose wavefronts wait longer for loads off 2-byte boundaries, at a clock of 1.85 to 1.9 GHz.
 // Before (both groups in step, halves of a super-block, split by 24-bit multiplies, tiles of 256 x 64 only where they filled the device) and now, us with x's
-// conversion, Q4_K | Q6_K: 655 x 4096 x 14336 244 -> 157 | 238 -> 166, 655 x 14336 x 4096 185 -> 155 | 177 -> 158, 2048 x 14336 x 4096 434 -> 360 (668 TFLOP/s) | 419 -> 362,
+// conversion, Q4_K | Q6_K: 655 x 4096 x 14336 244 -> 157 | 238 -> 166, 655 x 14336 x 4096 185 -> 155 | 177 -> 158, 2048 x 14336 x 4096 434 -> 360 (668 TFLOP/s; of bfloat16 x, copies of W in turn, 388) | 419 -> 362,
 // 1000 x 5120 x 5120 160 -> 109 | 148 -> 107, 128 x 14336 x 4096 42.1 -> 36.9 | 41.1 -> 39.1, 300 x 2048 x 8192 74 -> 61 | 70 -> 62.
 //
 // Both matrix instructions take, per lane, the

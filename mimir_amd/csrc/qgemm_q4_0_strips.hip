@@ -10,15 +10,16 @@
 // n - 8 of the lower and of the upper nibbles, exact in bfloat16 (as sixteenths, the scale times sixteen), and one FMA a result adds the
 // block's sum by its scale. A float32 x is the sum of three bfloat16, exactly, and a block six MFMAs.
 //
-// What bounds it: 30 instructions of unpacking, 16 FMAs and 64 cycles of MFMA a block and strip, with float32 another 150
-// instructions of splitting x (for two strips where they fill the chip) and 192 cycles. From some 1800 workgroups on the tile
+// What bounds it, by the counters: 75 vector instructions (30 of unpacking, 16 FMAs) and two MFMAs of 32 cycles a block and strip, half and a tenth of the SIMDs' cycles at
+// 128 x 14336 x 4096, the rest waits for loads, of which W's come past the L2 once for every 32 rows of x; with float32 310 instructions a block and two strips, some 150 of them
+// splitting x (for two strips where they fill the chip), and twelve MFMAs, 61 % and 19 % at 128 x 4096 x 4064. From some 1800 workgroups on the tile
 // kernels, which unpack W once for 128 rows, are the faster. Whole calls, us, before and now:
 //   bfloat16   16 x 4096 x 4096    61 -> 10      float32   16 x 4096 x 4064      31 -> 20
 //             256 x 4096 x 4096    62 -> 38               128 x 4096 x 4064     215 -> 30
 //             128 x 4096 x 14336  200 -> 70               512 x 14336 x 4064   3860 -> 370
-// Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 6.6e-8 at K = 4096 (7.4e-8 at 4064), 1.05e-6 -> 6.5e-8 at 14336;
-// float32 1.96e-7 -> 9.1e-8 at K = 4064, 2.0e-7 -> 1.34e-7 at 14368. With the runs' and the wavefronts' sums in 32 bits it was
-// 8.3e-8 of bfloat16 at K = 4096, more than the 7.4e-8 of the kernel for an odd number of blocks.
+// Errors against 64 bits, of the result: bfloat16 5.5e-7 -> 6.6e-8 at K = 4096, 1.05e-6 -> 6.5e-8 at 14336;
+// float32 1.96e-7 -> 9.1e-8 at K = 4064, 2.0e-7 -> 1.34e-7 at 14368. With the runs' and the wavefronts' sums of bfloat16 in 32 bits it was
+// 8.3e-8 at K = 4064, more than the 7.4e-8 of the float32 kernel that such rows took before.
 #include <atomic>
 
 #include "device_util.h"

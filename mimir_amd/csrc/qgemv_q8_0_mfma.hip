@@ -21,7 +21,8 @@
 //
 // What bounds it. Eight rows: the loads (143 MB of 32768 x 4096: 27 us at the rate of a copy), with four wavefronts
 // too few for them where the matrix is small. 32 rows: a conversion, a product and an fma for each sum and block, 192
-// cycles beside the MFMA's 32 and some 60 of unpacking; 315 TFLOP/s at 512 x 4096 x 14336. Whole calls, us, with W read for eight rows
+// cycles beside the MFMA's 32 and some 50 of unpacking (61 vector instructions a block by the counters, 57 % of the SIMDs' cycles at
+// 512 x 4096 x 14336, where LDS spends 28 % of them in bank conflicts); 315 TFLOP/s there. Whole calls, us, with W read for eight rows
 // by the vector unit (and by four zeroed copies of x on the matrix cores: 2 and 8 x 32768 x 4096) and now:
 //   2, 8 x 32768 x 4096    40, 43 -> 35, 37        8 x 4096 x 14336     71 -> 29
 //   32 x 32768 x 4096         122 -> 49            64 x 1024 x 4096     34 -> 14

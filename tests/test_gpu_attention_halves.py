@@ -163,6 +163,16 @@ def test_a_row_whose_features_lie_far_apart(B, H, Q, D, ratio, short):
     assert err <= 2e-6, err
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("size", [2.0 ** -99, 2.0 ** -101, 2.0 ** -130])
+def test_rows_of_next_to_nothing(size, D):
+    """Rows of Q at and below the smallest that the parts hold: scores of nought to float32, so that all weights are one. The results' error is that of 65 added values."""
+    rng = np.random.default_rng(D)
+    q = (rng.normal(size=(1, 2, 64, D)) * size).astype(np.float32)
+    k, v = (rng.normal(size=(1, 2, 65, D)).astype(np.float32) for _ in range(2))
+    check_rows(q, k, v, 1e-6)
+
+
 def max_row_error(got, want):
     return np.sqrt(np.mean((got.astype(np.float64) - want) ** 2, -1) / np.mean(want ** 2, -1)).max()
 

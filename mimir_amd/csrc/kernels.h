@@ -55,7 +55,7 @@ struct QGemvArgs {
     int64_t M, N, K;
     int64_t x_row_stride;
     int rows_per_wg;            // 0 = derived from the launch shape
-    const float* resid = nullptr;  // [M, N] added to the product (fixed-point Q4_0 kernel only)
+    const float* resid = nullptr;  // [M, N] added to the product (by the kernels whose _ok does not ask for none)
 };
 
 // The float32 Q4_0 product, any shape. tune: {rows, cols, waves, no_lds}; zeros

@@ -91,6 +91,8 @@ struct Decoder {
     virtual mi355x_status embed_next() { return MI355X_OK; }
     virtual void next_embedding(ChooseTail&) const {}
     virtual int step_variant() const { return 0; }
+    // Whether a call of one token a sequence is cheaper as a step() than as forward(1).
+    virtual bool one_token_as_step() const { return false; }
     // Whether calls longer than max_rows may be run in several passes.
     virtual bool runs_in_portions() const { return false; }
     // Empties what the sequences hold.
@@ -104,6 +106,11 @@ struct Decoder {
     mi355x_status check_tokens(const int32_t* tokens, int64_t n) const;
     // tokens [batch, n] -> logits of the wanted rows (b * n + t) to the host, in the order asked for.
     mi355x_status logits_at(const int32_t* tokens, int64_t n, const int64_t* want, int64_t n_want, float* logits_host);
+    // The same for one token a sequence, where one_token_as_step().
+    mi355x_status step_logits(const int32_t* tokens, const int64_t* want, int64_t n_want, float* logits_host);
+    ChooseTail choose_tail() const;
+    // Whether a recorded step ends with the next tokens' rows brought in, and so begins without embed_next().
+    bool step_embedded() const;
     mi355x_status generate(const int32_t* prompt, int64_t n_prompt, int64_t n_new, int32_t* out_tokens, double* seconds);
 };
 

@@ -55,6 +55,7 @@ mi355x_status Decoder::logits_at(const int32_t* tokens, int64_t n, const int64_t
     if (mi355x_status st = check_tokens(tokens, n)) return st;
     for (int64_t i = 0; i < n_want; i++)
         if (want[i] < 0 || want[i] >= (int64_t)batch * n) return capi_fail(MI355X_ERR_INDEX, "mi355x: %s: logits of row %lld of %lld", name, (long long)want[i], (long long)((int64_t)batch * n));
+    if (n == 1 && n_want > 0 && one_token_as_step() && g_llama_step_mode != 2) return step_logits(tokens, want, n_want, logits_host);
     const int64_t span = max_rows / batch;
     std::vector<int32_t> part;
     std::vector<int64_t> rows, place;
@@ -92,6 +93,38 @@ mi355x_status Decoder::logits_at(const int32_t* tokens, int64_t n, const int64_t
     return mi355x_sync(stream);
 }
 
+// One token a sequence, as the next decoding step that it is: a step's launches are fewer and fused where forward() has one for every operator and
+// row (a layer of one Q4_0 row is 5 launches for 16, of eight rows 8 for 16 whose products read W eight times). Replayed where generate has recorded it;
+// the choice that a recorded step ends in goes to `record` and `next_tok`, which the next caller sets anew.
+mi355x_status Decoder::step_logits(const int32_t* tokens, const int64_t* want, int64_t n_want, float* logits_host) {
+    DECODER_HIP(hipMemcpyAsync(next_tok.p, tokens, (size_t)batch * 4, hipMemcpyHostToDevice, stream), name, "upload tokens");
+    DECODER_HIP(set_state(state.as<int32_t>(), (int)cache_len, 0, stream), name, "step state");
+    const bool replay = step_graph && graph_variant == step_variant() && g_llama_step_mode == 0;
+    if (!replay || step_embedded())
+        if (mi355x_status st = embed_next()) return st;
+    if (replay) DECODER_HIP(hipGraphLaunch(step_graph, stream), name, "graph launch");
+    else if (mi355x_status st = step()) return st;
+    cache_len += 1;
+    for (int64_t i = 0; i < n_want;) {  // runs of neighbouring rows in one copy
+        int64_t j = i + 1;
+        while (j < n_want && want[j] == want[j - 1] + 1) j++;
+        DECODER_HIP(hipMemcpyAsync(logits_host + i * (int64_t)vocab, logits.as<float>() + want[i] * (int64_t)vocab, (size_t)(j - i) * (size_t)vocab * 4,
+                                   hipMemcpyDeviceToHost, stream), name, "download logits");
+        i = j;
+    }
+    return mi355x_sync(stream);
+}
+
+ChooseTail Decoder::choose_tail() const {
+    ChooseTail tail;
+    tail.state = state.as<int32_t>();
+    tail.record = record.as<int32_t>();
+    next_embedding(tail);
+    return tail;
+}
+
+bool Decoder::step_embedded() const { return argmax_choose_ok(batch, vocab, argmax_ws.p) && choose_tail().table; }
+
 // Greedy generation (examples/llama/generate.go:162-202 with Sample at :44-53):
 // the prompt [batch, n_prompt], then n_new steps. Each step's token is chosen on
 // the device and read by the next step's embedding lookup from device memory;
@@ -107,8 +140,6 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
     auto hip = [&](hipError_t e, const char* what) -> mi355x_status {
         return e == hipSuccess ? MI355X_OK : capi_fail((mi355x_status)e, "mi355x: %s: %s: %s", name, what, hipGetErrorName(e));
     };
-    DevBuf picked;  // [n_new, batch]
-    DECODER_HIP(picked.alloc((size_t)n_new * B * 4), name, "hipMalloc(tokens)");
     hipEvent_t e0, e1, e2;
     DECODER_HIP(hipEventCreate(&e0), name, "hipEventCreate");
     DECODER_HIP(hipEventCreate(&e1), name, "hipEventCreate");
@@ -133,19 +164,16 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
         if (mi355x_status s2 = head(last.data(), B)) return s2;
         return hip(argmax(logits.as<float>(), B, vocab, out, argmax_ws.p, stream), "argmax");
     };
-    if (!st) st = choose(picked.as<int32_t>(), last_s);
+    int32_t* picked = record.as<int32_t>();  // [n_new, batch]
+    if (!st) st = choose(use_fast ? next_tok.as<int32_t>() : picked, last_s);
     if (!st) (void)hipEventRecord(e1, stream);
     if (!st && use_fast) {
         // record[0] is the prompt's choice; each step then reads next_tok and the
         // position from the device, and leaves its own choice in both places
-        st = hip(hipMemcpyAsync(next_tok.p, picked.p, B * 4, hipMemcpyDeviceToDevice, stream), "step state");
-        if (!st) st = hip(set_state(state.as<int32_t>(), (int)cache_len, 0, stream), "step state");
-        if (!st) st = hip(advance(state.as<int32_t>(), next_tok.as<int32_t>(), record.as<int32_t>(), (int)B, 0, stream), "step state");
-        ChooseTail tail;
-        tail.state = state.as<int32_t>();
-        tail.record = record.as<int32_t>();
-        next_embedding(tail);
-        const bool chosen = argmax_choose_ok(B, vocab, argmax_ws.p), embedded = chosen && tail.table;
+        st = hip(set_state(state.as<int32_t>(), (int)cache_len, 0, stream), "step state");
+        if (!st) st = hip(advance(state.as<int32_t>(), next_tok.as<int32_t>(), picked, (int)B, 0, stream), "step state");
+        const ChooseTail tail = choose_tail();
+        const bool chosen = argmax_choose_ok(B, vocab, argmax_ws.p), embedded = step_embedded();
         if (!st && embedded && n_new > 1) st = embed_next();  // for the first step
         auto one_step = [&]() -> mi355x_status {
             if (!embedded)
@@ -175,17 +203,16 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
             st = step_graph && use_graph ? hip(hipGraphLaunch(step_graph, stream), "graph launch") : one_step();
             if (!st) cache_len += 1;
         }
-        if (!st) st = hip(hipMemcpyAsync(picked.p, record.p, (size_t)n_new * B * 4, hipMemcpyDeviceToDevice, stream), "copy record");
     } else
         for (int64_t t = 1; t < n_new && !st; t++) {
             // the step reads its tokens where the last step's argmax wrote them
-            st = hip(hipMemcpyAsync(tokens_dev.p, picked.as<int32_t>() + (t - 1) * B, B * 4, hipMemcpyDeviceToDevice, stream), "token copy");
+            st = hip(hipMemcpyAsync(tokens_dev.p, picked + (t - 1) * B, B * 4, hipMemcpyDeviceToDevice, stream), "token copy");
             if (!st) st = forward(1);
-            if (!st) st = choose(picked.as<int32_t>() + t * B, 1);
+            if (!st) st = choose(picked + t * B, 1);
         }
     if (!st) (void)hipEventRecord(e2, stream);
     std::vector<int32_t> host((size_t)n_new * B);
-    if (!st) st = hip(hipMemcpyAsync(host.data(), picked.p, host.size() * 4, hipMemcpyDeviceToHost, stream), "download tokens");
+    if (!st) st = hip(hipMemcpyAsync(host.data(), picked, host.size() * 4, hipMemcpyDeviceToHost, stream), "download tokens");
     if (!st) st = mi355x_sync(stream);
     if (!st) {
         for (int64_t t = 0; t < n_new; t++)

@@ -291,6 +291,44 @@ def test_fused_and_graph_replayed_steps_choose_the_per_operator_tokens(batch, ca
     assert all(same), (runs[2][0], runs[0][0])
 
 
+@pytest.mark.parametrize("batch,output_dt", [(1, O.Q4_0), (5, O.Q4_0), (16, O.Q8_0), (17, O.Q4_0)])
+def test_logits_of_one_token_as_a_decoding_step(batch, output_dt):
+    """One token a sequence goes through the decoding step's launches (of up to sixteen sequences), one by one before a generation
+    has recorded them and replayed after it, from an empty cache too, and leaves cache and logits as the per-operator pass does. A product is
+    within 2e-7 of the float32 one either way and a model has some tens: 1e-5 of the largest logit; a Q8_0 head rounds x to a 127th of a block's largest (0.02)."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    om = OL.synthetic(_oracle_config(c), seed=3, output_dt=output_dt)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(40)
+    rng = np.random.default_rng(batch)
+    prompts, one, two = rng.integers(0, c.vocab, (batch, 9)), rng.integers(0, c.vocab, (batch, 1)), rng.integers(0, c.vocab, (batch, 1))
+    want = [batch - 1, 0]
+    runs = {}
+    try:
+        for name, mode, recorded in (("operators", 2, False), ("launches", 0, False), ("replayed", 0, True), ("one by one", 1, True)):
+            gpu.say(f"one token as a step: {name}, batch {batch}")
+            capi.check(lib.mi355x_tune(b"llama.step", mode))
+            if recorded:
+                m.generate(prompts, 3)
+            m.reset()
+            first = m.logits(one)  # on empty caches
+            m.reset()
+            m.logits(prompts)
+            runs[name] = [first, m.logits(one), m.logits_at(two, want), m.logits_at(one, [0, 0]), m.logits(prompts)]
+            assert m.cache_len == 9 + 3 + 9
+    finally:
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    tol = 0.02 if output_dt == O.Q8_0 else 1e-5
+    for name, got in runs.items():
+        for i, (g, w) in enumerate(zip(got, runs["operators"])):
+            assert g.shape == w.shape and np.abs(g - w).max() <= tol * np.abs(w).max(), (name, i, float(np.abs(g - w).max() / np.abs(w).max()))
+    assert all(np.array_equal(a, b) for a, b in zip(runs["launches"], runs["replayed"]))
+    with pytest.raises(RuntimeError):
+        m.logits_at(one, [batch])
+
+
 @pytest.mark.parametrize("embed,batch", [(4160, 1), (8192, 1), (8192, 2)])
 def test_rows_longer_than_one_step_through_the_fused_rotation(embed, batch):
     """A llama-layout model whose rows of x are longer than 4096: the q|k|v product with the rotation and the cache

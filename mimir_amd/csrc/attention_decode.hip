@@ -11,17 +11,18 @@
 // Sixteen lanes share a key row, 16 or 32 bytes each, so a wavefront's load
 // covers four whole rows; the sixteen key groups of the workgroup take
 // consecutive keys. Scores go through LDS for the softmax, values are
-// accumulated per key group and summed through LDS. The rows of a share are
-// requested before the number of keys is read (shares are fixed ranges of the
-// cache, rows past the end clamped), so that load's round trip runs beside the
-// keys'. A share's (max, sum, weighted values) reach the combining workgroup one
+// accumulated per key group, summed within a wavefront by exchanges of
+// registers and over the four through LDS. Number of keys, queries, keys and
+// values are requested in that order before any of them is waited for (shares
+// are fixed ranges of the cache, rows past the end clamped): one trip to memory.
+// A share's (max, sum, weighted values) reach the combining workgroup one
 // of two ways. With flag slots (the decoder's steps): every float travels as an
 // 8-byte (value, flag) pair, stored and loaded as one word, so a pair that
-// reads as flagged is complete without any fence; the first share's workgroup
+// reads as flagged is complete without any fence; the last share's workgroup
 // polls the other shares' slots (all of them requested in one trip, a bounded
 // number of polls, the device's error word on a time-out), combines, and clears
 // the slots for the next launch. The workgroups it waits for never wait
-// themselves, and its own share is done before it polls. Without slots (the
+// themselves and start before it, and its own share is done before it polls. Without slots (the
 // boundary's call with its own workspace): each workgroup takes a ticket
 // (release-acquire at device scope) and the one that draws the last ticket of
 // its heads combines, so no workgroup waits at all. Either can leave the
@@ -30,6 +31,15 @@
 // (key head x query group, share, sequence): with eight key heads a head's
 // shares have workgroup indices congruent modulo eight, i.e. they run on one
 // die, and the head's rows and slots stay in that die's L2.
+//
+// What bounds it: a chain of waits, at one wavefront a SIMD. Clock readings of a launch between others that empty the caches, from the first
+// workgroup's start, heads of 128 features, binary16 cache, us: all loaded at 1.2, scores 1.9, softmax 2.3, values 3.4, the shares' put together 5.2, converted and stored 6.7
+// (one sequence, 576 positions in nine shares). Before, with each head's queries waited for in turn before the keys were requested, sums over
+// lanes and key groups one by one, and the first share's workgroup collecting: 2.5, 3.4, 3.9, 5.5, 8.2, 10.4. Whole launches: 64 positions 6.7 -> 4.4,
+// 128 9.7 -> 6.2, 576 11.0 -> 7.1, eight sequences of 544 15.3 -> 10.8, 2080 15.1 -> 10.8. Eight wavefronts a workgroup, a row of keys fewer each, were no
+// faster (6.4 at 128, 8.5 at 576), so were conversions kept apart from the products (v_fma_mix_f32).
+#include <type_traits>
+
 #include "device_util.h"
 #include "kernels.h"
 #include "kq_act.h"
@@ -63,13 +73,11 @@ struct DecParams {
     uint32_t* err;                // the device's error word (a hand-over that never completes sets kErrInternal)
 };
 
-__device__ __forceinline__ float group16_sum(float v) {
-    v += dpp_f32<0xb1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_f32<0x4e>(v);   // quad_perm [2,3,0,1]
-    v += dpp_f32<0x141>(v);  // row_half_mirror
-    v += dpp_f32<0x140>(v);  // row_mirror
-    return v;
-}
+// LDS in floats behind the scores: the wavefronts' values, and the results (or, before them, the shares' factors) beside them, so that
+// no wavefront waits for the others' reads before it writes its own.
+template <int D>
+constexpr int kFinal = kThreads / 64 * kHeads * D;
+constexpr int value_floats(int D) { return (kThreads / 64 + 1) * kHeads * D; }
 
 // Stores and loads that are coherent across the device on their own.
 __device__ __forceinline__ void coherent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -77,7 +85,7 @@ __device__ __forceinline__ float coherent_load(const float* p) { return __hip_at
 
 // A value and the flag that says it is there, in one 8-byte store: whoever loads the pair sees both or neither.
 constexpr uint32_t kShareReady = 1u;
-constexpr int kGather = 16;           // shares whose values the collecting workgroup requests together
+constexpr int kGather = 16;           // shares whose values the collecting workgroup requests together, at most
 constexpr int kShareSpins = 1 << 18;  // polls of a slot before the collecting workgroup gives up (some tenths of a second)
 __device__ __forceinline__ void flagged_store(unsigned long long* p, float v) {
     __hip_atomic_store(p, ((unsigned long long)kShareReady << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -140,10 +148,10 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                                                                uint32_t* __restrict__ counters, float* __restrict__ out,
                                                                float* __restrict__ lse, uint8_t* __restrict__ act, DecParams p) {
     constexpr int D = 16 * FPL;
-    constexpr int OPL = D / 64;  // results a lane holds of its wavefront's head
+    constexpr int OPL = D / 64;  // results a lane holds of its wavefront's head: features lane + 64 c
     extern __shared__ float smem[];
-    float* sc = smem;                  // [4][cmax] scores, then weights
-    float* osl = sc + kHeads * p.cmax; // [16][4][D] values per key group; later the combine's factors and results
+    float* sc = smem;                  // [cmax][4] scores, then weights: a key's four heads next to each other
+    float* osl = sc + kHeads * p.cmax; // [4][4][D] values per wavefront, and the results behind them
     __shared__ float red[2 * kHeads];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -163,18 +171,12 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
     // number before the queries, keys and values of the first batch have been requested (rows past the last key
     // seen are requested too, from within the caches, and ignored).
     const int j0 = split * cmax;
+    // Everything is requested before anything is waited for: the number of keys first (loads return in order), then the queries
+    // (those of a head that is not there: the first's), the keys and the values.
+    const int dyn_k = *(p.dyn_k ? p.dyn_k : (const int32_t*)q);
     float qr[kHeads][FPL];
 #pragma unroll
-    for (int g = 0; g < kHeads; g++) {
-        if (g < ng) {
-            load_row<float, FPL>(q + b * p.q_b + (int64_t)(hk * G + g0 + g) * p.q_h + part * FPL, qr[g]);
-#pragma unroll
-            for (int f = 0; f < FPL; f++) qr[g][f] = qr[g][f] * p.scale;
-        } else {
-#pragma unroll
-            for (int f = 0; f < FPL; f++) qr[g][f] = 0.f;
-        }
-    }
+    for (int g = 0; g < kHeads; g++) load_row<float, FPL>(q + b * p.q_b + (int64_t)(hk * G + g0 + (g < ng ? g : 0)) * p.q_h + part * FPL, qr[g]);
     // rows of a head's keys and values lie within 2^31 elements and fewer than 2^23 apart (checked by the host): 24-bit multiplies
     // and 32-bit offsets in place of 64-bit address arithmetic per row
     const int kp = (int)p.k_p, vp = (int)p.v_p;
@@ -198,13 +200,17 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
         load_raw<KV, FPL>(vbase + (uint32_t)__mul24(row < last_row ? row : last_row, vp), vraw[u]);
     }
     __builtin_amdgcn_sched_barrier(0);  // the requests above go out before the number of keys is waited for
-    int64_t seen = (int64_t)p.K + (p.dyn_k ? *p.dyn_k : 0);
+    int64_t seen = (int64_t)p.K + (p.dyn_k ? __builtin_amdgcn_readfirstlane(dyn_k) : 0);
     if (p.causal) {
         int64_t c = p.causal_offset + 1;
         seen = c < seen ? c : seen;
     }
     seen = seen < 0 ? 0 : seen > p.kmax ? p.kmax : seen;
     const int nj = seen > j0 ? (int)(seen - j0 < cmax ? seen - j0 : cmax) : 0;
+#pragma unroll
+    for (int g = 0; g < kHeads; g++)
+#pragma unroll
+        for (int f = 0; f < FPL; f++) qr[g][f] = g < ng ? qr[g][f] * p.scale : 0.f;
     for (int jj0 = 0; jj0 < nj; jj0 += U * kKeyGroups) {
         if (jj0 > 0) {
 #pragma unroll
@@ -213,19 +219,32 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                 load_raw<KV, FPL>(kbase + (uint32_t)__mul24(j0 + (jj < nj ? jj : 0), kp), kraw[u]);
             }
         }
+        // Four rows' scores for the four heads are sixteen sums over the row's sixteen lanes: a step within a quad keeps the head that
+        // its lane ends up with, so that they take 32 additions and one store for 64 and sixteen.
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int jj = jj0 + kKeyGroups * u + kg;
-            float kf[FPL];
-            raw_values<KV, FPL>(kraw[u], kf);
+        for (int u0 = 0; u0 < U; u0 += 4) {
+            float t[4];
 #pragma unroll
-            for (int g = 0; g < kHeads; g++) {
-                float s = 0.f;
+            for (int u = 0; u < 4; u++) {
+                float kf[FPL], s[kHeads];
+                raw_values<KV, FPL>(kraw[u0 + u], kf);
 #pragma unroll
-                for (int f = 0; f < FPL; f++) s = fmaf(qr[g][f], kf[f], s);
-                s = group16_sum(s);
-                if (part == 0 && jj < nj) sc[g * cmax + jj] = s;
+                for (int g = 0; g < kHeads; g++) {
+                    s[g] = 0.f;
+#pragma unroll
+                    for (int f = 0; f < FPL; f++) s[g] = fmaf(qr[g][f], kf[f], s[g]);
+                    s[g] += dpp_f32<0xb1>(s[g]);  // quad_perm [1,0,3,2]
+                }
+                float lo = part & 1 ? s[1] : s[0], hi = part & 1 ? s[3] : s[2];
+                lo += dpp_f32<0x4e>(lo);  // quad_perm [2,3,0,1]
+                hi += dpp_f32<0x4e>(hi);
+                t[u] = part & 2 ? hi : lo;    // head part & 3, over the quad
+                t[u] += dpp_f32<0x124>(t[u]);  // row_ror:4
+                t[u] += dpp_f32<0x128>(t[u]);  // row_ror:8
             }
+            const float mine = part & 8 ? (part & 4 ? t[3] : t[2]) : (part & 4 ? t[1] : t[0]);
+            const int jj = jj0 + kKeyGroups * (u0 + (part >> 2)) + kg;
+            if (jj < nj) sc[kHeads * jj + (part & 3)] = mine;
         }
     }
     __syncthreads();
@@ -233,17 +252,17 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
     // per head (wavefront g takes head g): max, exp, sum over the share's scores
     {
         float m = -__builtin_inff();
-        for (int jj = lane; jj < nj; jj += 64) m = fmaxf(m, sc[wave * cmax + jj]);
+        for (int jj = lane; jj < nj; jj += 64) m = fmaxf(m, sc[kHeads * jj + wave]);
         m = wave_max(m);
         float l = 0.f;
         if (nj > 0 && m > -__builtin_inff()) {
             for (int jj = lane; jj < nj; jj += 64) {
-                float e = __builtin_expf(sc[wave * cmax + jj] - m);
-                sc[wave * cmax + jj] = e;
+                float e = __builtin_expf(sc[kHeads * jj + wave] - m);
+                sc[kHeads * jj + wave] = e;
                 l += e;
             }
         } else {
-            for (int jj = lane; jj < nj; jj += 64) sc[wave * cmax + jj] = 0.f;
+            for (int jj = lane; jj < nj; jj += 64) sc[kHeads * jj + wave] = 0.f;
         }
         l = wave_sum(l);
         if (lane == 0) {
@@ -271,43 +290,56 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
         for (int u = 0; u < U; u++) {
             const int jj = jj0 + kKeyGroups * u + kg;
             const bool live = jj < nj;
+            // rows past the last key count nothing, whatever they hold
+            f32x4 pj = *(const f32x4*)(sc + kHeads * (live ? jj : 0));
+#pragma unroll
+            for (int g = 0; g < kHeads; g++) pj[g] = live ? pj[g] : 0.f;
+#pragma unroll
+            for (uint32_t& w : vraw[u].w) w = live ? w : 0u;
             float vf[FPL];
             raw_values<KV, FPL>(vraw[u], vf);
 #pragma unroll
-            for (int g = 0; g < kHeads; g++) {
-                float pj = live ? sc[g * cmax + jj] : 0.f;
+            for (int g = 0; g < kHeads; g++)
 #pragma unroll
-                for (int f = 0; f < FPL; f++) o[g][f] = fmaf(pj, live ? vf[f] : 0.f, o[g][f]);
-            }
+                for (int f = 0; f < FPL; f++) o[g][f] = fmaf(pj[g], vf[f], o[g][f]);
         }
     }
+    // the wavefront's four key groups: exchanges of half the registers each leave row r of sixteen lanes with head r, FPL features a lane
 #pragma unroll
-    for (int g = 0; g < kHeads; g++)
+    for (int f = 0; f < FPL; f++) {
+        swap_halves(o[0][f], o[2][f]);
+        swap_halves(o[1][f], o[3][f]);
+        float even = o[0][f] + o[2][f], odd = o[1][f] + o[3][f];
+        swap_rows(even, odd);
+        o[0][f] = even + odd;
+    }
 #pragma unroll
-        for (int f = 0; f < FPL; f++) osl[(kg * kHeads + g) * D + part * FPL + f] = o[g][f];
+    for (int f = 0; f < FPL; f += 4) {
+        const f32x4 v = {o[0][f], o[0][f + 1], o[0][f + 2], o[0][f + 3]};
+        *(f32x4*)(osl + (wave * kHeads + (lane >> 4)) * D + part * FPL + f) = v;
+    }
     __syncthreads();
-    // wavefront g now holds head g: lane takes features lane + 64 c
-    const int g = wave, h = hk * G + g0 + g;
-    float r[OPL];
+    const int g = wave, h = hk * G + g0 + g;  // wavefront g now holds head g
+    const bool mine = g < ng;
+    float r[OPL], M = red[g], L = red[kHeads + g];
 #pragma unroll
     for (int c = 0; c < OPL; c++) {
-        float s = 0.f;
+        r[c] = 0.f;
 #pragma unroll
-        for (int x = 0; x < kKeyGroups; x++) s += osl[(x * kHeads + g) * D + lane + 64 * c];
-        r[c] = s;
+        for (int w = 0; w < kThreads / 64; w++) r[c] += osl[(w * kHeads + g) * D + lane + 64 * c];
     }
-    float M = red[g], L = red[kHeads + g];
 
     if (nsplit > 1 && p.flagged) {
         // The shares travel as (value, flag) pairs, each one 8-byte store that is coherent at device scope on its own:
         // a pair is seen whole or not at all, so nothing has to be waited for between the data and a signal that it
-        // is there. The workgroups of shares 1.. store theirs and are done; the workgroup of share 0 keeps its own in
-        // registers, polls the others' slots until every pair shows its flag (a bounded number of times: all
-        // workgroups of a launch are resident together, the grid being far smaller than the chip), combines them in
-        // the shares' order and clears the slots for the next launch on the stream.
+        // is there. The workgroups of all shares but the last store theirs and are done; the last share's keeps its own in
+        // registers, polls the others' slots until every pair shows its flag (a bounded number of times), combines
+        // them in the shares' order and clears the slots for the next launch on the stream. Workgroups start in the order of their
+        // indices on every die, so those that it waits for have started before it and are running or done, however full the device is.
         unsigned long long* slots = p.flagged + ((int64_t)b * p.H + h) * nsplit * (D + 2);
-        if (split != 0) {
-            if (g < ng) {
+        const int last = nsplit - 1;
+        if (split != last) {
+            if (mine) {
                 unsigned long long* w = slots + (int64_t)split * (D + 2);
                 if (lane == 0) {
                     flagged_store(w, M);
@@ -319,72 +351,73 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
             return;
         }
         bool late = false;
-        float* fs = osl + g * 64;  // factor of share s of head g
-        float own[OPL];
-#pragma unroll
-        for (int c = 0; c < OPL; c++) own[c] = r[c];
         const unsigned long long ready = (unsigned long long)kShareReady << 32;
-        // Sixteen shares' values at a time, asked for again while any pair lacks its flag; with the first sixteen go the
-        // (max, sum) of every share, so that one trip to memory brings all a short context needs.
+        // Up to kGather shares' values at a time, asked for again while any pair lacks its flag; with the first go the
+        // (max, sum) of every share, so that one trip to memory brings all that most contexts need.
         unsigned long long raw[kGather][OPL], mraw = ready | __float_as_uint(M), lraw = ready | __float_as_uint(L);
-        auto gather = [&](int s0, bool with_sums) {
-            bool all = g >= ng;  // a wavefront without a head has nothing to wait for
+        auto gather = [&](auto few, int s0, bool with_sums) {  // few: so many shares, the last but one again past the end: no branch between the requests
+            constexpr int N = decltype(few)::value;
+            bool all = !mine;  // a wavefront without a head has nothing to wait for
             for (int spin = 0; !all && spin < kShareSpins; spin++) {
-                if (spin) __builtin_amdgcn_s_sleep(2);
-                all = true;
-                if (with_sums && lane < nsplit && lane > 0) {
+                if (spin) __builtin_amdgcn_s_sleep(1);
+                if (with_sums && lane < last) {
                     mraw = flagged_load(slots + lane * (D + 2));
                     lraw = flagged_load(slots + lane * (D + 2) + 1);
                 }
 #pragma unroll
-                for (int u = 0; u < kGather; u++) {
-                    const int sidx = s0 + u < nsplit ? s0 + u : nsplit - 1;
+                for (int u = 0; u < N; u++) {
+                    const int sidx = s0 + u < last ? s0 + u : last - 1;
 #pragma unroll
-                    for (int c = 0; c < OPL; c++)
-                        raw[u][c] = sidx == 0 ? ready | __float_as_uint(own[c]) : flagged_load(slots + (int64_t)sidx * (D + 2) + 2 + lane + 64 * c);
+                    for (int c = 0; c < OPL; c++) raw[u][c] = flagged_load(slots + (int64_t)sidx * (D + 2) + 2 + lane + 64 * c);
                 }
                 all = (uint32_t)(mraw >> 32) == kShareReady && (uint32_t)(lraw >> 32) == kShareReady;
 #pragma unroll
-                for (int u = 0; u < kGather; u++)
+                for (int u = 0; u < N; u++)
 #pragma unroll
                     for (int c = 0; c < OPL; c++) all = all && (uint32_t)(raw[u][c] >> 32) == kShareReady;
             }
             if (!all) late = true;
         };
-        gather(0, true);
+        if (last <= 4) gather(std::integral_constant<int, 4>{}, 0, true);
+        else if (last <= 8) gather(std::integral_constant<int, 8>{}, 0, true);
+        else if (last <= 12) gather(std::integral_constant<int, 12>{}, 0, true);
+        else gather(std::integral_constant<int, kGather>{}, 0, true);
         float f = 0.f, ls = 0.f, ms = -__builtin_inff();
-        if (g < ng && lane < nsplit) {
+        if (mine && lane < nsplit) {
             ms = __uint_as_float((uint32_t)mraw);
             ls = __uint_as_float((uint32_t)lraw);
         }
         M = wave_max(ms);
         if (ls != 0.f && M > -__builtin_inff()) f = __builtin_expf(ms - M);
         L = wave_sum(ls * f);
-        fs[lane] = f;
-        __syncthreads();
+        auto factor = [&](int s) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), s)); };
+        float total[OPL];
 #pragma unroll
-        for (int c = 0; c < OPL; c++) r[c] = 0.f;
-        if (g < ng) {
-            for (int s0 = 0; s0 < nsplit; s0 += kGather) {
-                if (s0 > 0) gather(s0, false);
+        for (int c = 0; c < OPL; c++) total[c] = 0.f;
+        if (mine) {
+            for (int s0 = 0; s0 < last; s0 += kGather) {
+                if (s0 > 0) gather(std::integral_constant<int, kGather>{}, s0, false);
 #pragma unroll
                 for (int u = 0; u < kGather; u++) {
-                    const float fsv = s0 + u < nsplit ? fs[s0 + u] : 0.f;
+                    if (s0 + u >= last) break;
+                    const float fsv = factor(s0 + u);
 #pragma unroll
-                    for (int c = 0; c < OPL; c++) r[c] = fmaf(__uint_as_float((uint32_t)raw[u][c]), fsv, r[c]);
+                    for (int c = 0; c < OPL; c++) total[c] = fmaf(__uint_as_float((uint32_t)raw[u][c]), fsv, total[c]);
                 }
             }
+            const float fsv = factor(last);
+#pragma unroll
+            for (int c = 0; c < OPL; c++) r[c] = fmaf(r[c], fsv, total[c]);
             // the slots are read: empty again for the next launch
-            if (lane < nsplit && lane > 0) {
+            if (lane < last) {
                 flagged_clear(slots + lane * (D + 2));
                 flagged_clear(slots + lane * (D + 2) + 1);
             }
-            for (int sidx = 1; sidx < nsplit; sidx++)
+            for (int sidx = 0; sidx < last; sidx++)
 #pragma unroll
                 for (int c = 0; c < OPL; c++) flagged_clear(slots + (int64_t)sidx * (D + 2) + 2 + lane + 64 * c);
         }
         if (late && p.err) atomicOr(p.err, kErrInternal);
-        __syncthreads();  // fs is read; the results go over it
     } else if (nsplit > 1) {
         // The shares travel between workgroups (and so between the L2 caches of
         // the chip's dies) through stores and loads that are coherent at device
@@ -393,7 +426,7 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
         // are waited on, then the barrier) before thread 0 takes the ticket, a
         // release-acquire operation at device scope, and the combining loads are
         // issued only after the last ticket is known.
-        if (g < ng) {
+        if (mine) {
             float* w = ws + (((int64_t)b * p.H + h) * nsplit + split) * (D + 2);
             if (p.fence == 2) {  // measurement aid: plain stores, made visible by the ticket's release
                 if (lane == 0) {
@@ -428,10 +461,9 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
         if (!s_last) return;
         // the last workgroup of these heads to get here combines the shares: their (max, sum) and the first eight shares'
         // values are requested together, one trip to memory for both
-        float* fs = osl + g * 64;  // factor of share s of head g
         float f = 0.f, ls = 0.f, ms = -__builtin_inff();
         const float* w0 = ws + ((int64_t)b * p.H + h) * nsplit * (D + 2);
-        if (g < ng && lane < nsplit) {
+        if (mine && lane < nsplit) {
             ms = p.fence == 2 ? w0[lane * (D + 2)] : coherent_load(w0 + lane * (D + 2));
             ls = p.fence == 2 ? w0[lane * (D + 2) + 1] : coherent_load(w0 + lane * (D + 2) + 1);
         }
@@ -444,41 +476,39 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                 for (int c = 0; c < OPL; c++) t[u][c] = p.fence == 2 ? w0[s * (D + 2) + 2 + lane + 64 * c] : coherent_load(w0 + s * (D + 2) + 2 + lane + 64 * c);
             }
         };
-        if (g < ng) load_shares(0);
+        if (mine) load_shares(0);
         M = wave_max(ms);
         if (ls != 0.f && M > -__builtin_inff()) f = __builtin_expf(ms - M);
         L = wave_sum(ls * f);
-        fs[lane] = f;
-        __syncthreads();
 #pragma unroll
         for (int c = 0; c < OPL; c++) r[c] = 0.f;
-        if (g < ng) {
+        if (mine) {
             for (int s0 = 0; s0 < nsplit; s0 += 8) {  // eight shares' loads in flight
                 if (s0 > 0) load_shares(s0);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
-                    const float fsv = s0 + u < nsplit ? fs[s0 + u] : 0.f;
+                    if (s0 + u >= nsplit) break;
+                    const float fsv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), s0 + u));
 #pragma unroll
                     for (int c = 0; c < OPL; c++) r[c] = fmaf(t[u][c], fsv, r[c]);
                 }
             }
         }
-        __syncthreads();  // fs is read; the results go over it
     }
 
     // (sum p v) * (1 / sum p); a row that sees no key gets zeros and -Inf
     const float inv = L == 0.f ? 0.f : 1.0f / L;
-    float* fin = osl;  // [4][D]
+    float* fin = osl + kFinal<D>;  // [4][D]
 #pragma unroll
     for (int c = 0; c < OPL; c++) {
-        float val = L == 0.f ? 0.f : r[c] * inv;
-        if (g < ng && out) out[b * p.o_b + (int64_t)h * p.o_h + lane + 64 * c] = val;
-        if (act) fin[g * D + lane + 64 * c] = g < ng ? val : 0.f;
+        const float val = L == 0.f ? 0.f : r[c] * inv;
+        if (mine && out) out[b * p.o_b + (int64_t)h * p.o_h + lane + 64 * c] = val;
+        if (act) fin[g * D + lane + 64 * c] = mine ? val : 0.f;
     }
-    if (g < ng && lse && lane == 0) lse[(int64_t)b * p.H + h] = L == 0.f ? -__builtin_inff() : M + __builtin_logf(L);
+    if (mine && lse && lane == 0) lse[(int64_t)b * p.H + h] = L == 0.f ? -__builtin_inff() : M + __builtin_logf(L);
     if (!act) return;
-    __syncthreads();
     if (p.act_kq) {
+        __syncthreads();
         // the heads of this workgroup are whole super-blocks of 256 of the row (checked by the host): a wavefront each
         const int nsup = ng * D / 256, wv = tid >> 6;
         if (wv < nsup) {
@@ -487,24 +517,21 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
         }
         return;
     }
-    // item t: head t / (D/8), block (t % (D/8)) / 4 of the head, dword t % 4
-    const int nit = ng * (D / 8);
-    if (tid < nit) {
-        const int gi = tid / (D / 8), rr = tid % (D / 8), blk = rr >> 2, dq = rr & 3;
-        float lo[4], hi[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            lo[e] = fin[gi * D + blk * 32 + 4 * dq + e];
-            hi[e] = fin[gi * D + blk * 32 + 16 + 4 * dq + e];
-        }
+    // every wavefront converts its own head, its values back from LDS in the order of the items: item `lane` is block lane / 4, dword lane % 4
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane < D / 8 && mine) {
+        const int blk = lane >> 2, dq = lane & 3;
+        const f32x4 vl = *(const f32x4*)(fin + g * D + blk * 32 + 4 * dq), vh = *(const f32x4*)(fin + g * D + blk * 32 + 16 + 4 * dq);
+        float lo[4] = {vl[0], vl[1], vl[2], vl[3]}, hi[4] = {vh[0], vh[1], vh[2], vh[3]};
         const int nb = p.H * D / 32, nbp = nb | 1;
         if (p.act_rows) {
             // sequence b: row b % 8 of its group of eight, which has a buffer of its own
-            rows_convert_item(lo, hi, act + (int64_t)(b >> 3) * q4_0_rows_act_size((int64_t)nb * 32), nb, b & 7, (hk * G + g0 + gi) * (D / 32) + blk, dq);
+            rows_convert_item(lo, hi, act + (int64_t)(b >> 3) * q4_0_rows_act_size((int64_t)nb * 32), nb, b & 7, h * (D / 32) + blk, dq);
         } else {
             u32x4* plane = (u32x4*)(act + (int64_t)b * p.act_row_bytes);
             float* xscale = (float*)(plane + kDigits * nbp);
-            q4_convert_item(lo, hi, plane, xscale, nbp, (hk * G + g0 + gi) * (D / 32) + blk, dq);
+            q4_convert_item(lo, hi, plane, xscale, nbp, h * (D / 32) + blk, dq);
         }
     }
 }
@@ -529,7 +556,7 @@ void attention_decode_plan(int64_t B, int H, int HK, int64_t kmax, int* nsplit, 
     // the scores and the weighted values of a share take half as long, the hand-over a little longer.
     const int64_t aim = g_share_keys.load(std::memory_order_relaxed);
     int64_t by_keys = (kmax + aim - 1) / aim;
-    const bool short_shares = by_keys <= kGather;
+    const bool short_shares = by_keys <= 16;
     if (!short_shares) by_keys = (kmax + 127) / 128;
     // Shares of 64 keys are worth three workgroups a compute unit (eight sequences at 768 positions: 12 shares of 64 keys
     // decode 1.7 % faster than 8 of 96), longer ones are not (at 2048 positions 8 shares of 256 keys: 90 us a layer,
@@ -562,7 +589,7 @@ bool attention_decode_ok(const AttnArgs& a, int64_t kmax) {
     if (((uintptr_t)a.k | (uintptr_t)a.v) % row_align || (uintptr_t)a.q % 16 || a.q_strides[0] % 4 || a.q_strides[1] % 4) return false;
     int ns, cm;
     attention_decode_plan(a.B, a.H, a.HK, kmax, &ns, &cm);
-    size_t lds = (size_t)(kHeads * cm + kKeyGroups * kHeads * a.D) * sizeof(float);
+    size_t lds = (size_t)(kHeads * cm + value_floats(a.D)) * sizeof(float);
     if (a.k_strides[2] <= 0 || a.v_strides[2] <= 0 || a.k_strides[2] >= (1 << 23) || a.v_strides[2] >= (1 << 23) || kmax >= (1 << 23) ||
         kmax * a.k_strides[2] >= ((int64_t)1 << 31) || kmax * a.v_strides[2] >= ((int64_t)1 << 31))
         return false;
@@ -609,7 +636,7 @@ hipError_t attention_decode(const AttnArgs& a, int64_t kmax, void* workspace, vo
     p.err = err;
     int G = a.H / a.HK, ngq = (G + kHeads - 1) / kHeads;
     dim3 grid((unsigned)(a.HK * ngq), (unsigned)p.nsplit, (unsigned)a.B);
-    size_t lds = (size_t)(kHeads * p.cmax + kKeyGroups * kHeads * a.D) * sizeof(float);
+    size_t lds = (size_t)(kHeads * p.cmax + value_floats(a.D)) * sizeof(float);
     uint32_t* counters = (uint32_t*)workspace;
     float* ws = (float*)((uint8_t*)workspace + kCounterBytes);
     // a thread keeps eight rows of binary16 keys (four of float32) under way, or half as many where a share is that short

@@ -51,16 +51,31 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// Halves (rows of 16) of two registers exchanged: a keeps its lower half (even rows) and gets b's in its upper (odd),
+// b keeps its upper and gets a's in its lower.
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    const uint32_t lo = r[0], hi = r[1];
+    a = __builtin_bit_cast(float, lo), b = __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    const uint32_t lo = r[0], hi = r[1];
+    a = __builtin_bit_cast(float, lo), b = __builtin_bit_cast(float, hi);
+}
+
 __device__ __forceinline__ float wave_max(float v) {
     // Butterfly over DPP where it reaches (within rows of 16), then two
-    // cross-row steps through the LDS crossbar.
+    // cross-row steps by exchanges of registers (through the LDS crossbar they cost a wavefront alone on its SIMD 0.1 us).
     v = fmaxf(v, dpp_f32<0xb1>(v));   // quad_perm [1,0,3,2]
     v = fmaxf(v, dpp_f32<0x4e>(v));   // quad_perm [2,3,0,1]
     v = fmaxf(v, dpp_f32<0x141>(v));  // row_half_mirror
     v = fmaxf(v, dpp_f32<0x140>(v));  // row_mirror
-    v = fmaxf(v, __shfl_xor(v, 16));
-    v = fmaxf(v, __shfl_xor(v, 32));
-    return v;
+    float w = v;
+    swap_rows(v, w);
+    v = w = fmaxf(v, w);
+    swap_halves(v, w);
+    return fmaxf(v, w);
 }
 
 // Sum and max over each aligned group of 8 lanes, returned to all 8.

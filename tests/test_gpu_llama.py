@@ -439,6 +439,37 @@ def test_steps_of_a_context_of_96_share_its_keys_between_two_workgroups(linear_d
     assert np.abs(got[0] - got[1]).max() <= (1e-3 if linear_dt == O.Q4_0 else 0.02) * scale
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,cache,batch", [(2, 1, 128, capi.F16, 1), (4, 1, 128, capi.F32, 3), (3, 3, 64, capi.F16, 1), (8, 1, 64, capi.F32, 2)])
+def test_shares_of_the_keys_are_put_together_for_every_number_of_them(heads, kv_heads, head_dim, cache, batch):
+    """A step's attention in up to 40 shares, handed over by flagged pairs (requests of 4, 8, 12 and 16 shares, and several of 16) or by tickets, of
+    heads that do not fill a workgroup's four: the logits of a model held to one share, to 1e-5 of the largest (float32 sums in another order, some 1e-7
+    each, of three blocks). Shares past the last key are empty; a second step finds the slots clear."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, cache)
+    c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.context = heads, kv_heads, head_dim, head_dim, 200
+    om = OL.synthetic(_oracle_config(c), seed=6, output_dt=O.Q4_0)
+    prompts = np.random.default_rng(31).integers(0, c.vocab, (batch, 70))
+    want = None
+    try:
+        for handover in (0, 1):
+            capi.check(lib.mi355x_tune(b"attention.handover", handover))
+            for shares in (1, 2, 4, 5, 6, 9, 10, 13, 14, 17, 18, 33, 34, 40):
+                gpu.say(f"{heads} heads of {head_dim}, batch {batch}, {shares} shares, handover {handover}")
+                capi.check(lib.mi355x_tune(b"attention.splits", shares))  # before the model sizes its workspaces
+                m = Llama(c)
+                _upload_synthetic(m, om)
+                m.finalize(70)
+                m.logits(prompts)
+                got = [m.logits(np.full((batch, 1), 7)) for _ in range(3)]
+                m.close()
+                want = want or got
+                for g, w in zip(got, want):
+                    assert np.abs(g - w).max() <= 1e-5 * np.abs(w).max(), (shares, handover, float(np.abs(g - w).max() / np.abs(w).max()))
+    finally:
+        capi.check(lib.mi355x_tune(b"attention.splits", 0))
+        capi.check(lib.mi355x_tune(b"attention.handover", 0))
+
+
 @pytest.mark.parametrize("embed,batch,rows", [(512, 1, 3), (512, 3, 2), (4160, 2, 5), (8192, 1, 9)])
 def test_the_heads_norm_and_conversion_in_one_launch_are_the_two_launches(embed, batch, rows):
     """A block of zeros leaves a token's embedding as it is: the logits of a Q8_0 head are, bit for bit, those of rmsnorm, conversion and product one by one, for all rows of a

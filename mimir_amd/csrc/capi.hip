@@ -125,7 +125,7 @@ mi355x_status gemm_scratch(void* stream, size_t bytes, void** out) {
     return stream_scratch(stream, &StreamScratch::gemm, bytes, 0, 0, 0, "gemm", out);
 }
 mi355x_status argmax_scratch(void* stream, size_t bytes, void** out) {
-    return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, 0, mimir::kArgmaxTicketBytes, "argmax", out);
+    return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, 0, (size_t)-1 /* all of it */, "argmax", out);
 }
 
 size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
@@ -653,7 +653,7 @@ mi355x_status mi355x_argmax(const float* logits, int64_t rows, int64_t n, int32_
     void* ws = nullptr;
     if (rows <= 1024)
         if (mi355x_status st = argmax_scratch(stream, mimir::argmax_workspace_bytes(1024), &ws)) return st;
-    HIP_TRY(mimir::argmax(logits, rows, n, out, ws, (hipStream_t)stream), "launch argmax");
+    HIP_TRY(mimir::argmax(logits, rows, n, out, ws, mimir::device_error_word(), (hipStream_t)stream), "launch argmax");
     return MI355X_OK;
 }
 

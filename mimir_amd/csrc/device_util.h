@@ -78,6 +78,19 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(v, w);
 }
 
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));
+    float a = __builtin_bit_cast(float, v), b = a;
+    swap_rows(a, b);
+    v = min(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b));
+    a = b = __builtin_bit_cast(float, v);
+    swap_halves(a, b);
+    return min(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b));
+}
+
 // Sum and max over each aligned group of 8 lanes, returned to all 8.
 __device__ __forceinline__ float group8_sum(float v) {
     v += dpp_f32<0xb1>(v);

@@ -107,24 +107,28 @@ __device__ __forceinline__ float group8_max(float v) {
 
 // A row's sum of squares as a workgroup of 256 threads adds it: thread t takes x[t], x[t + 256], ...
 // in that order (the wavefronts' and the workgroup's sums follow at the caller). The loads go out in
-// batches of sixteen (a row of 4096 in one): a loop of unknown length would wait for each before requesting the next.
-__device__ __forceinline__ float strided_sum_squares(const float* __restrict__ xr, int d, int t) {
+// batches of sixteen (a row of 4096 in one), of four for rows of at most 1024: a loop of unknown length would wait for
+// each before requesting the next, and a branch round each had the compiler wait for what the caller requested before the first.
+template <int BATCH>
+__device__ __forceinline__ float strided_sum_squares_by(const float* __restrict__ xr, int d, int t) {
     float ss = 0.f;
-    constexpr int kBatch = 16;
-    for (int i0 = t; i0 < d; i0 += kBatch * 256) {
-        float v[kBatch];
+    for (int i0 = t; i0 < d; i0 += BATCH * 256) {
+        float v[BATCH];
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
+        for (int u = 0; u < BATCH; u++) {
             const int i = i0 + 256 * u;
-            v[u] = i < d ? xr[i] : 0.f;  // + 0 changes no sum
+            v[u] = xr[i < d ? i : d - 1];
         }
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            float sq = v[u] * v[u];
-            ss = ss + sq;
+        for (int u = 0; u < BATCH; u++) {
+            const float sq = v[u] * v[u];
+            ss = ss + (i0 + 256 * u < d ? sq : 0.f);  // + 0 changes no sum
         }
     }
     return ss;
+}
+__device__ __forceinline__ float strided_sum_squares(const float* __restrict__ xr, int d, int t) {
+    return d <= 1024 ? strided_sum_squares_by<4>(xr, d, t) : strided_sum_squares_by<16>(xr, d, t);
 }
 
 // ---- half conversions -----------------------------------------------------

@@ -311,8 +311,9 @@ hipError_t qgemv_q4_0_rows_qkv_rope(const void* const W[3], const int64_t n[3], 
 hipError_t qgemv_q4_0_rows_swiglu_act(const void* gate, const void* up, const void* act, void* act_out, int64_t M, int64_t N, int64_t K,
                                       hipStream_t st);
 // Around that product in a decoding step of up to eight sequences, each leaving its result in the converted form:
-// RMSNorm (with shares > 0, x += parts[0] + parts[1] + ... first, parts [shares, rows, d], written back to x: the
+// RMSNorm (with shares = kRowsShares, not 0, x += parts[0] + parts[1] first, parts [shares, rows, d], written back to x: the
 // residual connection behind a product cut into shares), SiLU(g) * u, and the addition of the shares alone.
+constexpr int kRowsShares = 2;  // of K, where a product is cut and its sums are added here (measured against 3 and 4)
 hipError_t rows_norm_act(float* x, const float* parts, int shares, const float* w, void* act, int64_t rows, int64_t d, double eps,
                          hipStream_t st);
 hipError_t rows_swiglu_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st);

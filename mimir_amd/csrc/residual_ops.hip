@@ -120,22 +120,34 @@ __global__ __launch_bounds__(1024) void norm_chain_kernel(NormChain a) {
     }
 }
 
+constexpr int kAhead = 4;      // earlier results that the depth average requests at a time
+constexpr int kFewRows = 64;
+constexpr int kChainTaps = 4;  // taps of a convolution whose weights and inputs are requested ahead
+
 // The same for rows whose groups are whole wavefronts of 256 elements: a thread owns E runs of four neighbouring elements in
-// registers, everything that does not depend on a sum is requested at once, and a norm costs one barrier.
-template <int E, bool EMBED>
+// registers, and a norm costs one barrier. A launch of few rows is a chain of waits, so everything that does not depend on a sum is requested before
+// anything is waited for, earlier results and the convolution's inputs included: with those read where they are used, a trip to memory for each,
+// a step's launches of four rows of 2048 took 5.6 us in the mean by the profiler, the one with the embedding 8.2; now 4.8 and 5.0.
+// FEW: launches of few rows; those of many are bound by their instructions and are faster without (2048 rows of 4096: 13.6 us, 18.6 with).
+template <int E, bool EMBED, bool FEW>
 __global__ __launch_bounds__(1024) void norm_chain_wide_kernel(NormChain a) {
+    constexpr int N = FEW ? kAhead : 1;
     __shared__ float part[2][64];
     const int W = a.width, gs = W / a.groups, lane = threadIdx.x & 63;
     const int64_t r = blockIdx.x;
-    int at[E];
+    // all arguments in one go, not where each is used
+    if constexpr (FEW)
+        asm volatile("" ::"s"(a.y), "s"(a.x), "s"(a.w_post), "s"(a.w_next), "s"(a.dwa), "s"(a.streams), "s"(a.conv_w), "s"(a.conv_state), "s"(a.x_out),
+                     "s"(a.stream_out), "s"(a.h_f32), "s"(a.h_bf16));
+    int at[E], from[E];
     bool in[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
         at[e] = (threadIdx.x + e * blockDim.x) * 4;
         in[e] = at[e] < W;  // whole wavefronts
+        from[e] = in[e] ? at[e] : 0;
     }
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    auto read = [&](const float* p, int e) { return in[e] ? *(const f32x4*)(p + at[e]) : zero; };
     // sums of squares: one of each wavefront's run, then the runs of a thread's own group
     auto norm = [&](const f32x4 v[E], float* sums, f32x4 out[E]) {
 #pragma unroll
@@ -155,40 +167,74 @@ __global__ __launch_bounds__(1024) void norm_chain_wide_kernel(NormChain a) {
             out[e] = v[e] * scale;
         }
     };
-    f32x4 y[E], x[E], wp[E], wn[E], z[E], avg[E];
+    f32x4 y[E], x[E], wp[E], wn[E], z[E], avg[E], earlier[N][E], hist[kChainTaps - 1][E], taps_w[kChainTaps][E];
     const uint16_t* row = EMBED ? a.table + (int64_t)a.tokens[r] * a.table_ld : nullptr;
     const uint16_t* pair = EMBED && a.pairs.table ? pair_row(a.pairs, a.tokens, r, threadIdx.x == 0) : nullptr;
 #pragma unroll
     for (int e = 0; e < E; e++) {
         if constexpr (EMBED) {
-            u32x2 v = {0, 0};
-            if (in[e]) v = *(const u32x2*)(row + at[e]);
+            u32x2 v = *(const u32x2*)(row + from[e]);
             y[e] = f32x4{__uint_as_float(v[0] << 16), __uint_as_float(v[0] & 0xffff0000u), __uint_as_float(v[1] << 16), __uint_as_float(v[1] & 0xffff0000u)};
-            if (pair && in[e]) {
-                v = *(const u32x2*)(pair + at[e]);
+            if (pair) {
+                v = *(const u32x2*)(pair + from[e]);
                 y[e] = y[e] + f32x4{__uint_as_float(v[0] << 16), __uint_as_float(v[0] & 0xffff0000u), __uint_as_float(v[1] << 16), __uint_as_float(v[1] & 0xffff0000u)};
             }
             x[e] = zero;
         } else {
-            y[e] = a.y ? read(a.y + r * a.ldy, e) : zero;
-            x[e] = read(a.x + r * W, e);
+            y[e] = zero;
+            if (a.y) y[e] = *(const f32x4*)(a.y + r * a.ldy + from[e]);
+            x[e] = *(const f32x4*)(a.x + r * W + from[e]);
         }
-        wp[e] = a.w_post ? read(a.w_post, e) : zero;
-        wn[e] = a.w_next ? read(a.w_next, e) : zero;
-        avg[e] = zero;
+        wp[e] = wn[e] = avg[e] = zero;
+        if (a.w_post) wp[e] = *(const f32x4*)(a.w_post + from[e]);
+        if (a.w_next) wn[e] = *(const f32x4*)(a.w_next + from[e]);
     }
-    if (a.dwa)
-        for (int j = 0; j < a.n_streams; j++) {
-            const float w = a.dwa[j];
+    auto earlier_from = [&](int j0) {  // past the last: it again
 #pragma unroll
-            for (int e = 0; e < E; e++) {
-                const f32x4 v = read(a.streams + j * a.stream_stride + r * W, e);
+        for (int u = 0; u < N; u++) {
+            const int j = j0 + u < a.n_streams ? j0 + u : a.n_streams - 1;
 #pragma unroll
-                for (int i = 0; i < 4; i++) avg[e][i] = fmaf(w, v[i], avg[e][i]);
+            for (int e = 0; e < E; e++) earlier[u][e] = *(const f32x4*)(a.streams + j * a.stream_stride + r * W + from[e]);
+        }
+    };
+    const bool averages = a.dwa && a.n_streams > 0, ahead = FEW && a.conv_w && a.taps == kChainTaps;
+    float dw[N] = {}, own = 1.f;
+    if (averages) {
+        earlier_from(0);
+#pragma unroll
+        for (int u = 0; u < N; u++) dw[u] = a.dwa[u < a.n_streams ? u : a.n_streams - 1];
+    }
+    if (a.dwa) own = a.dwa[a.n_streams];
+    if (ahead) {
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+#pragma unroll
+            for (int j = 0; j < kChainTaps; j++) taps_w[j][e] = *(const f32x4*)(a.conv_w + (int64_t)from[e] * kChainTaps + 4 * j);  // channel from + j's
+#pragma unroll
+            for (int j = 0; j + 1 < kChainTaps; j++) hist[j][e] = *(const f32x4*)(a.conv_state + (r * (kChainTaps - 1) + j) * W + from[e]);
+        }
+    }
+    if constexpr (FEW) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < E; e++)
+        if (!in[e]) y[e] = x[e] = zero;
+    if (averages)
+        for (int j0 = 0; j0 < a.n_streams; j0 += N) {
+            if (j0 > 0) {
+                earlier_from(j0);
+#pragma unroll
+                for (int u = 0; u < N; u++) dw[u] = a.dwa[j0 + u < a.n_streams ? j0 + u : a.n_streams - 1];
+            }
+#pragma unroll
+            for (int u = 0; u < N; u++) {
+                if (j0 + u >= a.n_streams) break;
+#pragma unroll
+                for (int e = 0; e < E; e++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) avg[e][i] = fmaf(dw[u], earlier[u][e][i], avg[e][i]);
             }
         }
     if (a.w_post) norm(y, part[0], z);
-    const float own = a.dwa ? a.dwa[a.n_streams] : 1.f;
 #pragma unroll
     for (int e = 0; e < E; e++) {
         if (!in[e]) continue;
@@ -210,19 +256,31 @@ __global__ __launch_bounds__(1024) void norm_chain_wide_kernel(NormChain a) {
     for (int e = 0; e < E; e++) {
         if (!in[e]) continue;
         h[e] = h[e] * wn[e];
-        if (a.conv_w) {
+        if (ahead) {
+            f32x4 acc = zero;
+            float* to = a.conv_state + r * (kChainTaps - 1) * W + at[e];
+#pragma unroll
+            for (int j = 0; j + 1 < kChainTaps; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = fmaf(taps_w[i][e][j], hist[j][e][i], acc[i]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] = fmaf(taps_w[i][e][kChainTaps - 1], h[e][i], acc[i]);
+#pragma unroll
+            for (int j = 0; j + 1 < kChainTaps; j++) *(f32x4*)(to + (int64_t)j * W) = j + 2 < kChainTaps ? hist[j + 1][e] : h[e];
+            h[e] = h[e] + acc;
+        } else if (a.conv_w) {
             const float* w = a.conv_w + (int64_t)at[e] * a.taps;
-            float* hist = a.conv_state + r * (a.taps - 1) * W + at[e];
+            float* hist_at = a.conv_state + r * (a.taps - 1) * W + at[e];
             f32x4 acc = zero;
             for (int j = 0; j + 1 < a.taps; j++) {
-                const f32x4 old = *(const f32x4*)(hist + (int64_t)j * W);
+                const f32x4 old = *(const f32x4*)(hist_at + (int64_t)j * W);
 #pragma unroll
                 for (int i = 0; i < 4; i++) acc[i] = fmaf(w[i * a.taps + j], old[i], acc[i]);
-                if (j > 0) *(f32x4*)(hist + (int64_t)(j - 1) * W) = old;
+                if (j > 0) *(f32x4*)(hist_at + (int64_t)(j - 1) * W) = old;
             }
 #pragma unroll
             for (int i = 0; i < 4; i++) acc[i] = fmaf(w[(i + 1) * a.taps - 1], h[e][i], acc[i]);
-            if (a.taps > 1) *(f32x4*)(hist + (int64_t)(a.taps - 2) * W) = h[e];
+            if (a.taps > 1) *(f32x4*)(hist_at + (int64_t)(a.taps - 2) * W) = h[e];
             h[e] = h[e] + acc;
         }
         if (a.h_f32) *(f32x4*)(a.h_f32 + r * a.ldh + at[e]) = h[e];
@@ -286,7 +344,16 @@ __global__ __launch_bounds__(1024) void gated_norm_wide_kernel(const float* __re
         ss = 0.f;
         for (int k = 0; k < gs >> 8; k++) ss += part[(i / gs) * (gs >> 8) + k];
     } else {
-        for (int d = gs >> 3; d > 0; d >>= 1) ss += __shfl_xor(ss, d);
+        // gs / 4 lanes, a power of two: over pairs, quads, ... by exchanges of registers
+        if (gs >= 8) ss += dpp_f32<0xb1>(ss);    // quad_perm [1,0,3,2]
+        if (gs >= 16) ss += dpp_f32<0x4e>(ss);   // quad_perm [2,3,0,1]
+        if (gs >= 32) ss += dpp_f32<0x141>(ss);  // row_half_mirror
+        if (gs >= 64) ss += dpp_f32<0x140>(ss);  // row_mirror
+        if (gs >= 128) {
+            float other = ss;
+            swap_rows(ss, other);
+            ss += other;
+        }
     }
     const float scale = 1.f / __builtin_sqrtf(ss / (float)gs + eps);
     f32x4 y;
@@ -372,12 +439,14 @@ hipError_t norm_chain(const NormChain& a, int64_t rows, hipStream_t st) {
     if (rows == 0) return hipSuccess;
     auto whole = [](const void* p, int64_t ld) { return !p || (((uintptr_t)p & 15) == 0 && ld % 4 == 0); };
     if (a.width / a.groups % 256 == 0 && a.width <= 16384 && whole(a.table, a.table_ld) && whole(a.pairs.table, a.pairs.ld) && whole(a.y, a.ldy) && whole(a.x, 4) && whole(a.h_f32, a.ldh) &&
-        whole(a.h_bf16, a.ldh) && whole(a.streams, a.stream_stride) && whole(a.stream_out, 4) && whole(a.x_out, 4) && whole(a.conv_state, 4)) {
+        whole(a.h_bf16, a.ldh) && whole(a.streams, a.stream_stride) && whole(a.stream_out, 4) && whole(a.x_out, 4) && whole(a.conv_state, 4) && whole(a.conv_w, 4)) {
         const int threads = a.width < 4096 ? a.width / 4 : 1024;  // a multiple of 64
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(threads), 0, st, a); };
-        if (a.width <= 4096) a.tokens ? launch(norm_chain_wide_kernel<1, true>) : launch(norm_chain_wide_kernel<1, false>);
-        else if (a.width <= 8192) a.tokens ? launch(norm_chain_wide_kernel<2, true>) : launch(norm_chain_wide_kernel<2, false>);
-        else a.tokens ? launch(norm_chain_wide_kernel<4, true>) : launch(norm_chain_wide_kernel<4, false>);
+        // a thread of more than one run has no registers for what is requested ahead
+        if (a.width <= 4096 && rows <= kFewRows) a.tokens ? launch(norm_chain_wide_kernel<1, true, true>) : launch(norm_chain_wide_kernel<1, false, true>);
+        else if (a.width <= 4096) a.tokens ? launch(norm_chain_wide_kernel<1, true, false>) : launch(norm_chain_wide_kernel<1, false, false>);
+        else if (a.width <= 8192) a.tokens ? launch(norm_chain_wide_kernel<2, true, false>) : launch(norm_chain_wide_kernel<2, false, false>);
+        else a.tokens ? launch(norm_chain_wide_kernel<4, true, false>) : launch(norm_chain_wide_kernel<4, false, false>);
         return hipGetLastError();
     }
     const int threads = row_threads(a.width);

@@ -293,6 +293,23 @@ def test_greedy_generation(mixed):
     assert X.error(more, F.forward(c, w, np.concatenate([prompt, replayed[0]]))[-1:]) < TOL["float32"]
 
 
+@pytest.mark.parametrize("taps,width,layers", [(4, 512, 10), (3, 512, 5), (4, 1024, 2)])
+def test_steps_of_rows_in_whole_runs(tmp_path, taps, width, layers):
+    """Rows of whole runs of 256 elements a group, whose norms request a convolution's inputs (of four taps) and the earlier layers' results (four at a
+    time) ahead: a step's logits of five sequences, one to twelve positions on, and each of them in one call, against the plain forward."""
+    c = X.config([X.lightning(heads=2, decay=[0.9, 0.5], ff=96 if i % 2 else None) for i in range(layers)], width=width, groups=2, taps=taps)
+    w = X.weights(c, 13)
+    prompts = X.tokens(c, 9, 13, batch=5)
+    gpu.say(f"fuvolix whole runs {taps} {width} {layers}")
+    m = load(tmp_path, c, w, context=24, batch=5, max_tokens=9)
+    out, _ = m.generate(prompts, 12)
+    step = m.logits(out[:, -1:])
+    for b in range(5):
+        lg = F.forward(c, w, np.concatenate([prompts[b], out[b]]))
+        assert np.all(lg[8:-1].max(1) - lg[np.arange(8, 20), out[b]] < 1e-3 * lg.std())
+        assert X.error(step[b:b + 1], lg[-1:]) < TOL["float32"]
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_generation_of_several_sequences(mixed, dtype):
     """Each of the sequences chooses as it does alone (bfloat16: as long as no two logits are closer than its rounding)."""

@@ -226,6 +226,12 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
     if ((dtype == MI355X_Q4_K || dtype == MI355X_Q6_K) && g_tune_gemm != 1 && ((uintptr_t)X & 7) == 0 && x_row_stride % 4 == 0) {
         // the int8 rounding reads the bfloat16 rows directly and the matrix-core kernel rounds its results
         void* act;
+        if (mimir::qgemm_kquant_shared_pays(dtype, W, M, N, K)) {
+            if (mi355x_status s2 = act_scratch(stream, mimir::kq_lanes_bytes(M, K), &act)) return s2;
+            HIP_TRY(mimir::kq_convert_act_bf16(X, M, K, x_row_stride, act, st, true), "launch kq_convert_act");
+            HIP_TRY(mimir::qgemm_kquant_shared(dtype, mimir::QGemvArgs{W, nullptr, act, (float*)Y, M, N, K, 0, 0}, st, !f32), "launch qgemm_kquant_shared");
+            return MI355X_OK;
+        }
         if (mi355x_status s2 = act_scratch(stream, mimir::kq_act_bytes(K) * (size_t)M, &act)) return s2;
         mimir::QGemvArgs a{W, nullptr, act, (float*)Y, M, N, K, 0, 0};
         if (mimir::qgemv_kquant_rows_pays(dtype, a)) {  // a few rows: W read once per eight of them, the same bits, one rounding after
@@ -383,6 +389,13 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             return MI355X_OK;
         }
         void* act;
+        if (mimir::qgemm_kquant_shared_pays(dtype, W, M, N, K) && (!src.fixed || mimir::kq_lanes_bytes(M, K) <= kNoallocActBytes)) {
+            if (mi355x_status st = act_for(src, mimir::kq_lanes_bytes(M, K), &act)) return st;
+            HIP_TRY(mimir::kq_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream, true), "launch kq_convert_act");
+            a.act = act;
+            HIP_TRY(mimir::qgemm_kquant_shared(dtype, a, (hipStream_t)stream), "launch qgemm_kquant_shared");
+            return MI355X_OK;
+        }
         if (mi355x_status st = act_for(src, mimir::kq_act_bytes(K) * (size_t)M, &act)) return st;
         HIP_TRY(mimir::kq_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch kq_convert_act");
         a.act = act;
@@ -724,6 +737,10 @@ mi355x_status mi355x_tune(const char* key, int value) {
     }
     if (key && strcmp(key, "kquant.mfma_rows_waves") == 0) {
         mimir::set_kquant_rows_waves(value);
+        return MI355X_OK;
+    }
+    if (key && strcmp(key, "kquant.shared") == 0) {
+        mimir::set_kquant_shared(value);
         return MI355X_OK;
     }
     if (key && strcmp(key, "kquant.mfma_rows") == 0) {

@@ -143,19 +143,21 @@ hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st);
 // to int8 in super-blocks of 256 with the sums of each 16 quants
 // (kq_convert_act, kq_act_bytes(K) bytes per row), integer dot products.
 size_t kq_act_bytes(int64_t K);
-hipError_t kq_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
+size_t kq_lanes_bytes(int64_t M, int64_t K);  // with `lanes`, here and below: the rows in the order of the lanes (kq_act.h), for qgemm_kquant_shared
+hipError_t kq_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st, bool lanes = false);
 // RMSNorm then conversion, and SiLU(g) * u then conversion, each in one launch and with the separate
 // kernels' arithmetic (d and n multiples of 256; x, w, g, u 16-byte aligned).
-hipError_t rmsnorm_kq_act(const float* x, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st);
-hipError_t swiglu_kq_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st);
+hipError_t rmsnorm_kq_act(const float* x, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st, bool lanes = false);
+hipError_t swiglu_kq_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st, bool lanes = false);
 // The same from bfloat16 rows (8-byte aligned, a multiple of 4 elements apart).
-hipError_t kq_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
+hipError_t kq_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st, bool lanes = false);
 // With a.act null and qgemv_kquant_rope_ok(dt, a): one launch from float32 a.x (16-byte aligned rows), rounded by every workgroup.
 hipError_t qgemv_kquant_act(int dt, const QGemvArgs& a, hipStream_t st);
 // The same products for many rows of x on the matrix cores (qgemm_kquant.hip); qgemv_kquant_act
 // hands over to it where qgemm_kquant_pays says it is the faster of the two.
 bool qgemm_kquant_pays(int dt, const QGemvArgs& a);
 double qgemm_kquant_us(int64_t M, int64_t N, int64_t K);
+double qgemv_kquant_us(int dt, int64_t M, int64_t N, int64_t K);
 bool qgemm_kquant_ok(int dt, const QGemvArgs& a);
 // y float32, or with out_bf16 each result rounded once to bfloat16 into y taken as uint16_t*.
 hipError_t qgemm_kquant(int dt, const QGemvArgs& a, hipStream_t st, bool out_bf16 = false);
@@ -172,6 +174,15 @@ hipError_t qgemv_kquant_rows(int dt, const QGemvArgs& a, hipStream_t st, bool y_
 bool qgemv_kquant_rows_rope_ok(int dt, const QGemvArgs& a);
 hipError_t qgemv_kquant_rows_rope(int dt, const QGemvArgs& a, const Q4RopeTail& rope, hipStream_t st);
 void set_kquant_rows(int v);
+bool kquant_rows_by_rule();  // no measurement aid has a say, among those above
+bool kquant_by_rule();       // nor any of set_kquant_tune
+// Some rows of x, W read once for up to 64 of them (qgemm_kquant_shared.hip), the CPU's bits too. a.act: rows in the order of lanes, so that whoever
+// converts x asks qgemm_kquant_shared_pays first ("kquant.shared": 1 never, 2 always). It never pays for more than kSharedRows rows.
+constexpr int64_t kSharedRows = 512;
+bool qgemm_kquant_shared_ok(int dt, const void* W, int64_t M, int64_t N, int64_t K);
+bool qgemm_kquant_shared_pays(int dt, const void* W, int64_t M, int64_t N, int64_t K);
+hipError_t qgemm_kquant_shared(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);
+void set_kquant_shared(int v);
 void set_kquant_rows_waves(int v);
 
 // y = x . W^T for a float32, binary16 or bfloat16 W [N, K].

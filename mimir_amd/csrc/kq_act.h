@@ -5,6 +5,10 @@
 //   u32x4 q[nsb][16]     the 256 int8 quants
 //   uint32 sums[nsb][8]  sixteen int16 sums of 16 quants, packed in pairs
 //   float d[nsb]
+// Rows for a product of some of them (qgemm_kquant_shared.hip) lie in the order of the matrix instruction's lanes instead,
+// kq_lanes_bytes(M, K) bytes, per sixteen rows and super-block kLanesBlock bytes:
+//   q[4][64][16]         of step s, lane 16 k + r: quants 64 s + 16 k .. + 15 of row r
+//   float d[16]          of the sixteen rows
 #pragma once
 #include "device_util.h"
 
@@ -16,9 +20,10 @@ __device__ __forceinline__ int dpp_i32_quad_sum(int v) {
     return v;
 }
 
-// quantizeRow for one super-block of 256 with its sums: one wavefront, lane i holding values 4i..4i+3.
-// q: the super-block's 64 dwords of quants; sums: its 16 sums; d: its scale.
-__device__ __forceinline__ void kq_convert_superblock_to(const f32x4 v, int lane, uint32_t* q, uint16_t* sums, float* d_out) {
+constexpr int kLanesBlock = 4096 + 64;
+
+// quantizeRow for one super-block of 256: one wavefront, lane i holding values 4i..4i+3. packed: the lane's quants, local: their sum, returns the scale.
+__device__ __forceinline__ float kq_round_superblock(const f32x4 v, uint32_t& packed, int& local) {
     float amax = 0.f;
     bool finite = true;
 #pragma unroll
@@ -30,8 +35,8 @@ __device__ __forceinline__ void kq_convert_superblock_to(const f32x4 v, int lane
     amax = wave_max(amax);
     float bad = wave_max(finite ? 0.f : 1.f);
     float d = 0.f;
-    uint32_t packed = 0;
-    int local = 0;
+    packed = 0;
+    local = 0;
     if (bad != 0.f) {
         d = __builtin_nanf("");
     } else if (amax != 0.f) {
@@ -45,6 +50,14 @@ __device__ __forceinline__ void kq_convert_superblock_to(const f32x4 v, int lane
             local += r;
         }
     }
+    return d;
+}
+
+// The same with its sums. q: the super-block's 64 dwords of quants; sums: its 16 sums; d: its scale.
+__device__ __forceinline__ void kq_convert_superblock_to(const f32x4 v, int lane, uint32_t* q, uint16_t* sums, float* d_out) {
+    uint32_t packed;
+    int local;
+    const float d = kq_round_superblock(v, packed, local);
     q[lane] = packed;
     int s16 = dpp_i32_quad_sum(local);  // 16 quants = 4 consecutive lanes
     if ((lane & 3) == 0) sums[lane >> 2] = (uint16_t)(int16_t)s16;
@@ -55,6 +68,17 @@ __device__ __forceinline__ void kq_convert_superblock_to(const f32x4 v, int lane
 __device__ __forceinline__ void kq_convert_superblock(const f32x4 v, int sb, int lane, int nsb, uint8_t* __restrict__ row) {
     kq_convert_superblock_to(v, lane, (uint32_t*)row + (int64_t)sb * 64, (uint16_t*)(row + (int64_t)nsb * 256) + sb * 16,
                              (float*)(row + (int64_t)nsb * 288) + sb);
+}
+
+// Row m of the call's, into the form in the order of lanes.
+__device__ __forceinline__ void kq_convert_superblock_lanes(const f32x4 v, int64_t m, int sb, int lane, int nsb, uint8_t* __restrict__ act) {
+    uint32_t packed;
+    int local;
+    const float d = kq_round_superblock(v, packed, local);
+    const int r = (int)(m & 15);
+    uint8_t* block = act + ((m >> 4) * nsb + sb) * kLanesBlock;
+    *(uint32_t*)(block + (lane >> 4) * 1024 + ((lane >> 2) & 3) * 256 + 16 * r + 4 * (lane & 3)) = packed;
+    if (lane == 0) *(float*)(block + 4096 + 4 * r) = d;
 }
 
 }  // namespace mimir

@@ -36,8 +36,9 @@ namespace {
 #define LLM_HIP(expr, what) DECODER_HIP(expr, "llama", what)
 
 // The form of converted activations a weight's product reads.
-// kActFx: Q4_0 by many rows of x, on the int8 matrix cores; kActFxPairs: on the binary16 ones, x as pairs of binary16 numbers
-enum ActClass { kActNone = 0, kActQ4 = 1, kActQ8 = 2, kActKQ = 3, kActFx = 4, kActFxPairs = 5, kActClasses = 6 };
+// kActFx: Q4_0 by many rows of x, on the int8 matrix cores; kActFxPairs: on the binary16 ones, x as pairs of binary16 numbers;
+// kActKQLanes: K-quants by some rows of x, laid out for the matrix cores' lanes
+enum ActClass { kActNone = 0, kActQ4 = 1, kActQ8 = 2, kActKQ = 3, kActFx = 4, kActFxPairs = 5, kActKQLanes = 6, kActClasses = 7 };
 
 // qkv and gate_up: where q, k, v (gate, up) share a block dtype, finalize also keeps their rows in one
 // buffer, which a decoding step multiplies in one product (the reference concatenates the same
@@ -92,8 +93,11 @@ struct Model : Decoder {
     bool one_token_as_step() const override { return fast && c.batch <= 16; }
 };
 
+bool is_kquant(const Weight& w) { return w.set() && (w.dtype == kQ4_K || w.dtype == kQ6_K); }
+
 // panel_bytes: what the model holds as workspace for the fixed-point product's binary16 form (0: that form is not taken)
-int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0) {
+// lead: of the matrices that multiply one x the first, which decides the form of the K-quants' x for all of them
+int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0, const Weight* lead = nullptr) {
     switch (w.dtype) {
     case kQ4_0:
         if (rows > 1 && panel_bytes) {
@@ -103,7 +107,10 @@ int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0) {
         if (qgemm_q4_0_fx_pays(w.buf.p, rows, w.n, w.k)) return kActFx;
         return q4_0_fixed_point_ok(w.buf.p, w.k) ? kActQ4 : kActNone;
     case kQ8_0: return q8_act_fits(w.k) ? kActQ8 : kActNone;
-    case kQ4_K: case kQ6_K: return kActKQ;
+    case kQ4_K: case kQ6_K: {
+        const Weight& by = lead && is_kquant(*lead) ? *lead : w;
+        return qgemm_kquant_shared_pays(by.dtype, by.buf.p, rows, by.n, by.k) ? kActKQLanes : kActKQ;
+    }
     default: return kActNone;
     }
 }
@@ -111,6 +118,7 @@ int act_class(const Weight& w, int64_t rows = 1, size_t panel_bytes = 0) {
 // Bytes of `rows` converted rows of K.
 size_t act_bytes(int cls, int64_t rows, int64_t K) {
     if (cls == kActFxPairs) return q4_0_fx16_act_bytes(rows, K);
+    if (cls == kActKQLanes) return kq_lanes_bytes(rows, K);
     const size_t n = (size_t)rows;
     switch (cls) {
     case kActQ4: return n * q4_0_act_bytes(K);
@@ -127,7 +135,7 @@ const int kNoTune[5] = {0, 0, 0, 0, 0};
 mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std::initializer_list<const Weight*> ws, bool done[kActClasses]) {
     for (int i = 0; i < kActClasses; i++) done[i] = false;
     for (const Weight* w : ws) {
-        int cls = act_class(*w, rows, m.fx_panel.bytes);
+        int cls = act_class(*w, rows, m.fx_panel.bytes, *ws.begin());
         if (cls == kActNone || done[cls]) continue;
         size_t need = act_bytes(cls, rows, K);
         if (m.act[cls].bytes < need) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: activation scratch of %zu bytes, need %zu", m.act[cls].bytes, need);
@@ -137,7 +145,7 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
                        : cls == kActQ8 ? q8_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActFx ? q4_0_fx_convert_act(x, rows, K, K, m.act[cls].p, m.stream)
                        : cls == kActFxPairs ? q4_0_fx16_convert_act(x, rows, K, K, m.act[cls].p, form, m.stream)
-                                       : kq_convert_act(x, rows, K, K, m.act[cls].p, m.stream);
+                                       : kq_convert_act(x, rows, K, K, m.act[cls].p, m.stream, cls == kActKQLanes);
         LLM_HIP(e, "convert activations");
         done[cls] = true;
     }
@@ -146,8 +154,7 @@ mi355x_status convert_for(Model& m, const float* x, int64_t rows, int64_t K, std
 
 // y[rows, n] = x[rows, k] . W^T (nn/layers.go:49-55 -> tensor/quant.go:35-56).
 // With resid, y = product + resid (which may be y): every form of converted x has a kernel that adds it as it stores.
-mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_t rows, const float* resid = nullptr) {
-    int cls = act_class(w, rows, m.fx_panel.bytes);
+mi355x_status linear_by(Model& m, int cls, const Weight& w, const float* x, float* y, int64_t rows, const float* resid = nullptr) {
     if (resid && cls == kActNone) return capi_fail(MI355X_ERR_INTERNAL, "mi355x: llama: no residual epilogue for this product");
     QGemvArgs a{w.buf.p, x, m.act[cls].p, y, rows, w.n, w.k, w.k, 0};
     a.resid = resid;
@@ -168,12 +175,15 @@ mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_
         // several rows: W read once, on the matrix cores where the matrix is large
         e = qgemv_q8_0_mfma_pays(a) ? qgemv_q8_0_mfma(a, m.stream) : qgemv_q8_0_rows_ok(a) ? qgemv_q8_0_rows(a, m.stream) : qgemv_q8_0_act(a, kNoTune, m.stream);
         break;
-    case kQ4_K: case kQ6_K: e = qgemv_kquant_act(w.dtype, a, m.stream); break;
+    case kQ4_K: case kQ6_K: e = cls == kActKQLanes ? qgemm_kquant_shared(w.dtype, a, m.stream) : qgemv_kquant_act(w.dtype, a, m.stream); break;
     case kF32: case kF16: case kBF16: e = gemv_float(w.dtype, w.buf.p, x, y, rows, w.n, w.k, w.k, m.stream); break;
     default: return capi_fail(MI355X_ERR_DTYPE, "mi355x: llama: a linear weight of dtype %d", w.dtype);
     }
     LLM_HIP(e, "linear");
     return MI355X_OK;
+}
+mi355x_status linear(Model& m, const Weight& w, const float* x, float* y, int64_t rows, const float* resid = nullptr, const Weight* lead = nullptr) {
+    return linear_by(m, act_class(w, rows, m.fx_panel.bytes, lead), w, x, y, rows, resid);
 }
 
 // The products of one x by several Q4_0 matrices, or silu(gate) up of two, as one (qgemm_q4_0_fx16_parts), where that pays:
@@ -208,9 +218,6 @@ mi355x_status embed_rows(Model& m, const int32_t* idx_dev, int64_t rows, float* 
 
 }  // namespace
 
-// Matrices of one K-quant dtype kept in one buffer: their products are one, by x converted as it is normalized.
-static bool kq_together(const Weight& w) { return w.set() && (w.dtype == kQ4_K || w.dtype == kQ6_K); }
-
 // One pass of s tokens per sequence over the blocks (llm/model.go:391-437),
 // tokens already on the device at m.tokens_dev [batch, s]. Leaves the final
 // hidden state in m.x; advances the caches.
@@ -225,7 +232,7 @@ static mi355x_status forward(Model& m, int64_t s) {
     // x += in . W^T: the prompt-sized fixed-point products and the K-quants' add x as they store, the others leave it to a launch
     auto onto_x = [&](const Weight& w, const float* in) -> mi355x_status {
         const int cls = act_class(w, rows, m.fx_panel.bytes);
-        if (cls == kActFx || cls == kActFxPairs || cls == kActKQ) return linear(m, w, in, x, rows, x);
+        if (cls == kActFx || cls == kActFxPairs || cls == kActKQ || cls == kActKQLanes) return linear(m, w, in, x, rows, x);
         if (mi355x_status st = linear(m, w, in, o, rows)) return st;
         LLM_HIP(add(x, o, x, rows * c.embed, m.stream), "residual");
         return MI355X_OK;
@@ -236,18 +243,19 @@ static mi355x_status forward(Model& m, int64_t s) {
         if (mi355x_status st = linear_parts(m, {&b.q, &b.k, &b.v}, {q, k, v}, false, x, b.attn_norm, rows, &together)) return st;
         float *qp = q, *kp = k, *vp = v;
         int64_t qld = qd, kld = kvd;  // between positions
-        if (!together && kq_together(b.qkv) && qd + 2 * kvd <= 2 * (int64_t)c.hidden &&
+        if (!together && is_kquant(b.qkv) && qd + 2 * kvd <= 2 * (int64_t)c.hidden &&
             rope_kv_prompt_ok(gate, gate + qd, gate + qd + kvd, qd + 2 * kvd, qd + 2 * kvd, qd + 2 * kvd, c.head_dim, c.rope_dim)) {
-            LLM_HIP(rmsnorm_kq_act(x, b.attn_norm.buf.as<float>(), m.act[kActKQ].p, rows, c.embed, c.eps, m.stream), "attn_norm");
-            if (mi355x_status st = linear(m, b.qkv, h, gate, rows)) return st;
+            const int cls = act_class(b.qkv, rows);
+            LLM_HIP(rmsnorm_kq_act(x, b.attn_norm.buf.as<float>(), m.act[cls].p, rows, c.embed, c.eps, m.stream, cls == kActKQLanes), "attn_norm");
+            if (mi355x_status st = linear_by(m, cls, b.qkv, h, gate, rows)) return st;
             qp = gate, kp = gate + qd, vp = gate + qd + kvd;
             qld = kld = qd + 2 * kvd;
         } else if (!together) {
             LLM_HIP(rmsnorm(x, b.attn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "attn_norm");
             if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.q, &b.k, &b.v}, done)) return st;
             if (mi355x_status st = linear(m, b.q, h, q, rows)) return st;
-            if (mi355x_status st = linear(m, b.k, h, k, rows)) return st;
-            if (mi355x_status st = linear(m, b.v, h, v, rows)) return st;
+            if (mi355x_status st = linear(m, b.k, h, k, rows, nullptr, &b.q)) return st;
+            if (mi355x_status st = linear(m, b.v, h, v, rows, nullptr, &b.q)) return st;
         }
         const float* bias = b.biased() ? b.qkv_bias.as<float>() : nullptr;  // behind the product, before the rotation (nn/layers.go:49-55)
         if (rope_kv_prompt_ok(qp, kp, vp, qld, kld, kld, c.head_dim, c.rope_dim)) {
@@ -296,17 +304,18 @@ static mi355x_status forward(Model& m, int64_t s) {
         if (mi355x_status st = onto_x(b.o, a)) return st;
         if (mi355x_status st = linear_parts(m, {&b.gate, &b.up}, {sw, nullptr}, true, x, b.ffn_norm, rows, &together)) return st;
         bool converted = false;
-        if (!together && kq_together(b.gate_up)) {
-            LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[kActKQ].p, rows, c.embed, c.eps, m.stream), "ffn_norm");
-            if (mi355x_status st = linear(m, b.gate_up, h, gate, rows)) return st;
-            converted = act_class(b.down, rows, m.fx_panel.bytes) == kActKQ;
-            if (converted) LLM_HIP(swiglu_kq_act(gate, gate + c.hidden, m.act[kActKQ].p, rows, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
+        if (!together && is_kquant(b.gate_up)) {
+            const int cls = act_class(b.gate_up, rows), down = act_class(b.down, rows, m.fx_panel.bytes);
+            LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[cls].p, rows, c.embed, c.eps, m.stream, cls == kActKQLanes), "ffn_norm");
+            if (mi355x_status st = linear_by(m, cls, b.gate_up, h, gate, rows)) return st;
+            converted = down == kActKQ || down == kActKQLanes;
+            if (converted) LLM_HIP(swiglu_kq_act(gate, gate + c.hidden, m.act[down].p, rows, c.hidden, 2 * (int64_t)c.hidden, m.stream, down == kActKQLanes), "swiglu");
             else LLM_HIP(swiglu(gate, gate + c.hidden, sw, rows, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
         } else if (!together) {
             LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, rows, c.embed, c.eps, m.stream), "ffn_norm");
             if (mi355x_status st = convert_for(m, h, rows, c.embed, {&b.gate, &b.up}, done)) return st;
             if (mi355x_status st = linear(m, b.gate, h, gate, rows)) return st;
-            if (mi355x_status st = linear(m, b.up, h, up, rows)) return st;
+            if (mi355x_status st = linear(m, b.up, h, up, rows, nullptr, &b.gate)) return st;
             LLM_HIP(swiglu(gate, up, sw, rows, c.hidden, c.hidden, m.stream), "swiglu");
         }
         if (!converted)
@@ -499,7 +508,7 @@ static mi355x_status step_any(Model& m) {
     if (!one_launch) attention_plan(B, c.heads, c.kv_heads, 1, c.context, &at.chunk, &at.nsplit);
     for (int i = 0; i < c.layers; i++) {
         Block& b = m.blocks[i];
-        const bool qkv_kq = b.qkv.set() && act_class(b.qkv, B) == kActKQ;
+        const bool qkv_kq = is_kquant(b.qkv);  // x by rows: the rotation and the cache writes ride on that product
         if (qkv_kq) {  // norm and conversion in one launch
             LLM_HIP(rmsnorm_kq_act(x, b.attn_norm.buf.as<float>(), m.act[kActKQ].p, B, c.embed, c.eps, m.stream), "attn_norm");
         } else {
@@ -523,7 +532,7 @@ static mi355x_status step_any(Model& m) {
                 else LLM_HIP(qgemv_kquant_act_rope(b.qkv.dtype, qa, tail, m.stream), "q|k|v, rope and cache");
             } else {
                 // with biases (qwen2): one product, then the biases, the rotation and the cache writes in one launch
-                if (mi355x_status st = linear(m, b.qkv, h, qkv, B)) return st;
+                if (mi355x_status st = linear_by(m, qkv_kq ? (int)kActKQ : act_class(b.qkv, B, m.fx_panel.bytes), b.qkv, h, qkv, B)) return st;
                 LLM_HIP(rope_kv(qkv, m.keys[i].p, m.values[i].p, c.cache_dtype, B, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.interleaved,
                                 c.context, m.cos_t.as<float>(), m.sin_t.as<float>(), pos, m.stream,
                                 b.biased() ? b.qkv_bias.as<float>() : nullptr), "biases, rope and cache");
@@ -532,8 +541,8 @@ static mi355x_status step_any(Model& m) {
         } else {
             if (mi355x_status st = convert_for(m, h, B, c.embed, {&b.q, &b.k, &b.v}, done)) return st;
             if (mi355x_status st = linear(m, b.q, h, q, B)) return st;
-            if (mi355x_status st = linear(m, b.k, h, k, B)) return st;
-            if (mi355x_status st = linear(m, b.v, h, v, B)) return st;
+            if (mi355x_status st = linear(m, b.k, h, k, B, nullptr, &b.q)) return st;
+            if (mi355x_status st = linear(m, b.v, h, v, B, nullptr, &b.q)) return st;
             // biases (qwen2), rotation and cache writes in one launch
             LLM_HIP(rope_kv_split(q, k, v, m.keys[i].p, m.values[i].p, c.cache_dtype, B, c.heads, c.kv_heads, c.head_dim, c.rope_dim,
                                   c.interleaved, c.context, m.cos_t.as<float>(), m.sin_t.as<float>(), pos, m.stream,
@@ -542,7 +551,7 @@ static mi355x_status step_any(Model& m) {
         }
         at.k = m.keys[i].p; at.v = m.values[i].p;
         // K-quant output projection: attention leaves its result as the int8 super-blocks that product reads
-        const bool a_kq = one_launch && act_class(b.o, B) == kActKQ && attention_decode_kq_ok(at);
+        const bool a_kq = one_launch && is_kquant(b.o) && attention_decode_kq_ok(at);
         if (a_kq) {
             LLM_HIP(attention_decode(at, c.context, m.act[0].p, m.act[kActKQ].p, (int64_t)kq_act_bytes(qd), m.stream, kAttnActKQ, m.attn_flags.p, m.attn_flags.bytes, device_error_word()), "attention");
         } else {
@@ -550,30 +559,33 @@ static mi355x_status step_any(Model& m) {
             else LLM_HIP(attention(at, (uint8_t*)m.act[0].p + kAttnTicketBytes, m.stream), "attention");
             if (mi355x_status st = convert_for(m, a, B, qd, {&b.o}, done)) return st;
         }
-        if (act_class(b.o, B) != kActNone) {  // the residual rides on the product
-            if (mi355x_status st = linear(m, b.o, a, x, B, x)) return st;
+        const int o_cls = a_kq ? (int)kActKQ : act_class(b.o, B, m.fx_panel.bytes);
+        if (o_cls != kActNone) {  // the residual rides on the product
+            if (mi355x_status st = linear_by(m, o_cls, b.o, a, x, B, x)) return st;
         } else {
             if (mi355x_status st = linear(m, b.o, a, o, B)) return st;
             LLM_HIP(add(x, o, x, B * c.embed, m.stream), "residual");
         }
-        const bool down_kq = act_class(b.down, B) == kActKQ;  // then SwiGLU leaves its result converted
-        if (b.gate_up.set() && act_class(b.gate_up, B) == kActKQ) {
-            LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[kActKQ].p, B, c.embed, c.eps, m.stream), "ffn_norm");
-            if (mi355x_status st = linear(m, b.gate_up, h, gu, B)) return st;
-            if (down_kq) LLM_HIP(swiglu_kq_act(gu, gu + c.hidden, m.act[kActKQ].p, B, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
+        const int down = act_class(b.down, B);
+        const bool down_kq = down == kActKQ || down == kActKQLanes;  // then SwiGLU leaves its result converted
+        if (is_kquant(b.gate_up)) {
+            const int cls = act_class(b.gate_up, B);
+            LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[cls].p, B, c.embed, c.eps, m.stream, cls == kActKQLanes), "ffn_norm");
+            if (mi355x_status st = linear_by(m, cls, b.gate_up, h, gu, B)) return st;
+            if (down_kq) LLM_HIP(swiglu_kq_act(gu, gu + c.hidden, m.act[down].p, B, c.hidden, 2 * (int64_t)c.hidden, m.stream, down == kActKQLanes), "swiglu");
             else LLM_HIP(swiglu(gu, gu + c.hidden, sw, B, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
         } else if (b.gate_up.set()) {  // one product into [B, gate | up]
             LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, B, c.embed, c.eps, m.stream), "ffn_norm");
             if (mi355x_status st = convert_for(m, h, B, c.embed, {&b.gate_up}, done)) return st;
             if (mi355x_status st = linear(m, b.gate_up, h, gu, B)) return st;
-            if (down_kq) LLM_HIP(swiglu_kq_act(gu, gu + c.hidden, m.act[kActKQ].p, B, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
+            if (down_kq) LLM_HIP(swiglu_kq_act(gu, gu + c.hidden, m.act[down].p, B, c.hidden, 2 * (int64_t)c.hidden, m.stream, down == kActKQLanes), "swiglu");
             else LLM_HIP(swiglu(gu, gu + c.hidden, sw, B, c.hidden, 2 * (int64_t)c.hidden, m.stream), "swiglu");
         } else {
             LLM_HIP(rmsnorm(x, b.ffn_norm.buf.as<float>(), h, B, c.embed, c.eps, m.stream), "ffn_norm");
             if (mi355x_status st = convert_for(m, h, B, c.embed, {&b.gate, &b.up}, done)) return st;
             if (mi355x_status st = linear(m, b.gate, h, gate, B)) return st;
-            if (mi355x_status st = linear(m, b.up, h, up, B)) return st;
-            if (down_kq) LLM_HIP(swiglu_kq_act(gate, up, m.act[kActKQ].p, B, c.hidden, c.hidden, m.stream), "swiglu");
+            if (mi355x_status st = linear(m, b.up, h, up, B, nullptr, &b.gate)) return st;
+            if (down_kq) LLM_HIP(swiglu_kq_act(gate, up, m.act[down].p, B, c.hidden, c.hidden, m.stream, down == kActKQLanes), "swiglu");
             else LLM_HIP(swiglu(gate, up, sw, B, c.hidden, c.hidden, m.stream), "swiglu");
         }
         if (!down_kq)
@@ -786,8 +798,8 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
     LLM_HIP(m->hlast.alloc(rows * c.embed * 4), "hipMalloc");
     const int64_t kmax = c.hidden > qd ? (c.hidden > c.embed ? c.hidden : c.embed) : (qd > c.embed ? qd : c.embed);
     for (int cls = 1; cls < kActClasses; cls++) {
-        int64_t kk = cls == kActKQ ? (kmax + 255) / 256 * 256 : cls == kActFx || cls == kActFxPairs ? (kmax + 127) / 128 * 128 : (kmax + 63) / 64 * 64;
-        LLM_HIP(m->act[cls].alloc(act_bytes(cls, rows, kk) + 64), "hipMalloc(activations)");
+        int64_t kk = cls == kActKQ || cls == kActKQLanes ? (kmax + 255) / 256 * 256 : cls == kActFx || cls == kActFxPairs ? (kmax + 127) / 128 * 128 : (kmax + 63) / 64 * 64;
+        LLM_HIP(m->act[cls].alloc(act_bytes(cls, cls == kActKQLanes ? std::min<int64_t>(rows, kSharedRows) : rows, kk) + 64), "hipMalloc(activations)");
     }
     LLM_HIP(m->act2.alloc(q4_0_act_bytes((c.hidden + 63) / 64 * 64) * c.batch + 64), "hipMalloc(activations)");
     {

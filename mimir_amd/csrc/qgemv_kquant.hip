@@ -31,6 +31,7 @@ namespace mimir {
 //   u32x4 q[nsb][16]     the 256 int8 quants
 //   uint32 sums[nsb][8]  sixteen int16 sums of 16 quants, packed in pairs
 //   float d[nsb]
+size_t kq_lanes_bytes(int64_t M, int64_t K) { return (size_t)((M + 15) / 16 * (K / 256)) * kLanesBlock; }
 size_t kq_act_bytes(int64_t K) {
     int64_t nsb = K / 256;
     return (size_t)((nsb * (256 + 32 + 4) + 15) / 16 * 16);
@@ -54,6 +55,12 @@ __device__ __forceinline__ float add_in_order(float acc, float term) {
     return acc;
 }
 
+// Super-block sb of row blockIdx.y converted: rows act_row_bytes apart, or, where that is 0, in the order of lanes.
+__device__ __forceinline__ void kq_store(const f32x4 v, int sb, int lane, int nsb, uint8_t* __restrict__ act, int64_t act_row_bytes) {
+    if (act_row_bytes) kq_convert_superblock(v, sb, lane, nsb, act + (int64_t)blockIdx.y * act_row_bytes);
+    else kq_convert_superblock_lanes(v, blockIdx.y, sb, lane, nsb, act);
+}
+
 // One wavefront per super-block.
 template <bool BF16>  // x float32, or bfloat16 (widened exactly, as the cast in front of the product does: tensor/quant.go:45-48)
 __global__ __launch_bounds__(64) void kq_convert_act_kernel(const void* __restrict__ xv, int64_t x_row_stride, int nsb,
@@ -71,7 +78,7 @@ __global__ __launch_bounds__(64) void kq_convert_act_kernel(const void* __restri
     } else {
         __builtin_memcpy(&v, (const float*)xv + at, 16);
     }
-    kq_convert_superblock(v, sb, lane, nsb, act + (int64_t)blockIdx.y * act_row_bytes);
+    kq_store(v, sb, lane, nsb, act, act_row_bytes);
 }
 
 // RMSNorm (rmsnorm_kernel's arithmetic, operation for operation: nn/transformer.go:50-61) and the
@@ -100,14 +107,14 @@ __global__ __launch_bounds__(256) void rmsnorm_kq_act_kernel(const float* __rest
             float t = v[k] * scale;
             v[k] = t * wv[k];
         }
-        kq_convert_superblock(v, sb, lane, nsb, act + (int64_t)blockIdx.y * act_row_bytes);
+        kq_store(v, sb, lane, nsb, act, act_row_bytes);
     }
 }
 
-hipError_t rmsnorm_kq_act(const float* x, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st) {
+hipError_t rmsnorm_kq_act(const float* x, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st, bool lanes) {
     if (rows == 0) return hipSuccess;
     hipLaunchKernelGGL(rmsnorm_kq_act_kernel, dim3((unsigned)((d / 256 + 3) / 4), (unsigned)rows), dim3(256), 0, st, x, w, (int)d,
-                       (float)(1.0 / (double)d), (float)eps, (uint8_t*)act, (int64_t)kq_act_bytes(d));
+                       (float)(1.0 / (double)d), (float)eps, (uint8_t*)act, lanes ? 0 : (int64_t)kq_act_bytes(d));
     return hipGetLastError();
 }
 
@@ -128,28 +135,28 @@ __global__ __launch_bounds__(64) void swiglu_kq_act_kernel(const float* __restri
         float a = gv[k] * sg;
         v[k] = a * uv[k];
     }
-    kq_convert_superblock(v, sb, lane, nsb, act + (int64_t)blockIdx.y * act_row_bytes);
+    kq_store(v, sb, lane, nsb, act, act_row_bytes);
 }
 
-hipError_t swiglu_kq_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st) {
+hipError_t swiglu_kq_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st, bool lanes) {
     if (rows == 0) return hipSuccess;
     int nsb = (int)(n / 256);
     hipLaunchKernelGGL(swiglu_kq_act_kernel, dim3((unsigned)nsb, (unsigned)rows), dim3(64), 0, st, g, u, stride, nsb, (uint8_t*)act,
-                       (int64_t)kq_act_bytes(n));
+                       lanes ? 0 : (int64_t)kq_act_bytes(n));
     return hipGetLastError();
 }
 
-hipError_t kq_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
+hipError_t kq_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st, bool lanes) {
     int nsb = (int)(K / 256);
     hipLaunchKernelGGL(kq_convert_act_kernel<false>, dim3((unsigned)nsb, (unsigned)M), dim3(64), 0, st, (const void*)x, x_row_stride,
-                       nsb, (uint8_t*)act, (int64_t)kq_act_bytes(K));
+                       nsb, (uint8_t*)act, lanes ? 0 : (int64_t)kq_act_bytes(K));
     return hipGetLastError();
 }
 
-hipError_t kq_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
+hipError_t kq_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st, bool lanes) {
     int nsb = (int)(K / 256);
     hipLaunchKernelGGL(kq_convert_act_kernel<true>, dim3((unsigned)nsb, (unsigned)M), dim3(64), 0, st, x, x_row_stride, nsb,
-                       (uint8_t*)act, (int64_t)kq_act_bytes(K));
+                       (uint8_t*)act, lanes ? 0 : (int64_t)kq_act_bytes(K));
     return hipGetLastError();
 }
 
@@ -548,6 +555,7 @@ __global__ __launch_bounds__(kKqThreads) void qgemv_q6k_kernel(const uint8_t* __
 // [0] rows per wavefront (0: by shape). [1] 1: always the kernels without LDS, 2: never the
 // matrix-core kernel, 3: the matrix-core kernel for any number of rows.
 static std::atomic<int> g_kq_tune[2] = {{0}, {0}};
+bool kquant_by_rule() { return g_kq_tune[0] == 0 && g_kq_tune[1] == 0 && kquant_rows_by_rule(); }
 void set_kquant_tune(int which, int value) {
     if (which >= 0 && which < 2) g_kq_tune[which] = value;
 }

@@ -359,6 +359,7 @@ __global__ __launch_bounds__(64 * kWaves) void qgemv_kq_rows_kernel(const uint8_
 
 static std::atomic<int> g_kq_rows{0};  // measurement aid: 1 = never, 2 = for any number of rows the kernel takes
 void set_kquant_rows(int v) { g_kq_rows = v; }
+bool kquant_rows_by_rule() { return g_kq_rows == 0; }
 
 static std::atomic<int> g_kq_rows_waves{0};  // measurement aid: 4, 8 or 16 wavefronts to a workgroup where there is a form of that many
 void set_kquant_rows_waves(int v) { g_kq_rows_waves = v == 4 || v == 8 || v == 16 ? v : 0; }
@@ -391,16 +392,23 @@ static bool one_row_pays(int dt, const QGemvArgs& a) {
 // rows of more than 32 super-blocks leave LDS room for fewer workgroups; the tiled kernel qgemm_kquant_us. On 950 products of 9 to 512 rows, 512 x 1024 to 32768 x 8192
 // and 14336 x 14336, the choice takes 0.04 % longer than the faster kernel in the mean, 11 % at most. us, here | there: Q4_K 79 x 5248 x 1024 9.1 | 10.9, 58 x 4160 x 8960 48 | 55, 300 x 1152 x 4096 22.6 | 27,
 // 83 x 5632 x 13312 103 | 85, 205 x 2688 x 2560 22.3 | 19.2; Q6_K 25 x 22272 x 2048 25.5 | 31.2, 64 x 5184 x 2048 16.3 | 17.4, 41 x 10432 x 1792 21.0 | 16.0, 98 x 3520 x 3072 21.0 | 23.2.
+static double rows_us(int dt, int64_t M, int64_t N, int64_t nsb) {
+    const int64_t sixteens = (N + 15) / 16 * ((M + kRows - 1) / kRows);
+    const double each = (double)nsb + 0.5 * (double)(-nsb & 3), ns = dt == kQ4_K ? (nsb <= 8 ? 0.378 : 0.42) : 0.56;
+    return 3 + (double)sixteens * each * ns * 1e-3 * (nsb > 32 ? 1.1 : 1);
+}
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a) {
     if (!qgemv_kquant_rows_ok(dt, a)) return false;
     if (a.M == 1) return one_row_pays(dt, a);
     if (g_kq_rows == 2 || a.M <= 8) return true;
     if (a.M > 512) return false;
-    const bool q4 = dt == kQ4_K;
-    const int64_t nsb = a.K / 256, sixteens = (a.N + 15) / 16 * ((a.M + kRows - 1) / kRows);
-    const double each = (double)nsb + 0.5 * (double)(-nsb & 3), ns = q4 ? (nsb <= 8 ? 0.378 : 0.42) : 0.56;
-    const double rows_us = 3 + (double)sixteens * each * ns * 1e-3 * (nsb > 32 ? 1.1 : 1);
-    return rows_us < 3 + 1.4 * (double)nsb || rows_us < qgemm_kquant_us(a.M, a.N, a.K);  // no product takes less than one round of short tiles
+    const double us = rows_us(dt, a.M, a.N, a.K / 256);
+    return us < 3 + 1.4 * (double)(a.K / 256) || us < qgemm_kquant_us(a.M, a.N, a.K);  // no product takes less than one round of short tiles
+}
+// What 9 to 512 rows take by the one of these two.
+double qgemv_kquant_us(int dt, int64_t M, int64_t N, int64_t K) {
+    const double us = rows_us(dt, M, N, K / 256);
+    return us < 3 + 1.4 * (double)(K / 256) ? us : std::min(us, qgemm_kquant_us(M, N, K));
 }
 
 template <int DT, int TILES, int WAVES, int DEPTH, int ROUNDS, bool ROPE>

@@ -649,6 +649,32 @@ def test_a_prompt_by_k_quants_takes_matrices_of_one_x_together(linear_dt, batch,
         assert err.max() <= 0.05 and np.median(err) <= 0.01, err
 
 
+@pytest.mark.parametrize("linear_dt,batch,tokens", [(O.Q4_K, 11, 3), (O.Q6_K, 9, 5), (O.Q4_K, 2, 33), (O.Q6_K, 1, 77)])
+def test_k_quant_products_of_some_rows_in_a_decoder(linear_dt, batch, tokens):
+    """Prompts and steps whose products take W once for up to 64 rows, x left in the order of their lanes by the norms, SwiGLU and the conversion, the
+    residual added as they store: the same integers and the same sums in the same order, so the same bits as by the other kernels."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F32)
+    c.context = 100
+    m = Llama(c)
+    _upload_synthetic(m, OL.synthetic(_oracle_config(c), seed=4, linear_dt=linear_dt, output_dt=linear_dt))
+    m.finalize(tokens)
+    prompts = np.random.default_rng(tokens).integers(0, c.vocab, (batch, tokens))
+    runs = []
+    try:
+        for mode in (1, 2, 0):
+            gpu.say(f"k-quant rows in a decoder, dtype {linear_dt} {batch} x {tokens}, mode {mode}")
+            capi.check(lib.mi355x_tune(b"kquant.shared", mode))
+            m.reset()
+            logits = m.logits(prompts, all=True)
+            m.reset()
+            runs.append((logits, m.generate(prompts, 6)[0]))
+    finally:
+        capi.check(lib.mi355x_tune(b"kquant.shared", 0))
+    for logits, chosen in runs[1:]:
+        assert np.array_equal(logits.view(np.uint32), runs[0][0].view(np.uint32)) and np.array_equal(chosen, runs[0][1])
+
+
 @pytest.mark.parametrize("linear_dt", [O.Q4_K, O.Q6_K, O.Q8_0, O.Q4_0])
 def test_a_prompt_whose_products_round_to_int8_keeps_the_order_of_attentions_sums(linear_dt):
     """Rounding to int8 makes a step of a difference in the last place: a decoder of such products takes attention of a prompt over a binary16 cache on float32

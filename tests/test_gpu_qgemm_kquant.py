@@ -173,3 +173,38 @@ def tiles_run():
     cut = re.fullmatch(r"qgemm_kquant_kernel: (\d+) x (\d+) tiles of 256 x 64, (\d+) x (\d+) of 128 x 64", buf.value.decode())
     rows, cols, low_rows, low_cols = map(int, cut.groups())
     return rows * cols, low_rows * low_cols
+
+
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 256), (9, 17, 256 * 8), (16, 33, 256 * 9), (17, 130, 256 * 7), (32, 15, 512), (33, 128, 768), (48, 129, 256 * 17),
+                                   (49, 64, 256), (64, 200, 256 * 16), (65, 16, 256 * 3), (97, 70, 1280), (200, 48, 2304), (512, 40, 512)])
+def test_strips_of_sixteen_rows_of_w_by_some_rows_of_x(dt, m, n, k):
+    """The kernel between those for a few rows and the tall tiles: one to four tiles of rows, full and not, in one group or several, strips past the last row of W, super-blocks
+    in whole rounds of eight and not, blocks of Q6_K from either of the starts that two-byte alignment leaves, a row of zeros, NaN and infinity, bfloat16 in and out."""
+    import torch
+    l = gpu.lib()
+    rng = np.random.default_rng(m + n + k + dt)
+    raw = random_blocks(rng, dt, n * k)
+    xb = O.f32_to_bf16(rng.normal(size=(m, k)).astype(np.float32))
+    x = O.bf16_to_f32(xb)
+    x[m // 2, 256 * (k // 512):256 * (k // 512) + 256] = 0
+    if m > 40:
+        x[3, k // 2], x[40, 1] = np.nan, np.inf
+    want = O.qmatmul(dt, raw, x, n, k)
+    try:
+        capi.check(l.mi355x_tune(b"kquant.shared", 2))
+        for offset in (0, 2, 14) if dt == O.Q6_K else (0, 16):
+            gpu.say(f"kquant strips dt={dt} M={m} N={n} K={k} offset {offset}")
+            got = product(dt, raw, x, n, k, offset=offset)
+            assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(got).any() == (m > 40)
+            ok = ~np.isnan(want)
+            assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32))
+        xd = torch.from_numpy(O.f32_to_bf16(O.bf16_to_f32(xb)).view(np.int16)).to("cuda:0")
+        y = torch.zeros((m, n), dtype=torch.int16, device="cuda:0")
+        wbuf, wp = gpu.dev_bytes_at(raw, 0)
+        gpu.say(f"kquant strips of bfloat16 dt={dt} M={m} N={n} K={k}")
+        capi.check(l.mi355x_qgemm_bf16(dt, wp, xd.data_ptr(), y.data_ptr(), m, n, k, k, capi.BF16, gpu.stream()))
+        gpu.sync()
+        assert np.array_equal(y.cpu().numpy().view(np.uint16), O.f32_to_bf16(O.qmatmul(dt, raw, O.bf16_to_f32(xb), n, k)))
+    finally:
+        capi.check(l.mi355x_tune(b"kquant.shared", 0))

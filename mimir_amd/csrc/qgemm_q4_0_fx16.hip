@@ -5,7 +5,7 @@
 //
 // What bounds it: four MFMAs of 32 cycles and sixteen FMAs of 4 per 32 x 32 outputs and block of 32, which hardly overlap
 // on a SIMD (128 + 64 cycles; one wide tile alone takes 1.3 us a block, those cycles at the full clock; with every unit at work
-// the clock falls and it is 1.75 us. Counters: 3097 cycles a block, 2048 of MFMA and 1426 of all vector instructions, 1024 of them FMAs). The form with the int8 form's bits (x as two 12-bit integer
+// the clock falls and it was 1.75 us. Counters, with the barrier between blocks: 3097 cycles a block, 2048 of MFMA and 1426 of all vector instructions, 1024 of them FMAs). The form with the int8 form's bits (x as two 12-bit integer
 // digits with a float32 scale a block: two sums, an MFMA for dw dx and two FMAs an output: 128 + 32 + 128 cycles) is taken where mi355x_qgemv_noalloc
 // multiplies in that form. Whole calls, conversion and the pass over W included, fifty of a shape back to back (among other shapes, as bench.py has them, a
 // tenth more: 498 us for the first), digits and halves:
@@ -20,6 +20,9 @@
 // into LDS (global_load_lds_dwordx4). A workgroup of eight wavefronts owns 256 x 256 outputs (a wavefront 64 x 128, three
 // stages of one block) where tiles are many, 128 x 256 (64 x 64, four stages) where they are few: 8 KB of fragments
 // from LDS per 16 MFMAs against 12. One barrier a block; a sub-tile's MFMAs are issued with the FMAs of the sub-tile before.
+// The barrier is in a block's middle and fragments are read up to a block ahead. With it between blocks, both wavefronts of a SIMD waited
+// behind it for all eight's fragments, 96 or 128 KB at 256 bytes a cycle: 512 x 14336 x 4096 159 us a call, now 153; 2048 x 14336 x 4096 458, now 451; 4096 x 14336 x
+// 4096 874, now 843. (FMAs set between the MFMAs one by one, which alone in a loop take a tenth less: 158, 465, 864.)
 // Where even those leave units idle, K is cut into shares whose sums a third launch adds.
 //
 // Several matrices by the same x (q, k and v; gate and up, SwiGLU included) are one product: Parts.
@@ -321,65 +324,105 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
         from[j] += (j < S::kX ? kGranuleX * 2 : kGranuleP * 2) * step;
     };
     if (has_sw) load_to_lds(sw_from, lane16, sw_into);
-    uint32_t fill = 0;  // the stage that is loaded next
-    for (int i = 0; i < S::STAGES - 1; i++) {
-#pragma unroll
-        for (int j = 0; j < S::kLoads; j++) load_stage(j, fill, i + 1 < count ? 1 : 0);
-        fill += S::stage;
-    }
-    if (FORM != kHalves && tid < S::BM) ((float*)(lds + S::sx))[tid] = *xscale;
-    f32x16 c[2];  // kHalves: the sums of a sub-tile, finished with the next one's products
-    c[1] = zero;
-    float dlast = 0.f;
-    uint32_t use = 0;  // the stage that is multiplied
-    // No branches around the loads: past the end the last block is requested again, into a stage that is not read any more.
-    for (int i = 0; i < count; i++) {
-        wait_loads<S::kLoads*(S::STAGES - 2)>();  // this wavefront's part of block i has landed, and W's scales
-        lds_barrier();                             // everyone's has, and everyone has read the block before for the last time
-        const int step = i + S::STAGES < count ? 1 : 0;
-        const char* st = lds + use;
-        if (has_sw && (i & (kGroup - 1)) == 0 && i + kGroup < count) {  // the next group of W's scales, over the one before this
+    auto next_scales = [&](int i) {  // in block i: the next group of W's scales, over the one before this
+        if (has_sw && (i & (kGroup - 1)) == 0 && i + kGroup < count) {
             sw_from += 1024;
             load_to_lds(sw_from, lane16, sw_into + ((i / kGroup + 1) & 1) * S::sw_group);
         }
-        float next_dx = 0.f;
-        if (FORM != kHalves) {
-            xscale += i + 1 < count ? 1 : 0;
-            next_dx = *xscale;
-        }
-        f16x8 a[MT][2][2], b[2][2];  // a[mt][part][half], b[nt % 2][half]
-        auto read_b = [&](int nt) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) b[nt & 1][h] = *(const f16x8*)(st + b_off + nt * 2048 + h * 1024);
-        };
-        read_b(0);
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+    };
+    f32x16 c[2];  // kHalves: the sums of a sub-tile, finished with the next one's products
+    c[1] = zero;
+    float dlast = 0.f;
+    // No branches around the loads: past the end the last block is requested again, into a stage that is not read any more.
+    if constexpr (FORM == kHalves) {
+        // Fragments are in registers before they are wanted, x's a sub-tile row and W's a block ahead, so that no product waits behind the barrier while
+        // every wavefront reads at once. The barrier is in a block's middle: by then its stage has been read, and is filled anew.
+        static_assert(MT == 2, "two rows of sub-tiles a block");
+        f16x8 a[MT][2][2], b[NT][2];  // a[mt][part][half], b[nt][half]
+        auto read_a = [&](int mt, const char* st) {
 #pragma unroll
             for (int p = 0; p < 4; p++) a[mt][p >> 1][p & 1] = *(const f16x8*)(st + mt * 4096 + piece_off[p]);
-        read_b(1);
-        const char* sw = lds + S::sw + (i / kGroup & 1) * S::sw_group + wn * NT * 1024 + (i & (kGroup - 1)) * 128;
-        if (FORM == kHalves) {
-            float dw[NT];
+        };
+        auto read_b = [&](int nt, const char* st) {
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++) dw[nt] = *(const float*)(sw + nt * 1024 + r32 * 4);
-            // A sub-tile's products are issued with the FMAs of the one before it, so that the vector unit works while the
-            // matrix cores do. What h0 leaves first: the smaller terms.
+            for (int h = 0; h < 2; h++) b[nt][h] = *(const f16x8*)(st + b_off + nt * 2048 + h * 1024);
+        };
+        for (int i = 0; i < S::STAGES; i++)
 #pragma unroll
-            for (int sub = 0; sub < MT * NT; sub++) {
-                const int nt = sub / MT, mt = sub % MT, was = (sub + MT * NT - 1) % (MT * NT);
-                if (mt == 0 && nt > 0 && nt + 1 < NT) read_b(nt + 1);
-                if (sub < S::kLoads) load_stage(sub, fill, step);
+            for (int j = 0; j < S::kLoads; j++) load_stage(j, i * S::stage, i + 1 < count ? 1 : 0);
+        wait_loads<S::kLoads*(S::STAGES - 1)>();
+        lds_barrier();
+        read_a(0, lds);
 #pragma unroll
-                for (int p = 0; p < 4; p++)
-                    c[sub & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1 - (p >> 1)][p & 1], b[nt & 1][p & 1], p == 0 ? zero : c[sub & 1], 0, 0, 0);
-                const float d = sub == 0 ? dlast : dw[was / MT];
+        for (int nt = 0; nt < NT; nt++) read_b(nt, lds);
+        float dw[NT];
+        // A sub-tile's products are issued with the FMAs of the one before it, so that the vector unit works while the
+        // matrix cores do. What h0 leaves first: the smaller terms.
+        auto sub_tile = [&](int sub) {
+            const int mt = sub / NT, nt = sub % NT, was = (sub + MT * NT - 1) % (MT * NT);
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[was % MT][was / MT][e] = fmaf(d, c[(sub + 1) & 1][e], acc[was % MT][was / MT][e]);
+            for (int p = 0; p < 4; p++)
+                c[sub & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt][1 - (p >> 1)][p & 1], b[nt][p & 1], p == 0 ? zero : c[sub & 1], 0, 0, 0);
+            const float d = sub == 0 ? dlast : dw[was % NT];
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[was / NT][was % NT][e] = fmaf(d, c[(sub + 1) & 1][e], acc[was / NT][was % NT][e]);
+        };
+        uint32_t use = 0;  // the stage that is multiplied
+        for (int i = 0; i < count; i++) {
+            const uint32_t next = use + S::stage == S::sw ? 0 : use + S::stage;
+            const int step = i + S::STAGES + 1 < count ? 1 : 0;
+            next_scales(i);
+            read_a(1, lds + use);
+            const char* sw = lds + S::sw + (i / kGroup & 1) * S::sw_group + wn * NT * 1024 + (i & (kGroup - 1)) * 128;
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                sub_tile(nt);
+                if (nt == 0)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) dw[t] = *(const float*)(sw + t * 1024 + r32 * 4);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            wait_loads<S::kLoads*(S::STAGES - 2)>();  // this wavefront's part of block i + 1 has landed, and W's scales
+            lds_barrier();                             // everyone's has, and everyone has read block i for the last time
+            read_a(0, lds + next);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+#pragma unroll
+                for (int j = nt * S::kLoads / NT; j < (nt + 1) * S::kLoads / NT; j++) load_stage(j, use, step);
+                sub_tile(NT + nt);
+                read_b(nt, lds + next);
                 __builtin_amdgcn_sched_barrier(0);
             }
             dlast = dw[NT - 1];
-        } else {
+            use = next;
+        }
+    } else {
+        uint32_t fill = 0;  // the stage that is loaded next
+        for (int i = 0; i < S::STAGES - 1; i++) {
+#pragma unroll
+            for (int j = 0; j < S::kLoads; j++) load_stage(j, fill, i + 1 < count ? 1 : 0);
+            fill += S::stage;
+        }
+        if (tid < S::BM) ((float*)(lds + S::sx))[tid] = *xscale;
+        uint32_t use = 0;  // the stage that is multiplied
+        for (int i = 0; i < count; i++) {
+            wait_loads<S::kLoads*(S::STAGES - 2)>();  // this wavefront's part of block i has landed, and W's scales
+            lds_barrier();                             // everyone's has, and everyone has read the block before for the last time
+            const int step = i + S::STAGES < count ? 1 : 0;
+            const char* st = lds + use;
+            next_scales(i);
+            xscale += i + 1 < count ? 1 : 0;
+            const float next_dx = *xscale;
+            f16x8 a[MT][2][2], b[2][2];  // a[mt][part][half], b[nt][half]
+#pragma unroll
+            for (int nt = 0; nt < 2; nt++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) b[nt][h] = *(const f16x8*)(st + b_off + nt * 2048 + h * 1024);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int p = 0; p < 4; p++) a[mt][p >> 1][p & 1] = *(const f16x8*)(st + mt * 4096 + piece_off[p]);
+            const char* sw = lds + S::sw + (i / kGroup & 1) * S::sw_group + wn * NT * 1024 + (i & (kGroup - 1)) * 128;
 #pragma unroll
             for (int j = 0; j < S::kLoads; j++) load_stage(j, fill, step);
             // The products of the two scales, dw dx, are an outer product: v_mfma_f32_32x32x1_2b_f32 makes two (one exact product
@@ -418,9 +461,9 @@ __device__ __forceinline__ void tile_body(const Operands& o, int m0, int n0, int
             // the next block's scales, at the end: by now their loads have landed with everything requested before them
             __builtin_amdgcn_sched_barrier(0);
             if (tid < S::BM) ((float*)(lds + S::sx))[((i + 1) & 1) * S::BM + tid] = next_dx;
+            use = use + S::stage == S::sw ? 0 : use + S::stage;
+            fill = fill + S::stage == S::sw ? 0 : fill + S::stage;
         }
-        use = use + S::stage == S::sw ? 0 : use + S::stage;
-        fill = fill + S::stage == S::sw ? 0 : fill + S::stage;
     }
     if (FORM == kHalves) {
 #pragma unroll

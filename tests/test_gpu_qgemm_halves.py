@@ -87,6 +87,12 @@ def test_pairs_of_halves(m, n, k, kernel, rows):
     assert ((got - want).abs() <= bound)[good].all()
 
 
+@pytest.mark.parametrize("k", [384, 640])
+def test_tiles_of_256_by_256_over_groups_of_scales(k):
+    """Twelve and twenty blocks: a stage's refill from the fourth on, the scales' second and third group of eight, fragments read past the last block's stage."""
+    test_pairs_of_halves(1000, 16500, k, PANEL + "4 x 64 tiles of 256 x 256, 8 x 1 tiles of 128 x 256", "even")
+
+
 @pytest.mark.parametrize("m,kernel", [(20, DIRECT + "<1>"), (64, PARTS + "<4>"), (77, PARTS + "<5>"), (128, PARTS + "<4>"), (200, DIRECT + "<4>")])
 def test_rows_held_by_block_among_others(m, kernel):
     """One row with a block 2^17 above its others, which is held with an exponent a block, beside ordinary rows, a row of zeros and one with

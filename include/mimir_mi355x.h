@@ -504,6 +504,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * workgroup where it has a form of that many (0: by shape). "kquant.shared" = 1
  * keeps products of up to 512 rows of x off the kernel that reads sixteen rows of
  * W once for up to 64 of x, 2 sends them all there (0: by shape).
+ * "kquant.stream" = 1 keeps products of one row of x off the kernel with a
+ * workgroup per compute unit, 4 to 16 sends all it takes there, with that many
+ * wavefronts a workgroup (0: by shape).
  * "qgemm.path" = 1 makes mi355x_qgemm_bf16 take its general route for every shape.
  * "qgemm.f16" = 1 makes mi355x_qgemm_bf16's Q4_0 matrix-core kernel round every
  * weight once to binary16 instead of multiplying it exactly (each weight within

@@ -382,9 +382,10 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
     }
     case MI355X_Q4_K:
     case MI355X_Q6_K: {
-        // One row against a small matrix: one launch, every workgroup rounding x itself (a.act stays null). Measured at
-        // K = 4096: 4.7 against 6.5 us at N = 1024, level at N = 4096, 2 us behind at N = 14336.
-        if (M == 1 && N * K <= (8ll << 20) && ((uintptr_t)x & 15) == 0 && mimir::qgemv_kquant_rope_ok(dtype, a)) {
+        // One row: one launch, every workgroup rounding x itself (a.act stays null); by the kernels of short workgroups
+        // against a small matrix alone (at K = 2048 3.4 us for N = 1024 where the rounding's launch and the product took 5).
+        if (M == 1 && (mimir::qgemv_kquant_stream_pays(dtype, a, mimir::KqStream{}) ||
+                       (N * K <= (8ll << 20) && ((uintptr_t)x & 15) == 0 && mimir::qgemv_kquant_rope_ok(dtype, a)))) {
             HIP_TRY(mimir::qgemv_kquant_act(dtype, a, (hipStream_t)stream), "launch qgemv_kquant");
             return MI355X_OK;
         }
@@ -700,6 +701,10 @@ mi355x_status mi355x_tune(const char* key, int value) {
         }
     if (key && (strcmp(key, "kquant.rows") == 0 || strcmp(key, "kquant.path") == 0)) {
         mimir::set_kquant_tune(key[7] == 'p', value);
+        return MI355X_OK;
+    }
+    if (key && strcmp(key, "kquant.stream") == 0) {
+        mimir::set_kquant_stream(value);
         return MI355X_OK;
     }
     if (key && strcmp(key, "qgemm.path") == 0) {

@@ -151,7 +151,7 @@ hipError_t rmsnorm_kq_act(const float* x, const float* w, void* act, int64_t row
 hipError_t swiglu_kq_act(const float* g, const float* u, void* act, int64_t rows, int64_t n, int64_t stride, hipStream_t st, bool lanes = false);
 // The same from bfloat16 rows (8-byte aligned, a multiple of 4 elements apart).
 hipError_t kq_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st, bool lanes = false);
-// With a.act null and qgemv_kquant_rope_ok(dt, a): one launch from float32 a.x (16-byte aligned rows), rounded by every workgroup.
+// With a.act null and qgemv_kquant_rope_ok(dt, a) or qgemv_kquant_stream_pays: one launch from float32 a.x (16-byte aligned rows), rounded by every workgroup.
 hipError_t qgemv_kquant_act(int dt, const QGemvArgs& a, hipStream_t st);
 // The same products for many rows of x on the matrix cores (qgemm_kquant.hip); qgemv_kquant_act
 // hands over to it where qgemm_kquant_pays says it is the faster of the two.
@@ -165,7 +165,7 @@ hipError_t qgemm_kquant(int dt, const QGemvArgs& a, hipStream_t st, bool out_bf1
 // global memory, 2 = never the matrix-core kernel, 3 = always the matrix-core kernel.
 void set_kquant_tune(int which, int value);
 // Two rows of x or more against Q4_K or Q6_K weights, eight to a pass over W, on the int8 matrix cores with the CPU's bits
-// (qgemv_kquant_rows.hip), and one row where its rows of W are short and many; qgemv_kquant_act hands over where qgemv_kquant_rows_pays says so
+// (qgemv_kquant_rows.hip), and one row of bfloat16 x where its rows of W are short and many; qgemv_kquant_act hands over where qgemv_kquant_rows_pays says so
 // ("kquant.mfma_rows": 1 never, 2 wherever the kernel takes two rows or more).
 bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a);
 bool qgemv_kquant_rows_pays(int dt, const QGemvArgs& a);
@@ -183,6 +183,20 @@ bool qgemm_kquant_shared_ok(int dt, const void* W, int64_t M, int64_t N, int64_t
 bool qgemm_kquant_shared_pays(int dt, const void* W, int64_t M, int64_t N, int64_t K);
 hipError_t qgemm_kquant_shared(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);
 void set_kquant_shared(int v);
+// One row of x with a workgroup per compute unit (qgemv_kquant_stream.hip), the CPU's bits too. a.act: a converted row; null: float32 a.x (16-byte aligned), which every
+// workgroup rounds for itself, and with norm_w normalizes before (rows of at most 4096). Its tails beside a.resid: the rotation with the cache writes (as
+// qgemv_kquant_act_rope, from a converted row or with the norm), or y[N] = SiLU(W . x)[0, N) times (W . x)[N, 2 N) of a W of 2 N rows (the same).
+// qgemv_kquant_act hands over where qgemv_kquant_stream_pays says so ("kquant.stream": 1 never, 4 to 16 wherever it takes the product, with that many wavefronts).
+struct KqStream {
+    const float* norm_w = nullptr;
+    double eps = 0;
+    const Q4RopeTail* rope = nullptr;
+    bool swiglu = false;
+};
+bool qgemv_kquant_stream_ok(int dt, const QGemvArgs& a, const KqStream& s);
+bool qgemv_kquant_stream_pays(int dt, const QGemvArgs& a, const KqStream& s);
+hipError_t qgemv_kquant_stream(int dt, const QGemvArgs& a, const KqStream& s, hipStream_t st);
+void set_kquant_stream(int v);
 void set_kquant_rows_waves(int v);
 
 // y = x . W^T for a float32, binary16 or bfloat16 W [N, K].

@@ -509,25 +509,35 @@ static mi355x_status step_any(Model& m) {
     for (int i = 0; i < c.layers; i++) {
         Block& b = m.blocks[i];
         const bool qkv_kq = is_kquant(b.qkv);  // x by rows: the rotation and the cache writes ride on that product
-        if (qkv_kq) {  // norm and conversion in one launch
+        const bool pairs = c.interleaved && c.head_dim % 2 == 0 && c.rope_dim % 2 == 0;
+        KqStream lone;  // of one sequence the norm rides on it as well
+        Q4RopeTail tail;
+        tail.cosv = m.cos_t.as<float>(); tail.sinv = m.sin_t.as<float>(); tail.pos = pos;
+        tail.kcache = m.keys[i].p; tail.vcache = m.values[i].p;
+        tail.cache_dt = c.cache_dtype; tail.H = c.heads; tail.HK = c.kv_heads; tail.dim = c.head_dim; tail.rope_dim = c.rope_dim;
+        tail.cap = c.context;
+        lone.norm_w = b.attn_norm.buf.as<float>();
+        lone.eps = c.eps;
+        lone.rope = &tail;
+        const QGemvArgs normed{b.qkv.buf.p, x, nullptr, qkv, B, b.qkv.n, b.qkv.k, b.qkv.k, 0};
+        const bool norm_qkv = B == 1 && qkv_kq && pairs && !b.biased() && qgemv_kquant_stream_pays(b.qkv.dtype, normed, lone);
+        if (norm_qkv) {
+            LLM_HIP(qgemv_kquant_stream(b.qkv.dtype, normed, lone, m.stream), "norm, q|k|v, rope and cache");
+        } else if (qkv_kq) {  // norm and conversion in one launch
             LLM_HIP(rmsnorm_kq_act(x, b.attn_norm.buf.as<float>(), m.act[kActKQ].p, B, c.embed, c.eps, m.stream), "attn_norm");
         } else {
             LLM_HIP(rmsnorm(x, b.attn_norm.buf.as<float>(), h, B, c.embed, c.eps, m.stream), "attn_norm");
             if (b.qkv.set())
                 if (mi355x_status st = convert_for(m, h, B, c.embed, {&b.qkv}, done)) return st;
         }
-        if (b.qkv.set()) {  // one product into [B, q | k | v]
+        if (norm_qkv) {
+            at.q = qkv; at.q_strides[0] = qd + 2 * kvd;
+        } else if (b.qkv.set()) {  // one product into [B, q | k | v]
             QGemvArgs qa{b.qkv.buf.p, nullptr, m.act[kActKQ].p, qkv, B, b.qkv.n, b.qkv.k, b.qkv.k, 0};
             // From three sequences on, where W can be read once for eight of them, that beats the tail that saves a launch.
             const bool read_once = B >= 3 && qkv_kq && qgemv_kquant_rows_pays(b.qkv.dtype, qa);
-            const bool pairs = c.interleaved && c.head_dim % 2 == 0 && c.rope_dim % 2 == 0;
             const bool once_rope = read_once && pairs && qgemv_kquant_rows_rope_ok(b.qkv.dtype, qa);
             if (!b.biased() && (once_rope || (qkv_kq && !read_once && pairs && qgemv_kquant_rope_ok(b.qkv.dtype, qa)))) {
-                Q4RopeTail tail;  // the rotation and the cache writes ride on the product
-                tail.cosv = m.cos_t.as<float>(); tail.sinv = m.sin_t.as<float>(); tail.pos = pos;
-                tail.kcache = m.keys[i].p; tail.vcache = m.values[i].p;
-                tail.cache_dt = c.cache_dtype; tail.H = c.heads; tail.HK = c.kv_heads; tail.dim = c.head_dim; tail.rope_dim = c.rope_dim;
-                tail.cap = c.context;
                 if (once_rope) LLM_HIP(qgemv_kquant_rows_rope(b.qkv.dtype, qa, tail, m.stream), "q|k|v, rope and cache");
                 else LLM_HIP(qgemv_kquant_act_rope(b.qkv.dtype, qa, tail, m.stream), "q|k|v, rope and cache");
             } else {
@@ -551,16 +561,23 @@ static mi355x_status step_any(Model& m) {
         }
         at.k = m.keys[i].p; at.v = m.values[i].p;
         // K-quant output projection: attention leaves its result as the int8 super-blocks that product reads
-        const bool a_kq = one_launch && is_kquant(b.o) && attention_decode_kq_ok(at);
+        // (one sequence's rounds it for itself)
+        QGemvArgs from_a{b.o.buf.p, a, nullptr, x, B, c.embed, qd, qd, 0};
+        from_a.resid = x;
+        const bool round_a = B == 1 && is_kquant(b.o) && qgemv_kquant_stream_pays(b.o.dtype, from_a, KqStream{});
+        const bool a_kq = one_launch && !round_a && is_kquant(b.o) && attention_decode_kq_ok(at);
         if (a_kq) {
             LLM_HIP(attention_decode(at, c.context, m.act[0].p, m.act[kActKQ].p, (int64_t)kq_act_bytes(qd), m.stream, kAttnActKQ, m.attn_flags.p, m.attn_flags.bytes, device_error_word()), "attention");
         } else {
             if (one_launch) LLM_HIP(attention_decode(at, c.context, m.act[0].p, nullptr, 0, m.stream, kAttnActQ4, m.attn_flags.p, m.attn_flags.bytes, device_error_word()), "attention");
             else LLM_HIP(attention(at, (uint8_t*)m.act[0].p + kAttnTicketBytes, m.stream), "attention");
-            if (mi355x_status st = convert_for(m, a, B, qd, {&b.o}, done)) return st;
+            if (!round_a)
+                if (mi355x_status st = convert_for(m, a, B, qd, {&b.o}, done)) return st;
         }
         const int o_cls = a_kq ? (int)kActKQ : act_class(b.o, B, m.fx_panel.bytes);
-        if (o_cls != kActNone) {  // the residual rides on the product
+        if (round_a) {
+            LLM_HIP(qgemv_kquant_stream(b.o.dtype, from_a, KqStream{}, m.stream), "attn_output");
+        } else if (o_cls != kActNone) {  // the residual rides on the product
             if (mi355x_status st = linear_by(m, o_cls, b.o, a, x, B, x)) return st;
         } else {
             if (mi355x_status st = linear(m, b.o, a, o, B)) return st;
@@ -568,6 +585,20 @@ static mi355x_status step_any(Model& m) {
         }
         const int down = act_class(b.down, B);
         const bool down_kq = down == kActKQ || down == kActKQLanes;  // then SwiGLU leaves its result converted
+        // one sequence: the norm and SwiGLU ride on the first product, the rounding of its results on the second
+        KqStream ffn;
+        ffn.norm_w = b.ffn_norm.buf.as<float>();
+        ffn.eps = c.eps;
+        ffn.swiglu = true;
+        const QGemvArgs gate_up{b.gate_up.buf.p, x, nullptr, sw, B, c.hidden, c.embed, c.embed, 0};
+        QGemvArgs from_sw{b.down.buf.p, sw, nullptr, x, B, c.embed, c.hidden, c.hidden, 0};
+        from_sw.resid = x;
+        if (B == 1 && is_kquant(b.gate_up) && is_kquant(b.down) && qgemv_kquant_stream_pays(b.gate_up.dtype, gate_up, ffn) &&
+            qgemv_kquant_stream_pays(b.down.dtype, from_sw, KqStream{})) {
+            LLM_HIP(qgemv_kquant_stream(b.gate_up.dtype, gate_up, ffn, m.stream), "norm, gate|up and swiglu");
+            LLM_HIP(qgemv_kquant_stream(b.down.dtype, from_sw, KqStream{}, m.stream), "ffn_down");
+            continue;
+        }
         if (is_kquant(b.gate_up)) {
             const int cls = act_class(b.gate_up, B);
             LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[cls].p, B, c.embed, c.eps, m.stream, cls == kActKQLanes), "ffn_norm");

@@ -17,7 +17,8 @@
 // a kernel built from dword loads). The loads of the next pass are requested
 // before the current pass is multiplied. A second pair of kernels, one
 // wavefront per row with x read from global memory, serves rows of x too long
-// for the LDS.
+// for the LDS. One row of x by all but small matrices is
+// qgemv_kquant_stream.hip's.
 #include "device_util.h"
 #include "kernels.h"
 #include "kq_act.h"
@@ -591,11 +592,15 @@ bool qgemv_kquant_rope_ok(int dt, const QGemvArgs& a) {
 // The q|k|v product of a decoding step with the rotation and the cache writes as its tail: y receives
 // the rotated queries only (see Q4RopeTail; interleaved pairs, even widths).
 hipError_t qgemv_kquant_act_rope(int dt, const QGemvArgs& a, const Q4RopeTail& rope, hipStream_t st) {
+    KqStream s;
+    s.rope = &rope;
+    if (qgemv_kquant_stream_pays(dt, a, s)) return qgemv_kquant_stream(dt, a, s, st);
     return launch_kq<2>(dt, a, (int)(a.K / 256), &rope, st);
 }
 
 hipError_t qgemv_kquant_act(int dt, const QGemvArgs& a, hipStream_t st) {
     int nsb = (int)(a.K / 256);
+    if (a.M == 1 && qgemv_kquant_stream_pays(dt, a, KqStream{})) return qgemv_kquant_stream(dt, a, KqStream{}, st);
     // Float32 x in place of converted rows (a.act null): only the kernels that stage the row in LDS round it themselves.
     if (!a.act) {
         if (!qgemv_kquant_rope_ok(dt, a) || ((uintptr_t)a.x & 15) || a.x_row_stride % 4) return hipErrorInvalidValue;

@@ -378,7 +378,7 @@ bool qgemv_kquant_rows_ok(int dt, const QGemvArgs& a) {
            rows_lds(dt, nsb, 1, 4) <= 160 * 1024;
 }
 
-// One converted row: the kernels that give a row of W to a wavefront (qgemv_kquant.hip) have little to read a wavefront where rows are short and many. us, there | here,
+// One converted row of bfloat16 x (of float32 x they are qgemv_kquant_stream.hip's): the kernels that give a row of W to a wavefront (qgemv_kquant.hip) have little to read a wavefront where rows are short and many. us, there | here,
 // Q4_K: 8192 x 256 5.5 | 4.2, 8192 x 2048 6.2 | 5.5, 12288 x 2048 8.0 | 6.8, 32768 x 2048 17.3 | 13.0, 128256 x 2048 56 | 36; Q6_K: 8192 x 2048 6.0 | 5.9, 12288 x 2048 9.3 | 8.7,
 // 32768 x 2048 20.4 | 18.0; but Q6_K 9216 x 2048 7.2 | 7.6, 10240 x 1536 6.8 | 7.0, and of longer rows Q4_K 16384 x 3072 11.2 | 11.9, 4096 x 14336 11.5 | 11.7,
 // 4096 x 20480 14.2 | 16.6; Q6_K 4096 x 14336 15.8 | 17.1.

@@ -760,6 +760,35 @@ def test_kquant_gemv_single_row_rounds_x_in_the_product(dt):
             assert bits_equal(one, want) and bits_equal(two, want)
 
 
+@pytest.mark.parametrize("waves", [4, 8, 12, 16])
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+def test_kquant_one_row_by_a_workgroup_a_compute_unit(dt, waves):
+    """Several rows of W a load (K up to 8 or 16 super-blocks), rows cut over wavefronts evenly and not (9, 17, 56), counts of rows that no workgroup
+    shares evenly (odd, fewer than workgroups, more than 256 times the least); x with a super-block of zeros, ties, values so small that 127 / amax overflows,
+    an infinity and a NaN: the CPU's bits from float32 and from converted x, and those of the kernels of short workgroups."""
+    l = gpu.lib()
+    rng = np.random.default_rng(31 * dt + waves)
+    for n, k in ((1, 256), (515, 256), (2051, 256 * 3), (700, 256 * 5), (259, 256 * 8), (4097, 256 * 9), (1031, 256 * 16), (130, 256 * 17), (37, 256 * 56)):
+        raw = random_blocks(rng, dt, n * k)
+        x = rng.normal(size=k).astype(np.float32)
+        x[k - 256:] = (rng.integers(0, 254, 256) - 127) / 2; x[k - 1] = 127
+        if k >= 1280: x[256:512] = 0; x[512:768] *= np.float32(1e-38)
+        buf, ptr = gpu.dev_bytes_at(raw, 2 if dt == O.Q6_K else 0)  # Q6_K: W on any even address
+        for poison in (None, np.inf, np.nan):
+            if poison is not None: x[k // 2] = poison
+            want = O.qmatmul(dt, raw, x, n, k)
+            try:
+                capi.check(l.mi355x_tune(b"kquant.stream", waves))
+                gpu.say(f"kquant one row dt={dt} N={n} K={k} waves={waves} x={poison}")
+                got = gpu.qgemv(dt, ptr, gpu.dev(x), n, k)
+                got_act = gpu.qgemv_act(dt, ptr, gpu.dev(x), n, k)
+                capi.check(l.mi355x_tune(b"kquant.stream", 1))
+                other = gpu.qgemv_act(dt, ptr, gpu.dev(x), n, k)
+            finally:
+                capi.check(l.mi355x_tune(b"kquant.stream", 0))
+            assert bits_equal(got, want) and bits_equal(got_act, want) and bits_equal(other, want)
+
+
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("m,n,k", [(2, 33, 256), (5, 100, 512), (8, 203, 4096), (11, 64, 256 * 9), (20, 31, 256 * 56), (40, 130, 1024),
                                    (3, 40, 256 * 37), (4, 33, 256 * 70), (9, 300, 256 * 33)])

@@ -183,9 +183,9 @@ bool qgemm_kquant_shared_ok(int dt, const void* W, int64_t M, int64_t N, int64_t
 bool qgemm_kquant_shared_pays(int dt, const void* W, int64_t M, int64_t N, int64_t K);
 hipError_t qgemm_kquant_shared(int dt, const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);
 void set_kquant_shared(int v);
-// One row of x with a workgroup per compute unit (qgemv_kquant_stream.hip), the CPU's bits too. a.act: a converted row; null: float32 a.x (16-byte aligned), which every
-// workgroup rounds for itself, and with norm_w normalizes before (rows of at most 4096). Its tails beside a.resid: the rotation with the cache writes (as
-// qgemv_kquant_act_rope, from a converted row or with the norm), or y[N] = SiLU(W . x)[0, N) times (W . x)[N, 2 N) of a W of 2 N rows (the same).
+// One to three rows of x with a workgroup per compute unit (qgemv_kquant_stream.hip), the CPU's bits too. a.act: converted rows; null: float32 a.x (16-byte aligned), one row, which
+// every workgroup rounds for itself, or with norm_w rows that it normalizes before (of at most 4096, with one of the two tails). Its tails beside a.resid: the rotation with the cache writes (as
+// qgemv_kquant_act_rope, from converted rows or with the norm), or y[N] = SiLU(W . x)[0, N) times (W . x)[N, 2 N) of a W of 2 N rows (with the norm).
 // qgemv_kquant_act hands over where qgemv_kquant_stream_pays says so ("kquant.stream": 1 never, 4 to 16 wherever it takes the product, with that many wavefronts).
 struct KqStream {
     const float* norm_w = nullptr;

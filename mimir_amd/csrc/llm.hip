@@ -510,7 +510,7 @@ static mi355x_status step_any(Model& m) {
         Block& b = m.blocks[i];
         const bool qkv_kq = is_kquant(b.qkv);  // x by rows: the rotation and the cache writes ride on that product
         const bool pairs = c.interleaved && c.head_dim % 2 == 0 && c.rope_dim % 2 == 0;
-        KqStream lone;  // of one sequence the norm rides on it as well
+        KqStream lone;  // of few sequences the norm rides on it as well
         Q4RopeTail tail;
         tail.cosv = m.cos_t.as<float>(); tail.sinv = m.sin_t.as<float>(); tail.pos = pos;
         tail.kcache = m.keys[i].p; tail.vcache = m.values[i].p;
@@ -520,7 +520,7 @@ static mi355x_status step_any(Model& m) {
         lone.eps = c.eps;
         lone.rope = &tail;
         const QGemvArgs normed{b.qkv.buf.p, x, nullptr, qkv, B, b.qkv.n, b.qkv.k, b.qkv.k, 0};
-        const bool norm_qkv = B == 1 && qkv_kq && pairs && !b.biased() && qgemv_kquant_stream_pays(b.qkv.dtype, normed, lone);
+        const bool norm_qkv = qkv_kq && pairs && !b.biased() && qgemv_kquant_stream_pays(b.qkv.dtype, normed, lone);
         if (norm_qkv) {
             LLM_HIP(qgemv_kquant_stream(b.qkv.dtype, normed, lone, m.stream), "norm, q|k|v, rope and cache");
         } else if (qkv_kq) {  // norm and conversion in one launch
@@ -585,7 +585,7 @@ static mi355x_status step_any(Model& m) {
         }
         const int down = act_class(b.down, B);
         const bool down_kq = down == kActKQ || down == kActKQLanes;  // then SwiGLU leaves its result converted
-        // one sequence: the norm and SwiGLU ride on the first product, the rounding of its results on the second
+        // few sequences: the norm and SwiGLU ride on the first product, with one the rounding of its results on the second
         KqStream ffn;
         ffn.norm_w = b.ffn_norm.buf.as<float>();
         ffn.eps = c.eps;
@@ -593,13 +593,14 @@ static mi355x_status step_any(Model& m) {
         const QGemvArgs gate_up{b.gate_up.buf.p, x, nullptr, sw, B, c.hidden, c.embed, c.embed, 0};
         QGemvArgs from_sw{b.down.buf.p, sw, nullptr, x, B, c.embed, c.hidden, c.hidden, 0};
         from_sw.resid = x;
-        if (B == 1 && is_kquant(b.gate_up) && is_kquant(b.down) && qgemv_kquant_stream_pays(b.gate_up.dtype, gate_up, ffn) &&
-            qgemv_kquant_stream_pays(b.down.dtype, from_sw, KqStream{})) {
+        const bool ffn_rides = is_kquant(b.gate_up) && qgemv_kquant_stream_pays(b.gate_up.dtype, gate_up, ffn);
+        if (ffn_rides) {
             LLM_HIP(qgemv_kquant_stream(b.gate_up.dtype, gate_up, ffn, m.stream), "norm, gate|up and swiglu");
-            LLM_HIP(qgemv_kquant_stream(b.down.dtype, from_sw, KqStream{}, m.stream), "ffn_down");
-            continue;
-        }
-        if (is_kquant(b.gate_up)) {
+            if (is_kquant(b.down) && qgemv_kquant_stream_pays(b.down.dtype, from_sw, KqStream{})) {
+                LLM_HIP(qgemv_kquant_stream(b.down.dtype, from_sw, KqStream{}, m.stream), "ffn_down");
+                continue;
+            }
+        } else if (is_kquant(b.gate_up)) {
             const int cls = act_class(b.gate_up, B);
             LLM_HIP(rmsnorm_kq_act(x, b.ffn_norm.buf.as<float>(), m.act[cls].p, B, c.embed, c.eps, m.stream, cls == kActKQLanes), "ffn_norm");
             if (mi355x_status st = linear_by(m, cls, b.gate_up, h, gu, B)) return st;
@@ -619,7 +620,7 @@ static mi355x_status step_any(Model& m) {
             if (down_kq) LLM_HIP(swiglu_kq_act(gate, up, m.act[down].p, B, c.hidden, c.hidden, m.stream, down == kActKQLanes), "swiglu");
             else LLM_HIP(swiglu(gate, up, sw, B, c.hidden, c.hidden, m.stream), "swiglu");
         }
-        if (!down_kq)
+        if (ffn_rides || !down_kq)
             if (mi355x_status st = convert_for(m, sw, B, c.hidden, {&b.down}, done)) return st;
         if (act_class(b.down, B) != kActNone) {
             if (mi355x_status st = linear(m, b.down, sw, x, B, x)) return st;

@@ -600,7 +600,7 @@ hipError_t qgemv_kquant_act_rope(int dt, const QGemvArgs& a, const Q4RopeTail& r
 
 hipError_t qgemv_kquant_act(int dt, const QGemvArgs& a, hipStream_t st) {
     int nsb = (int)(a.K / 256);
-    if (a.M == 1 && qgemv_kquant_stream_pays(dt, a, KqStream{})) return qgemv_kquant_stream(dt, a, KqStream{}, st);
+    if (qgemv_kquant_stream_pays(dt, a, KqStream{})) return qgemv_kquant_stream(dt, a, KqStream{}, st);
     // Float32 x in place of converted rows (a.act null): only the kernels that stage the row in LDS round it themselves.
     if (!a.act) {
         if (!qgemv_kquant_rope_ok(dt, a) || ((uintptr_t)a.x & 15) || a.x_row_stride % 4) return hipErrorInvalidValue;

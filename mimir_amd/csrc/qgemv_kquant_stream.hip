@@ -1,4 +1,4 @@
-// One row of x by Q4_K or Q6_K weights with a workgroup per compute unit, for
+// One to three rows of x by Q4_K or Q6_K weights with a workgroup per compute unit, for
 // gfx950: the arithmetic of qgemv_kquant.hip (the CPU's bits: integers exact, a
 // row's super-blocks added in their order; backend/cpu/qmatmul.go:141-254), what
 // differs is the launch. A lane keeps its part of x in registers for all rows of W
@@ -31,7 +31,8 @@ namespace mimir {
 
 namespace {
 
-constexpr int kMostWaves = 16;
+constexpr int kMostWaves = 16, kFewWaves = 8;  // a workgroup, with one row of x and with more
+constexpr int kMostRows = 3;
 constexpr int kStride = 256 + 16;    // a super-block's quants of x in LDS
 constexpr uint32_t kPast = 1u << 31; // an offset past every buffer: the load is not made
 constexpr int kMaxLds = 160 * 1024;
@@ -162,46 +163,61 @@ __device__ __forceinline__ void fetch(Raw<kQ6_K>& f, __amdgpu_buffer_rsrc_t w, u
 }
 
 // qdotQ4KGo's integers (qmatmul.go:148-172). Lane j of a super-block: sub-blocks 2 g, 2 g + 1, 2 g + 4, 2 g + 5, g = j / 2, their chunk h = j % 2.
-__device__ __forceinline__ void dot(const Raw<kQ4_K>& f, const X<kQ4_K>& x, uint32_t, int j, int& sumi, int& summ) {
+template <int ROWS>
+__device__ __forceinline__ void dot(const Raw<kQ4_K>& f, const X<kQ4_K> (&x)[ROWS], uint32_t, int j, int (&sumi)[ROWS], int (&summ)[ROWS]) {
     const int sh = 16 * (j >> 1);
     const uint32_t s0 = f.hdr[1] >> sh, s1 = f.hdr[2] >> sh, s2 = f.hdr[3] >> sh;
     // scale_min_k4 (backend/cpu/quant.go:129-134)
     const int sc_a = s0 & 63, sc_b = (s0 >> 8) & 63, m_a = s1 & 63, m_b = (s1 >> 8) & 63;
     const int sc_c = (s2 & 0xf) | ((s0 >> 2) & 0x30), sc_e = ((s2 >> 8) & 0xf) | ((s0 >> 10) & 0x30);
     const int m_c = ((s2 >> 4) & 0xf) | ((s1 >> 2) & 0x30), m_e = ((s2 >> 12) & 0xf) | ((s1 >> 10) & 0x30);
-    int lo0 = 0, hi0 = 0, lo1 = 0, hi1 = 0;
+    int w[4][4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t w0 = f.q[0][i], w1 = f.q[1][i];
-        lo0 = __builtin_amdgcn_sdot4((int)(w0 & 0x0F0F0F0Fu), (int)x.q[0][i], lo0, false);
-        hi0 = __builtin_amdgcn_sdot4((int)((w0 >> 4) & 0x0F0F0F0Fu), (int)x.q[1][i], hi0, false);
-        lo1 = __builtin_amdgcn_sdot4((int)(w1 & 0x0F0F0F0Fu), (int)x.q[2][i], lo1, false);
-        hi1 = __builtin_amdgcn_sdot4((int)((w1 >> 4) & 0x0F0F0F0Fu), (int)x.q[3][i], hi1, false);
+        w[0][i] = (int)(w0 & 0x0F0F0F0Fu);
+        w[1][i] = (int)((w0 >> 4) & 0x0F0F0F0Fu);
+        w[2][i] = (int)(w1 & 0x0F0F0F0Fu);
+        w[3][i] = (int)((w1 >> 4) & 0x0F0F0F0Fu);
     }
-    // 24-bit multiplies: scales and mins below 64, sums within 16 x 15 x 127
-    sumi = __mul24(sc_a, lo0) + __mul24(sc_b, hi0) + __mul24(sc_c, lo1) + __mul24(sc_e, hi1);
-    summ = __mul24(m_a, x.s[0]) + __mul24(m_b, x.s[1]) + __mul24(m_c, x.s[2]) + __mul24(m_e, x.s[3]);
-    sumi = dpp_i32_quad_sum(sumi);
-    summ = dpp_i32_quad_sum(summ);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        int q[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) q[c] = __builtin_amdgcn_sdot4(w[c][i], (int)x[r].q[c][i], q[c], false);
+        // 24-bit multiplies: scales and mins below 64, sums within 16 x 15 x 127
+        sumi[r] = dpp_i32_quad_sum(__mul24(sc_a, q[0]) + __mul24(sc_b, q[1]) + __mul24(sc_c, q[2]) + __mul24(sc_e, q[3]));
+        summ[r] = dpp_i32_quad_sum(__mul24(m_a, x[r].s[0]) + __mul24(m_b, x[r].s[1]) + __mul24(m_c, x[r].s[2]) + __mul24(m_e, x[r].s[3]));
+    }
 }
 // qdotQ6KGo's (qmatmul.go:180-200). Lane j = 4 n + c: chunks 8 n + c and 8 n + c + 4.
-__device__ __forceinline__ void dot(const Raw<kQ6_K>& f, const X<kQ6_K>& x, uint32_t at, int j, int& sumi, int&) {
+template <int ROWS>
+__device__ __forceinline__ void dot(const Raw<kQ6_K>& f, const X<kQ6_K> (&x)[ROWS], uint32_t at, int j, int (&sumi)[ROWS], int (&)[ROWS]) {
     const uint32_t mis = at & 3;
     const int c = j & 3, shl = c & 2;
-    int dl = 0, dh = 0;
+    int w[2][4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t a = __builtin_amdgcn_alignbyte(i == 3 ? f.ql_top : f.ql[i < 3 ? i + 1 : 3], f.ql[i], mis);
         const uint32_t b = __builtin_amdgcn_alignbyte(i == 3 ? f.qh_top : f.qh[i < 3 ? i + 1 : 3], f.qh[i], mis) >> shl;
-        const uint32_t vl = (a & 0x0F0F0F0Fu) | ((b & 0x03030303u) << 4), vh = ((a >> 4) & 0x0F0F0F0Fu) | (b & 0x30303030u);  // 0..63 a byte
-        dl = __builtin_amdgcn_sdot4((int)vl, (int)x.q[0][i], dl, false);
-        dh = __builtin_amdgcn_sdot4((int)vh, (int)x.q[1][i], dh, false);
+        w[0][i] = (int)((a & 0x0F0F0F0Fu) | ((b & 0x03030303u) << 4));  // 0..63 a byte
+        w[1][i] = (int)(((a >> 4) & 0x0F0F0F0Fu) | (b & 0x30303030u));
     }
     const uint32_t low = __builtin_amdgcn_alignbyte(f.sc[1], f.sc[0], mis), high = __builtin_amdgcn_alignbyte(f.sc[2], f.sc[1], mis);
     const int sc_l = (int)(int8_t)(low >> (8 * c)), sc_h = (int)(int8_t)(high >> (8 * c));
-    sumi = __mul24(sc_l, dl - 32 * x.s[0]) + __mul24(sc_h, dh - 32 * x.s[1]);
-    sumi = dpp_i32_quad_sum(sumi);
-    sumi += __builtin_amdgcn_update_dpp(0, sumi, 0x141, 0xf, 0xf, true);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        int dl = 0, dh = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            dl = __builtin_amdgcn_sdot4(w[0][i], (int)x[r].q[0][i], dl, false);
+            dh = __builtin_amdgcn_sdot4(w[1][i], (int)x[r].q[1][i], dh, false);
+        }
+        const int sum = dpp_i32_quad_sum(__mul24(sc_l, dl - 32 * x[r].s[0]) + __mul24(sc_h, dh - 32 * x[r].s[1]));
+        sumi[r] = sum + __builtin_amdgcn_update_dpp(0, sum, 0x141, 0xf, 0xf, true);
+    }
 }
 
 // The lane's part of x of super-block sb, from LDS.
@@ -245,51 +261,71 @@ __device__ __forceinline__ float add_row(const uint8_t* terms, int nsb) {
     return DT == kQ4_K ? acc - under : acc;
 }
 
-template <int DT, int DEPTH, int HEAD, int TAIL>
-__global__ __launch_bounds__(64 * kMostWaves) void qgemv_kquant_stream_kernel(Job a) {
+constexpr int kDepth = 2;  // rows of W, or packs of them, under way a wavefront
+
+// x's rows converted, end to end in LDS, the terms behind them.
+__host__ __device__ __forceinline__ int x_bytes(int nsb) { return (nsb * (kStride + 36) + 15) / 16 * 16; }
+
+template <int DT, int ROWS, int HEAD, int TAIL>
+__global__ __launch_bounds__(64 * (ROWS > 1 ? kFewWaves : kMostWaves)) void qgemv_kquant_stream_kernel(Job a) {
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int BB = DT == kQ4_K ? 144 : 210, kLanes = DT == kQ4_K ? 4 : 8;  // bytes and lanes of a super-block
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m = blockIdx.y;
-    const int nsb = a.nsb, R = a.rows, first = blockIdx.x * R;
-    const uint8_t* xr = a.x + (int64_t)m * a.x_row;
-    uint8_t *x_sums = smem + nsb * kStride, *x_d = x_sums + nsb * 32;
-    uint8_t* terms = smem + (nsb * (kStride + 36) + 15) / 16 * 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m0 = blockIdx.y;  // several of x only with ROWS 1
+    const int nsb = a.nsb, R = a.rows, first = blockIdx.x * R, threads = 64 * a.waves, xb = x_bytes(nsb);
+    const int live = a.N - first < R ? a.N - first : R;  // results of a row of x
+    const uint8_t* xr = a.x + (int64_t)m0 * a.x_row;
+    uint8_t* terms = smem + ROWS * xb;
     const int stride = term_row<DT>(nsb);
+    const int local = TAIL == kTailSwiglu ? 2 * R : R;  // rows of W
 
     // What does not depend on W is requested first: loads come back in order.
     int pos = 0;
     if (TAIL == kTailRope) pos = *a.rope.pos;
-    float res = 0.f;
-    if (TAIL == kTailPlain && a.resid && tid < R && first + tid < a.N) res = a.resid[(int64_t)m * a.N + first + tid];
+    float res = 0.f;  // of the first result that this thread puts together
+    const int my_row = ROWS > 1 ? tid / R : 0, my_result = tid - my_row * R;
+    if (TAIL == kTailPlain && a.resid && (ROWS > 1 ? my_row < ROWS : tid < R) && my_result < live) res = a.resid[(int64_t)(m0 + my_row) * a.N + first + my_result];
+    // Four super-blocks are a wavefront's task. The norm's sums are a row of x for every 256 threads, its tasks from the last wavefront down.
+    constexpr int kTurns = HEAD == kHeadNorm ? (ROWS + 1) / 2 : 1;
     const int tasks = (nsb + 3) / 4, l16 = lane & 15;
-    const int task0 = HEAD == kHeadNorm ? a.waves - 1 - wave : wave;  // four super-blocks each; the first wavefronts have the norm's sum
-    f32x4 v[4], nw[4];
-    float sq[16];
+    const int squares = a.waves / 4, square0 = wave / 4;
+    const int sides = HEAD == kHeadNorm ? a.waves / tasks : 1;
+    const int task0 = HEAD == kHeadNorm ? (a.waves - 1 - wave) % tasks : wave, side = HEAD == kHeadNorm ? (a.waves - 1 - wave) / tasks : 0;
+    f32x4 v[kTurns][4], nw[4];
+    float sq[kTurns][16];
+    u32x4 xq[ROWS];
+    uint32_t xt[ROWS];
     auto request = [&](int task, f32x4 to[4], const float* from) {
         const int sb = 4 * task + (lane >> 4) < nsb ? 4 * task + (lane >> 4) : nsb - 1;
 #pragma unroll
         for (int i = 0; i < 4; i++) to[i] = *(const f32x4*)(from + 256 * sb + 64 * i + 4 * l16);
     };
-    u32x4 xq;
-    uint32_t xt;
     if constexpr (HEAD == kHeadAct) {
-        if (tid < 16 * nsb) xq = ((const u32x4*)xr)[tid];
-        if (tid < 9 * nsb) xt = ((const uint32_t*)(xr + nsb * 256))[tid];
-    } else {
-        if (HEAD == kHeadNorm && tid < 256) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) sq[i] = ((const float*)xr)[tid + 256 * i < 256 * nsb ? tid + 256 * i : 0];
+        for (int r = 0; r < ROWS; r++) {
+            if (tid < 16 * nsb) xq[r] = ((const u32x4*)(xr + r * a.x_row))[tid];
+            if (tid < 9 * nsb) xt[r] = ((const uint32_t*)(xr + r * a.x_row + nsb * 256))[tid];
         }
-        if (task0 < tasks) {
-            request(task0, v, (const float*)xr);
-            if (HEAD == kHeadNorm) request(task0, nw, a.norm_w);
-        }
+    } else if constexpr (HEAD == kHeadNorm) {
+#pragma unroll
+        for (int u = 0; u < kTurns; u++)
+            if (square0 < squares && square0 + u * squares < ROWS) {
+                const float* row = (const float*)(xr + (square0 + u * squares) * a.x_row);
+                const int t = tid & 255;
+#pragma unroll
+                for (int i = 0; i < 16; i++) sq[u][i] = row[t + 256 * i < 256 * nsb ? t + 256 * i : 0];
+            }
+#pragma unroll
+        for (int u = 0; u < kTurns; u++)
+            if (side + u * sides < ROWS) request(task0, v[u], (const float*)(xr + (side + u * sides) * a.x_row));
+        if (side < ROWS) request(task0, nw, a.norm_w);
+    } else if (task0 < tasks) {
+        request(task0, v[0], (const float*)xr);
     }
 
     // This wavefront's rows of W: packs of `packed` rows, every groups-th; this lane's super-block of them
     const int groups = a.waves / a.cuts, group = wave / a.cuts, cut = wave - group * a.cuts;
     const int j = lane & (kLanes - 1), unit = lane / kLanes, in_pack = unit / a.each, sb = cut * a.each + unit - in_pack * a.each;
-    const int local = TAIL == kTailSwiglu ? 2 * R : R, packs = (local + a.packed - 1) / a.packed;
+    const int packs = (local + a.packed - 1) / a.packed;
     const int turns = group < groups ? (packs - group + groups - 1) / groups : 0;
     const bool mine = in_pack < a.packed && sb < nsb;
     const int sbx = sb < nsb ? sb : nsb - 1;
@@ -302,115 +338,140 @@ __global__ __launch_bounds__(64 * kMostWaves) void qgemv_kquant_stream_kernel(Jo
         row = (group + turn * groups) * a.packed + in_pack;
         const bool upper = TAIL == kTailSwiglu && row >= R;
         const int result = upper ? row - R : row;
-        const bool there = mine && turn < turns && row < local && first + result < a.N;
+        const bool there = mine && turn < turns && row < local && result < live;
         const uint32_t at = lead + __umul24((uint32_t)(upper ? a.N + result : result), row_bytes) + (uint32_t)(sb * BB);
         return there ? at : kPast;
     };
-    X<DT> x;
-    Raw<DT> slot[DEPTH];
+    Raw<DT> slot[kDepth];
     int row;
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) fetch(slot[d], w, place(d, row), j);
+    for (int d = 0; d < kDepth; d++) fetch(slot[d], w, place(d, row), j);
     __builtin_amdgcn_sched_barrier(0);
 
     if constexpr (HEAD == kHeadAct) {
-        const int threads = 64 * a.waves;
-        for (int c = tid; c < 16 * nsb; c += threads) *(u32x4*)(smem + (c >> 4) * kStride + (c & 15) * 16) = c == tid ? xq : ((const u32x4*)xr)[c];
-        for (int c = tid; c < 9 * nsb; c += threads) ((uint32_t*)x_sums)[c] = c == tid ? xt : ((const uint32_t*)(xr + nsb * 256))[c];
-    } else {
-        float scale = 1.f;
-        if constexpr (HEAD == kHeadNorm) {  // rmsnorm_kernel's arithmetic (nn/transformer.go:50-61)
-            float* part = (float*)terms;
-            if (tid < 256) {
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const uint8_t* from = xr + r * a.x_row;
+            uint8_t* to = smem + r * xb;
+            for (int c = tid; c < 16 * nsb; c += threads) *(u32x4*)(to + (c >> 4) * kStride + (c & 15) * 16) = c == tid ? xq[r] : ((const u32x4*)from)[c];
+            for (int c = tid; c < 9 * nsb; c += threads) ((uint32_t*)(to + nsb * kStride))[c] = c == tid ? xt[r] : ((const uint32_t*)(from + nsb * 256))[c];
+        }
+    } else if constexpr (HEAD == kHeadNorm) {  // rmsnorm_kernel's arithmetic (nn/transformer.go:50-61)
+        float* part = (float*)terms;
+#pragma unroll
+        for (int u = 0; u < kTurns; u++)
+            if (square0 < squares && square0 + u * squares < ROWS) {
                 float ss = 0.f;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const float s = sq[i] * sq[i];
-                    ss = ss + (tid + 256 * i < 256 * nsb ? s : 0.f);
+                    const float s = sq[u][i] * sq[u][i];
+                    ss = ss + ((tid & 255) + 256 * i < 256 * nsb ? s : 0.f);
                 }
                 ss = wave_sum(ss);
-                if (lane == 0) part[wave] = ss;
+                if (lane == 0) part[4 * (square0 + u * squares) + (wave & 3)] = ss;
             }
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            const float total = (part[0] + part[1]) + (part[2] + part[3]);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int to = 4 * task0 + (lane >> 4);
+#pragma unroll
+        for (int u = 0; u < kTurns; u++) {
+            const int r = side + u * sides;
+            if (r >= ROWS) break;
+            const float total = (part[4 * r] + part[4 * r + 1]) + (part[4 * r + 2] + part[4 * r + 3]);
             const float ms = total * a.inv_d;
-            scale = 1.0f / __builtin_sqrtf(ms + a.eps);
+            const float scale = 1.0f / __builtin_sqrtf(ms + a.eps);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float t = v[u][i][k] * scale;
+                    v[u][i][k] = t * nw[i][k];
+                }
+            uint8_t* x = smem + r * xb;
+            if (to < nsb) round_by_sixteen(v[u], l16, x + to * kStride, (uint16_t*)(x + nsb * kStride) + 16 * to, (float*)(x + nsb * (kStride + 32)) + to);
         }
+    } else {
         for (int task = task0; task < tasks; task += a.waves) {
-            if (task != task0) request(task, v, (const float*)xr);
-            if constexpr (HEAD == kHeadNorm) {
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const float t = v[i][k] * scale;
-                        v[i][k] = t * nw[i][k];
-                    }
-            }
+            if (task != task0) request(task, v[0], (const float*)xr);
             const int to = 4 * task + (lane >> 4);
-            if (to < nsb) round_by_sixteen(v, l16, smem + to * kStride, (uint16_t*)x_sums + 16 * to, (float*)x_d + to);
+            if (to < nsb) round_by_sixteen(v[0], l16, smem + to * kStride, (uint16_t*)(smem + nsb * kStride) + 16 * to, (float*)(smem + nsb * (kStride + 32)) + to);
         }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    read_x<DT>(x, smem, x_sums, x_d, sbx, j);
+    X<DT> x[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) read_x<DT>(x[r], smem + r * xb, smem + r * xb + nsb * kStride, smem + r * xb + nsb * (kStride + 32), sbx, j);
+    const int pairs = R >> 1;
     float cosine = 1.f, sine = 0.f;
     bool rotates = false;
-    if (TAIL == kTailRope && 2 * tid < R && first + 2 * tid < a.N) rotates = q4_rope_coeffs(a.rope, pos, first + 2 * tid, &cosine, &sine);
+    const int my_pair = TAIL == kTailRope ? tid % pairs : 0;
+    if (TAIL == kTailRope && tid < ROWS * pairs && 2 * my_pair < live) rotates = q4_rope_coeffs(a.rope, pos, first + 2 * my_pair, &cosine, &sine);
 
     auto multiply = [&](const Raw<DT>& f, int turn) {
         const uint32_t at = place(turn, row);
-        int sumi, summ = 0;
-        dot(f, x, at, j, sumi, summ);
+        int sumi[ROWS], summ[ROWS];
+        dot<ROWS>(f, x, at, j, sumi, summ);
         uint32_t dw;
         if constexpr (DT == kQ4_K) dw = f.hdr[0];
         else dw = f.d >> (8 * (at & 3));
         if (j == 0 && at != kPast) {
-            const float dd = f16_bits_to_f32((uint16_t)dw) * x.d;
             uint8_t* to = terms + row * stride + sb * (DT == kQ4_K ? 8 : 4);
-            *(float*)to = dd * (float)sumi;
-            if (DT == kQ4_K) {
-                const float dm = f16_bits_to_f32((uint16_t)(dw >> 16)) * x.d;
-                *(float*)(to + 4) = dm * (float)summ;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++, to += local * stride) {
+                const float dd = f16_bits_to_f32((uint16_t)dw) * x[r].d;
+                *(float*)to = dd * (float)sumi[r];
+                if (DT == kQ4_K) {
+                    const float dm = f16_bits_to_f32((uint16_t)(dw >> 16)) * x[r].d;
+                    *(float*)(to + 4) = dm * (float)summ[r];
+                }
             }
         }
     };
     // Whole rounds without a branch, so that each wait counts the loads that may still be out; the rest asks for nothing more.
     int t0 = 0;
-    for (; t0 + DEPTH <= turns; t0 += DEPTH) {
+    for (; t0 + kDepth <= turns; t0 += kDepth) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
+        for (int d = 0; d < kDepth; d++) {
             multiply(slot[d], t0 + d);
             int ahead;
-            fetch(slot[d], w, place(t0 + d + DEPTH, ahead), j);
+            fetch(slot[d], w, place(t0 + d + kDepth, ahead), j);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; d++) {
+    for (int d = 0; d < kDepth - 1; d++) {
         if (t0 + d >= turns) break;
         multiply(slot[d], t0 + d);
         __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (TAIL == kTailRope) {  // pairs of rows
-        if (2 * tid < R && first + 2 * tid < a.N) {
-            const float p = add_row<DT>(terms + 2 * tid * stride, nsb), q = add_row<DT>(terms + (2 * tid + 1) * stride, nsb);
-            q4_rope_store_with(a.rope, pos, m, first + 2 * tid, p, q, rotates, cosine, sine, a.y + (int64_t)m * a.N);
+    if constexpr (TAIL == kTailRope) {  // pairs of rows
+        for (int t = tid; t < ROWS * pairs; t += threads) {
+            const int r = t / pairs, pair = t - r * pairs;
+            if (2 * pair >= live) continue;
+            if (t != tid) rotates = q4_rope_coeffs(a.rope, pos, first + 2 * pair, &cosine, &sine);
+            const uint8_t* from = terms + (r * local + 2 * pair) * stride;
+            const float p = add_row<DT>(from, nsb), q = add_row<DT>(from + stride, nsb);
+            q4_rope_store_with(a.rope, pos, m0 + r, first + 2 * pair, p, q, rotates, cosine, sine, a.y + (int64_t)(m0 + r) * a.N);
         }
         return;
     }
-    if (tid >= R || first + tid >= a.N) return;
-    float out = add_row<DT>(terms + tid * stride, nsb);
-    if (TAIL == kTailSwiglu) {  // swiglu_kernel's arithmetic (llm/model.go:446-448)
-        const float u = add_row<DT>(terms + (R + tid) * stride, nsb);
-        const float e = __builtin_exp2f(out * (float)(-1.4426950408889634));
-        const float sg = 1.0f / (1.0f + e);
-        const float silu = out * sg;
-        out = silu * u;
-    } else if (a.resid) {
-        out = out + res;
+    for (int t = tid; t < ROWS * R; t += threads) {
+        const int r = ROWS > 1 ? t / R : 0, result = t - r * R;
+        if (result >= live) continue;
+        const uint8_t* from = terms + (r * local + result) * stride;
+        const int64_t at = (int64_t)(m0 + r) * a.N + first + result;
+        float out = add_row<DT>(from, nsb);
+        if (TAIL == kTailSwiglu) {  // swiglu_kernel's arithmetic (llm/model.go:446-448)
+            const float u = add_row<DT>(from + R * stride, nsb);
+            const float e = __builtin_exp2f(out * (float)(-1.4426950408889634));
+            const float sg = 1.0f / (1.0f + e);
+            const float silu = out * sg;
+            out = silu * u;
+        } else if (a.resid) {
+            out = out + (t == tid ? res : a.resid[at]);
+        }
+        a.y[at] = out;
     }
-    a.y[(int64_t)m * a.N + first + tid] = out;
 }
 
 // How a product is laid out: a workgroup a compute unit, more where its rows are more than kMaxRows.
@@ -420,28 +481,38 @@ int results_of(int64_t N, bool swiglu) {
     const int64_t r = (N + kUnits * turns - 1) / (kUnits * turns);
     return (int)((r + 1) & ~1);
 }
-int lds_of(int dt, int64_t nsb, int rows) {
-    const int64_t x = (nsb * (kStride + 36) + 15) / 16 * 16;
-    return (int)std::min<int64_t>(x + (int64_t)rows * (dt == kQ4_K ? term_row<kQ4_K>((int)nsb) : term_row<kQ6_K>((int)nsb)), 1 << 30);
+int lds_of(int dt, int64_t nsb, int x_rows, int rows) {
+    const int64_t terms = dt == kQ4_K ? term_row<kQ4_K>((int)nsb) : term_row<kQ6_K>((int)nsb);
+    return (int)std::min<int64_t>(x_rows * (x_bytes((int)nsb) + rows * terms), 1 << 30);
 }
 
-template <int DT, int HEAD, int TAIL>
+template <int DT, int ROWS, int HEAD, int TAIL>
 hipError_t launch(const Job& j, int64_t M, hipStream_t st) {
-    const auto kernel = qgemv_kquant_stream_kernel<DT, 2, HEAD, TAIL>;
+    const auto kernel = qgemv_kquant_stream_kernel<DT, ROWS, HEAD, TAIL>;
     static LdsLimit limit;
-    const int lds = lds_of(DT, j.nsb, TAIL == kTailSwiglu ? 2 * j.rows : j.rows);
+    const int lds = lds_of(DT, j.nsb, ROWS, TAIL == kTailSwiglu ? 2 * j.rows : j.rows);
     if (lds > 48 * 1024)
         if (hipError_t e = limit.raise(kMaxLds, {(const void*)kernel})) return e;
-    note_kernel("qgemv_kquant_stream_kernel");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((j.N + j.rows - 1) / j.rows), (unsigned)M), dim3(64 * (unsigned)j.waves), lds, st, j);
+    note_kernel("qgemv_kquant_stream_kernel<%d>", ROWS);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((j.N + j.rows - 1) / j.rows), (unsigned)(ROWS > 1 ? 1 : M)), dim3(64 * (unsigned)j.waves), lds, st, j);
     return hipGetLastError();
 }
-template <int HEAD, int TAIL>
+template <int ROWS, int HEAD, int TAIL>
 hipError_t launch(int dt, const Job& j, int64_t M, hipStream_t st) {
-    return dt == kQ4_K ? launch<kQ4_K, HEAD, TAIL>(j, M, st) : launch<kQ6_K, HEAD, TAIL>(j, M, st);
+    return dt == kQ4_K ? launch<kQ4_K, ROWS, HEAD, TAIL>(j, M, st) : launch<kQ6_K, ROWS, HEAD, TAIL>(j, M, st);
+}
+template <int HEAD, int TAIL>
+hipError_t launch_rows(int dt, const Job& j, int64_t M, int x_rows, hipStream_t st) {
+    switch (x_rows) {
+    case 1: return launch<1, HEAD, TAIL>(dt, j, M, st);
+    case 2: return launch<2, HEAD, TAIL>(dt, j, M, st);
+    default: return launch<3, HEAD, TAIL>(dt, j, M, st);
+    }
 }
 
 int head_of(const QGemvArgs& a, const KqStream& s) { return a.act ? kHeadAct : s.norm_w ? kHeadNorm : kHeadRound; }
+// Rows of x a workgroup: all, but for the forms that have one of them a workgroup.
+int x_rows_of(const QGemvArgs& a, const KqStream& s) { return a.act && s.rope ? 1 : (int)std::min<int64_t>(a.M, 1 << 16); }
 
 }  // namespace
 
@@ -451,26 +522,32 @@ void set_kquant_stream(int v) { g_kq_stream = v; }
 bool qgemv_kquant_stream_ok(int dt, const QGemvArgs& a, const KqStream& s) {
     if ((dt != kQ4_K && dt != kQ6_K) || a.K <= 0 || a.K % 256 || a.N <= 0 || a.N > (1 << 22) || a.M <= 0 || a.M > 65535) return false;
     const int64_t nsb = a.K / 256, lanes = dt == kQ4_K ? 4 : 8, rows = results_of(a.N, s.swiglu) * (s.swiglu ? 2 : 1);
-    if (nsb * lanes > 64 * kMostWaves || ((uintptr_t)a.W & (dt == kQ4_K ? 15 : 1))) return false;
+    const int x_rows = x_rows_of(a, s);
+    if (x_rows > kMostRows || (x_rows > 1 && head_of(a, s) == kHeadRound)) return false;
+    if (nsb * lanes > 64 * (x_rows > 1 ? kFewWaves : kMostWaves) || ((uintptr_t)a.W & (dt == kQ4_K ? 15 : 1))) return false;
     const int64_t row_bytes = nsb * (dt == kQ4_K ? 144 : 210);
     if ((s.swiglu ? a.N + rows : rows) * row_bytes >= kMaxBytes) return false;
     const int head = head_of(a, s);
     if (head != kHeadAct && (((uintptr_t)a.x & 15) || a.x_row_stride % 4)) return false;
     if (head == kHeadNorm && (nsb > 16 || ((uintptr_t)s.norm_w & 15))) return false;
-    if ((s.swiglu && (s.rope || a.resid)) || (head == kHeadRound && (s.swiglu || s.rope)) || (s.rope && a.N % 2)) return false;
-    return lds_of(dt, nsb, (int)rows) <= kMaxLds;
+    if ((s.swiglu && (s.rope || a.resid)) || (head == kHeadRound && s.rope) || (head != kHeadNorm && s.swiglu) || (head == kHeadNorm && !s.swiglu && !s.rope) || (s.rope && a.N % 2)) return false;
+    return lds_of(dt, nsb, x_rows, (int)rows) <= kMaxLds;
 }
 
 // From a converted row where W has more rows than the kernels of short workgroups can be spread over at once, from float32 x where their rounding of x, by four wavefronts a
 // workgroup or a launch of its own, is what takes the time; always where a launch before the product goes with it. us, there | here, converted row: Q4_K 1024 x 4096 3.2 | 3.8,
 // 2048 x 2048 3.5 | 3.6, 2500 x 1024 3.9 | 3.4, 4096 x 4096 4.9 | 4.6, 28672 x 4096 18.9 | 14.4, 128256 x 2048 37 | 28; Q6_K 2048 x 4096 4.4 | 4.5, 2048 x 8192 6.8 | 6.4,
 // 8192 x 2048 6.0 | 6.0, 28672 x 4096 26.7 | 21.8; float32 x: Q4_K 1024 x 2048 3.45 | 3.60, 512 x 4096 4.1 | 3.8, 2048 x 2048 4.1 | 3.85, 4096 x 14336 13.5 | 10.8;
-// Q6_K 2048 x 1024 3.7 | 3.9, 512 x 4096 4.6 | 4.0, 4096 x 14336 16.5 | 14.7.
+// Q6_K 2048 x 1024 3.7 | 3.9, 512 x 4096 4.6 | 4.0, 4096 x 14336 16.5 | 14.7. Two and three converted rows where the kernel that reads W once for eight has four wavefronts a workgroup,
+// two rows there | here: Q4_K 8192 x 4096 7.3 | 7.4, 14336 x 4096 12.7 | 10.2, 14336 x 14336 35.6 | 26.1, Q6_K 14336 x 4096 16.2 | 13.7; three: Q4_K 14336 x 2048 7.7 | 7.9,
+// 14336 x 4096 12.7 | 11.3, Q6_K 14336 x 8192 29.4 | 26.5; four are level, eight (28672 x 4096 Q4_K 22.4) twice as slow here but with the spills of eight rows in registers.
+// A step of two, three and four sequences with its norms here: 10.4 | 9.3, 10.5 | 9.95 and 10.75 | 10.75 ms for 32 of four Q4_K blocks of 4096 features.
 bool qgemv_kquant_stream_pays(int dt, const QGemvArgs& a, const KqStream& s) {
     if (g_kq_stream == 1 || !kquant_by_rule() || !qgemv_kquant_stream_ok(dt, a, s)) return false;
     if (g_kq_stream) return true;
     const int head = head_of(a, s);
     if (head == kHeadNorm) return true;
+    if (a.M > 1 && !s.rope) return a.N > 8192 && a.K >= 2048 * (a.M - 1);
     return head == kHeadAct ? a.N > 2048 : a.N * a.K > (2ll << 20) || a.K >= 3072;
 }
 
@@ -490,18 +567,18 @@ hipError_t qgemv_kquant_stream(int dt, const QGemvArgs& a, const KqStream& s, hi
     j.cuts = (j.nsb + units - 1) / units;
     j.each = (j.nsb + j.cuts - 1) / j.cuts;
     j.packed = j.cuts == 1 ? units / j.each : 1;
-    const int forced = g_kq_stream;
+    const int forced = g_kq_stream, x_rows = x_rows_of(a, s);
     // A wavefront for each load of the first turn where they are few. Else eight, which wait for each other less (28672 x 4096 Q4_K 15.0 us, 15.5 with sixteen), but for long rows,
     // whose rounding takes all there are (4096 x 14336 Q4_K 10.8 with sixteen, 11.3 with eight; Q6_K 14.65 with twelve, 14.8, 15.2 with sixteen).
     const int tasks = ((s.swiglu ? 2 : 1) * j.rows + j.packed - 1) / j.packed * j.cuts;
-    j.waves = forced >= 4 && forced <= kMostWaves ? forced : tasks <= kMostWaves ? std::max(tasks, 8) : j.nsb <= 16 ? 8 : dt == kQ4_K ? kMostWaves : 12;
+    j.waves = x_rows > 1 ? kFewWaves : forced >= 4 && forced <= kMostWaves ? forced : tasks <= kMostWaves ? std::max(tasks, 8) : j.nsb <= 16 ? 8 : dt == kQ4_K ? kMostWaves : 12;
     j.waves = std::max(j.waves, j.cuts);
     j.inv_d = (float)(1.0 / (double)a.K);
     j.eps = (float)s.eps;
     if (s.rope) j.rope = *s.rope;
-    if (s.rope) return head == kHeadAct ? launch<kHeadAct, kTailRope>(dt, j, a.M, st) : head == kHeadNorm ? launch<kHeadNorm, kTailRope>(dt, j, a.M, st) : hipErrorInvalidValue;
-    if (s.swiglu) return head == kHeadAct ? launch<kHeadAct, kTailSwiglu>(dt, j, a.M, st) : head == kHeadNorm ? launch<kHeadNorm, kTailSwiglu>(dt, j, a.M, st) : hipErrorInvalidValue;
-    return head == kHeadAct ? launch<kHeadAct, kTailPlain>(dt, j, a.M, st) : head == kHeadRound ? launch<kHeadRound, kTailPlain>(dt, j, a.M, st) : hipErrorInvalidValue;
+    if (s.rope) return head == kHeadAct ? launch<1, kHeadAct, kTailRope>(dt, j, a.M, st) : launch_rows<kHeadNorm, kTailRope>(dt, j, a.M, x_rows, st);
+    if (s.swiglu) return launch_rows<kHeadNorm, kTailSwiglu>(dt, j, a.M, x_rows, st);
+    return head == kHeadAct ? launch_rows<kHeadAct, kTailPlain>(dt, j, a.M, x_rows, st) : launch<1, kHeadRound, kTailPlain>(dt, j, a.M, st);
 }
 
 }  // namespace mimir

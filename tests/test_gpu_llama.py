@@ -530,6 +530,32 @@ def test_the_choice_brings_in_the_next_embedding(embed, vocab, batch):
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
 
 
+@pytest.mark.parametrize("linear_dt,batch", [(O.Q4_K, 1), (O.Q6_K, 1), (O.Q4_K, 2), (O.Q6_K, 3)])
+def test_kquant_steps_with_norms_and_swiglu_in_the_products_have_the_bits_of_those_without(linear_dt, batch):
+    """One to three sequences: the norms and SwiGLU as parts of the products (rows of three super-blocks, 1280 results) against launches of their own."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.head_dim, c.rope_dim, c.vocab, c.context = 768, 1280, 2, 6, 2, 128, 128, 301, 32
+    om = OL.synthetic(_oracle_config(c), seed=5, linear_dt=linear_dt)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(8 * batch)
+    prompts = np.random.default_rng(7).integers(0, c.vocab, (batch, 5))
+    runs = []
+    try:
+        for stream in (0, 1):
+            capi.check(lib.mi355x_tune(b"kquant.stream", stream))
+            capi.check(lib.mi355x_tune(b"llama.step", 1))  # launches, which a graph of the other choice would stand in for
+            gpu.say(f"steps dt={linear_dt} batch={batch} stream={stream}")
+            m.reset()
+            tokens, _ = m.generate(prompts, 12)
+            runs.append((tokens, np.asarray(m.logits(tokens[:, -1:]))))
+    finally:
+        capi.check(lib.mi355x_tune(b"kquant.stream", 0))
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1].view(np.uint32), runs[1][1].view(np.uint32))
+
+
 def test_fused_steps_without_their_riders_choose_the_per_operator_tokens():
     """The fused step lets the rotation, the norms and the conversion of SwiGLU's results ride on the products
     only where their shapes allow: interleaved pairs, rows of x one step of a wavefront long. A model with

@@ -789,6 +789,28 @@ def test_kquant_one_row_by_a_workgroup_a_compute_unit(dt, waves):
             assert bits_equal(got, want) and bits_equal(got_act, want) and bits_equal(other, want)
 
 
+@pytest.mark.parametrize("m", [2, 3])
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+def test_kquant_two_and_three_rows_by_a_workgroup_a_compute_unit(dt, m):
+    """The same kernel with more rows of x, at rows of W packed, whole and cut, shares of workgroups that do not come out even, and one row with a NaN."""
+    l = gpu.lib()
+    rng = np.random.default_rng(13 * dt + m)
+    for n, k in ((2, 256), (1027, 256 * 3), (513, 256 * 16), (261, 256 * 17), (37, 256 * 56), (9000, 2048 * (m - 1))):
+        raw = random_blocks(rng, dt, n * k)
+        x = rng.normal(size=(m, k)).astype(np.float32)
+        x[0, :256] = 0
+        x[m - 1, k // 2] = np.nan
+        buf, ptr = gpu.dev_bytes_at(raw, 2 if dt == O.Q6_K else 0)
+        want = O.qmatmul(dt, raw, x, n, k)
+        try:
+            capi.check(l.mi355x_tune(b"kquant.stream", 8 if n < 9000 else 0))  # the last by the rule
+            gpu.say(f"kquant few rows dt={dt} M={m} N={n} K={k}")
+            got, got_act = gpu.qgemv(dt, ptr, gpu.dev(x), n, k), gpu.qgemv_act(dt, ptr, gpu.dev(x), n, k)
+        finally:
+            capi.check(l.mi355x_tune(b"kquant.stream", 0))
+        assert bits_equal(got, want) and bits_equal(got_act, want)
+
+
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
 @pytest.mark.parametrize("m,n,k", [(2, 33, 256), (5, 100, 512), (8, 203, 4096), (11, 64, 256 * 9), (20, 31, 256 * 56), (40, 130, 1024),
                                    (3, 40, 256 * 37), (4, 33, 256 * 70), (9, 300, 256 * 33)])

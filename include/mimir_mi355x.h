@@ -504,6 +504,8 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * workgroup where it has a form of that many (0: by shape). "kquant.shared" = 1
  * keeps products of up to 512 rows of x off the kernel that reads sixteen rows of
  * W once for up to 64 of x, 2 sends them all there (0: by shape).
+ * "q4_0.few" = 1 keeps Q4_0 products of two to four rows of x, and steps of two
+ * sequences, off the kernel for so few, 2 sends all products it takes there.
  * "kquant.stream" = 1 keeps products of one row of x off the kernel with a
  * workgroup per compute unit, 4 to 16 sends all it takes there, with that many
  * wavefronts a workgroup (0: by shape).

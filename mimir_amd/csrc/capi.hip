@@ -295,6 +295,11 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             const size_t plain = rows ? mimir::q4_0_rows_act_bytes(K) * (size_t)(one_launch ? (M + 7) / 8 : 1)
                                       : (fx ? mimir::q4_0_fx_act_bytes(K) : mimir::q4_0_act_bytes(K)) * (size_t)M;
             const size_t scratch = src.fixed ? 0 : q4_0_scratch_bytes(W, M, N, K, wide_x);
+            // two to four of them: x's digits in registers, one launch
+            if (rows && g_rows_max == 0 && mimir::qgemv_q4_0_few_pays(a, mimir::Q4Few{})) {
+                HIP_TRY(mimir::qgemv_q4_0_few(a, mimir::Q4Few{}, (hipStream_t)stream), "launch qgemv_q4_0_few");
+                return MI355X_OK;
+            }
             // some tens of rows, where W read where it lies by pairs of binary16 undercuts both
             if (M >= 16 && M <= mimir::kInPlaceRows && wide_x && !fx_forced && g_tune_q4[4] != 2 && g_rows_path != 1 && g_rows_max == 0 && q4_0_in_place_pays(W, M, N, K, rows)) {
                 const size_t act_bytes = rounded(mimir::q4_0_fx16_act_bytes(M, K)), ws = mimir::qgemm_q4_0_in_place_sums_bytes(M, N, K);
@@ -701,6 +706,10 @@ mi355x_status mi355x_tune(const char* key, int value) {
         }
     if (key && (strcmp(key, "kquant.rows") == 0 || strcmp(key, "kquant.path") == 0)) {
         mimir::set_kquant_tune(key[7] == 'p', value);
+        return MI355X_OK;
+    }
+    if (key && strcmp(key, "q4_0.few") == 0) {
+        mimir::set_q4_few(value);
         return MI355X_OK;
     }
     if (key && strcmp(key, "kquant.stream") == 0) {

@@ -112,6 +112,22 @@ struct Q4RopeTail {
 };
 hipError_t qgemv_q4_0_act_qkv_rope(const void* const W[3], const int64_t n[3], const void* act, float* y, int64_t M, int64_t K,
                                    const Q4RopeTail& rope, const Q4NormHead& norm, const int* tune, hipStream_t st);
+// Two to four rows of x by Q4_0 with a workgroup per compute unit (qgemv_q4_0_few.hip), the bits of one row's kernel. a.act: rows of q4_0_convert_act; null: float32 a.x (16-byte
+// aligned), which every workgroup converts for itself. Two rows alone: a.act, and with norm_w the RMSNorm in front as well (q4_0_norm_head_ok(K)), and then one of the tails: a.W, W1 and W2 q, k (n1 rows)
+// and v behind n0 rows of q, a.N in all, with the rotation and the cache writes; or a.W gate and W1 up of a.N rows, y = SiLU(gate . x) (up . x). ("q4_0.few": 1 never, 2 always)
+struct Q4Few {
+    const void *W1 = nullptr, *W2 = nullptr;
+    int64_t n0 = 0, n1 = 0;
+    const float* norm_w = nullptr;
+    double eps = 0;
+    const Q4RopeTail* rope = nullptr;
+    bool swiglu = false;
+};
+bool qgemv_q4_0_few_ok(const QGemvArgs& a, const Q4Few& q);
+bool qgemv_q4_0_few_pays(const QGemvArgs& a, const Q4Few& q);
+hipError_t qgemv_q4_0_few(const QGemvArgs& a, const Q4Few& q, hipStream_t st);
+void set_q4_few(int v);
+bool q4_0_few_on();  // not switched off
 // The same tail behind a Q4_K or Q6_K product (qgemv_kquant_rope_ok says whether the shape qualifies).
 bool qgemv_kquant_rope_ok(int dt, const QGemvArgs& a);
 hipError_t qgemv_kquant_act_rope(int dt, const QGemvArgs& a, const Q4RopeTail& rope, hipStream_t st);

@@ -88,10 +88,14 @@ struct Model : Decoder {
     mi355x_status embed_next() override;
     void next_embedding(ChooseTail& tail) const override;
     int step_variant() const override;
+    bool few_fit = false;  // a rows model of so few sequences that step_few takes it
+    bool few() const;
     // A step of Q4_0 linears is some 5 launches a block, 8 of several sequences, that read W once for eight of them; forward(1) has 16, of a row at a time: 300 us
     // a call against 520 (four blocks of 4096 features), 8 sequences 500 against 1000. Blocks of other dtypes and the stacks are within 1 % either way. Measured up to 16 sequences.
     bool one_token_as_step() const override { return fast && c.batch <= 16; }
 };
+
+constexpr int kFewSequences = 2;  // of more the step with kernels for eight is level or faster (qgemv_q4_0_few.hip)
 
 bool is_kquant(const Weight& w) { return w.set() && (w.dtype == kQ4_K || w.dtype == kQ6_K); }
 
@@ -479,6 +483,75 @@ static mi355x_status step_rows(Model& m) {
     return MI355X_OK;
 }
 
+// Two sequences of the same models: step_fast's operations with every weight read once for all of them and the norms in the products
+// (qgemv_q4_0_few.hip), six launches a block: norm, q|k|v, rotation and cache write; attention with conversion; output projection; norm, gate|up and
+// SiLU * up; conversion; down projection. The products of block i, whose y, resid and converted x are left to the launch:
+struct FewProducts {
+    QGemvArgs qkv, o, gate_up, down;
+    Q4Few qkv_q, gate_up_q;
+    Q4RopeTail rope;
+};
+static void few_products(const Model& m, int i, FewProducts* f) {
+    const auto& c = m.c;
+    const Block& b = m.blocks[i];
+    const int64_t B = c.batch, qd = (int64_t)c.heads * c.head_dim, kvd = (int64_t)c.kv_heads * c.head_dim;
+    float* x = m.x.as<float>();
+    Q4RopeTail& tail = f->rope;
+    tail.cosv = m.cos_t.as<float>(); tail.sinv = m.sin_t.as<float>(); tail.pos = m.state.as<int32_t>();
+    tail.kcache = m.keys[i].p; tail.vcache = m.values[i].p;
+    tail.cache_dt = c.cache_dtype; tail.H = c.heads; tail.HK = c.kv_heads; tail.dim = c.head_dim; tail.rope_dim = c.rope_dim;
+    tail.cap = c.context;
+    f->qkv = QGemvArgs{b.q.buf.p, x, nullptr, m.qkv.as<float>(), B, qd + 2 * kvd, c.embed, c.embed, 0};
+    f->qkv_q.W1 = b.k.buf.p; f->qkv_q.W2 = b.v.buf.p; f->qkv_q.n0 = qd; f->qkv_q.n1 = kvd;
+    f->qkv_q.norm_w = b.attn_norm.buf.as<float>(); f->qkv_q.eps = c.eps; f->qkv_q.rope = &tail;
+    f->o = QGemvArgs{b.o.buf.p, nullptr, m.act[kActQ4].p, x, B, c.embed, qd, 0, 0};
+    f->o.resid = x;
+    f->gate_up = QGemvArgs{b.gate.buf.p, x, nullptr, m.s.as<float>(), B, c.hidden, c.embed, c.embed, 0};
+    f->gate_up_q.W1 = b.up.buf.p;
+    f->gate_up_q.norm_w = b.ffn_norm.buf.as<float>(); f->gate_up_q.eps = c.eps; f->gate_up_q.swiglu = true;
+    f->down = QGemvArgs{b.down.buf.p, nullptr, m.act[kActQ4].p, x, B, c.embed, c.hidden, 0, 0};
+    f->down.resid = x;
+}
+static bool few_sequences(const Model& m) {
+    const auto& c = m.c;
+    if (!m.rows || c.batch > kFewSequences || !c.interleaved || c.head_dim % 2 || c.rope_dim % 2) return false;
+    if (m.act[kActQ4].bytes < (size_t)c.batch * q4_0_act_bytes(std::max<int64_t>((int64_t)c.heads * c.head_dim, c.hidden))) return false;
+    for (int i = 0; i < c.layers; i++) {
+        FewProducts f;
+        few_products(m, i, &f);
+        if (!qgemv_q4_0_few_ok(f.qkv, f.qkv_q) || !qgemv_q4_0_few_ok(f.o, Q4Few{}) || !qgemv_q4_0_few_ok(f.gate_up, f.gate_up_q) || !qgemv_q4_0_few_ok(f.down, Q4Few{})) return false;
+    }
+    return true;
+}
+static mi355x_status step_few(Model& m) {
+    const auto& c = m.c;
+    const int64_t B = c.batch, qd = (int64_t)c.heads * c.head_dim, kvd = (int64_t)c.kv_heads * c.head_dim, row = qd + 2 * kvd;
+    void* act = m.act[kActQ4].p;
+    AttnArgs at;
+    at.q = m.qkv.as<float>(); at.kv_dtype = c.cache_dtype; at.out = nullptr; at.lse = nullptr;
+    at.q_strides[0] = row; at.q_strides[1] = c.head_dim; at.q_strides[2] = 0;
+    at.k_strides[0] = at.v_strides[0] = (int64_t)c.kv_heads * c.context * c.head_dim;
+    at.k_strides[1] = at.v_strides[1] = (int64_t)c.context * c.head_dim;
+    at.k_strides[2] = at.v_strides[2] = c.head_dim;
+    at.o_strides[0] = qd; at.o_strides[1] = c.head_dim; at.o_strides[2] = 0;
+    at.B = B; at.Q = 1; at.K = 1; at.H = c.heads; at.HK = c.kv_heads; at.D = c.head_dim;
+    at.scale = 1.0 / std::sqrt((double)c.head_dim);
+    at.causal = 0; at.causal_offset = 0;
+    at.dyn_k = m.state.as<int32_t>();  // position p holds p keys before this step's own
+    for (int i = 0; i < c.layers; i++) {
+        FewProducts f;
+        few_products(m, i, &f);
+        LLM_HIP(qgemv_q4_0_few(f.qkv, f.qkv_q, m.stream), "norm, q|k|v, rope and cache");
+        at.k = m.keys[i].p; at.v = m.values[i].p;
+        LLM_HIP(attention_decode(at, c.context, m.act[0].p, act, (int64_t)q4_0_act_bytes(qd), m.stream, kAttnActQ4, m.attn_flags.p, m.attn_flags.bytes, device_error_word()), "attention");
+        LLM_HIP(qgemv_q4_0_few(f.o, Q4Few{}, m.stream), "attn_output");
+        LLM_HIP(qgemv_q4_0_few(f.gate_up, f.gate_up_q, m.stream), "norm, gate|up and swiglu");
+        LLM_HIP(q4_0_convert_act(m.s.as<float>(), B, c.hidden, c.hidden, act, m.stream), "convert");
+        LLM_HIP(qgemv_q4_0_few(f.down, Q4Few{}, m.stream), "ffn_down");
+    }
+    return MI355X_OK;
+}
+
 // One decoding step of every sequence for blocks of any supported dtypes: the per-operator launches of
 // forward() for one position, but with the position read from m.state on the device (rotation, cache
 // write, number of keys), so that the step can be captured once and replayed as a graph like step_fast
@@ -679,12 +752,14 @@ void Model::next_embedding(ChooseTail& tail) const {
 }
 
 mi355x_status Model::step() {
-    if (mi355x_status st = rows && !g_llama_rows_off ? step_rows(*this) : fast ? step_fast(*this) : step_any(*this)) return st;
+    if (mi355x_status st = rows && !g_llama_rows_off ? (few() ? step_few(*this) : step_rows(*this)) : fast ? step_fast(*this) : step_any(*this)) return st;
     return mimir::head(*this, x.as<float>(), c.batch, c.embed);
 }
 
-// 0 step_fast or step_any, 1 step_rows, more: step_rows without its riders
-int Model::step_variant() const { return rows && !g_llama_rows_off ? 1 + g_llama_rows_plain : 0; }
+// (no measurement aid asks for the step of kernels for eight rows)
+bool Model::few() const { return few_fit && g_llama_rows_plain == 0 && q4_0_few_on(); }
+// 0 step_fast or step_any, -1 step_few, 1 step_rows, more: step_rows without its riders
+int Model::step_variant() const { return rows && !g_llama_rows_off ? (few() ? -1 : 1 + g_llama_rows_plain) : 0; }
 
 }  // namespace mimir
 
@@ -973,6 +1048,7 @@ mi355x_status mimir::Model::finalize(int64_t max_tokens) {
         LLM_HIP(m->rows_act2.alloc(ab), "hipMalloc(activations)");
         LLM_HIP(hipMemset(m->rows_act2.p, 0, ab), "hipMemset(activations)");
         LLM_HIP(m->parts.alloc((size_t)2 * c.batch * c.embed * 4), "hipMalloc");
+        m->few_fit = few_sequences(*m);
     }
     m->ready = true;
     return MI355X_OK;

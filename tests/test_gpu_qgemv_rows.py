@@ -47,6 +47,34 @@ def test_rows_kernel_matches_oracle_and_one_row_kernel(m, n, k):
     assert np.all(np.abs(got - one) <= 1e-6 * mag + 1e-30)  # the same integers, another order of float32 additions
 
 
+@pytest.mark.parametrize("m", [2, 3, 4])
+@pytest.mark.parametrize("n,k", [(1, 64), (257, 4096), (513, 4096 + 64), (1100, 1024), (2051, 192), (35, 14336), (9000, 2112)])
+def test_two_to_four_rows_by_a_workgroup_a_compute_unit(m, n, k):
+    """One pair of blocks a row of W, a wavefront's worth, one more (cut over two wavefronts), four cuts; shares of workgroups that do not come out even: the bound of the kernel
+    for eight rows, by that kernel too, and the one-row kernel's integers. One row with a NaN is NaN, the others are as they were."""
+    l = gpu.lib()
+    rng = np.random.default_rng(m * 100 + n + k)
+    raw = random_blocks(rng, O.Q4_0, n * k)
+    x = (rng.normal(size=(m, k)) * np.exp(rng.normal(size=(m, 1)) * 3)).astype(np.float32)
+    x[0, :32] = 0
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    want = O.qmatmul(O.Q4_0, raw, x, n, k)
+    mag = np.abs(x.astype(np.float64)) @ np.abs(O.dequantize(O.Q4_0, raw).reshape(n, k).astype(np.float64)).T
+    one = per_row(l, ptr, gpu.dev(x), n, k)
+    bad = x.copy()
+    bad[m - 1, k // 2] = np.nan
+    try:
+        for few in (2, 1):
+            capi.check(l.mi355x_tune(b"q4_0.few", few))
+            gpu.say(f"q4_0 few rows M={m} N={n} K={k} few={few}")
+            got = gpu.qgemv(O.Q4_0, ptr, gpu.dev(x), n, k)
+            assert np.all(np.abs(got - want) <= 2e-6 * mag + 1e-30) and np.all(np.abs(got - one) <= 1e-6 * mag + 1e-30)
+            worse = gpu.qgemv(O.Q4_0, ptr, gpu.dev(bad), n, k)
+            assert np.isnan(worse[m - 1]).all() and np.array_equal(worse[:-1].view(np.uint32), got[:-1].view(np.uint32))
+    finally:
+        capi.check(l.mi355x_tune(b"q4_0.few", 0))
+
+
 def test_rows_kernel_at_the_model_shapes():
     """Bench-generated weights at the 8B shapes, eight rows: within the path's 1e-3 of the oracle."""
     rng = np.random.default_rng(3)

@@ -247,6 +247,21 @@ def test_other_sizes(tmp_path, name, dtype):
         assert e < TOL[dtype], (sizes, e)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rank,vdim", [(520, 40), (1000, 72), (64, 7)])
+def test_latent_steps_over_more_shares_than_are_requested_ahead(tmp_path, rank, vdim, dtype):
+    """Steps at 65, 512, 513 and 600 positions (2, 8, 9 and 10 shares of the keys) with latents of one, two and four columns a thread, and of values that
+    come out even among the wavefronts and not."""
+    c = X.config([X.latent(heads=2, dim=24, rot_dim=8, vdim=vdim, kv_rank=rank)])
+    w = X.weights(c, 9)
+    toks = X.tokens(c, 600, 9)
+    want = F.forward(c, w, toks)
+    gpu.say(f"fuvolix latent shares rank={rank} {dtype}")
+    m = load(tmp_path, c, w, context=600, dtype=dtype)
+    for sizes in ([64, 1, 446, 1, 1, 86, 1], [597, 1, 1, 1]):
+        assert X.error(in_portions(m, toks, sizes), want) < TOL[dtype], sizes
+
+
 def test_gates_and_states_far_from_one(tmp_path):
     """Gates driven to their cap in both directions, and a state that decays to nothing and starts anew. A state of one
     key only gives o = v sign(k . q): the few rows where k . q is within its rounding of zero are not looked at."""

@@ -245,6 +245,18 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
             return MI355X_OK;
         }
     }
+    if (dtype == MI355X_Q8_0 && g_tune_gemm != 1 && g_rows_path != 1 && ((uintptr_t)X & 7) == 0 && x_row_stride % 4 == 0 && mimir::q8_act_fits(K)) {
+        // the same without the casts' launches and their float32 copies, where several rows go to the int8 matrix cores (32 x 4096 x 4096 18.1 us, now 13.7)
+        mimir::QGemvArgs a{W, nullptr, (void*)256, (float*)Y, M, N, K, 0, 0};
+        if (mimir::qgemv_q8_0_mfma_pays(a)) {
+            void* act;
+            if (mi355x_status s2 = act_scratch(stream, mimir::q8_act_bytes(K) * (size_t)M, &act)) return s2;
+            a.act = act;
+            HIP_TRY(mimir::q8_convert_act_bf16(X, M, K, x_row_stride, act, st), "launch q8_convert_act");
+            HIP_TRY(mimir::qgemv_q8_0_mfma(a, st, !f32), "launch qgemv_q8_0_mfma");
+            return MI355X_OK;
+        }
+    }
     // Any other shape or dtype: the activations as float32 through mi355x_qgemv, then one rounding. For
     // Q8_0, Q4_K and Q6_K that is the reference's own sequence (cast, int8 rounding of x, integer dot
     // products, cast), and the K-quants take their matrix-core kernel from a few rows on.

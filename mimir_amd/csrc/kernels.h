@@ -140,6 +140,7 @@ hipError_t qgemv_q4_0_act_swiglu(const void* gate, const void* up, const void* a
 bool q8_act_fits(int64_t K);
 size_t q8_act_bytes(int64_t K);
 hipError_t q8_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);
+hipError_t q8_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st);  // of bfloat16 x, rows on 8 bytes
 // The same of rmsnorm's result, rows of x x_row_stride floats apart, d a multiple of 32, x and w 16-byte aligned.
 hipError_t rmsnorm_q8_act(const float* x, int64_t x_row_stride, const float* w, void* act, int64_t rows, int64_t d, double eps, hipStream_t st);
 hipError_t qgemv_q8_0_act(const QGemvArgs& a, const int* tune, hipStream_t st);
@@ -153,7 +154,7 @@ hipError_t qgemv_q8_0_rows(const QGemvArgs& a, hipStream_t st);
 bool qgemv_q8_0_mfma_ok(const QGemvArgs& a);
 bool qgemv_q8_0_mfma_pays(const QGemvArgs& a);
 void set_q8_mfma(int v);
-hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st);
+hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st, bool y_bf16 = false);  // y_bf16: results rounded once, into y taken as uint16_t*
 
 // The Q4_K and Q6_K products as the reference's CPU computes them: x rounded
 // to int8 in super-blocks of 256 with the sums of each 16 quants

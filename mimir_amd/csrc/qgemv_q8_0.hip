@@ -65,24 +65,39 @@ __device__ __forceinline__ void q8_convert_item(const f32x4 v, uint32_t* q, floa
     if (i == 0) dscale[b] = d;
 }
 
-__global__ __launch_bounds__(256) void q8_convert_act_kernel(const float* __restrict__ x, int64_t x_row_stride, int nb,
+template <bool BF16>  // x float32, or bfloat16 (widened exactly, as the cast in front of the product does: tensor/quant.go:45-48)
+__global__ __launch_bounds__(256) void q8_convert_act_kernel(const void* __restrict__ x, int64_t x_row_stride, int nb,
                                                              uint8_t* __restrict__ act, int64_t act_row_bytes) {
-    const float* xr = x + (int64_t)blockIdx.y * x_row_stride;
+    const int64_t row = (int64_t)blockIdx.y * x_row_stride;
     uint32_t* q = (uint32_t*)(act + (int64_t)blockIdx.y * act_row_bytes);
     const int nbp = nb | 1;
     float* dscale = (float*)(q + 2 * nbp * 4);
     const int nq = nb * 8;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nq; t += gridDim.x * blockDim.x) {
         f32x4 v;
-        __builtin_memcpy(&v, xr + 4 * (int64_t)t, 16);
+        if (BF16) {
+            u32x2 h;
+            __builtin_memcpy(&h, (const uint16_t*)x + row + 4 * (int64_t)t, 8);
+            const uint32_t low = h[0], high = h[1];
+            v = f32x4{__uint_as_float(low << 16), __uint_as_float(low & 0xffff0000u), __uint_as_float(high << 16), __uint_as_float(high & 0xffff0000u)};
+        } else {
+            __builtin_memcpy(&v, (const float*)x + row + 4 * (int64_t)t, 16);
+        }
         q8_convert_item(v, q, dscale, nbp, t);
     }
+}
+
+hipError_t q8_convert_act_bf16(const void* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
+    int nb = (int)(K / 32);
+    int gx = (nb * 8 + 255) / 256;
+    hipLaunchKernelGGL(q8_convert_act_kernel<true>, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, nb, (uint8_t*)act, (int64_t)q8_act_bytes(K));
+    return hipGetLastError();
 }
 
 hipError_t q8_convert_act(const float* x, int64_t M, int64_t K, int64_t x_row_stride, void* act, hipStream_t st) {
     int nb = (int)(K / 32);
     int gx = (nb * 8 + 255) / 256;
-    hipLaunchKernelGGL(q8_convert_act_kernel, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, nb,
+    hipLaunchKernelGGL(q8_convert_act_kernel<false>, dim3((unsigned)gx, (unsigned)M), dim3(256), 0, st, x, x_row_stride, nb,
                        (uint8_t*)act, (int64_t)q8_act_bytes(K));
     return hipGetLastError();
 }

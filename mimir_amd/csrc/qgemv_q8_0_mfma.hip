@@ -55,8 +55,8 @@ constexpr int kWaveLds = kSlabBytes + kRunBlocks * XR * 4 + (XR == kManyRows ? X
 // XR: rows of x a workgroup (8 or 32); WAVES: its wavefronts, among which the runs of K go round. AHEAD: a run's loads stay a run ahead, which takes the
 // registers of two wavefronts: for so few workgroups that no more are on a compute unit (four sums, us, without and with: 4 x 8192 x 14336 48, 33).
 template <int XR, int WAVES, bool FOUR = false, bool AHEAD = false>
-__global__ __launch_bounds__(64 * WAVES, XR == kManyRows || AHEAD ? 2 : 4) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, float* y, int M,
-                                                                                             int N, int nb, int64_t act_row_bytes) {
+__global__ __launch_bounds__(64 * WAVES, XR == kManyRows || AHEAD ? 2 : 4) void qgemv_q8_0_mfma_kernel(const uint8_t* __restrict__ W, const uint8_t* act, void* yv, int M,
+                                                                                             int N, int nb, int64_t act_row_bytes, int y_bf16) {
     constexpr bool kMany = XR == kManyRows;
     constexpr int kSums = FOUR ? 16 : XR / 2;  // of a lane
     static_assert(!FOUR || XR == 8, "four sums of each of a lane's four rows");
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows || AHEAD ? 2 : 4) void 
     float* dxs = (float*)(slab + kSlabBytes);
     uint8_t* xslab = slab + kSlabBytes + kRunBlocks * XR * 4;
     act += (int64_t)XR * group * act_row_bytes;
-    y += (int64_t)XR * group * N;
+    const int64_t y0 = (int64_t)XR * group * N;
     M = M - XR * group < XR ? M - XR * group : XR;
 
     // piece p = 64 i + lane of a run: row p / 17 of the 32, bytes 16 (p % 17).. of its 272
@@ -244,7 +244,11 @@ __global__ __launch_bounds__(64 * WAVES, XR == kManyRows || AHEAD ? 2 : 4) void 
     for (int s = wave; s < (FOUR ? 4 : kSums); s += WAVES) {
         const float v = FOUR ? (sum_of(s) + sum_of(8 + s)) + (sum_of(4 + s) + sum_of(12 + s)) : sum_of(s);
         const int m = 8 * (s >> 2) + 4 * lh + (s & 3);
-        if (n < N && m < M) y[(int64_t)m * N + n] = v;
+        if (n < N && m < M) {
+            const int64_t at = y0 + (int64_t)m * N + n;
+            if (y_bf16) ((uint16_t*)yv)[at] = f32_to_bf16_bits(v);
+            else ((float*)yv)[at] = v;
+        }
     }
 }
 
@@ -274,28 +278,28 @@ bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
 }
 
 template <int XR, int WAVES, bool FOUR = false, bool AHEAD = false>
-static hipError_t launch(const QGemvArgs& a, int64_t wgs, hipStream_t st) {
+static hipError_t launch(const QGemvArgs& a, int64_t wgs, bool bf16, hipStream_t st) {
     constexpr int kLds = WAVES * kWaveLds<XR>;
     if (kLds > 64 * 1024) {
         static LdsLimit limit;
         if (hipError_t e = limit.raise(kLds, {(const void*)qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>})) return e;
     }
-    hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, a.y,
-                       (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K));
+    hipLaunchKernelGGL((qgemv_q8_0_mfma_kernel<XR, WAVES, FOUR, AHEAD>), dim3((unsigned)wgs), dim3(64 * WAVES), kLds, st, (const uint8_t*)a.W, (const uint8_t*)a.act, (void*)a.y,
+                       (int)a.M, (int)a.N, (int)(a.K / 32), (int64_t)q8_act_bytes(a.K), bf16 ? 1 : 0);
     return hipGetLastError();
 }
 
 // Eight wavefronts a workgroup where all workgroups then are on the chip at once, two a compute unit of eight rows, one of 32
 // (us with four, with eight: 2 x 14336 x 4064 21, 20; 32 x 4096 x 14336 65, 45; past it, 64 x 8192 x 4096 26, 30), else four.
-hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st) {
+hipError_t qgemv_q8_0_mfma(const QGemvArgs& a, hipStream_t st, bool bf16) {
     const int rows = a.M > kFewRows ? kManyRows : 8;
     const int64_t wgs = ((a.N + 31) / 32) * ((a.M + rows - 1) / rows);
     if (wgs > 0x7fffffff) return hipErrorInvalidValue;
     // from 64 M weights on, of whole runs: sums in the order in which they always were
     if (a.M <= kFewRows && a.N * a.K >= ((int64_t)64 << 20) && a.K % 256 == 0 && ((uintptr_t)a.W & 15) == 0)
-        return wgs <= 512 ? launch<8, 4, true, true>(a, wgs, st) : launch<8, 4, true>(a, wgs, st);
-    if (rows == 8) return wgs <= 512 ? launch<8, 8>(a, wgs, st) : launch<8, 4>(a, wgs, st);
-    return wgs <= 256 ? launch<kManyRows, 8>(a, wgs, st) : launch<kManyRows, 4>(a, wgs, st);
+        return wgs <= 512 ? launch<8, 4, true, true>(a, wgs, bf16, st) : launch<8, 4, true>(a, wgs, bf16, st);
+    if (rows == 8) return wgs <= 512 ? launch<8, 8>(a, wgs, bf16, st) : launch<8, 4>(a, wgs, bf16, st);
+    return wgs <= 256 ? launch<kManyRows, 8>(a, wgs, bf16, st) : launch<kManyRows, 4>(a, wgs, bf16, st);
 }
 
 }  // namespace mimir

@@ -538,3 +538,32 @@ def test_rows_with_an_infinity_or_a_nan_leave_the_others_sums_alone(half, m, n, 
         want = O.bf16_to_f32(bf16_bits(x)).astype(np.float64) @ O.dequantize(O.Q4_0, w).reshape(n, k).astype(np.float64).T
         fits = np.abs(want[bad[0]]) < 3e38
         assert fits.any() and np.allclose(product(x)[bad[0]][fits], want[bad[0]][fits], rtol=1e-4)
+
+
+@pytest.mark.parametrize("m,n,k,stride,offset", [(16, 2048, 256, 256, 0), (33, 1001, 288, 300, 2), (9, 4097, 1056, 1056, 0), (100, 512, 4096, 4104, 0), (4, 8192, 4096, 4096, 0)])
+def test_q8_0_bfloat16_rows_on_the_int8_matrix_cores(m, n, k, stride, offset):
+    """Rows rounded from bfloat16 and results rounded as they are stored: the bits of the general route (casts around the float32 product), for both output types, with
+    a NaN, an infinity and a block of zeros, W on an even address, rows apart."""
+    l = gpu.lib()
+    rng = np.random.default_rng(m + n + k)
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[0, :32] = 0
+    x[1, 40] = np.inf
+    x[2, 50] = np.nan
+    wbuf, wp = gpu.dev_bytes_at(raw, offset)
+    xs = torch.zeros(m, stride, dtype=torch.bfloat16, device="cuda:0")
+    xs[:, :k] = torch.from_numpy(x).to("cuda:0").to(torch.bfloat16)
+    for out, kind in ((capi.BF16, torch.int16), (capi.F32, torch.int32)):
+        got = []
+        try:
+            for path in (0, 1):
+                capi.check(l.mi355x_tune(b"qgemm.path", path))
+                y = torch.full((m, n), -1, dtype=kind, device="cuda:0")
+                gpu.say(f"q8_0 bf16 M={m} N={n} K={k} out={out} path={path}")
+                capi.check(l.mi355x_qgemm_bf16(capi.Q8_0, wp, xs.data_ptr(), y.data_ptr(), m, n, k, stride, out, gpu.stream()))
+                gpu.sync()
+                got.append(y.cpu().numpy())
+        finally:
+            capi.check(l.mi355x_tune(b"qgemm.path", 0))
+        assert np.array_equal(got[0], got[1])

@@ -95,6 +95,17 @@ mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, s
     return MI355X_OK;
 }
 
+// Whether act_scratch(stream, bytes) would not have to grow a block under capture.
+bool act_at_hand(void* stream, size_t bytes) {
+    DeviceState* s;
+    if (current_state(&s) != MI355X_OK) return false;
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (s->scratch[stream].act.bytes >= bytes) return true;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) (void)hipGetLastError();
+    return capture == hipStreamCaptureStatusNone;
+}
+
 mi355x_status act_scratch(void* stream, size_t bytes, void** out, size_t wish = 0) {
     return stream_scratch(stream, &StreamScratch::act, bytes, wish, kActFloorBytes, 0, "activation", out);
 }
@@ -378,7 +389,12 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
         if (!mimir::q8_act_fits(K)) return capi_fail(MI355X_ERR_SHAPE, "mi355x: qgemv by q8_0 with K = %lld: rows longer than 57344 are not supported", (long long)K);
         // Small products in one launch (a.act stays null: every workgroup rounds x for itself, its first weights under way meanwhile); on large
         // ones that many workgroups' rounding costs more than a conversion launch of its own (measured).
-        if (M <= kConvertInProductRows && N * K <= (int64_t)24 << 20 && ((uintptr_t)x & 15) == 0 && (M == 1 || x_row_stride % 4 == 0)) {
+        mimir::QGemvArgs converted = a;
+        converted.act = (void*)256;
+        bool matrix = g_rows_path != 1 && mimir::qgemv_q8_0_mfma_pays(converted);  // a large matrix or many rows: the int8 matrix cores
+        const bool in_product = M <= kConvertInProductRows && N * K <= (int64_t)24 << 20 && ((uintptr_t)x & 15) == 0 && (M == 1 || x_row_stride % 4 == 0);
+        if (matrix && in_product && !src.fixed) matrix = act_at_hand(stream, mimir::q8_act_bytes(K) * (size_t)M);  // which the one launch does without
+        if (!matrix && in_product) {
             HIP_TRY(mimir::qgemv_q8_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q8_0");
             return MI355X_OK;
         }
@@ -386,7 +402,7 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
         if (mi355x_status st = act_for(src, mimir::q8_act_bytes(K) * (size_t)M, &act)) return st;
         HIP_TRY(mimir::q8_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q8_convert_act");
         a.act = act;
-        if (g_rows_path != 1 && mimir::qgemv_q8_0_mfma_pays(a)) {  // a large matrix or many rows: the int8 matrix cores
+        if (matrix) {
             HIP_TRY(mimir::qgemv_q8_0_mfma(a, (hipStream_t)stream), "launch qgemv_q8_0_mfma");
             return MI355X_OK;
         }

@@ -266,14 +266,17 @@ bool qgemv_q8_0_mfma_ok(const QGemvArgs& a) {
 static std::atomic<int> g_q8_mfma{0};  // measurement aid: 1 = wherever the kernel takes the shape, 2 = never
 void set_q8_mfma(int v) { g_q8_mfma = v; }
 
-// Up to eight rows: matrices of 32 M weights and more that give the chip 128 workgroups, for two and three rows 192
-// (us by the vector unit, here; 8 rows: 8192 x 4096 34, 13; 4 rows: 4096 x 8192 19, 17, 2048 x 16384 18, 28; 2 rows:
-// 6144 x 8192 20, 18, 4096 x 14336 24, 26). More rows: from 32768 results (9 x 4096 x 4096 31, 12; 32 x 1024 x 14336
-// 42, 28; 128 x 256 x 1024 18, 8; against 9 x 1024 x 4096 11.3, 11.8; 64 x 64 x 14336 20, 28).
+// Up to eight rows: matrices of 32 M weights and more that give the chip 128 workgroups, for two and three rows 192 (us by the vector unit, here; 8 rows: 8192 x 4096 34, 13; 4 rows:
+// 4096 x 8192 19, 17, 2048 x 16384 18, 28; 2 rows: 6144 x 8192 20, 18, 4096 x 14336 24, 26), and of short rows, of which the vector unit has as much to do whatever their length: eight rows
+// 14336 x 1024 29.7, 8.1, 14336 x 2048 49.7, 12.1, 4096 x 1024 10.5, 6.5; four 4096 x 1024 6.4, 6.4, 8192 x 2048 12.6, 8.3; three 8192 x 1024 8.4, 6.7, but 4096 x 2048 6.3, 7.3; two 14336 x
+// 1024 9.3, 7.9, but 12288 x 2048 10.9, 11.0, 8192 x 2048 7.8, 8.2. Other few rows keep the bits that a row alone has.
+// More rows, of which the vector unit takes eight a pass over W: from 64 rows of W on nearly always; nine rows 512 x 1024 10.6, 7.5, 64 x 2048 10.3, 8.3, 1280 x 4096 15.6, 11.7, 3072 x 14336 46, 30,
+// 17 rows 1024 x 4096 17.2, 12.1, but sixteen 1024 x 4096 11.3, 12.0, 512 x 8192 10.8, 17.5, twelve 1536 x 8192 16.8, 17.7 (2048 x 8192 19.8, 17.7), nine 2048 x 14336 27.5, 29.4 (twelve 32.7, 29.7).
 bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
     if (g_q8_mfma == 2 || !qgemv_q8_0_mfma_ok(a)) return false;
     if (g_q8_mfma == 1) return true;
-    if (a.M > kFewRows) return a.M * a.N >= 32768;
+    if (a.M > kFewRows) return a.M * a.N >= 32768 || (a.N >= 64 && (a.K <= 2048 || (a.K <= 6144 ? a.N >= 1280 || a.M * a.N >= 17000 : a.M * a.N >= 24000)));
+    if (a.K <= 2048 && a.N >= (a.M == 2 ? 14336 : a.M == 3 ? 6144 : 4096)) return true;
     return a.N * a.K >= ((int64_t)32 << 20) && a.N >= (a.M >= 4 ? 4096 : 6144);
 }
 

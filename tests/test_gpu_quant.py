@@ -612,8 +612,33 @@ def test_q8_0_rows_on_the_matrix_cores(m, n, k):
     assert np.all(np.abs(got - rows) <= 2e-6 * mag + 1e-30)
 
 
+def test_q8_0_few_rows_captured_on_a_stream_without_scratch():
+    """A product that one launch serves where there is no memory for converted rows: recorded on a stream that has none, as before it went to the matrix cores elsewhere."""
+    l = gpu.lib()
+    rng = np.random.default_rng(8)
+    m, n, k = 8, 4096, 512
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    xd, y = gpu.dev(x), torch.zeros((m, n), device="cuda:0")
+    want = O.qmatmul(O.Q8_0, raw, x, n, k)
+    mag = np.abs(x.astype(np.float64)) @ np.abs(O.dequantize(O.Q8_0, raw).reshape(n, k).astype(np.float64)).T
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    gpu.say("q8_0 few rows captured")
+    with torch.cuda.graph(graph, stream=stream):
+        capi.check(l.mi355x_qgemv(O.Q8_0, ptr, xd.data_ptr(), y.data_ptr(), m, n, k, k, stream.cuda_stream))
+    for _ in range(2):
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.all(np.abs(y.cpu().numpy() - want) <= 2e-6 * mag + 1e-30)
+    again = gpu.qgemv(O.Q8_0, ptr, xd, n, k)  # by the matrix cores
+    assert np.all(np.abs(again - want) <= 2e-6 * mag + 1e-30)
+
+
 @pytest.mark.parametrize("m,n,k,offset", [(9, 4097, 256, 0), (32, 1024, 288, 2), (33, 1000, 4064, 0), (64, 513, 2304, 4), (65, 8200, 480, 2), (520, 70, 992, 0),
-                                          (3, 8193, 4128, 2), (2, 16500, 2080, 0)])
+                                          (3, 8193, 4128, 2), (2, 16500, 2080, 0), (8, 4097, 1056, 0), (7, 2049, 4096, 2), (3, 6145, 288, 0), (9, 64, 256, 0), (9, 1281, 4128, 0),
+                                          (17, 1003, 4096, 0), (12, 2049, 8224, 2)])
 def test_q8_0_products_of_any_rows_on_the_matrix_cores(m, n, k, offset):
     """32 rows of x and 32 of W a workgroup, eight blocks a run: remainders of each, a W on two bytes, four and eight
     wavefronts, on the route that the size selects. The integers are the CPU's; a result's float32 sums pass through

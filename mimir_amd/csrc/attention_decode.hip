@@ -11,8 +11,9 @@
 // Sixteen lanes share a key row, 16 or 32 bytes each, so a wavefront's load
 // covers four whole rows; the sixteen key groups of the workgroup take
 // consecutive keys. Scores go through LDS for the softmax, values are
-// accumulated per key group, summed within a wavefront by exchanges of
-// registers and over the four through LDS. Number of keys, queries, keys and
+// accumulated per key group and summed through LDS, the sixteen groups one
+// after the other: K-quant products round the result to int8, so that another
+// order of sums is another model's logits by some hundredths. Number of keys, queries, keys and
 // values are requested in that order before any of them is waited for (shares
 // are fixed ranges of the cache, rows past the end clamped): one trip to memory.
 // A share's (max, sum, weighted values) reach the combining workgroup one
@@ -32,12 +33,13 @@
 // shares have workgroup indices congruent modulo eight, i.e. they run on one
 // die, and the head's rows and slots stay in that die's L2.
 //
-// What bounds it: a chain of waits, at one wavefront a SIMD. Clock readings of a launch between others that empty the caches, from the first
-// workgroup's start, heads of 128 features, binary16 cache, us: all loaded at 1.2, scores 1.9, softmax 2.3, values 3.4, the shares' put together 5.2, converted and stored 6.7
+// What bounds it: a chain of waits, at one wavefront a SIMD, and where several workgroups share a compute unit the sixteen groups' values through LDS. Clock readings of a launch
+// between others that empty the caches, from the first workgroup's start, heads of 128 features, binary16 cache, us: all loaded at 1.2, scores 1.9, softmax 2.3, values 3.4
 // (one sequence, 576 positions in nine shares). Before, with each head's queries waited for in turn before the keys were requested, sums over
-// lanes and key groups one by one, and the first share's workgroup collecting: 2.5, 3.4, 3.9, 5.5, 8.2, 10.4. Whole launches: 64 positions 6.7 -> 4.4,
-// 128 9.7 -> 6.2, 576 11.0 -> 7.1, eight sequences of 544 15.3 -> 10.8, 2080 15.1 -> 10.8. Eight wavefronts a workgroup, a row of keys fewer each, were no
-// faster (6.4 at 128, 8.5 at 576), so were conversions kept apart from the products (v_fma_mix_f32).
+// lanes one by one, and the first share's workgroup collecting: 2.5, 3.4, 3.9, 5.5. Whole launches by the profiler, us, in the mean of a generation: one sequence of
+// 37 to 101 positions 7.1, 512 to 576 8.6, 2048 to 2080 12.0, eight of 512 to 544 12.9. With a wavefront's four groups summed by exchanges of registers, another order, these took 6.5, 8.0, 11.5
+// and 11.5; in this order wider reads by half the lanes took longer (7.7, 9.4, 13.0, 15.2), values stored a head at a time were level (6.9, 8.6, 12.4, 12.8). Eight wavefronts a workgroup, a row
+// of keys fewer each, were no faster, so were conversions kept apart from the products (v_fma_mix_f32).
 #include <type_traits>
 
 #include "device_util.h"
@@ -69,15 +71,15 @@ struct DecParams {
     int act_rows;  // the converted result in the form for a few rows of x (q4_rows_act.h), all sequences in one buffer
     int act_kq;    // the converted result as int8 super-blocks for Q4_K / Q6_K products (kq_act.h), rows act_row_bytes apart
     int fence;     // 1: the ticket is a release-acquire operation at device scope (the default); 0, 2: measurement aids, see the ticket
-    unsigned long long* flagged;  // not null: shares travel as (value, flag) pairs and the first share's workgroup collects them (no ticket)
+    unsigned long long* flagged;  // not null: shares travel as (value, flag) pairs and the last share's workgroup collects them (no ticket)
     uint32_t* err;                // the device's error word (a hand-over that never completes sets kErrInternal)
 };
 
-// LDS in floats behind the scores: the wavefronts' values, and the results (or, before them, the shares' factors) beside them, so that
-// no wavefront waits for the others' reads before it writes its own.
+// LDS in floats behind the scores: the key groups' values, and the results beside them, so that no wavefront waits for the others'
+// reads before it writes its own.
 template <int D>
-constexpr int kFinal = kThreads / 64 * kHeads * D;
-constexpr int value_floats(int D) { return (kThreads / 64 + 1) * kHeads * D; }
+constexpr int kFinal = kKeyGroups * kHeads * D;
+constexpr int value_floats(int D) { return (kKeyGroups + 1) * kHeads * D; }
 
 // Stores and loads that are coherent across the device on their own.
 __device__ __forceinline__ void coherent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -148,10 +150,10 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                                                                uint32_t* __restrict__ counters, float* __restrict__ out,
                                                                float* __restrict__ lse, uint8_t* __restrict__ act, DecParams p) {
     constexpr int D = 16 * FPL;
-    constexpr int OPL = D / 64;  // results a lane holds of its wavefront's head: features lane + 64 c
+    constexpr int OPL = D / 64;  // results a lane holds of its wavefront's head: features feature0 + 4 c
     extern __shared__ float smem[];
     float* sc = smem;                  // [cmax][4] scores, then weights: a key's four heads next to each other
-    float* osl = sc + kHeads * p.cmax; // [4][4][D] values per wavefront, and the results behind them
+    float* osl = sc + kHeads * p.cmax; // [16][4][D] values per key group, and the results behind them
     __shared__ float red[2 * kHeads];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -239,8 +241,9 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                 lo += dpp_f32<0x4e>(lo);  // quad_perm [2,3,0,1]
                 hi += dpp_f32<0x4e>(hi);
                 t[u] = part & 2 ? hi : lo;    // head part & 3, over the quad
-                t[u] += dpp_f32<0x124>(t[u]);  // row_ror:4
-                t[u] += dpp_f32<0x128>(t[u]);  // row_ror:8
+                // (q0 + q1) + (q2 + q3) of the quads, in quad u, which keeps it: its neighbour's, then the other pair's
+                t[u] += u & 1 ? dpp_f32<0x124>(t[u]) : dpp_f32<0x12c>(t[u]);  // row_ror:4, row_ror:12
+                t[u] += dpp_f32<0x128>(t[u]);                                 // row_ror:8
             }
             const float mine = part & 8 ? (part & 4 ? t[3] : t[2]) : (part & 4 ? t[1] : t[0]);
             const int jj = jj0 + kKeyGroups * (u0 + (part >> 2)) + kg;
@@ -304,29 +307,24 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
                 for (int f = 0; f < FPL; f++) o[g][f] = fmaf(pj[g], vf[f], o[g][f]);
         }
     }
-    // the wavefront's four key groups: exchanges of half the registers each leave row r of sixteen lanes with head r, FPL features a lane
+    // Features 4 c .. + 3 of each lane's are 64 c .. of a row in LDS, so that a wavefront's stores fall on all banks
 #pragma unroll
-    for (int f = 0; f < FPL; f++) {
-        swap_halves(o[0][f], o[2][f]);
-        swap_halves(o[1][f], o[3][f]);
-        float even = o[0][f] + o[2][f], odd = o[1][f] + o[3][f];
-        swap_rows(even, odd);
-        o[0][f] = even + odd;
-    }
+    for (int g = 0; g < kHeads; g++)
 #pragma unroll
-    for (int f = 0; f < FPL; f += 4) {
-        const f32x4 v = {o[0][f], o[0][f + 1], o[0][f + 2], o[0][f + 3]};
-        *(f32x4*)(osl + (wave * kHeads + (lane >> 4)) * D + part * FPL + f) = v;
-    }
+        for (int f = 0; f < FPL; f += 4) {
+            const f32x4 v = {o[g][f], o[g][f + 1], o[g][f + 2], o[g][f + 3]};
+            *(f32x4*)(osl + (kg * kHeads + g) * D + 16 * f + 4 * part) = v;
+        }
     __syncthreads();
     const int g = wave, h = hk * G + g0 + g;  // wavefront g now holds head g
     const bool mine = g < ng;
+    const int feature0 = FPL * (lane >> 2) + (lane & 3);
     float r[OPL], M = red[g], L = red[kHeads + g];
 #pragma unroll
-    for (int c = 0; c < OPL; c++) {
+    for (int c = 0; c < OPL; c++) {  // the key groups one after the other, whatever wavefront they are of
         r[c] = 0.f;
 #pragma unroll
-        for (int w = 0; w < kThreads / 64; w++) r[c] += osl[(w * kHeads + g) * D + lane + 64 * c];
+        for (int x = 0; x < kKeyGroups; x++) r[c] += osl[(x * kHeads + g) * D + lane + 64 * c];
     }
 
     if (nsplit > 1 && p.flagged) {
@@ -502,8 +500,9 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const float* __re
 #pragma unroll
     for (int c = 0; c < OPL; c++) {
         const float val = L == 0.f ? 0.f : r[c] * inv;
-        if (mine && out) out[b * p.o_b + (int64_t)h * p.o_h + lane + 64 * c] = val;
-        if (act) fin[g * D + lane + 64 * c] = mine ? val : 0.f;
+        const int feature = feature0 + 4 * c;
+        if (mine && out) out[b * p.o_b + (int64_t)h * p.o_h + feature] = val;
+        if (act) fin[g * D + feature] = mine ? val : 0.f;
     }
     if (mine && lse && lane == 0) lse[(int64_t)b * p.H + h] = L == 0.f ? -__builtin_inff() : M + __builtin_logf(L);
     if (!act) return;
@@ -589,7 +588,7 @@ bool attention_decode_ok(const AttnArgs& a, int64_t kmax) {
     if (((uintptr_t)a.k | (uintptr_t)a.v) % row_align || (uintptr_t)a.q % 16 || a.q_strides[0] % 4 || a.q_strides[1] % 4) return false;
     int ns, cm;
     attention_decode_plan(a.B, a.H, a.HK, kmax, &ns, &cm);
-    size_t lds = (size_t)(kHeads * cm + value_floats(a.D)) * sizeof(float);
+    const size_t lds = (size_t)(kHeads * cm + kKeyGroups * kHeads * a.D) * sizeof(float);  // and two kilobytes at most for the results
     if (a.k_strides[2] <= 0 || a.v_strides[2] <= 0 || a.k_strides[2] >= (1 << 23) || a.v_strides[2] >= (1 << 23) || kmax >= (1 << 23) ||
         kmax * a.k_strides[2] >= ((int64_t)1 << 31) || kmax * a.v_strides[2] >= ((int64_t)1 << 31))
         return false;

@@ -171,6 +171,56 @@ def attention(q, k, v, scale, causal=False, offset=0, kv_dt=capi.F32, k_len=None
     return out.cpu().numpy(), lse.cpu().numpy()
 
 
+def _chain(start, terms):
+    """float32 sums one after the other, each term exact in float64."""
+    s = start
+    for t in terms:
+        s = (s.astype(np.float64) + t).astype(np.float32)
+    return s
+
+
+@pytest.mark.parametrize("handover", [0, 1])
+@pytest.mark.parametrize("D,kv_dt,K,shares", [(128, capi.F16, 37, 1), (128, capi.F16, 100, 2), (128, capi.F32, 64, 1), (64, capi.F16, 300, 3), (64, capi.F32, 200, 7)])
+def test_decode_attention_adds_in_a_fixed_order(D, kv_dt, K, shares, handover):
+    """One query position, bit for bit: int8 products that read the result make steps of its last bits. Scores: a lane's D / 16 features as a chain, then (q0 + q1) + (q2 + q3)
+    of the quads' (l0 + l1) + (l2 + l3); seen alone in the logsumexp where all other keys' weights underflow. Values under equal weights of one: keys 16 apart as a
+    chain, the sixteen chains one after the other, then the shares."""
+    rng = np.random.default_rng(D + K)
+    l = gpu.lib()
+    rounded = lambda a: a.astype(np.float16).astype(np.float32)
+    store = lambda a: O.f32_to_f16(a) if kv_dt == capi.F16 else a
+    H, HK = 6, 2
+    try:
+        capi.check(l.mi355x_tune(b"attention.splits", shares))
+        capi.check(l.mi355x_tune(b"attention.handover", handover))
+        # scores: sequence b sees its key b alone, the others' products are below -1000
+        q = rng.normal(size=(K, H, 1, D)).astype(np.float32)
+        q[..., 0] = 8
+        k = rounded(rng.normal(size=(K, HK, K, D)).astype(np.float32))
+        k[..., 0] = -1000
+        k[np.arange(K), :, np.arange(K), 0] = rounded(rng.normal(size=(K, HK)).astype(np.float32))
+        gpu.say(f"attention order D={D} dt={kv_dt} K={K} shares={shares} handover={handover}")
+        _, lse = attention(q, store(k), store(np.zeros_like(k)), 1.0, kv_dt=kv_dt)
+        own = np.repeat(k[np.arange(K), :, np.arange(K)], H // HK, axis=1)  # [K, H, D]
+        exact = (q[:, :, 0].astype(np.float64) * own).reshape(K, H, 16, D // 16)
+        lanes = _chain(np.zeros((K, H, 16), np.float32), [exact[..., f] for f in range(D // 16)])
+        quads = lanes.reshape(K, H, 4, 4)
+        quads = (quads[..., 0] + quads[..., 1]) + (quads[..., 2] + quads[..., 3])
+        assert bits_equal(lse[:, :, 0], (quads[..., 0] + quads[..., 1]) + (quads[..., 2] + quads[..., 3]))
+        # values: keys of nought weigh the same
+        v = rounded((rng.normal(size=(3, HK, K, D)) * np.exp(rng.normal(size=(3, HK, K, 1)))).astype(np.float32))
+        out, lse = attention(rng.normal(size=(3, H, 1, D)).astype(np.float32), store(np.zeros_like(v)), store(v), 1.0, kv_dt=kv_dt)
+        total, each = np.zeros((3, HK, D), np.float32), -(-K // shares)
+        for s in range(shares):
+            part = v[:, :, s * each:(s + 1) * each].astype(np.float64)
+            groups = [_chain(np.zeros((3, HK, D), np.float32), [part[:, :, j] for j in range(x, part.shape[2], 16)]) for x in range(16)]
+            total = _chain(total, [_chain(np.zeros((3, HK, D), np.float32), groups)])
+        assert bits_equal(out[:, :, 0], np.repeat(total * (np.float32(1) / np.float32(K)), H // HK, axis=1))
+    finally:
+        capi.check(l.mi355x_tune(b"attention.splits", 0))
+        capi.check(l.mi355x_tune(b"attention.handover", 0))
+
+
 def test_attention_golden_mask(cases):
     """The reference's masked case (nn/transformer_test.go:36-38): an additive float mask as In[3]."""
     c = cases["sdpa_mask"]

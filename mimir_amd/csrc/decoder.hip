@@ -94,7 +94,7 @@ mi355x_status Decoder::logits_at(const int32_t* tokens, int64_t n, const int64_t
 }
 
 // One token a sequence, as the next decoding step that it is: a step's launches are fewer and fused where forward() has one for every operator and
-// row (a layer of one Q4_0 row is 5 launches for 16, of eight rows 8 for 16 whose products read W eight times). Replayed where generate has recorded it;
+// row (a layer of one Q4_0 row is 5 launches for 16). Replayed where generate has recorded it;
 // the choice that a recorded step ends in goes to `record` and `next_tok`, which the next caller sets anew.
 mi355x_status Decoder::step_logits(const int32_t* tokens, const int64_t* want, int64_t n_want, float* logits_host) {
     DECODER_HIP(hipMemcpyAsync(next_tok.p, tokens, (size_t)batch * 4, hipMemcpyHostToDevice, stream), name, "upload tokens");

@@ -90,9 +90,11 @@ struct Model : Decoder {
     int step_variant() const override;
     bool few_fit = false;  // a rows model of so few sequences that step_few takes it
     bool few() const;
-    // A step of Q4_0 linears is some 5 launches a block, 8 of several sequences, that read W once for eight of them; forward(1) has 16, of a row at a time: 300 us
-    // a call against 520 (four blocks of 4096 features), 8 sequences 500 against 1000. Blocks of other dtypes and the stacks are within 1 % either way. Measured up to 16 sequences.
-    bool one_token_as_step() const override { return fast && c.batch <= 16; }
+    // A step of Q4_0 linears of one or two sequences is five or six launches a block where forward(1) has 16, of a row at a time: 300 us a call against 520 (one sequence, four blocks of
+    // 4096 features), by products that have the one-row kernel's integers. Of more sequences the step's rows kernel adds in two shares of K; its logits are as far from 64 bits in the mean
+    // (forty models each of 1024, 2048 and 4096 features and one, two and eight sequences: 0.90 to 1.02 of the others' error), but not the ones that a sequence alone has, and a Q8_0 head
+    // makes a step of its int8 rounding of a difference: those keep forward's kernels. Blocks of other dtypes and the stacks are within 1 % either way.
+    bool one_token_as_step() const override { return fast && (c.batch == 1 || few()); }
 };
 
 constexpr int kFewSequences = 2;  // of more the step with kernels for eight is level or faster (qgemv_q4_0_few.hip)

@@ -291,9 +291,9 @@ def test_fused_and_graph_replayed_steps_choose_the_per_operator_tokens(batch, ca
     assert all(same), (runs[2][0], runs[0][0])
 
 
-@pytest.mark.parametrize("batch,output_dt", [(1, O.Q4_0), (5, O.Q4_0), (16, O.Q8_0), (17, O.Q4_0)])
+@pytest.mark.parametrize("batch,output_dt", [(1, O.Q4_0), (2, O.Q4_0), (5, O.Q4_0), (16, O.Q8_0), (17, O.Q4_0)])
 def test_logits_of_one_token_as_a_decoding_step(batch, output_dt):
-    """One token a sequence goes through the decoding step's launches (of up to sixteen sequences), one by one before a generation
+    """One token a sequence goes through the decoding step's launches (of one and two sequences; of more through the operators'), one by one before a generation
     has recorded them and replayed after it, from an empty cache too, and leaves cache and logits as the per-operator pass does. A product is
     within 2e-7 of the float32 one either way and a model has some tens: 1e-5 of the largest logit; a Q8_0 head rounds x to a 127th of a block's largest (0.02)."""
     lib = gpu.lib()
@@ -327,6 +327,33 @@ def test_logits_of_one_token_as_a_decoding_step(batch, output_dt):
     assert all(np.array_equal(a, b) for a, b in zip(runs["launches"], runs["replayed"]))
     with pytest.raises(RuntimeError):
         m.logits_at(one, [batch])
+
+
+@pytest.mark.parametrize("batch,output_dt", [(3, O.Q8_0), (8, O.Q8_0), (16, O.Q4_0)])
+def test_logits_of_one_token_of_several_sequences_are_the_operators(batch, output_dt):
+    """Bit for bit: a Q8_0 head's rounding of x makes a step of any difference before it. With a recorded step at hand and without."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    om = OL.synthetic(_oracle_config(c), seed=4, output_dt=output_dt)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(16)
+    rng = np.random.default_rng(batch)
+    prompts, one = rng.integers(0, c.vocab, (batch, 9)), rng.integers(0, c.vocab, (batch, 1))
+    runs = []
+    try:
+        for mode, recorded in ((2, False), (0, False), (0, True)):
+            gpu.say(f"one token of {batch} sequences, step mode {mode}")
+            capi.check(lib.mi355x_tune(b"llama.step", mode))
+            if recorded:
+                m.generate(prompts, 3)
+            m.reset()
+            m.logits(prompts)
+            runs.append([m.logits(one), m.logits(one)])
+    finally:
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    for got in runs[1:]:
+        assert all(np.array_equal(g.view(np.uint32), w.view(np.uint32)) for g, w in zip(got, runs[0]))
 
 
 @pytest.mark.parametrize("embed,batch", [(4160, 1), (8192, 1), (8192, 2)])

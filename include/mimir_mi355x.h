@@ -509,6 +509,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * "kquant.stream" = 1 keeps products of one row of x off the kernel with a
  * workgroup per compute unit, 4 to 16 sends all it takes there, with that many
  * wavefronts a workgroup (0: by shape).
+ * "argmax.spins" = n has the workgroup that chooses a row's index poll n times for
+ * the others' candidates before it looks over the row itself (below 0: as often as
+ * it was, some tenths of a second).
  * "qgemm.path" = 1 makes mi355x_qgemm_bf16 take its general route for every shape.
  * "qgemm.f16" = 1 makes mi355x_qgemm_bf16's Q4_0 matrix-core kernel round every
  * weight once to binary16 instead of multiplying it exactly (each weight within

@@ -700,7 +700,7 @@ mi355x_status mi355x_argmax(const float* logits, int64_t rows, int64_t n, int32_
     void* ws = nullptr;
     if (rows <= 1024)
         if (mi355x_status st = argmax_scratch(stream, mimir::argmax_workspace_bytes(1024), &ws)) return st;
-    HIP_TRY(mimir::argmax(logits, rows, n, out, ws, mimir::device_error_word(), (hipStream_t)stream), "launch argmax");
+    HIP_TRY(mimir::argmax(logits, rows, n, out, ws, (hipStream_t)stream), "launch argmax");
     return MI355X_OK;
 }
 
@@ -734,6 +734,10 @@ mi355x_status mi355x_tune(const char* key, int value) {
         }
     if (key && (strcmp(key, "kquant.rows") == 0 || strcmp(key, "kquant.path") == 0)) {
         mimir::set_kquant_tune(key[7] == 'p', value);
+        return MI355X_OK;
+    }
+    if (key && strcmp(key, "argmax.spins") == 0) {
+        mimir::set_argmax_spins(value);
         return MI355X_OK;
     }
     if (key && strcmp(key, "q4_0.few") == 0) {

@@ -469,8 +469,8 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ 
 }
 
 // The same over many workgroups per row: each scans a span of the row and
-// leaves its candidate; the row's last one picks among them. slots: a zeroed
-// word per candidate, which the last workgroup zeroes again.
+// leaves its candidate; the row's last one picks among them. slots: 64 words a
+// row, zeroed; the last workgroup zeroes the candidates' again.
 constexpr int kArgmaxBlocks = 64;  // at most, per row
 
 __device__ __forceinline__ void argmax_better(float& best, int& at, float v, int i) {
@@ -486,16 +486,32 @@ __device__ __forceinline__ void wave_argmax(float& best, int& at) {
     best = top;
 }
 
-constexpr int kArgmaxSpins = 1 << 18;  // polls of a row's candidates before the workgroup that chooses gives up (some tenths of a second)
+// The best of row[lo, hi) among threads t, t + step, ...: eight loads under way a thread.
+__device__ __forceinline__ void scan_span(const float* __restrict__ row, int64_t lo, int64_t hi, int t, int step, float& best, int& at) {
+    for (int64_t i0 = lo + t; i0 < hi; i0 += 8 * step) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = row[i0 + step * u < hi ? i0 + step * u : hi - 1];
+#pragma unroll
+        for (int u = 0; u < 8; u++) argmax_better(best, at, v[u], (int)(i0 + step * u < hi ? i0 + step * u : hi - 1));
+    }
+}
+
+// Polls of a row's candidates before the workgroup that chooses looks for itself (some tenths of a second). "argmax.spins"
+constexpr int kArgmaxSpins = 1 << 18;
+static std::atomic<int> g_argmax_spins{kArgmaxSpins};
+void set_argmax_spins(int n) { g_argmax_spins = n < 0 ? kArgmaxSpins : n; }
 
 // The candidates travel as one 8-byte word each, stored and loaded whole at device scope: the value, and the index plus one, which says that
 // it is there. A row's last workgroup keeps its own and polls for the others', which start before it and wait for nothing; it empties the slots for the next launch.
+// Where one does not arrive in time it looks over the row by itself. That candidate still comes, into a slot that the next launch would take for its own, so the
+// row's last slot, which no candidate has, says from then on that its slots are not to be used.
 // TAIL: it also does what follows the choice (ChooseTail); as launches of their own the bookkeeping and the embedding of a decoding step took 4.0 and 4.6 us.
 // All latency. A step's choice among 32768 logits, us by the profiler: 7.2 with candidates stored, waited for and counted by a release-acquire ticket, the
 // wavefronts' best by twelve exchanges through the LDS crossbar each, row[0] and the state read where they are used; now 4.0 (eight rows 8.4 -> 5.5).
 template <bool TAIL>
 __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restrict__ logits, int64_t n, int span, int32_t* __restrict__ out,
-                                                           unsigned long long* __restrict__ slots, uint32_t* err, const ChooseTail tail) {
+                                                           unsigned long long* __restrict__ slots, int spins, const ChooseTail tail) {
     __shared__ float bv[4];
     __shared__ int bi[4];
     __shared__ int s_token;
@@ -503,17 +519,13 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
     const float* row = logits + (int64_t)r * n;
     const int64_t lo = (int64_t)blockIdx.x * span, hi = lo + span < n ? lo + span : n;
     const float first = row[0];
+    unsigned long long* slot = slots + (int64_t)r * kArgmaxBlocks;
+    const unsigned long long spoilt = __hip_atomic_load(slot + kArgmaxBlocks - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int32_t pos = 0, step = 0;
     if (TAIL) pos = tail.state[0], step = tail.state[1];  // read before this row is counted, moved on behind the last row that is
     float best = -__builtin_inff();
     int at = 0x7fffffff;
-    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += 8 * 256) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = row[i0 + 256 * u < hi ? i0 + 256 * u : hi - 1];
-#pragma unroll
-        for (int u = 0; u < 8; u++) argmax_better(best, at, v[u], (int)(i0 + 256 * u < hi ? i0 + 256 * u : hi - 1));
-    }
+    scan_span(row, lo, hi, threadIdx.x, 256, best, at);
     wave_argmax(best, at);
     if (lane == 0) {
         bv[threadIdx.x >> 6] = best;
@@ -526,17 +538,23 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
         best = bv[0], at = bi[0];
 #pragma unroll
         for (int w = 1; w < 4; w++) argmax_better(best, at, bv[w], bi[w]);
-        unsigned long long* slot = slots + (int64_t)r * kArgmaxBlocks;
         if (!last) {
-            __hip_atomic_store(slot + blockIdx.x, (unsigned long long)__float_as_uint(best) << 32 | ((uint32_t)at + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!spoilt) __hip_atomic_store(slot + blockIdx.x, (unsigned long long)__float_as_uint(best) << 32 | ((uint32_t)at + 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
+        bool there = true;
         if (lane < nblk - 1) {  // nblk is at most 64
             unsigned long long c = 0;
-            for (int spin = 0; c == 0 && spin < kArgmaxSpins; spin++) c = __hip_atomic_load(slot + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(slot + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (c == 0) atomicOr(err, kErrInternal);
-            else argmax_better(best, at, __uint_as_float((uint32_t)(c >> 32)), (int)((uint32_t)c - 1u));
+            if (!spoilt) {
+                for (int spin = 0; c == 0 && spin < spins; spin++) c = __hip_atomic_load(slot + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(slot + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            there = c != 0;
+            if (there) argmax_better(best, at, __uint_as_float((uint32_t)(c >> 32)), (int)((uint32_t)c - 1u));
+        }
+        if (!__all(there)) {
+            if (lane == 0) __hip_atomic_store(slot + kArgmaxBlocks - 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            scan_span(row, 0, n, lane, 64, best, at);
         }
         wave_argmax(best, at);
         if (first != first || at == 0x7fffffff) at = 0;  // NaN at 0, or nothing but NaNs
@@ -591,35 +609,36 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
 size_t argmax_workspace_bytes(int64_t rows) { return (size_t)rows * kArgmaxBlocks * 8; }
 
 // Workgroups of 2048 values, one round of eight loads a thread, up to 64 a row (one lane each in the last step).
-static void argmax_split(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail* tail, uint32_t* err, hipStream_t st) {
+static void argmax_split(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail* tail, hipStream_t st) {
     int64_t nblk = (n + 2047) / 2048;
     nblk = nblk > kArgmaxBlocks ? kArgmaxBlocks : nblk;
     int64_t span = ((n + nblk - 1) / nblk + 255) / 256 * 256;
     nblk = (n + span - 1) / span;
+    const int spins = g_argmax_spins.load(std::memory_order_relaxed);
     if (tail)
         hipLaunchKernelGGL(argmax_split_kernel<true>, dim3((unsigned)nblk, (unsigned)rows), dim3(256), 0, st, logits, n, (int)span, out,
-                           (unsigned long long*)workspace, err, *tail);
+                           (unsigned long long*)workspace, spins, *tail);
     else
         hipLaunchKernelGGL(argmax_split_kernel<false>, dim3((unsigned)nblk, (unsigned)rows), dim3(256), 0, st, logits, n, (int)span, out,
-                           (unsigned long long*)workspace, err, ChooseTail{});
+                           (unsigned long long*)workspace, spins, ChooseTail{});
 }
 
 // workspace: argmax_workspace_bytes(rows) bytes that were zero before the first
 // launch, or null for the one-workgroup kernel.
-hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, uint32_t* err, hipStream_t st) {
+hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, hipStream_t st) {
     if (rows == 0) return hipSuccess;
     if (!argmax_choose_ok(rows, n, workspace)) {
         hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)rows), dim3(1024), 0, st, logits, n, out);
         return hipGetLastError();
     }
-    argmax_split(logits, rows, n, out, workspace, nullptr, err, st);
+    argmax_split(logits, rows, n, out, workspace, nullptr, st);
     return hipGetLastError();
 }
 
 bool argmax_choose_ok(int64_t rows, int64_t n, const void* workspace) { return workspace && rows > 0 && rows <= kArgmaxRows && n >= 8192; }
 
-hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, uint32_t* err, hipStream_t st) {
-    argmax_split(logits, rows, n, out, workspace, &tail, err, st);
+hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, hipStream_t st) {
+    argmax_split(logits, rows, n, out, workspace, &tail, st);
     return hipGetLastError();
 }
 

@@ -162,7 +162,7 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
     auto choose = [&](int32_t* out, int64_t s) -> mi355x_status {  // from the last row of every sequence of a pass of s tokens
         for (int64_t b = 0; b < B; b++) last[b] = b * s + s - 1;
         if (mi355x_status s2 = head(last.data(), B)) return s2;
-        return hip(argmax(logits.as<float>(), B, vocab, out, argmax_ws.p, device_error_word(), stream), "argmax");
+        return hip(argmax(logits.as<float>(), B, vocab, out, argmax_ws.p, stream), "argmax");
     };
     int32_t* picked = record.as<int32_t>();  // [n_new, batch]
     if (!st) st = choose(use_fast ? next_tok.as<int32_t>() : picked, last_s);
@@ -179,8 +179,8 @@ mi355x_status Decoder::generate(const int32_t* prompt, int64_t n_prompt, int64_t
             if (!embedded)
                 if (mi355x_status s2 = embed_next()) return s2;
             if (mi355x_status s2 = step()) return s2;
-            if (chosen) return hip(argmax_choose(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, tail, device_error_word(), stream), "choice");
-            if (mi355x_status s2 = hip(argmax(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, device_error_word(), stream), "argmax")) return s2;
+            if (chosen) return hip(argmax_choose(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, tail, stream), "choice");
+            if (mi355x_status s2 = hip(argmax(logits.as<float>(), B, vocab, next_tok.as<int32_t>(), argmax_ws.p, stream), "argmax")) return s2;
             return hip(advance(state.as<int32_t>(), next_tok.as<int32_t>(), record.as<int32_t>(), (int)B, 1, stream), "advance");
         };
         if (step_graph && graph_variant != step_variant()) {  // a measurement aid changed which step runs

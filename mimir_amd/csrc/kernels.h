@@ -264,13 +264,14 @@ hipError_t swiglu(const float* g, const float* u, float* out, int64_t rows, int6
 hipError_t add(const float* a, const float* b, float* out, int64_t n, hipStream_t st);
 hipError_t add_bias(float* y, const float* bias, int64_t rows, int64_t n, hipStream_t st);  // y[r, :] += bias
 // workspace: argmax_workspace_bytes(rows) bytes, zero before the first launch (they restore themselves), of at most kArgmaxRows rows, or null for
-// one workgroup a row. err: the device's error word (candidates that never arrive set kErrInternal).
+// one workgroup a row.
 constexpr int64_t kArgmaxRows = 1024;
 size_t argmax_workspace_bytes(int64_t rows);
-hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, uint32_t* err, hipStream_t st);
+hipError_t argmax(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, hipStream_t st);
+void set_argmax_spins(int n);  // measurement aid: polls before a row's last workgroup looks for itself; below 0: as many as it was
 // argmax and its tail in one launch (the workspace is needed); whether it takes rows of n.
 bool argmax_choose_ok(int64_t rows, int64_t n, const void* workspace);
-hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, uint32_t* err, hipStream_t st);
+hipError_t argmax_choose(const float* logits, int64_t rows, int64_t n, int32_t* out, void* workspace, const ChooseTail& tail, hipStream_t st);
 
 // Attention of queries [B, H, Q, D] over keys and values [B, HK, K, D], each
 // read through strides {batch, head, position} (features contiguous). chunk

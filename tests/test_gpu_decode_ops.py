@@ -502,6 +502,33 @@ def test_swiglu_add_argmax():
     assert idx.cpu().tolist()[:2] == [0, 0]
 
 
+@pytest.mark.parametrize("rows,n", [(1, 8192), (3, 32768), (2, 300007)])
+def test_a_choice_without_its_candidates_looks_for_itself(rows, n):
+    """A row's last workgroup that gives up on the others' candidates scans the row, and what they leave behind is no later call's: with no polls at all, then with as many
+    as ever on the same workspace, other logits each time. No call fails, and a stream of its own is not slowed down."""
+    l = gpu.lib()
+    rng = np.random.default_rng(n)
+    stream = torch.cuda.Stream()
+    idx = torch.full((rows,), -1, dtype=torch.int32, device="cuda:0")
+    data = [rng.normal(size=(rows, n)).astype(np.float32) for _ in range(5)]
+    for i, d in enumerate(data):
+        d[:, 17 + i] = 9 - i  # the largest of each call below that of the one before
+    data[1][0, n - 1] = data[1][0, 18] = 8.5
+    data[2][rows - 1, 0] = np.nan
+    try:
+        for spins, d in zip((0, -1, 0, -1, -1), data):
+            capi.check(l.mi355x_tune(b"argmax.spins", spins))
+            gpu.say(f"argmax {rows} x {n} spins={spins}")
+            dd = gpu.dev(d)
+            torch.cuda.synchronize()
+            capi.check(l.mi355x_argmax(dd.data_ptr(), rows, n, idx.data_ptr(), stream.cuda_stream))
+            capi.check(l.mi355x_sync(stream.cuda_stream))
+            assert idx.cpu().tolist() == [O.argmax(r) for r in d]
+    finally:
+        capi.check(l.mi355x_tune(b"argmax.spins", -1))
+        capi.check(l.mi355x_stream_release(stream.cuda_stream))
+
+
 @pytest.mark.parametrize("K,off", [(64, 20), (256, 254), (288, 100), (8192, 8190), (8224, 8222), (8224, -1)])
 def test_shares_of_the_keys_are_put_together(K, off):
     """Two query positions over shares of 32 keys: 2, 8, 9, 256 and 257 of them (eight are read ahead, 256 are a round of the threads), some or all of them

@@ -557,6 +557,33 @@ def test_the_choice_brings_in_the_next_embedding(embed, vocab, batch):
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
 
 
+@pytest.mark.parametrize("batch", [1, 3])
+def test_a_generation_whose_choices_give_up_on_their_candidates(batch):
+    """With no polls, recorded so, and with as many as ever on the same workspace: the same tokens."""
+    lib = gpu.lib()
+    c = _small_q4_config(batch, capi.F16)
+    c.vocab, c.context = 9000, 32
+    om = OL.synthetic(_oracle_config(c), seed=3, output_dt=O.Q8_0)
+    prompts = np.random.default_rng(23).integers(0, c.vocab, (batch, 5))
+    runs = []
+    try:
+        for spins in ((-1,), (0, -1)):
+            m = Llama(c)
+            _upload_synthetic(m, om)
+            m.finalize(16)
+            for n in spins:
+                capi.check(lib.mi355x_tune(b"argmax.spins", n))
+                capi.check(lib.mi355x_tune(b"llama.step", 1 if n < 0 else 0))
+                gpu.say(f"generation of {batch}, argmax.spins {n}")
+                m.reset()
+                runs.append(m.generate(prompts, 12)[0])
+            m.close()
+    finally:
+        capi.check(lib.mi355x_tune(b"argmax.spins", -1))
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+
+
 @pytest.mark.parametrize("linear_dt,batch", [(O.Q4_K, 1), (O.Q6_K, 1), (O.Q4_K, 2), (O.Q6_K, 3)])
 def test_kquant_steps_with_norms_and_swiglu_in_the_products_have_the_bits_of_those_without(linear_dt, batch):
     """One to three sequences: the norms and SwiGLU as parts of the products (rows of three super-blocks, 1280 results) against launches of their own."""

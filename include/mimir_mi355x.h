@@ -106,8 +106,9 @@ MI355X_API mi355x_status mi355x_stream_release(void* stream);
  * x by Q4_0 or by a small Q8_0, Q4_K or Q6_K matrix; Q8_0 weights are read
  * once for up to eight rows) or kernels on the int8 matrix cores (Q4_0 from two
  * rows on: up to some tens of rows a kernel that reads W once per eight rows,
- * beyond them a tiled one; Q8_0 from two rows on by a large matrix, from nine on
- * by all but the smallest, W read once for eight or for 32 rows; Q4_K, Q6_K
+ * beyond them a tiled one; Q8_0 from two rows on by a large matrix or by many
+ * rows of W of at most 2048, from nine on by all but the smallest, W read once
+ * for eight or for 32 rows; Q4_K, Q6_K
  * from enough rows on), on the bfloat16 ones (Q4_0 from five rows on where rows
  * of W are an odd number of blocks or W is on two bytes: a float32 x as the sum of
  * three bfloat16, W and x read where they lie and no scratch) or, for other Q4_0,
@@ -119,7 +120,9 @@ MI355X_API mi355x_status mi355x_stream_release(void* stream);
  * additions (Q4_0, Q8_0) and, for Q4_0, by how x is held (fixed point per block,
  * or pairs of binary16: either within the bound below; or exactly), or not at all (Q8_0 among
  * its row kernels, Q4_K, Q6_K). The choice depends on the sizes, the
- * alignment of W and x, and mi355x_tune alone. */
+ * alignment of W and x, and mi355x_tune alone, under capture too (two to eight
+ * rows by a Q8_0 matrix of up to 24 M weights, which need no scratch by the row
+ * kernels, have theirs allocated there, or take those if there is no memory). */
 MI355X_API mi355x_status mi355x_qgemv(int dtype, const void* W, const float* x, float* y, int64_t M, int64_t N, int64_t K,
                            int64_t x_row_stride, void* stream);
 

@@ -95,19 +95,18 @@ mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, s
     return MI355X_OK;
 }
 
-// Whether act_scratch(stream, bytes) would not have to grow a block under capture.
-bool act_at_hand(void* stream, size_t bytes) {
-    DeviceState* s;
-    if (current_state(&s) != MI355X_OK) return false;
-    std::lock_guard<std::mutex> lock(g_mu);
-    if (s->scratch[stream].act.bytes >= bytes) return true;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) (void)hipGetLastError();
-    return capture == hipStreamCaptureStatusNone;
-}
-
 mi355x_status act_scratch(void* stream, size_t bytes, void** out, size_t wish = 0) {
     return stream_scratch(stream, &StreamScratch::act, bytes, wish, kActFloorBytes, 0, "activation", out);
+}
+// The stream's block for a product that has a form without one: allocated under capture too (the thread's calls are relaxed meanwhile), so that the form
+// depends on no earlier call. False: there is no memory.
+bool act_always(void* stream, size_t bytes, void** out) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const mi355x_status st = act_scratch(stream, bytes, out);
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (st) (void)hipGetLastError();  // which the next launch's check would report
+    return st == MI355X_OK;
 }
 // Where a product's converted activations go: the stream's growing block, or a fixed block of
 // kNoallocScratchBytes (then nothing is allocated, and activations of more than kNoallocActBytes are an error).
@@ -391,15 +390,16 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
         // ones that many workgroups' rounding costs more than a conversion launch of its own (measured).
         mimir::QGemvArgs converted = a;
         converted.act = (void*)256;
-        bool matrix = g_rows_path != 1 && mimir::qgemv_q8_0_mfma_pays(converted);  // a large matrix or many rows: the int8 matrix cores
+        bool matrix = g_rows_path != 1 && mimir::qgemv_q8_0_mfma_pays(converted);  // a large matrix, short rows of W or many rows: the int8 matrix cores
         const bool in_product = M <= kConvertInProductRows && N * K <= (int64_t)24 << 20 && ((uintptr_t)x & 15) == 0 && (M == 1 || x_row_stride % 4 == 0);
-        if (matrix && in_product && !src.fixed) matrix = act_at_hand(stream, mimir::q8_act_bytes(K) * (size_t)M);  // which the one launch does without
+        void* act = nullptr;
+        if (matrix && in_product && !src.fixed) matrix = act_always(stream, mimir::q8_act_bytes(K) * (size_t)M, &act);
         if (!matrix && in_product) {
             HIP_TRY(mimir::qgemv_q8_0_act(a, g_tune_q4, (hipStream_t)stream), "launch qgemv_q8_0");
             return MI355X_OK;
         }
-        void* act;
-        if (mi355x_status st = act_for(src, mimir::q8_act_bytes(K) * (size_t)M, &act)) return st;
+        if (!act)
+            if (mi355x_status st = act_for(src, mimir::q8_act_bytes(K) * (size_t)M, &act)) return st;
         HIP_TRY(mimir::q8_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch q8_convert_act");
         a.act = act;
         if (matrix) {

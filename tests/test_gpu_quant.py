@@ -636,6 +636,43 @@ def test_q8_0_few_rows_captured_on_a_stream_without_scratch():
     assert np.all(np.abs(again - want) <= 2e-6 * mag + 1e-30)
 
 
+@pytest.mark.parametrize("m,n,k", [(8, 4096, 512), (2, 14336, 256), (5, 5000, 2048)])
+def test_q8_0_few_rows_are_the_same_product_whatever_the_stream_holds(m, n, k):
+    """Bits eager on a stream of some history, eager on a new one, and recorded first on another new one (a graph keeps the kernels it was recorded with); the product by
+    mi355x_qgemv_noalloc too."""
+    l = gpu.lib()
+    rng = np.random.default_rng(k)
+    raw = random_blocks(rng, O.Q8_0, n * k)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    xd, y = gpu.dev(rng.normal(size=(m, k)).astype(np.float32)), torch.empty((m, n), device="cuda:0")
+    want = gpu.qgemv(O.Q8_0, ptr, xd, n, k)
+
+    def got():
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+    gpu.say(f"q8_0 {m} x {n} x {k} on new streams")
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    try:
+        for s in streams:
+            capi.check(l.mi355x_stream_release(s.cuda_stream))  # torch hands streams out again
+        capi.check(l.mi355x_qgemv(O.Q8_0, ptr, xd.data_ptr(), y.data_ptr(), m, n, k, k, streams[0].cuda_stream))
+        assert bits_equal(got(), want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=streams[1]):
+            capi.check(l.mi355x_qgemv(O.Q8_0, ptr, xd.data_ptr(), y.data_ptr(), m, n, k, k, streams[1].cuda_stream))
+        for _ in range(3):
+            y.fill_(float("nan"))
+            graph.replay()
+            assert bits_equal(got(), want)
+        y.fill_(float("nan"))
+        capi.check(l.mi355x_qgemv_noalloc(O.Q8_0, ptr, xd.data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream()))
+        assert bits_equal(got(), want)
+    finally:
+        graph = None
+        for s in streams:
+            capi.check(l.mi355x_stream_release(s.cuda_stream))
+
+
 @pytest.mark.parametrize("m,n,k,offset", [(9, 4097, 256, 0), (32, 1024, 288, 2), (33, 1000, 4064, 0), (64, 513, 2304, 4), (65, 8200, 480, 2), (520, 70, 992, 0),
                                           (3, 8193, 4128, 2), (2, 16500, 2080, 0), (8, 4097, 1056, 0), (7, 2049, 4096, 2), (3, 6145, 288, 0), (9, 64, 256, 0), (9, 1281, 4128, 0),
                                           (17, 1003, 4096, 0), (12, 2049, 8224, 2)])

@@ -108,6 +108,21 @@ bool act_always(void* stream, size_t bytes, void** out) {
     if (st) (void)hipGetLastError();  // which the next launch's check would report
     return st == MI355X_OK;
 }
+// The stream's block grown for later calls, by a product that does without: one of fewer rows, or of x elsewhere, may need it, and whoever records that
+// has run the largest call before. Under capture, or where there is no memory, the block stays as it is.
+void reserve(void* stream, ScratchBlock StreamScratch::*which, size_t bytes, size_t floor, const char* what) {
+    DeviceState* s;
+    if (current_state(&s) != MI355X_OK) return;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        if ((s->scratch[stream].*which).bytes >= bytes) return;
+    }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    void* p;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess || (capture == hipStreamCaptureStatusNone && stream_scratch(stream, which, bytes, 0, floor, 0, what, &p)))
+        (void)hipGetLastError();
+}
+void reserve_act(void* stream, size_t bytes) { reserve(stream, &StreamScratch::act, bytes, kActFloorBytes, "activation"); }
 // Where a product's converted activations go: the stream's growing block, or a fixed block of
 // kNoallocScratchBytes (then nothing is allocated, and activations of more than kNoallocActBytes are an error).
 struct ActSource {
@@ -319,6 +334,8 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             const size_t scratch = src.fixed ? 0 : q4_0_scratch_bytes(W, M, N, K, wide_x);
             // two to four of them: x's digits in registers, one launch
             if (rows && g_rows_max == 0 && mimir::qgemv_q4_0_few_pays(a, mimir::Q4Few{})) {
+                if (!src.fixed) reserve_act(stream, std::max(plain, scratch));
+                else if (mi355x_status st = fixed_holds(plain)) return st;
                 HIP_TRY(mimir::qgemv_q4_0_few(a, mimir::Q4Few{}, (hipStream_t)stream), "launch qgemv_q4_0_few");
                 return MI355X_OK;
             }

@@ -636,6 +636,46 @@ def test_q8_0_few_rows_captured_on_a_stream_without_scratch():
     assert np.all(np.abs(again - want) <= 2e-6 * mag + 1e-30)
 
 
+def recorded_after(eager, recorded, want):
+    """`eager` on a new stream, then `recorded` in a graph on it: its scratch is there, as whoever runs the largest call first may expect. Either takes a stream."""
+    l = gpu.lib()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    capi.check(l.mi355x_stream_release(stream.cuda_stream))  # torch hands streams out again
+    try:
+        eager(stream.cuda_stream)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            y = recorded(stream.cuda_stream)
+        for _ in range(2):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bits_equal(y.cpu().numpy(), want)
+    finally:
+        graph = None
+        capi.check(l.mi355x_stream_release(stream.cuda_stream))
+
+
+def test_q4_0_few_rows_leave_their_scratch_to_calls_that_need_it():
+    """Two rows in one launch that needs none, then two whose x is on four bytes, recorded."""
+    l = gpu.lib()
+    rng = np.random.default_rng(2)
+    m, n, k = 2, 4096, 4096
+    buf, ptr = gpu.dev_bytes_at(random_blocks(rng, O.Q4_0, n * k), 0)
+    x = gpu.dev(rng.normal(size=m * k + 1).astype(np.float32))
+    y = torch.empty((m, n), device="cuda:0")
+
+    def call(at, st):
+        gpu.say(f"q4_0 {m} x {n} x {k}, x at {at}")
+        capi.check(l.mi355x_qgemv(O.Q4_0, ptr, x.data_ptr() + at, y.data_ptr(), m, n, k, k, st))
+        return y
+    call(4, gpu.stream())
+    gpu.sync()
+    want = y.cpu().numpy()
+    recorded_after(lambda st: call(0, st), lambda st: call(4, st), want)
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 4096, 512), (2, 14336, 256), (5, 5000, 2048)])
 def test_q8_0_few_rows_are_the_same_product_whatever_the_stream_holds(m, n, k):
     """Bits eager on a stream of some history, eager on a new one, and recorded first on another new one (a graph keeps the kernels it was recorded with); the product by

@@ -153,6 +153,9 @@ mi355x_status argmax_scratch(void* stream, size_t bytes, void** out) {
     return stream_scratch(stream, &StreamScratch::argmax, bytes, 0, 0, (size_t)-1 /* all of it */, "argmax", out);
 }
 
+// The stream's scratch that a K-quant product asks for: as much as either form of these rows or of fewer takes.
+size_t kq_scratch_bytes(int64_t M, int64_t K) { return std::max(mimir::kq_act_bytes(K) * (size_t)M, mimir::kq_lanes_bytes(M, K)); }
+
 size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 // About what a Q4_0 product of M rows takes on the row kernel or the int8 form, the shorter; it never falls as M grows.
@@ -252,12 +255,12 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
         // the int8 rounding reads the bfloat16 rows directly and the matrix-core kernel rounds its results
         void* act;
         if (mimir::qgemm_kquant_shared_pays(dtype, W, M, N, K)) {
-            if (mi355x_status s2 = act_scratch(stream, mimir::kq_lanes_bytes(M, K), &act)) return s2;
+            if (mi355x_status s2 = act_scratch(stream, mimir::kq_lanes_bytes(M, K), &act, kq_scratch_bytes(M, K))) return s2;
             HIP_TRY(mimir::kq_convert_act_bf16(X, M, K, x_row_stride, act, st, true), "launch kq_convert_act");
             HIP_TRY(mimir::qgemm_kquant_shared(dtype, mimir::QGemvArgs{W, nullptr, act, (float*)Y, M, N, K, 0, 0}, st, !f32), "launch qgemm_kquant_shared");
             return MI355X_OK;
         }
-        if (mi355x_status s2 = act_scratch(stream, mimir::kq_act_bytes(K) * (size_t)M, &act)) return s2;
+        if (mi355x_status s2 = act_scratch(stream, mimir::kq_act_bytes(K) * (size_t)M, &act, kq_scratch_bytes(M, K))) return s2;
         mimir::QGemvArgs a{W, nullptr, act, (float*)Y, M, N, K, 0, 0};
         if (mimir::qgemv_kquant_rows_pays(dtype, a)) {  // a few rows: W read once per eight of them, the same bits, one rounding after
             HIP_TRY(mimir::kq_convert_act_bf16(X, M, K, x_row_stride, act, st), "launch kq_convert_act");
@@ -436,18 +439,19 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
         // against a small matrix alone (at K = 2048 3.4 us for N = 1024 where the rounding's launch and the product took 5).
         if (M == 1 && (mimir::qgemv_kquant_stream_pays(dtype, a, mimir::KqStream{}) ||
                        (N * K <= (8ll << 20) && ((uintptr_t)x & 15) == 0 && mimir::qgemv_kquant_rope_ok(dtype, a)))) {
+            if (!src.fixed && N * K > (8ll << 20)) reserve_act(stream, kq_scratch_bytes(M, K));
             HIP_TRY(mimir::qgemv_kquant_act(dtype, a, (hipStream_t)stream), "launch qgemv_kquant");
             return MI355X_OK;
         }
         void* act;
         if (mimir::qgemm_kquant_shared_pays(dtype, W, M, N, K) && (!src.fixed || mimir::kq_lanes_bytes(M, K) <= kNoallocActBytes)) {
-            if (mi355x_status st = act_for(src, mimir::kq_lanes_bytes(M, K), &act)) return st;
+            if (mi355x_status st = act_for(src, mimir::kq_lanes_bytes(M, K), &act, kq_scratch_bytes(M, K))) return st;
             HIP_TRY(mimir::kq_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream, true), "launch kq_convert_act");
             a.act = act;
             HIP_TRY(mimir::qgemm_kquant_shared(dtype, a, (hipStream_t)stream), "launch qgemm_kquant_shared");
             return MI355X_OK;
         }
-        if (mi355x_status st = act_for(src, mimir::kq_act_bytes(K) * (size_t)M, &act)) return st;
+        if (mi355x_status st = act_for(src, mimir::kq_act_bytes(K) * (size_t)M, &act, kq_scratch_bytes(M, K))) return st;
         HIP_TRY(mimir::kq_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream), "launch kq_convert_act");
         a.act = act;
         HIP_TRY(mimir::qgemv_kquant_act(dtype, a, (hipStream_t)stream), "launch qgemv_kquant_act");

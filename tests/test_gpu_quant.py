@@ -676,6 +676,25 @@ def test_q4_0_few_rows_leave_their_scratch_to_calls_that_need_it():
     recorded_after(lambda st: call(0, st), lambda st: call(4, st), want)
 
 
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q6_K])
+def test_kquant_one_row_leaves_its_scratch_to_calls_that_need_it(dt):
+    """One row by a matrix of more than 8 M weights, rounded by the product, then one on four bytes, recorded: the same bits."""
+    l = gpu.lib()
+    rng = np.random.default_rng(3)
+    n, k = 4096, 4096
+    raw = random_blocks(rng, dt, n * k)
+    buf, ptr = gpu.dev_bytes_at(raw, 0)
+    x = rng.normal(size=k).astype(np.float32)
+    xd, y = gpu.dev(np.concatenate([x, x, x[:1]])), torch.empty(n, device="cuda:0")
+    xd[k + 1:] = xd[:k].clone()
+
+    def call(at, st):
+        gpu.say(f"kquant dt={dt} 1 x {n} x {k}, x at element {at}")
+        capi.check(l.mi355x_qgemv(dt, ptr, xd.data_ptr() + 4 * at, y.data_ptr(), 1, n, k, k, st))
+        return y
+    recorded_after(lambda st: call(0, st), lambda st: call(k + 1, st), O.qmatmul(dt, raw, x, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 4096, 512), (2, 14336, 256), (5, 5000, 2048)])
 def test_q8_0_few_rows_are_the_same_product_whatever_the_stream_holds(m, n, k):
     """Bits eager on a stream of some history, eager on a new one, and recorded first on another new one (a graph keeps the kernels it was recorded with); the product by

@@ -444,6 +444,8 @@ static mi355x_status qgemv_impl(int dtype, const void* W, const float* x, float*
             return MI355X_OK;
         }
         void* act;
+        if (src.fixed)  // by the form of which mi355x_act_bytes tells the size
+            if (mi355x_status st = fixed_holds(mimir::kq_act_bytes(K) * (size_t)M)) return st;
         if (mimir::qgemm_kquant_shared_pays(dtype, W, M, N, K) && (!src.fixed || mimir::kq_lanes_bytes(M, K) <= kNoallocActBytes)) {
             if (mi355x_status st = act_for(src, mimir::kq_lanes_bytes(M, K), &act, kq_scratch_bytes(M, K))) return st;
             HIP_TRY(mimir::kq_convert_act(x, M, K, x_row_stride, act, (hipStream_t)stream, true), "launch kq_convert_act");

@@ -116,6 +116,19 @@ def test_noalloc_rejects_what_the_block_cannot_hold():
     gpu.sync()
 
 
+def test_noalloc_rejects_by_the_size_that_act_bytes_tells():
+    """K-quant rows of which sixteen laid out for the matrix cores would fit the block, though mi355x_act_bytes a row says more than 1 MiB."""
+    l = gpu.lib()
+    m, n, k = 128, 4096, 31 * 256
+    w = torch.zeros(n * k // 256 * 144, dtype=torch.uint8, device="cuda:0")
+    x, y = torch.zeros((m, k), device="cuda:0"), torch.zeros((m, n), device="cuda:0")
+    assert m * l.mi355x_act_bytes(capi.Q4_K, k) > 1 << 20
+    st = l.mi355x_qgemv_noalloc(capi.Q4_K, w.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream())
+    assert st == capi.ERR_SHAPE and "fixed scratch" in capi.last_error()
+    capi.check(l.mi355x_qgemv_noalloc(capi.Q4_K, w.data_ptr(), x.data_ptr(), y.data_ptr(), m - 16, n, k, k, gpu.stream()))
+    gpu.sync()
+
+
 def test_a_call_of_more_rows_under_capture_after_one_of_few():
     """What a stream's first call leaves is enough for whatever fills no more than 1 MiB in fixed point: 32 rows by W read where it lies,
     whose rows and shares of K take 4.8 MB, recorded into a graph after a call of eight rows, and replayed."""

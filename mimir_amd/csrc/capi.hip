@@ -233,6 +233,7 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
         return MI355X_OK;
     }
     void* ws;
+    const size_t xb = rounded((size_t)M * K * 4), yb = rounded((size_t)M * N * 4);  // of the general route
     if (dtype == MI355X_Q4_0 && g_tune_gemm != 1 && g_tune_gemm_f16 == 0 && !mimir::q4_0_blocks_chosen() && mimir::qgemm_q4_0_strips_pays(W, X, true, M, N, K, x_row_stride)) {
         HIP_TRY(mimir::qgemm_q4_0_strips(W, X, true, Y, !f32, M, N, K, x_row_stride, st), "launch qgemm_q4_0_strips");
         return MI355X_OK;
@@ -279,6 +280,7 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
         if (mimir::qgemv_q8_0_mfma_pays(a)) {
             void* act;
             if (mi355x_status s2 = act_scratch(stream, mimir::q8_act_bytes(K) * (size_t)M, &act)) return s2;
+            reserve(stream, &StreamScratch::gemm, xb + yb, 0, "gemm");  // fewer rows take the general route
             a.act = act;
             HIP_TRY(mimir::q8_convert_act_bf16(X, M, K, x_row_stride, act, st), "launch q8_convert_act");
             HIP_TRY(mimir::qgemv_q8_0_mfma(a, st, !f32), "launch qgemv_q8_0_mfma");
@@ -288,7 +290,6 @@ mi355x_status mi355x_qgemm_bf16(int dtype, const void* W, const void* X, void* Y
     // Any other shape or dtype: the activations as float32 through mi355x_qgemv, then one rounding. For
     // Q8_0, Q4_K and Q6_K that is the reference's own sequence (cast, int8 rounding of x, integer dot
     // products, cast), and the K-quants take their matrix-core kernel from a few rows on.
-    const size_t xb = ((size_t)M * K * 4 + 255) & ~(size_t)255, yb = ((size_t)M * N * 4 + 255) & ~(size_t)255;
     if (mi355x_status s2 = gemm_scratch(stream, xb + yb, &ws)) return s2;
     float* xf = (float*)ws;
     float* yf = f32 ? (float*)Y : (float*)((uint8_t*)ws + xb);

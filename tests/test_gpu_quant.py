@@ -695,6 +695,25 @@ def test_kquant_one_row_leaves_its_scratch_to_calls_that_need_it(dt):
     recorded_after(lambda st: call(0, st), lambda st: call(k + 1, st), O.qmatmul(dt, raw, x, n, k))
 
 
+def test_q8_0_bfloat16_rows_leave_their_scratch_to_fewer():
+    """Sixteen bfloat16 rows without the casts around them, then one of them, which has those, recorded."""
+    l = gpu.lib()
+    rng = np.random.default_rng(4)
+    m, n, k = 16, 2048, 1024
+    buf, ptr = gpu.dev_bytes_at(random_blocks(rng, O.Q8_0, n * k), 0)
+    x = gpu.dev(rng.normal(size=(m, k)).astype(np.float32)).to(torch.bfloat16)
+    ys = {rows: torch.empty((rows, n), device="cuda:0") for rows in (1, m)}
+
+    def call(rows, st):
+        gpu.say(f"q8_0 bf16 {rows} x {n} x {k}")
+        capi.check(l.mi355x_qgemm_bf16(capi.Q8_0, ptr, x.data_ptr(), ys[rows].data_ptr(), rows, n, k, k, capi.F32, st))
+        return ys[rows]
+    call(1, gpu.stream())
+    gpu.sync()
+    want = ys[1].cpu().numpy()
+    recorded_after(lambda st: call(m, st), lambda st: call(1, st), want)
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 4096, 512), (2, 14336, 256), (5, 5000, 2048)])
 def test_q8_0_few_rows_are_the_same_product_whatever_the_stream_holds(m, n, k):
     """Bits eager on a stream of some history, eager on a new one, and recorded first on another new one (a graph keeps the kernels it was recorded with); the product by

@@ -264,15 +264,29 @@ bool qgemv_q4_0_few_ok(const QGemvArgs& a, const Q4Few& q) {
     if ((q.rope || q.swiglu) != (head == kHeadNorm) || ((q.rope || q.swiglu) && a.resid)) return false;
     return lds_of(a.K, (int)a.M, head, q.swiglu ? 2 * R : R, cuts) <= kMaxLds;
 }
-// float32 x. A row of W costs as much however short it is, and a row of x more as much again: us, by the kernel for eight rows | here, two rows of x 14336 x 1024 8.1 | 8.9,
-// 32768 x 1024 13.8 | 16.3, but 4096 x 1024 6.5 | 5.1, 32768 x 2048 18.6 | 16.3, 4096 x 4096 9.6 | 5.6, 14336 x 4096 16.6 | 10.3, 4096 x 14336 22.9 | 14.7, 14336 x 14336 43 | 32; three
-// 8192 x 1024 6.9 | 8.4, 8192 x 2048 8.4 | 8.5, but 4096 x 2048 7.9 | 6.4, 8192 x 4096 12.2 | 9.3, 5120 x 5120 12.1 | 11.9, 14336 x 14336 43 | 41.5; four 4096 x 1024 6.6 | 7.6,
-// 5120 x 5120 12.4 | 14.6, 14336 x 8192 26.6 | 29.5, but 3000 x 2048 7.9 | 6.8, 1024 x 6144 11.3 | 8.8, 4096 x 4096 9.7 | 8.6, 14336 x 4096 16.7 | 16.3.
+// float32 x. A turn of a workgroup's wavefronts takes as long however many of their lanes have a pair of blocks, and a row of x more as much again, where the kernel for eight rows takes
+// what W's bytes take: here where that share of the lanes is large, or the rows of W are few. us, there | here, of all lanes (K = 4096, 8192 of them): two rows 4096 x 4096 9.6 | 5.6, 14336 x
+// 4096 16.6 | 10.3; three 8192 x 4096 12.2 | 9.3, 28672 x 8192 44 | 36; four 4096 x 4096 9.7 | 8.7, but 38912 x 4096 31.3 | 31.9, 14336 x 8192 26.3 | 29.5. Of less than half of them, two
+// rows 5120 x 256 5.4 | 5.2, 11008 x 1024 10.0 | 8.8, 14336 x 1536 10.1 | 9.4, but 8192 x 256 5.5 | 6.8, 28672 x 1024 12.0 | 16.6; three 2048 x 256 5.3 | 5.1, 4096 x 1024 6.5 | 6.5, 6144 x 2048 8.1 | 7.5, but
+// 28672 x 2048 15.9 | 17.6; four 1024 x 512 5.6 | 5.3, 4096 x 2048 7.9 | 7.7. Of 0.63 to 0.75 (K = 5120, 6144, 11008): two rows 14336 x 5120 19.2 | 16.9; three 3072 x 5120 10.5 | 9.8, but 14336 x 5120
+// 19.2 | 22.1, 38912 x 11008 75 | 90; four 1024 x 11008 13.0 | 11.8, but 3072 x 11008 15.8 | 19.5. K = 3072, whose rows fit a wavefront: three 14336 x 3072 13.3 | 12.6, four 4096 x 3072 8.8 | 8.7, but 128256 x 3072 71 | 94.
+// All that where K is a multiple of 256, whole runs of that kernel; else it takes up to twice as long: two 32704 x 640 17.7 | 18.5, 22528 x 11072 66 | 32; three 18688 x 448 17.4 | 14.0, 16640 x 14528 104 | 49,
+// but 15962 x 640 14.6 | 18.2; four 2688 x 384 7.7 | 6.6, 25280 x 6592 78 | 46, 11098 x 1728 13.8 | 12.8, but 4608 x 320 7.6 | 8.7, 20544 x 1152 16 | 20.
 bool qgemv_q4_0_few_pays(const QGemvArgs& a, const Q4Few& q) {
     if (g_few == 1 || !qgemv_q4_0_few_ok(a, q)) return false;
-    if (g_few == 2 || a.N <= 3072) return true;
-    if (a.M == 2) return a.K >= 2048 || a.N <= 8192;
-    return a.M == 3 ? a.K >= 4096 || a.N <= 4096 : a.K > 2048 && a.K <= 4096;
+    if (g_few == 2) return true;
+    const int64_t pairs = a.K / 64, cuts = (pairs + 63) / 64;
+    const double lanes = (double)(pairs * (kWaves / cuts)) / (64 * kWaves);  // that work, in the workgroup
+    const bool runs = a.K % 256 == 0;
+    if (a.M == 2) return !runs || lanes >= 0.5 || (double)a.N <= 4096 + 28000 * lanes;
+    if (a.M == 3) {
+        if (!runs) return lanes >= 0.25 || a.N <= 12288;
+        if (lanes >= (cuts == 1 ? 0.75 : 0.85)) return true;
+        return cuts == 1 ? (double)a.N <= 1536 + 10500 * lanes : a.N <= (lanes >= 0.75 ? 4096 : 3072);
+    }
+    if (!runs) return a.K > 1536 || a.N <= 3072;
+    if (lanes >= 1) return a.N <= (cuts == 1 ? 28672 : 2048);
+    return cuts == 1 ? (double)a.N <= std::min(4096.0, 600 + 7000 * lanes) : a.N <= (lanes >= 0.75 ? 2048 : 1024);
 }
 
 hipError_t qgemv_q4_0_few(const QGemvArgs& a, const Q4Few& q, hipStream_t st) {

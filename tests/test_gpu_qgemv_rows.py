@@ -2,6 +2,8 @@
 reads W once for eight rows on the int8 matrix cores, against the oracle's float32 product with the
 dequantized weights (io/mim/dtype.go:118-123, backend/cpu/gemv.go:73-104; bound 1e-3) and against
 the one-row kernel, whose integers it shares."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -73,6 +75,22 @@ def test_two_to_four_rows_by_a_workgroup_a_compute_unit(m, n, k):
             assert np.isnan(worse[m - 1]).all() and np.array_equal(worse[:-1].view(np.uint32), got[:-1].view(np.uint32))
     finally:
         capi.check(l.mi355x_tune(b"q4_0.few", 0))
+
+
+@pytest.mark.parametrize("m,n,k,few", [(2, 4096, 4096, True), (2, 28672, 1024, False), (3, 28672, 8192, True), (3, 38912, 5120, False), (3, 14336, 11008, False),
+                                       (3, 16640, 14528, True), (4, 2048, 4096, True), (4, 3072, 11008, False), (4, 65536, 3072, False), (4, 25280, 6592, True)])
+def test_two_to_four_rows_go_where_they_are_faster(m, n, k, few):
+    """By the kernel for few rows where most of its lanes have a pair of blocks, rows of W are few, or the kernel for eight rows has no whole runs."""
+    l = gpu.lib()
+    w = torch.zeros(n * k // 32 * 18, dtype=torch.uint8, device="cuda:0")
+    x, y = torch.zeros((m, k), device="cuda:0"), torch.empty((m, n), device="cuda:0")
+    gpu.say(f"q4_0 route of {m} x {n} x {k}")
+    name = ctypes.create_string_buffer(200)
+    gpu.qgemv(O.Q4_0, w.data_ptr(), x[:1], 16, k)  # a kernel of another name
+    capi.check(l.mi355x_qgemv(O.Q4_0, w.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, k, k, gpu.stream()))
+    capi.check(l.mi355x_last_kernel(name, 200))
+    gpu.sync()
+    assert name.value.decode().startswith("qgemv_q4_0_few_kernel") == few
 
 
 def test_rows_kernel_at_the_model_shapes():

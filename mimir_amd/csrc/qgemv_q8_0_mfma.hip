@@ -271,11 +271,12 @@ void set_q8_mfma(int v) { g_q8_mfma = v; }
 // 14336 x 1024 29.7, 8.1, 14336 x 2048 49.7, 12.1, 4096 x 1024 10.5, 6.5; four 4096 x 1024 6.4, 6.4, 8192 x 2048 12.6, 8.3; three 8192 x 1024 8.4, 6.7, but 4096 x 2048 6.3, 7.3; two 14336 x
 // 1024 9.3, 7.9, but 12288 x 2048 10.9, 11.0, 8192 x 2048 7.8, 8.2. Other few rows keep the bits that a row alone has.
 // More rows, of which the vector unit takes eight a pass over W: from 64 rows of W on nearly always; nine rows 512 x 1024 10.6, 7.5, 64 x 2048 10.3, 8.3, 1280 x 4096 15.6, 11.7, 3072 x 14336 46, 30,
-// 17 rows 1024 x 4096 17.2, 12.1, but sixteen 1024 x 4096 11.3, 12.0, 512 x 8192 10.8, 17.5, twelve 1536 x 8192 16.8, 17.7 (2048 x 8192 19.8, 17.7), nine 2048 x 14336 27.5, 29.4 (twelve 32.7, 29.7).
+// 17 rows 1024 x 4096 17.2, 12.1; of an odd number of blocks, which the vector unit takes a row of x at a time, from 12000 results on (17 rows 874 x 672 8.8, 7.8, 12 rows 1408 x 352 8.4, 7.0, but 26 x 192 x 1696
+// 6.3, 9.9, 9 x 1088 x 1184 7.5, 8.7); but sixteen 1024 x 4096 11.3, 12.0, 512 x 8192 10.8, 17.5, twelve 1536 x 8192 16.8, 17.7 (2048 x 8192 19.8, 17.7), nine 2048 x 14336 27.5, 29.4 (twelve 32.7, 29.7).
 bool qgemv_q8_0_mfma_pays(const QGemvArgs& a) {
     if (g_q8_mfma == 2 || !qgemv_q8_0_mfma_ok(a)) return false;
     if (g_q8_mfma == 1) return true;
-    if (a.M > kFewRows) return a.M * a.N >= 32768 || (a.N >= 64 && (a.K <= 2048 || (a.K <= 6144 ? a.N >= 1280 || a.M * a.N >= 17000 : a.M * a.N >= 24000)));
+    if (a.M > kFewRows) return a.M * a.N >= 32768 || (a.N >= 64 && (a.K <= 2048 ? qgemv_q8_0_rows_ok(a) || a.M * a.N >= 12000 : (a.K <= 6144 ? a.N >= 1280 || a.M * a.N >= 17000 : a.M * a.N >= 24000)));
     if (a.K <= 2048 && a.N >= (a.M == 2 ? 14336 : a.M == 3 ? 6144 : 4096)) return true;
     return a.N * a.K >= ((int64_t)32 << 20) && a.N >= (a.M >= 4 ? 4096 : 6144);
 }

@@ -714,6 +714,18 @@ def test_q8_0_bfloat16_rows_leave_their_scratch_to_fewer():
     recorded_after(lambda st: call(m, st), lambda st: call(1, st), want)
 
 
+@pytest.mark.parametrize("m,n,k,row_bits", [(26, 192, 1696, True), (9, 1088, 1184, True), (17, 874, 672, False), (26, 192, 1664, False)])
+def test_q8_0_rows_of_an_odd_number_of_blocks_go_where_they_are_faster(m, n, k, row_bits):
+    """More than eight rows by few rows of W of an odd number of blocks: the one-row kernel, whose bits each row alone has; the matrix cores from 12000 results on, and for an even number."""
+    rng = np.random.default_rng(k)
+    buf, ptr = gpu.dev_bytes_at(random_blocks(rng, O.Q8_0, n * k), 0)
+    x = gpu.dev(rng.normal(size=(m, k)).astype(np.float32))
+    gpu.say(f"q8_0 route of {m} x {n} x {k}")
+    got = gpu.qgemv(O.Q8_0, ptr, x, n, k)
+    alone = np.stack([gpu.qgemv(O.Q8_0, ptr, x[i:i + 1], n, k)[0] for i in range(m)])
+    assert bits_equal(got, alone) == row_bits
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 4096, 512), (2, 14336, 256), (5, 5000, 2048)])
 def test_q8_0_few_rows_are_the_same_product_whatever_the_stream_holds(m, n, k):
     """Bits eager on a stream of some history, eager on a new one, and recorded first on another new one (a graph keeps the kernels it was recorded with); the product by

@@ -365,6 +365,8 @@ bool qgemm_kquant_shared_ok(int dt, const void* W, int64_t M, int64_t N, int64_t
 // units has workgroups, 0.7 us and per eight super-blocks 0.3 (Q4_K) or 0.6 (Q6_K) and 0.68 for each tile of rows. On 1350 products of 9 to 512 rows, 384 to 24768 x 512 to 14848,
 // the choice takes 0.6 % (Q4_K) or 1.6 % (Q6_K) longer than the faster side in the mean. us, here | by the kernel that had them: Q4_K 16 x 4096 x 14336 13.4 | 19.5, 64 x 4096 x 4096 11.2 | 18.6,
 // 64 x 4096 x 14336 26.9 | 59.7, 128 x 14336 x 4096 56 | 34, 256 x 4096 x 14336 92 | 100, 512 x 4096 x 4096 65 | 38; Q6_K 16 x 14336 x 4096 17.7 | 22.4, 64 x 4096 x 14336 27.4 | 83, 128 x 14336 x 4096 56 | 36.
+// Not where one tile of rows leaves half the compute units idle (16 x 2048 x 14336 Q4_K 13.4 | 11.9, Q6_K 18.2 | 14.8), nor where seven turns and more are one round of super-blocks each, whose
+// beginnings take longer than the model's (64 x 28672 x 2048 Q4_K 45.7 | 37.5, 9 rows 21.3 | 18.4; Q6_K 64 45.8 | 41.7, but 48 37 | 40).
 bool qgemm_kquant_shared_pays(int dt, const void* W, int64_t M, int64_t N, int64_t K) {
     if (M > kSharedRows || !qgemm_kquant_shared_ok(dt, W, M, N, K) || g_kq_shared == 1 || !kquant_by_rule()) return false;
     if (g_kq_shared == 2) return true;
@@ -372,6 +374,8 @@ bool qgemm_kquant_shared_pays(int dt, const void* W, int64_t M, int64_t N, int64
     int64_t groups;
     const int tiles = tiles_of(M, &groups);
     const int64_t turns = ((N + 127) / 128 * 8 * groups + 255) / 256, rounds = (K / 256 + kWaves - 1) / kWaves;
+    if (M <= kStrip && N <= 2048) return false;
+    if (rounds == 1 && turns > 6 && (dt == kQ4_K || tiles == 4)) return false;
     return 2 + (double)turns * (0.7 + (double)rounds * ((dt == kQ4_K ? 0.3 : 0.6) + 0.68 * tiles)) < qgemv_kquant_us(dt, M, N, K);
 }
 

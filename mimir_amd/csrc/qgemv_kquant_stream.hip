@@ -510,6 +510,12 @@ hipError_t launch_rows(int dt, const Job& j, int64_t M, int x_rows, hipStream_t 
     }
 }
 
+// The share of the lanes of kFewWaves wavefronts that have a super-block in a turn.
+double lanes_used(int dt, int nsb) {
+    const int units = dt == kQ4_K ? 16 : 8, cuts = (nsb + units - 1) / units;
+    if (cuts == 1) return (double)(units / nsb * nsb) / units;
+    return (double)(nsb * (kFewWaves / cuts)) / (units * kFewWaves);
+}
 int head_of(const QGemvArgs& a, const KqStream& s) { return a.act ? kHeadAct : s.norm_w ? kHeadNorm : kHeadRound; }
 // Rows of x a workgroup: all, but for the forms that have one of them a workgroup.
 int x_rows_of(const QGemvArgs& a, const KqStream& s) { return a.act && s.rope ? 1 : (int)std::min<int64_t>(a.M, 1 << 16); }
@@ -538,16 +544,19 @@ bool qgemv_kquant_stream_ok(int dt, const QGemvArgs& a, const KqStream& s) {
 // workgroup or a launch of its own, is what takes the time; always where a launch before the product goes with it. us, there | here, converted row: Q4_K 1024 x 4096 3.2 | 3.8,
 // 2048 x 2048 3.5 | 3.6, 2500 x 1024 3.9 | 3.4, 4096 x 4096 4.9 | 4.6, 28672 x 4096 18.9 | 14.4, 128256 x 2048 37 | 28; Q6_K 2048 x 4096 4.4 | 4.5, 2048 x 8192 6.8 | 6.4,
 // 8192 x 2048 6.0 | 6.0, 28672 x 4096 26.7 | 21.8; float32 x: Q4_K 1024 x 2048 3.45 | 3.60, 512 x 4096 4.1 | 3.8, 2048 x 2048 4.1 | 3.85, 4096 x 14336 13.5 | 10.8;
-// Q6_K 2048 x 1024 3.7 | 3.9, 512 x 4096 4.6 | 4.0, 4096 x 14336 16.5 | 14.7. Two and three converted rows where the kernel that reads W once for eight has four wavefronts a workgroup,
-// two rows there | here: Q4_K 8192 x 4096 7.3 | 7.4, 14336 x 4096 12.7 | 10.2, 14336 x 14336 35.6 | 26.1, Q6_K 14336 x 4096 16.2 | 13.7; three: Q4_K 14336 x 2048 7.7 | 7.9,
-// 14336 x 4096 12.7 | 11.3, Q6_K 14336 x 8192 29.4 | 26.5; four are level, eight (28672 x 4096 Q4_K 22.4) twice as slow here but with the spills of eight rows in registers.
-// A step of two, three and four sequences with its norms here: 10.4 | 9.3, 10.5 | 9.95 and 10.75 | 10.75 ms for 32 of four Q4_K blocks of 4096 features.
+// Q6_K 2048 x 1024 3.7 | 3.9, 512 x 4096 4.6 | 4.0, 4096 x 14336 16.5 | 14.7. Two and three converted rows where the kernel that reads W once for eight has four wavefronts a workgroup, and where
+// enough lanes here have a super-block (K = 4096, 8192 and 14336; of Q4_K as well where W is read by two rows): two rows there | here: Q4_K 8192 x 4096 7.3 | 7.4, 14336 x 4096 12.7 | 10.2, 14336 x
+// 14336 35.6 | 26.1, 38912 x 5120 33 | 29, Q6_K 14336 x 4096 16.2 | 13.7, but 20480 x 3072 17.7 | 19.0, 20480 x 5120 27.6 | 30.4; three: Q4_K 14336 x 2048 7.7 | 7.9, 14336 x 4096 12.7 | 11.3, Q6_K
+// 14336 x 8192 29.4 | 26.5, but Q4_K 38912 x 5120 33 | 39.3, Q6_K 28672 x 5120 37 | 44; four are level, eight (28672 x 4096 Q4_K 22.4) twice as slow here but with the spills of eight rows in registers.
+// A step with its norms here, us, four blocks: two sequences Q4_K of 512, 1024, 2048 and 4096 features 122 | 114, 140 | 126, 163 | 147, 243 | 225, Q6_K 123 | 115, 141 | 131, 189 | 165, 301 | 274; three Q4_K 117 | 115,
+// 134 | 128, 163 | 153, 246 | 241, Q6_K 118 | 116, 140 | 132, 174 | 171, 306 | 288, but of 2560 features, whose rows leave three lanes in eight idle, 181 | 185 and 206 | 210; four of 4096 336 | 336.
 bool qgemv_kquant_stream_pays(int dt, const QGemvArgs& a, const KqStream& s) {
     if (g_kq_stream == 1 || !kquant_by_rule() || !qgemv_kquant_stream_ok(dt, a, s)) return false;
     if (g_kq_stream) return true;
     const int head = head_of(a, s);
-    if (head == kHeadNorm) return true;
-    if (a.M > 1 && !s.rope) return a.N > 8192 && a.K >= 2048 * (a.M - 1);
+    const double lanes = lanes_used(dt, (int)(a.K / 256));
+    if (head == kHeadNorm) return a.M < 3 || lanes >= 0.7;
+    if (a.M > 1 && !s.rope) return a.N > 8192 && a.K >= 2048 * (a.M - 1) && (lanes >= 0.8 || (a.M == 2 && (dt == kQ4_K || a.K > 8192)));
     return head == kHeadAct ? a.N > 2048 : a.N * a.K > (2ll << 20) || a.K >= 3072;
 }
 

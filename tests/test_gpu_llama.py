@@ -610,6 +610,67 @@ def test_kquant_steps_with_norms_and_swiglu_in_the_products_have_the_bits_of_tho
     assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1].view(np.uint32), runs[1][1].view(np.uint32))
 
 
+@pytest.mark.parametrize("embed", [2304, 3072, 4096])
+@pytest.mark.parametrize("linear_dt", [O.Q4_K, O.Q6_K])
+def test_kquant_norms_in_the_products_of_several_tasks(linear_dt, embed):
+    """Rows of nine, twelve and sixteen super-blocks, a norm's three tasks (of which two wavefronts share one) and four, two turns of them for three sequences, rows of Q6_K cut over two
+    wavefronts behind a norm: caches and logits of one to three sequences bit for bit those of launches of their own."""
+    lib = gpu.lib()
+    c = _small_q4_config(1, capi.F16)
+    c.embed, c.hidden, c.layers, c.heads, c.kv_heads, c.vocab, c.context = embed, 1280, 2, 6, 2, 301, 32
+    om = OL.synthetic(_oracle_config(c), seed=5, linear_dt=linear_dt)
+    for batch in (1, 2, 3):
+        c.batch = batch
+        m = Llama(c)
+        _upload_synthetic(m, om)
+        m.finalize(8 * batch)
+        prompts = np.random.default_rng(7).integers(0, c.vocab, (batch, 5))
+        runs = []
+        try:
+            capi.check(lib.mi355x_tune(b"llama.step", 1))
+            for stream in (8, 1):
+                capi.check(lib.mi355x_tune(b"kquant.stream", stream))
+                gpu.say(f"steps dt={linear_dt} embed={embed} batch={batch} stream={stream}")
+                m.reset()
+                tokens, _ = m.generate(prompts, 8)
+                capi.check(lib.mi355x_tune(b"kquant.stream", 1))
+                runs.append((tokens, np.asarray(m.logits(tokens[:, -1:]))))
+        finally:
+            capi.check(lib.mi355x_tune(b"kquant.stream", 0))
+            capi.check(lib.mi355x_tune(b"llama.step", 0))
+        m.close()
+        assert np.array_equal(runs[0][0], runs[1][0]) and np.array_equal(runs[0][1].view(np.uint32), runs[1][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("embed,hidden,heads", [(4096, 4608, 36), (2304, 14336, 4), (256, 768, 4)])
+def test_steps_of_two_q4_0_sequences_by_the_kernel_for_few_rows(embed, hidden, heads):
+    """Two sequences: rows of a wavefront's 64 pairs of blocks and of more (72 and 224, cut over two and four wavefronts), of converted rows with the residual, of two norm items a
+    thread; and rows of four pairs. Tokens of the steps by the kernel for eight rows, logits of the next token within 1e-5 of the largest (a product is within 2e-7, and a model has some tens)."""
+    lib = gpu.lib()
+    c = _small_q4_config(2, capi.F16)
+    c.embed, c.hidden, c.layers, c.heads, c.vocab, c.context = embed, hidden, 2, heads, 515, 40
+    om = OL.synthetic(_oracle_config(c), seed=9, output_dt=O.Q4_0)
+    m = Llama(c)
+    _upload_synthetic(m, om)
+    m.finalize(16)
+    prompts = np.random.default_rng(8).integers(0, c.vocab, (2, 7))
+    runs = []
+    try:
+        for few, step in ((1, 1), (0, 1), (0, 0)):
+            capi.check(lib.mi355x_tune(b"q4_0.few", few))
+            capi.check(lib.mi355x_tune(b"llama.step", step))
+            gpu.say(f"two sequences of {embed} features, few={few}, step={step}")
+            m.reset()
+            tokens, _ = m.generate(prompts, 9)
+            runs.append((tokens, m.logits(tokens[:, -1:])))
+    finally:
+        capi.check(lib.mi355x_tune(b"q4_0.few", 0))
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    for tokens, logits in runs[1:]:
+        assert np.array_equal(tokens, runs[0][0]) and np.abs(logits - runs[0][1]).max() <= 1e-5 * np.abs(runs[0][1]).max()
+    assert np.array_equal(runs[1][1], runs[2][1]) and not np.array_equal(runs[0][1], runs[1][1])
+
+
 def test_fused_steps_without_their_riders_choose_the_per_operator_tokens():
     """The fused step lets the rotation, the norms and the conversion of SwiGLU's results ride on the products
     only where their shapes allow: interleaved pairs, rows of x one step of a wavefront long. A model with
@@ -745,14 +806,19 @@ def test_k_quant_products_of_some_rows_in_a_decoder(linear_dt, batch, tokens):
         for mode in (1, 2, 0):
             gpu.say(f"k-quant rows in a decoder, dtype {linear_dt} {batch} x {tokens}, mode {mode}")
             capi.check(lib.mi355x_tune(b"kquant.shared", mode))
+            capi.check(lib.mi355x_tune(b"llama.step", 1))  # launches, which a graph of the first mode would stand in for
             m.reset()
             logits = m.logits(prompts, all=True)
             m.reset()
-            runs.append((logits, m.generate(prompts, 6)[0]))
+            chosen = m.generate(prompts, 6)[0]
+            capi.check(lib.mi355x_tune(b"kquant.shared", 1))
+            runs.append((logits, chosen, m.logits(chosen[:, -1:])))  # by the same kernels from what the steps have left in the caches
     finally:
         capi.check(lib.mi355x_tune(b"kquant.shared", 0))
-    for logits, chosen in runs[1:]:
+        capi.check(lib.mi355x_tune(b"llama.step", 0))
+    for logits, chosen, after in runs[1:]:
         assert np.array_equal(logits.view(np.uint32), runs[0][0].view(np.uint32)) and np.array_equal(chosen, runs[0][1])
+        assert np.array_equal(after.view(np.uint32), runs[0][2].view(np.uint32))
 
 
 @pytest.mark.parametrize("linear_dt", [O.Q4_K, O.Q6_K, O.Q8_0, O.Q4_0])

@@ -208,3 +208,24 @@ def test_strips_of_sixteen_rows_of_w_by_some_rows_of_x(dt, m, n, k):
         assert np.array_equal(y.cpu().numpy().view(np.uint16), O.f32_to_bf16(O.qmatmul(dt, raw, O.bf16_to_f32(xb), n, k)))
     finally:
         capi.check(l.mi355x_tune(b"kquant.shared", 0))
+
+
+@pytest.mark.parametrize("dt,m,n,k,kernel", [
+    (O.Q4_K, 3, 14336, 4096, "stream"), (O.Q4_K, 3, 38912, 5120, ""), (O.Q4_K, 2, 38912, 5120, "stream"), (O.Q6_K, 3, 14336, 8192, "stream"), (O.Q6_K, 2, 20480, 3072, ""),
+    (O.Q6_K, 3, 28672, 6144, ""), (O.Q4_K, 16, 4096, 4096, "shared"), (O.Q4_K, 16, 2048, 14336, ""), (O.Q6_K, 9, 2048, 4096, ""), (O.Q4_K, 64, 28672, 2048, ""),
+    (O.Q6_K, 64, 28672, 2048, ""), (O.Q6_K, 48, 28672, 2048, "shared")])
+def test_some_rows_go_where_they_are_faster(dt, m, n, k, kernel):
+    """Two and three rows by the kernel of a workgroup a compute unit where enough of its lanes have a super-block; more by the one of sixteen rows of W where it has a unit's work for
+    each, and not many short turns. (Other kernels for a few rows have no name.)"""
+    l = gpu.lib()
+    w = gpu.dev(np.zeros(n * k // 256 * (144 if dt == O.Q4_K else 210), np.uint8))
+    gpu.say(f"kquant route of dt={dt} {m} x {n} x {k}")
+    name = ctypes.create_string_buffer(200)
+    x = gpu.dev(np.zeros((m, k), np.float32))
+    gpu.qgemv(O.Q4_0, w.data_ptr(), x[:1], 16, k)  # a kernel of another name
+    gpu.qgemv(dt, w.data_ptr(), x, n, k)
+    capi.check(l.mi355x_last_kernel(name, 200))
+    name = name.value.decode()
+    assert name.startswith({"stream": "qgemv_kquant_stream_kernel", "shared": "qgemm_kquant_shared_kernel"}.get(kernel, "q")), name
+    if not kernel:
+        assert not name.startswith(("qgemv_kquant_stream_kernel", "qgemm_kquant_shared_kernel")), name

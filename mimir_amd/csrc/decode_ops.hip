@@ -371,20 +371,14 @@ hipError_t set_state(int32_t* state, int pos, int step, hipStream_t st) {
 }
 
 // ---- SwiGLU: llm/model.go:446-448; tensor/elementwise.go:520-525,583-585 ----------
-// out = (g * recip(1 + exp2(g * -log2e))) * u, each step a float32. Rows of g
-// and u are `stride` floats apart (they may be the halves of one fused
-// product); out is contiguous.
+// silu_times of every element. Rows of g and u are `stride` floats apart (they
+// may be the halves of one fused product); out is contiguous.
 __global__ __launch_bounds__(256) void swiglu_kernel(const float* __restrict__ g, const float* __restrict__ u,
                                                      float* __restrict__ out, int64_t rows, int64_t n, int64_t stride) {
-    const float nl2e = (float)(-1.4426950408889634);
     int64_t total = rows * n;
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
         int64_t r = t / n, i = t % n;
-        float gv = g[r * stride + i];
-        float e = __builtin_exp2f(gv * nl2e);
-        float s = 1.0f / (1.0f + e);
-        float a = gv * s;
-        out[t] = a * u[r * stride + i];
+        out[t] = silu_times(g[r * stride + i], u[r * stride + i]);
     }
 }
 

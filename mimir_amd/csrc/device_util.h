@@ -131,6 +131,19 @@ __device__ __forceinline__ float strided_sum_squares(const float* __restrict__ x
     return d <= 1024 ? strided_sum_squares_by<4>(xr, d, t) : strided_sum_squares_by<16>(xr, d, t);
 }
 
+// SiLU(g) u (llm/model.go:446-448; tensor/elementwise.go:520-525, 583-585): (g recip(1 + exp2(-g log2 e))) u, each step a float32.
+__device__ __forceinline__ float silu_times(float g, float u) {
+    const float e = __builtin_exp2f(g * (float)(-1.4426950408889634));
+    const float s = 1.0f / (1.0f + e);
+    const float a = g * s;
+    return a * u;
+}
+
+// Memory whose loads past `bytes` give zeros and touch nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
+}
+
 // ---- half conversions -----------------------------------------------------
 // The hardware's cvt instructions round to nearest even and keep subnormals
 // (the f16 denormal mode is on), which is what half.go computes for every

@@ -54,13 +54,6 @@ struct Operands {
     Parts parts;
 };
 
-__device__ __forceinline__ float silu_times(float g, float u) {  // as swiglu_kernel's
-    const float e = __builtin_exp2f(g * (float)(-1.4426950408889634));
-    const float s = 1.0f / (1.0f + e);
-    const float a = g * s;
-    return a * u;
-}
-
 // Where column 0 of a strip goes: its part, and the column it is there. SwiGLU: of both gate's and up's strips, the result's.
 __device__ __forceinline__ int part_of(const Parts& p, int strip, int* n) {
     const int part = p.swiglu ? 0 : strip >= p.begin[2] ? 2 : strip >= p.begin[1] ? 1 : 0;

@@ -125,17 +125,11 @@ __global__ __launch_bounds__(64) void swiglu_kq_act_kernel(const float* __restri
                                                            uint8_t* __restrict__ act, int64_t act_row_bytes) {
     const int sb = blockIdx.x, lane = threadIdx.x;
     const int64_t at = (int64_t)blockIdx.y * stride + 256 * (int64_t)sb + 4 * lane;
-    const float nl2e = (float)(-1.4426950408889634);
     f32x4 gv, uv, v;
     __builtin_memcpy(&gv, g + at, 16);
     __builtin_memcpy(&uv, u + at, 16);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        float e = __builtin_exp2f(gv[k] * nl2e);
-        float sg = 1.0f / (1.0f + e);
-        float a = gv[k] * sg;
-        v[k] = a * uv[k];
-    }
+    for (int k = 0; k < 4; k++) v[k] = silu_times(gv[k], uv[k]);
     kq_store(v, sb, lane, nsb, act, act_row_bytes);
 }
 

@@ -45,10 +45,6 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 constexpr int kRows = 8;    // rows of x a group holds
 constexpr uint32_t kBeyond = 1u << 30;  // an offset, or a bit of one, past every buffer's end: the load gives zeros and touches no memory
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
-}
-
 // The sums of lanes 32 apart: lanes of the lower half get v[0] and v[1] of both, lanes of the upper half v[2] and v[3].
 __device__ __forceinline__ void add_halves(const int v[4], int out[2]) {
 #pragma unroll

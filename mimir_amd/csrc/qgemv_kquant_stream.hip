@@ -139,10 +139,6 @@ __device__ __forceinline__ void round_by_sixteen(const f32x4 v[4], int l, uint8_
     if (l == 0) *d_out = !finite ? __builtin_nanf("") : some ? d : 0.f;
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
-}
-
 // Of the block at `at` from the buffer's start. j: the lane's place among those of a super-block.
 __device__ __forceinline__ void fetch(Raw<kQ4_K>& f, __amdgpu_buffer_rsrc_t w, uint32_t at, int j) {
     f.hdr = __builtin_amdgcn_raw_buffer_load_b128(w, at, 0, 0);
@@ -461,12 +457,8 @@ __global__ __launch_bounds__(64 * (ROWS > 1 ? kFewWaves : kMostWaves)) void qgem
         const uint8_t* from = terms + (r * local + result) * stride;
         const int64_t at = (int64_t)(m0 + r) * a.N + first + result;
         float out = add_row<DT>(from, nsb);
-        if (TAIL == kTailSwiglu) {  // swiglu_kernel's arithmetic (llm/model.go:446-448)
-            const float u = add_row<DT>(from + R * stride, nsb);
-            const float e = __builtin_exp2f(out * (float)(-1.4426950408889634));
-            const float sg = 1.0f / (1.0f + e);
-            const float silu = out * sg;
-            out = silu * u;
+        if (TAIL == kTailSwiglu) {
+            out = silu_times(out, add_row<DT>(from + R * stride, nsb));
         } else if (a.resid) {
             out = out + (t == tid ? res : a.resid[at]);
         }

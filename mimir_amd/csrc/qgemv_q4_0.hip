@@ -434,11 +434,7 @@ __global__ __launch_bounds__(512) void qgemv_q4_0_i4_kernel(Q4Job job, const uin
         for (int r = 0; r < R; r++) {
             float s = wave_sum(acc[r]);
             if (MODE == kSwiGLU) {
-                const float u = wave_sum(acc[R + r]);
-                const float e = __builtin_exp2f(s * (float)(-1.4426950408889634));
-                const float sg = 1.0f / (1.0f + e);
-                const float a = s * sg;
-                s = a * u;
+                s = silu_times(s, wave_sum(acc[R + r]));
             }
             if (MODE == kSwiGLU && job.act_out) {
                 if (lane == 0) ((float*)(lds_i4 + n16))[r0 + r] = s;  // behind the staged activations
@@ -586,11 +582,7 @@ __global__ __launch_bounds__(512) void qgemv_q4_0_i4_batch_kernel(Q4Job job, con
             for (int r = 0; r < R; r++) {
                 float s = wave_sum(acc[mi][r]);
                 if (MODE == kSwiGLU) {
-                    const float u = wave_sum(acc[mi][R + r]);
-                    const float e = __builtin_exp2f(s * (float)(-1.4426950408889634));
-                    const float sg = 1.0f / (1.0f + e);
-                    const float a = s * sg;
-                    s = a * u;
+                    s = silu_times(s, wave_sum(acc[mi][R + r]));
                 }
                 if (MODE == kSwiGLU && job.act_out) {
                     if (lane == 0) outv[32 * mi + r0 + r] = s;

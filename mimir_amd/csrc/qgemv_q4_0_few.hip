@@ -45,10 +45,6 @@ struct Few {
 };
 enum { kTailPlain = 0, kTailRope = 1, kTailSwiglu = 2 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
-}
-
 template <int ROWS, int HEAD, int TAIL>
 __global__ __launch_bounds__(kThreads) void qgemv_q4_0_few_kernel(Few a) {
     extern __shared__ u32x4 smem[];
@@ -211,12 +207,8 @@ __global__ __launch_bounds__(kThreads) void qgemv_q4_0_few_kernel(Few a) {
         if (result >= live) continue;
         const int64_t at = (int64_t)r * a.N + first + result;
         float out = sum_of(result, r);
-        if (TAIL == kTailSwiglu) {  // swiglu_kernel's arithmetic (llm/model.go:446-448)
-            const float u = sum_of(R + result, r);
-            const float e = __builtin_exp2f(out * (float)(-1.4426950408889634));
-            const float sg = 1.0f / (1.0f + e);
-            const float silu = out * sg;
-            out = silu * u;
+        if (TAIL == kTailSwiglu) {
+            out = silu_times(out, sum_of(R + result, r));
         } else if (a.resid) {
             out = out + (t == tid ? res : a.resid[at]);
         }

@@ -473,18 +473,11 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3)))
         // hold its elements. Largest magnitude and sum over the half's 32 lanes, digits through LDS into the operand's
         // 16-byte pieces (lane 32 h + 8 d + m of the block: digit d of elements 16 h.. of row m).
         uint8_t* stage = smem + 2 * WAVES * 64 * 16;  // 64 pieces
-        const float nl2e = (float)(-1.4426950408889634);
         float scale_j[4];
         int sum_j[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            float v = 0.f;
-            if (n < N) {
-                const float e = __builtin_exp2f(sum[j] * nl2e);
-                const float sg = 1.0f / (1.0f + e);
-                const float a = sum[j] * sg;
-                v = a * up[j];
-            }
+            float v = n < N ? silu_times(sum[j], up[j]) : 0.f;
             // magnitudes as integers order like the floats, with infinities and NaNs above every finite value
             uint32_t mag = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
             mag = max(mag, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mag, 0xb1, 0xf, 0xf, true));
@@ -632,7 +625,6 @@ __global__ __launch_bounds__(256) void rows_norm_act_kernel(float* __restrict__ 
 // rows `stride` floats apart, n a multiple of 32.
 __global__ __launch_bounds__(256) void rows_swiglu_act_kernel(const float* __restrict__ g, const float* __restrict__ u, int64_t stride,
                                                               uint8_t* act, int n) {
-    const float nl2e = (float)(-1.4426950408889634);
     const int m = blockIdx.y, nq = n >> 3, nb = n >> 5;
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= nq) return;  // whole quads: nq is a multiple of 4
@@ -646,14 +638,8 @@ __global__ __launch_bounds__(256) void rows_swiglu_act_kernel(const float* __res
     float l4[4], h4[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        float e = __builtin_exp2f(gl[k] * nl2e);
-        float sg = 1.0f / (1.0f + e);
-        float a = gl[k] * sg;
-        l4[k] = a * ul[k];
-        e = __builtin_exp2f(gh[k] * nl2e);
-        sg = 1.0f / (1.0f + e);
-        a = gh[k] * sg;
-        h4[k] = a * uh[k];
+        l4[k] = silu_times(gl[k], ul[k]);
+        h4[k] = silu_times(gh[k], uh[k]);
     }
     rows_convert_item(l4, h4, act, nb, m % kRows, t >> 2, t & 3);
 }

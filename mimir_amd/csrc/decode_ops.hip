@@ -514,7 +514,7 @@ __global__ __launch_bounds__(256) void argmax_split_kernel(const float* __restri
     const int64_t lo = (int64_t)blockIdx.x * span, hi = lo + span < n ? lo + span : n;
     const float first = row[0];
     unsigned long long* slot = slots + (int64_t)r * kArgmaxBlocks;
-    const unsigned long long spoilt = __hip_atomic_load(slot + kArgmaxBlocks - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long spoilt = slot[kArgmaxBlocks - 1];  // of earlier launches
     int32_t pos = 0, step = 0;
     if (TAIL) pos = tail.state[0], step = tail.state[1];  // read before this row is counted, moved on behind the last row that is
     float best = -__builtin_inff();

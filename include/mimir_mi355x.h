@@ -83,7 +83,7 @@ MI355X_API mi355x_status mi355x_download(void* dst, const void* src, size_t byte
  * MI355X_ERR_INDEX if a gather read an index out of range. */
 MI355X_API mi355x_status mi355x_sync(void* stream);
 /* Frees the scratch memory the library keeps for `stream` on the current device: converted activations,
- * attention's and argmax's partial results and tickets, qgemm_bf16's float32 copies, and the blocks kept aside
+ * attention's partial results and tickets, argmax's candidates, qgemm_bf16's float32 copies, and the blocks kept aside
  * when one of them grew. Waits for the stream first. For hosts that create and destroy streams (the library
  * otherwise keeps a stream's scratch, some 20 MiB and up, for the life of the process). After it, no HIP graph
  * recorded over this library's calls on that stream may be replayed: such a graph points into these blocks.
@@ -509,9 +509,9 @@ MI355X_API int64_t mi355x_backend_graph_replays(void* backend);
  * W once for up to 64 of x, 2 sends them all there (0: by shape).
  * "q4_0.few" = 1 keeps Q4_0 products of two to four rows of x, and steps of two
  * sequences, off the kernel for so few, 2 sends all products it takes there.
- * "kquant.stream" = 1 keeps products of one row of x off the kernel with a
- * workgroup per compute unit, 4 to 16 sends all it takes there, with that many
- * wavefronts a workgroup (0: by shape).
+ * "kquant.stream" = 1 keeps products of one to three rows of x, and the norms in
+ * front of them, off the kernel with a workgroup per compute unit, 4 to 16 sends
+ * all it takes there, one row with that many wavefronts a workgroup (0: by shape).
  * "argmax.spins" = n has the workgroup that chooses a row's index poll n times for
  * the others' candidates before it looks over the row itself (below 0: as often as
  * it was, some tenths of a second).

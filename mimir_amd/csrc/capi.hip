@@ -48,7 +48,7 @@ void set_llama_rows_off(int v);      // llm.hip
 namespace {
 
 // Returns the calling stream's block `which` of the current device, at least `bytes` long, and, where that much is to be had, `wish`
-// bytes (at least `floor` when it has to be allocated); the first `zero_prefix` bytes of a new block are zeroed (tickets).
+// bytes (at least `floor` when it has to be allocated); the first `zero_prefix` bytes of a new block are zeroed (tickets, candidates).
 // Allocates, so it fails under stream capture when the block has to grow: a caller that records a
 // graph runs the call once beforehand, as run_batch does.
 mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, size_t bytes, size_t wish, size_t floor, size_t zero_prefix, const char* what,
@@ -79,12 +79,12 @@ mi355x_status stream_scratch(void* stream, ScratchBlock StreamScratch::*which, s
         }
         if (e != hipSuccess) return capi_fail((mi355x_status)e, "mi355x: hipMalloc(%s scratch, %zu bytes): %s", what, want, hipGetErrorName(e));
         if (zero_prefix) {
-            // on the calling stream, so that the zeros are in place before the first kernel that takes a ticket there
+            // on the calling stream, so that the zeros are in place before the first kernel that reads it
             // (never under capture: the allocation above fails first)
             e = hipMemsetAsync(p, 0, zero_prefix < want ? zero_prefix : want, (hipStream_t)stream);
             if (e != hipSuccess) {
                 (void)hipFree(p);  // nothing has seen it yet
-                return capi_fail((mi355x_status)e, "mi355x: hipMemset(%s tickets): %s", what, hipGetErrorName(e));
+                return capi_fail((mi355x_status)e, "mi355x: hipMemset(%s scratch): %s", what, hipGetErrorName(e));
             }
         }
         if (b.p) mine.retired.push_back(b.p);
@@ -729,7 +729,7 @@ mi355x_status mi355x_argmax(const float* logits, int64_t rows, int64_t n, int32_
 }
 
 // Frees the scratch memory the library holds for `stream` on the current device (converted activations, attention's
-// and argmax's partial results and tickets, qgemm_bf16's float32 copies), blocks kept aside after growth included.
+// partial results and tickets, argmax's candidates, qgemm_bf16's float32 copies), blocks kept aside after growth included.
 // Waits for the stream first. The caller promises that no HIP graph recorded over this library's calls on that
 // stream will be replayed afterwards: such a graph points into these blocks.
 mi355x_status mi355x_stream_release(void* stream) {

@@ -112,7 +112,7 @@ struct Q4RopeTail {
 };
 hipError_t qgemv_q4_0_act_qkv_rope(const void* const W[3], const int64_t n[3], const void* act, float* y, int64_t M, int64_t K,
                                    const Q4RopeTail& rope, const Q4NormHead& norm, const int* tune, hipStream_t st);
-// Two to four rows of x by Q4_0 with a workgroup per compute unit (qgemv_q4_0_few.hip), the bits of one row's kernel. a.act: rows of q4_0_convert_act; null: float32 a.x (16-byte
+// Two to four rows of x by Q4_0 with a workgroup per compute unit (qgemv_q4_0_few.hip): the integers of one row's kernel, their float32 sums within rounding of its. a.act: rows of q4_0_convert_act; null: float32 a.x (16-byte
 // aligned), which every workgroup converts for itself. Two rows alone: a.act, and with norm_w the RMSNorm in front as well (q4_0_norm_head_ok(K)), and then one of the tails: a.W, W1 and W2 q, k (n1 rows)
 // and v behind n0 rows of q, a.N in all, with the rotation and the cache writes; or a.W gate and W1 up of a.N rows, y = SiLU(gate . x) (up . x). ("q4_0.few": 1 never, 2 always)
 struct Q4Few {
@@ -321,7 +321,7 @@ void attention_decode_plan(int64_t B, int H, int HK, int64_t kmax, int* nsplit, 
 size_t attention_decode_workspace_bytes(int64_t B, int H, int D, int nsplit);
 enum { kAttnActQ4 = 0, kAttnActRows = 1, kAttnActKQ = 2 };
 // flagged, if not null: flagged_bytes bytes (at least attention_decode_flagged_bytes, else the tickets are used), zero before the first launch and left zero by every launch, that no
-// other kernel writes: the shares of the keys then travel as (value, flag) pairs to the first share's workgroup, which polls for
+// other kernel writes: the shares of the keys then travel as (value, flag) pairs to the last share's workgroup, which polls for
 // them (a bounded number of times; a pair that never arrives sets kErrInternal in *err), instead of through tickets.
 size_t attention_decode_flagged_bytes(int64_t B, int H, int D, int nsplit);
 void set_attention_decode_handover(int v);  // measurement aid: 1 keeps the ticket protocol

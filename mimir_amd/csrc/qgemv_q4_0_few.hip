@@ -1,6 +1,7 @@
 // Two to four rows of x by Q4_0 weights with a workgroup per compute unit, for gfx950:
-// the integers and float32 operations of one row's kernel (qgemv_q4_0_stream.hip,
-// io/mim/dtype.go:118-123 and backend/cpu/gemv.go:73-104) for each row of x, W read once.
+// the integers and a block's float32 operations of one row's kernel (qgemv_q4_0_stream.hip,
+// io/mim/dtype.go:118-123 and backend/cpu/gemv.go:73-104) for each row of x, W read once; the blocks'
+// sums are within rounding of its (lanes and cuts of a row of W are other ones).
 //
 // The kernel that reads W once for eight rows (qgemv_q4_0_rows.hip) has 32 rows of W a
 // workgroup, so that 4096 rows of W are half the compute units, and works on eight rows of x

@@ -40,11 +40,11 @@ constexpr size_t kActFloorBytes = (size_t)19 << 20;
 constexpr size_t kNoallocScratchBytes = kActFloorBytes;
 
 // Scratch memory of the entry points that need some beyond their arguments (converted activations,
-// partial results and tickets of split attention and argmax, float32 copies of qgemm_bf16's general
+// split attention's partial results and tickets, argmax's candidates, float32 copies of qgemm_bf16's general
 // route). One set per device and stream: calls on different streams never share a block, calls on one
 // stream are ordered by it. A block that has become too small is replaced by a larger one and kept
 // aside: work already queued, and HIP graphs a caller has instantiated over an entry point, may still
-// read and write it, tickets included (a graph keeps the block it was recorded with and stays valid).
+// read and write it, tickets and candidates included (a graph keeps the block it was recorded with and stays valid).
 // Growth at least doubles a block, so what is kept aside stays below the size of the live block.
 // mi355x_stream_release frees everything a stream holds, live and kept aside.
 struct ScratchBlock {
